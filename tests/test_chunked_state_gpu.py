@@ -1,0 +1,183 @@
+"""The recurrences in chunks (chunked_state.hip) against a token-by-token walk in float64, at the
+edges of their tiles and chunks: errors are held to those of the kernels that walk in float32."""
+
+import dataclasses
+
+import pytest
+import torch
+
+from tokensprint_amd.cache import CacheManager, CacheStorage
+from tokensprint_amd.engine.batch import BatchBuilder, StepEntry
+from tokensprint_amd.kernels import load_hip_ops
+from tokensprint_amd.parts.base import SlotStateNeed
+
+pytestmark = pytest.mark.gpu
+
+
+def walk(q, k, v, g, beta, S):
+    """q, k [T, H, N], v [T, H, P], g [T, H, N or 1], beta [T, H] or None, S [H, N, P], float64."""
+    out = torch.empty_like(v)
+    for t in range(q.shape[0]):
+        S = S * g[t].unsqueeze(-1)
+        u = v[t] if beta is None else beta[t, :, None] * (v[t] - (S * k[t].unsqueeze(-1)).sum(1))
+        S = S + k[t].unsqueeze(-1) * u.unsqueeze(1)
+        out[t] = (S * q[t].unsqueeze(-1)).sum(1)
+    return out, S
+
+
+class Requests:
+    def __init__(self, device, shape, count):
+        self.storage = CacheStorage([SlotStateNeed(shape, torch.float32, "s")], 16, 8, count + 2,
+                                    torch.float32, device)
+        self.manager = CacheManager(self.storage.groups, 16, 8, count + 2)
+        self.manager.admit("in front")                     # so that slots do not start at 0
+        self.caches = [self.manager.admit(i) for i in range(count)]
+        self.builder = BatchBuilder(device, len(self.storage.groups))
+        self.state = self.storage.views[0].states["s"]
+        self.state.fill_(3.0)                              # what others left in the slots
+
+    def step(self, spans):
+        entries = []
+        for rc, n in zip(self.caches, spans):
+            self.manager.extend(rc, rc.num_tokens + n)
+            entries.append(StepEntry(rc, [1] * n, rc.num_tokens - n, [n - 1]))
+        return self.builder.build(entries)
+
+
+def in_chunks_and_walked(ops, call, state):
+    """`call`'s output and the state it leaves, by the chunked kernels and by those that walk."""
+    before, kept = state.clone(), ops.dispatch
+    results = []
+    try:
+        for whole in (16, 1 << 30):
+            ops.dispatch = dataclasses.replace(kept, scan_whole_tokens=whole,
+                                               state_space_whole_tokens=whole)
+            state.copy_(before)
+            results.append((call(), state.clone()))
+    finally:
+        ops.dispatch = kept
+    state.copy_(results[0][1])
+    return results
+
+
+def no_further_off(chunked, walked, want):
+    """Both are float32 sums of the same products, in other orders: what the walk is off by is what
+    the sizes and the data give, and a few units in the last place of the largest value."""
+    scale = want.abs().max().item()
+    off = [(x.double().cpu() - want).norm().item() / max(want.norm().item(), 1e-30)
+           for x in (chunked, walked)]
+    top = (chunked.double().cpu() - want).abs().max().item()
+    assert off[0] <= 2 * off[1] + 1e-6, off
+    assert top <= 1e-4 * scale, (top, scale)
+
+
+SPANS = [[130, 1, 64, 17], [1, 65, 3, 200]]
+SIZES = [(4, 2, 128, 128), (2, 2, 64, 64), (3, 1, 10, 6), (2, 1, 36, 70), (1, 1, 65, 17)]
+
+
+@pytest.mark.parametrize("mode", ["fixed", "per_head_plain", "turned", "delta", "delta_per_channel"])
+@pytest.mark.parametrize("heads, kv_heads, dim, vdim", SIZES + [(2, 2, 200, 33)])
+def test_linear_recurrence_in_chunks(gpu_device, mode, heads, kv_heads, dim, vdim):
+    if dim > 128 and mode.startswith("delta"):
+        pytest.skip("the delta rule runs in chunks up to 128 rows")
+    ops = load_hip_ops(gpu_device)
+    qk, inner = kv_heads * dim, heads * vdim
+    requests = Requests(gpu_device, (heads, dim, vdim), 4)
+    want_state = [None] * 4
+    gen = torch.Generator().manual_seed(7)
+    pad = 4 if dim % 4 == 0 else 3                         # rows that can be read 16 bytes wide, or not
+    pairs = dim // 2 - (dim // 2 > 3)
+    angles = torch.outer(torch.arange(400.0), 0.3 ** torch.arange(pairs))
+    table = torch.stack([angles.cos(), angles.sin()], -1).contiguous()
+    for spans in SPANS:
+        batch = requests.step(spans)
+        T = batch.num_tokens
+        x = torch.randn(T, pad + 2 * qk + inner, generator=gen)
+        kw = dict(heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, silu_inputs=mode == "fixed")
+        if mode == "turned" and pairs > 0:
+            kw.update(turn=table.to(gpu_device), k_scale=0.5)
+        beta = None
+        if mode in ("fixed", "turned"):
+            decay = torch.tensor([1.0, 0.0, 0.9, 0.999])[:heads]
+            kw["decay"] = decay.to(gpu_device)
+            g = decay.double()[None, :, None].expand(T, heads, 1)
+        else:
+            n = heads * dim if mode == "delta_per_channel" else heads
+            gates = torch.cat([torch.rand(T, heads, generator=gen),
+                               torch.rand(T, n, generator=gen) ** 0.1], 1)
+            gates[T // 3, heads:] = 0.0                    # everything is forgotten
+            gates[T // 2:, heads:] **= 20                  # and most of it in a few tokens
+            kw.update(gates=gates.to(gpu_device), per_channel=n > heads,
+                      delta=mode.startswith("delta"))
+            g = gates[:, heads:].double().view(T, heads, -1)
+            beta = gates[:, :heads].double() if kw["delta"] else None
+        if beta is not None:                               # unit keys, as the rule has them
+            k = x[:, pad + qk:pad + 2 * qk].view(T, kv_heads, dim)
+            k /= k.norm(dim=-1, keepdim=True)
+        xd = x.double()
+        if mode == "fixed":
+            xd = torch.nn.functional.silu(xd)
+        q, k, v = xd[:, pad:pad + qk], xd[:, pad + qk:pad + 2 * qk], xd[:, pad + 2 * qk:]
+        q, k = (t.reshape(T, kv_heads, dim).repeat_interleave(heads // kv_heads, 1) for t in (q, k))
+        if "turn" in kw:
+            pos = batch.positions.cpu().long()
+            c, s = (table[pos, :, i].double()[:, None] for i in (0, 1))
+
+            def turned(t):
+                t = t.clone()
+                even, odd = t[..., 0:2 * pairs:2].clone(), t[..., 1:2 * pairs:2].clone()
+                t[..., 0:2 * pairs:2], t[..., 1:2 * pairs:2] = even * c - odd * s, odd * c + even * s
+                return t
+            q, k = turned(q), turned(k) * 0.5
+        v = v.reshape(T, heads, vdim)
+        x = x.to(gpu_device)
+        (got, st), (walked, st_walked) = in_chunks_and_walked(
+            ops, lambda: ops.linear_recurrence(x, pad, pad + qk, pad + 2 * qk, batch,
+                                               requests.state, **kw), requests.state)
+        at, want = 0, torch.empty(T, heads, vdim, dtype=torch.float64)
+        for i, n in enumerate(spans):
+            S = want_state[i] if want_state[i] is not None else torch.zeros(heads, dim, vdim,
+                                                                            dtype=torch.float64)
+            rows = slice(at, at + n)
+            want[rows], want_state[i] = walk(q[rows], k[rows], v[rows], g[rows],
+                                             None if beta is None else beta[rows], S)
+            at += n
+        no_further_off(got, walked, want.view(T, inner))
+        slots = batch.slot_ids.long()
+        no_further_off(st[slots], st_walked[slots], torch.stack(want_state))
+        others = [i for i in range(st.shape[0]) if i not in slots.tolist()]
+        assert (st[others] == 3.0).all()
+
+
+@pytest.mark.parametrize("heads, groups, rows, vdim", [(8, 2, 128, 64), (3, 3, 10, 6), (4, 1, 200, 20),
+                                                       (6, 1, 64, 33)])
+def test_state_space_scan_in_chunks(gpu_device, heads, groups, rows, vdim):
+    ops = load_hip_ops(gpu_device)
+    inner, gen = heads * vdim, torch.Generator().manual_seed(8)
+    requests = Requests(gpu_device, (heads, rows, vdim), 4)
+    want_state = [torch.zeros(heads, rows, vdim, dtype=torch.float64) for _ in range(4)]
+    bias, a_log, skip = (torch.randn(heads, generator=gen) for _ in range(3))
+    for spans in SPANS:
+        batch = requests.step(spans)
+        T = batch.num_tokens
+        xbc = torch.randn(T, inner + 2 * groups * rows, generator=gen)
+        proj = torch.randn(T, 5 + heads, generator=gen)
+        args = [t.to(gpu_device) for t in (xbc, proj)]
+        consts = [t.to(gpu_device) for t in (bias, a_log, skip)]
+        (got, st), (walked, st_walked) = in_chunks_and_walked(
+            ops, lambda: ops.ssm_scan(*args, 5, *consts, batch, requests.state, heads=heads,
+                                      vdim=vdim, state_rows=rows, groups=groups), requests.state)
+        d = torch.nn.functional.softplus(proj[:, 5:].double() + bias.double())
+        g = torch.exp(-torch.exp(a_log.double()) * d)[..., None]
+        x = xbc[:, :inner].double().view(T, heads, vdim)
+        B, C = (t.reshape(T, groups, rows).repeat_interleave(heads // groups, 1)
+                for t in xbc[:, inner:].double().split(groups * rows, 1))
+        at, want = 0, torch.empty(T, heads, vdim, dtype=torch.float64)
+        for i, n in enumerate(spans):
+            r = slice(at, at + n)
+            y, want_state[i] = walk(C[r], B[r], d[r][..., None] * x[r], g[r], None, want_state[i])
+            want[r] = y + skip.double()[:, None] * x[r]
+            at += n
+        no_further_off(got, walked, want.view(T, inner))
+        slots = batch.slot_ids.long()
+        no_further_off(st[slots], st_walked[slots], torch.stack(want_state))

@@ -14,15 +14,7 @@
 //
 // A request's state is read only where a portion does not start at position 0, and is
 // written once a portion, by the thread that owns the element.
-#include "common.h"
-#include <type_traits>
-
-struct BatchView {
-  const int* positions;       // [T]
-  const int* entry_of_token;  // [T]
-  const int* q_start;         // [B + 1]
-  const int* slot_ids;        // [B]
-};
+#include "chunked_state.h"
 
 __device__ __forceinline__ float sigmoid_f(float v) { return 1.0f / (1.0f + expf(-v)); }
 __device__ __forceinline__ float silu_f(float v) { return v / (1.0f + expf(-v)); }
@@ -40,19 +32,7 @@ struct RecurrenceArgs {
   const float2* turn;    // [max_pos, turn_dims / 2]: cosine and sine of a pair's angle, or null
   int turn_dims;         // leading channels of q and k that are turned, neighbours in pairs
   float k_scale;         // a factor on k behind its rotation
-  const int* chunks;        // [num_chunks, 3]: first token, one past the last, entry
-  const int* entry_chunks;  // [B + 1]: the chunks of entry e are [entry_chunks[e], entry_chunks[e+1])
-  float* chunk_state;       // [num_chunks, heads, N, P]: local contribution, then start state
-  float* chunk_decay;       // [num_chunks, heads]
 };
-
-// Without the delta rule the recurrence is linear in S, and a long portion is cut into
-// chunks of 64 tokens that run side by side, in three launches: every chunk's recurrence
-// from an empty state (its own contribution and the product of its decays, kRecLocal); per
-// entry, the state in front of every chunk, one after the other, and the state the portion
-// leaves (combine); every chunk once more from its true start state, now writing o
-// (kRecOutput).  Twice the arithmetic, a sixty-fourth of the chain.
-constexpr int kRecWhole = 0, kRecLocal = 1, kRecOutput = 2;
 
 constexpr int kRecThreads = 128;
 constexpr int kRecStage = 16;              // tokens staged in LDS at a time
@@ -103,7 +83,7 @@ __device__ __forceinline__ void read_rows(const float* p, float (&r)[NI]) {
 // TURN: the operands are turned by their token's position as they are staged: channels 2i
 // and 2i + 1 (they stand in neighbouring lanes) by the angle of row `position` of the table,
 // and k is scaled.
-template <int NI, int CPT, int SL, bool DELTA, bool PER_ROW, int MODE = kRecWhole, bool TURN = false>
+template <int NI, int CPT, int SL, bool DELTA, bool PER_ROW, bool TURN = false>
 __global__ __launch_bounds__(kRecThreads) void recurrence_kernel(RecurrenceArgs a) {
   constexpr int kRecSlices = SL, kRecGroups = kRecThreads / SL;
   constexpr int EPT = kRecStage * SL * NI / kRecThreads;   // elements of q a thread stages
@@ -124,21 +104,9 @@ __global__ __launch_bounds__(kRecThreads) void recurrence_kernel(RecurrenceArgs 
   const int col0 = blockIdx.z * BC;
   const int p0 = col0 + cg * CPT;
   const int hk = h / (a.heads / a.kv_heads);
-  int first, end, e;
-  if (MODE == kRecWhole) {
-    e = blockIdx.y;
-    first = a.b.q_start[e];
-    end = a.b.q_start[e + 1];
-  } else {
-    first = a.chunks[3 * blockIdx.y];
-    end = a.chunks[3 * blockIdx.y + 1];
-    e = a.chunks[3 * blockIdx.y + 2];
-  }
-  float* st = MODE == kRecWhole
-      ? a.state + ((int64_t)a.b.slot_ids[e] * a.heads + h) * N * a.P
-      : a.chunk_state + ((int64_t)blockIdx.y * a.heads + h) * N * a.P;
-  const bool fresh = MODE == kRecLocal || (MODE == kRecWhole && a.b.positions[first] == 0);
-  float total_decay = 1.f;
+  const int e = blockIdx.y, first = a.b.q_start[e], end = a.b.q_start[e + 1];
+  float* st = a.state + ((int64_t)a.b.slot_ids[e] * a.heads + h) * N * a.P;
+  const bool fresh = a.b.positions[first] == 0;
   float S[NI][CPT];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
@@ -169,7 +137,7 @@ __global__ __launch_bounds__(kRecThreads) void recurrence_kernel(RecurrenceArgs 
       if (TURN) pt[j] = make_float2(1.f, 0.f);
       if (tt < nt && n < N) {
         const float* row = a.x + (int64_t)(t0 + tt) * a.ld;
-        if (MODE != kRecLocal) pq[j] = row[a.q_col + hk * N + n];     // (a chunk alone gives no o)
+        pq[j] = row[a.q_col + hk * N + n];
         pk[j] = row[a.k_col + hk * N + n];
         if (TURN && n < a.turn_dims)
           pt[j] = a.turn[(int64_t)(pos0 + t0 + tt) * (a.turn_dims / 2) + n / 2];
@@ -198,10 +166,10 @@ __global__ __launch_bounds__(kRecThreads) void recurrence_kernel(RecurrenceArgs 
         // (element n's partner of the pair is the neighbouring lane's; EPT x threads is whole
         // tokens, so the two always hold the same token)
         const float s = (i % NP) & 1 ? pt[j].y : -pt[j].y;
-        if (MODE != kRecLocal) buf[kQ + at] = fmaf(swap_pair(pq[j]), s, pq[j] * pt[j].x);
+        buf[kQ + at] = fmaf(swap_pair(pq[j]), s, pq[j] * pt[j].x);
         buf[kK + at] = a.k_scale * fmaf(swap_pair(pk[j]), s, pk[j] * pt[j].x);
       } else {
-        if (MODE != kRecLocal) buf[kQ + at] = a.silu ? silu_f(pq[j]) : pq[j];
+        buf[kQ + at] = a.silu ? silu_f(pq[j]) : pq[j];
         buf[kK + at] = a.silu ? silu_f(pk[j]) : pk[j];
       }
       if (PER_ROW) buf[kG + at] = pg[j];
@@ -227,7 +195,7 @@ __global__ __launch_bounds__(kRecThreads) void recurrence_kernel(RecurrenceArgs 
     for (int tt = 0; tt < nt; ++tt) {
       float kr[NI], qr[NI], u[CPT], acc[CPT];
       read_rows<NI>(buf + kK + tt * LP + s * SP, kr);
-      if (MODE != kRecLocal) read_rows<NI>(buf + kQ + tt * LP + s * SP, qr);   // one trip to LDS a token
+      read_rows<NI>(buf + kQ + tt * LP + s * SP, qr);   // one trip to LDS a token
 #pragma unroll
       for (int c = 0; c < CPT; ++c) u[c] = buf[kV + tt * BC + cg * CPT + c];
       const float g_all = PER_ROW ? 1.f : buf[kG + tt];
@@ -259,10 +227,6 @@ __global__ __launch_bounds__(kRecThreads) void recurrence_kernel(RecurrenceArgs 
 #pragma unroll
           for (int c = 0; c < CPT; ++c) S[i][c] = fmaf(g_all, S[i][c], kr[i] * u[c]);
       }
-      if (MODE == kRecLocal) {
-        total_decay *= g_all;
-        continue;
-      }
 #pragma unroll
       for (int c = 0; c < CPT; ++c) {
         float a0 = 0.f, a1 = 0.f;
@@ -278,7 +242,6 @@ __global__ __launch_bounds__(kRecThreads) void recurrence_kernel(RecurrenceArgs 
     if (more) commit(lds + (which ^ 1) * kBuf);
     __syncthreads();
   }
-  if (MODE == kRecOutput) return;
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int n = s * NI + i;
@@ -286,42 +249,6 @@ __global__ __launch_bounds__(kRecThreads) void recurrence_kernel(RecurrenceArgs 
     for (int c = 0; c < CPT; ++c)
       if (n < N && p0 + c < a.P) st[(int64_t)n * a.P + p0 + c] = S[i][c];
   }
-  if (MODE == kRecLocal && blockIdx.z == 0 && threadIdx.x == 0)
-    a.chunk_decay[(int64_t)blockIdx.y * a.heads + h] = total_decay;
-}
-
-// A thread per element of S and (head, entry): walks the entry's chunks in order.
-// chunk_state[c] holds the chunk's own contribution and receives the state in front of the
-// chunk; the state behind the last chunk goes to the request's slot.
-__global__ __launch_bounds__(256) void recurrence_combine_kernel(RecurrenceArgs a) {
-  const int h = blockIdx.x, e = blockIdx.y;
-  const int idx = blockIdx.z * blockDim.x + threadIdx.x;
-  const int size = a.N * a.P;
-  if (idx >= size) return;
-  float* st = a.state + ((int64_t)a.b.slot_ids[e] * a.heads + h) * size;
-  float S = a.b.positions[a.b.q_start[e]] == 0 ? 0.f : st[idx];
-  for (int c = a.entry_chunks[e]; c < a.entry_chunks[e + 1]; ++c) {
-    float* cs = a.chunk_state + ((int64_t)c * a.heads + h) * size;
-    const float local = cs[idx];
-    cs[idx] = S;
-    S = fmaf(a.chunk_decay[(int64_t)c * a.heads + h], S, local);
-  }
-  st[idx] = S;
-}
-
-template <int NI, int CPT, bool TURN>
-static void launch_recurrence_chunked(const RecurrenceArgs& a, int num_entries, int num_chunks,
-                                      hipStream_t stream) {
-  constexpr int SL = 8, LP = SL * (NI + 4), BC = kRecThreads / SL * CPT;
-  const dim3 grid(a.heads, num_chunks, (a.P + BC - 1) / BC);
-  const int buf = (kRecStage * (2 * LP + 1 + BC + 1) + 3) / 4 * 4;
-  const size_t lds = (size_t)2 * buf * sizeof(float);
-  hipLaunchKernelGGL((recurrence_kernel<NI, CPT, 8, false, false, kRecLocal, TURN>), grid,
-                     dim3(kRecThreads), lds, stream, a);
-  hipLaunchKernelGGL(recurrence_combine_kernel, dim3(a.heads, num_entries, (a.N * a.P + 255) / 256),
-                     dim3(256), 0, stream, a);
-  hipLaunchKernelGGL((recurrence_kernel<NI, CPT, 8, false, false, kRecOutput, TURN>), grid,
-                     dim3(kRecThreads), lds, stream, a);
 }
 
 template <int NI, int CPT, int SL>
@@ -334,7 +261,7 @@ static int launch_recurrence_cols(const RecurrenceArgs& a, int num_entries, bool
   const size_t lds = (size_t)2 * buf * sizeof(float);
   const void* fn = delta && per_row ? (const void*)recurrence_kernel<NI, CPT, SL, true, true>
                    : delta          ? (const void*)recurrence_kernel<NI, CPT, SL, true, false>
-                   : a.turn ? (const void*)recurrence_kernel<NI, CPT, SL, false, false, kRecWhole, true>
+                   : a.turn ? (const void*)recurrence_kernel<NI, CPT, SL, false, false, true>
                                     : (const void*)recurrence_kernel<NI, CPT, SL, false, false>;
   if (lds > 64 * 1024 &&
       hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
@@ -344,7 +271,7 @@ static int launch_recurrence_cols(const RecurrenceArgs& a, int num_entries, bool
   else if (delta)
     hipLaunchKernelGGL((recurrence_kernel<NI, CPT, SL, true, false>), grid, block, lds, stream, a);
   else if (a.turn)
-    hipLaunchKernelGGL((recurrence_kernel<NI, CPT, SL, false, false, kRecWhole, true>), grid, block,
+    hipLaunchKernelGGL((recurrence_kernel<NI, CPT, SL, false, false, true>), grid, block,
                        lds, stream, a);
   else
     hipLaunchKernelGGL((recurrence_kernel<NI, CPT, SL, false, false>), grid, block, lds, stream, a);
@@ -372,10 +299,11 @@ static int launch_recurrence(const RecurrenceArgs& a, int num_entries, bool delt
 // `gates` [T, ldg] holds beta (heads; read by the delta rule only) and then the decays, one
 // per head or (`per_row`) one per head and row of S.  out [T, heads*P].  `max_q_len`: the
 // most tokens an entry brings (it chooses the launch's shape, never a result).
-// `num_chunks` 0: every entry is walked whole.  Else (without the delta rule) `chunks`
-// [num_chunks, 3] cuts every entry into runs of tokens (first, one past the last, entry), in
-// order, `entry_chunks` [B + 1] says which are whose, and chunk_state [num_chunks, heads, N,
-// P], chunk_decay [num_chunks, heads] are scratch.
+// `num_chunks` 0: every entry is walked whole.  Else `chunks` [num_chunks, 3] cuts every entry
+// into runs of ts_chunk_tokens() tokens, the last of them shorter (first, one past the last,
+// entry), in order,
+// `entry_chunks` [B + 1] says which are whose, and `scratch` has ts_chunked_scratch floats
+// (chunked_state.hip: up to 256 rows of S, with the delta rule up to 128).
 // `turn` [turn_rows, turn_dims / 2] (cosine, sine), or null: without the delta rule and without
 // `silu`, the first `turn_dims` channels of every q and k head are turned by the row of the
 // token's position, channels 2i and 2i + 1 in pairs, and k is multiplied by k_scale.  (The host
@@ -387,8 +315,8 @@ extern "C" int ts_linear_recurrence(const float* x, int ld, int q_col, int k_col
                                     int num_entries, int max_q_len, int heads, int kv_heads,
                                     int N, int P, int silu, int delta, int per_row,
                                     const int* chunks, const int* entry_chunks, int num_chunks,
-                                    float* chunk_state, float* chunk_decay, const float* turn,
-                                    int turn_dims, float k_scale, hipStream_t stream) {
+                                    float* scratch, const float* turn, int turn_dims,
+                                    float k_scale, hipStream_t stream) {
   if (num_tokens <= 0) return 0;
   if (heads <= 0 || kv_heads <= 0 || heads % kv_heads || N <= 0 || P <= 0)
     TS_FAIL("linear_recurrence: bad sizes heads=%d kv_heads=%d dim=%d vdim=%d", heads, kv_heads, N, P);
@@ -405,30 +333,25 @@ extern "C" int ts_linear_recurrence(const float* x, int ld, int q_col, int k_col
   RecurrenceArgs a{x, decay, gates, state, out,
                    BatchView{positions, entry_of_token, q_start, slot_ids},
                    ld, q_col, k_col, v_col, ldg, heads, kv_heads, N, P, silu,
-                   (const float2*)turn, turn_dims, k_scale,
-                   chunks, entry_chunks, chunk_state, chunk_decay};
+                   (const float2*)turn, turn_dims, k_scale};
   if (turn && (delta || per_row || silu || turn_dims < 2 || turn_dims % 2 || turn_dims > N))
     TS_FAIL("linear_recurrence: a rotation of %d of %d channels goes with plain operands and without "
             "the delta rule", turn_dims, N);
   if (!turn && k_scale != 1.f) TS_FAIL("linear_recurrence: a factor on k comes with a rotation");
-  const int ni = (N + 7) / 8;
   if (num_chunks > 0) {
-    if (delta) TS_FAIL("linear_recurrence: the delta rule is not linear in S and runs whole");
-    if (!chunks || !entry_chunks || !chunk_state || !chunk_decay)
+    if (!chunks || !entry_chunks || !scratch)
       TS_FAIL("linear_recurrence: chunked without its lists and scratch");
-    if (ni > 16) TS_FAIL("linear_recurrence: chunks are built for up to 128 key channels");
-    auto run = [&](auto turned) {
-      constexpr bool T = decltype(turned)::value;
-      if (ni <= 2) launch_recurrence_chunked<2, 4, T>(a, num_entries, num_chunks, stream);
-      else if (ni <= 4) launch_recurrence_chunked<4, 4, T>(a, num_entries, num_chunks, stream);
-      else if (ni <= 8) launch_recurrence_chunked<8, 4, T>(a, num_entries, num_chunks, stream);
-      else launch_recurrence_chunked<16, 4, T>(a, num_entries, num_chunks, stream);
-    };
-    if (turn) run(std::true_type{});
-    else run(std::false_type{});
-    TS_CHECK_LAUNCH("linear_recurrence (chunked)");
-    return 0;
+    ChunkedArgs c{};
+    c.x = x, c.state = state, c.out = out, c.b = a.b;
+    c.ld = ld, c.q_col = q_col, c.k_col = k_col, c.v_col = v_col;
+    c.heads = heads, c.kv_heads = kv_heads, c.N = N, c.P = P, c.silu = silu;
+    c.decay = decay, c.gates = gates, c.ldg = ldg, c.delta = delta, c.per_row = per_row;
+    c.turn = a.turn, c.turn_dims = turn_dims, c.k_scale = k_scale;
+    c.chunks = chunks, c.entry_chunks = entry_chunks;
+    c.num_chunks = num_chunks, c.num_entries = num_entries, c.scratch = scratch;
+    return launch_chunked(c, stream);
   }
+  const int ni = (N + 7) / 8;
   const int64_t wide_groups = (int64_t)heads * num_entries * ((P + 63) / 64);
   const bool narrow = max_q_len >= 8 && wide_groups < 1024;
   int rc;

@@ -5,14 +5,7 @@
 //
 // A request's state is read only where a portion does not start at position 0, and is
 // written once a portion, by the thread that owns the element.
-#include "common.h"
-
-struct BatchView {
-  const int* positions;       // [T]
-  const int* entry_of_token;  // [T]
-  const int* q_start;         // [B + 1]
-  const int* slot_ids;        // [B]
-};
+#include "chunked_state.h"
 
 __device__ __forceinline__ float silu_f(float v) { return v / (1.0f + expf(-v)); }
 __device__ __forceinline__ float softplus_f(float v) { return v > 20.f ? v : log1pf(expf(v)); }
@@ -208,12 +201,8 @@ extern "C" int ts_conv_silu(const float* proj, int ld, int col, int channels, in
 // rows of four columns in registers, walks the tokens in order and adds the eight slices of
 // a column's dot product through the wavefront.
 //
-// Steps of few tokens per entry walk each entry whole (kScanWhole).  A long portion is cut
-// into chunks of 64 tokens that run side by side, in three launches: every chunk's
-// recurrence from an empty state (its own contribution and the product of its decays,
-// kScanLocal); per entry, the state in front of every chunk, one after the other, and the
-// state the portion leaves (combine); every chunk once more from its true start state,
-// now writing y (kScanOutput).  Twice the arithmetic, a sixty-fourth of the chain.
+// Steps of few tokens per entry walk each entry whole here; long portions run in chunks of 64
+// tokens as products of matrices (chunked_state.hip).
 struct ScanArgs {
   const float* xbc;       // [T, channels]: x (heads*P) | B (groups*N) | C (groups*N)
   const float* proj;      // [T, ld]: dt at column dt_col
@@ -224,30 +213,21 @@ struct ScanArgs {
   float* y;               // [T, heads*P]
   BatchView b;
   int ld, dt_col, channels, heads, P, N, groups;
-  const int* chunks;      // [num_chunks, 3]: first token, one past the last, entry
-  const int* entry_chunks;  // [B + 1]: the chunks of entry e are [entry_chunks[e], entry_chunks[e+1])
-  float* chunk_state;     // [num_chunks, heads, N, P]: local contribution, then start state
-  float* chunk_decay;     // [num_chunks, heads]
 };
 
 constexpr int kScanSlices = 8;
-constexpr int kScanCols = 32;              // columns of a workgroup of the combine kernel
-constexpr int kScanWhole = 0, kScanLocal = 1, kScanOutput = 2;
 constexpr int kScanThreads = 128;          // the walking kernel: 8 slices x 16 groups of columns
 constexpr int kScanPerThread = 4;          // columns a thread owns
 constexpr int kScanBlockCols = kScanThreads / kScanSlices * kScanPerThread;   // 64
 constexpr int kScanStage = 16;             // tokens staged in LDS at a time
 static_assert(kScanStage * kScanBlockCols == 8 * kScanThreads, "a stage's x: eight loads a thread");
 
-// (The output pass is held to 168 registers so that three wavefronts share a SIMD: its
-// time went from 292 to 220 us at 64 heads of 64 columns and 128 state rows, 2,048 tokens.)
 // Thread (cg, s) = (tid / 8, tid % 8) keeps rows s, s + 8, ... of four columns in registers.
 // Sixteen tokens' operands (B, C, the workgroup's columns of x, the step and the decay,
 // computed once a token) are staged in LDS by all threads together, then walked in order:
 // a token costs a thread 2 NI + 3 LDS reads for 8 NI multiply-adds.
-template <int NI, int MODE>
-__global__ __launch_bounds__(kScanThreads, (MODE == kScanOutput && NI <= 16) ? 3 : 1)
-void ssm_scan_kernel(ScanArgs a) {
+template <int NI>
+__global__ __launch_bounds__(kScanThreads) void ssm_scan_kernel(ScanArgs a) {
   extern __shared__ float lds[];
   const int N = a.N;
   float* B_s = lds;                                  // [stage][N]
@@ -260,22 +240,11 @@ void ssm_scan_kernel(ScanArgs a) {
   const int col0 = blockIdx.z * kScanBlockCols;
   const int p0 = col0 + cg * kScanPerThread;
   const int g = h / (a.heads / a.groups);
-  int first, end, e;
-  if (MODE == kScanWhole) {
-    e = blockIdx.y;
-    first = a.b.q_start[e];
-    end = a.b.q_start[e + 1];
-  } else {
-    first = a.chunks[3 * blockIdx.y];
-    end = a.chunks[3 * blockIdx.y + 1];
-    e = a.chunks[3 * blockIdx.y + 2];
-  }
+  const int e = blockIdx.y, first = a.b.q_start[e], end = a.b.q_start[e + 1];
   const int inner = a.heads * a.P;
-  float* st = MODE == kScanWhole
-      ? a.state + ((int64_t)a.b.slot_ids[e] * a.heads + h) * N * a.P
-      : a.chunk_state + ((int64_t)blockIdx.y * a.heads + h) * N * a.P;
+  float* st = a.state + ((int64_t)a.b.slot_ids[e] * a.heads + h) * N * a.P;
   float S[NI][kScanPerThread];
-  const bool fresh = MODE == kScanLocal || (MODE == kScanWhole && a.b.positions[first] == 0);
+  const bool fresh = a.b.positions[first] == 0;
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int n = s + kScanSlices * i;
@@ -286,7 +255,6 @@ void ssm_scan_kernel(ScanArgs a) {
   const float decay_rate = -expf(a.a_log[h]);
   const float bias = a.dt_bias[h], skip = a.d_skip[h];
   const int b_col = inner + g * N, c_col = inner + a.groups * N + g * N;
-  float total_decay = 1.f;
 
   for (int t0 = first; t0 < end; t0 += kScanStage) {
     const int nt = min(kScanStage, end - t0);
@@ -305,7 +273,7 @@ void ssm_scan_kernel(ScanArgs a) {
           if (i < total) {
             const float* row = a.xbc + (int64_t)(t0 + i / N) * a.channels;
             vb[u] = row[b_col + i % N];
-            if (MODE != kScanLocal) vc[u] = row[c_col + i % N];
+            vc[u] = row[c_col + i % N];
           }
         }
 #pragma unroll
@@ -313,7 +281,7 @@ void ssm_scan_kernel(ScanArgs a) {
           const int i = base + u * kScanThreads + threadIdx.x;
           if (i < total) {
             B_s[i] = vb[u];
-            if (MODE != kScanLocal) C_s[i] = vc[u];
+            C_s[i] = vc[u];
           }
         }
       }
@@ -343,17 +311,6 @@ void ssm_scan_kernel(ScanArgs a) {
         dx[c] = d * x[c];
         acc[c] = 0.f;
       }
-      if (MODE == kScanLocal) {
-        total_decay *= decay;
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-          const int n = s + kScanSlices * i;
-          const float Bv = n < N ? B_s[tt * N + n] : 0.f;
-#pragma unroll
-          for (int c = 0; c < kScanPerThread; ++c) S[i][c] = fmaf(decay, S[i][c], Bv * dx[c]);
-        }
-        continue;
-      }
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
         const int n = s + kScanSlices * i;
@@ -375,7 +332,6 @@ void ssm_scan_kernel(ScanArgs a) {
       }
     }
   }
-  if (MODE == kScanOutput) return;
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int n = s + kScanSlices * i;
@@ -383,111 +339,52 @@ void ssm_scan_kernel(ScanArgs a) {
     for (int c = 0; c < kScanPerThread; ++c)
       if (n < N && p0 + c < a.P) st[(int64_t)n * a.P + p0 + c] = S[i][c];
   }
-  if (MODE == kScanLocal && blockIdx.z == 0 && threadIdx.x == 0)
-    a.chunk_decay[(int64_t)blockIdx.y * a.heads + h] = total_decay;
-}
-
-// Per (head, entry, 32 columns): walks the entry's chunks in order.  chunk_state[c] holds
-// the chunk's own contribution and receives the state in front of the chunk; the state
-// behind the last chunk goes to the request's slot.
-template <int NI>
-__global__ __launch_bounds__(kScanSlices* kScanCols) void ssm_combine_kernel(ScanArgs a) {
-  const int h = blockIdx.x, e = blockIdx.y;
-  const int p = blockIdx.z * kScanCols + threadIdx.x / kScanSlices;
-  const int s = threadIdx.x % kScanSlices;
-  if (p >= a.P) return;
-  const int N = a.N;
-  float* st = a.state + ((int64_t)a.b.slot_ids[e] * a.heads + h) * N * a.P;
-  const bool fresh = a.b.positions[a.b.q_start[e]] == 0;
-  float S[NI];
-#pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const int n = s + kScanSlices * i;
-    S[i] = (!fresh && n < N) ? st[(int64_t)n * a.P + p] : 0.f;
-  }
-  const int c_begin = a.entry_chunks[e], c_end = a.entry_chunks[e + 1];
-  float next[NI], next_decay = 0.f;
-  auto fetch = [&](int c) {                 // a chunk's contribution, ahead of its turn
-    const float* cs = a.chunk_state + ((int64_t)c * a.heads + h) * N * a.P;
-    next_decay = a.chunk_decay[(int64_t)c * a.heads + h];
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int n = s + kScanSlices * i;
-      next[i] = n < N ? cs[(int64_t)n * a.P + p] : 0.f;
-    }
-  };
-  if (c_begin < c_end) fetch(c_begin);
-  for (int c = c_begin; c < c_end; ++c) {
-    float* cs = a.chunk_state + ((int64_t)c * a.heads + h) * N * a.P;
-    float local[NI];
-    const float decay = next_decay;
-#pragma unroll
-    for (int i = 0; i < NI; ++i) local[i] = next[i];
-    if (c + 1 < c_end) fetch(c + 1);
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int n = s + kScanSlices * i;
-      if (n < N) {
-        cs[(int64_t)n * a.P + p] = S[i];
-        S[i] = fmaf(decay, S[i], local[i]);
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const int n = s + kScanSlices * i;
-    if (n < N) st[(int64_t)n * a.P + p] = S[i];
-  }
 }
 
 template <int NI>
-static void launch_scan(const ScanArgs& a, int num_entries, int num_chunks, hipStream_t stream) {
-  const dim3 block(kScanThreads);
+static void launch_scan(const ScanArgs& a, int num_entries, hipStream_t stream) {
   const unsigned z = (a.P + kScanBlockCols - 1) / kScanBlockCols;
   const size_t lds = (size_t)(kScanStage * (2 * a.N + kScanBlockCols + 2)) * sizeof(float);
-  if (num_chunks <= 0) {
-    hipLaunchKernelGGL((ssm_scan_kernel<NI, kScanWhole>), dim3(a.heads, num_entries, z), block,
-                       lds, stream, a);
-    return;
-  }
-  hipLaunchKernelGGL((ssm_scan_kernel<NI, kScanLocal>), dim3(a.heads, num_chunks, z), block, lds,
-                     stream, a);
-  hipLaunchKernelGGL(ssm_combine_kernel<NI>, dim3(a.heads, num_entries, (a.P + kScanCols - 1) / kScanCols),
-                     dim3(kScanSlices * kScanCols), 0, stream, a);
-  hipLaunchKernelGGL((ssm_scan_kernel<NI, kScanOutput>), dim3(a.heads, num_chunks, z), block, lds,
+  hipLaunchKernelGGL(ssm_scan_kernel<NI>, dim3(a.heads, num_entries, z), dim3(kScanThreads), lds,
                      stream, a);
 }
 
-extern "C" int ts_ssm_scan_chunk() { return 64; }
-
 // `num_chunks` 0: every entry is walked whole.  Else `chunks` [num_chunks, 3] cuts every
-// entry into runs of tokens (first, one past the last, entry), in order, `entry_chunks`
-// [B + 1] says which are whose, and chunk_state [num_chunks, heads, N, P], chunk_decay
-// [num_chunks, heads] are scratch.
+// entry into runs of ts_chunk_tokens() tokens, the last one shorter (first, one past the last, entry), in
+// order, `entry_chunks` [B + 1] says which are whose, and `scratch` has ts_chunked_scratch
+// floats.
 extern "C" int ts_ssm_scan(const float* xbc, const float* proj, int ld, int dt_col,
                            const float* dt_bias, const float* a_log, const float* d_skip,
                            float* state, float* y, const int* positions,
                            const int* entry_of_token, const int* q_start, const int* slot_ids,
                            int num_tokens, int num_entries, int heads, int P, int N, int groups,
                            const int* chunks, const int* entry_chunks, int num_chunks,
-                           float* chunk_state, float* chunk_decay, hipStream_t stream) {
+                           float* scratch, hipStream_t stream) {
   if (num_tokens <= 0) return 0;
   if (heads <= 0 || P <= 0 || N <= 0 || groups <= 0 || heads % groups)
     TS_FAIL("ssm_scan: bad sizes heads=%d vdim=%d state=%d groups=%d", heads, P, N, groups);
   if (N > kScanSlices * 32) TS_FAIL("ssm_scan: state of %d rows, at most %d are built", N, kScanSlices * 32);
   if (dt_col < 0 || dt_col + heads > ld) TS_FAIL("ssm_scan: dt columns outside the projection");
-  if (num_chunks > 0 && (!chunks || !entry_chunks || !chunk_state || !chunk_decay))
-    TS_FAIL("ssm_scan: chunked without its lists and scratch");
-  ScanArgs a{xbc, proj, dt_bias, a_log, d_skip, state, y,
-             BatchView{positions, entry_of_token, q_start, slot_ids},
-             ld, dt_col, heads * P + 2 * groups * N, heads, P, N, groups,
-             chunks, entry_chunks, chunk_state, chunk_decay};
+  const BatchView b{positions, entry_of_token, q_start, slot_ids};
+  const int channels = heads * P + 2 * groups * N;
+  if (num_chunks > 0) {
+    if (!chunks || !entry_chunks || !scratch) TS_FAIL("ssm_scan: chunked without its lists and scratch");
+    ChunkedArgs c{};                     // q: C, k: B, v: x times its step size
+    c.x = xbc, c.state = state, c.out = y, c.b = b;
+    c.ld = channels, c.v_col = 0, c.k_col = heads * P, c.q_col = heads * P + groups * N;
+    c.heads = heads, c.kv_heads = groups, c.N = N, c.P = P;
+    c.dt = proj + dt_col, c.ldg = ld, c.dt_bias = dt_bias, c.a_log = a_log, c.d_skip = d_skip;
+    c.k_scale = 1.f, c.chunks = chunks, c.entry_chunks = entry_chunks;
+    c.num_chunks = num_chunks, c.num_entries = num_entries, c.scratch = scratch;
+    return launch_chunked(c, stream);
+  }
+  ScanArgs a{xbc, proj, dt_bias, a_log, d_skip, state, y, b, ld, dt_col, channels, heads, P, N, groups};
   const int ni = (N + kScanSlices - 1) / kScanSlices;
-  if (ni <= 2) launch_scan<2>(a, num_entries, num_chunks, stream);
-  else if (ni <= 4) launch_scan<4>(a, num_entries, num_chunks, stream);
-  else if (ni <= 8) launch_scan<8>(a, num_entries, num_chunks, stream);
-  else if (ni <= 16) launch_scan<16>(a, num_entries, num_chunks, stream);
-  else launch_scan<32>(a, num_entries, num_chunks, stream);
+  if (ni <= 2) launch_scan<2>(a, num_entries, stream);
+  else if (ni <= 4) launch_scan<4>(a, num_entries, stream);
+  else if (ni <= 8) launch_scan<8>(a, num_entries, stream);
+  else if (ni <= 16) launch_scan<16>(a, num_entries, stream);
+  else launch_scan<32>(a, num_entries, stream);
   TS_CHECK_LAUNCH("ssm_scan");
   return 0;
 }

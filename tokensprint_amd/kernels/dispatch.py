@@ -78,12 +78,17 @@ class Dispatch:
     cooperative_workgroups: int = 512
     per_wave_workgroups: int = 4096
 
-    # ---- state-space recurrence.  A step whose longest portion has more tokens than this
-    # is cut into chunks of 64 tokens that run side by side (three launches, twice the
-    # arithmetic); below it every entry is walked whole by one launch.  At 64 heads of 64
-    # columns and 128 state rows a walked token costs about 0.3 us, a chunked portion about
-    # as much as 130 walked tokens whatever its length.
+    # ---- recurrences.  A step whose longest portion has more tokens than this runs in chunks of
+    # 64 tokens as products of matrices, below it every entry is walked whole by one launch.
+    # Three launches have a length of their own (25 to 45 us to the first 64 tokens), a walked
+    # token costs 0.28 us (delta rule, 16 heads of 128 x 128: 128 tokens 44 walked, 47 in chunks;
+    # 512 tokens 155 / 63), 0.23 (8 heads of 64 x 128, a decay per row: 35 / 38 and 123 / 44),
+    # 0.25 (fixed decays, 16 heads of 128 x 128: 38 / 40 and 132 / 44).
     scan_whole_tokens: int = 128
+    #: the state-space scan, whose workgroup walks 64 columns: 1.5 us a token at 64 heads of
+    #: 128 x 64 (16 tokens 30 us walked, 26 in chunks; 64 tokens 98 / 34; 32 heads of 64 x 64:
+    #: 23 / 22 and 70 / 25)
+    state_space_whole_tokens: int = 16
 
     # ---- latent attention on the matrix cores: a wavefront per tile of 16 (token, head)
     # rows.  A step with fewer tiles than `latent_full_tiles` gives every tile a workgroup

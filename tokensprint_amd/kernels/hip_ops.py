@@ -77,6 +77,7 @@ def _load_library() -> ctypes.CDLL:
         path = build()
     lib = ctypes.CDLL(str(path))
     lib.ts_last_error.restype = ctypes.c_char_p
+    lib.ts_chunked_scratch.restype = c_int64
     if lib.ts_abi_version() != ABI_VERSION:
         raise KernelError(f"{path} has interface version {lib.ts_abi_version()}, "
                           f"this package needs {ABI_VERSION}")
@@ -1274,26 +1275,31 @@ class HipOps:
         y = torch.empty(T, inner, dtype=torch.float32, device=self.device)
         # a step with a long portion runs its entries in chunks side by side (the lists are
         # the step's: every recurrent layer of the model uses the same)
-        chunks, entry_chunks, num_chunks = self._scan_chunks(batch)
-        scratch = decays = None
-        if num_chunks:
-            scratch = torch.empty(num_chunks, heads, N, vdim, dtype=torch.float32,
-                                  device=self.device)
-            decays = torch.empty(num_chunks, heads, dtype=torch.float32, device=self.device)
+        chunks, entry_chunks, num_chunks = self._scan_chunks(
+            batch, self.dispatch.state_space_whole_tokens)
+        scratch = self._chunk_scratch(num_chunks, heads, N, vdim)
         self._call(self.lib.ts_ssm_scan, _ptr(xbc), _ptr(proj), proj.shape[1], dt_col,
                    _ptr(dt_bias), _ptr(a_log), _ptr(d_skip), _ptr(state), _ptr(y), pos, eot, qs,
                    slots, T, batch.num_entries, heads, vdim, N, groups, _ptr(chunks),
-                   _ptr(entry_chunks), num_chunks, _ptr(scratch), _ptr(decays), self._stream())
+                   _ptr(entry_chunks), num_chunks, _ptr(scratch), self._stream())
         return y
 
-    def _scan_chunks(self, batch):
-        """(chunk list, chunks of each entry, number of chunks) for a step with a portion long
-        enough to run in chunks side by side, else (None, None, 0).  The lists are the
-        step's: every recurrent layer of the model uses the same."""
-        if batch.max_q_len <= self.dispatch.scan_whole_tokens:
+    def _chunk_scratch(self, num_chunks, heads, rows, cols, delta=False, per_row=False):
+        """What the kernels of a recurrence in chunks hand each other; None without chunks."""
+        if not num_chunks:
+            return None
+        count = self.lib.ts_chunked_scratch(num_chunks, heads, rows, cols, int(delta), int(per_row))
+        return torch.empty(count, dtype=torch.float32, device=self.device)
+
+    def _scan_chunks(self, batch, whole=None):
+        """(chunk list, chunks of each entry, number of chunks) for a step with a portion of more
+        than `whole` tokens (default: the dispatch's), long enough to run in chunks, else
+        (None, None, 0).  The lists are the step's: every recurrent layer of the model uses the
+        same."""
+        if batch.max_q_len <= (self.dispatch.scan_whole_tokens if whole is None else whole):
             return None, None, 0
         if "scan_chunks" not in batch.plans:
-            size, rows, firsts, t0 = self.lib.ts_ssm_scan_chunk(), [], [0], 0
+            size, rows, firsts, t0 = self.lib.ts_chunk_tokens(), [], [0], 0
             for e, n in enumerate(batch.q_lens):
                 rows += [(t0 + c, min(t0 + c + size, t0 + n), e) for c in range(0, n, size)]
                 firsts.append(len(rows))
@@ -1372,20 +1378,16 @@ class HipOps:
             self._check("gates", gates, torch.float32, shape=(T, ldg))
         pos, eot, qs, slots = self._batch_ptrs(batch, T)
         out = torch.empty(T, heads * vdim, dtype=torch.float32, device=self.device)
-        # without the delta rule a long portion runs in chunks side by side
-        chunks = entry_chunks = scratch = decays = None
-        num_chunks = 0
-        if not delta and dim <= 128:
+        # a long portion runs in chunks, as products of matrices
+        chunks, entry_chunks, num_chunks = None, None, 0
+        if dim <= (128 if delta else 256):
             chunks, entry_chunks, num_chunks = self._scan_chunks(batch)
-        if num_chunks:
-            scratch = torch.empty(num_chunks, heads, dim, vdim, dtype=torch.float32,
-                                  device=self.device)
-            decays = torch.empty(num_chunks, heads, dtype=torch.float32, device=self.device)
+        scratch = self._chunk_scratch(num_chunks, heads, dim, vdim, delta, per_channel)
         self._call(self.lib.ts_linear_recurrence, _ptr(x), ld, int(q_col), int(k_col), int(v_col),
                    _ptr(decay), _ptr(gates), ldg, _ptr(state), _ptr(out), pos, eot, qs, slots, T,
                    batch.num_entries, int(batch.max_q_len), heads, kv_heads, dim, vdim,
                    int(bool(silu_inputs)), int(bool(delta)), int(bool(per_channel)),
-                   _ptr(chunks), _ptr(entry_chunks), num_chunks, _ptr(scratch), _ptr(decays),
+                   _ptr(chunks), _ptr(entry_chunks), num_chunks, _ptr(scratch),
                    _ptr(turn), 2 * turn.shape[1] if turn is not None else 0, c_float(k_scale),
                    self._stream())
         return out
