@@ -1,0 +1,99 @@
+"""The float32 path's products and attention on the float32 matrix cores, at the edges of their
+tiles, runs of K and key blocks: against float64, and a row the same to the bit however it is
+batched."""
+
+import pytest
+import torch
+
+from scenarios import paged_scenario
+from tokensprint_amd.kernels import load_hip_ops
+
+pytestmark = pytest.mark.gpu
+
+
+def rand(shape, seed, dtype=torch.float32):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed)).to(dtype)
+
+
+@pytest.mark.parametrize("K", [4, 12, 16, 20, 124, 128, 132, 512, 1024, 1092, 3072])
+@pytest.mark.parametrize("N", [5, 64, 150, 4100])
+def test_product_rows_do_not_depend_on_the_number_of_rows(gpu_device, N, K):
+    """Every kernel that a row count chooses (16, 32 and 64 rows, three tiles) and its edges."""
+    ops = load_hip_ops(gpu_device)
+    x, w = rand((600, K), 1), rand((N, K), 2) * 0.05
+    # |x| |w| summed, times a unit in the last place for every addition on an element's way
+    bound = (x.abs().double() @ w.abs().double().T) * (2.0 ** -24) * (64 + 8 + K / 512)
+    want = x.double() @ w.double().T
+    x, w = x.to(gpu_device), w.to(gpu_device)
+    full = ops.linear(x, w, torch.float32)
+    assert ((full.double().cpu() - want).abs() <= bound).all()
+    for M in (1, 8, 16, 17, 32, 33, 64, 65, 96, 129, 257):
+        assert torch.equal(ops.linear(x[:M].contiguous(), w, torch.float32), full[:M]), M
+        assert torch.equal(ops.linear(x[600 - M:].contiguous(), w, torch.float32), full[600 - M:]), M
+
+
+@pytest.mark.parametrize("x_type, w_type", [(torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16)])
+@pytest.mark.parametrize("M", [3, 40, 70, 300])
+def test_product_of_mixed_types(gpu_device, M, x_type, w_type):
+    ops = load_hip_ops(gpu_device)
+    x, w = rand((M, 200), 3, x_type), (rand((150, 200), 4) * 0.05).to(w_type)
+    want = x.double() @ w.double().T
+    out = ops.linear(x.to(gpu_device), w.to(gpu_device), torch.float32)
+    torch.testing.assert_close(out.double().cpu(), want, rtol=1e-5, atol=1e-5)
+
+
+SPANS = [(0, 1), (63, 1), (64, 1), (0, 70), (15, 130), (500, 33), (0, 17)]
+
+
+@pytest.mark.parametrize("nq, nkv, hd, page", [(16, 8, 128, 16), (6, 2, 48, 32), (5, 1, 16, 16),
+                                               (4, 4, 64, 64), (16, 1, 80, 16), (7, 7, 112, 48)])
+@pytest.mark.parametrize("form", ["plain", "window", "chunk_sink", "extras"])
+def test_attention_against_the_general_kernel(gpu_device, monkeypatch, nq, nkv, hd, page, form):
+    ops = load_hip_ops(gpu_device)
+    batch, cache, table, _ = paged_scenario(gpu_device, torch.float32, nkv=nkv, hd=hd, page_size=page,
+                                            spans=SPANS, seed=5)
+    q = rand((batch.num_tokens, nq, hd), 6).to(gpu_device)
+    kw = dict(num_heads=nq, num_kv_heads=nkv, head_dim=hd, scale=hd ** -0.5, window=None)
+    if form == "window":
+        kw["window"] = 37
+    elif form == "chunk_sink":
+        kw.update(chunk=50, sink=rand((nq,), 7).to(gpu_device))
+    elif form == "extras":
+        kw.update(softcap=3.0, slopes=(0.1 * rand((nq,), 8).abs()).to(gpu_device), q_temp=(0.3, 40),
+                  window=200)
+    assert ops.lib.ts_attention_f32_fits(hd, nq // nkv, page, nkv, 0) == 1
+    # places behind an entry's last key hold whatever the page's last owner left
+    for b, (start, n) in enumerate(SPANS):
+        rest = (start + n) % page
+        if rest:
+            last = table[b, (start + n) // page].item()
+            cache.k_pages[last, :, rest:] = float("nan")
+            cache.v_pages[last, :, :, rest:] = float("nan")
+    out = ops.paged_attention(q, batch, table, cache, **kw)
+    monkeypatch.setattr(ops.lib, "ts_attention_f32_fits", lambda *a: 0)
+    want = ops.paged_attention(q, batch, table, cache, **kw)
+    torch.testing.assert_close(out, want, rtol=2e-5, atol=2e-6)
+
+
+def test_attention_of_a_token_does_not_depend_on_its_step(gpu_device):
+    """Keys counted from position 0 in fixed blocks: a token alone, at the end of a portion and
+    beside others adds up the same."""
+    ops = load_hip_ops(gpu_device)
+    kw = dict(num_heads=16, num_kv_heads=8, head_dim=128, scale=128 ** -0.5, window=None)
+    batch, cache, table, _ = paged_scenario(gpu_device, torch.float32, nkv=8, hd=128, page_size=16,
+                                            spans=[(0, 700), (40, 3)], seed=9)
+    q = rand((batch.num_tokens, 16, 128), 10).to(gpu_device)
+    for window in (None, 100):
+        kw["window"] = window
+        whole = ops.paged_attention(q, batch, table, cache, **kw)
+        for t in (0, 63, 64, 333, 699):
+            import copy
+            one = copy.copy(batch)
+            one.num_tokens = one.num_entries = one.max_q_len = 1
+            one.q_lens, one.starts, one.plans = [1], [t], {}
+            one.positions = batch.positions[t:t + 1].contiguous()
+            one.entry_of_token = torch.zeros(1, dtype=torch.int32, device=gpu_device)
+            one.q_start = torch.tensor([0, 1], dtype=torch.int32, device=gpu_device)
+            one.ctx_len = torch.tensor([t + 1], dtype=torch.int32, device=gpu_device)
+            alone = ops.paged_attention(q[t:t + 1].contiguous(), one, table[:1].contiguous(), cache, **kw)
+            assert torch.equal(alone[0], whole[t]), t

@@ -1,10 +1,14 @@
-// C[M,N] = A[M,K] * W[N,K]^T with float32 fused multiply-adds only: no matrix-core
-// instruction and no reduced-precision mode, whatever the operand types.  This is the
-// product of the float32 path and of any bfloat16 run whose weights are held in 32-bit.
-// Every output element adds its K products in an order fixed by K alone (per lane in
-// index order and then across the lanes of a wavefront; in index order with one
-// accumulator in the tiled kernel, which serves a K that is no multiple of 4), so its value
-// does not depend on which other rows are in the call.
+// C[M,N] = A[M,K] * W[N,K]^T in float32: float32 operands (bfloat16 ones are widened), float32
+// products and sums, no reduced-precision mode.  This is the product of the float32 path and of
+// any bfloat16 run whose weights are held in 32-bit.
+//
+// Every output element adds its K products in an order fixed by K alone, so its value does not
+// depend on which other rows are in the call nor on the kernel that the number of rows chooses.
+// Where K is a multiple of 4: K is cut into stretches of 64, the stretches into eight runs of
+// equal length; a stretch is one chain of float32 matrix-core products (v_mfma_f32_16x16x4_f32;
+// the four products of a step of 16 take elements 4 g + r, g = 0..3, in product r), a run adds its
+// stretches' sums in order and the result the eight runs' sums in order.  Another K adds in index
+// order in one accumulator.
 #include "common.h"
 
 constexpr int kTile = 64;   // output tile edge per workgroup
@@ -56,14 +60,9 @@ __global__ __launch_bounds__(256) void gemm_fma_kernel(const TA* __restrict__ A,
   }
 }
 
-// The kernel for every K that is a multiple of 4: a wavefront per four output columns and
-// up to 16 rows of A, so that a row of W is read by 64 lanes side by side (a kilobyte a load
-// instruction) and a decode step's columns spread over the chip.  Lane l takes elements
-// 4 l .. 4 l + 3 of every stretch of 256 of K, adds its products in index order, and the 64
-// lanes' sums are added in a fixed butterfly: the order depends on K alone, never on M or
-// on which other rows are in the call, so a row's result is the same to the bit however
-// the rows are batched (more than 16 rows are further workgroups along y).  The rows of A
-// are the same for every wavefront and come out of the caches.
+// ---------------------------------------------------------------- K a multiple of 4
+// Matrix operands: lane (g, l) = (lane / 16, lane % 16) holds row l of A or W, elements
+// 4 g .. 4 g + 3 of a step, and rows 4 g + r, column l of the sums.
 typedef __attribute__((ext_vector_type(4))) float f32x4_fma;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4_fma;
 __device__ __forceinline__ f32x4_fma load4_fma(const float* p) { return *(const f32x4_fma*)p; }
@@ -72,125 +71,311 @@ __device__ __forceinline__ f32x4_fma load4_fma(const bf16_t* p) {
   return f32x4_fma{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
 }
 
-constexpr int kColumnsPerWave = 4;
+constexpr int kRuns = 8, kStretch = 4;     // runs of K, steps of a stretch
 
-template <typename TA, typename TW, typename TC, int MR>
-__global__ __launch_bounds__(256) void gemm_fma_rows_kernel(const TA* __restrict__ A,
-                                                            const TW* __restrict__ W,
-                                                            TC* __restrict__ C, int M, int N, int K) {
-  constexpr int CPW = kColumnsPerWave;
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int64_t n0 = ((int64_t)blockIdx.x * 4 + wave) * CPW;
-  if (n0 >= N) return;
-  const int m0 = blockIdx.y * MR;
-  A += (int64_t)m0 * K;
-  C += (int64_t)m0 * N;
-  M -= m0;
-  float acc[MR][CPW];
+// Stretches of a run: the last runs may be shorter or empty.
+__host__ __device__ __forceinline__ int stretches_of_run(int K) {
+  const int stretches = (K + 16 * kStretch - 1) / (16 * kStretch);
+  return (stretches + kRuns - 1) / kRuns;
+}
+
+// Few rows (up to 16 MT): a workgroup takes 16 columns, each of its eight wavefronts a run of K, so
+// a weight is read once, straight into the matrix cores' operands, a stretch ahead of its use.
+// Bound by the rate at which a compute unit takes load instructions: one of W and MT of A
+// (cached) a step.
+template <typename TA, typename TW, typename TC, int MT>
+__global__ __launch_bounds__(kRuns* kWave) void gemm_f32_rows_kernel(
+    const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, int M, int N, int K) {
+  __shared__ __align__(16) float part[kRuns][MT][256];
+  const int run = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int l = lane % 16, g = lane / 16;
+  const int64_t n0 = (int64_t)blockIdx.x * 16;
+  const int m0 = blockIdx.y * 16 * MT;
+  const int steps = (K + 15) / 16, per = stretches_of_run(K) * kStretch;
+  const int begin = run * per, end = min(begin + per, steps);
+  const TW* w_row = W + min(n0 + l, (int64_t)N - 1) * K + 4 * g;
+  const TA* a_row[MT];
 #pragma unroll
-  for (int m = 0; m < MR; ++m)
+  for (int i = 0; i < MT; ++i) a_row[i] = A + (int64_t)min(m0 + 16 * i + l, M - 1) * K + 4 * g;
+  const f32x4_fma zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4_fma sum[MT], w[2][kStretch], a[2][kStretch][MT];
 #pragma unroll
-    for (int c = 0; c < CPW; ++c) acc[m][c] = 0.f;
-  // Few rows (a decode step): the rows of W are read once and come from memory; four
-  // stretches of them are asked for before the first is used, and each again four ahead, so
-  // that a compute unit's few waves keep enough bytes on the way (a decode step's product
-  // has one workgroup a unit; stretch after stretch it ran at a tenth of the memory's
-  // rate).  The rows of A, the same for every wave, come out of the caches one stretch
-  // ahead.  The sums' order is that of the plain loop.
-  if constexpr (MR > 8) {
-    // many rows (a prompt's portion, workgroups enough to hide the waits): stretch after
-    // stretch, a row at a time, so that the sums and not the rows hold the registers
-    for (int k = lane * 4; k < K; k += kWave * 4) {
-      f32x4_fma w[CPW];
+  for (int i = 0; i < MT; ++i) sum[i] = zero;
+  auto fetch = [&](int half, int step0) {
 #pragma unroll
-      for (int c = 0; c < CPW; ++c) w[c] = load4_fma(W + min(n0 + c, (int64_t)N - 1) * K + k);
+    for (int u = 0; u < kStretch; ++u) {
+      // (a step behind the run is read from the run's last place and not used)
+      const int k = min(min(step0 + u, end - 1) * 16, K - 4 - 4 * g);
+      w[half][u] = load4_fma(w_row + k);
 #pragma unroll
-      for (int m = 0; m < MR; ++m) {
-        const f32x4_fma a = load4_fma(A + (int64_t)min(m, M - 1) * K + k);
-#pragma unroll
-        for (int c = 0; c < CPW; ++c)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) acc[m][c] = fmaf(a[e], w[c][e], acc[m][c]);
-      }
+      for (int i = 0; i < MT; ++i) a[half][u][i] = load4_fma(a_row[i] + k);
     }
-  } else {
-    constexpr int kAhead = 4;
-    const int stretches = (K - lane * 4 + kWave * 4 - 1) / (kWave * 4);     // of this lane
-    // (a lane without a stretch i reads the row's last four elements and drops them)
-    auto w_at = [&](int i, int c) {
-      return load4_fma(W + min(n0 + c, (int64_t)N - 1) * K + min(lane * 4 + i * kWave * 4, K - 4));
-    };
-    auto a_at = [&](int i, int m) {
-      return load4_fma(A + (int64_t)min(m, M - 1) * K + min(lane * 4 + i * kWave * 4, K - 4));
-    };
-    f32x4_fma w[kAhead][CPW], a_next[MR];
+  };
+  auto multiply = [&](int half, int step0) {
+    f32x4_fma chain[MT];
 #pragma unroll
-    for (int p = 0; p < kAhead; ++p)
+    for (int i = 0; i < MT; ++i) chain[i] = zero;
 #pragma unroll
-      for (int c = 0; c < CPW; ++c) w[p][c] = w_at(p, c);
+    for (int u = 0; u < kStretch; ++u) {
+      if (step0 + u >= end) break;
+      const bool inside = (step0 + u) * 16 + 4 * g < K;      // (K's last step may be cut)
+      const f32x4_fma wv = inside ? w[half][u] : zero;
 #pragma unroll
-    for (int m = 0; m < MR; ++m) a_next[m] = a_at(0, m);
-    for (int i0 = 0; i0 < stretches; i0 += kAhead) {
+      for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int p = 0; p < kAhead; ++p) {
-        const int i = i0 + p;
-        if (i >= stretches) break;
-        f32x4_fma a[MR];
+        for (int i = 0; i < MT; ++i)
+          chain[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(inside ? a[half][u][i][r] : 0.f, wv[r],
+                                                          chain[i], 0, 0, 0);
+    }
 #pragma unroll
-        for (int m = 0; m < MR; ++m) a[m] = a_next[m];
-        if (i + 1 < stretches) {
-#pragma unroll
-          for (int m = 0; m < MR; ++m) a_next[m] = a_at(i + 1, m);
-        }
-#pragma unroll
-        for (int m = 0; m < MR; ++m)
-#pragma unroll
-          for (int c = 0; c < CPW; ++c)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[m][c] = fmaf(a[m][e], w[p][c][e], acc[m][c]);
-        if (i + kAhead < stretches) {
-#pragma unroll
-          for (int c = 0; c < CPW; ++c) w[p][c] = w_at(i + kAhead, c);
-        }
-      }
+    for (int i = 0; i < MT; ++i) sum[i] += chain[i];
+  };
+  if (begin < end) {
+    fetch(0, begin);
+    for (int s = begin; s < end; s += 2 * kStretch) {
+      if (s + kStretch < end) fetch(1, s + kStretch);
+      multiply(0, s);
+      if (s + kStretch >= end) break;
+      if (s + 2 * kStretch < end) fetch(0, s + 2 * kStretch);
+      multiply(1, s + kStretch);
     }
   }
 #pragma unroll
-  for (int m = 0; m < MR; ++m)
+  for (int i = 0; i < MT; ++i) *(f32x4_fma*)&part[run][i][lane * 4] = sum[i];
+  __syncthreads();
+  for (int e = threadIdx.x; e < MT * 256; e += kRuns * kWave) {
+    const int i = e / 256, row = e % 256 / 16, col = e % 16;
+    const int at = (row / 4 * 16 + col) * 4 + row % 4;
+    float v = 0.f;
 #pragma unroll
-    for (int c = 0; c < CPW; ++c) {
-      float v = acc[m][c];
+    for (int r = 0; r < kRuns; ++r) v += part[r][i][at];
+    const int m = m0 + 16 * i + row;
+    if (m < M && n0 + col < N) C[(int64_t)m * N + n0 + col] = from_f32<TC>(v);
+  }
+}
+
+// Many rows: a BM x BN tile a workgroup.  Its wavefronts stand in G groups of four, a group takes
+// 8 / G runs of K, a wavefront a quarter of the tile, operands through two LDS buffers of KS
+// elements of K a group, those of the turn after the next on their way in registers.  The float32 matrix rate (256
+// operations a cycle and unit) is low enough that LDS and memory keep up with any tile; what
+// counts is that tiles fill the units and that a SIMD has wavefronts enough to hide the trips to
+// LDS and memory, so small products take small tiles and more groups (o and down of the 0.6B
+// shape, 501 rows: 43 us with one group of a 32 x 64 tile, which is as long with 130 rows).
+template <typename TA, typename TW, typename TC, int BM, int BN, int KS, int G>
+__global__ __launch_bounds__(256 * G, BM == 32 ? 4 : BM == 64 ? 2 : 1) void gemm_f32_tile_kernel(
+    const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, int M, int N, int K) {
+  constexpr int TM = BM / 32, TN = BN / 32, LD = KS + 4, Q = KS / 4, ROWS = BM + BN;
+  constexpr int COUNT = ROWS * Q / 256, STEP = 256 / Q, OWN = kRuns / G, SUMS = G == 1 ? 1 : OWN;
+  constexpr int STEPS = KS / 16, TURNS = kStretch / STEPS;       // steps a turn, turns a stretch
+  static_assert(ROWS * Q % 256 == 0 && 256 % Q == 0 && BM % STEP == 0, "whole rows a turn");
+  static_assert(STEPS % 2 == 0 && kStretch % STEPS == 0, "operands in two sets by turns");
+  extern __shared__ __align__(16) float lds[];
+  const int group = __builtin_amdgcn_readfirstlane(threadIdx.x / 256), tid = threadIdx.x % 256;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
+  const int l = lane % 16, g = lane / 16, wm = wave / 2, wn = wave % 2;
+  const int64_t m0 = (int64_t)blockIdx.y * BM, n0 = (int64_t)blockIdx.x * BN;
+  const int per = stretches_of_run(K);
+  const f32x4_fma zero = {0.f, 0.f, 0.f, 0.f};
+  const int row0 = tid / Q;
+  // (a group's part of K; what lies behind K is zeros, which change no sum)
+  int k = group * OWN * per * 16 * kStretch + tid % Q * 4;
+  float* buffers = lds + group * 2 * ROWS * LD;
+  f32x4_fma next[COUNT];
+  auto fetch = [&] {
 #pragma unroll
-      for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-      if (lane == 0 && m < M && n0 + c < N) C[(int64_t)m * N + n0 + c] = from_f32<TC>(v);
+    for (int u = 0; u < COUNT; ++u) {
+      const int row = row0 + u * STEP;     // of A's BM rows, then of W's BN
+      next[u] = zero;
+      if (k < K) {
+        if (u * STEP < BM) next[u] = load4_fma(A + min(m0 + row, (int64_t)M - 1) * K + k);
+        else next[u] = load4_fma(W + min(n0 + row - BM, (int64_t)N - 1) * K + k);
+      }
     }
+    k += KS;
+  };
+  float* put = buffers + row0 * LD + tid % Q * 4;
+  auto commit = [&](int which) {
+#pragma unroll
+    for (int u = 0; u < COUNT; ++u)
+      *(f32x4_fma*)(put + which * ROWS * LD + u * STEP * LD) = next[u];
+  };
+  fetch();
+  commit(0);
+  fetch();
+  __syncthreads();
+  // A step's operands are read from LDS while the step before is multiplied, a turn's first
+  // while the last step of the turn before is: the barrier that says that every wavefront has
+  // put the next turn's operands down, and has read the last of this one's, stands in front
+  // of that step's products.
+  f32x4_fma af[2][TM], wf[2][TN];
+  const float* a_s = buffers + (wm * 16 * TM + l) * LD + 4 * g;
+  const float* w_s = buffers + (BM + wn * 16 * TN + l) * LD + 4 * g;
+  auto read = [&](int which, int u) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+      af[u & 1][i] = *(const f32x4_fma*)(a_s + which * ROWS * LD + 16 * u + 16 * i * LD);
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      wf[u & 1][j] = *(const f32x4_fma*)(w_s + which * ROWS * LD + 16 * u + 16 * j * LD);
+  };
+  read(0, 0);
+  int which = 0;
+  f32x4_fma chain[TM][TN], run[TM][TN], all[SUMS][TM][TN];
+  auto stretch = [&] {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) chain[i][j] = zero;
+#pragma unroll
+    for (int turn = 0; turn < TURNS; ++turn) {
+      commit(which ^ 1);
+      fetch();
+#pragma unroll
+      for (int u = 0; u < STEPS; ++u) {
+        if (u + 1 < STEPS) {
+          read(which, u + 1);
+        } else {
+          __syncthreads();
+          which ^= 1;
+          read(which, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+              chain[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[u & 1][i][r], wf[u & 1][j][r],
+                                                                 chain[i][j], 0, 0, 0);
+      }
+    }
+  };
+  auto whole_run = [&] {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) run[i][j] = zero;
+    for (int s = 0; s < per; ++s) {
+      stretch();
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) run[i][j] += chain[i][j];
+    }
+  };
+  // (one group adds its runs up as they end, several keep theirs apart until all are there)
+#pragma unroll
+  for (int o = 0; o < SUMS; ++o)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) all[o][i][j] = zero;
+  if constexpr (G == 1) {
+    for (int o = 0; o < OWN && o * per * 16 * kStretch < K; ++o) {
+      whole_run();
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) all[0][i][j] += run[i][j];
+    }
+  } else {
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) {
+      whole_run();
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) all[o][i][j] = run[i][j];
+    }
+  }
+  __syncthreads();
+  if (G > 1) {
+    // the other groups' runs through LDS, [group - 1][run][wave][tile][lane]
+    auto at = [&](int gr, int o, int i, int j) {
+      return (f32x4_fma*)(lds + (((((gr - 1) * OWN + o) * 4 + wave) * TM + i) * TN + j) * 256 + lane * 4);
+    };
+    if (group > 0) {
+#pragma unroll
+      for (int o = 0; o < OWN; ++o)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) *at(group, o, i, j) = all[o][i][j];
+    }
+    __syncthreads();
+    if (group > 0) return;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        f32x4_fma v = zero;
+#pragma unroll
+        for (int o = 0; o < OWN; ++o) v += all[o][i][j];
+        for (int gr = 1; gr < G; ++gr)
+#pragma unroll
+          for (int o = 0; o < OWN; ++o) v += *at(gr, o, i, j);
+        all[0][i][j] = v;
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t m = m0 + (wm * TM + i) * 16 + 4 * g + r, n = n0 + (wn * TN + j) * 16 + l;
+        if (m < M && n < N) C[m * N + n] = from_f32<TC>(all[0][i][j][r]);
+      }
+}
+
+template <typename TA, typename TW, typename TC, int BM, int BN, int KS, int G>
+static int launch_tile(const TA* A, const TW* W, TC* C, int M, int N, int K, hipStream_t stream) {
+  constexpr int operands = G * 2 * (BM + BN) * (KS + 4), sums = (G - 1) * (kRuns / G) * BM * BN;
+  const size_t lds = (size_t)(operands > sums ? operands : sums) * sizeof(float);
+  auto* fn = gemm_f32_tile_kernel<TA, TW, TC, BM, BN, KS, G>;
+  if (lds > 64 * 1024 &&
+      hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+    return -1;
+  hipLaunchKernelGGL(fn, dim3((N + BN - 1) / BN, (M + BM - 1) / BM), dim3(256 * G), lds, stream, A, W, C, M, N, K);
+  return 0;
 }
 
 template <typename TA, typename TW, typename TC>
-static void launch_rows(const TA* A, const TW* W, TC* C, int M, int N, int K, hipStream_t stream) {
-  const int columns = (N + 4 * kColumnsPerWave - 1) / (4 * kColumnsPerWave);
-  const dim3 grid(columns, M <= 16 ? 1 : (M + 15) / 16);
-  if (M == 1)
-    hipLaunchKernelGGL((gemm_fma_rows_kernel<TA, TW, TC, 1>), grid, dim3(256), 0, stream, A, W, C, M, N, K);
-  else if (M <= 4)
-    hipLaunchKernelGGL((gemm_fma_rows_kernel<TA, TW, TC, 4>), grid, dim3(256), 0, stream, A, W, C, M, N, K);
-  else if (M <= 8)
-    hipLaunchKernelGGL((gemm_fma_rows_kernel<TA, TW, TC, 8>), grid, dim3(256), 0, stream, A, W, C, M, N, K);
-  else
-    hipLaunchKernelGGL((gemm_fma_rows_kernel<TA, TW, TC, 16>), grid, dim3(256), 0, stream, A, W, C, M, N, K);
+static int launch_f32(const TA* A, const TW* W, TC* C, int M, int N, int K, hipStream_t stream) {
+  const dim3 block(kRuns * kWave), grid((N + 15) / 16);
+  if (M <= 16) {
+    hipLaunchKernelGGL((gemm_f32_rows_kernel<TA, TW, TC, 1>), grid, block, 0, stream, A, W, C, M, N, K);
+    return 0;
+  }
+  if (M <= 32) {
+    hipLaunchKernelGGL((gemm_f32_rows_kernel<TA, TW, TC, 2>), grid, block, 0, stream, A, W, C, M, N, K);
+    return 0;
+  }
+  if (M <= 64) {
+    hipLaunchKernelGGL((gemm_f32_rows_kernel<TA, TW, TC, 4>), grid, block, 0, stream, A, W, C, M, N, K);
+    return 0;
+  }
+  // the largest tile that still gives every unit one
+  auto tiles = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  if (tiles(128, 128) >= 256) return launch_tile<TA, TW, TC, 128, 128, 32, 1>(A, W, C, M, N, K, stream);
+  if (tiles(64, 64) >= 256) return launch_tile<TA, TW, TC, 64, 64, 64, 1>(A, W, C, M, N, K, stream);
+  return launch_tile<TA, TW, TC, 32, 64, 32, 4>(A, W, C, M, N, K, stream);
 }
 
 extern "C" int ts_gemm_fma(const void* a, int a_type, const void* w, int w_type, void* c,
                            int c_type, int M, int N, int K, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0) TS_FAIL("gemm: K=%d", K);
-  // rows of 4 elements must start on 16 (float32) or 8 (bfloat16) bytes for the row kernel
+  // rows of 4 elements must start on 16 (float32) or 8 (bfloat16) bytes for these kernels
   // (a property of K and of the buffers, not of M: which kernel serves a weight never
   // depends on the number of rows)
-  const bool rows_ok = K % 4 == 0 && (((uintptr_t)a | (uintptr_t)w) & 15) == 0 && (M + 15) / 16 <= 65535;
+  const bool rows_ok = K % 4 == 0 && (((uintptr_t)a | (uintptr_t)w) & 15) == 0 && (M + 31) / 32 <= 65535;
   if (rows_ok) {
+    int rc = 0;
     TS_DISPATCH_TYPE(a_type, TA, TS_DISPATCH_TYPE(w_type, TW, TS_DISPATCH_TYPE(c_type, TC,
-        launch_rows<TA, TW, TC>((const TA*)a, (const TW*)w, (TC*)c, M, N, K, stream))));
+        rc = launch_f32<TA, TW, TC>((const TA*)a, (const TW*)w, (TC*)c, M, N, K, stream))));
+    if (rc != 0) TS_FAIL("gemm: a tile needs more LDS than the device gives");
     TS_CHECK_LAUNCH("gemm_fma");
     return 0;
   }

@@ -769,6 +769,19 @@ class HipOps:
                 self._attention_decode(a, batch, num_heads // num_kv_heads)
             else:
                 self._attention_mfma(a, batch, num_heads // num_kv_heads, extras)
+        elif (q.dtype == torch.float32 and cache.k_pages.dtype == torch.float32
+                and self.lib.ts_attention_f32_fits(head_dim, num_heads // num_kv_heads,
+                                                   cache.page_size, num_kv_heads, a.keep) == 1):
+            # the same kernel for portions and single tokens: what a row adds up depends on its
+            # position and window alone
+            m = AttentionMfmaArgs()
+            m.base = a
+            m.rows_per_token, m.num_tiles = num_heads // num_kv_heads, batch.num_entries
+            if batch.max_q_len > 1:
+                tiles, m.num_tiles = self._attention_tiles(batch, 16 // m.rows_per_token,
+                                                           longest_first=True)
+                m.tiles = tiles.data_ptr()
+            self._call(self.lib.ts_attention_f32, byref(m), self._stream())
         else:
             self._call(self.lib.ts_attention_generic, byref(a), _TYPE_CODE[q.dtype],
                        _TYPE_CODE[cache.k_pages.dtype], self._stream())
