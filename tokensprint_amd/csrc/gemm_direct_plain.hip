@@ -6,18 +6,12 @@ static int plain(const DirectArgs& a, hipStream_t stream) {
   const bool deep = layout_deep(a.N, a.K);
   const int mt = gemm_direct_row_tiles(a.M, a.N, 4);
   if (mt == 1) {
-    // float32 results are the output head's, which has columns enough
-    const int cw = std::is_same<TC, float>::value ? 16 : gemm_direct_columns(a.M, a.N);
+    const int cw = gemm_direct_columns(a.M, a.N);
     TS_DIRECT_ROWS(a.M, {
-      if constexpr (std::is_same<TC, float>::value) {
-        if (deep) launch<1, 8, TC, false, false, 4, 4, false, false, 16, AR>(a, stream);
-        else launch<1, 4, TC, false, false, 4, 4, false, false, 16, AR>(a, stream);
-      } else {
-        TS_DIRECT_COLUMNS(cw, {
-          if (deep) launch<1, 8, TC, false, false, 4, 4, false, false, CW, AR>(a, stream);
-          else launch<1, 4, TC, false, false, 4, 4, false, false, CW, AR>(a, stream);
-        })
-      }
+      TS_DIRECT_COLUMNS(cw, {
+        if (deep) launch<1, 8, TC, false, false, 4, 4, false, false, CW, AR>(a, stream);
+        else launch<1, 4, TC, false, false, 4, 4, false, false, CW, AR>(a, stream);
+      })
     })
   } else if (deep) {
     if (mt == 2) launch<2, 8, TC, false, false, 4, 3>(a, stream);

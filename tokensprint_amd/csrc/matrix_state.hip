@@ -15,6 +15,8 @@
 // A request's state is read only where a portion does not start at position 0, and is
 // written once a portion, by the thread that owns the element.
 #include "chunked_state.h"
+#include "gated_norm.h"
+#include <algorithm>
 
 __device__ __forceinline__ float sigmoid_f(float v) { return 1.0f / (1.0f + expf(-v)); }
 __device__ __forceinline__ float silu_f(float v) { return v / (1.0f + expf(-v)); }
@@ -370,20 +372,41 @@ extern "C" int ts_linear_recurrence(const float* x, int ld, int q_col, int k_col
 // it) becomes x / sqrt(sum(x^2) + 1e-6), q also times N^-1/2.  Into gates [T, ldg]:
 // beta = sigmoid(proj[beta_col + h]); g = exp(-exp(A_log[h]) softplus(z[z_col + j] +
 // dt_bias[j])), j over heads or (`per_row`) over heads x N.
-__global__ __launch_bounds__(256) void delta_gates_kernel(
+__global__ __launch_bounds__(1024) void delta_gates_kernel(
     float* __restrict__ qkv, int ld, const float* __restrict__ proj, int ldp, int beta_col,
     const float* __restrict__ z, int ldz, int z_col, const float* __restrict__ a_log,
     const float* __restrict__ dt_bias, float* __restrict__ gates, int ldg, int heads,
     int kv_heads, int N, int per_row) {
   const int64_t t = blockIdx.x;
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, waves = blockDim.x / kWave;
+  // a wavefront's heads: the first kKeep lane-fuls of each in registers between sum and write,
+  // and the next head's on their way while one is summed
+  constexpr int kKeep = 2;
+  const float q_scale = 1.0f / sqrtf((float)N);
+  float next[kKeep];
+  auto fetch = [&](int u) {
+#pragma unroll
+    for (int j = 0; j < kKeep; ++j) {
+      const int i = lane + j * kWave;
+      next[j] = u < 2 * kv_heads && i < N ? qkv[t * ld + (int64_t)u * N + i] : 0.f;
+    }
+  };
+  fetch(wave);
   for (int u = wave; u < 2 * kv_heads; u += waves) {
     float* v = qkv + t * ld + (int64_t)u * N;
-    float ss = 0.f;
-    for (int i = lane; i < N; i += kWave) ss = fmaf(v[i], v[i], ss);
+    float keep[kKeep], ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < kKeep; ++j) keep[j] = next[j];
+    fetch(u + waves);
+#pragma unroll
+    for (int j = 0; j < kKeep; ++j) ss = fmaf(keep[j], keep[j], ss);
+    for (int i = lane + kKeep * kWave; i < N; i += kWave) ss = fmaf(v[i], v[i], ss);
     ss = wave_sum(ss);
-    const float r = (1.0f / sqrtf(ss + 1e-6f)) * (u < kv_heads ? 1.0f / sqrtf((float)N) : 1.f);
-    for (int i = lane; i < N; i += kWave) v[i] *= r;
+    const float r = (1.0f / sqrtf(ss + 1e-6f)) * (u < kv_heads ? q_scale : 1.f);
+#pragma unroll
+    for (int j = 0; j < kKeep; ++j)
+      if (lane + j * kWave < N) v[lane + j * kWave] = keep[j] * r;
+    for (int i = lane + kKeep * kWave; i < N; i += kWave) v[i] *= r;
   }
   const int ng = per_row ? heads * N : heads;
   for (int c = threadIdx.x; c < heads + ng; c += blockDim.x) {
@@ -407,7 +430,9 @@ extern "C" int ts_delta_gates(float* qkv, int ld, const float* proj, int ldp, in
   if (heads <= 0 || kv_heads <= 0 || N <= 0 || 2 * kv_heads * N > ld || beta_col < 0 ||
       beta_col + heads > ldp || z_col < 0 || z_col + ng > ldz || ldg < heads + ng)
     TS_FAIL("delta_gates: sizes do not fit (heads=%d kv_heads=%d dim=%d)", heads, kv_heads, N);
-  hipLaunchKernelGGL(delta_gates_kernel, dim3(rows), dim3(256), 0, stream, qkv, ld, proj, ldp,
+  // few rows: a wavefront a head (16 heads in four rounds of four took 7 us a decode step)
+  const int threads = rows >= 512 ? 256 : std::min(1024, std::max(4, 2 * kv_heads) * kWave);
+  hipLaunchKernelGGL(delta_gates_kernel, dim3(rows), dim3(threads), 0, stream, qkv, ld, proj, ldp,
                      beta_col, z, ldz, z_col, a_log, dt_bias, gates, ldg, heads, kv_heads, N,
                      per_row);
   TS_CHECK_LAUNCH("delta_gates");
@@ -418,7 +443,7 @@ extern "C" int ts_delta_gates(float* qkv, int ld, const float* proj, int ldp, in
 // Each of `groups` equal parts of a row of y is divided by its root mean square, weighed by
 // w (w_len values: one per column of a part, shared by the parts, or one per column of the
 // row; null: not weighed) and multiplied by act(gate[gate_col + column]); act: 0 sigmoid, 1 SiLU.
-// One wavefront per (row, part).
+// One wavefront per (row, part): sizes and places that gated_norm.h does not take.
 template <typename TO>
 __global__ __launch_bounds__(256) void norm_gate_kernel(
     const float* __restrict__ y, const float* __restrict__ gate, int ldgate, int gate_col,
@@ -451,6 +476,13 @@ extern "C" int ts_norm_gate(const float* y, const float* gate, int ldgate, int g
     TS_FAIL("norm_gate: bad sizes inner=%d groups=%d weight=%d gate columns %d..%d of %d", inner,
             groups, w_len, gate_col, gate_col + inner, ldgate);
   const int64_t units = (int64_t)rows * groups;
+  const GatedNormArgs n{y, gate, w, out, units, ldgate, gate_col, w_len == inner / groups,
+                        inner / groups, groups, act, eps};
+  if (gated_norm_fits(n)) {
+    TS_DISPATCH_TYPE(out_type, TO, (launch_gated_norm<TO, false>(n, stream)));
+    TS_CHECK_LAUNCH("norm_gate");
+    return 0;
+  }
   TS_DISPATCH_TYPE(out_type, TO,
                    hipLaunchKernelGGL(norm_gate_kernel<TO>, dim3((unsigned)((units + 3) / 4)),
                                       dim3(256), 0, stream, y, gate, ldgate, gate_col, w, w_len,

@@ -460,26 +460,37 @@ __global__ __launch_bounds__(1024) void norm_token_shift_kernel(
     const int* __restrict__ q_start, const int* __restrict__ slot_ids, int width, float eps) {
   __shared__ float scratch[16];
   const int t = blockIdx.x, nt = blockDim.x;
-  const int e = entry_of_token[t];
-  const int first = q_start[e], last = q_start[e + 1] - 1;
-  const bool is_first = t == first;
-  const bool from_state = is_first && positions[t] > 0;
-  const bool other_last = is_first && last != t;
   const float* x = resid + (int64_t)t * width;
-  const float* xp = resid + (int64_t)(t - 1) * width;
-  const float* xl = resid + (int64_t)last * width;
-  float* st = state + (int64_t)slot_ids[e] * width;
-  // the row, and the one other row this workgroup needs (the row before, or the portion's
-  // last row whose norm goes into the state), both kept in registers
-  const float* y = !is_first ? xp : xl;
-  const bool need_y = !is_first || other_last;
-  float xc[kRowItems], yc[kRowItems];
-  float ss = 0.f, ssy = 0.f;
+  // the row and the weights, asked for before it is known which other rows are wanted
+  float xc[kRowItems], yc[kRowItems], sc[kRowItems], wc[kRowItems], mc[kRowItems];
 #pragma unroll
   for (int k = 0; k < kRowItems; ++k) {
     const int i = threadIdx.x + k * nt;
     xc[k] = i < width ? x[i] : 0.f;
+    wc[k] = i < width ? norm_w[i] : 0.f;
+    mc[k] = i < width ? shift_w[i] : 0.f;
+  }
+  const int e = entry_of_token[t], slot = slot_ids[e];
+  const int first = q_start[e], last = q_start[e + 1] - 1;
+  const bool is_first = t == first;
+  const bool from_state = is_first && positions[t] > 0;
+  const bool other_last = is_first && last != t;
+  const float* xp = resid + (int64_t)(t - 1) * width;
+  const float* xl = resid + (int64_t)last * width;
+  float* st = state + (int64_t)slot * width;
+  // the one other row this workgroup needs (the row before, or the portion's last row whose
+  // norm goes into the state), and the state's where the portion goes on from it
+  const float* y = !is_first ? xp : xl;
+  const bool need_y = !is_first || other_last;
+  float ss = 0.f, ssy = 0.f;
+#pragma unroll
+  for (int k = 0; k < kRowItems; ++k) {
+    const int i = threadIdx.x + k * nt;
     yc[k] = (need_y && i < width) ? y[i] : 0.f;
+    sc[k] = (from_state && i < width) ? st[i] : 0.f;
+  }
+#pragma unroll
+  for (int k = 0; k < kRowItems; ++k) {
     ss += xc[k] * xc[k];
     ssy += yc[k] * yc[k];
   }
@@ -491,22 +502,21 @@ __global__ __launch_bounds__(1024) void norm_token_shift_kernel(
   float ry = r;
   if (need_y) ry = inv_rms(block_sum(ssy, scratch), width, eps);
   TO* o = out + (int64_t)t * width;
-  auto finish = [&](int i, float xv, float yv) {
-    const float w = norm_w[i];
+  auto finish = [&](int i, float xv, float yv, float sv, float w, float mix) {
     const float h = xv * r * w;
     float prev = 0.f;
     if (!is_first) prev = yv * ry * w;
-    else if (from_state) prev = st[i];
-    o[i] = from_f32<TO>(h + (prev - h) * shift_w[i]);
+    else if (from_state) prev = sv;
+    o[i] = from_f32<TO>(h + (prev - h) * mix);
     if (is_first) st[i] = other_last ? yv * ry * w : h;
   };
 #pragma unroll
   for (int k = 0; k < kRowItems; ++k) {
     const int i = threadIdx.x + k * nt;
-    if (i < width) finish(i, xc[k], yc[k]);
+    if (i < width) finish(i, xc[k], yc[k], sc[k], wc[k], mc[k]);
   }
   for (int i = threadIdx.x + kRowItems * nt; i < width; i += nt)
-    finish(i, x[i], need_y ? y[i] : 0.f);
+    finish(i, x[i], need_y ? y[i] : 0.f, from_state ? st[i] : 0.f, norm_w[i], shift_w[i]);
 }
 
 extern "C" int ts_norm_token_shift(const float* resid, const float* norm_w, float eps,

@@ -45,18 +45,28 @@ __global__ __launch_bounds__(256) void stream_add_norm_kernel(
   constexpr int kKeep = 8;
   const int64_t base = (int64_t)blockIdx.x * width;
   if (row) row += (int64_t)blockIdx.x * row_stride;
-  float keep[kKeep], ss = 0.f;
+  // (everything is asked for before the first store, which every later wait would wait for)
+  float keep[kKeep], av[kKeep], bv[kKeep], rv[kKeep], wv[kKeep], ss = 0.f;
 #pragma unroll
   for (int j = 0; j < kKeep; ++j) {
     const int c = j * blockDim.x + threadIdx.x;
-    keep[j] = 0.f;
-    if (c < width) {
-      float v = resid[base + c];
-      v += b ? to_f32(a[base + c]) + to_f32(b[base + c]) : to_f32(a[base + c]);
-      if (row) v += row[c];
-      resid[base + c] = keep[j] = v;
-      ss = fmaf(v, v, ss);
-    }
+    const bool in = c < width;
+    keep[j] = in ? resid[base + c] : 0.f;
+    av[j] = in ? to_f32(a[base + c]) : 0.f;
+    bv[j] = in && b ? to_f32(b[base + c]) : 0.f;
+    rv[j] = in && row ? row[c] : 0.f;
+    wv[j] = in ? w[c] : 0.f;
+  }
+#pragma unroll
+  for (int j = 0; j < kKeep; ++j) {
+    keep[j] += b ? av[j] + bv[j] : av[j];
+    if (row) keep[j] += rv[j];
+    ss = fmaf(keep[j], keep[j], ss);
+  }
+#pragma unroll
+  for (int j = 0; j < kKeep; ++j) {
+    const int c = j * blockDim.x + threadIdx.x;
+    if (c < width) resid[base + c] = keep[j];
   }
   for (int c = kKeep * blockDim.x + threadIdx.x; c < width; c += blockDim.x) {
     float v = resid[base + c];
@@ -69,7 +79,7 @@ __global__ __launch_bounds__(256) void stream_add_norm_kernel(
 #pragma unroll
   for (int j = 0; j < kKeep; ++j) {
     const int c = j * blockDim.x + threadIdx.x;
-    if (c < width) out[base + c] = from_f32<TO>(keep[j] * r * w[c]);
+    if (c < width) out[base + c] = from_f32<TO>(keep[j] * r * wv[j]);
   }
   for (int c = kKeep * blockDim.x + threadIdx.x; c < width; c += blockDim.x)
     out[base + c] = from_f32<TO>(resid[base + c] * r * w[c]);

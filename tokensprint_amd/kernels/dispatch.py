@@ -86,9 +86,12 @@ class Dispatch:
     # 0.25 (fixed decays, 16 heads of 128 x 128: 38 / 40 and 132 / 44).
     scan_whole_tokens: int = 128
     #: the state-space scan, whose workgroup walks 64 columns: 1.5 us a token at 64 heads of
-    #: 128 x 64 (16 tokens 30 us walked, 26 in chunks; 64 tokens 98 / 34; 32 heads of 64 x 64:
-    #: 23 / 22 and 70 / 25)
-    state_space_whole_tokens: int = 16
+    #: 128 x 64 (64 tokens 98 us walked, 34 in chunks), 1.1 at 32 heads of 64 x 64 (70 / 25).
+    #: The line lies higher than that says because a step that short is eager and as long as
+    #: its launches: two more a layer cost it more on the host than the walk does on the GPU
+    #: (45 tokens beside 11 single ones, six such layers of the smaller size: 1.31 ms walked,
+    #: 1.41 in chunks)
+    state_space_whole_tokens: int = 96
 
     # ---- latent attention on the matrix cores: a wavefront per tile of 16 (token, head)
     # rows.  A step with fewer tiles than `latent_full_tiles` gives every tile a workgroup
