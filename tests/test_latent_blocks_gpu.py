@@ -1,0 +1,69 @@
+"""Latent attention of many tiles: every size that has a kernel of its own, rows shorter than
+one, windows and portions that begin and end inside a block of keys, against float32 torch."""
+
+import dataclasses
+
+import pytest
+import torch
+
+from tokensprint_amd.cache import CacheManager, CacheStorage
+from tokensprint_amd.engine.batch import BatchBuilder, StepEntry
+from tokensprint_amd.kernels import load_hip_ops
+from tokensprint_amd.parts.base import PagedLatentNeed
+
+pytestmark = pytest.mark.gpu
+
+
+def rand(shape, seed, scale=1.0):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed)) * scale
+
+
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("window", [None, 1, 63, 65, 130])
+@pytest.mark.parametrize("heads, kv_rank, rot_dim", [
+    (3, 64, 32), (5, 128, 32), (4, 256, 32), (2, 256, 64), (16, 512, 64),
+    (3, 48, 24), (2, 96, 32), (7, 200, 16), (2, 448, 64), (3, 512, 128)])
+def test_tiles_of_one_entry_walk_their_keys_together(gpu_device, monkeypatch, heads, kv_rank,
+                                                     rot_dim, window, out_dtype):
+    ops = load_hip_ops(gpu_device)
+    monkeypatch.setattr(ops, "dispatch", dataclasses.replace(ops.dispatch, latent_full_tiles=1))
+    dl, page = kv_rank + rot_dim, 16
+    scale = 2.0 / dl ** 0.5
+    storage = CacheStorage([PagedLatentNeed(dl, None)], page, 40, 3, torch.bfloat16, gpu_device)
+    manager = CacheManager(storage.groups, page, 40, 3)
+    builder = BatchBuilder(gpu_device, len(storage.groups))
+    view = storage.views[0]
+    view.k_pages.copy_(rand(view.k_pages.shape, 1).to(gpu_device).bfloat16())
+    caches, at = [manager.admit(i) for i in range(3)], [0, 0, 0]
+    sink = rand((heads,), 2).to(gpu_device)
+    for spans in ([63, 1, 17], [2, 64, 47], [66, 65, 1]):
+        entries = []
+        for i, n in enumerate(spans):
+            manager.extend(caches[i], at[i] + n)
+            entries.append(StepEntry(caches[i], [1] * n, at[i], [n - 1]))
+            at[i] += n
+        batch = builder.build(entries)
+        T = batch.num_tokens
+        rows = rand((T, heads * dl), 3, 1.5).to(gpu_device)
+        got = ops.latent_attention(rows, batch, batch.tables[0], view, heads=heads, kv_rank=kv_rank,
+                                   rot_dim=rot_dim, scale=scale, window=window, sink=sink,
+                                   out_dtype=out_dtype).float().view(T, heads, kv_rank)
+        row = 0
+        for b, e in enumerate(entries):
+            keys = torch.arange(e.start + len(e.tokens), device=gpu_device)
+            kv = view.k_pages[batch.tables[0][b, keys // page].long(), keys % page].float()
+            for i in range(len(e.tokens)):
+                p = e.start + i
+                lo = 0 if window is None else max(0, p - window + 1)
+                mine = kv[lo:p + 1]
+                q = rows[row].view(heads, dl).bfloat16().float()
+                w = torch.softmax(torch.cat([(mine @ q.T) * scale, sink.view(1, -1)]), 0)[:-1]
+                want = w.T @ mine[:, :kv_rank]
+                # each weight is rounded to bfloat16 once (8 significant bits: half a unit is 2^-8
+                # of the value), and the result where it is bfloat16
+                bound = 2 ** -8 * (w.T @ mine[:, :kv_rank].abs()) + 1e-4
+                if out_dtype == torch.bfloat16:
+                    bound = bound + 2 ** -8 * (want.abs() + bound)
+                assert bool(((got[row] - want).abs() <= bound).all()), (spans, b, i)
+                row += 1
+

@@ -359,7 +359,9 @@ struct LatentMfmaArgs {
   const float* sink;        // [heads] or null: a score that joins a row's denominator once
 };
 
-constexpr int kLatentPad = 8;     // elements between staged rows: operand reads spread over banks
+// elements between staged rows: with rows of a multiple of 32 elements they lie 8 odd banks of 4
+// bytes apart, eight rows' pieces of 32 bytes (a transposing read's) beside one another
+constexpr int kLatentPad = 16;
 
 // The query operand of a row: elements 32 s + 8 g .. + 7.  (The row's length is a multiple of
 // 8: eight elements are there together or not at all.)
@@ -376,50 +378,89 @@ __device__ __forceinline__ void load_query_row(bf16x8_l (&q)[KS], const float* q
       q[s][j] = (__bf16)(there ? lo4[j] : 0.f);
       q[s][4 + j] = (__bf16)(there ? hi4[j] : 0.f);
     }
+    if (s % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // eight loads in registers at a time
   }
+}
+
+// The four lanes r, r + 16, r + 32, r + 48 hold a row: the sum and the largest of what they
+// have, by the instructions that swap rows of 16 and halves of 32 lanes of two operands.
+__device__ __forceinline__ float row_total(float v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+__device__ __forceinline__ float row_max(float v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
 // Scores, in units of log2, of row r with keys kb + 16 (e / 4) + 4 g + e % 4, the keys staged
 // as rows of `stride` elements at k_s; -inf where the row does not see a key.  Returns the
-// largest of the row's 32.
-template <int KS>
-__device__ __forceinline__ float score_block(float (&sc)[8], const bf16x8_l (&q)[KS],
+// largest of the row's 16 BLK.  FULL: a row of exactly 32 KS elements, whose operands are asked
+// for AHEAD steps before the product that takes them (one read after the other with a branch
+// between them left the matrix cores idle for an LDS latency a step).
+template <int KS, bool FULL, int BLK>
+__device__ __forceinline__ float score_block(float (&sc)[4 * BLK], const bf16x8_l (&q)[KS],
                                              const bf16_t* k_s, int stride, int kb, int dl,
                                              float scale_log2, int pos, int lo, int r, int g) {
-  // two blocks of 16 keys, the reduction over the row in two chains each
-  f32x4_l st[2][2];
+  // BLK blocks of 16 keys, the reduction over the row in two chains each
+  f32x4_l st[BLK][2];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) st[c / 2][c % 2] = f32x4_l{0.f, 0.f, 0.f, 0.f};
+  for (int c = 0; c < 2 * BLK; ++c) st[c / 2][c % 2] = f32x4_l{0.f, 0.f, 0.f, 0.f};
   const bf16_t* kr = k_s + r * stride + 8 * g;
+  constexpr int AHEAD = KS > 10 ? 2 : 3;
+  if constexpr (FULL) {
+    bf16x8_l kop[AHEAD + 1][BLK];
 #pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    if (32 * s < dl) {
-      // (past the row's end the query's elements are zeros: the row's last eight stand in)
-      const int d0 = min(32 * s, dl - 8 - 8 * g);
+    for (int s = 0; s < KS + AHEAD; ++s) {
+      if (s < KS) {
 #pragma unroll
-      for (int blk = 0; blk < 2; ++blk) {
-        const bf16x8_l kop = *(const bf16x8_l*)(kr + 16 * blk * stride + d0);
-        st[blk][s & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kop, q[s], st[blk][s & 1], 0, 0, 0);
+        for (int blk = 0; blk < BLK; ++blk)
+          kop[s % (AHEAD + 1)][blk] = *(const bf16x8_l*)(kr + 16 * blk * stride + 32 * s);
+      }
+      if (s >= AHEAD) {
+        __builtin_amdgcn_sched_barrier(0);
+        const int u = s - AHEAD;
+#pragma unroll
+        for (int blk = 0; blk < BLK; ++blk)
+          st[blk][u & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kop[u % (AHEAD + 1)][blk], q[u],
+                                                                   st[blk][u & 1], 0, 0, 0);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      if (32 * s < dl) {
+        // (past the row's end the query's elements are zeros: the row's last eight stand in)
+        const int d0 = min(32 * s, dl - 8 - 8 * g);
+#pragma unroll
+        for (int blk = 0; blk < BLK; ++blk) {
+          const bf16x8_l kop = *(const bf16x8_l*)(kr + 16 * blk * stride + d0);
+          st[blk][s & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kop, q[s], st[blk][s & 1], 0, 0, 0);
+        }
       }
     }
   }
   float mx = -INFINITY;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
+  for (int e = 0; e < 4 * BLK; ++e) {
     const int key = kb + 16 * (e / 4) + 4 * g + e % 4;
     const float dot = st[e / 4][0][e % 4] + st[e / 4][1][e % 4];
     sc[e] = (key <= pos && key >= lo) ? dot * scale_log2 : -INFINITY;
     mx = fmaxf(mx, sc[e]);
   }
-  mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-  return fmaxf(mx, __shfl_xor(mx, 32, kWave));
+  return row_max(mx);
 }
 
 // Weights of the block's scores relative to m_use; returns this lane's share of their sum.
-__device__ __forceinline__ float weigh_block(bf16x8_l& pv, const float (&sc)[8], float m_use) {
+template <int N>
+__device__ __forceinline__ float weigh_block(__bf16 (&pv)[N], const float (&sc)[N], float m_use) {
   float sum = 0.f;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
+  for (int e = 0; e < N; ++e) {
     const float p = __builtin_amdgcn_exp2f(sc[e] - m_use);
     sum += p;
     pv[e] = (__bf16)p;
@@ -427,32 +468,28 @@ __device__ __forceinline__ float weigh_block(bf16x8_l& pv, const float (&sc)[8],
   return sum;
 }
 
-// O^T += C^T P^T for `DB` blocks of 16 columns from `db0` on.  A lane's column of four keys
-// comes out of LDS by the transposing read (sixteen lanes name four rows' runs of sixteen
-// elements, four elements a lane, and each gets one column of the four rows; columns from
-// kv_rank on, which belong to the key part or the padding, give results that nobody stores).
-template <int DB>
-__device__ __forceinline__ void value_block(f32x4_l (&o)[DB], bf16x8_l pv, const bf16_t* k_s,
-                                            int stride, int kv_rank, int db0, int r, int g) {
+// The C^T operand of 32 keys and 16 columns from `vcol` on.  A lane's column of four keys comes
+// out of LDS by the transposing read (sixteen lanes name four rows' runs of sixteen elements,
+// four elements a lane, and each gets one column of the four rows; columns from kv_rank on,
+// which belong to the key part or the padding, give results that nobody stores).
+__device__ __forceinline__ bf16x8_l value_operand(const bf16_t* vcol, int stride) {
   typedef short s16x4 __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) s16x4* Lds4;
-  const bf16_t* vrow = k_s + (4 * g + r / 4) * stride + 4 * (r % 4) + 16 * db0;
-#pragma unroll
-  for (int db = 0; db < DB; ++db) {
-    if (16 * (db0 + db) < kv_rank) {
-      const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lds4)(vrow + 16 * db));
-      const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lds4)(vrow + 16 * stride + 16 * db));
-      const auto both = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
-      o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_l, both), pv,
-                                                      o[db], 0, 0, 0);
-    }
-  }
+  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lds4)vcol);
+  const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lds4)(vcol + 16 * stride));
+  return __builtin_bit_cast(bf16x8_l, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-// The four lanes r, r + 16, r + 32, r + 48 hold a row: the sum of their shares.
-__device__ __forceinline__ float row_total(float v) {
-  v += __shfl_xor(v, 16, kWave);
-  return v + __shfl_xor(v, 32, kWave);
+// O^T += C^T P^T for `DB` blocks of 16 columns from `db0` on.
+template <int DB, bool FULL>
+__device__ __forceinline__ void value_block(f32x4_l (&o)[DB], bf16x8_l pv, const bf16_t* k_s,
+                                            int stride, int kv_rank, int db0, int r, int g) {
+  const bf16_t* vrow = k_s + (4 * g + r / 4) * stride + 4 * (r % 4) + 16 * db0;
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+    if (FULL || 16 * (db0 + db) < kv_rank)
+      o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(value_operand(vrow + 16 * db, stride), pv,
+                                                      o[db], 0, 0, 0);
 }
 
 // A sink's weight relative to `m_log2`, a largest score in units of log2.
@@ -460,21 +497,32 @@ __device__ __forceinline__ float sink_weight_log2(float sink, float m_log2) {
   return __builtin_amdgcn_exp2f(fminf(sink * 1.44269504088896f - m_log2, 100.f));
 }
 
-// Many tiles: the four wavefronts of a workgroup take four tiles of one entry (the last of an
-// entry's may be empty: such a wavefront only helps load) and walk the union of their keys
-// together.  Each block of 32 cached rows passes through registers into one of two LDS
-// buffers, eight threads a row, sent for while the block before it is worked on; the page of
-// the block after that is looked up meanwhile.
-template <int KS, int DB, typename TO>
-__global__ __launch_bounds__(4 * kWave) void latent_attention_mfma_kernel(LatentMfmaArgs a) {
-  constexpr int PIECES = (4 * KS + 7) / 8;                // 16-byte pieces of a row a thread brings
+// Many tiles: the eight wavefronts of a workgroup take four tiles of one entry (the last of an
+// entry's may be empty) and walk the union of their keys together, blocks of BK cached rows
+// through registers into one of two LDS areas, sent for while the block before is worked on.
+// Two wavefronts score a tile, half of a block's keys each; the largest scores and the weights
+// go through LDS, and for the values every wavefront takes OWN blocks of 16 columns of TILES
+// tiles, so that a value read serves up to four products.  What bounds it is the LDS: 488 KB
+// are read and written for 64 keys and 64 rows of 512 + 64 elements, 3,900 cycles at 128 bytes
+// a cycle beside 2,200 of products, and the two barriers a block.  2,048 tokens of 16 heads
+// over a window of 1,024: 122 us against 317 of the form with four wavefronts, a tile each from
+// first to last, whose reads waited one by one and whose values were read once a tile.
+template <int KS, int DB, int BLK, bool FULL, typename TO>
+__global__ __launch_bounds__(8 * kWave) void latent_attention_mfma_kernel(LatentMfmaArgs a) {
+  constexpr int BK = 32 * BLK, PER_ROW = 8 * kWave / BK;  // threads that bring a row
+  constexpr int PIECES = (4 * KS + PER_ROW - 1) / PER_ROW;   // its 16-byte pieces a thread brings
+  constexpr int GROUPS = DB < 8 ? DB : 8;                 // of columns
+  constexpr int TILES = 4 * GROUPS / 8, OWN = DB / GROUPS;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-  const int dl = a.kv_rank + a.rot_dim, P = a.page_size;
+  __shared__ bf16x8_l p_s[4][BLK][kWave];
+  __shared__ float m_s[4][2][16], c_s[4][16];
+  const int dl = FULL ? 32 * KS : a.kv_rank + a.rot_dim, P = a.page_size;
   const int stride = dl + kLatentPad;
-  bf16_t* bufs = (bf16_t*)lds_raw;                        // [2][32][stride]
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
-  const int tile0 = blockIdx.x * 4, tile = tile0 + wave;
-  const int row0 = a.tiles[3 * tile], nrows = a.tiles[3 * tile + 1];
+  bf16_t* bufs = (bf16_t*)lds_raw;                        // [2][BK][stride]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
+  const int tile0 = blockIdx.x * 4, mine = wave / 2, half = wave % 2;
+  const int row0 = a.tiles[3 * (tile0 + mine)], nrows = a.tiles[3 * (tile0 + mine) + 1];
   const int* tab = a.table + (int64_t)a.tiles[3 * tile0 + 2] * a.table_width;
   const bool row_ok = r < nrows;
   const int my_row = row0 + max(0, min(r, nrows - 1));
@@ -482,97 +530,171 @@ __global__ __launch_bounds__(4 * kWave) void latent_attention_mfma_kernel(Latent
   const int pos_r = a.positions[my_token];
   const int my_pos = row_ok ? pos_r : -1;
   const int lo_r = a.window > 0 ? max(0, pos_r - a.window + 1) : 0;
-  // the keys of the whole workgroup: from the first tile's first token to the last token
-  const int pos_first = a.positions[a.tiles[3 * tile0] / a.heads];
-  const int lo_t = a.window > 0 ? max(0, pos_first - a.window + 1) : 0;
-  int hi_t = pos_first;
-  for (int w = 0; w < 4; ++w) {
-    const int n = a.tiles[3 * (tile0 + w) + 1];
-    if (n > 0) hi_t = max(hi_t, a.positions[(a.tiles[3 * (tile0 + w)] + n - 1) / a.heads]);
-  }
-  const int k_begin = (lo_t / 32) * 32, k_end = hi_t + 1;
-  // the wavefront's own first and last visible keys: blocks outside are not its business
-  const int tile_last = __builtin_amdgcn_readfirstlane(nrows) > 0
-      ? a.positions[(row0 + nrows - 1) / a.heads] : -1;
-  const int tile_lo = __builtin_amdgcn_readfirstlane(a.window > 0
-      ? max(0, a.positions[row0 / a.heads] - a.window + 1) : 0);
-
-  const int key_l = threadIdx.x / 8, piece = threadIdx.x % 8;
-  const int parts = dl / 8;
-  auto look_up = [&](int kb) {
-    const int j = kb + key_l;
-    return (j >= lo_t && j <= hi_t) ? tab[j / P] : -1;
-  };
-  bf16x8_l held[PIECES];
-  auto fetch = [&](int kb, int page) {
-    const bf16_t* row = a.pages + ((int64_t)max(page, 0) * P + (kb + key_l) % P) * dl;
+  // the tiles' first and last visible keys (blocks outside are not a tile's business), and the
+  // keys of the whole workgroup: from the first tile's first token to the last token
+  int first[4], last[4], hi_t = 0;
 #pragma unroll
-    for (int i = 0; i < PIECES; ++i) held[i] = *(const bf16x8_l*)(row + 8 * min(piece + 8 * i, parts - 1));
-  };
-  auto commit = [&](bf16_t* buf, int page) {
-    const bf16x8_l zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  for (int t = 0; t < 4; ++t) {
+    const int at = a.tiles[3 * (tile0 + t)], n = a.tiles[3 * (tile0 + t) + 1];
+    const int p0 = a.positions[at / a.heads];
+    const int p1 = n > 0 ? a.positions[(at + n - 1) / a.heads] : -1;
+    first[t] = __builtin_amdgcn_readfirstlane(a.window > 0 ? max(0, p0 - a.window + 1) : 0);
+    last[t] = __builtin_amdgcn_readfirstlane(p1);
+    hi_t = max(hi_t, last[t]);
+  }
+  const int lo_t = first[0];
+  const int k_begin = (lo_t / 32) * 32, k_end = hi_t + 1;
+
+  const int key_l = threadIdx.x / PER_ROW, piece = threadIdx.x % PER_ROW;
+  const int parts = dl / 8;
+  // (rows that no tile sees are stood in for by the nearest that one does)
+  auto visible = [&](int kb) { return max(lo_t, min(kb + key_l, hi_t)); };
+  auto look_up = [&](int kb) { return tab[visible(kb) / P]; };
+  typedef bf16x8_l Pieces[PIECES];
+  auto fetch = [&](Pieces& held, int kb, int page) {
+    const bf16_t* row = a.pages + ((int64_t)page * P + visible(kb) % P) * dl;
 #pragma unroll
     for (int i = 0; i < PIECES; ++i)
-      if (piece + 8 * i < parts)
-        *(bf16x8_l*)(buf + key_l * stride + 8 * (piece + 8 * i)) = page >= 0 ? held[i] : zero;
+      held[i] = *(const bf16x8_l*)(row + 8 * min(piece + PER_ROW * i, parts - 1));
   };
-  int page = look_up(k_begin), page_next = look_up(k_begin + 32);
-  fetch(k_begin, page);
+  auto commit = [&](bf16_t* buf, const Pieces& held) {
+    bf16_t* row = buf + key_l * stride + 8 * piece;
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i)
+      if (piece + PER_ROW * i < parts) *(bf16x8_l*)(row + 8 * PER_ROW * i) = held[i];
+  };
+  int page = look_up(k_begin + BK);
+  {
+    Pieces held;
+    fetch(held, k_begin, look_up(k_begin));
+    commit(bufs, held);
+  }
   bf16x8_l q[KS];
   load_query_row<KS>(q, a.qa + (int64_t)my_token * a.q_ld + my_head * dl, dl, g);
-  f32x4_l o[DB];
+  const int t0 = wave / GROUPS * TILES, col0 = wave % GROUPS * OWN;
+  f32x4_l o[TILES][OWN];
 #pragma unroll
-  for (int db = 0; db < DB; ++db) o[db] = f32x4_l{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < TILES; ++t)
+#pragma unroll
+    for (int db = 0; db < OWN; ++db) o[t][db] = f32x4_l{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;            // l: this lane's share of the row's sum
-  commit(bufs, page);
   __syncthreads();
   const float scale_log2 = a.scale * 1.44269504088896341f;
   int which = 0;
-  for (int kb = k_begin; kb < k_end; kb += 32, which ^= 1) {
-    const bool more = kb + 32 < k_end;
-    if (more) {
-      page = page_next;
-      fetch(kb + 32, page);
-      page_next = look_up(kb + 64);
+  for (int kb = k_begin; kb < k_end; kb += BK, which ^= 1) {
+    // the next block's rows, in flight while this one is scored (behind the last block the last
+    // row again: under a condition the registers would be taken through the whole loop)
+    Pieces held;
+    fetch(held, kb + BK, page);
+    page = look_up(kb + 2 * BK);
+    const bf16_t* k_s = bufs + which * BK * stride;
+    bool sees[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) sees[t] = kb <= last[t] && kb + BK - 1 >= first[t];
+    const bool scoring = mine == 0 ? sees[0] : mine == 1 ? sees[1] : mine == 2 ? sees[2] : sees[3];
+    float sc[4 * BLK];
+    if (scoring) {
+      const float mx = score_block<KS, FULL, BLK>(sc, q, k_s + half * 16 * BLK * stride, stride,
+                                                  kb + half * 16 * BLK, dl, scale_log2, my_pos, lo_r, r, g);
+      if (g == 0) m_s[mine][half][r] = mx;
     }
-    if (kb <= tile_last && kb + 31 >= tile_lo) {
-      const bf16_t* k_s = bufs + which * 32 * stride;
-      float sc[8];
-      bf16x8_l pv;
-      const float m_new = fmaxf(m, score_block<KS>(sc, q, k_s, stride, kb, dl, scale_log2, my_pos, lo_r, r, g));
+    __syncthreads();                       // the largest scores are there, the values before read
+    if (scoring) {
+      const float m_new = fmaxf(m, fmaxf(m_s[mine][0][r], m_s[mine][1][r]));
       // (a finite stand-in while the row has seen no key makes every exponential zero)
       const float m_use = fmaxf(m_new, -1e30f);
       const float corr = __builtin_amdgcn_exp2f(m - m_use);
+      __bf16 pv[4 * BLK];
       l = l * corr + weigh_block(pv, sc, m_use);
       m = m_new;
-      if (__builtin_amdgcn_ballot_w64(corr != 1.f) != 0) {
+      __bf16* at = (__bf16*)&p_s[mine][BLK == 2 ? half : 0][lane] + (BLK == 2 ? 0 : 4 * half);
 #pragma unroll
-        for (int db = 0; db < DB; ++db) o[db] = o[db] * corr;
+      for (int e = 0; e < 4 * BLK; ++e) at[e] = pv[e];
+      if (half == 0 && g == 0) c_s[mine][r] = corr;
+    }
+    commit(bufs + (which ^ 1) * BK * stride, held);
+    __syncthreads();                       // the weights and the next block's rows are there
+    // everything the values' products take is asked for before the first of them
+    const bf16_t* vrow = k_s + (4 * g + r / 4) * stride + 4 * (r % 4) + 16 * col0;
+    bf16x8_l v[BLK][OWN], pv[BLK][TILES];
+    float corr[TILES];
+    bool seen[TILES], turn = false;
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+      seen[t] = TILES == 4 || t0 == 0 ? sees[t] : sees[(t + TILES) % 4];
+      corr[t] = c_s[t0 + t][r];
+    }
+#pragma unroll
+    for (int c = 0; c < BLK; ++c) {
+#pragma unroll
+      for (int db = 0; db < OWN; ++db)
+        if (FULL || 16 * (col0 + db) < a.kv_rank)
+          v[c][db] = value_operand(vrow + 32 * c * stride + 16 * db, stride);
+#pragma unroll
+      for (int t = 0; t < TILES; ++t) pv[c][t] = p_s[t0 + t][c][lane];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+      if (!seen[t]) corr[t] = 1.f;
+      turn = turn || corr[t] != 1.f;
+    }
+    if (__builtin_amdgcn_ballot_w64(turn) != 0) {
+#pragma unroll
+      for (int t = 0; t < TILES; ++t)
+#pragma unroll
+        for (int db = 0; db < OWN; ++db) o[t][db] = o[t][db] * corr[t];
+    }
+#pragma unroll
+    for (int t = 0; t < TILES; ++t)
+      if (seen[t]) {
+#pragma unroll
+        for (int c = 0; c < BLK; ++c)
+#pragma unroll
+          for (int db = 0; db < OWN; ++db)
+            if (FULL || 16 * (col0 + db) < a.kv_rank)
+              o[t][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[c][db], pv[c][t], o[t][db], 0, 0, 0);
       }
-      value_block<DB>(o, pv, k_s, stride, a.kv_rank, 0, r, g);
-    }
-    if (more) commit(bufs + (which ^ 1) * 32 * stride, page);
-    __syncthreads();
   }
-  l = row_total(l);
-  if (!row_ok) return;
-  if (a.sink) l += sink_weight_log2(a.sink[my_head], m);
-  const float inv = l > 0.f ? 1.0f / l : 0.f;
-  TO* orow = (TO*)a.out + (int64_t)my_row * a.kv_rank;
+  // the rows' sums, then what a row's result is multiplied by
+  const float share = row_total(l);
+  __syncthreads();
+  if (g == 0) m_s[mine][half][r] = share;
+  __syncthreads();
+  if (half == 0 && g == 0) {
+    float sum = m_s[mine][0][r] + m_s[mine][1][r];
+    if (a.sink) sum += sink_weight_log2(a.sink[my_head], m);
+    c_s[mine][r] = sum > 0.f ? 1.0f / sum : 0.f;
+  }
+  __syncthreads();
+  typedef TO out4 __attribute__((ext_vector_type(4)));
 #pragma unroll
-  for (int db = 0; db < DB; ++db)
+  for (int t = 0; t < TILES; ++t) {
+    if (r >= a.tiles[3 * (tile0 + t0 + t) + 1]) continue;
+    const float inv = c_s[t0 + t][r];
+    TO* orow = (TO*)a.out + (int64_t)(a.tiles[3 * (tile0 + t0 + t)] + r) * a.kv_rank;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int d = 16 * db + 4 * g + e;
-      if (d < a.kv_rank) orow[d] = from_f32<TO>(o[db][e] * inv);
+    for (int db = 0; db < OWN; ++db) {
+      const int d = 16 * (col0 + db) + 4 * g;
+      if constexpr (FULL) {
+        out4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = from_f32<TO>(o[t][db][e] * inv);
+        *(out4*)(orow + d) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (d + e < a.kv_rank) orow[d + e] = from_f32<TO>(o[t][db][e] * inv);
+      }
     }
+  }
 }
 
 // Few tiles: a workgroup per (tile, share of its keys).  Of every 32 NW keys each of the NW
 // wavefronts stages and scores 32; with the rows' largest scores and the weights exchanged
 // through LDS, each then adds up its share of the columns over all of them.  With one share
 // of the keys the rows are finished here, else the share's results go to the merge kernel.
-template <int KS, int DB, int NW, typename TO>
+template <int KS, int DB, bool FULL, int NW, typename TO>
 __global__ __launch_bounds__(NW* kWave) void latent_attention_split_kernel(LatentMfmaArgs a) {
   constexpr int PIECES = (4 * KS + 7) / 8, OWN = (DB + NW - 1) / NW;
   // rows a lane's loads are in flight for at once: as many as registers allow
@@ -580,7 +702,7 @@ __global__ __launch_bounds__(NW* kWave) void latent_attention_split_kernel(Laten
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];   // [NW][32][stride]
   __shared__ bf16x8_l p_s[NW][kWave];
   __shared__ float m_s[NW][16], l_s[NW][16];
-  const int dl = a.kv_rank + a.rot_dim, P = a.page_size;
+  const int dl = FULL ? 32 * KS : a.kv_rank + a.rot_dim, P = a.page_size;
   const int stride = dl + kLatentPad;
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
   bf16_t* all_s = (bf16_t*)lds_raw;
@@ -644,7 +766,7 @@ __global__ __launch_bounds__(NW* kWave) void latent_attention_split_kernel(Laten
     if (kb0 == k_begin) load_query_row<KS>(q, a.qa + (int64_t)my_token * a.q_ld + my_head * dl, dl, g);
     // (a wavefront's LDS accesses are carried out in order: its own rows need no barrier)
     float sc[8];
-    const float mx = score_block<KS>(sc, q, k_s, stride, kb, dl, scale_log2, my_pos, lo_r, r, g);
+    const float mx = score_block<KS, FULL, 2>(sc, q, k_s, stride, kb, dl, scale_log2, my_pos, lo_r, r, g);
     if (g == 0) m_s[wave][r] = mx;
     __syncthreads();                       // every wavefront's rows and largest scores are there
     float m_new = m;
@@ -652,16 +774,17 @@ __global__ __launch_bounds__(NW* kWave) void latent_attention_split_kernel(Laten
     for (int w = 0; w < NW; ++w) m_new = fmaxf(m_new, m_s[w][r]);
     const float m_use = fmaxf(m_new, -1e30f);
     const float corr = __builtin_amdgcn_exp2f(m - m_use);
-    bf16x8_l pv;
+    __bf16 pv[8];
     l = l * corr + weigh_block(pv, sc, m_use);
     m = m_new;
-    p_s[wave][lane] = pv;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) p_s[wave][lane][e] = pv[e];
     __syncthreads();                       // and every wavefront's weights
 #pragma unroll
     for (int db = 0; db < OWN; ++db) o[db] = o[db] * corr;
 #pragma unroll 1
     for (int w = 0; w < NW; ++w)
-      value_block<OWN>(o, p_s[w][lane], all_s + w * 32 * stride, stride, a.kv_rank, wave * OWN, r, g);
+      value_block<OWN, FULL>(o, p_s[w][lane], all_s + w * 32 * stride, stride, a.kv_rank, wave * OWN, r, g);
     __syncthreads();                       // before the areas are written again
   }
   const float share = row_total(l);
@@ -752,20 +875,22 @@ static int allow_lds(const void* kernel, size_t bytes, size_t* allowed) {
 
 constexpr size_t kLatentLds = 154 * 1024;      // of a compute unit's 160 KB, beside weights and statistics
 
-template <int KS, int DB, typename TO>
+template <int KS, int DB, bool FULL, typename TO>
 static int launch_latent_typed(const LatentMfmaArgs& a, int num_tiles, int waves, hipStream_t stream) {
   const size_t block = (size_t)32 * (a.kv_rank + a.rot_dim + kLatentPad) * sizeof(bf16_t);
   if (waves == 4) {
+    // two areas of 64 rows where they fit, else of 32
+    constexpr int BLK = (size_t)4 * 32 * (32 * KS + kLatentPad) * sizeof(bf16_t) <= kLatentLds ? 2 : 1;
     static size_t allowed = 48 * 1024;         // per instantiation, here and below
-    auto kernel = latent_attention_mfma_kernel<KS, DB, TO>;
-    if (allow_lds((const void*)kernel, 2 * block, &allowed)) return -1;
-    hipLaunchKernelGGL(kernel, dim3(num_tiles / 4), dim3(4 * kWave), 2 * block, stream, a);
+    auto kernel = latent_attention_mfma_kernel<KS, DB, BLK, FULL, TO>;
+    if (allow_lds((const void*)kernel, 2 * BLK * block, &allowed)) return -1;
+    hipLaunchKernelGGL(kernel, dim3(num_tiles / 4), dim3(8 * kWave), 2 * BLK * block, stream, a);
     return 0;
   }
   // four wavefronts' rows in LDS at once where a row is short enough, else two's
   constexpr int NW = (size_t)4 * 32 * (32 * KS + kLatentPad) * sizeof(bf16_t) <= kLatentLds ? 4 : 2;
   static size_t allowed = 48 * 1024;
-  auto kernel = latent_attention_split_kernel<KS, DB, NW, TO>;
+  auto kernel = latent_attention_split_kernel<KS, DB, FULL, NW, TO>;
   if (allow_lds((const void*)kernel, NW * block, &allowed)) return -1;
   hipLaunchKernelGGL(kernel, dim3(num_tiles, a.splits), dim3(NW * kWave), NW * block, stream, a);
   if (a.splits > 1)
@@ -774,10 +899,10 @@ static int launch_latent_typed(const LatentMfmaArgs& a, int num_tiles, int waves
   return 0;
 }
 
-template <int KS, int DB>
+template <int KS, int DB, bool FULL>
 static int launch_latent_mfma(const LatentMfmaArgs& a, int num_tiles, int waves, int out_type,
                               hipStream_t stream) {
-  TS_DISPATCH_TYPE(out_type, TO, return (launch_latent_typed<KS, DB, TO>(a, num_tiles, waves, stream)));
+  TS_DISPATCH_TYPE(out_type, TO, return (launch_latent_typed<KS, DB, FULL, TO>(a, num_tiles, waves, stream)));
   return 0;
 }
 
@@ -813,11 +938,21 @@ extern "C" int ts_latent_attention_mfma(const float* qa, const void* pages, void
                    scale, q_ld, sink};
   const int dl = kv_rank + rot_dim;
   int rc;
-  if (dl <= 96 && kv_rank <= 64) rc = launch_latent_mfma<3, 4>(a, num_tiles, waves, out_type, stream);
-  else if (dl <= 160 && kv_rank <= 128) rc = launch_latent_mfma<5, 8>(a, num_tiles, waves, out_type, stream);
-  else if (dl <= 320 && kv_rank <= 256) rc = launch_latent_mfma<10, 16>(a, num_tiles, waves, out_type, stream);
-  else if (dl <= 576) rc = launch_latent_mfma<18, 32>(a, num_tiles, waves, out_type, stream);
-  else rc = launch_latent_mfma<20, 32>(a, num_tiles, waves, out_type, stream);
+  // rows of exactly an instance's size take its form without a branch a step
+  const bool even = ((uintptr_t)out & 15) == 0;
+#define TS_LATENT(KS, DB, FULL) \
+  rc = launch_latent_mfma<KS, DB, FULL>(a, num_tiles, waves, out_type, stream)
+  if (even && dl == 96 && kv_rank == 64) TS_LATENT(3, 4, true);
+  else if (even && dl == 160 && kv_rank == 128) TS_LATENT(5, 8, true);
+  else if (even && dl == 288 && kv_rank == 256) TS_LATENT(9, 16, true);
+  else if (even && dl == 320 && kv_rank == 256) TS_LATENT(10, 16, true);
+  else if (even && dl == 576 && kv_rank == 512) TS_LATENT(18, 32, true);
+  else if (dl <= 96 && kv_rank <= 64) TS_LATENT(3, 4, false);
+  else if (dl <= 160 && kv_rank <= 128) TS_LATENT(5, 8, false);
+  else if (dl <= 320 && kv_rank <= 256) TS_LATENT(10, 16, false);
+  else if (dl <= 576) TS_LATENT(18, 32, false);
+  else TS_LATENT(20, 32, false);
+#undef TS_LATENT
   if (rc) return rc;
   TS_CHECK_LAUNCH("latent_attention_mfma");
   return 0;
