@@ -149,22 +149,28 @@ __global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgs g
   };
 
   // TAIL with a small part of the tile per wave: the stream's values and the norm's
-  // weights are asked for now (before every direct load, so that the waits that count
-  // those see them gone first) and wait in registers for the epilogue
+  // weights are asked for behind the last direct loads, a ring's length of K steps before
+  // the epilogue that takes them out of registers (EARLY loads a lane, which the waits for
+  // the last steps count).  Asked for before the first direct loads they were 8 MB of 2,048
+  // rows of 1,024 that every tile waited for with its first step (23.1 us a product, 22.0 so).
   constexpr bool kEarlyStream = FORM == kTail && TM * TN <= 16;
+  constexpr int EARLY = kEarlyStream ? TN * TM + TN : 0;
+  static_assert(LOADS * (STAGES - 2) + EARLY < 64, "the load counter has six bits");
   f32x4 early_x[kEarlyStream ? TN : 1][kEarlyStream ? TM : 1], early_w[kEarlyStream ? TN : 1];
-  if constexpr (kEarlyStream) {
+  auto early_loads = [&]() {
+    if constexpr (kEarlyStream) {
 #pragma unroll
-    for (int tn = 0; tn < TN; ++tn) {
-      const int n = min(tile_n * BN + wn * WN + tn * 16 + gq * 4, g.N - 4);
-      early_w[tn] = *(const f32x4*)(g.norm_w + n);
+      for (int tn = 0; tn < TN; ++tn) {
+        const int n = min(tile_n * BN + wn * WN + tn * 16 + gq * 4, g.N - 4);
+        early_w[tn] = *(const f32x4*)(g.norm_w + n);
 #pragma unroll
-      for (int tm = 0; tm < TM; ++tm) {
-        const int m = min(m0 + wm * WM + tm * 16 + r, g.M - 1);
-        early_x[tn][tm] = *(const f32x4*)(g.resid + (int64_t)m * g.N + n);
+        for (int tm = 0; tm < TM; ++tm) {
+          const int m = min(m0 + wm * WM + tm * 16 + r, g.M - 1);
+          early_x[tn][tm] = *(const f32x4*)(g.resid + (int64_t)m * g.N + n);
+        }
       }
     }
-  }
+  };
 
   // column of W (row of the stacked weight) that LDS row `j` of the W slab holds
   auto w_row = [&](int j) {
@@ -312,27 +318,48 @@ __global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgs g
   asm volatile("" ::: "memory");
   Frags f0, f1;
   read(f0, 0, 0);
-  for (int kt0 = 0; kt0 < KT; kt0 += STAGES) {
+  // a turn's middle: step kt + 1 has arrived when at most IN_FLIGHT loads are on their way
+  auto next_step = [&](auto in_flight, int stage) {
+    wait_loads<decltype(in_flight)::value>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // this wave has read step kt
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read(f0, stage, 0);
+  };
+  for (int kt0 = 0; kt0 < KT - STAGES; kt0 += STAGES) {
 #pragma unroll
     for (int s = 0; s < STAGES; ++s) {
       const int kt = kt0 + s;
-      if (kt < KT) {
+      if (kt < KT - STAGES) {
         read(f1, s, 1);
         mma(f0, std::false_type{}, 0, 0);
-        const bool more = kt + 1 < KT;
-        if (more) {
-          // step kt + 1 has arrived when at most the younger steps' loads are in flight
-          wait_steps<LOADS, STAGES - 2>(min(STAGES - 2, KT - 2 - kt));
-          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");    // this wave has read step kt
-          __builtin_amdgcn_s_barrier();
-          asm volatile("" ::: "memory");
-          read(f0, (s + 1) % STAGES, 0);
-        }
-        if (kt + STAGES < KT) mma(f1, std::true_type{}, s, kt + STAGES);
-        else mma(f1, std::false_type{}, 0, 0);
+        next_step(std::integral_constant<int, LOADS * (STAGES - 2)>{}, (s + 1) % STAGES);
+        mma(f1, std::true_type{}, s, kt + STAGES);
       }
     }
   }
+  // the last STAGES turns, for which nothing is sent any more: written out, so that the turns
+  // before them have one wait and no branch (2,048 x 2,048 x 2,048 in 128 x 128 tiles 22.1 ->
+  // 19.6 us, 2,048 x 1,024 x 2,048 in 128 x 64 13.0 -> 12.6)
+  early_loads();
+  // (they have to lie in front of the waits that count them)
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  const int last = (KT - STAGES) % STAGES;
+  auto last_turn = [&](auto turn) {
+    constexpr int t = decltype(turn)::value;
+    const int stage = (last + t) % STAGES;
+    read(f1, stage, 1);
+    mma(f0, std::false_type{}, 0, 0);
+    if constexpr (t + 1 < STAGES)
+      next_step(std::integral_constant<int, LOADS * (STAGES - 2 - t) + EARLY>{}, (last + t + 1) % STAGES);
+    mma(f1, std::false_type{}, 0, 0);
+  };
+  last_turn(std::integral_constant<int, 0>{});
+  last_turn(std::integral_constant<int, 1>{});
+  if constexpr (STAGES > 2) last_turn(std::integral_constant<int, 2>{});
+  if constexpr (STAGES > 3) last_turn(std::integral_constant<int, 3>{});
+  static_assert(STAGES <= 4, "the last turns are written out");
   }
 
   // acc[tn][tm][e] = C[m0 + wm WM + 16 tm + r][column block tn, column 4 gq + e]
