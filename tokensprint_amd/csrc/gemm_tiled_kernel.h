@@ -79,18 +79,6 @@ __device__ __forceinline__ void wait_loads() {
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
 }
 
-// Waits until at most the loads of `younger` K steps (of LOADS each; at most MOST steps)
-// are in flight.
-template <int LOADS, int MOST>
-__device__ __forceinline__ void wait_steps(int younger) {
-  if constexpr (MOST <= 0) {
-    wait_loads<0>();
-  } else {
-    if (younger >= MOST) wait_loads<LOADS * MOST>();
-    else wait_steps<LOADS, MOST - 1>(younger);
-  }
-}
-
 template <int BM, int BN, int GM, int GN, int STAGES, bool PAIR, typename TO, int FORM = kPlain>
 __global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgs g) {
   static_assert(!(FORM == kTail && PAIR), "the product that ends a sub-layer has one weight");
@@ -269,43 +257,49 @@ __global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgs g
 #pragma unroll
       for (int i = 0; i < LOADS; ++i) issue_one(s, s, i);
     row_scales();
-    for (int kt0 = 0; kt0 < KT; kt0 += STAGES) {
+    // a turn; `in_flight`: the loads that may still be on their way when step kt has arrived.
+    // (The last one, which sends nothing, apart: no branch in the others.  The gate/up product
+    // of 2,048 rows at 2 x 3,072 x 1,024 in 256 x 192 tiles 31.6 -> 30.4 us.)
+    auto turn = [&](auto in_flight, auto with_loads, int s, int kt) {
+      constexpr bool load = decltype(with_loads)::value;
+      wait_loads<decltype(in_flight)::value>();
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      const unsigned char* slab = tiled_lds + s * STAGE_BYTES;
 #pragma unroll
-      for (int s = 0; s < STAGES; ++s) {
-        const int kt = kt0 + s;
-        if (kt >= KT) break;
-        wait_steps<LOADS, STAGES - 2>(min(STAGES - 2, KT - 1 - kt));
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        const bool load = kt + STAGES - 1 < KT;
-        const unsigned char* slab = tiled_lds + s * STAGE_BYTES;
+      for (int ks = 0; ks < 2; ++ks) {
+        const unsigned char* sa = slab + wm * WM * 128 + (ks ? read1 : read0);
+        const unsigned char* sw = slab + (BM + wn * WN) * 128 + (ks ? read1 : read0);
+        bf16x8 fw[TN], fa = *(const bf16x8*)sa, fb;
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-          const unsigned char* sa = slab + wm * WM * 128 + (ks ? read1 : read0);
-          const unsigned char* sw = slab + (BM + wn * WN) * 128 + (ks ? read1 : read0);
-          bf16x8 fw[TN], fa = *(const bf16x8*)sa, fb;
+        for (int tn = 0; tn < TN; ++tn) fw[tn] = *(const bf16x8*)(sw + tn * 2048);
 #pragma unroll
-          for (int tn = 0; tn < TN; ++tn) fw[tn] = *(const bf16x8*)(sw + tn * 2048);
+        for (int tm = 0; tm < TM; ++tm) {
+          if (tm + 1 < TM) fb = *(const bf16x8*)(sa + (tm + 1) * 2048);
 #pragma unroll
-          for (int tm = 0; tm < TM; ++tm) {
-            if (tm + 1 < TM) fb = *(const bf16x8*)(sa + (tm + 1) * 2048);
+          for (int tn = 0; tn < TN; ++tn)
+            acc[tn][tm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[tn], fa, acc[tn][tm], 0, 0, 0);
+          fa = fb;
+          constexpr int PER = (LOADS + 2 * TM - 1) / (2 * TM);      // loads per row block
+          if constexpr (load) {
 #pragma unroll
-            for (int tn = 0; tn < TN; ++tn)
-              acc[tn][tm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[tn], fa, acc[tn][tm], 0, 0, 0);
-            fa = fb;
-            constexpr int PER = (LOADS + 2 * TM - 1) / (2 * TM);      // loads per row block
-            if (load) {
-#pragma unroll
-              for (int j = 0; j < PER; ++j) {
-                const int i = (ks * TM + tm) * PER + j;
-                if (i < LOADS) issue_one((s + STAGES - 1) % STAGES, kt + STAGES - 1, i);
-              }
+            for (int j = 0; j < PER; ++j) {
+              const int i = (ks * TM + tm) * PER + j;
+              if (i < LOADS) issue_one((s + STAGES - 1) % STAGES, kt + STAGES - 1, i);
             }
           }
         }
       }
+    };
+    static_assert(STAGES == 2, "the turns are written out for a ring of two");
+    using none = std::integral_constant<int, 0>;
+    for (int kt = 0; kt + 2 < KT; kt += 2) {
+      turn(none{}, std::true_type{}, 0, kt);
+      turn(none{}, std::true_type{}, 1, kt + 1);
     }
+    if (KT % 2 == 0) turn(none{}, std::true_type{}, 0, KT - 2);
+    turn(none{}, std::false_type{}, (KT - 1) % 2, KT - 1);
   } else {
 #pragma unroll
   for (int s = 0; s < STAGES; ++s)
