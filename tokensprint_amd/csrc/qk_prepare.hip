@@ -107,6 +107,26 @@ __global__ void qk_prepare_kernel(QkPrepareArgs a) {
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_qk;
 typedef __attribute__((ext_vector_type(4))) float f32x4_qk;
 
+// Eight consecutive elements of a row as they are loaded, and as they are stored.
+template <typename T>
+struct Eight;
+template <>
+struct Eight<bf16_t> {
+  bf16x8_qk x;
+  __device__ __forceinline__ void load(const bf16_t* p) { x = *(const bf16x8_qk*)p; }
+  __device__ __forceinline__ void store(bf16_t* p) const { *(bf16x8_qk*)p = x; }
+  __device__ __forceinline__ float get(int j) const { return (float)x[j]; }
+  __device__ __forceinline__ void set(int j, float v) { x[j] = (bf16_t)v; }
+};
+template <>
+struct Eight<float> {
+  f32x4_qk lo, hi;
+  __device__ __forceinline__ void load(const float* p) { lo = *(const f32x4_qk*)p; hi = *(const f32x4_qk*)(p + 4); }
+  __device__ __forceinline__ void store(float* p) const { *(f32x4_qk*)p = lo; *(f32x4_qk*)(p + 4) = hi; }
+  __device__ __forceinline__ float get(int j) const { return j < 4 ? lo[j] : hi[j - 4]; }
+  __device__ __forceinline__ void set(int j, float v) { if (j < 4) lo[j] = v; else hi[j - 4] = v; }
+};
+
 // Values of many tokens into their pages (bfloat16 to bfloat16).  A page holds values
 // transposed, [head element][position], so a token's head vector lands two bytes at a
 // time, hd rows apart: here 16 lanes take 16 consecutive tokens for the same 8 head
@@ -114,6 +134,7 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_qk;
 // two-byte stores of one row fall into one 32-byte run of the page.  A workgroup of 256
 // takes (tile of 16 tokens, key/value head); its 16 lane groups take 8 head elements
 // each, in rounds.
+template <typename T>
 __device__ __forceinline__ void v_store_tile(const QkPrepareArgs& a, int tile, int kvh) {
   const int j = threadIdx.x % 16;
   const int t = tile * 16 + j;
@@ -122,14 +143,15 @@ __device__ __forceinline__ void v_store_tile(const QkPrepareArgs& a, int tile, i
   const int page = a.table[(int64_t)a.entry_of_token[t] * a.table_width + pos / a.page_size];
   if (page < 0) return;
   const int hd = a.hd;
-  const bf16_t* src = (const bf16_t*)a.qkv + (int64_t)t * ((a.nq + 2 * a.nkv) * hd + a.row_extra) +
-                      (int64_t)(a.nq + a.nkv + kvh) * hd;
-  bf16_t* dst = (bf16_t*)a.v_dst + ((int64_t)page * a.nkv + kvh) * a.page_size * hd +
-                pos % a.page_size;
+  const T* src = (const T*)a.qkv + (int64_t)t * ((a.nq + 2 * a.nkv) * hd + a.row_extra) +
+                 (int64_t)(a.nq + a.nkv + kvh) * hd;
+  T* dst = (T*)a.v_dst + ((int64_t)page * a.nkv + kvh) * a.page_size * hd +
+           pos % a.page_size;
   for (int d0 = (threadIdx.x / 16) * 8; d0 < hd; d0 += 128) {
-    const bf16x8_qk x = *(const bf16x8_qk*)(src + d0);
+    Eight<T> x;
+    x.load(src + d0);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) dst[(int64_t)(d0 + i) * a.page_size] = x[i];
+    for (int i = 0; i < 8; ++i) dst[(int64_t)(d0 + i) * a.page_size] = (T)x.get(i);
   }
 }
 
@@ -138,14 +160,14 @@ __device__ __forceinline__ void v_store_tile(const QkPrepareArgs& a, int tile, i
 // elements, the position, the norm weight, the entry), then what hangs on the position
 // (cos and sin, the page), then the arithmetic and the stores.  A piece so costs two
 // trips to memory, not one per use.
-template <typename TC, int N>
+template <typename T, typename TC, int N>
 __global__ __launch_bounds__(256) void qk_prepare_vec_kernel(QkPrepareArgs a, int lanes_log2,
                                                              int with_v, int v_first_block) {
   // with_v = 0 and v_first_block >= 0: the workgroups from that one on store the values
   // tile by tile (one launch for both: a second launch costs more than its work here)
   if (v_first_block >= 0 && (int)blockIdx.x >= v_first_block) {
     const int idx = blockIdx.x - v_first_block;
-    v_store_tile(a, idx / a.nkv, idx % a.nkv);
+    v_store_tile<T>(a, idx / a.nkv, idx % a.nkv);
     return;
   }
   const int L = 1 << lanes_log2;                     // lanes per head
@@ -160,7 +182,7 @@ __global__ __launch_bounds__(256) void qk_prepare_vec_kernel(QkPrepareArgs a, in
   struct Piece {
     bool live, norm, rotate, to_page;
     int t, h, kind, pos, entry, page;
-    bf16x8_qk x;
+    Eight<T> x;
     f32x4_qk w0, w1, c0, c1, s0, s1;
   };
   Piece pc[N];
@@ -172,8 +194,7 @@ __global__ __launch_bounds__(256) void qk_prepare_vec_kernel(QkPrepareArgs a, in
     const int64_t it = p.live ? item : 0;
     p.t = (int)(it / heads), p.h = (int)(it % heads);
     p.kind = p.h < a.nq ? 0 : (p.h < a.nq + a.nkv ? 1 : 2);
-    const bf16_t* src = (const bf16_t*)a.qkv + (int64_t)p.t * ((a.nq + 2 * a.nkv) * hd + a.row_extra) + (int64_t)p.h * hd;
-    p.x = *(const bf16x8_qk*)(src + sub * 8);
+    p.x.load((const T*)a.qkv + (int64_t)p.t * ((a.nq + 2 * a.nkv) * hd + a.row_extra) + (int64_t)p.h * hd + sub * 8);
     p.pos = a.positions[p.t];
     const float* w = p.kind == 0 ? a.q_weight : a.k_weight;
     p.norm = p.kind != 2 && w, p.rotate = p.kind != 2 && a.cos;
@@ -202,7 +223,7 @@ __global__ __launch_bounds__(256) void qk_prepare_vec_kernel(QkPrepareArgs a, in
     const Piece& p = pc[i];
     float v[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = (float)p.x[j];
+    for (int j = 0; j < 8; ++j) v[j] = p.x.get(j);
     if (p.norm) {
       float ss = 0.f;
 #pragma unroll
@@ -225,10 +246,10 @@ __global__ __launch_bounds__(256) void qk_prepare_vec_kernel(QkPrepareArgs a, in
     if (!p.live) continue;
     const int t = p.t, h = p.h;
     if (p.kind == 0) {
-      bf16x8_qk o;
+      Eight<T> o;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] = (bf16_t)v[j];
-      *(bf16x8_qk*)((bf16_t*)a.q_out + ((int64_t)t * a.nq + h) * hd + sub * 8) = o;
+      for (int j = 0; j < 8; ++j) o.set(j, v[j]);
+      o.store((T*)a.q_out + ((int64_t)t * a.nq + h) * hd + sub * 8);
       continue;
     }
     const int kvh = p.kind == 1 ? h - a.nq : h - a.nq - a.nkv;
@@ -243,15 +264,10 @@ __global__ __launch_bounds__(256) void qk_prepare_vec_kernel(QkPrepareArgs a, in
     const int slot = p.pos % a.page_size;
     if (p.kind == 1) {
       TC* dst = (TC*)a.k_dst + head_base + (int64_t)slot * hd + sub * 8;
-      if constexpr (sizeof(TC) == 2) {     // one 16-byte store (pages and rows are 16-byte aligned)
-        bf16x8_qk o;
+      Eight<TC> o;                         // 16-byte stores (pages and rows are 16-byte aligned)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) o[j] = (bf16_t)v[j];
-        *(bf16x8_qk*)dst = o;
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) dst[j] = from_f32<TC>(v[j]);
-      }
+      for (int j = 0; j < 8; ++j) o.set(j, v[j]);
+      o.store(dst);
     } else {
       TC* dst = (TC*)a.v_dst + head_base + slot;
 #pragma unroll
@@ -275,21 +291,25 @@ extern "C" int ts_qk_prepare(const QkPrepareArgs* args, int act_type, int cache_
   const int heads = a.nq + (a.store_kv ? 2 * a.nkv : 0);
   const int64_t items = (int64_t)a.num_tokens * heads;
   const int waves_per_block = 4;
-  if (act_type == TS_BF16 && a.hd >= 16 && a.hd <= 256 && (a.hd & (a.hd - 1)) == 0 &&
-      ((uintptr_t)a.qkv & 15) == 0 && ((uintptr_t)a.q_out & 15) == 0) {
+  // (float32 rows of 16 + 2 x 8 heads of 128: 501 of them 6.3 us, where a wavefront per head and an
+  // element at a time took 36.7 for 2,048; the step of 501 tokens 6.86 -> 6.65 ms)
+  if (a.hd >= 16 && a.hd <= 256 && (a.hd & (a.hd - 1)) == 0 && ((uintptr_t)a.qkv & 15) == 0 &&
+      ((uintptr_t)a.q_out & 15) == 0 && ((uintptr_t)a.k_dst & 15) == 0 &&
+      ((uintptr_t)a.q_weight & 15) == 0 && ((uintptr_t)a.k_weight & 15) == 0 &&
+      ((uintptr_t)a.cos & 15) == 0 && ((uintptr_t)a.sin & 15) == 0) {
     // portions of prompts: the values go tile by tile, by further workgroups of the same
     // launch
-    const bool v_tiles = a.store_kv && a.paged && cache_type == TS_BF16 && a.num_tokens >= 64;
+    const bool v_tiles = a.store_kv && a.paged && cache_type == act_type && a.num_tokens >= 64;
     const int lanes_log2 = __builtin_ctz(a.hd / 8);
     const int heads_per_block = waves_per_block * (kWave >> lanes_log2);
     const int64_t vec_items = v_tiles ? (int64_t)a.num_tokens * (a.nq + a.nkv) : items;
     const int64_t vblocks = (vec_items + heads_per_block - 1) / heads_per_block;
     const int64_t tiles = v_tiles ? (int64_t)((a.num_tokens + 15) / 16) * a.nkv : 0;
     if (vblocks + tiles > 2147483647LL) TS_FAIL("qk_prepare: too many tokens");
-    TS_DISPATCH_TYPE(cache_type, TC,
-        hipLaunchKernelGGL((qk_prepare_vec_kernel<TC, 1>), dim3((unsigned)(vblocks + tiles)),
+    TS_DISPATCH_TYPE(act_type, T, TS_DISPATCH_TYPE(cache_type, TC,
+        hipLaunchKernelGGL((qk_prepare_vec_kernel<T, TC, 1>), dim3((unsigned)(vblocks + tiles)),
                            dim3(waves_per_block * kWave), 0, stream, a, lanes_log2,
-                           v_tiles ? 0 : 1, v_tiles ? (int)vblocks : -1));
+                           v_tiles ? 0 : 1, v_tiles ? (int)vblocks : -1)));
     TS_CHECK_LAUNCH("qk_prepare");
     return 0;
   }
