@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from tokensprint_amd.cache import CacheManager, CacheStorage
-from tokensprint_amd.engine.batch import BatchBuilder, StepEntry
+from tokensprint_amd.engine.batch import BatchBuilder, StaticDecodeBatch, StepEntry
 from tokensprint_amd.kernels import load_hip_ops
 from tokensprint_amd.parts.base import PagedLatentNeed
 
@@ -67,3 +67,37 @@ def test_tiles_of_one_entry_walk_their_keys_together(gpu_device, monkeypatch, he
                 assert bool(((got[row] - want).abs() <= bound).all()), (spans, b, i)
                 row += 1
 
+
+
+@pytest.mark.parametrize("heads, kv_rank, rot_dim", [(16, 512, 64), (5, 128, 32), (16, 448, 64),
+                                                     (3, 512, 128)])
+def test_lanes_without_pages_read_none(gpu_device, monkeypatch, heads, kv_rank, rot_dim):
+    """A captured decode step's idle lanes: position 0, no pages.  Their rows see nothing but
+    zeros, and the lanes beside them what the form for few tiles gives."""
+    ops = load_hip_ops(gpu_device)
+    dl, page = kv_rank + rot_dim, 16
+    # (the second of two runs: a page in front of its first is the first run's last)
+    storage = CacheStorage([PagedLatentNeed(dl, None)] * 2, page, 12, 3, torch.bfloat16, gpu_device)
+    manager = CacheManager(storage.groups, page, 12, 3)
+    for i, view in enumerate(storage.views):
+        view.k_pages.copy_(rand(view.k_pages.shape, 4 + i).to(gpu_device).bfloat16())
+    view = storage.views[1]
+    entries = []
+    for i, n in enumerate((70, 1, 33)):
+        cache = manager.admit(i)
+        manager.extend(cache, n)
+        entries.append(StepEntry(cache, [1], n - 1, [0]))
+    static = StaticDecodeBatch(gpu_device, 6, [8], idle_slot=storage.idle_slot)
+    static.batch.max_ctx_len = 128
+    static.fill(entries)
+    rows = rand((6, heads * dl), 6, 1.5).to(gpu_device)
+    kept, outs = ops.dispatch, []
+    for full in (1, 1 << 30):
+        monkeypatch.setattr(ops, "dispatch", dataclasses.replace(kept, latent_full_tiles=full))
+        outs.append(ops.latent_attention(
+            rows, static.batch, static.batch.tables[0], view, heads=heads, kv_rank=kv_rank,
+            rot_dim=rot_dim, scale=2.0 / dl ** 0.5, window=None))
+    assert (outs[0][3:] == 0).all() and (outs[1][3:] == 0).all()
+    # a weight is rounded to bfloat16 once in either form, 2^-8 of it: the values are up to 5
+    assert ((outs[0] - outs[1]).abs() <= 2 * 2 ** -8 * 5).all()
+    assert (outs[0][:3] != 0).any(dim=(1, 2)).all()

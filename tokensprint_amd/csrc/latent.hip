@@ -547,17 +547,22 @@ __global__ __launch_bounds__(8 * kWave) void latent_attention_mfma_kernel(Latent
 
   const int key_l = threadIdx.x / PER_ROW, piece = threadIdx.x % PER_ROW;
   const int parts = dl / 8;
-  // (rows that no tile sees are stood in for by the nearest that one does)
+  // (rows that no tile sees are stood in for by the nearest that one does; rows of a page that
+  // the table does not have, as an idle lane's, are zeros, read from page 0's place)
   auto visible = [&](int kb) { return max(lo_t, min(kb + key_l, hi_t)); };
   auto look_up = [&](int kb) { return tab[visible(kb) / P]; };
   typedef bf16x8_l Pieces[PIECES];
   auto fetch = [&](Pieces& held, int kb, int page) {
-    const bf16_t* row = a.pages + ((int64_t)page * P + visible(kb) % P) * dl;
+    const bf16_t* row = a.pages + ((int64_t)max(page, 0) * P + visible(kb) % P) * dl;
 #pragma unroll
     for (int i = 0; i < PIECES; ++i)
       held[i] = *(const bf16x8_l*)(row + 8 * min(piece + PER_ROW * i, parts - 1));
   };
-  auto commit = [&](bf16_t* buf, const Pieces& held) {
+  auto commit = [&](bf16_t* buf, Pieces& held, int page) {
+    if (page < 0) {
+#pragma unroll
+      for (int i = 0; i < PIECES; ++i) held[i] = bf16x8_l{0, 0, 0, 0, 0, 0, 0, 0};
+    }
     bf16_t* row = buf + key_l * stride + 8 * piece;
 #pragma unroll
     for (int i = 0; i < PIECES; ++i)
@@ -566,8 +571,9 @@ __global__ __launch_bounds__(8 * kWave) void latent_attention_mfma_kernel(Latent
   int page = look_up(k_begin + BK);
   {
     Pieces held;
-    fetch(held, k_begin, look_up(k_begin));
-    commit(bufs, held);
+    const int page0 = look_up(k_begin);
+    fetch(held, k_begin, page0);
+    commit(bufs, held, page0);
   }
   bf16x8_l q[KS];
   load_query_row<KS>(q, a.qa + (int64_t)my_token * a.q_ld + my_head * dl, dl, g);
@@ -585,7 +591,8 @@ __global__ __launch_bounds__(8 * kWave) void latent_attention_mfma_kernel(Latent
     // the next block's rows, in flight while this one is scored (behind the last block the last
     // row again: under a condition the registers would be taken through the whole loop)
     Pieces held;
-    fetch(held, kb + BK, page);
+    const int held_page = page;
+    fetch(held, kb + BK, held_page);
     page = look_up(kb + 2 * BK);
     const bf16_t* k_s = bufs + which * BK * stride;
     bool sees[4];
@@ -612,7 +619,7 @@ __global__ __launch_bounds__(8 * kWave) void latent_attention_mfma_kernel(Latent
       for (int e = 0; e < 4 * BLK; ++e) at[e] = pv[e];
       if (half == 0 && g == 0) c_s[mine][r] = corr;
     }
-    commit(bufs + (which ^ 1) * BK * stride, held);
+    commit(bufs + (which ^ 1) * BK * stride, held, held_page);
     __syncthreads();                       // the weights and the next block's rows are there
     // everything the values' products take is asked for before the first of them
     const bf16_t* vrow = k_s + (4 * g + r / 4) * stride + 4 * (r % 4) + 16 * col0;
