@@ -101,3 +101,35 @@ def test_lanes_without_pages_read_none(gpu_device, monkeypatch, heads, kv_rank, 
     # a weight is rounded to bfloat16 once in either form, 2^-8 of it: the values are up to 5
     assert ((outs[0] - outs[1]).abs() <= 2 * 2 ** -8 * 5).all()
     assert (outs[0][:3] != 0).any(dim=(1, 2)).all()
+
+
+@pytest.mark.parametrize("window", [None, 37, 64, 100])
+@pytest.mark.parametrize("heads, kv_rank, rot_dim", [(16, 512, 64), (2, 128, 32), (5, 200, 16),
+                                                     (16, 512, 128)])
+def test_rows_do_not_depend_on_how_a_prompt_is_cut(gpu_device, monkeypatch, heads, kv_rank, rot_dim,
+                                                   window):
+    """Which tokens share a workgroup decides nothing: blocks of keys lie at fixed positions."""
+    ops = load_hip_ops(gpu_device)
+    monkeypatch.setattr(ops, "dispatch", dataclasses.replace(ops.dispatch, latent_full_tiles=1))
+    dl, page, T = kv_rank + rot_dim, 16, 300
+    rows = rand((T, heads * dl), 7, 1.5).to(gpu_device)
+
+    def whole(portions):
+        storage = CacheStorage([PagedLatentNeed(dl, None)], page, 20, 1, torch.bfloat16, gpu_device)
+        manager = CacheManager(storage.groups, page, 20, 1)
+        builder, view = BatchBuilder(gpu_device, len(storage.groups)), storage.views[0]
+        view.k_pages.copy_(rand(view.k_pages.shape, 8).to(gpu_device).bfloat16())
+        cache, at, outs = manager.admit(0), 0, []
+        for n in portions:
+            manager.extend(cache, at + n)
+            batch = builder.build([StepEntry(cache, [1] * n, at, [n - 1])])
+            outs.append(ops.latent_attention(
+                rows[at:at + n].contiguous(), batch, batch.tables[0], view, heads=heads,
+                kv_rank=kv_rank, rot_dim=rot_dim, scale=2.0 / dl ** 0.5, window=window))
+            at += n
+        assert at == T
+        return torch.cat(outs)
+
+    want = whole([T])
+    for portions in ([33, 67, 200], [1, 2, 3, 93, 1, 95, 105], [131, 169]):
+        assert torch.equal(whole(portions), want), portions

@@ -336,8 +336,9 @@ extern "C" int ts_latent_attention(const float* qa, const void* pages, int cache
 // S^T[key 4g + t][row r], which is, in place, its part of the second product's B operand;
 // its softmax statistics are shared with lanes r + 16, r + 32, r + 48; its part of O^T is
 // [columns 16 db + 4g + t][row r], so rescaling needs nothing from other lanes.
-// Keys are walked in blocks of 32 at absolute multiples of 32, staged in LDS, from where both
-// operands come: the K operand as 16 bytes of a row, the C^T operand by the transposing read.
+// Keys are walked in blocks at absolute multiples of the block's size (32; 64 in the form for
+// many tiles where two blocks of that size fit), staged in LDS, from where both operands come:
+// the K operand as 16 bytes of a row, the C^T operand by the transposing read.
 // Where a step has few tiles, a tile's keys are shared out in runs of `keys_per_split` over
 // several workgroups, whose unnormalised results and statistics (the largest score in units
 // of log2) a second kernel merges.
@@ -542,8 +543,10 @@ __global__ __launch_bounds__(8 * kWave) void latent_attention_mfma_kernel(Latent
     last[t] = __builtin_amdgcn_readfirstlane(p1);
     hi_t = max(hi_t, last[t]);
   }
+  // (blocks begin at absolute multiples of BK: a row's running maximum, the rounding of its
+  // weights and the order of its sums do not depend on which tokens share the workgroup)
   const int lo_t = first[0];
-  const int k_begin = (lo_t / 32) * 32, k_end = hi_t + 1;
+  const int k_begin = lo_t / BK * BK, k_end = hi_t + 1;
 
   const int key_l = threadIdx.x / PER_ROW, piece = threadIdx.x % PER_ROW;
   const int parts = dl / 8;
