@@ -97,3 +97,24 @@ def test_attention_of_a_token_does_not_depend_on_its_step(gpu_device):
             one.ctx_len = torch.tensor([t + 1], dtype=torch.int32, device=gpu_device)
             alone = ops.paged_attention(q[t:t + 1].contiguous(), one, table[:1].contiguous(), cache, **kw)
             assert torch.equal(alone[0], whole[t]), t
+
+
+@pytest.mark.parametrize("which", ["q", "k_pages", "v_pages"])
+def test_attention_takes_buffers_that_do_not_begin_on_16_bytes(gpu_device, which):
+    ops = load_hip_ops(gpu_device)
+    kw = dict(num_heads=6, num_kv_heads=2, head_dim=32, scale=32 ** -0.5, window=None)
+    batch, cache, table, _ = paged_scenario(gpu_device, torch.float32, nkv=2, hd=32, page_size=16,
+                                            spans=[(0, 70), (33, 1), (5, 20)], seed=11)
+    q = rand((batch.num_tokens, 6, 32), 12).to(gpu_device)
+    want = ops.paged_attention(q, batch, table, cache, **kw)
+
+    def moved(x):
+        flat = torch.empty(x.numel() + 1, dtype=x.dtype, device=x.device)[1:]
+        return flat.view(x.shape).copy_(x)
+
+    if which == "q":
+        q = moved(q)
+    else:
+        setattr(cache, which, moved(getattr(cache, which)))
+    out = ops.paged_attention(q, batch, table, cache, **kw)
+    torch.testing.assert_close(out, want, rtol=2e-5, atol=2e-6)

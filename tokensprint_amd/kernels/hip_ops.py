@@ -770,6 +770,8 @@ class HipOps:
             else:
                 self._attention_mfma(a, batch, num_heads // num_kv_heads, extras)
         elif (q.dtype == torch.float32 and cache.k_pages.dtype == torch.float32
+                # (its loads are of 16 bytes; buffers that begin elsewhere take the general kernel)
+                and (q.data_ptr() | cache.k_pages.data_ptr() | cache.v_pages.data_ptr()) % 16 == 0
                 and self.lib.ts_attention_f32_fits(head_dim, num_heads // num_kv_heads,
                                                    cache.page_size, num_kv_heads, a.keep) == 1):
             # the same kernel for portions and single tokens: what a row adds up depends on its
