@@ -181,3 +181,29 @@ def test_state_space_scan_in_chunks(gpu_device, heads, groups, rows, vdim):
         no_further_off(got, walked, want.view(T, inner))
         slots = batch.slot_ids.long()
         no_further_off(st[slots], st_walked[slots], torch.stack(want_state))
+
+
+@pytest.mark.parametrize("per_channel", [False, True])
+def test_delta_rule_takes_silu_of_its_operands_in_long_portions(gpu_device, per_channel):
+    ops, gen = load_hip_ops(gpu_device), torch.Generator().manual_seed(9)
+    heads, dim, vdim = 2, 36, 20
+    requests, spans = Requests(gpu_device, (heads, dim, vdim), 2), [150, 70]
+    batch = requests.step(spans)
+    T, n = batch.num_tokens, heads * dim if per_channel else heads
+    x = torch.randn(T, heads * (2 * dim + vdim), generator=gen)
+    x[:, :2 * heads * dim] *= 0.2
+    gates = torch.cat([torch.rand(T, heads, generator=gen), torch.rand(T, n, generator=gen) ** 0.1], 1)
+    out = ops.linear_recurrence(
+        x.to(gpu_device), 0, heads * dim, 2 * heads * dim, batch, requests.state, heads=heads,
+        kv_heads=heads, dim=dim, vdim=vdim, silu_inputs=True, delta=True, per_channel=per_channel,
+        gates=gates.to(gpu_device))
+    q, k, v = torch.nn.functional.silu(x.double()).split([heads * dim] * 2 + [heads * vdim], 1)
+    q, k, v = q.view(T, heads, dim), k.view(T, heads, dim), v.view(T, heads, vdim)
+    g, beta = gates[:, heads:].double().view(T, heads, -1), gates[:, :heads].double()
+    want, at = [], 0
+    for rows in spans:
+        r = slice(at, at + rows)
+        want.append(walk(q[r], k[r], v[r], g[r], beta[r],
+                         torch.zeros(heads, dim, vdim, dtype=torch.float64))[0])
+        at += rows
+    torch.testing.assert_close(out.double().cpu(), torch.cat(want).view(T, -1), rtol=1e-5, atol=1e-5)

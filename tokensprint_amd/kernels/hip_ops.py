@@ -1393,9 +1393,10 @@ class HipOps:
             self._check("gates", gates, torch.float32, shape=(T, ldg))
         pos, eot, qs, slots = self._batch_ptrs(batch, T)
         out = torch.empty(T, heads * vdim, dtype=torch.float32, device=self.device)
-        # a long portion runs in chunks, as products of matrices
+        # a long portion runs in chunks, as products of matrices (the delta rule with operands as
+        # they stand: with their SiLU taken on the way it is walked)
         chunks, entry_chunks, num_chunks = None, None, 0
-        if dim <= (128 if delta else 256):
+        if dim <= (128 if delta else 256) and not (delta and silu_inputs):
             chunks, entry_chunks, num_chunks = self._scan_chunks(batch)
         scratch = self._chunk_scratch(num_chunks, heads, dim, vdim, delta, per_channel)
         self._call(self.lib.ts_linear_recurrence, _ptr(x), ld, int(q_col), int(k_col), int(v_col),
