@@ -9,6 +9,7 @@ import torch
 from tokensprint_amd.cache import CacheManager, CacheStorage
 from tokensprint_amd.engine.batch import BatchBuilder, StepEntry
 from tokensprint_amd.kernels import load_hip_ops
+from tokensprint_amd.kernels.hip_ops import KernelError
 from tokensprint_amd.parts.base import SlotStateNeed
 
 pytestmark = pytest.mark.gpu
@@ -207,3 +208,16 @@ def test_delta_rule_takes_silu_of_its_operands_in_long_portions(gpu_device, per_
                          torch.zeros(heads, dim, vdim, dtype=torch.float64))[0])
         at += rows
     torch.testing.assert_close(out.double().cpu(), torch.cat(want).view(T, -1), rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("tokens", [3, 200])
+def test_states_of_more_rows_are_refused_with_a_message(gpu_device, tokens):
+    ops = load_hip_ops(gpu_device)
+    heads, rows, vdim = 2, 260, 4
+    requests = Requests(gpu_device, (heads, rows, vdim), 1)
+    batch = requests.step([tokens])
+    xbc = torch.zeros(tokens, heads * vdim + 2 * rows, device=gpu_device)
+    proj, consts = torch.zeros(tokens, heads, device=gpu_device), torch.zeros(heads, device=gpu_device)
+    with pytest.raises(KernelError, match="260"):
+        ops.ssm_scan(xbc, proj, 0, consts, consts, consts, batch, requests.state, heads=heads,
+                     vdim=vdim, state_rows=rows, groups=1)

@@ -1304,6 +1304,8 @@ class HipOps:
         if not num_chunks:
             return None
         count = self.lib.ts_chunked_scratch(num_chunks, heads, rows, cols, int(delta), int(per_row))
+        if count < 0:
+            raise KernelError(f"recurrence in chunks: {rows} x {cols} states are not built")
         return torch.empty(count, dtype=torch.float32, device=self.device)
 
     def _scan_chunks(self, batch, whole=None):
