@@ -118,3 +118,33 @@ def test_attention_takes_buffers_that_do_not_begin_on_16_bytes(gpu_device, which
         setattr(cache, which, moved(getattr(cache, which)))
     out = ops.paged_attention(q, batch, table, cache, **kw)
     torch.testing.assert_close(out, want, rtol=2e-5, atol=2e-6)
+
+
+@pytest.mark.parametrize("nq, nkv, hd, page", [(16, 8, 128, 16), (5, 1, 48, 32), (2, 2, 16, 16)])
+@pytest.mark.parametrize("form", ["plain", "window", "chunk_sink"])
+def test_values_that_are_not_finite_stay_with_the_rows_that_see_them(gpu_device, monkeypatch, nq, nkv,
+                                                                    hd, page, form):
+    ops = load_hip_ops(gpu_device)
+    spans = [(0, 130), (40, 37), (0, 9), (70, 1)]
+    batch, cache, table, _ = paged_scenario(gpu_device, torch.float32, nkv=nkv, hd=hd, page_size=page,
+                                            spans=spans, seed=13)
+    q = rand((batch.num_tokens, nq, hd), 14).to(gpu_device)
+    kw = dict(num_heads=nq, num_kv_heads=nkv, head_dim=hd, scale=hd ** -0.5, window=None)
+    if form == "window":
+        kw["window"] = 21
+    elif form == "chunk_sink":
+        kw.update(chunk=50, sink=rand((nq,), 15).to(gpu_device))
+    finite = ops.paged_attention(q, batch, table, cache, **kw)
+    spoilt = {0: [(45, float("inf")), (77, float("nan")), (101, float("-inf"))],
+              1: [(60, float("nan"))], 2: [(5, float("inf"))], 3: [(3, float("inf"))]}
+    for e, places in spoilt.items():
+        for key, value in places:
+            cache.v_pages[table[e, key // page].item(), -1, key % hd, key % page] = value
+    cache.k_pages[table[0, 118 // page].item(), -1, 118 % page, 0] = float("nan")
+    out = ops.paged_attention(q, batch, table, cache, **kw)
+    monkeypatch.setattr(ops.lib, "ts_attention_f32_fits", lambda *a: 0)
+    want = ops.paged_attention(q, batch, table, cache, **kw)
+    torch.testing.assert_close(out, want, rtol=2e-5, atol=2e-6, equal_nan=True)
+    kept = out.isfinite()
+    assert torch.equal(out[kept], finite[kept])
+    assert kept[:45].all() and not kept.all()

@@ -18,6 +18,7 @@
 // each of its blocks.  The kernel before it, a workgroup per token and head with a key a lane,
 // read every key row 32 times as 16-byte pieces 512 bytes apart.
 #include "attention_mfma.h"
+#include <type_traits>
 
 int ts_check_attention_args(const AttentionArgs& a, const char* who);
 
@@ -59,88 +60,119 @@ __global__ __launch_bounds__(kWaves* kWave) void attention_f32_kernel(AttentionM
   if (EXTRAS) x = score_extra(a, head, pos);
   f32x4 qf[NT], o[NT];
 #pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    qf[j] = read4(q + 16 * j);
-    o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  float top = -INFINITY, sum = 0.f;        // of column l; `sum` of this lane's keys only
-  int b = begin / kBlock;
-  b += (w - b) & (kWaves - 1);             // the first block of this wavefront's
-  for (; b * kBlock <= last; b += kWaves) {
-    // (every load is made, from page 0 where there is none: what it brings is not used)
-    int64_t row[4];                        // of the block's four tiles of 16 keys: their page
-    bool have[4];
+  for (int j = 0; j < NT; ++j) qf[j] = read4(q + 16 * j);
+  float top, sum;                          // of column l; `sum` of this lane's keys only
+  // The wavefront's blocks.  A key that a row does not see has no weight with it, but nothing times
+  // a value that is not finite is not nothing: APART makes the product with the values once a
+  // row, without the keys that the row does not see, and takes the row's column of it.
+  auto walk = [&](auto apart) {
+    constexpr bool APART = decltype(apart)::value;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int key = b * kBlock + 16 * t;
-      const int page = __builtin_amdgcn_readfirstlane(table[min(key, last) / P]);
-      have[t] = key <= last && page >= 0;
-      row[t] = ((int64_t)max(page, 0) * a.nkv + kvh) * P * HD;
-    }
-    f32x4 kf[4][NT], vf[4][NT], s[4];
+    for (int j = 0; j < NT; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    top = -INFINITY, sum = 0.f;
+    int b = begin / kBlock;
+    b += (w - b) & (kWaves - 1);             // the first block of this wavefront's
+    for (; b * kBlock <= last; b += kWaves) {
+      // (every load is made, from page 0 where there is none: what it brings is not used)
+      int64_t row[4];                        // of the block's four tiles of 16 keys: their page
+      bool have[4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const float* k = (const float*)a.k_pages + row[t] + (int64_t)((b * kBlock + 16 * t) % P + l) * HD + 4 * g;
-#pragma unroll
-      for (int j = 0; j < NT; ++j) kf[t][j] = read4(k + 16 * j);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int j = 0; j < NT; ++j) s[t] = mfma4(kf[t][j], qf[j], s[t]);
-    }
-    __builtin_amdgcn_sched_barrier(0);     // (the values in the keys' registers)
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const float* v = (const float*)a.v_pages + row[t] + (int64_t)l * P + (b * kBlock + 16 * t) % P + 4 * g;
-#pragma unroll
-      for (int c = 0; c < NT; ++c) vf[t][c] = read4(v + (int64_t)16 * c * P);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    float high = top;
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int key = b * kBlock + 16 * t + 4 * g + r;
-        const float v = EXTRAS ? extra_score(x, s[t][r], key) : s[t][r] * a.scale;
-        s[t][r] = have[t] && mine && key <= pos && key >= from ? v : -INFINITY;
-        high = fmaxf(high, s[t][r]);
+      for (int t = 0; t < 4; ++t) {
+        const int key = b * kBlock + 16 * t;
+        const int page = __builtin_amdgcn_readfirstlane(table[min(key, last) / P]);
+        have[t] = key <= last && page >= 0;
+        row[t] = ((int64_t)max(page, 0) * a.nkv + kvh) * P * HD;
       }
-    high = fmaxf(high, __shfl_xor(high, 16, kWave));
-    high = fmaxf(high, __shfl_xor(high, 32, kWave));
-    // (`high` stays -inf only while the row has seen no key: zeros are kept)
-    const float fall = high == -INFINITY ? 1.f : expf(top - high);
-    top = high;
-    sum *= fall;
+      f32x4 kf[4][NT], vf[4][NT], s[4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < 4; ++t) {
+        const float* k = (const float*)a.k_pages + row[t] + (int64_t)((b * kBlock + 16 * t) % P + l) * HD + 4 * g;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        s[t][r] = s[t][r] == -INFINITY ? 0.f : expf(s[t][r] - high);
-        sum += s[t][r];
+        for (int j = 0; j < NT; ++j) kf[t][j] = read4(k + 16 * j);
       }
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int c = 0; c < NT; ++c) o[c] *= fall;
+      for (int t = 0; t < 4; ++t) {
+        s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int key = b * kBlock + 16 * t;
-      if (!have[t] || key + 15 > last) {   // a page's places behind the last key hold anything
+        for (int j = 0; j < NT; ++j) s[t] = mfma4(kf[t][j], qf[j], s[t]);
+      }
+      __builtin_amdgcn_sched_barrier(0);     // (the values in the keys' registers)
 #pragma unroll
-        for (int c = 0; c < NT; ++c)
+      for (int t = 0; t < 4; ++t) {
+        const float* v = (const float*)a.v_pages + row[t] + (int64_t)l * P + (b * kBlock + 16 * t) % P + 4 * g;
+#pragma unroll
+        for (int c = 0; c < NT; ++c) vf[t][c] = read4(v + (int64_t)16 * c * P);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      float high = top;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int key = b * kBlock + 16 * t + 4 * g + r;
+          const float v = EXTRAS ? extra_score(x, s[t][r], key) : s[t][r] * a.scale;
+          s[t][r] = have[t] && mine && key <= pos && key >= from ? v : -INFINITY;
+          high = fmaxf(high, s[t][r]);
+        }
+      high = fmaxf(high, __shfl_xor(high, 16, kWave));
+      high = fmaxf(high, __shfl_xor(high, 32, kWave));
+      // (`high` stays -inf only while the row has seen no key: zeros are kept)
+      const float fall = high == -INFINITY ? 1.f : expf(top - high);
+      top = high;
+      sum *= fall;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          s[t][r] = s[t][r] == -INFINITY ? 0.f : expf(s[t][r] - high);
+          sum += s[t][r];
+        }
+#pragma unroll
+      for (int c = 0; c < NT; ++c) o[c] *= fall;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int key = b * kBlock + 16 * t;
+        if (!have[t] || key + 15 > last) {   // a page's places behind the last key hold anything
+#pragma unroll
+          for (int c = 0; c < NT; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (!have[t] || key + 4 * g + r > last) vf[t][c][r] = 0.f;
+        }
+        if constexpr (APART) {
+#pragma unroll 1
+          for (int row = 0; row < tokens * group; ++row) {
+            const int to = __shfl(pos, row, kWave), lo = __shfl(from, row, kWave);
+#pragma unroll
+            for (int c = 0; c < NT; ++c) {
+              f32x4 sums = o[c];
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                const bool sees = key + 4 * g + r <= to && key + 4 * g + r >= lo;
+                sums = __builtin_amdgcn_mfma_f32_16x16x4f32(sees ? vf[t][c][r] : 0.f, s[t][r], sums, 0, 0, 0);
+              }
+              if (l == row) o[c] = sums;
+            }
+          }
+        } else {
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            if (!have[t] || key + 4 * g + r > last) vf[t][c][r] = 0.f;
+#pragma unroll
+            for (int c = 0; c < NT; ++c)
+              o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][c][r], s[t][r], o[c], 0, 0, 0);
+        }
       }
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int c = 0; c < NT; ++c)
-          o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][c][r], s[t][r], o[c], 0, 0, 0);
     }
-  }
+  };
+  walk(std::false_type{});
+  // (a value of that kind leaves NaN in every row that meets it, whatever comes behind)
+  bool nan = false;
+#pragma unroll
+  for (int c = 0; c < NT; ++c)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) nan = nan || o[c][r] != o[c][r];
+  if (__builtin_amdgcn_ballot_w64(nan && mine) != 0) walk(std::true_type{});
   sum += __shfl_xor(sum, 16, kWave);
   sum += __shfl_xor(sum, 32, kWave);
   if (g == 0) {
@@ -163,6 +195,7 @@ __global__ __launch_bounds__(kWaves* kWave) void attention_f32_kernel(AttentionM
       const float mu = m_s[u * 16 + r];
       if (mu == -INFINITY) continue;       // a wavefront without keys
       const float weight = expf(mu - all);
+      if (weight == 0.f) continue;         // (its sums may be infinite)
       den += l_s[u * 16 + r] * weight;
       num += read4(o_s + (u * 16 + r) * LD + d) * weight;
     }
