@@ -221,3 +221,62 @@ def test_states_of_more_rows_are_refused_with_a_message(gpu_device, tokens):
     with pytest.raises(KernelError, match="260"):
         ops.ssm_scan(xbc, proj, 0, consts, consts, consts, batch, requests.state, heads=heads,
                      vdim=vdim, state_rows=rows, groups=1)
+
+
+@pytest.mark.parametrize("what", ["q", "k", "v", "gates"])
+@pytest.mark.parametrize("mode", ["fixed", "turned", "per_head", "delta", "delta_per_channel", "scan"])
+def test_what_is_not_finite_does_not_reach_earlier_tokens(gpu_device, mode, what):
+    """Infinities and NaN in a token's operands: the tokens before it and the other requests come
+    out the same to the bit, a q reaches its own token alone."""
+    ops, gen = load_hip_ops(gpu_device), torch.Generator().manual_seed(10)
+    ops_dispatch = dataclasses.replace(ops.dispatch, scan_whole_tokens=16, state_space_whole_tokens=16)
+    heads, kv_heads, dim, vdim, spans = 4, 2, 64, 33, [150, 70]
+    n_gates = heads * dim if mode == "delta_per_channel" else heads
+    x = torch.randn(sum(spans), 2 * kv_heads * dim + heads * vdim, generator=gen)
+    x[:, :2 * kv_heads * dim] *= 0.15
+    gates = torch.cat([torch.rand(sum(spans), heads, generator=gen),
+                       torch.rand(sum(spans), n_gates, generator=gen) ** 0.1], 1)
+    q_col, k_col, v_col = 0, kv_heads * dim, 2 * kv_heads * dim
+    if mode == "scan":                                     # x | B | C, and the step sizes
+        v_col, k_col, q_col = 0, heads * vdim, heads * vdim + kv_heads * dim
+    column = {"q": q_col, "k": k_col, "v": v_col}
+    consts = [torch.randn(heads, generator=gen).to(gpu_device) for _ in range(3)]
+    angles = torch.outer(torch.arange(200.0), 0.3 ** torch.arange(dim // 2))
+    table = torch.stack([angles.cos(), angles.sin()], -1).contiguous().to(gpu_device)
+
+    def run(x, gates):
+        requests = Requests(gpu_device, (heads, dim, vdim), 2)
+        batch, kept = requests.step(spans), ops.dispatch
+        x, gates = x.to(gpu_device), gates.to(gpu_device)
+        ops.dispatch = ops_dispatch
+        try:
+            if mode == "scan":
+                return ops.ssm_scan(x, gates, heads, *consts, batch, requests.state, heads=heads,
+                                    vdim=vdim, state_rows=dim, groups=kv_heads)
+            kw = dict(gates=gates, per_channel=n_gates > heads, delta=mode.startswith("delta"))
+            if mode in ("fixed", "turned"):
+                kw = dict(decay=0.9 + 0.02 * consts[0].tanh(), silu_inputs=mode == "fixed")
+            if mode == "turned":
+                kw.update(turn=table, k_scale=0.5)
+            return ops.linear_recurrence(x, q_col, k_col, v_col, batch, requests.state, heads=heads,
+                                         kv_heads=kv_heads, dim=dim, vdim=vdim,
+                                         **{"silu_inputs": False, **kw})
+        finally:
+            ops.dispatch = kept
+
+    want = run(x, gates)
+    for t in (0, 5, 37, 63, 64, 79, 140):
+        for value in (float("inf"), float("nan")):
+            xs, gs = x.clone(), gates.clone()
+            if what == "gates":
+                if mode in ("fixed", "turned"):
+                    return
+                gs[t, heads:] = value
+            else:
+                xs[t, column[what]] = value
+            out = run(xs, gs)
+            assert torch.equal(out[:t], want[:t]), (t, value)
+            assert torch.equal(out[150:], want[150:]), (t, value)
+            assert not out[t].isfinite().all() or (mode == "scan" and what == "gates"), (t, value)
+            if what == "q":
+                assert torch.equal(out[t + 1:], want[t + 1:]), (t, value)

@@ -253,6 +253,26 @@ __device__ __forceinline__ void read_run(const float* p, float (&v)[PER]) {
   }
 }
 
+// acc + T u for a diagonal tile T in LDS, zero above its diagonal: row t takes u of its own and of
+// earlier tokens.  Zero times what is not finite is not zero, so where such u are among the
+// sixteen a row at a time is made, with the later ones left out, and taken.
+__device__ __forceinline__ f32x4 causal_product(const float* tile, f32x4 u, f32x4 acc, int l, int g) {
+  const f32x4 a = read4(tile + l * kTileLd + 4 * g);
+  if (__builtin_amdgcn_ballot_w64(!(fabsf(u[0]) + fabsf(u[1]) + fabsf(u[2]) + fabsf(u[3]) < INFINITY)) == 0)
+    return mfma4(a, u, acc);
+  f32x4 out = acc;
+#pragma unroll 1
+  for (int t = 0; t < 16; ++t) {
+    f32x4 seen;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) seen[r] = 4 * g + r <= t ? u[r] : 0.f;
+    const f32x4 sums = mfma4(a, seen, acc);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) out[r] = 4 * g + r == t ? sums[r] : out[r];
+  }
+  return out;
+}
+
 // Decays per row: the diagonal tiles (wavefront w takes block w), the products' decays
 // multiplied up pair by pair.  left: q or k rows.  STRICT leaves the diagonal out.  Sixteen lanes
 // share a column s (a run of channels each), four columns at a time.
@@ -581,7 +601,7 @@ __device__ __forceinline__ void solve_chunk(const ChunkedArgs& a, const ChunkRan
       for (int m = 0; m < i; ++m)
         acc = mfma4(read4(tiles + tri(i, m) * kTile + l * kTileLd + 4 * g), X[m], acc);
       const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-      X[i] = mfma4(read4(tiles + tri(i, i) * kTile + l * kTileLd + 4 * g), acc, zero);
+      X[i] = causal_product(tiles + tri(i, i) * kTile, acc, zero, l, g);
       if (ct < NT) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
@@ -887,7 +907,8 @@ __device__ __forceinline__ void output_chunk(const ChunkedArgs& a, const ChunkRa
 #pragma unroll
         for (int j = 0; j <= i; ++j) {
           const f32x4 u = DELTA ? v[j] : v[j] * read4(d.vs() + 16 * j + 4 * g);
-          acc[i] = mfma4(read4(tiles + tri(i, j) * kTile + l * kTileLd + 4 * g), u, acc[i]);
+          if (i == j) acc[i] = causal_product(tiles + tri(i, i) * kTile, u, acc[i], l, g);
+          else acc[i] = mfma4(read4(tiles + tri(i, j) * kTile + l * kTileLd + 4 * g), u, acc[i]);
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
