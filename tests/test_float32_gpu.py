@@ -148,3 +148,17 @@ def test_values_that_are_not_finite_stay_with_the_rows_that_see_them(gpu_device,
     kept = out.isfinite()
     assert torch.equal(out[kept], finite[kept])
     assert kept[:45].all() and not kept.all()
+
+
+@pytest.mark.parametrize("M", [1, 40, 501])
+@pytest.mark.parametrize("N, K", [(1024, 1024), (512, 2048), (512, 3072)])
+def test_product_rounds_no_more_than_short_chains_do(gpu_device, N, K, M):
+    """Additions of random signs: a rounding is 2^-24 of what it rounds at most, in the mean square
+    less than 0.45 of that, and K / 8 chains of eight products, a run's K / 128 steps and four
+    pairs of runs give (8 / 2 + 1 + K / 256 + 3.5) such squares of the result's."""
+    ops = load_hip_ops(gpu_device)
+    x, w = rand((M, K), 16), rand((N, K), 17)
+    want = x.double() @ w.double().T
+    got = ops.linear(x.to(gpu_device), w.to(gpu_device), torch.float32).double().cpu()
+    bound = 0.45 * 2.0 ** -24 * (8.5 + K / 256) ** 0.5 * 1.1
+    assert (got - want).norm() <= bound * want.norm()

@@ -4,11 +4,13 @@
 //
 // Every output element adds its K products in an order fixed by K alone, so its value does not
 // depend on which other rows are in the call nor on the kernel that the number of rows chooses.
-// Where K is a multiple of 4: K is cut into stretches of 64, the stretches into eight runs of
-// equal length; a stretch is one chain of float32 matrix-core products (v_mfma_f32_16x16x4_f32;
-// the four products of a step of 16 take elements 4 g + r, g = 0..3, in product r), a run adds its
-// stretches' sums in order and the result the eight runs' sums in order.  Another K adds in index
-// order in one accumulator.
+// Where K is a multiple of 4: K is cut into steps of 16, four of them a stretch, the stretches into
+// eight runs of equal length.  A step is four float32 matrix-core products
+// (v_mfma_f32_16x16x4_f32; elements 4 g + r, g = 0..3, in product r) in two chains from zero, the
+// even and the odd r; a run adds the steps' sums in order, the result the sums of pairs of runs in
+// order.  Chains of eight products and not of a stretch's 64, because their roundings are what an
+// element's error mostly is: 9.6e-8 of the result at K = 1,024 against 1.58e-7, 1.1e-7 against
+// 1.6e-7 at 2,048, for 4 to 10 % of the tiles' time.  Another K adds in index order in one accumulator.
 #include "common.h"
 
 constexpr int kTile = 64;   // output tile edge per workgroup
@@ -90,13 +92,12 @@ __global__ __launch_bounds__(kRuns* kWave) void gemm_f32_rows_kernel(
   const int run = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
   const int l = lane % 16, g = lane / 16;
   const int64_t n0 = (int64_t)blockIdx.x * 16;
-  const int m0 = blockIdx.y * 16 * MT;
   const int steps = (K + 15) / 16, per = stretches_of_run(K) * kStretch;
   const int begin = run * per, end = min(begin + per, steps);
   const TW* w_row = W + min(n0 + l, (int64_t)N - 1) * K + 4 * g;
   const TA* a_row[MT];
 #pragma unroll
-  for (int i = 0; i < MT; ++i) a_row[i] = A + (int64_t)min(m0 + 16 * i + l, M - 1) * K + 4 * g;
+  for (int i = 0; i < MT; ++i) a_row[i] = A + (int64_t)min(16 * i + l, M - 1) * K + 4 * g;
   const f32x4_fma zero = {0.f, 0.f, 0.f, 0.f};
   f32x4_fma sum[MT], w[2][kStretch], a[2][kStretch][MT];
 #pragma unroll
@@ -112,23 +113,21 @@ __global__ __launch_bounds__(kRuns* kWave) void gemm_f32_rows_kernel(
     }
   };
   auto multiply = [&](int half, int step0) {
-    f32x4_fma chain[MT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i) chain[i] = zero;
 #pragma unroll
     for (int u = 0; u < kStretch; ++u) {
       if (step0 + u >= end) break;
       const bool inside = (step0 + u) * 16 + 4 * g < K;      // (K's last step may be cut)
       const f32x4_fma wv = inside ? w[half][u] : zero;
+      f32x4_fma chain[MT][2];
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
         for (int i = 0; i < MT; ++i)
-          chain[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(inside ? a[half][u][i][r] : 0.f, wv[r],
-                                                          chain[i], 0, 0, 0);
-    }
+          chain[i][r & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              inside ? a[half][u][i][r] : 0.f, wv[r], r < 2 ? zero : chain[i][r & 1], 0, 0, 0);
 #pragma unroll
-    for (int i = 0; i < MT; ++i) sum[i] += chain[i];
+      for (int i = 0; i < MT; ++i) sum[i] += chain[i][0] + chain[i][1];
+    }
   };
   if (begin < end) {
     fetch(0, begin);
@@ -148,8 +147,8 @@ __global__ __launch_bounds__(kRuns* kWave) void gemm_f32_rows_kernel(
     const int at = (row / 4 * 16 + col) * 4 + row % 4;
     float v = 0.f;
 #pragma unroll
-    for (int r = 0; r < kRuns; ++r) v += part[r][i][at];
-    const int m = m0 + 16 * i + row;
+    for (int r = 0; r < kRuns; r += 2) v += part[r][i][at] + part[r + 1][i][at];
+    const int m = 16 * i + row;
     if (m < M && n0 + col < N) C[(int64_t)m * N + n0 + col] = from_f32<TC>(v);
   }
 }
@@ -162,13 +161,14 @@ __global__ __launch_bounds__(kRuns* kWave) void gemm_f32_rows_kernel(
 // LDS and memory, so small products take small tiles and more groups (o and down of the 0.6B
 // shape, 501 rows: 43 us with one group of a 32 x 64 tile, which is as long with 130 rows).
 template <typename TA, typename TW, typename TC, int BM, int BN, int KS, int G>
-__global__ __launch_bounds__(256 * G, BM == 32 ? 4 : BM == 64 ? 2 : 1) void gemm_f32_tile_kernel(
+__global__ __launch_bounds__(256 * G, BM == 32 ? 4 : BM == 64 ? (KS == 32 ? 3 : 2) : 1) void gemm_f32_tile_kernel(
     const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, int M, int N, int K) {
   constexpr int TM = BM / 32, TN = BN / 32, LD = KS + 4, Q = KS / 4, ROWS = BM + BN;
-  constexpr int COUNT = ROWS * Q / 256, STEP = 256 / Q, OWN = kRuns / G, SUMS = G == 1 ? 1 : OWN;
+  constexpr int COUNT = ROWS * Q / 256, STEP = 256 / Q, OWN = kRuns / G;
   constexpr int STEPS = KS / 16, TURNS = kStretch / STEPS;       // steps a turn, turns a stretch
   static_assert(ROWS * Q % 256 == 0 && 256 % Q == 0 && BM % STEP == 0, "whole rows a turn");
   static_assert(STEPS % 2 == 0 && kStretch % STEPS == 0, "operands in two sets by turns");
+  static_assert(G == 1 || OWN == 2, "a group's runs are one pair, or it has all of them");
   extern __shared__ __align__(16) float lds[];
   const int group = __builtin_amdgcn_readfirstlane(threadIdx.x / 256), tid = threadIdx.x % 256;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
@@ -220,103 +220,96 @@ __global__ __launch_bounds__(256 * G, BM == 32 ? 4 : BM == 64 ? 2 : 1) void gemm
   };
   read(0, 0);
   int which = 0;
-  f32x4_fma chain[TM][TN], run[TM][TN], all[SUMS][TM][TN];
-  auto stretch = [&] {
+  // A row of tiles is multiplied while the row before is added to its run.
+  f32x4_fma chain[2][TN][2], run[TM][TN], pair[TM][TN], all[TM][TN];
+  auto add = [&](int row, int set) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int j = 0; j < TN; ++j) run[row][j] += chain[set][j][0] + chain[set][j][1];
+  };
+  auto turn = [&] {
+    commit(which ^ 1);
+    fetch();
 #pragma unroll
-      for (int j = 0; j < TN; ++j) chain[i][j] = zero;
+    for (int u = 0; u < STEPS; ++u) {
+      if (u + 1 < STEPS) {
+        read(which, u + 1);
+      } else {
+        __syncthreads();
+        which ^= 1;
+        read(which, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int turn = 0; turn < TURNS; ++turn) {
-      commit(which ^ 1);
-      fetch();
-#pragma unroll
-      for (int u = 0; u < STEPS; ++u) {
-        if (u + 1 < STEPS) {
-          read(which, u + 1);
-        } else {
-          __syncthreads();
-          which ^= 1;
-          read(which, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
+      for (int i = 0; i < TM; ++i) {
+        const int set = (u * TM + i) & 1;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
-          for (int i = 0; i < TM; ++i)
+          for (int j = 0; j < TN; ++j)
+            chain[set][j][r & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                af[u & 1][i][r], wf[u & 1][j][r], r < 2 ? zero : chain[set][j][r & 1], 0, 0, 0);
+        add(i > 0 ? i - 1 : TM - 1, set ^ 1);
+        // (the additions in the products' shadow, from the fourth product on, when the last ones
+        // of the row before have ended)
+        __builtin_amdgcn_sched_group_barrier(8, 3, 0);
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
-              chain[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[u & 1][i][r], wf[u & 1][j][r],
-                                                                 chain[i][j], 0, 0, 0);
+        for (int m = 3; m < 4 * TN; ++m) {
+          __builtin_amdgcn_sched_group_barrier(8, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(2, TN == 2 ? 4 : 3, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
   };
-  auto whole_run = [&] {
+  auto clear = [&](f32x4_fma (&sums)[TM][TN]) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) run[i][j] = zero;
-    for (int s = 0; s < per; ++s) {
-      stretch();
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) run[i][j] += chain[i][j];
-    }
+      for (int j = 0; j < TN; ++j) sums[i][j] = zero;
   };
-  // (one group adds its runs up as they end, several keep theirs apart until all are there)
-#pragma unroll
-  for (int o = 0; o < SUMS; ++o)
+  auto gather = [&](f32x4_fma (&sums)[TM][TN], const f32x4_fma (&more)[TM][TN]) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) all[o][i][j] = zero;
-  if constexpr (G == 1) {
-    for (int o = 0; o < OWN && o * per * 16 * kStretch < K; ++o) {
-      whole_run();
+      for (int j = 0; j < TN; ++j) sums[i][j] += more[i][j];
+  };
+  clear(all);
+  // (of one group, runs behind K are left out; several meet at the same barriers and make theirs)
+  auto there = [&](int own) { return G > 1 || own * per * 16 * kStretch < K; };
+#pragma unroll 1
+  for (int o = 0; o < OWN && there(o); o += 2) {
+    clear(pair);
+#pragma unroll 1
+    for (int half = 0; half < 2; ++half) {
+      clear(run);
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) all[0][i][j] += run[i][j];
+      for (int j = 0; j < TN; ++j) chain[1][j][0] = chain[1][j][1] = zero;
+#pragma unroll 1
+      for (int t = 0; t < per * TURNS; ++t) turn();
+      add(TM - 1, 1);
+      gather(pair, run);
     }
-  } else {
-#pragma unroll
-    for (int o = 0; o < OWN; ++o) {
-      whole_run();
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) all[o][i][j] = run[i][j];
-    }
+    gather(all, pair);
   }
   __syncthreads();
   if (G > 1) {
-    // the other groups' runs through LDS, [group - 1][run][wave][tile][lane]
-    auto at = [&](int gr, int o, int i, int j) {
-      return (f32x4_fma*)(lds + (((((gr - 1) * OWN + o) * 4 + wave) * TM + i) * TN + j) * 256 + lane * 4);
+    // the other groups' pair of runs through LDS, [group - 1][wave][tile][lane]
+    auto at = [&](int gr, int i, int j) {
+      return (f32x4_fma*)(lds + ((((gr - 1) * 4 + wave) * TM + i) * TN + j) * 256 + lane * 4);
     };
     if (group > 0) {
 #pragma unroll
-      for (int o = 0; o < OWN; ++o)
+      for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) *at(group, o, i, j) = all[o][i][j];
+        for (int j = 0; j < TN; ++j) *at(group, i, j) = all[i][j];
     }
     __syncthreads();
     if (group > 0) return;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        f32x4_fma v = zero;
-#pragma unroll
-        for (int o = 0; o < OWN; ++o) v += all[o][i][j];
-        for (int gr = 1; gr < G; ++gr)
-#pragma unroll
-          for (int o = 0; o < OWN; ++o) v += *at(gr, o, i, j);
-        all[0][i][j] = v;
-      }
+      for (int j = 0; j < TN; ++j)
+        for (int gr = 1; gr < G; ++gr) all[i][j] += *at(gr, i, j);
   }
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -325,13 +318,13 @@ __global__ __launch_bounds__(256 * G, BM == 32 ? 4 : BM == 64 ? 2 : 1) void gemm
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int64_t m = m0 + (wm * TM + i) * 16 + 4 * g + r, n = n0 + (wn * TN + j) * 16 + l;
-        if (m < M && n < N) C[m * N + n] = from_f32<TC>(all[0][i][j][r]);
+        if (m < M && n < N) C[m * N + n] = from_f32<TC>(all[i][j][r]);
       }
 }
 
 template <typename TA, typename TW, typename TC, int BM, int BN, int KS, int G>
 static int launch_tile(const TA* A, const TW* W, TC* C, int M, int N, int K, hipStream_t stream) {
-  constexpr int operands = G * 2 * (BM + BN) * (KS + 4), sums = (G - 1) * (kRuns / G) * BM * BN;
+  constexpr int operands = G * 2 * (BM + BN) * (KS + 4), sums = (G - 1) * BM * BN;
   const size_t lds = (size_t)(operands > sums ? operands : sums) * sizeof(float);
   auto* fn = gemm_f32_tile_kernel<TA, TW, TC, BM, BN, KS, G>;
   if (lds > 64 * 1024 &&
@@ -359,6 +352,10 @@ static int launch_f32(const TA* A, const TW* W, TC* C, int M, int N, int K, hipS
   // the largest tile that still gives every unit one
   auto tiles = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   if (tiles(128, 128) >= 256) return launch_tile<TA, TW, TC, 128, 128, 32, 1>(A, W, C, M, N, K, stream);
+  // (64 x 64: half as many turns, or the third workgroup of a unit where there is one: 512 and 768
+  // tiles of K = 1,024 54.5 and 84.0 us with turns of 64, 54.6 and 78.1 with turns of 32; 256 of
+  // K = 8,192 232 and 246)
+  if (tiles(64, 64) > 512) return launch_tile<TA, TW, TC, 64, 64, 32, 1>(A, W, C, M, N, K, stream);
   if (tiles(64, 64) >= 256) return launch_tile<TA, TW, TC, 64, 64, 64, 1>(A, W, C, M, N, K, stream);
   return launch_tile<TA, TW, TC, 32, 64, 32, 4>(A, W, C, M, N, K, stream);
 }
