@@ -280,3 +280,29 @@ def test_what_is_not_finite_does_not_reach_earlier_tokens(gpu_device, mode, what
             assert not out[t].isfinite().all() or (mode == "scan" and what == "gates"), (t, value)
             if what == "q":
                 assert torch.equal(out[t + 1:], want[t + 1:]), (t, value)
+
+
+@pytest.mark.parametrize("shift", [6, 9, 11])
+def test_equal_decays_do_not_add_up_their_roundings(gpu_device, shift):
+    """A chunk's whole decay is rounded once, by 2^-24 of itself at most, and what is j chunks old
+    has met it j times: 1 / (1 - g^64) times on average; beside it the sums' own roundings (the mean
+    square of 64 in a chain is 32, each less than 0.45 x 2^-24; as many again for the products)."""
+    ops, gen = load_hip_ops(gpu_device), torch.Generator().manual_seed(11)
+    heads, dim, vdim, T, g = 2, 64, 32, 1500, 1 - 2.0 ** -shift
+    requests = Requests(gpu_device, (heads, dim, vdim), 1)
+    batch = requests.step([T])
+    x = torch.randn(T, heads * (2 * dim + vdim), generator=gen)
+    x[:, :2 * heads * dim] *= dim ** -0.25
+    out = ops.linear_recurrence(
+        x.to(gpu_device), 0, heads * dim, 2 * heads * dim, batch, requests.state, heads=heads,
+        kv_heads=heads, dim=dim, vdim=vdim, silu_inputs=False,
+        decay=torch.full((heads,), g).to(gpu_device))
+    q, k, v = x.double().split([heads * dim] * 2 + [heads * vdim], 1)
+    want, S = walk(q.view(T, heads, dim), k.view(T, heads, dim), v.view(T, heads, vdim),
+                   torch.full((T, heads, 1), g, dtype=torch.float64), None,
+                   torch.zeros(heads, dim, vdim, dtype=torch.float64))
+    bound = 2.0 ** -24 * (1 / (1 - g ** 64) + 0.45 * 64 ** 0.5)
+    state = requests.state[batch.slot_ids.long()][0].double().cpu()
+    assert (state - S).norm() <= bound * S.norm()
+    want = want.view(T, -1)
+    assert (out.double().cpu() - want).norm() <= 2 * bound * want.norm()

@@ -174,25 +174,28 @@ struct HeadDecays {
   __device__ float* total() const { return at + 6 * kTok; }   // of the four blocks
 };
 
-// One wavefront, a token a lane (dec 1 behind the chunk's end), fills them in.
+// One wavefront, a token a lane (dec 1 behind the chunk's end), fills them in.  The products are
+// made by doubling, in 64 bits: equal decays have equal roundings, which every doubling doubles (a
+// chunk's whole decay was off by up to 32 of them, and every chunk's by the same: with decays of
+// 1 - 2^-9 outputs by 1.7e-6 instead of 4.6e-7).
 __device__ __forceinline__ void spread_decays(HeadDecays d, float dec, float vs, int lane) {
   const int l = lane % 16, blk = lane / 16;
-  float p = dec, q = dec;
+  double p = dec, q = dec;
 #pragma unroll
   for (int o = 1; o < 16; o <<= 1) {
-    const float x = __shfl_up(p, o, 16), y = __shfl_down(q, o, 16);
-    p *= l >= o ? x : 1.f;
-    q *= l + o < 16 ? y : 1.f;
+    const double x = __shfl_up(p, o, 16), y = __shfl_down(q, o, 16);
+    p *= l >= o ? x : 1.;
+    q *= l + o < 16 ? y : 1.;
   }
-  const float behind = __shfl_down(q, 1, 16), suf = l < 15 ? behind : 1.f;
-  const float t0 = __shfl(p, 15, 64), t1 = __shfl(p, 31, 64), t2 = __shfl(p, 47, 64), t3 = __shfl(p, 63, 64);
+  const double behind = __shfl_down(q, 1, 16), suf = l < 15 ? behind : 1.;
+  const double t0 = __shfl(p, 15, 64), t1 = __shfl(p, 31, 64), t2 = __shfl(p, 47, 64), t3 = __shfl(p, 63, 64);
   d.g()[lane] = dec;
-  d.pre()[lane] = p;
-  d.suf()[lane] = suf;
+  d.pre()[lane] = (float)p;
+  d.suf()[lane] = (float)suf;
   d.vs()[lane] = vs;
-  d.d0()[lane] = p * (blk == 0 ? 1.f : blk == 1 ? t0 : blk == 2 ? t0 * t1 : t0 * t1 * t2);
-  d.es()[lane] = suf * (blk == 3 ? 1.f : blk == 2 ? t3 : blk == 1 ? t2 * t3 : t1 * t2 * t3);
-  if (l == 15) d.total()[blk] = p;
+  d.d0()[lane] = (float)(p * (blk == 0 ? 1. : blk == 1 ? t0 : blk == 2 ? t0 * t1 : t0 * t1 * t2));
+  d.es()[lane] = (float)(suf * (blk == 3 ? 1. : blk == 2 ? t3 : blk == 1 ? t2 * t3 : t1 * t2 * t3));
+  if (l == 15) d.total()[blk] = (float)p;
 }
 
 // M(t, s) for rows t = 4 g + r and column s = l of tile (i, j), j <= i; zero above the diagonal.
@@ -395,15 +398,15 @@ __global__ __launch_bounds__(kThreads, 2) void chunk_local_kernel(ChunkedArgs a,
   for (int i = w; i < heads_each; i += 4) {
     float dec = 1.f, vs = 0.f;
     if (lane < c.nt) token_scalars(a, c.first + lane, h0 + i, dec, vs);
-    float p = dec;                         // the product from this token through the last
-#pragma unroll
+    double p = dec;                        // the product from this token through the last (64 bits:
+#pragma unroll                             // see spread_decays)
     for (int o = 1; o < 64; o <<= 1) {
-      const float q = __shfl_down(p, o, 64);
-      p *= lane + o < 64 ? q : 1.f;
+      const double q = __shfl_down(p, o, 64);
+      p *= lane + o < 64 ? q : 1.;
     }
-    const float behind = __shfl_down(p, 1, 64);
-    scale[i * kTok + lane] = vs * (lane < 63 ? behind : 1.f);
-    if (lane == 0) a.scratch[parts.totals + ((int64_t)chunk * a.heads + h0 + i) * NP] = p;
+    const double behind = __shfl_down(p, 1, 64);
+    scale[i * kTok + lane] = vs * (float)(lane < 63 ? behind : 1.);
+    if (lane == 0) a.scratch[parts.totals + ((int64_t)chunk * a.heads + h0 + i) * NP] = (float)p;
   }
   stage_rows<NP, FORM>(a, Ks, a.k_col + hk * a.N, c.first, c.nt, c.pos0, true, wide);
   __syncthreads();
