@@ -64,6 +64,9 @@ __device__ __forceinline__ f32x4 mfma4(f32x4 a, f32x4 b, f32x4 c) {
   for (int r = 0; r < 4; ++r) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], c, 0, 0, 0);
   return c;
 }
+// A product of 16 by itself, to be added to others: chains of 16, or an element's error is that of
+// one chain over all of them.
+__device__ __forceinline__ f32x4 product4(f32x4 a, f32x4 b) { return mfma4(a, b, f32x4{0.f, 0.f, 0.f, 0.f}); }
 __device__ __forceinline__ f32x4 read4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 __device__ __forceinline__ void write4(float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
 __device__ __forceinline__ int tri(int i, int j) { return i * (i + 1) / 2 + j; }
@@ -223,7 +226,7 @@ __device__ __forceinline__ f32x4 gram_tile(const float* a, const float* b, int l
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
   for (int j = 0; j < NT; ++j)
-    acc = mfma4(read4(a + l * LD + 16 * j + 4 * g), read4(b + l * LD + 16 * j + 4 * g), acc);
+    acc += product4(read4(a + l * LD + 16 * j + 4 * g), read4(b + l * LD + 16 * j + 4 * g));
   return acc;
 }
 
@@ -256,20 +259,20 @@ __device__ __forceinline__ void read_run(const float* p, float (&v)[PER]) {
   }
 }
 
-// acc + T u for a diagonal tile T in LDS, zero above its diagonal: row t takes u of its own and of
+// T u for a diagonal tile T in LDS, zero above its diagonal: row t takes u of its own and of
 // earlier tokens.  Zero times what is not finite is not zero, so where such u are among the
 // sixteen a row at a time is made, with the later ones left out, and taken.
-__device__ __forceinline__ f32x4 causal_product(const float* tile, f32x4 u, f32x4 acc, int l, int g) {
+__device__ __forceinline__ f32x4 causal_product(const float* tile, f32x4 u, int l, int g) {
   const f32x4 a = read4(tile + l * kTileLd + 4 * g);
   if (__builtin_amdgcn_ballot_w64(!(fabsf(u[0]) + fabsf(u[1]) + fabsf(u[2]) + fabsf(u[3]) < INFINITY)) == 0)
-    return mfma4(a, u, acc);
-  f32x4 out = acc;
+    return product4(a, u);
+  f32x4 out;
 #pragma unroll 1
   for (int t = 0; t < 16; ++t) {
     f32x4 seen;
 #pragma unroll
     for (int r = 0; r < 4; ++r) seen[r] = 4 * g + r <= t ? u[r] : 0.f;
-    const f32x4 sums = mfma4(a, seen, acc);
+    const f32x4 sums = product4(a, seen);
 #pragma unroll
     for (int r = 0; r < 4; ++r) out[r] = 4 * g + r == t ? sums[r] : out[r];
   }
@@ -347,7 +350,7 @@ __device__ __forceinline__ f32x4 split_tile(const float* pre, const float* post,
     const int n = 16 * c + 4 * g;
     f32x4 b = read4(post + (16 * j + l) * LD + n);
     for (int m = j + 1; m < i; ++m) b *= read4(blocks + m * NP + n);
-    acc = mfma4(read4(pre + (16 * i + l) * LD + n), b, acc);
+    acc += product4(read4(pre + (16 * i + l) * LD + n), b);
   }
   return acc;
 }
@@ -444,7 +447,7 @@ __global__ __launch_bounds__(kThreads, 2) void chunk_local_kernel(ChunkedArgs a,
           if (w + 4 * o >= NT) break;
           f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int j = 0; j < 4; ++j) acc = mfma4(kf[o][j], vf[j], acc);
+          for (int j = 0; j < 4; ++j) acc += product4(kf[o][j], vf[j]);
           write4(share + ((int64_t)(c0 / 16 + ct) * NT + w + 4 * o) * 256 + lane * 4, acc);
         }
       }
@@ -602,9 +605,8 @@ __device__ __forceinline__ void solve_chunk(const ChunkedArgs& a, const ChunkRan
       if (ROW && ct < NT) whole *= blocks[i * NP + n];
 #pragma unroll
       for (int m = 0; m < i; ++m)
-        acc = mfma4(read4(tiles + tri(i, m) * kTile + l * kTileLd + 4 * g), X[m], acc);
-      const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-      X[i] = causal_product(tiles + tri(i, i) * kTile, acc, zero, l, g);
+        acc += product4(read4(tiles + tri(i, m) * kTile + l * kTileLd + 4 * g), X[m]);
+      X[i] = causal_product(tiles + tri(i, i) * kTile, acc, l, g);
       if (ct < NT) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
@@ -719,20 +721,21 @@ __global__ __launch_bounds__(kThreads, 1) void chunk_walk_kernel(ChunkedArgs a) 
     for (int o = 0; o < OWN; ++o)
       if (owns(o)) write4(&s_lds[w + 4 * o][lane * 4], S[o]);
     __syncthreads();
-    f32x4 acc[2] = {f.y, zero}, s[NT];     // two chains
+    f32x4 mine = f.y, part[2], s[NT];
 #pragma unroll
     for (int j = 0; j < NT; ++j) s[j] = read4(&s_lds[j][lane * 4]);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-      acc[j & 1] = mfma4(f.w[j], s[j], acc[j & 1]);
+      part[j & 1] = product4(f.w[j], s[j]);
+      if (j > 0) mine += part[(j - 1) & 1];
       fetch_w(ahead, later, j);
       __builtin_amdgcn_sched_barrier(0);
     }
-    const f32x4 mine = acc[0] + acc[1];
+    mine += part[(NT - 1) & 1];
     write4(&u_lds[w][lane * 4], mine);
     __syncthreads();
-    f32x4 u[4];
+    f32x4 u[4], more[2][OWN];
 #pragma unroll
     for (int i = 0; i < 4; ++i) u[i] = read4(&u_lds[i][lane * 4]);
     write4(a.scratch + parts.u + ((unit * PT + ct) * 4 + w) * 256 + lane * 4, mine);
@@ -748,10 +751,16 @@ __global__ __launch_bounds__(kThreads, 1) void chunk_walk_kernel(ChunkedArgs a) 
       for (int r = 0; r < 4; ++r)
 #pragma unroll
         for (int o = 0; o < OWN; ++o)
-          S[o] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.kt[o][i][r], u[i][r], S[o], 0, 0, 0);
+          more[i & 1][o] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.kt[o][i][r], u[i][r],
+                                                                r ? more[i & 1][o] : zero, 0, 0, 0);
+#pragma unroll
+      for (int o = 0; o < OWN; ++o)
+        if (i > 0) S[o] += more[(i - 1) & 1][o];
       fetch_kt(ahead, later, i);
       __builtin_amdgcn_sched_barrier(0);
     }
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) S[o] += more[1][o];
   };
   WalkOperands<NT> ring[4];
 #pragma unroll
@@ -875,7 +884,7 @@ __device__ __forceinline__ void output_chunk(const ChunkedArgs& a, const ChunkRa
             v[j][r] = t < nt && p < a.P ? col[(int64_t)t * a.ld] : 0.f;
           }
       }
-      f32x4 acc[RT], q[2][RT];
+      f32x4 acc[RT], part[2][RT], q[2][RT];
       auto fetch = [&](int j) {
 #pragma unroll
         for (int i = 0; i < RT; ++i) {
@@ -894,9 +903,27 @@ __device__ __forceinline__ void output_chunk(const ChunkedArgs& a, const ChunkRa
         for (int r = 0; r < 4; ++r)
 #pragma unroll
           for (int i = 0; i < RT; ++i)
-            acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[j & 1][i][r], s0[j][r], acc[i], 0, 0, 0);
+            part[j & 1][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[j & 1][i][r], s0[j][r],
+                                                                  r ? part[j & 1][i] : zero, 0, 0, 0);
+        // (the sixteen before are added meanwhile; put off to the end by the compiler otherwise, which
+        // then has no registers left)
+        if (j > 0) {
+#pragma unroll
+          for (int i = 0; i < RT; ++i) {
+            acc[i] += part[(j - 1) & 1][i];
+            asm volatile("" : "+v"(acc[i]));
+          }
+        }
+        __builtin_amdgcn_sched_group_barrier(8, 3, 0);
+#pragma unroll
+        for (int m = 3; m < 4 * RT; ++m) {
+          __builtin_amdgcn_sched_group_barrier(8, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(2, 2, 0);
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
+#pragma unroll
+      for (int i = 0; i < RT; ++i) acc[i] += part[(NT - 1) & 1][i];
       if (FORM == kSilu) {
 #pragma unroll
         for (int j = 0; j < RT; ++j)
@@ -910,8 +937,8 @@ __device__ __forceinline__ void output_chunk(const ChunkedArgs& a, const ChunkRa
 #pragma unroll
         for (int j = 0; j <= i; ++j) {
           const f32x4 u = DELTA ? v[j] : v[j] * read4(d.vs() + 16 * j + 4 * g);
-          if (i == j) acc[i] = causal_product(tiles + tri(i, i) * kTile, u, acc[i], l, g);
-          else acc[i] = mfma4(read4(tiles + tri(i, j) * kTile + l * kTileLd + 4 * g), u, acc[i]);
+          acc[i] += i == j ? causal_product(tiles + tri(i, i) * kTile, u, l, g)
+                           : product4(read4(tiles + tri(i, j) * kTile + l * kTileLd + 4 * g), u);
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
