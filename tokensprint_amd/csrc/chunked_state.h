@@ -37,5 +37,5 @@ struct ChunkedArgs {
 };
 
 // Floats of scratch that launch_chunked wants; -1: these sizes are not built in chunks.
-int64_t chunked_scratch_floats(int num_chunks, int heads, int N, int P, int delta, int per_row);
+int64_t chunked_scratch_floats(int num_chunks, int heads, int N, int P, int delta);
 int launch_chunked(ChunkedArgs a, hipStream_t stream);

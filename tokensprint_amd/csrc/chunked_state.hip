@@ -1016,20 +1016,19 @@ int launch_delta(const ChunkedArgs& a, int wide, hipStream_t stream) {
 
 }  // namespace
 
-int64_t chunked_scratch_floats(int num_chunks, int heads, int N, int P, int delta, int per_row) {
+int64_t chunked_scratch_floats(int num_chunks, int heads, int N, int P, int delta) {
   if (N < 1 || P < 1 || N > (delta ? 128 : 256)) return -1;
-  (void)per_row;
   return parts_of(num_chunks, heads, N, P, delta).end;
 }
 
-extern "C" int64_t ts_chunked_scratch(int num_chunks, int heads, int N, int P, int delta, int per_row) {
-  return chunked_scratch_floats(num_chunks, heads, N, P, delta, per_row);
+extern "C" int64_t ts_chunked_scratch(int num_chunks, int heads, int N, int P, int delta) {
+  return chunked_scratch_floats(num_chunks, heads, N, P, delta);
 }
 
 extern "C" int ts_chunk_tokens() { return kChunkTokens; }
 
 int launch_chunked(ChunkedArgs a, hipStream_t stream) {
-  if (chunked_scratch_floats(a.num_chunks, a.heads, a.N, a.P, a.delta, a.per_row) < 0)
+  if (chunked_scratch_floats(a.num_chunks, a.heads, a.N, a.P, a.delta) < 0)
     TS_FAIL("chunked recurrence: %d rows of S are not built", a.N);
   if (a.num_chunks > 65535 || a.num_entries > 65535 || a.P > 1 << 19)
     TS_FAIL("chunked recurrence: %d chunks, %d entries, %d columns", a.num_chunks, a.num_entries, a.P);

@@ -257,12 +257,12 @@ __global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgs g
 #pragma unroll
       for (int i = 0; i < LOADS; ++i) issue_one(s, s, i);
     row_scales();
-    // a turn; `in_flight`: the loads that may still be on their way when step kt has arrived.
-    // (The last one, which sends nothing, apart: no branch in the others.  The gate/up product
-    // of 2,048 rows at 2 x 3,072 x 1,024 in 256 x 192 tiles 31.6 -> 30.4 us.)
-    auto turn = [&](auto in_flight, auto with_loads, int s, int kt) {
+    // a turn: everything that was sent for has to have arrived.  (The last one, which sends
+    // nothing, apart: no branch in the others.  The gate/up product of 2,048 rows at
+    // 2 x 3,072 x 1,024 in 256 x 192 tiles 31.6 -> 30.4 us.)
+    auto turn = [&](auto with_loads, int s, int kt) {
       constexpr bool load = decltype(with_loads)::value;
-      wait_loads<decltype(in_flight)::value>();
+      wait_loads<0>();
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
@@ -286,20 +286,19 @@ __global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgs g
 #pragma unroll
             for (int j = 0; j < PER; ++j) {
               const int i = (ks * TM + tm) * PER + j;
-              if (i < LOADS) issue_one((s + STAGES - 1) % STAGES, kt + STAGES - 1, i);
+              if (i < LOADS) issue_one(s ^ 1, kt + 1, i);
             }
           }
         }
       }
     };
     static_assert(STAGES == 2, "the turns are written out for a ring of two");
-    using none = std::integral_constant<int, 0>;
     for (int kt = 0; kt + 2 < KT; kt += 2) {
-      turn(none{}, std::true_type{}, 0, kt);
-      turn(none{}, std::true_type{}, 1, kt + 1);
+      turn(std::true_type{}, 0, kt);
+      turn(std::true_type{}, 1, kt + 1);
     }
-    if (KT % 2 == 0) turn(none{}, std::true_type{}, 0, KT - 2);
-    turn(none{}, std::false_type{}, (KT - 1) % 2, KT - 1);
+    if (KT % 2 == 0) turn(std::true_type{}, 0, KT - 2);
+    turn(std::false_type{}, (KT - 1) % 2, KT - 1);
   } else {
 #pragma unroll
   for (int s = 0; s < STAGES; ++s)

@@ -127,11 +127,11 @@ struct Eight<float> {
   __device__ __forceinline__ void set(int j, float v) { if (j < 4) lo[j] = v; else hi[j - 4] = v; }
 };
 
-// Values of many tokens into their pages (bfloat16 to bfloat16).  A page holds values
-// transposed, [head element][position], so a token's head vector lands two bytes at a
+// Values of many tokens into their pages (of the rows' own type).  A page holds values
+// transposed, [head element][position], so a token's head vector lands an element at a
 // time, hd rows apart: here 16 lanes take 16 consecutive tokens for the same 8 head
-// elements, and since consecutive tokens of a prompt sit at consecutive positions, the 16
-// two-byte stores of one row fall into one 32-byte run of the page.  A workgroup of 256
+// elements, and since consecutive tokens of a prompt sit at consecutive positions, the
+// stores of one row fall into one run of 16 elements of the page.  A workgroup of 256
 // takes (tile of 16 tokens, key/value head); its 16 lane groups take 8 head elements
 // each, in rounds.
 template <typename T>

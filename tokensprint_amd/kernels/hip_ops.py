@@ -446,7 +446,7 @@ class HipOps:
     @staticmethod
     def _mfma_ok(x, weight):
         """The matrix-core product takes bfloat16 operands with K a multiple of 8;
-        everything else (float32 anywhere) goes to the float32 multiply-add kernel."""
+        everything else (float32 anywhere) goes to the float32 kernels."""
         return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
                 and x.shape[1] % 8 == 0)
 
@@ -1299,11 +1299,11 @@ class HipOps:
                    _ptr(entry_chunks), num_chunks, _ptr(scratch), self._stream())
         return y
 
-    def _chunk_scratch(self, num_chunks, heads, rows, cols, delta=False, per_row=False):
+    def _chunk_scratch(self, num_chunks, heads, rows, cols, delta=False):
         """What the kernels of a recurrence in chunks hand each other; None without chunks."""
         if not num_chunks:
             return None
-        count = self.lib.ts_chunked_scratch(num_chunks, heads, rows, cols, int(delta), int(per_row))
+        count = self.lib.ts_chunked_scratch(num_chunks, heads, rows, cols, int(delta))
         if count < 0:
             raise KernelError(f"recurrence in chunks: {rows} x {cols} states are not built")
         return torch.empty(count, dtype=torch.float32, device=self.device)
@@ -1400,7 +1400,7 @@ class HipOps:
         chunks, entry_chunks, num_chunks = None, None, 0
         if dim <= (128 if delta else 256) and not (delta and silu_inputs):
             chunks, entry_chunks, num_chunks = self._scan_chunks(batch)
-        scratch = self._chunk_scratch(num_chunks, heads, dim, vdim, delta, per_channel)
+        scratch = self._chunk_scratch(num_chunks, heads, dim, vdim, delta)
         self._call(self.lib.ts_linear_recurrence, _ptr(x), ld, int(q_col), int(k_col), int(v_col),
                    _ptr(decay), _ptr(gates), ldg, _ptr(state), _ptr(out), pos, eot, qs, slots, T,
                    batch.num_entries, int(batch.max_q_len), heads, kv_heads, dim, vdim,

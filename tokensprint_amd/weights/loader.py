@@ -95,7 +95,7 @@ def held_dtype(decl: TensorDecl, stored: torch.dtype, run_dtype: torch.dtype,
     Small vectors are held in float32 (exact for bfloat16 values) and integer
     tables in int32.  Matrices follow the run dtype, except that in a bfloat16 run
     a matrix the file stores in 32-bit stays 32-bit (its products then run on the
-    float32 multiply-add kernels) unless `cast_32bit` asks for it to be rounded.
+    float32 kernels) unless `cast_32bit` asks for it to be rounded.
     """
     if decl.role == "table" or not stored.is_floating_point:
         return torch.int32
@@ -141,7 +141,7 @@ def load_weights(model, source, run_dtype: torch.dtype, device, cast_32bit: bool
         tensors[name] = t.to(device=device, dtype=held).contiguous()
     if kept_wide:
         log.warning("%d matrices are stored in 32-bit and stay so in this bfloat16 run (%s, ...): "
-                    "their products run on the float32 multiply-add kernels, many times slower "
-                    "than the bfloat16 ones; load with cast_32bit=True (--cast-weights True) to "
+                    "their products run on the float32 kernels, which read twice the bytes and "
+                    "multiply at a sixteenth of the bfloat16 rate; load with cast_32bit=True (--cast-weights True) to "
                     "round them to bfloat16", len(kept_wide), kept_wide[0])
     model.load_tensors(tensors)
