@@ -309,7 +309,7 @@ class TorchOps:
 
     def linear_recurrence(self, x, q_col, k_col, v_col, batch, state, *, heads, kv_heads, dim,
                           vdim, silu_inputs, decay=None, gates=None, per_channel=False,
-                          delta=False, turn=None, k_scale=1.0):
+                          delta=False, turn=None, k_scale=1.0, walk=False):
         T = x.shape[0]
         rep = heads // kv_heads
 

@@ -336,3 +336,31 @@ def test_chunks_round_no_more_than_chains_of_sixteen_do(gpu_device, mode):
     assert (out.double().cpu() - want).norm() <= bound * want.norm()
     state = requests.state[batch.slot_ids.long()][0].double().cpu()
     assert (state - S).norm() <= bound * S.norm()
+
+
+@pytest.mark.parametrize("per_channel", [False, True])
+def test_walked_portions_do_not_depend_on_the_cut(gpu_device, per_channel):
+    """The same sums in the same order, so the same to the bit, for portions that the same number of
+    lanes walks (from eight tokens on)."""
+    ops, gen = load_hip_ops(gpu_device), torch.Generator().manual_seed(13)
+    heads, dim, vdim, T = 3, 48, 40, 210
+    n = heads * dim if per_channel else heads
+    x = torch.randn(T, heads * (2 * dim + vdim), generator=gen)
+    x[:, heads * dim:2 * heads * dim] *= dim ** -0.5
+    gates = torch.cat([torch.rand(T, heads, generator=gen), torch.rand(T, n, generator=gen) ** 0.1], 1)
+    x, gates = x.to(gpu_device), gates.to(gpu_device)
+
+    def run(portions):
+        requests, at, outs = Requests(gpu_device, (heads, dim, vdim), 1), 0, []
+        for rows in portions:
+            outs.append(ops.linear_recurrence(
+                x[at:at + rows].contiguous(), 0, heads * dim, 2 * heads * dim, requests.step([rows]),
+                requests.state, heads=heads, kv_heads=heads, dim=dim, vdim=vdim, silu_inputs=False,
+                delta=True, per_channel=per_channel, gates=gates[at:at + rows].contiguous(), walk=True))
+            at += rows
+        assert at == T
+        return torch.cat(outs)
+
+    whole = run([T])
+    for portions in ([70, 13, 127], [8, 9, 64, 129]):
+        assert torch.equal(run(portions), whole), portions

@@ -1366,7 +1366,7 @@ class HipOps:
 
     def linear_recurrence(self, x, q_col, k_col, v_col, batch, state, *, heads, kv_heads, dim,
                           vdim, silu_inputs, decay=None, gates=None, per_channel=False,
-                          delta=False, turn=None, k_scale=1.0):
+                          delta=False, turn=None, k_scale=1.0, walk=False):
         """Per head and entry, a token at a time: S <- g S; u = v, or (`delta`)
         u = beta (v - S^T k); S <- S + k u^T; o = S^T q -> float32 [T, heads * vdim].
         `x` (float32 [T, ld]) holds q and k (kv_heads x dim; head h reads q/k head
@@ -1376,7 +1376,9 @@ class HipOps:
         S).  `state` [slots, heads, dim, vdim] float32 carries S from step to step.  `turn`
         (float32 [positions, pairs, 2], cosines and sines): channels 2i and 2i + 1 of every q
         and k head, i < pairs, are turned as a pair by the row of their token's position, and
-        k is multiplied by `k_scale` (plain operands, no delta rule)."""
+        k is multiplied by `k_scale` (plain operands, no delta rule).  `walk`: portions of any
+        length a token at a time, none in chunks, so that a token adds up the same sums however
+        its request is cut (their order differs with the lanes that share a column alone)."""
         self._check("x", x, torch.float32, ndim=2)
         T, ld = x.shape
         if turn is not None:
@@ -1398,7 +1400,7 @@ class HipOps:
         # a long portion runs in chunks, as products of matrices (the delta rule with operands as
         # they stand: with their SiLU taken on the way it is walked)
         chunks, entry_chunks, num_chunks = None, None, 0
-        if dim <= (128 if delta else 256) and not (delta and silu_inputs):
+        if dim <= (128 if delta else 256) and not walk and not (delta and silu_inputs):
             chunks, entry_chunks, num_chunks = self._scan_chunks(batch)
         scratch = self._chunk_scratch(num_chunks, heads, dim, vdim, delta)
         self._call(self.lib.ts_linear_recurrence, _ptr(x), ld, int(q_col), int(k_col), int(v_col),
