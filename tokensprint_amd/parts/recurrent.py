@@ -27,6 +27,17 @@ from tokensprint_amd.parts.base import (MIXERS, Mixer, SlotStateNeed, TensorDecl
                                         flat_needs, register)
 
 
+def walks_portions(ctx) -> bool:
+    """Whether long portions are walked a token at a time and not run in chunks: in float32 runs,
+    whose logits then do not hang on how a request is cut.  (Twelve small models with large
+    weights, requests whole against portions and against steps beside others: where recurrences
+    are all that a cut changes, largest differences of 0.2 to 1.1 times 5e-5 + 1e-4 of the value
+    in chunks, 0.00 to 0.01 walked.  In a bfloat16 run the rounding of operands hides it.  Heads
+    of 128 x 128, 2,048 tokens: 498 us a layer walked, 78 in chunks, 230 in chunks of
+    multiply-adds; the delta rule's 590 and 125.)"""
+    return ctx.dtype == torch.float32
+
+
 class FixedDecayAttention(Mixer):
     """Linear attention with a fixed decay per head: S <- decay_h S + k v^T, o = S^T q, with q,
     k, v and a gate from one product; o passes an RMS norm and the gate, then the output
@@ -92,7 +103,8 @@ class FixedDecayAttention(Mixer):
         o = ops.linear_recurrence(
             proj, 0, self.qk, 2 * self.qk, batch, cache.states[self.state_name],
             heads=self.heads, kv_heads=self.heads, dim=self.dim, vdim=self.vdim,
-            silu_inputs=self.silu_inputs, decay=self.decay, **self.turning)
+            silu_inputs=self.silu_inputs, decay=self.decay, walk=walks_portions(self.ctx),
+            **self.turning)
         gated = ops.norm_gate(o, proj, 2 * self.qk + self.inner, self.norm_w,
                               groups=self.norm_groups, gate=self.gate, eps=self.eps,
                               out_dtype=self.ctx.dtype)
@@ -239,14 +251,11 @@ class GatedDeltaRule(Mixer):
         beta_g = ops.delta_gates(qkv, proj, b_col, z, z_col, self.a_log, self.dt_bias,
                                  heads=H, kv_heads=self.kv_heads, dim=self.dim,
                                  per_channel=self.per_channel)
-        # (a float32 run walks its portions.  In chunks, a request whole and the same request in
-        # portions gave logits further apart, over eight small models with large weights 5.0e-5
-        # on average against 2.2e-5 walked; in a bfloat16 run the rounding of operands hides it.)
         o = ops.linear_recurrence(
             qkv, 0, self.qk, 2 * self.qk, batch, cache.states[self.state_name],
             heads=H, kv_heads=self.kv_heads, dim=self.dim, vdim=self.vdim,
             silu_inputs=False, gates=beta_g, per_channel=self.per_channel, delta=True,
-            walk=self.ctx.dtype == torch.float32)
+            walk=walks_portions(self.ctx))
         gated = ops.norm_gate(o, gate, gate_col, self.norm_w, groups=H,
                               gate="sigmoid" if self.per_channel else "silu", eps=self.eps,
                               out_dtype=self.ctx.dtype)
