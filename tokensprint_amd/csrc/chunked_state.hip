@@ -31,10 +31,12 @@
 // What bounds them: the float32 matrix rate (64 operations a cycle and SIMD) and, in chunk_walk,
 // the chain of two products and two meetings in LDS a chunk.  The kernels before these walked a
 // token at a time (the linear forms in chunks side by side, twice the arithmetic) and were bound
-// by the chain of a token's multiply-adds and sums.  At 2,048 tokens, before and now: delta rule,
-// 16 heads of 128 x 128, 592 and 112 us (solve 30, walk 52, output 33); 8 heads of 64 x 128 with
-// a decay per row 469 and 77; fixed decays, 16 heads of 128 x 128, 230 and 76 (local 26, carry
-// 16, output 40); state space, 64 heads of 128 x 64, 386 and 121 (38, 22, 60).
+// by the chain of a token's multiply-adds and sums.  At 2,048 tokens, before and now (alone; in
+// brackets the launches as they run in a prompt's step): delta rule, 16 heads of 128 x 128, 592 and
+// 126 us (solve 37, walk 60, output 37); 8 heads of 64 x 128 with a decay per row 469 and 81 (27,
+// 35, 24); fixed decays, 16 heads of 128 x 128, 230 and 78 (local 29, carry 22, output 44); state
+// space, 64 heads of 128 x 64, 386 and 123 (41, 31, 67).  The short chains of product_step and the
+// decays in 64 bits are 1 to 10 us of that.
 //
 // Matrix operands: lane (g, l) = (lane / 16, lane % 16) holds row l of A, column l of B, and rows
 // 4 g + r, column l of the sum.  The four steps of a 16-deep product take k = 4 g + r in step r
@@ -59,14 +61,31 @@ constexpr int kTiles = 10;                 // tiles on and below the diagonal of
 __device__ __forceinline__ float silu(float v) { return v / (1.0f + expf(-v)); }
 __device__ __forceinline__ float softplus(float v) { return v > 20.f ? v : log1pf(expf(v)); }
 
-__device__ __forceinline__ f32x4 mfma4(f32x4 a, f32x4 b, f32x4 c) {
-#pragma unroll
-  for (int r = 0; r < 4; ++r) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], c, 0, 0, 0);
-  return c;
+// One of the four steps of a product of 16 by itself, to be added to others: the even and the odd
+// steps are a chain of eight products each.  An element's error is mostly that of its chains and
+// of the decays that it is multiplied with: 600 tokens, outputs of the delta rule (128 rows) off by
+// 1.40e-7 of themselves, 1.58 in chains of sixteen with decays in 32 bits, 3.4 in one chain, 1.40
+// walked; a decay per row and 64 rows 1.33, 1.54, 2.6, 1.35; fixed decays (128) 1.03, 1.24 (1.06 in
+// chunks of multiply-adds); state space (128) 1.07, 1.22 (1.15).
+__device__ __forceinline__ void product_step(f32x4 (&chain)[2], f32x4 a, f32x4 b, int r) {
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  chain[r & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], r < 2 ? zero : chain[r & 1], 0, 0, 0);
 }
-// A product of 16 by itself, to be added to others: chains of 16, or an element's error is that of
-// one chain over all of them.
-__device__ __forceinline__ f32x4 product4(f32x4 a, f32x4 b) { return mfma4(a, b, f32x4{0.f, 0.f, 0.f, 0.f}); }
+__device__ __forceinline__ f32x4 product2(f32x4 a, f32x4 b) {
+  f32x4 chain[2];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) product_step(chain, a, b, r);
+  return chain[0] + chain[1];
+}
+// The same with every step a chain of its own, where few products are made or many results hang on
+// one: the products of keys and queries, the triangular systems.
+__device__ __forceinline__ f32x4 product4(f32x4 a, f32x4 b) {
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 step[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) step[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], zero, 0, 0, 0);
+  return (step[0] + step[1]) + (step[2] + step[3]);
+}
 __device__ __forceinline__ f32x4 read4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 __device__ __forceinline__ void write4(float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
 __device__ __forceinline__ int tri(int i, int j) { return i * (i + 1) / 2 + j; }
@@ -201,22 +220,27 @@ __device__ __forceinline__ void spread_decays(HeadDecays d, float dec, float vs,
   if (l == 15) d.total()[blk] = (float)p;
 }
 
-// M(t, s) for rows t = 4 g + r and column s = l of tile (i, j), j <= i; zero above the diagonal.
+// M(t, s) times vs(s) for rows t = 4 g + r and column s = l of tile (i, j), j <= i; zero above the
+// diagonal.  Multiplied up in 64 bits and rounded once.
 __device__ __forceinline__ f32x4 tile_decays(HeadDecays d, int i, int j, int l, int g) {
   f32x4 m;
+  const double vs = d.vs()[16 * j + l];
   if (i == j) {
     const float* gb = d.g() + 16 * i;
-    float run = 1.f;
+    double run = 1.;
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
-      run = u > l ? run * gb[u] : 1.f;
-      if (u / 4 == g) m[u % 4] = u >= l ? run : 0.f;
+      run = u > l ? run * gb[u] : 1.;
+      if (u / 4 == g) m[u % 4] = u >= l ? (float)(run * vs) : 0.f;
     }
     return m;
   }
-  float col = d.suf()[16 * j + l];
+  double col = d.suf()[16 * j + l] * vs;
   for (int b = j + 1; b < i; ++b) col *= d.total()[b];
-  return read4(d.pre() + 16 * i + 4 * g) * col;
+  const f32x4 row = read4(d.pre() + 16 * i + 4 * g);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) m[r] = (float)(row[r] * col);
+  return m;
 }
 
 // One 16 x 16 tile of rows a . rows b over NP columns, both in LDS.
@@ -224,9 +248,11 @@ template <int NT>
 __device__ __forceinline__ f32x4 gram_tile(const float* a, const float* b, int l, int g) {
   constexpr int LD = 16 * NT + 4;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int j = 0; j < NT; ++j)
-    acc += product4(read4(a + l * LD + 16 * j + 4 * g), read4(b + l * LD + 16 * j + 4 * g));
+  auto part = [&](int j) {
+    return product4(read4(a + l * LD + 16 * j + 4 * g), read4(b + l * LD + 16 * j + 4 * g));
+  };
+#pragma unroll 2
+  for (int j = 0; j < NT; j += 2) acc += part(j) + part(j + 1);
   return acc;
 }
 
@@ -322,17 +348,17 @@ __device__ __forceinline__ void split_decays(float* pre, const float* post, floa
       g[t] = gr[(16 * blk + t) * LD + n];
       k[t] = post[(16 * blk + t) * LD + n];
     }
-    float m = 1.f;
+    double m = 1.;                         // (rounded where it is used, not at every step)
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
       m *= g[t];
-      pre[(16 * blk + t) * LD + n] *= m;
+      pre[(16 * blk + t) * LD + n] = (float)(pre[(16 * blk + t) * LD + n] * m);
     }
-    blocks[i] = m;
-    m = 1.f;
+    blocks[i] = (float)m;
+    m = 1.;
 #pragma unroll
     for (int t = 15; t >= 0; --t) {
-      gr[(16 * blk + t) * LD + n] = k[t] * m;
+      gr[(16 * blk + t) * LD + n] = (float)(k[t] * m);
       m *= g[t];
     }
   }
@@ -345,13 +371,14 @@ __device__ __forceinline__ f32x4 split_tile(const float* pre, const float* post,
                                             int i, int j, int l, int g) {
   constexpr int NP = 16 * NT, LD = NP + 4;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int c = 0; c < NT; ++c) {
+  auto part = [&](int c) {
     const int n = 16 * c + 4 * g;
     f32x4 b = read4(post + (16 * j + l) * LD + n);
     for (int m = j + 1; m < i; ++m) b *= read4(blocks + m * NP + n);
-    acc += product4(read4(pre + (16 * i + l) * LD + n), b);
-  }
+    return product4(read4(pre + (16 * i + l) * LD + n), b);
+  };
+#pragma unroll 2
+  for (int c = 0; c < NT; c += 2) acc += part(c) + part(c + 1);
   return acc;
 }
 
@@ -445,9 +472,8 @@ __global__ __launch_bounds__(kThreads, 2) void chunk_local_kernel(ChunkedArgs a,
 #pragma unroll
         for (int o = 0; o < OWN; ++o) {
           if (w + 4 * o >= NT) break;
-          f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int j = 0; j < 4; ++j) acc += product4(kf[o][j], vf[j]);
+          const f32x4 early = product2(kf[o][0], vf[0]) + product2(kf[o][1], vf[1]);
+          const f32x4 acc = early + (product2(kf[o][2], vf[2]) + product2(kf[o][3], vf[3]));
           write4(share + ((int64_t)(c0 / 16 + ct) * NT + w + 4 * o) * 256 + lane * 4, acc);
         }
       }
@@ -721,21 +747,22 @@ __global__ __launch_bounds__(kThreads, 1) void chunk_walk_kernel(ChunkedArgs a) 
     for (int o = 0; o < OWN; ++o)
       if (owns(o)) write4(&s_lds[w + 4 * o][lane * 4], S[o]);
     __syncthreads();
-    f32x4 mine = f.y, part[2], s[NT];
+    f32x4 mine = f.y, part[2][2], s[NT];
 #pragma unroll
     for (int j = 0; j < NT; ++j) s[j] = read4(&s_lds[j][lane * 4]);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-      part[j & 1] = product4(f.w[j], s[j]);
-      if (j > 0) mine += part[(j - 1) & 1];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) product_step(part[j & 1], f.w[j], s[j], r);
+      if (j > 0) mine += part[(j - 1) & 1][0] + part[(j - 1) & 1][1];
       fetch_w(ahead, later, j);
       __builtin_amdgcn_sched_barrier(0);
     }
-    mine += part[(NT - 1) & 1];
+    mine += part[(NT - 1) & 1][0] + part[(NT - 1) & 1][1];
     write4(&u_lds[w][lane * 4], mine);
     __syncthreads();
-    f32x4 u[4], more[2][OWN];
+    f32x4 u[4], more[2][OWN][2];
 #pragma unroll
     for (int i = 0; i < 4; ++i) u[i] = read4(&u_lds[i][lane * 4]);
     write4(a.scratch + parts.u + ((unit * PT + ct) * 4 + w) * 256 + lane * 4, mine);
@@ -751,16 +778,15 @@ __global__ __launch_bounds__(kThreads, 1) void chunk_walk_kernel(ChunkedArgs a) 
       for (int r = 0; r < 4; ++r)
 #pragma unroll
         for (int o = 0; o < OWN; ++o)
-          more[i & 1][o] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.kt[o][i][r], u[i][r],
-                                                                r ? more[i & 1][o] : zero, 0, 0, 0);
+          product_step(more[i & 1][o], f.kt[o][i], u[i], r);
 #pragma unroll
       for (int o = 0; o < OWN; ++o)
-        if (i > 0) S[o] += more[(i - 1) & 1][o];
+        if (i > 0) S[o] += more[(i - 1) & 1][o][0] + more[(i - 1) & 1][o][1];
       fetch_kt(ahead, later, i);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int o = 0; o < OWN; ++o) S[o] += more[1][o];
+    for (int o = 0; o < OWN; ++o) S[o] += more[1][o][0] + more[1][o][1];
   };
   WalkOperands<NT> ring[4];
 #pragma unroll
@@ -884,7 +910,7 @@ __device__ __forceinline__ void output_chunk(const ChunkedArgs& a, const ChunkRa
             v[j][r] = t < nt && p < a.P ? col[(int64_t)t * a.ld] : 0.f;
           }
       }
-      f32x4 acc[RT], part[2][RT], q[2][RT];
+      f32x4 acc[RT], part[2][RT][2], q[2][RT];
       auto fetch = [&](int j) {
 #pragma unroll
         for (int i = 0; i < RT; ++i) {
@@ -903,14 +929,13 @@ __device__ __forceinline__ void output_chunk(const ChunkedArgs& a, const ChunkRa
         for (int r = 0; r < 4; ++r)
 #pragma unroll
           for (int i = 0; i < RT; ++i)
-            part[j & 1][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[j & 1][i][r], s0[j][r],
-                                                                  r ? part[j & 1][i] : zero, 0, 0, 0);
+            product_step(part[j & 1][i], q[j & 1][i], s0[j], r);
         // (the sixteen before are added meanwhile; put off to the end by the compiler otherwise, which
         // then has no registers left)
         if (j > 0) {
 #pragma unroll
           for (int i = 0; i < RT; ++i) {
-            acc[i] += part[(j - 1) & 1][i];
+            acc[i] += part[(j - 1) & 1][i][0] + part[(j - 1) & 1][i][1];
             asm volatile("" : "+v"(acc[i]));
           }
         }
@@ -918,12 +943,12 @@ __device__ __forceinline__ void output_chunk(const ChunkedArgs& a, const ChunkRa
 #pragma unroll
         for (int m = 3; m < 4 * RT; ++m) {
           __builtin_amdgcn_sched_group_barrier(8, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(2, 2, 0);
+          __builtin_amdgcn_sched_group_barrier(2, 3, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
-      for (int i = 0; i < RT; ++i) acc[i] += part[(NT - 1) & 1][i];
+      for (int i = 0; i < RT; ++i) acc[i] += part[(NT - 1) & 1][i][0] + part[(NT - 1) & 1][i][1];
       if (FORM == kSilu) {
 #pragma unroll
         for (int j = 0; j < RT; ++j)
@@ -934,11 +959,13 @@ __device__ __forceinline__ void output_chunk(const ChunkedArgs& a, const ChunkRa
 #pragma unroll
       for (int i = 0; i < RT; ++i) {
         if (!ROW) acc[i] *= read4(d.d0() + 16 * i + 4 * g);
+        f32x4 pair = zero;
 #pragma unroll
         for (int j = 0; j <= i; ++j) {
-          const f32x4 u = DELTA ? v[j] : v[j] * read4(d.vs() + 16 * j + 4 * g);
-          acc[i] += i == j ? causal_product(tiles + tri(i, i) * kTile, u, l, g)
-                           : product4(read4(tiles + tri(i, j) * kTile + l * kTileLd + 4 * g), u);
+          const f32x4 p = i == j ? causal_product(tiles + tri(i, i) * kTile, v[j], l, g)
+                                 : product2(read4(tiles + tri(i, j) * kTile + l * kTileLd + 4 * g), v[j]);
+          pair = j & 1 ? pair + p : p;
+          if (j & 1 || j == i) acc[i] += pair;
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
