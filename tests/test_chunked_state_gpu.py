@@ -372,3 +372,22 @@ def test_walked_portions_do_not_depend_on_the_cut(gpu_device, per_channel):
     whole = run([T])
     for portions in ([70, 13, 127], [8, 9, 64, 129]):
         assert torch.equal(run(portions), whole), portions
+
+
+@pytest.mark.parametrize("tokens, walked", [(128, True), (160, True), (161, False)])
+def test_delta_rule_walks_portions_that_its_chunks_are_slower_for(gpu_device, tokens, walked):
+    ops, gen = load_hip_ops(gpu_device), torch.Generator().manual_seed(14)
+    heads, dim, vdim = 2, 64, 32
+    x = torch.randn(tokens, heads * (2 * dim + vdim), generator=gen).to(gpu_device)
+    x[:, heads * dim:2 * heads * dim] *= dim ** -0.5
+    gates = torch.rand(tokens, 2 * heads, generator=gen).to(gpu_device)
+    outs = []
+    for walk in (False, True):
+        requests = Requests(gpu_device, (heads, dim, vdim), 1)
+        batch = requests.step([tokens])
+        outs.append(ops.linear_recurrence(
+            x, 0, heads * dim, 2 * heads * dim, batch, requests.state, heads=heads, kv_heads=heads,
+            dim=dim, vdim=vdim, silu_inputs=False, delta=True, gates=gates, walk=walk))
+        assert ("scan_chunks" in batch.plans) == (not walk and not walked)
+    assert torch.equal(*outs) == walked
+    torch.testing.assert_close(*outs, rtol=1e-4, atol=1e-4)

@@ -80,11 +80,14 @@ class Dispatch:
 
     # ---- recurrences.  A step whose longest portion has more tokens than this runs in chunks of
     # 64 tokens as products of matrices, below it every entry is walked whole by one launch.
-    # Three launches have a length of their own (25 to 45 us to the first 64 tokens), a walked
-    # token costs 0.28 us (delta rule, 16 heads of 128 x 128: 128 tokens 44 walked, 47 in chunks;
-    # 512 tokens 155 / 63), 0.23 (8 heads of 64 x 128, a decay per row: 35 / 38 and 123 / 44),
-    # 0.25 (fixed decays, 16 heads of 128 x 128: 38 / 40 and 132 / 44).
+    # Three launches have a length of their own, a walked token costs 0.24 to 0.28 us (16 heads
+    # of 128 x 128, a decay per head: 128 tokens 38 us walked, 40 in chunks; 144 tokens 42 / 41;
+    # 512 tokens 130 / 45).
     scan_whole_tokens: int = 128
+    #: so many more for the delta rule, whose launches take longer: 16 heads of 128 x 128, 128
+    #: tokens 43 us walked, 52 in chunks; 160 tokens 53 / 54; 192 tokens 62 / 54; 512 tokens
+    #: 153 / 69.  8 heads of 64 x 128, a decay per row: 35 / 39, 42 / 40, 49 / 41, 121 / 46.
+    delta_whole_more: int = 32
     #: the state-space scan, whose workgroup walks 64 columns: 1.5 us a token at 64 heads of
     #: 128 x 64 (64 tokens 98 us walked, 34 in chunks), 1.1 at 32 heads of 64 x 64 (70 / 25).
     #: The line lies higher than that says because a step that short is eager and as long as

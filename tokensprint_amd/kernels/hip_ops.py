@@ -1401,7 +1401,8 @@ class HipOps:
         # they stand: with their SiLU taken on the way it is walked)
         chunks, entry_chunks, num_chunks = None, None, 0
         if dim <= (128 if delta else 256) and not walk and not (delta and silu_inputs):
-            chunks, entry_chunks, num_chunks = self._scan_chunks(batch)
+            whole = self.dispatch.scan_whole_tokens + delta * self.dispatch.delta_whole_more
+            chunks, entry_chunks, num_chunks = self._scan_chunks(batch, whole)
         scratch = self._chunk_scratch(num_chunks, heads, dim, vdim, delta)
         self._call(self.lib.ts_linear_recurrence, _ptr(x), ld, int(q_col), int(k_col), int(v_col),
                    _ptr(decay), _ptr(gates), ldg, _ptr(state), _ptr(out), pos, eot, qs, slots, T,
