@@ -88,12 +88,15 @@ class Dispatch:
     #: tokens 43 us walked, 52 in chunks; 160 tokens 53 / 54; 192 tokens 62 / 54; 512 tokens
     #: 153 / 69.  8 heads of 64 x 128, a decay per row: 35 / 39, 42 / 40, 49 / 41, 121 / 46.
     delta_whole_more: int = 32
-    #: the state-space scan, whose workgroup walks 64 columns: 1.5 us a token at 64 heads of
-    #: 128 x 64 (64 tokens 98 us walked, 34 in chunks), 1.1 at 32 heads of 64 x 64 (70 / 25).
-    #: The line lies higher than that says because a step that short is eager and as long as
-    #: its launches: two more a layer cost it more on the host than the walk does on the GPU
-    #: (45 tokens beside 11 single ones, six such layers of the smaller size: 1.31 ms walked,
-    #: 1.41 in chunks)
+    #: the state-space scan, whose workgroup walks 64 columns: 1.45 us a token at 64 heads of
+    #: 128 x 64 (64 tokens 96 us walked, 33 in chunks), 1.05 at 32 heads of 64 x 64 (68 / 23).
+    #: The line lies higher than that says because a step that short is eager and mostly as long
+    #: as its launches: two more a layer cost it more on the host than the walk does on the GPU.
+    #: Steps of one portion, six such layers, walked and in chunks: the smaller size 45 tokens
+    #: 1.12 / 1.21 ms, 64 tokens 1.12 / 1.21, 96 tokens 1.34 / 1.44; the larger 45 tokens
+    #: 1.30 / 1.39, 64 tokens 1.48 / 1.39, 96 tokens 1.77 / 1.44 (beside 11 single tokens, 64:
+    #: 1.55 / 1.61).  One line for both sizes: what is lost at the larger, up to a third of a
+    #: millisecond at 96, is won back at smaller ones, which would rather have it higher.
     state_space_whole_tokens: int = 96
 
     # ---- latent attention on the matrix cores: a wavefront per tile of 16 (token, head)
