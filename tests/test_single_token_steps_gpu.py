@@ -1,0 +1,123 @@
+"""Kernels of steps in which every entry brings one token against the ones that take entries of
+any length, at the edges of their sizes.  They add the same sums in the same order, so outputs
+and the states that are left are equal to the bit (operands that do not begin on 16 bytes go to
+the general kernels)."""
+
+import pytest
+import torch
+
+from tokensprint_amd.cache import CacheManager, CacheStorage
+from tokensprint_amd.engine.batch import BatchBuilder, StepEntry
+from tokensprint_amd.kernels import load_hip_ops
+from tokensprint_amd.parts.base import SlotStateNeed
+
+pytestmark = pytest.mark.gpu
+
+
+def rand(shape, seed, scale=1.0):
+    return (torch.randn(shape, generator=torch.Generator().manual_seed(seed)) * scale).cuda()
+
+
+def steps(device, entries, count):
+    """`count` steps of one token an entry; slots do not start at 0."""
+    storage = CacheStorage([SlotStateNeed((1,), torch.float32, "s")], 16, 8, entries + 2,
+                           torch.float32, device)
+    manager = CacheManager(storage.groups, 16, 8, entries + 2)
+    manager.admit("in front")
+    caches = [manager.admit(i) for i in range(entries)]
+    builder = BatchBuilder(device, len(storage.groups))
+    for _ in range(count):
+        out = []
+        for rc in caches:
+            manager.extend(rc, rc.num_tokens + 1)
+            out.append(StepEntry(rc, [1], rc.num_tokens - 1, [0]))
+        yield builder.build(out)
+
+
+def off_by_one(t):
+    """A copy of t that begins 4 bytes behind a 16-byte boundary."""
+    buf = torch.empty(t.numel() + 4, dtype=t.dtype, device=t.device)
+    view = buf[1:1 + t.numel()].view(t.shape)
+    view.copy_(t)
+    return view
+
+
+def stale(entries, shape):
+    """What others left in the slots: not numbers, which a new sequence must not see."""
+    return torch.full((entries + 2, *shape), float("nan"), device="cuda")
+
+
+@pytest.mark.parametrize("form", ["fixed", "silu", "turn", "per_head", "delta", "per_row"])
+@pytest.mark.parametrize("heads, kv_heads, N, P, entries", [
+    (2, 1, 16, 4, 1), (4, 2, 32, 60, 3), (2, 2, 64, 64, 2), (3, 1, 64, 68, 5), (4, 2, 128, 128, 2),
+    (2, 1, 128, 132, 1), (2, 2, 24, 64, 2)])
+def test_recurrence(gpu_device, form, heads, kv_heads, N, P, entries):
+    ops = load_hip_ops(gpu_device)
+    if form in ("fixed", "silu", "turn"):
+        kv_heads = heads
+    qk = kv_heads * N
+    kw = dict(heads=heads, kv_heads=kv_heads, dim=N, vdim=P, silu_inputs=form == "silu")
+    if form in ("fixed", "silu", "turn"):
+        kw["decay"] = torch.rand(heads, generator=torch.Generator().manual_seed(1)).cuda()
+    if form == "turn":
+        kw.update(turn=rand((8, N // 2 - 2, 2), 2), k_scale=0.3)
+    one, other = stale(entries, (heads, N, P)), stale(entries, (heads, N, P))
+    other = off_by_one(other)
+    for i, batch in enumerate(steps(gpu_device, entries, 3)):
+        x = rand((entries, 4 + 2 * qk + heads * P), 10 + i, 0.5)
+        if form in ("per_head", "delta", "per_row"):
+            n = heads * N if form == "per_row" else heads
+            kw.update(gates=torch.sigmoid(rand((entries, heads + n), 20 + i)),
+                      delta=form != "per_head", per_channel=form == "per_row")
+        got = ops.linear_recurrence(x, 4, 4 + qk, 4 + 2 * qk, batch, one, **kw)
+        want = ops.linear_recurrence(x, 4, 4 + qk, 4 + 2 * qk, batch, other, **kw)
+        assert not got.isnan().any()
+        assert torch.equal(got, want) and torch.equal(one[1:-1], other[1:-1])
+
+
+@pytest.mark.parametrize("heads, groups, N, P, entries", [
+    (2, 1, 16, 4, 1), (4, 2, 32, 60, 3), (4, 4, 64, 64, 2), (8, 2, 128, 64, 5), (2, 1, 128, 68, 2),
+    (2, 1, 24, 64, 2)])
+def test_state_space(gpu_device, heads, groups, N, P, entries):
+    ops = load_hip_ops(gpu_device)
+    args = [rand((heads,), 1), rand((heads,), 2), rand((heads,), 3)]
+    kw = dict(heads=heads, vdim=P, state_rows=N, groups=groups)
+    one = stale(entries, (heads, N, P))
+    other = off_by_one(one)
+    for i, batch in enumerate(steps(gpu_device, entries, 3)):
+        xbc = rand((entries, heads * P + 2 * groups * N), 10 + i)
+        proj = rand((entries, 3 + heads), 20 + i)
+        got = ops.ssm_scan(xbc, proj, 3, *args, batch, one, **kw)
+        want = ops.ssm_scan(xbc, proj, 3, *args, batch, other, **kw)
+        assert not got.isnan().any()
+        assert torch.equal(got, want) and torch.equal(one[1:-1], other[1:-1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("per_channel", [False, True])
+@pytest.mark.parametrize("heads, kv_heads, N, P, entries", [
+    (2, 1, 16, 64, 1), (4, 2, 32, 128, 3), (2, 2, 64, 64, 2), (6, 2, 128, 128, 5)])
+def test_delta_rule_whole(gpu_device, heads, kv_heads, N, P, entries, per_channel, dtype):
+    """From the convolved rows to the gated ones against the three kernels one after the other."""
+    ops = load_hip_ops(gpu_device)
+    qk, inner, n = kv_heads * N, heads * P, heads * N if per_channel else heads
+    a_log, dt_bias, w = rand((heads,), 1), rand((n,), 2), 1 + 0.1 * rand((P,), 3)
+    one, other = stale(entries, (heads, N, P)), stale(entries, (heads, N, P))
+    sizes = dict(heads=heads, kv_heads=kv_heads, dim=N)
+    out = dict(gate="sigmoid" if per_channel else "silu", eps=1e-6, out_dtype=dtype)
+    for i, batch in enumerate(steps(gpu_device, entries, 3)):
+        qkv, proj = rand((entries, 2 * qk + inner), 10 + i), rand((entries, 5 + heads), 20 + i)
+        z, gate = rand((entries, 3 + n), 30 + i), rand((entries, 8 + inner), 40 + i)
+        kept = qkv.clone()
+        got = ops.delta_step(qkv, proj, 5, z, 3, a_log, dt_bias, gate, 8, w, batch, one,
+                             per_channel=per_channel, vdim=P, **sizes, **out)
+        assert torch.equal(qkv, kept)
+        gates = ops.delta_gates(qkv, proj, 5, z, 3, a_log, dt_bias, per_channel=per_channel, **sizes)
+        o = ops.linear_recurrence(qkv, 0, qk, 2 * qk, batch, other, vdim=P, silu_inputs=False,
+                                  gates=gates, per_channel=per_channel, delta=True, **sizes)
+        want = ops.norm_gate(o, gate, 8, w, groups=heads, **out)
+        assert not got.isnan().any()
+        assert torch.equal(got, want) and torch.equal(one[1:-1], other[1:-1])
+        # rows that the kernel does not take are left to the others
+        assert ops.delta_step(qkv, proj, 5, z, 3, a_log, dt_bias, gate, 7, w, batch, one,
+                              per_channel=per_channel, vdim=P, **sizes, **out) is None

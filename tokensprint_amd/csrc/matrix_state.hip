@@ -16,6 +16,7 @@
 // written once a portion, by the thread that owns the element.
 #include "chunked_state.h"
 #include "gated_norm.h"
+#include "recurrence_step.h"
 #include <algorithm>
 
 __device__ __forceinline__ float sigmoid_f(float v) { return 1.0f / (1.0f + expf(-v)); }
@@ -352,6 +353,19 @@ extern "C" int ts_linear_recurrence(const float* x, int ld, int q_col, int k_col
     c.chunks = chunks, c.entry_chunks = entry_chunks;
     c.num_chunks = num_chunks, c.num_entries = num_entries, c.scratch = scratch;
     return launch_chunked(c, stream);
+  }
+  if (max_q_len == 1 && num_tokens == num_entries) {       // a token an entry
+    RecurrenceStepArgs one{};
+    one.x = x, one.decay = decay, one.gates = gates, one.state = state, one.out = out;
+    one.positions = positions, one.slot_ids = slot_ids;
+    one.ld = ld, one.q_col = q_col, one.k_col = k_col, one.v_col = v_col, one.ldg = ldg;
+    one.heads = heads, one.kv_heads = kv_heads, one.N = N, one.P = P, one.silu = silu;
+    one.turn = a.turn, one.turn_dims = turn_dims, one.k_scale = k_scale;
+    if (recurrence_step_fits(one)) {
+      launch_recurrence_step(one, num_entries, delta, per_row, stream);
+      TS_CHECK_LAUNCH("linear_recurrence (one token)");
+      return 0;
+    }
   }
   const int ni = (N + 7) / 8;
   const int64_t wide_groups = (int64_t)heads * num_entries * ((P + 63) / 64);

@@ -7,6 +7,7 @@
 // written once a portion, by the thread that owns the element.
 #include "chunked_state.h"
 #include "gated_norm.h"
+#include "recurrence_step.h"
 
 __device__ __forceinline__ float silu_f(float v) { return v / (1.0f + expf(-v)); }
 __device__ __forceinline__ float softplus_f(float v) { return v > 20.f ? v : log1pf(expf(v)); }
@@ -434,7 +435,8 @@ extern "C" int ts_ssm_scan(const float* xbc, const float* proj, int ld, int dt_c
                            const float* dt_bias, const float* a_log, const float* d_skip,
                            float* state, float* y, const int* positions,
                            const int* entry_of_token, const int* q_start, const int* slot_ids,
-                           int num_tokens, int num_entries, int heads, int P, int N, int groups,
+                           int num_tokens, int num_entries, int max_q_len, int heads, int P,
+                           int N, int groups,
                            const int* chunks, const int* entry_chunks, int num_chunks,
                            float* scratch, hipStream_t stream) {
   if (num_tokens <= 0) return 0;
@@ -454,6 +456,13 @@ extern "C" int ts_ssm_scan(const float* xbc, const float* proj, int ld, int dt_c
     c.k_scale = 1.f, c.chunks = chunks, c.entry_chunks = entry_chunks;
     c.num_chunks = num_chunks, c.num_entries = num_entries, c.scratch = scratch;
     return launch_chunked(c, stream);
+  }
+  const ScanStepArgs one{xbc, proj + dt_col, dt_bias, a_log, d_skip, state, y, positions, slot_ids,
+                         ld, heads, P, N, groups};
+  if (max_q_len == 1 && num_tokens == num_entries && scan_step_fits(one)) {       // a token an entry
+    launch_scan_step(one, num_entries, stream);
+    TS_CHECK_LAUNCH("ssm_scan (one token)");
+    return 0;
   }
   ScanArgs a{xbc, proj, dt_bias, a_log, d_skip, state, y, b, ld, dt_col, channels, heads, P, N, groups};
   const int ni = (N + kScanSlices - 1) / kScanSlices;

@@ -1081,6 +1081,11 @@ class HipOps:
         return (_ptr(batch.positions), _ptr(batch.entry_of_token), _ptr(batch.q_start),
                 _ptr(batch.slot_ids))
 
+    @staticmethod
+    def _single_tokens(batch):
+        """Whether every entry of the step brings one token (row t is then entry t's)."""
+        return batch.max_q_len == 1 and batch.num_tokens == batch.num_entries
+
     def _check_state(self, name, state, shape, dtype=torch.float32):
         self._check(name, state, dtype, ndim=len(shape) + 1)
         if tuple(state.shape[1:]) != tuple(shape):
@@ -1295,8 +1300,8 @@ class HipOps:
         scratch = self._chunk_scratch(num_chunks, heads, N, vdim)
         self._call(self.lib.ts_ssm_scan, _ptr(xbc), _ptr(proj), proj.shape[1], dt_col,
                    _ptr(dt_bias), _ptr(a_log), _ptr(d_skip), _ptr(state), _ptr(y), pos, eot, qs,
-                   slots, T, batch.num_entries, heads, vdim, N, groups, _ptr(chunks),
-                   _ptr(entry_chunks), num_chunks, _ptr(scratch), self._stream())
+                   slots, T, batch.num_entries, int(batch.max_q_len), heads, vdim, N, groups,
+                   _ptr(chunks), _ptr(entry_chunks), num_chunks, _ptr(scratch), self._stream())
         return y
 
     def _chunk_scratch(self, num_chunks, heads, rows, cols, delta=False):
@@ -1363,6 +1368,39 @@ class HipOps:
                    _ptr(gates), heads + n, T, heads, kv_heads, dim, int(bool(per_channel)),
                    self._stream())
         return gates
+
+    def delta_step(self, qkv, proj, beta_col, z, z_col, a_log, dt_bias, gate_rows, gate_col, norm_w,
+                   batch, state, *, heads, kv_heads, dim, vdim, per_channel, gate, eps, out_dtype):
+        """`delta_gates`, `linear_recurrence` with the delta rule and `norm_gate` over the heads
+        (a weight they share) in one kernel, for steps in which every entry brings one token
+        and sizes that are built; else None, and nothing has been done.  `qkv` stays as it is."""
+        T = qkv.shape[0]
+        if not (self._single_tokens(batch) and self.lib.ts_delta_step_fits(dim, vdim) == 1
+                and qkv.shape[1] % 4 == 0 and gate_rows.shape[1] % 4 == 0 and gate_col % 4 == 0
+                and norm_w is not None and norm_w.shape == (vdim,)
+                and not any(t.data_ptr() % 16 for t in (qkv, gate_rows, norm_w, state))):
+            return None
+        self._check("qkv", qkv, torch.float32, ndim=2)
+        for name, rows in (("proj", proj), ("z", z), ("gate rows", gate_rows)):
+            self._check(name, rows, torch.float32, ndim=2)
+            if rows.shape[0] != T:
+                raise ValueError("delta_step: row counts differ")
+        self._check("A_log", a_log, torch.float32, shape=(heads,))
+        self._check("dt_bias", dt_bias, torch.float32,
+                    shape=(heads * dim if per_channel else heads,))
+        self._check("norm weight", norm_w, torch.float32)
+        if gate not in ("sigmoid", "silu"):
+            raise ValueError(f"delta_step: gate {gate!r}; built are sigmoid and silu")
+        self._check_state("recurrent state", state, (heads, dim, vdim))
+        pos, _, _, slots = self._batch_ptrs(batch, T)
+        out = torch.empty(T, heads * vdim, dtype=out_dtype, device=self.device)
+        self._call(self.lib.ts_delta_step, _ptr(qkv), qkv.shape[1], _ptr(proj), proj.shape[1],
+                   int(beta_col), _ptr(z), z.shape[1], int(z_col), _ptr(a_log), _ptr(dt_bias),
+                   _ptr(gate_rows), gate_rows.shape[1], int(gate_col), _ptr(norm_w),
+                   0 if gate == "sigmoid" else 1, c_float(eps), _ptr(state), _ptr(out),
+                   _TYPE_CODE[out_dtype], pos, slots, T, heads, kv_heads, dim, vdim,
+                   int(bool(per_channel)), self._stream())
+        return out
 
     def linear_recurrence(self, x, q_col, k_col, v_col, batch, state, *, heads, kv_heads, dim,
                           vdim, silu_inputs, decay=None, gates=None, per_channel=False,

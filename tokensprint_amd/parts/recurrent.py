@@ -234,7 +234,7 @@ class GatedDeltaRule(Mixer):
             raise RuntimeError(f"{self.prefix}: a recurrence cannot read another run's state")
         ops, H = self.ops, self.heads
         proj = ops.linear(h, self.w_in, torch.float32)
-        b_col = self.channels
+        b_col, state = self.channels, cache.states[self.state_name]
         qkv = ops.conv_silu(proj, 0, self.channels, self.conv_w, None, batch,
                             cache.states[self.state_name + ".conv"])
         if self.per_channel:
@@ -248,17 +248,25 @@ class GatedDeltaRule(Mixer):
         else:
             z, z_col = proj, b_col + H
             gate, gate_col = proj, b_col + 2 * H
+        gate_kind = "sigmoid" if self.per_channel else "silu"
+        if hasattr(ops, "delta_step"):       # steps of single tokens: the rest in one kernel
+            gated = ops.delta_step(qkv, proj, b_col, z, z_col, self.a_log, self.dt_bias, gate,
+                                   gate_col, self.norm_w, batch, state, heads=H,
+                                   kv_heads=self.kv_heads, dim=self.dim, vdim=self.vdim,
+                                   per_channel=self.per_channel, gate=gate_kind, eps=self.eps,
+                                   out_dtype=self.ctx.dtype)
+            if gated is not None:
+                return ops.linear(gated, self.w_o, torch.float32)
         beta_g = ops.delta_gates(qkv, proj, b_col, z, z_col, self.a_log, self.dt_bias,
                                  heads=H, kv_heads=self.kv_heads, dim=self.dim,
                                  per_channel=self.per_channel)
         o = ops.linear_recurrence(
-            qkv, 0, self.qk, 2 * self.qk, batch, cache.states[self.state_name],
+            qkv, 0, self.qk, 2 * self.qk, batch, state,
             heads=H, kv_heads=self.kv_heads, dim=self.dim, vdim=self.vdim,
             silu_inputs=False, gates=beta_g, per_channel=self.per_channel, delta=True,
             walk=walks_portions(self.ctx))
-        gated = ops.norm_gate(o, gate, gate_col, self.norm_w, groups=H,
-                              gate="sigmoid" if self.per_channel else "silu", eps=self.eps,
-                              out_dtype=self.ctx.dtype)
+        gated = ops.norm_gate(o, gate, gate_col, self.norm_w, groups=H, gate=gate_kind,
+                              eps=self.eps, out_dtype=self.ctx.dtype)
         return ops.linear(gated, self.w_o, torch.float32)
 
 
