@@ -121,3 +121,26 @@ def test_delta_rule_whole(gpu_device, heads, kv_heads, N, P, entries, per_channe
         # rows that the kernel does not take are left to the others
         assert ops.delta_step(qkv, proj, 5, z, 3, a_log, dt_bias, gate, 7, w, batch, one,
                               per_channel=per_channel, vdim=P, **sizes, **out) is None
+
+
+@pytest.mark.parametrize("bias, in_bias, plain", [(True, False, False), (False, True, True),
+                                                  (False, False, False)])
+@pytest.mark.parametrize("entries", [1, 4, 5, 8, 9, 16, 17])
+@pytest.mark.parametrize("N, K, col, channels", [(3088, 512, 4, 3084), (1100, 1096, 20, 64),
+                                                 (2500, 2048, 0, 2500), (1040, 2056, 1036, 4)])
+def test_product_and_convolution(gpu_device, N, K, col, channels, entries, bias, in_bias, plain):
+    ops = load_hip_ops(gpu_device)
+    weight = (rand((N, K), 1) * K ** -0.5).bfloat16()
+    conv_w = rand((channels, 4), 2)
+    b = rand((channels,), 3) if bias else None
+    ib = rand((channels,), 4) if in_bias else None
+    one, other = stale(entries, (3, channels)), stale(entries, (3, channels))
+    for i, batch in enumerate(steps(gpu_device, entries, 5)):
+        x = rand((entries, K), 10 + i).bfloat16()
+        proj, got = ops.linear_conv_silu(x, weight, col, channels, conv_w, b, batch, one,
+                                         in_bias=ib, plain=plain)
+        rows = ops.linear(x, weight, torch.float32)
+        want = ops.conv_silu(rows, col, channels, conv_w, b, batch, other, in_bias=ib, plain=plain)
+        assert not got.isnan().any()
+        assert torch.equal(proj, rows) and torch.equal(got, want)
+        assert torch.equal(one[1:-1], other[1:-1])

@@ -64,11 +64,23 @@ struct DirectArgs {
   const int* merge_pos;     // [M]: position of each row's token
   int merge_splits, merge_nkv, merge_group, merge_hd, merge_window, merge_chunk;
   float limit;              // pair: gated_unit's limit (0: silu, below: gelu)
+  // convolved form (conv_out set; at most 16 rows, each the only token of its entry): columns
+  // [conv_col, conv_col + conv_channels) of the product pass a causal convolution of four taps a
+  // channel (bias, SiLU unless conv_plain) on their way out, as ts_conv_silu takes it
+  const float* conv_w;      // [channels, 4]
+  const float* conv_b;      // [channels] or null
+  const float* conv_in_b;   // [channels] or null
+  float* conv_state;        // [slots, 3, channels]
+  float* conv_out;          // [M, channels]
+  const int *conv_pos, *conv_slots;     // [M]
+  int conv_col, conv_channels, conv_plain;
 };
 
 // Launches it; `norm` (the fused form) takes at most 16 rows.  Returns 0 or -1 with the
 // error text set.
 int gemm_direct_launch(const DirectArgs& a, int c_type, bool pair, bool norm, hipStream_t stream);
+// Whether the convolved form takes a product of this shape.
+bool gemm_direct_conv_fits(int M, int N, int K, int col, int channels, int taps);
 // Whether the tail and the scaled form take a product of this shape (up to 64 rows).
 bool gemm_direct_tail_fits(int M, int N, int K);
 int gemm_direct_tail_parts(int M, int N);      // slices the tail form leaves per row

@@ -29,10 +29,11 @@ __device__ __forceinline__ bf16x8 row_down_by(bf16x8 v, int n) {
 }
 
 template <int MT, int WK, typename TC, bool PAIR, bool NORM, int S, int PD, bool SCALED = false,
-          bool TAIL = false, int CW = 16, int AR = 16, bool MERGE = false>
+          bool TAIL = false, int CW = 16, int AR = 16, bool MERGE = false, bool CONV = false>
 __global__ __launch_bounds__(WK* kWave) void gemm_direct_kernel(DirectArgs a) {
   static_assert(!NORM || MT == 1, "the fused form holds one tile of rows");
   static_assert(!MERGE || (TAIL && MT == 1), "the merged form: a tail product of one tile of rows");
+  static_assert(!CONV || (MT == 1 && !PAIR && !NORM && !SCALED && !TAIL), "the convolved form is a plain product");
   // Packed operands.  A compute unit takes a wave's 16-byte load in about 28 cycles
   // whatever its lanes ask for, and that rate, not the bytes, bounds these products.  An
   // operand with fewer than 16 rows (AR rows of A that exist, CW rows of W that this
@@ -108,6 +109,41 @@ __global__ __launch_bounds__(WK* kWave) void gemm_direct_kernel(DirectArgs a) {
       tail_x[mt] = *(const f32x4*)(a.resid + (int64_t)min(m_base + mt * 16 + r, M - 1) * N + tail_n);
     tail_w4 = *(const f32x4*)(a.tail_w + tail_n);
   }
+  // convolved form: the rows' slots and positions come by scalar loads (the counter of the
+  // operands' loads stays theirs), a row's is picked out below; then wave 0 asks for its four
+  // channels' weights and last inputs, behind the first operands, for use at the end
+  const int conv_c = CONV ? max(min(n0 + g * 4 - a.conv_col, a.conv_channels - 4), 0) : 0;
+  float* conv_st = nullptr;
+  int conv_at = 0;
+  f32x4 conv_hist[CONV ? 3 : 1], conv_wt[CONV ? 4 : 1], conv_bias, conv_ib;
+  auto load_conv = [&]() {
+    if constexpr (CONV) {
+      if (wk != 0) return;
+      typedef const __attribute__((address_space(4))) int* scalar_ints;
+      int slots[AR], at[AR], slot = 0;
+#pragma unroll
+      for (int i = 0; i < AR; ++i) {
+        const int row = min(m_base + i, M - 1);
+        slots[i] = ((scalar_ints)a.conv_slots)[row], at[i] = ((scalar_ints)a.conv_pos)[row];
+      }
+      // (all of them first: left alone, each is loaded under the condition that picks it)
+#pragma unroll
+      for (int i = 0; i < AR; ++i) asm volatile("" ::"s"(slots[i]), "s"(at[i]));
+#pragma unroll
+      for (int i = 0; i < AR; ++i) {
+        slot = r % AR == i ? slots[i] : slot;
+        conv_at = r % AR == i ? at[i] : conv_at;
+      }
+      conv_st = a.conv_state + (int64_t)slot * 3 * a.conv_channels + conv_c;
+#pragma unroll
+      for (int j = 0; j < 3; ++j) conv_hist[j] = *(const f32x4*)(conv_st + (int64_t)j * a.conv_channels);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) conv_wt[t] = *(const f32x4*)(a.conv_w + (conv_c + t) * 4);
+      // (without a bias the weights' first are read instead and dropped)
+      conv_bias = *(const f32x4*)((a.conv_b ? a.conv_b : a.conv_w) + conv_c);
+      conv_ib = *(const f32x4*)((a.conv_in_b ? a.conv_in_b : a.conv_w) + conv_c);
+    }
+  };
   // scaled form: a row's slices lie side by side (rows of `parts` rounded up to four);
   // four of them, 4 j .. 4 j + 3, go to wave (j / 4) % WK, lane group j % 4 in one load; a
   // four past the last reads the last again and is dropped
@@ -363,6 +399,7 @@ __global__ __launch_bounds__(WK* kWave) void gemm_direct_kernel(DirectArgs a) {
       __builtin_amdgcn_sched_barrier(0);
     }
     load_parts();
+    load_conv();
     __builtin_amdgcn_sched_barrier(0);
     for (; kb + (2 * PD - 1) * stride < kfull; kb += PD * stride) {
 #pragma unroll
@@ -376,6 +413,7 @@ __global__ __launch_bounds__(WK* kWave) void gemm_direct_kernel(DirectArgs a) {
     for (int p = 0; p < PD; ++p)
       if (kb0 + p * stride < kfull) load(st[p], kb0 + p * stride);
     load_parts();
+    load_conv();
   }
   // the last steps (all of them, for a short K)
   for (; kb < kfull; kb += PD * stride) {
@@ -510,14 +548,35 @@ __global__ __launch_bounds__(WK* kWave) void gemm_direct_kernel(DirectArgs a) {
       }
     }
     store4<TC>(C + (int64_t)m * N + n, v, N - n);
+    if constexpr (CONV) {
+      if (n < a.conv_col || n >= a.conv_col + a.conv_channels) continue;
+      f32x4 x, out;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        x[t] = v[t] + (a.conv_in_b ? conv_ib[t] : 0.f);
+        float sum = a.conv_b ? conv_bias[t] : 0.f;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          // (inputs in front of the sequence are zero, whatever the slot holds)
+          if (conv_at - 3 + j < 0) conv_hist[j][t] = 0.f;
+          sum = fmaf(conv_wt[t][j], conv_hist[j][t], sum);
+        }
+        sum = fmaf(conv_wt[t][3], x[t], sum);
+        out[t] = a.conv_plain ? sum : sum / (1.0f + expf(-sum));
+      }
+      *(f32x4*)(a.conv_out + (int64_t)m * a.conv_channels + conv_c) = out;
+      *(f32x4*)conv_st = conv_hist[1];
+      *(f32x4*)(conv_st + a.conv_channels) = conv_hist[2];
+      *(f32x4*)(conv_st + 2 * (int64_t)a.conv_channels) = x;
+    }
   }
 }
 
 template <int MT, int WK, typename TC, bool PAIR, bool NORM, int S, int PD, bool SCALED = false,
-          bool TAIL = false, int CW = 16, int AR = 16>
+          bool TAIL = false, int CW = 16, int AR = 16, bool CONV = false>
 static inline void launch(const DirectArgs& a, hipStream_t stream) {
   dim3 grid((a.N + CW - 1) / CW, (a.M + MT * 16 - 1) / (MT * 16));
-  hipLaunchKernelGGL((gemm_direct_kernel<MT, WK, TC, PAIR, NORM, S, PD, SCALED, TAIL, CW, AR>),
+  hipLaunchKernelGGL((gemm_direct_kernel<MT, WK, TC, PAIR, NORM, S, PD, SCALED, TAIL, CW, AR, false, CONV>),
                      grid, dim3(WK * kWave), 0, stream, a);
 }
 
@@ -547,6 +606,7 @@ static inline int gemm_direct_packed_rows(int M) { return M <= 4 ? 4 : M <= 8 ? 
 
 // The forms' dispatchers, one per translation unit.
 int gemm_direct_plain(const DirectArgs& a, int c_type, hipStream_t stream);
+int gemm_direct_conv(const DirectArgs& a, hipStream_t stream);
 int gemm_direct_tail(const DirectArgs& a, hipStream_t stream);
 int gemm_direct_merged(const DirectArgs& a, hipStream_t stream);
 int gemm_direct_scaled(const DirectArgs& a, int c_type, bool pair, hipStream_t stream);

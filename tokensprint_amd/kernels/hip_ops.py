@@ -1273,6 +1273,36 @@ class HipOps:
                    self._stream())
         return out
 
+    def linear_conv_silu(self, x, weight, col, channels, conv_w, bias, batch, state, in_bias=None,
+                         plain=False):
+        """(proj, conv): x weight^T in float32, and `conv_silu` of its columns [col, col +
+        channels).  A decode step's few bfloat16 rows are convolved in the product's epilogue."""
+        x = self._rows(x)
+        self._check("x", x, self._FLOATS, ndim=2)
+        self._check("weight", weight, self._FLOATS, ndim=2)
+        (M, K), N = x.shape, weight.shape[0]
+        taps = conv_w.shape[1]
+        if not (weight.shape[1] == K and self._single_tokens(batch) and self._mfma_ok(x, weight)
+                and not self._library_rows(M, N, K)
+                and self.lib.ts_gemm_conv_fits(M, N, K, int(col), channels, taps) == 1
+                and not any(t is not None and t.data_ptr() % 16 for t in
+                            (x, weight, conv_w, bias, in_bias, state))):
+            proj = self.linear(x, weight, torch.float32)
+            return proj, self.conv_silu(proj, col, channels, conv_w, bias, batch, state,
+                                        in_bias=in_bias, plain=plain)
+        self._check("conv weight", conv_w, torch.float32, shape=(channels, taps))
+        for name, b in (("conv bias", bias), ("conv input bias", in_bias)):
+            if b is not None:
+                self._check(name, b, torch.float32, shape=(channels,))
+        self._check_state("conv state", state, (taps - 1, channels))
+        pos, _, _, slots = self._batch_ptrs(batch, M)
+        proj = torch.empty(M, N, dtype=torch.float32, device=self.device)
+        out = torch.empty(M, channels, dtype=torch.float32, device=self.device)
+        self._call(self.lib.ts_gemm_conv_silu, _ptr(x), _ptr(weight), _ptr(proj), M, N, K,
+                   int(col), channels, taps, _ptr(conv_w), _ptr(bias), _ptr(in_bias), _ptr(state),
+                   _ptr(out), pos, slots, int(bool(plain)), self._stream())
+        return proj, out
+
     def ssm_scan(self, xbc, proj, dt_col, dt_bias, a_log, d_skip, batch, state, *, heads, vdim,
                  state_rows, groups):
         """The recurrence S <- exp(-exp(A_log) d) S + d B x^T, y = S^T C + D x per head,

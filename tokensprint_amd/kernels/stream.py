@@ -159,3 +159,13 @@ class StreamProducts:
             if prepared is not None:
                 return prepared
         return self.ops.linear(x, weight, self.ctx.dtype)
+
+
+def product_and_conv(ops, x, weight, col, channels, conv_w, bias, batch, state):
+    """(x weight^T in float32, the short convolution of its columns [col, col + channels)); a
+    provider that has the two in one call chooses how."""
+    fused = getattr(ops, "linear_conv_silu", None)
+    if fused is not None:
+        return fused(x, weight, col, channels, conv_w, bias, batch, state)
+    proj = ops.linear(x, weight, torch.float32)
+    return proj, ops.conv_silu(proj, col, channels, conv_w, bias, batch, state)

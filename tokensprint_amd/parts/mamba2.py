@@ -21,6 +21,7 @@ import math
 
 import torch
 
+from tokensprint_amd.kernels.stream import product_and_conv
 from tokensprint_amd.parts.base import MIXERS, Mixer, SlotStateNeed, TensorDecl, register
 
 
@@ -74,9 +75,8 @@ class Mamba2(Mixer):
         if not write_cache:
             raise RuntimeError(f"{self.prefix}: a recurrence cannot read another run's state")
         ops = self.ops
-        proj = ops.linear(h, self.w_in, torch.float32)
-        xbc = ops.conv_silu(proj, self.inner, self.channels, self.conv_w, self.conv_b, batch,
-                            cache.states["conv"])
+        proj, xbc = product_and_conv(ops, h, self.w_in, self.inner, self.channels, self.conv_w,
+                                     self.conv_b, batch, cache.states["conv"])
         y = ops.ssm_scan(xbc, proj, 2 * self.inner + 2 * self.bc, self.dt_bias, self.a_log,
                          self.d_skip, batch, cache.states["ssm"], heads=self.heads,
                          vdim=self.vdim, state_rows=self.state, groups=self.groups)

@@ -22,7 +22,8 @@ import math
 
 import torch
 
-from tokensprint_amd.kernels.stream import NormedPair, StreamProducts, fused_rmsnorm_of
+from tokensprint_amd.kernels.stream import (NormedPair, StreamProducts, fused_rmsnorm_of,
+                                            product_and_conv)
 from tokensprint_amd.parts.base import (MIXERS, Mixer, SlotStateNeed, TensorDecl, build_part,
                                         flat_needs, register)
 
@@ -233,10 +234,9 @@ class GatedDeltaRule(Mixer):
         if not write_cache:
             raise RuntimeError(f"{self.prefix}: a recurrence cannot read another run's state")
         ops, H = self.ops, self.heads
-        proj = ops.linear(h, self.w_in, torch.float32)
+        proj, qkv = product_and_conv(ops, h, self.w_in, 0, self.channels, self.conv_w, None, batch,
+                                     cache.states[self.state_name + ".conv"])
         b_col, state = self.channels, cache.states[self.state_name]
-        qkv = ops.conv_silu(proj, 0, self.channels, self.conv_w, None, batch,
-                            cache.states[self.state_name + ".conv"])
         if self.per_channel:
             # the second steps of the two low-rank projections, on the first steps' columns
             a1 = ops.take_columns(proj, b_col + H, self.decay_rank, self.ctx.dtype)
