@@ -144,3 +144,20 @@ def test_product_and_convolution(gpu_device, N, K, col, channels, entries, bias,
         assert not got.isnan().any()
         assert torch.equal(proj, rows) and torch.equal(got, want)
         assert torch.equal(one[1:-1], other[1:-1])
+
+
+@pytest.mark.parametrize("delta_type", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width, entries", [(4, 1), (100, 3), (2048, 8), (8192, 2), (8200, 2)])
+def test_add_norm_and_shift(gpu_device, width, entries, delta_type):
+    ops = load_hip_ops(gpu_device)
+    post, norm, shift = (1 + 0.1 * rand((width,), s) for s in (1, 2, 3))
+    one, other = stale(entries, (width,)), stale(entries, (width,))
+    for i, batch in enumerate(steps(gpu_device, entries, 3)):
+        a, delta = rand((entries, width), 10 + i), rand((entries, width), 20 + i).to(delta_type)
+        b = a.clone()
+        got = ops.postnorm_add_shift(a, delta, post, 1e-5, norm, 1e-6, shift, batch, one,
+                                     torch.bfloat16)
+        ops.postnorm_add(b, delta, post, 1e-5)
+        want = ops.norm_token_shift(b, norm, 1e-6, shift, batch, other, torch.bfloat16)
+        assert not got.isnan().any()
+        assert torch.equal(a, b) and torch.equal(got, want) and torch.equal(one[1:-1], other[1:-1])

@@ -95,22 +95,33 @@ extern "C" int ts_bigram_embed(const void* table, const void* bigram, int table_
 // ---------------------------------------------------------------- add of a normalised output
 // resid += delta / rms(delta) * post_w; then, by THEN, nothing more, or also
 // out = resid / rms(resid) * norm_w, or out = resid itself (rounded to out's type, for a
-// sub-layer that reads the stream as it is).
-constexpr int kThenNothing = 0, kThenNorm = 1, kThenRows = 2;
+// sub-layer that reads the stream as it is), or the norm behind a token shift (below), for steps
+// whose rows are each their request's only token: the row before is then the state's.
+constexpr int kThenNothing = 0, kThenNorm = 1, kThenRows = 2, kThenShift = 3;
+
+struct ShiftArgs {
+  const float* weight;      // [width]
+  float* state;             // [slots, width]
+  const int *positions, *slot_ids;      // of the rows
+};
 
 template <typename TD, typename TO, int THEN>
 __global__ __launch_bounds__(1024) void postnorm_add_kernel(
     float* __restrict__ resid, const TD* __restrict__ delta, const float* __restrict__ post_w,
     const float* __restrict__ norm_w, TO* __restrict__ out, int width, float post_eps,
-    float norm_eps) {
+    float norm_eps, ShiftArgs shift) {
+  constexpr bool kNorm = THEN == kThenNorm || THEN == kThenShift, kShift = THEN == kThenShift;
   __shared__ float scratch[16];
   const int64_t row = blockIdx.x;
   const int nt = blockDim.x;
+  float* st = kShift ? shift.state + (int64_t)shift.slot_ids[row] * width : nullptr;
+  const bool from_state = kShift && shift.positions[row] > 0;
   float* x = resid + row * width;
   const TD* d = delta + row * width;
   TO* o = out + row * width;
   // (the weights are asked for with the row, not behind the sum that they wait for)
   float dc[kRowItems], xc[kRowItems], pc[kRowItems], nc[kRowItems];
+  float mc[kShift ? kRowItems : 1], sc[kShift ? kRowItems : 1];
   float ss = 0.f;
 #pragma unroll
   for (int k = 0; k < kRowItems; ++k) {
@@ -118,7 +129,11 @@ __global__ __launch_bounds__(1024) void postnorm_add_kernel(
     dc[k] = i < width ? to_f32(d[i]) : 0.f;
     xc[k] = i < width ? x[i] : 0.f;
     pc[k] = i < width ? post_w[i] : 0.f;
-    nc[k] = THEN == kThenNorm && i < width ? norm_w[i] : 0.f;
+    nc[k] = kNorm && i < width ? norm_w[i] : 0.f;
+    if constexpr (kShift) {
+      mc[k] = i < width ? shift.weight[i] : 0.f;
+      sc[k] = i < width && from_state ? st[i] : 0.f;
+    }
   }
 #pragma unroll
   for (int k = 0; k < kRowItems; ++k) ss += dc[k] * dc[k];
@@ -144,16 +159,21 @@ __global__ __launch_bounds__(1024) void postnorm_add_kernel(
     if (THEN == kThenRows) o[i] = from_f32<TO>(v);
     ss2 += v * v;
   }
-  if (THEN == kThenNorm) {
+  if (kNorm) {
     const float r2 = inv_rms(block_sum(ss2, scratch), width, norm_eps);
+    auto finish = [&](int i, float h, float prev, float mix) {
+      if (!kShift) { o[i] = from_f32<TO>(h); return; }
+      o[i] = from_f32<TO>(h + (prev - h) * mix);
+      st[i] = h;
+    };
 #pragma unroll
     for (int k = 0; k < kRowItems; ++k) {
       const int i = threadIdx.x + k * nt;
-      if (i < width) o[i] = from_f32<TO>(xc[k] * r2 * nc[k]);
+      if (i < width) finish(i, xc[k] * r2 * nc[k], kShift ? sc[kShift ? k : 0] : 0.f, kShift ? mc[kShift ? k : 0] : 0.f);
     }
     // each thread reads back the elements it wrote itself
     for (int i = threadIdx.x + kRowItems * nt; i < width; i += nt)
-      o[i] = from_f32<TO>(x[i] * r2 * norm_w[i]);
+      finish(i, x[i] * r2 * norm_w[i], from_state ? st[i] : 0.f, kShift ? shift.weight[i] : 0.f);
   }
 }
 
@@ -169,20 +189,39 @@ extern "C" int ts_postnorm_add(float* resid, const void* delta, int delta_type,
   TS_DISPATCH_TYPE(delta_type, TD, {
     if (!out) {
       hipLaunchKernelGGL((postnorm_add_kernel<TD, float, kThenNothing>), grid, block, 0, stream,
-                         resid, (const TD*)delta, post_w, nullptr, nullptr, width, post_eps, 0.f);
+                         resid, (const TD*)delta, post_w, nullptr, nullptr, width, post_eps, 0.f, ShiftArgs{});
     } else if (norm_w) {
       TS_DISPATCH_TYPE(out_type, TO,
                        hipLaunchKernelGGL((postnorm_add_kernel<TD, TO, kThenNorm>), grid, block, 0,
                                           stream, resid, (const TD*)delta, post_w, norm_w,
-                                          (TO*)out, width, post_eps, norm_eps));
+                                          (TO*)out, width, post_eps, norm_eps, ShiftArgs{}));
     } else {
       TS_DISPATCH_TYPE(out_type, TO,
                        hipLaunchKernelGGL((postnorm_add_kernel<TD, TO, kThenRows>), grid, block, 0,
                                           stream, resid, (const TD*)delta, post_w, nullptr,
-                                          (TO*)out, width, post_eps, 0.f));
+                                          (TO*)out, width, post_eps, 0.f, ShiftArgs{}));
     }
   });
   TS_CHECK_LAUNCH("postnorm_add");
+  return 0;
+}
+
+// The add and what ts_norm_token_shift makes of the new stream, in one kernel, for steps in which
+// row t is the only token of the request in slot slot_ids[t].  (8 rows of 2,048: 5.3 us, as two
+// kernels 4.6 and 4.7: each is a launch, trips to memory and sums over a row.)
+extern "C" int ts_postnorm_add_shift(float* resid, const void* delta, int delta_type,
+                                     const float* post_w, float post_eps, const float* norm_w,
+                                     float norm_eps, const float* shift_w, float* state, void* out,
+                                     int out_type, const int* positions, const int* slot_ids,
+                                     int rows, int width, hipStream_t stream) {
+  if (rows <= 0) return 0;
+  if (width <= 0) TS_FAIL("postnorm_add_shift: bad width %d", width);
+  const ShiftArgs shift{shift_w, state, positions, slot_ids};
+  TS_DISPATCH_TYPE(delta_type, TD, TS_DISPATCH_TYPE(out_type, TO,
+      hipLaunchKernelGGL((postnorm_add_kernel<TD, TO, kThenShift>), dim3(rows),
+                         dim3(row_threads(width)), 0, stream, resid, (const TD*)delta, post_w,
+                         norm_w, (TO*)out, width, post_eps, norm_eps, shift)));
+  TS_CHECK_LAUNCH("postnorm_add_shift");
   return 0;
 }
 

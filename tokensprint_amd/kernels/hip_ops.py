@@ -1202,6 +1202,29 @@ class HipOps:
                    slots, T, W, self._stream())
         return out
 
+    def postnorm_add_shift(self, resid, delta, post_w, post_eps, norm_w, norm_eps, shift_w, batch,
+                           state, out_dtype):
+        """`postnorm_add`, then `norm_token_shift` of the new resid; one kernel where every
+        entry brings one token."""
+        if not self._single_tokens(batch):
+            self.postnorm_add(resid, delta, post_w, post_eps)
+            return self.norm_token_shift(resid, norm_w, norm_eps, shift_w, batch, state, out_dtype)
+        delta = self._rows(delta)
+        self._check("resid", resid, torch.float32, ndim=2)
+        self._check("delta", delta, self._FLOATS, shape=resid.shape)
+        T, W = resid.shape
+        for name, w in (("post-norm weight", post_w), ("norm weight", norm_w),
+                        ("shift weight", shift_w)):
+            self._check(name, w, torch.float32, shape=(W,))
+        self._check_state("shift state", state, (W,))
+        pos, _, _, slots = self._batch_ptrs(batch, T)
+        out = torch.empty(T, W, dtype=out_dtype, device=self.device)
+        self._call(self.lib.ts_postnorm_add_shift, _ptr(resid), _ptr(delta),
+                   _TYPE_CODE[delta.dtype], _ptr(post_w), c_float(post_eps), _ptr(norm_w),
+                   c_float(norm_eps), _ptr(shift_w), _ptr(state), _ptr(out),
+                   _TYPE_CODE[out_dtype], pos, slots, T, W, self._stream())
+        return out
+
     def polynorm(self, z, coef, eps, out_dtype):
         """a N(z) + b N(z^2) + c N(z^3) + e with N(v) = v / rms(v) per row; coef = (a, b, c, e)."""
         self._check("z", z, torch.float32, ndim=2)

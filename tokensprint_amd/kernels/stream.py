@@ -6,7 +6,7 @@ between parts that do."""
 
 from __future__ import annotations
 
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 
 import torch
 
@@ -52,6 +52,23 @@ class NormAhead:
 
     def entering(self, row: torch.Tensor) -> "NormAhead":
         return NormAhead(self.norm_weight, self.eps, row)
+
+
+@dataclass(frozen=True)
+class ShiftAhead:
+    """What a block that opens with an RMSNorm and a token shift behind it tells the block before
+    it: the norm's weight and eps, the shift's weight, and (`at_cache`, from whoever knows which
+    run reads next) the requests' last rows.  A block of the same kind in front may then make the
+    shifted rows in the kernel of its last add."""
+
+    norm_weight: torch.Tensor
+    eps: float
+    weight: torch.Tensor
+    state: torch.Tensor | None = None
+
+    def at_cache(self, cache) -> "ShiftAhead | None":
+        state = cache.states.get("shift") if cache is not None else None
+        return None if state is None else replace(self, state=state)
 
 
 @dataclass(frozen=True)

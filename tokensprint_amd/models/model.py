@@ -116,6 +116,9 @@ class Model:
                 # may have its norm taken ahead
                 next_hint = next_hint.entering(entering(nxt)) \
                     if hasattr(next_hint, "entering") else None
+            if hasattr(next_hint, "at_cache"):
+                next_hint = next_hint.at_cache(
+                    caches[r + 1 if nxt.cache_of is None else nxt.cache_of])
             if run.enter is not None and not getattr(delta, "entered", False):
                 # what is still to be added, then the row of this pass
                 ops.stream_add(resid, delta, None, entering(run))

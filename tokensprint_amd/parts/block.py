@@ -8,8 +8,8 @@ from __future__ import annotations
 
 import torch
 
-from tokensprint_amd.kernels.stream import (NormAhead, NormedPair, NormedRows, RowsAhead, StreamRows,
-                                            fused_rmsnorm_of)
+from tokensprint_amd.kernels.stream import (NormAhead, NormedPair, NormedRows, RowsAhead, ShiftAhead,
+                                            StreamRows,                                            fused_rmsnorm_of)
 from tokensprint_amd.parts.base import (BLOCKS, FEED_FORWARDS, FILTERS, MIXERS, NORMS, SIDES, Block,
                                         StreamFilter, TensorDecl, SlotStateNeed, register)
 
@@ -72,8 +72,22 @@ class SandwichNormBlock(Block):
             raise ValueError("sandwich_norm: a side input and its norm come together")
 
     def entry_hint(self):
-        fused = fused_rmsnorm_of(self.mixer_norm) if self.mixer_filter is None else None
+        if self.mixer_filter is not None:
+            probe = getattr(self.mixer_filter, "stream_hint", None)
+            return probe(self.mixer_norm) if callable(probe) else None
+        fused = fused_rmsnorm_of(self.mixer_norm)
         return None if fused is None else NormAhead(fused[0], fused[1])
+
+    def _post_add_shift(self, resid, out, post, shift, batch):
+        """resid += post(out); the shifted rows of its norm that `shift` asks for."""
+        ops, dtype = self.ctx.ops, self.ctx.dtype
+        fused = fused_rmsnorm_of(post)
+        if fused is not None and not isinstance(out, NormedPair):
+            return ops.postnorm_add_shift(resid, out, fused[0], fused[1], shift.norm_weight,
+                                          shift.eps, shift.weight, batch, shift.state, dtype)
+        self._post_add(resid, out, post)
+        return ops.norm_token_shift(resid, shift.norm_weight, shift.eps, shift.weight, batch,
+                                    shift.state, dtype)
 
     def _post_add(self, resid, out, post, then=None, rows=False):
         """resid += post(out); then, if given, the norm `then` (weight, eps) of the sum, or with
@@ -115,22 +129,29 @@ class SandwichNormBlock(Block):
         # front of that block would have to be added first)
         ahead = (next_hint.norm_weight, next_hint.eps) \
             if isinstance(next_hint, NormAhead) and next_hint.row is None else None
+        shift = next_hint if isinstance(next_hint, ShiftAhead) else None
         side_reads = self.side is not None
+
+        def last_add(out, post):
+            if shift is not None:
+                return self._post_add_shift(resid, out, post, shift, batch)
+            return self._post_add(resid, out, post, ahead)
+
         out = self.mixer.forward(h, batch, cache, write_cache)
         if self.feed_forward is None:
-            h = self._post_add(resid, out, self.mixer_post_norm,
-                               None if side_reads else ahead, rows=side_reads)
+            h = self._post_add(resid, out, self.mixer_post_norm, rows=True) if side_reads \
+                else last_add(out, self.mixer_post_norm)
         else:
             norm = fused_rmsnorm_of(self.ffn_norm)
             h = self._post_add(resid, out, self.mixer_post_norm, norm)
             if norm is None:
                 h = self.ffn_norm.forward(resid)
             out = self.feed_forward.forward(h, batch)
-            h = self._post_add(resid, out, self.ffn_post_norm,
-                               None if side_reads else ahead, rows=side_reads)
+            h = self._post_add(resid, out, self.ffn_post_norm, rows=True) if side_reads \
+                else last_add(out, self.ffn_post_norm)
         if side_reads:
-            h = self._post_add(resid, self.side.forward(h, batch), self.side_post_norm, ahead)
-        return resid, NormedRows(h, False) if ahead else None
+            h = last_add(self.side.forward(h, batch), self.side_post_norm)
+        return resid, NormedRows(h, False) if ahead or shift is not None else None
 
 
 @register(BLOCKS, "post_norm")
@@ -243,6 +264,14 @@ class TokenShift(StreamFilter):
 
     def cache_need(self):
         return SlotStateNeed((self.dim,), torch.float32, "shift")
+
+    def stream_hint(self, norm):
+        """For the block in front: the norm and the shift, if its provider has them behind an
+        add."""
+        fused = fused_rmsnorm_of(norm)
+        if fused is None or not hasattr(self.ops, "postnorm_add_shift"):
+            return None
+        return ShiftAhead(fused[0], fused[1], self.weight)
 
     def forward_from_stream(self, resid, norm, batch, cache):
         fused = fused_rmsnorm_of(norm)
