@@ -13,7 +13,7 @@ bool gemm_direct_conv_fits(int M, int N, int K, int col, int channels, int taps)
          col >= 0 && col + channels <= N;
 }
 
-int gemm_direct_conv(const DirectArgs& a, hipStream_t stream) {
+int gemm_direct_conv(const ConvArgs& a, hipStream_t stream) {
   const bool deep = layout_deep(a.N, a.K), narrow = gemm_direct_columns(a.M, a.N) == 8;
   TS_DIRECT_ROWS(a.M, {
     if (deep && narrow) launch<1, 8, float, false, false, 4, 4, false, false, 8, AR, true>(a, stream);
@@ -43,7 +43,7 @@ extern "C" int ts_gemm_conv_silu(const void* a, const void* w, float* c, int M, 
   if (((uintptr_t)a | (uintptr_t)w | (uintptr_t)conv_w | (uintptr_t)bias | (uintptr_t)in_bias |
        (uintptr_t)state | (uintptr_t)out) & 15)
     TS_FAIL("gemm_conv_silu: operands must be 16-byte aligned");
-  DirectArgs d = {};
+  ConvArgs d = {};
   d.A = (const bf16_t*)a, d.W = (const bf16_t*)w, d.C = c, d.M = M, d.N = N, d.K = K;
   d.conv_w = conv_w, d.conv_b = bias, d.conv_in_b = in_bias, d.conv_state = state, d.conv_out = out;
   d.conv_pos = positions, d.conv_slots = slot_ids;

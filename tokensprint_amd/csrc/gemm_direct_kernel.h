@@ -30,7 +30,8 @@ __device__ __forceinline__ bf16x8 row_down_by(bf16x8 v, int n) {
 
 template <int MT, int WK, typename TC, bool PAIR, bool NORM, int S, int PD, bool SCALED = false,
           bool TAIL = false, int CW = 16, int AR = 16, bool MERGE = false, bool CONV = false>
-__global__ __launch_bounds__(WK* kWave) void gemm_direct_kernel(DirectArgs a) {
+__global__ __launch_bounds__(WK* kWave) void gemm_direct_kernel(
+    std::conditional_t<CONV, ConvArgs, DirectArgs> a) {
   static_assert(!NORM || MT == 1, "the fused form holds one tile of rows");
   static_assert(!MERGE || (TAIL && MT == 1), "the merged form: a tail product of one tile of rows");
   static_assert(!CONV || (MT == 1 && !PAIR && !NORM && !SCALED && !TAIL), "the convolved form is a plain product");
@@ -112,7 +113,8 @@ __global__ __launch_bounds__(WK* kWave) void gemm_direct_kernel(DirectArgs a) {
   // convolved form: the rows' slots and positions come by scalar loads (the counter of the
   // operands' loads stays theirs), a row's is picked out below; then wave 0 asks for its four
   // channels' weights and last inputs, behind the first operands, for use at the end
-  const int conv_c = CONV ? max(min(n0 + g * 4 - a.conv_col, a.conv_channels - 4), 0) : 0;
+  int conv_c = 0;
+  if constexpr (CONV) conv_c = max(min(n0 + g * 4 - a.conv_col, a.conv_channels - 4), 0);
   float* conv_st = nullptr;
   int conv_at = 0;
   f32x4 conv_hist[CONV ? 3 : 1], conv_wt[CONV ? 4 : 1], conv_bias, conv_ib;
@@ -574,7 +576,7 @@ __global__ __launch_bounds__(WK* kWave) void gemm_direct_kernel(DirectArgs a) {
 
 template <int MT, int WK, typename TC, bool PAIR, bool NORM, int S, int PD, bool SCALED = false,
           bool TAIL = false, int CW = 16, int AR = 16, bool CONV = false>
-static inline void launch(const DirectArgs& a, hipStream_t stream) {
+static inline void launch(const std::conditional_t<CONV, ConvArgs, DirectArgs>& a, hipStream_t stream) {
   dim3 grid((a.N + CW - 1) / CW, (a.M + MT * 16 - 1) / (MT * 16));
   hipLaunchKernelGGL((gemm_direct_kernel<MT, WK, TC, PAIR, NORM, S, PD, SCALED, TAIL, CW, AR, false, CONV>),
                      grid, dim3(WK * kWave), 0, stream, a);
@@ -606,7 +608,7 @@ static inline int gemm_direct_packed_rows(int M) { return M <= 4 ? 4 : M <= 8 ? 
 
 // The forms' dispatchers, one per translation unit.
 int gemm_direct_plain(const DirectArgs& a, int c_type, hipStream_t stream);
-int gemm_direct_conv(const DirectArgs& a, hipStream_t stream);
+int gemm_direct_conv(const ConvArgs& a, hipStream_t stream);
 int gemm_direct_tail(const DirectArgs& a, hipStream_t stream);
 int gemm_direct_merged(const DirectArgs& a, hipStream_t stream);
 int gemm_direct_scaled(const DirectArgs& a, int c_type, bool pair, hipStream_t stream);
