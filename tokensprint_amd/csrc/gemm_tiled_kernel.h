@@ -47,7 +47,7 @@ struct TiledArgs {
   void* c;
   int M, N, K;          // N: columns of C (with PAIR: of each half of W)
   int tiles_m, tiles_n;
-  int groups_n;         // the tile grid is cut into 8 regions, 8 / groups_n by groups_n
+  int panel;            // tiles of a panel along M
   // SCALED: the sums of squares of A's rows [parts, M]
   const float* sumsq_in;
   int parts;
@@ -101,15 +101,15 @@ __global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgs g
   const int wm = wave / GN, wn = wave % GN;
 
   // Which tile: workgroups go round the 8 XCDs by their index, each XCD has an L2 of its
-  // own, so each XCD gets a compact region of the tile grid (its workgroups share rows of
-  // A and W), walked row by row.
-  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
-  const int groups_m = 8 / g.groups_n;
-  const int region_m = (g.tiles_m + groups_m - 1) / groups_m;
-  const int region_n = (g.tiles_n + g.groups_n - 1) / g.groups_n;
-  const int tile_m = (xcd / g.groups_n) * region_m + local / region_n;
-  const int tile_n = (xcd % g.groups_n) * region_n + local % region_n;
-  if (local >= region_m * region_n || tile_m >= g.tiles_m || tile_n >= g.tiles_n) return;
+  // own, so each XCD gets an eighth of the tiles that lie together (its workgroups share rows
+  // of A and W): the tile grid is walked in panels of `panel` tiles along M, down a panel's
+  // columns.
+  const int local = blockIdx.x >> 3, per_xcd = gridDim.x >> 3;
+  const int tile = (blockIdx.x & 7) * per_xcd + local;
+  if (tile >= g.tiles_m * g.tiles_n) return;
+  const int panel = tile / (g.panel * g.tiles_n), in_panel = tile - panel * g.panel * g.tiles_n;
+  const int height = min(g.panel, g.tiles_m - panel * g.panel);
+  const int tile_m = panel * g.panel + in_panel % height, tile_n = in_panel / height;
   const int m0 = tile_m * BM;
 
   // SCALED: the factors of this tile's rows.  Called once the first direct loads are on
@@ -160,6 +160,16 @@ __global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgs g
     }
   };
 
+  // row of the tile that LDS row `j` of the A slab holds: the upper halves of all waves' parts,
+  // then the lower ones, where a turn takes them apart
+  auto a_row = [&](int j) {
+    if constexpr (TM * TN > 16) {
+      const int in = j % (BM / 2);
+      return in / (WM / 2) * WM + j / (BM / 2) * (WM / 2) + in % (WM / 2);
+    } else {
+      return j;
+    }
+  };
   // column of W (row of the stacked weight) that LDS row `j` of the W slab holds
   auto w_row = [&](int j) {
     if constexpr (PAIR) {
@@ -179,7 +189,7 @@ __global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgs g
   for (int i = 0; i < LA; ++i) {
     const int row = (NW * i + wave) * 8 + (lane >> 3);
     const int piece = (lane & 7) ^ ((row >> 1) & 7);
-    off_a[i] = (unsigned)min(m0 + row, g.M - 1) * row_bytes + piece * 16;
+    off_a[i] = (unsigned)min(m0 + a_row(row), g.M - 1) * row_bytes + piece * 16;
   }
 #pragma unroll
   for (int i = 0; i < LW; ++i) {
@@ -246,59 +256,99 @@ __global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgs g
   // into the buffer that step kt has left.
   const int KT = g.K / 64;                              // at least STAGES (the launcher's check)
   if constexpr (TM * TN > 16) {
-    // A wave's part is too large to hold two K steps' operands beside its sums: the
-    // column operands of a K step of 32 are read first, the row operands one ahead of
-    // their products, and a turn is: step kt has arrived and step kt - 1 has been read by
-    // everyone (barrier); multiply step kt while the loads of step kt + STAGES - 1 go out
-    // into the buffer that step kt - 1 has left.  Two waves share a SIMD and fill each
-    // other's waits.
+    // A wave's part is too large to hold two K steps' operands beside its sums.  A turn (one K
+    // step) is walked in blocks of TN products, a row block of A against the wave's columns:
+    // the upper half of its row blocks with the first 32 of K, with the second, then the lower
+    // half.  The columns' operands stay in registers for the turn, a row block's comes out of
+    // LDS H blocks before its products, also across the turns' border.  So a step's W and
+    // upper A have been read an eighth of a turn after their first use, its lower A an eighth
+    // after its own, and two meetings a turn say so: the loads that go into their places have
+    // about a turn to arrive with two buffers, and no wave waits for LDS in front of its products.
+    // (With one meeting a turn, at its border, everything was waited for there and every half
+    // began with a trip to LDS.  256 x 256 tiles, products of zeros, 2,048 x 24,576 x 4,096: 285 ->
+    // 232 us, of ordinary data, where the card's power holds it back, 333 -> 314; 8,192 x 51,200 x
+    // 5,120 3,986 -> 3,124, of that 125 by panels of eight tiles instead of four.  Four wavefronts
+    // of 128 x 128, with two thirds of the reads of LDS, are as fast; a higher priority of half the
+    // wavefronts, or of the products, changes nothing.)
+    static_assert(STAGES == 2 && TM % 2 == 0 && LA % 2 == 0, "two buffers, whole halves of A");
+    constexpr int H = TM / 2, LOWER = LA / 2, FIRST = LW + LOWER;
+    // Load i of a step: the columns, the upper half of the rows, then the lower half.  A unit
+    // takes a load in about 28 cycles, so a turn's are spread over its blocks, from block H on
+    // (where the places of the first are free) and through block H - 1 of the next turn.
+    auto issue = [&](int stage, int kt, int i) {
+      issue_one(stage, kt, i < LW ? LA + i : i - LW);
+    };
+    auto at = [](int i) constexpr { return i * (4 * H) / LOADS; };   // blocks behind block H
+    auto issued_before = [at](int q) constexpr {                     // of a step's loads
+      int n = 0;
+      for (int i = 0; i < LOADS; ++i) n += at(i) < q;
+      return n;
+    };
+    static_assert(at(FIRST) >= 2 * H, "a place is free when it is sent for");
+    constexpr int EARLY_LOADS = issued_before(3 * H), BY_MEETING = issued_before(2 * H);
 #pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s)
+    for (int i = 0; i < LOADS; ++i) issue(0, 0, i);
 #pragma unroll
-      for (int i = 0; i < LOADS; ++i) issue_one(s, s, i);
+    for (int i = 0; i < EARLY_LOADS; ++i) issue(1, 1, i);
     row_scales();
-    // a turn: everything that was sent for has to have arrived.  (The last one, which sends
-    // nothing, apart: no branch in the others.  The gate/up product of 2,048 rows at
-    // 2 x 3,072 x 1,024 in 256 x 192 tiles 31.6 -> 30.4 us.)
-    auto turn = [&](auto with_loads, int s, int kt) {
-      constexpr bool load = decltype(with_loads)::value;
-      wait_loads<0>();
+    auto meet = [&](auto in_flight) {
+      __builtin_amdgcn_sched_barrier(0);
+      wait_loads<decltype(in_flight)::value>();
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      const unsigned char* slab = tiled_lds + s * STAGE_BYTES;
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    bf16x8 fw[2][TN], fa[H];
+    auto read_columns = [&](int stage, int ks) {
+      const unsigned char* sw = tiled_lds + stage * STAGE_BYTES + (BM + wn * WN) * 128 + (ks ? read1 : read0);
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        const unsigned char* sa = slab + wm * WM * 128 + (ks ? read1 : read0);
-        const unsigned char* sw = slab + (BM + wn * WN) * 128 + (ks ? read1 : read0);
-        bf16x8 fw[TN], fa = *(const bf16x8*)sa, fb;
+      for (int tn = 0; tn < TN; ++tn) fw[ks][tn] = *(const bf16x8*)(sw + tn * 2048);
+    };
+    auto read_rows = [&](int stage, int half, int ks, int t) {
+      fa[t] = *(const bf16x8*)(tiled_lds + stage * STAGE_BYTES +
+                               (half * (BM / 2) + wm * (WM / 2) + t * 16) * 128 + (ks ? read1 : read0));
+    };
+    meet(std::integral_constant<int, LOWER + EARLY_LOADS>{});
+    read_columns(0, 0);
 #pragma unroll
-        for (int tn = 0; tn < TN; ++tn) fw[tn] = *(const bf16x8*)(sw + tn * 2048);
+    for (int t = 0; t < H; ++t) read_rows(0, 0, 0, t);
+    // behind: steps that follow this one (2: two or more)
+    auto turn = [&](auto steps_behind, int s, int kt) {
+      constexpr int behind = decltype(steps_behind)::value;
+      read_columns(s, 1);
 #pragma unroll
-        for (int tm = 0; tm < TM; ++tm) {
-          if (tm + 1 < TM) fb = *(const bf16x8*)(sa + (tm + 1) * 2048);
+      for (int b = 0; b < 4 * H; ++b) {
+        const int half = b / (2 * H), ks = b / H % 2, t = b % H;
 #pragma unroll
-          for (int tn = 0; tn < TN; ++tn)
-            acc[tn][tm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[tn], fa, acc[tn][tm], 0, 0, 0);
-          fa = fb;
-          constexpr int PER = (LOADS + 2 * TM - 1) / (2 * TM);      // loads per row block
-          if constexpr (load) {
-#pragma unroll
-            for (int j = 0; j < PER; ++j) {
-              const int i = (ks * TM + tm) * PER + j;
-              if (i < LOADS) issue_one(s ^ 1, kt + 1, i);
-            }
+        for (int tn = 0; tn < TN; ++tn)
+          acc[tn][half * H + t] =
+              __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[ks][tn], fa[t], acc[tn][half * H + t], 0, 0, 0);
+        // the lower half of this step has arrived; its W and upper half have been read
+        if (b == H) meet(std::integral_constant<int, behind >= 1 ? LOADS : 0>{});
+        if constexpr (behind >= 1) {
+          // the next step's W and upper half have arrived; this one's lower half has been read
+          if (b == 3 * H) {
+            meet(std::integral_constant<int, behind >= 2 ? LOWER + BY_MEETING : LOWER>{});
+            read_columns(s ^ 1, 0);
           }
         }
+        if (b < 3 * H) read_rows(s, (b + H) / (2 * H), (b + H) / H % 2, t);
+        else if constexpr (behind >= 1) read_rows(s ^ 1, 0, 0, t);
+        if constexpr (behind >= 1) {
+#pragma unroll
+          for (int i = 0; i < LOADS; ++i) {
+            if (b < H && at(i) == 3 * H + b) issue(s ^ 1, kt + 1, i);
+            if (behind >= 2 && b >= H && at(i) == b - H) issue(s, kt + 2, i);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
     };
-    static_assert(STAGES == 2, "the turns are written out for a ring of two");
-    for (int kt = 0; kt + 2 < KT; kt += 2) {
-      turn(std::true_type{}, 0, kt);
-      turn(std::true_type{}, 1, kt + 1);
-    }
-    if (KT % 2 == 0) turn(std::true_type{}, 0, KT - 2);
-    turn(std::false_type{}, (KT - 1) % 2, KT - 1);
+    int kt = 0;
+    for (; kt + 2 < KT; ++kt) turn(std::integral_constant<int, 2>{}, kt & 1, kt);
+    turn(std::integral_constant<int, 1>{}, kt & 1, kt);
+    turn(std::integral_constant<int, 0>{}, (kt + 1) & 1, kt + 1);
   } else {
 #pragma unroll
   for (int s = 0; s < STAGES; ++s)
@@ -473,20 +523,17 @@ int launch_tiled(TiledArgs g, hipStream_t stream) {
   if (g.K / 64 < STAGES) TS_FAIL("gemm_tiled: K=%d is too short for %d buffers", g.K, STAGES);
   g.tiles_m = (g.M + BM - 1) / BM;
   g.tiles_n = (g.N + (PAIR ? BN / 2 : BN) - 1) / (PAIR ? BN / 2 : BN);
-  // regions of the tile grid, one per XCD: the cut that brings the fewest bytes of A and W
-  // into an L2
-  int best = 1;
-  int64_t best_cost = -1;
-  for (int gn = 1; gn <= 8; gn *= 2) {
-    const int gm = 8 / gn;
-    const int64_t rm = (g.tiles_m + gm - 1) / gm, rn = (g.tiles_n + gn - 1) / gn;
-    const int64_t cost = rm * BM + rn * BN;
-    if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = gn; }
+  // the height of a panel: the one with which the tiles that an XCD's units hold at a time (32)
+  // bring the fewest rows of A and W into its L2.  (Regions of the grid, one an XCD, came before
+  // it: where they divided the tiles unevenly one XCD had a round more than the others.
+  // 1,536 x 10,304 x 2,048 in 246 tiles of 256 x 256: 92 -> 58 us.)
+  const int per_xcd = (int)(((int64_t)g.tiles_m * g.tiles_n + 7) / 8), held = per_xcd < 32 ? per_xcd : 32;
+  int64_t best_rows = -1;
+  for (int p = 1; p <= 16; p *= 2) {
+    const int64_t rows = (int64_t)(p < g.tiles_m ? p : g.tiles_m) * BM + (int64_t)((held + p - 1) / p) * BN;
+    if (best_rows < 0 || rows < best_rows) { best_rows = rows; g.panel = p; }
   }
-  g.groups_n = best;
-  const int gm = 8 / best;
-  const int region = ((g.tiles_m + gm - 1) / gm) * ((g.tiles_n + best - 1) / best);
-  hipLaunchKernelGGL(kernel, dim3(8 * region), dim3(64 * GM * GN), lds, stream, g);
+  hipLaunchKernelGGL(kernel, dim3(8 * per_xcd), dim3(64 * GM * GN), lds, stream, g);
   TS_CHECK_LAUNCH("gemm_tiled");
   return 0;
 }
@@ -495,36 +542,44 @@ int launch_tiled(TiledArgs g, hipStream_t stream) {
 // the smallest estimate of rounds x time of a tile, a round being one tile on every
 // compute unit.  A tile's time is a fixed part (launch, first loads, epilogue and the
 // stores' way to memory; the SiLU of the paired form on top) and a part per K step of 64,
-// both measured on an MI355X at 512 to 8,192 rows with the weights of the 0.6B shape
-// (N 1,024 to 6,144, K 1,024 to 3,072): a large tile needs fewer bytes from L2 per
-// product and its steps are bound by the matrix cores (1.2 us for 256 x 256), a small
-// one's by the rate at which a unit takes direct loads (0.28 us for 128 x 64, 2.3 times
-// the matrix cores' time), but a tile is one workgroup and a unit without one idles.
+// both fitted to an MI355X at 65 to 8,192 rows of 23 weights (N 1,024 to 51,200, K 1,024 to
+// 25,600) in memory, where the estimate's choice is the fastest tile but for 0.02 % of the time:
+// a large tile needs fewer bytes from L2 per product and its steps are bound by the matrix cores
+// (1.1 us for 256 x 256 on average; at what the card's power allows with all units busy on
+// ordinary data up to 1.5, with zeros 1.2), a small one's by the rate at which a unit takes
+// direct loads (0.33 us for 128 x 64, 2.3 times the matrix cores' time), but a tile is one
+// workgroup and a unit without one idles.
 struct TileCost {
   int tile, bm, bn;
   float fixed_us, step_us, pair_us;
 };
 constexpr TileCost kTileCosts[] = {
-    {3, 128, 64, 4.4f, 0.275f, 1.f}, {2, 128, 128, 6.3f, 0.39f, 1.5f}, {1, 256, 128, 7.8f, 0.66f, 2.f},
-    {5, 256, 192, 8.f, 1.1f, 3.f},   {4, 256, 256, 7.f, 1.19f, 4.f},
+    {3, 128, 64, 1.2f, 0.329f, 0.5f}, {2, 128, 128, 2.4f, 0.491f, 0.8f}, {1, 256, 128, 4.5f, 0.721f, 1.4f},
+    {5, 256, 192, 6.6f, 0.931f, 1.1f}, {4, 256, 256, 7.7f, 1.126f, 1.6f},
 };
 
-inline int cheapest_tile(const TiledArgs& g, bool pair) {
+// Compute units of the current device (256 where it cannot be asked).
+inline int compute_units() {
   static int units[64] = {};
   int device = 0;
-  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return 3;
+  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return 256;
   if (units[device] == 0) {
     int n = 0;
     if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0)
       n = 256;
     units[device] = n;
   }
+  return units[device];
+}
+
+inline int cheapest_tile(const TiledArgs& g, bool pair) {
+  const int units = compute_units();
   const int64_t cols = pair ? 2 * (int64_t)g.N : g.N;
   int best = 3;
   float best_us = -1.f;
   for (const TileCost& t : kTileCosts) {
     const int64_t tiles = (int64_t)((g.M + t.bm - 1) / t.bm) * ((cols + t.bn - 1) / t.bn);
-    const int64_t rounds = (tiles + units[device] - 1) / units[device];
+    const int64_t rounds = (tiles + units - 1) / units;
     const float us = rounds * (t.fixed_us + (pair ? t.pair_us : 0.f) + t.step_us * (g.K / 64));
     if (best_us < 0.f || us < best_us) { best_us = us; best = t.tile; }
   }
