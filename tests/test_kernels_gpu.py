@@ -207,7 +207,7 @@ def test_linear_silu_mul(ops, gpu_device, dtype, M, I, K):
                                    (513, 4096, 1024), (1000, 48, 4096), (640, 1296, 640)])
 def test_gemm_tiled(ops, gpu_device, out_dtype, M, N, K):
     """The LDS-tiled product at sizes whose edges cut tiles in both directions and whose
-    tile grids do not divide into the eight regions evenly, with every tile size: against
+    tile grids do not divide into eighths evenly, with every tile size: against
     float32 sums of the same bfloat16 operands, and every tile size the same to the bit
     (one accumulator per element sums K in index order whatever the tile)."""
     x = rand((M, K), torch.bfloat16, gpu_device, 50)
@@ -245,6 +245,34 @@ def test_gemm_tiled_with_silu_mul(ops, gpu_device, M, I, K):
     # the engine's entry takes this kernel from 65 rows on at weights of this size
     if 2 * I * K <= ops.dispatch.tiled_pair_weight:
         assert torch.equal(ops.linear_silu_mul(x, w, torch.bfloat16), first)
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 400, 256), (130, 4640, 320), (1000, 2064, 4224),
+                                   (1024, 4096, 2176), (512, 8192, 1088)])
+def test_plain_products_that_the_tiled_kernel_takes(ops, gpu_device, M, N, K):
+    """Columns that are no multiple of 256 from 65 rows on, and weights above
+    `tiled_plain_weight` whose tiles fill their rounds: `linear` is the tiled kernel there."""
+    assert ops.lib.ts_gemm_tiled_ahead(M, N, K, 1) == 1
+    x = rand((M, K), torch.bfloat16, gpu_device, 57)
+    w = rand((N, K), torch.bfloat16, gpu_device, 58, scale=0.05)
+    out = ops.linear(x, w, torch.bfloat16)
+    assert torch.equal(out, ops.gemm_tiled(x, w, torch.bfloat16))
+    torch.testing.assert_close(out.float(), x.float() @ w.float().T, rtol=1e-2, atol=1e-2)
+
+
+@pytest.mark.parametrize("M", [15, 16, 64, 65, 200])
+def test_gate_up_of_a_large_weight(ops, gpu_device, M):
+    """Around the row counts at which a gate/up product above `large_weight` elements goes from
+    the weight-streaming kernel to the tiled one."""
+    inner, K = 4128, 1088
+    x = rand((M, K), torch.bfloat16, gpu_device, 59)
+    w = rand((2 * inner, K), torch.bfloat16, gpu_device, 60, scale=0.05)
+    assert w.numel() > ops.dispatch.large_weight
+    out = ops.linear_silu_mul(x, w, torch.bfloat16)
+    if M >= ops.dispatch.library_rows_large:
+        assert torch.equal(out, ops.gemm_tiled(x, w, torch.bfloat16, pair=True))
+    torch.testing.assert_close(out.float(), REF.linear_silu_mul(x, w, torch.bfloat16).float(),
+                               rtol=2e-2, atol=2e-2)
 
 
 @pytest.mark.parametrize("M,N,K,next_n,silu", [(2051, 1024, 2048, 3072, True),

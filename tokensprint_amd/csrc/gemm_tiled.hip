@@ -9,6 +9,32 @@ extern "C" int ts_gemm_tiled_fits(int M, int N, int K, int pair) {
          (int64_t)M * K * 2 < (1ll << 32) && rows_w * K * 2 < (1ll << 32);
 }
 
+// 1 if the plain product of these sizes (that ts_gemm_tiled_fits) is this kernel's rather than
+// the library's.  Both timed at 65 to 8,192 rows of 18 weights (N 1,024 to 10,304, K 1,024 to
+// 25,600), the weights in memory, bfloat16 out: where N is no multiple of 256 (4,384, 4,640,
+// 6,176, 10,304) this kernel takes 0.59 to 1.11 of the library's time, 0.86 in the mean; where
+// N is one and the chosen tiles fill four fifths of the rounds that they take 0.67 to 1.11,
+// 0.92 in the mean (5,120 x 25,600 at 8,192 rows 1,610 / 2,090 us), but for products that the
+// library's tile of 256 x 256 cuts in whole rounds of the units: 0.97 to 1.11, 1.08 in the
+// mean, so those stay the library's (with float32 out, whose stores it does worse, they do
+// not: 2,048 x 8,192 x 2,048 59 / 66 us).  With emptier rounds neither is ahead by a rule.
+extern "C" int ts_gemm_tiled_ahead(int M, int N, int K, int c_type) {
+  if (!ts_gemm_tiled_fits(M, N, K, 0)) return 0;
+  if (N % 256 != 0) return 1;
+  const int units = compute_units();
+  const int64_t squares = (int64_t)((M + 255) / 256) * (N / 256);
+  if (c_type == TS_BF16 && squares % units == 0) return 0;
+  TiledArgs g{};
+  g.M = M, g.N = N, g.K = K;
+  const int tile = cheapest_tile(g, false);
+  for (const TileCost& t : kTileCosts) {
+    if (t.tile != tile) continue;
+    const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    return 5 * tiles >= 4 * ((tiles + units - 1) / units) * units;
+  }
+  return 0;
+}
+
 // C[M, N] = A[M, K] W[N, K]^T, or with `pair` C[M, N] = silu(A Wg^T) * (A Wu^T) (or, with a
 // `limit` other than 0, gated_unit's other forms) for W = [Wg; Wu] of 2 N rows.  `c_type`: bfloat16 or float32 (float32 not with `pair`).
 // `tile`: 0 lets the sizes choose; 1 to 5 name a tile (for measuring; the result is the

@@ -25,9 +25,16 @@ class Dispatch:
     #: in the wide layout (a short K: four waves along N) the library is ahead from 17 rows
     library_rows_wide: int = 17
     #: at the output head (N from `head_columns`: every one of thousands of workgroups
-    #: reads all rows of x) from 5 rows; measured at N = 151,936, K = 1,024
-    library_rows_head: int = 5
+    #: reads all rows of x) from 9 rows; float32 logits of 8 and 10 rows here and with the
+    #: library, us: N = 151,936 and K = 1,024 59.8 and 64.9 / 60.5 and 61.9, K = 4,096 224 and
+    #: 254 / 251 and 253; 65,536 x 2,048 52.4 and 56.9 / 66.5 and 66.7; 32,000 x 2,048 26.6 / 32.0
+    library_rows_head: int = 9
     head_columns: int = 16384
+    #: a gate/up product, whose SiLU-multiply is then a kernel of its own, goes there only where
+    #: its weight is above `pair_head_weight` elements, from 5 rows: 8 rows, here and with the
+    #: library, 16,384 x 2,048 15.3 / 20.5 us, 24,576 x 4,096 38.3 / 46.2, 51,200 x 5,120 108 / 93
+    library_rows_pair: int = 5
+    pair_head_weight: int = 1 << 27
     #: weights above `large_weight` elements (the layer shapes of the 8B and 32B models:
     #: products bound by bandwidth, not latency): every workgroup's reading of the rows of
     #: x costs as much as the weights from 16 rows on, and the library is ahead from there
@@ -37,22 +44,27 @@ class Dispatch:
     library_rows_large: int = 16
     large_weight: int = 1 << 23
 
-    # ---- gate/up product of many rows with the SiLU-multiply in its epilogue: stacked
-    # weights up to this many elements take the LDS-tiled kernel.  Against the library's
-    # product followed by the SiLU-multiply kernel: at the 0.6B shape (2 x 3,072 x 1,024)
-    # 0.56 to 0.87 of their time from 128 to 8,192 rows, because the [M, 2 I] intermediate
-    # is neither written nor read; at the 8B shape 0.85 to 1.07, at the 32B shape 1.02 to
-    # 1.20, the library's product itself being 10 to 20 % ahead at large sizes.
-    tiled_pair_weight: int = 1 << 23
+    # ---- products of many rows (from `library_rows`), the LDS-tiled kernel or the library.
+    #: A gate/up product with the SiLU-multiply in its epilogue is the tiled kernel's: neither
+    #: is the [M, 2 I] intermediate written nor read.  Against the library's product and the
+    #: SiLU-multiply kernel, 65 to 8,192 rows: 2 x 3,072 x 1,024 0.46 to 0.80 of their time,
+    #: 2 x 8,192 x 2,048 0.71 to 0.93, 2 x 12,288 x 4,096 0.80 to 0.98 (from `library_rows_large`
+    #: rows already: 24 to 64 rows 17.6 to 17.9 / 21.2 to 22.1 and 43.4 to 45.4 / 49.6 us); only
+    #: the largest weights (2 x 25,600 x 5,120: 0.83 to 0.94 from 512 rows on, 0.85 to 1.12 below)
+    #: wait for `tiled_pair_rows_large` rows.
+    tiled_pair_weight: int = 1 << 27
+    tiled_pair_rows_large: int = 512
     #: rows from which, and elements of a weight [N, K] up to which, the product that ends a
     #: sub-layer is the LDS-tiled kernel's tail form (it adds itself into the float32 stream
     #: and prepares the rows for the norm behind it, whose product then takes the scaled
-    #: form) instead of the library's product and a norm kernel.  Plain products of such
-    #: sizes (a model's first layer, whose norm nothing prepares) take the tiled kernel too:
-    #: the same time on the GPU (22.5 against 22.4 us for qkv at 2,048 rows) and a fifth of
-    #: the library call's 20 to 30 us on the host, which the GPU waits for at a step's start.
+    #: form) instead of the library's product and a norm kernel.
     tiled_stream_rows: int = 512
-    tiled_stream_weight: int = 1 << 23
+    tiled_stream_weight: int = 1 << 28
+    #: Plain products: from `tiled_stream_rows` rows and up to so many elements the tiled
+    #: kernel's (the same time on the GPU, 22.5 against 22.4 us for the 0.6B model's qkv at 2,048
+    #: rows, and a fifth of the library call's 20 to 30 us on the host, which the GPU waits for
+    #: at a step's start); others where `ts_gemm_tiled_ahead` says so.
+    tiled_plain_weight: int = 1 << 23
 
     # ---- attention.  Measured at 16 query / 8 key-value heads of 128, page size 16.
     #: workgroups (entries x key/value heads) up to which a decode step takes the decode

@@ -386,22 +386,29 @@ class HipOps:
     def _tiled_pair_ok(self, x, weight, out_dtype):
         M, K = x.shape
         inner = weight.shape[0] // 2
+        d = self.dispatch
         return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
-                and out_dtype == torch.bfloat16 and weight.numel() <= self.dispatch.tiled_pair_weight
-                and self._library_rows(M, weight.shape[0], K)
+                and out_dtype == torch.bfloat16
+                and (weight.numel() <= d.large_weight or M >= (
+                    d.library_rows_large if weight.numel() <= d.tiled_pair_weight
+                    else d.tiled_pair_rows_large))
+                and self._library_rows(M, weight.shape[0], K, weight.numel())
                 and self.lib.ts_gemm_tiled_fits(M, inner, K, 1) == 1)
 
     def _tiled_plain_ok(self, M, N, K, x_dtype, w_dtype, out_dtype):
         d = self.dispatch
         return (x_dtype == torch.bfloat16 and w_dtype == torch.bfloat16
                 and out_dtype in (torch.bfloat16, torch.float32)
-                and M >= d.tiled_stream_rows and N * K <= d.tiled_stream_weight
-                and self.lib.ts_gemm_tiled_fits(M, N, K, 0) == 1)
+                and self.lib.ts_gemm_tiled_fits(M, N, K, 0) == 1
+                and (M >= d.tiled_stream_rows and N * K <= d.tiled_plain_weight
+                     or M >= d.library_rows
+                     and self.lib.ts_gemm_tiled_ahead(M, N, K, _TYPE_CODE[out_dtype]) == 1))
 
-    def _library_ok(self, x, weight, out_dtype=None):
+    def _library_ok(self, x, weight, pair=False):
         if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
             return False
-        return self._library_rows(x.shape[0], weight.shape[0], weight.shape[1])
+        return self._library_rows(x.shape[0], weight.shape[0], weight.shape[1],
+                                  weight.numel() if pair else 0)
 
     def large_weight_choices(self):
         """Row counts from which products with a large weight may go to the library, for the
@@ -427,12 +434,16 @@ class HipOps:
         self._large_undecided = set()
         self._large_trial = None
 
-    def _library_rows(self, M, N, K):
-        """Whether a bfloat16 product of M rows with a weight [N, K] is the library's."""
+    def _library_rows(self, M, N, K, pair=0):
+        """Whether a bfloat16 product of M rows with a weight [N, K] is the library's; `pair`:
+        the elements of a stacked gate/up weight whose SiLU-multiply belongs to the product."""
         d = self.dispatch
         if M >= d.library_rows:
             return True
-        if M >= d.library_rows_head and N >= d.head_columns:
+        if pair:
+            if M >= d.library_rows_pair and pair > d.pair_head_weight:
+                return True
+        elif M >= d.library_rows_head and N >= d.head_columns:
             return True
         if N * K > d.large_weight:
             rows = self._large_rows.get((N, K))
@@ -486,7 +497,7 @@ class HipOps:
             return PreparedRows(rows, sumsq, sumsq.shape[0], hint)
         parts = self.lib.ts_gemm_tail_parts(M, N)
         if hint.weight.shape[1] != N or self._library_rows(M, N, K) \
-                or self._library_rows(M, next_n, N) \
+                or self._library_rows(M, next_n, N, hint.weight.numel() if hint.silu_mul else 0) \
                 or self.lib.ts_gemm_tail_fits(M, N, K) != 1 \
                 or self.lib.ts_gemm_scaled_fits(M, next_n, N, int(hint.silu_mul), parts) != 1:
             return None
@@ -503,7 +514,7 @@ class HipOps:
         and product behind it, are the LDS-tiled kernel's tail and scaled forms."""
         d = self.dispatch
         if M < d.tiled_stream_rows or hint.weight.shape[1] != N \
-                or N * K > d.tiled_stream_weight or hint.weight.numel() > d.tiled_pair_weight:
+                or max(N * K, hint.weight.numel()) > d.tiled_stream_weight:
             return False
         next_n = hint.weight.shape[0] // 2 if hint.silu_mul else hint.weight.shape[0]
         return (self.lib.ts_gemm_tiled_tail_fits(M, N, K) == 1
@@ -521,7 +532,8 @@ class HipOps:
             return None
         next_n = hint.weight.shape[0] // 2 if hint.silu_mul else hint.weight.shape[0]
         parts = self.lib.ts_gemm_tail_parts(M, N)
-        if self._library_rows(M, N, K) or self._library_rows(M, next_n, N) \
+        if self._library_rows(M, N, K) \
+                or self._library_rows(M, next_n, N, hint.weight.numel() if hint.silu_mul else 0) \
                 or self.lib.ts_gemm_tail_merged_fits(M, N, a.nq, a.hd) != 1 \
                 or self.lib.ts_gemm_scaled_fits(M, next_n, N, int(hint.silu_mul), parts) != 1:
             return None
@@ -616,7 +628,7 @@ class HipOps:
         if self._tiled_pair_ok(x, weight, out_dtype):
             return self.gemm_tiled(x, weight, out_dtype, pair=True, limit=limit, act=act)
         if (self._mfma_ok(x, weight) and out_dtype == torch.bfloat16
-                and not self._library_ok(x, weight, out_dtype)):
+                and not self._library_ok(x, weight, pair=True)):
             out = torch.empty(M, inner, dtype=out_dtype, device=self.device)
             self._call(self.lib.ts_gemm_mfma_bf16, _ptr(x), _ptr(weight), _ptr(out),
                        _TYPE_CODE[out_dtype], M, inner, K, 1, self._unit(limit, act), self._stream())
