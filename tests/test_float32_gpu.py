@@ -162,3 +162,34 @@ def test_product_rounds_no_more_than_short_chains_do(gpu_device, N, K, M):
     got = ops.linear(x.to(gpu_device), w.to(gpu_device), torch.float32).double().cpu()
     bound = 0.45 * 2.0 ** -24 * (8.5 + K / 256) ** 0.5 * 1.1
     assert (got - want).norm() <= bound * want.norm()
+
+
+@pytest.mark.parametrize("K", [64, 192, 1088])
+@pytest.mark.parametrize("M", [1, 17, 33, 64, 65, 200, 513])
+@pytest.mark.parametrize("N", [3, 130, 1100])
+def test_products_of_numbers_cut_in_three_parts(gpu_device, M, N, K):
+    """Runs that are empty or shorter than others, edges of every tile; results are not off to one
+    side: the mean error of M N elements, each rounded by itself, is within five standard errors."""
+    ops = load_hip_ops(gpu_device)
+    x, w = rand((M, K), 20).to(gpu_device), (rand((N, K), 21) * 0.05).to(gpu_device)
+    want = x.double() @ w.double().T
+    off = ops.linear(x, w, torch.float32).double() - want
+    # a rounding of each of K / 32 sums in a run and of five sums of runs, three standard deviations
+    # of a normal number times sqrt(K) 0.05, the largest of M N (less than 2^20) such
+    assert float(off.abs().max()) <= 2.0 ** -24 * (K / 256 + 5) * 5.0 * K ** 0.5 * 0.05
+    assert abs(float(off.mean())) <= 5.0 * float(off.pow(2).mean().sqrt()) / (M * N) ** 0.5 + 1e-12
+
+
+@pytest.mark.parametrize("M", [9, 40, 70, 300])
+def test_products_with_numbers_that_have_no_three_parts(gpu_device, M):
+    """Infinities, NaN and numbers that bfloat16 rounds to an infinity: results as float32 has them."""
+    ops = load_hip_ops(gpu_device)
+    x, w = rand((M, 1024), 22), rand((300, 1024), 23)
+    x[3, 5], x[4, 7], w[9, 100], x[6, 100], x[8, 2] = float("inf"), float("nan"), -3.4e38, 1.5, 3.402e38
+    x[7], w[:, 2] = 0.0, 0.25
+    want = (x.double() @ w.double().T).float()
+    out = ops.linear(x.to(gpu_device), w.to(gpu_device), torch.float32).cpu()
+    assert torch.equal(torch.isnan(out), torch.isnan(want))
+    assert torch.equal(torch.isinf(out), torch.isinf(want))
+    fine = torch.isfinite(want)
+    torch.testing.assert_close(out[fine], want[fine], rtol=1e-5, atol=1e-3)

@@ -1,6 +1,7 @@
 // C[M,N] = A[M,K] * W[N,K]^T in float32: float32 operands (bfloat16 ones are widened), float32
 // products and sums, no reduced-precision mode.  This is the product of the float32 path and of
-// any bfloat16 run whose weights are held in 32-bit.
+// any bfloat16 run whose weights are held in 32-bit; where both operands are float32 and K is a
+// multiple of 64, gemm_f32_split.hip takes it.
 //
 // Every output element adds its K products in an order fixed by K alone, so its value does not
 // depend on which other rows are in the call nor on the kernel that the number of rows chooses.
@@ -11,7 +12,10 @@
 // order.  Chains of eight products and not of a stretch's 64, because their roundings are what an
 // element's error mostly is: 9.6e-8 of the result at K = 1,024 against 1.58e-7, 1.1e-7 against
 // 1.6e-7 at 2,048, for 4 to 10 % of the tiles' time.  Another K adds in index order in one accumulator.
+#include <type_traits>
+
 #include "common.h"
+#include "gemm_f32_split.h"
 
 constexpr int kTile = 64;   // output tile edge per workgroup
 constexpr int kStep = 16;   // K elements staged per iteration
@@ -336,6 +340,9 @@ static int launch_tile(const TA* A, const TW* W, TC* C, int M, int N, int K, hip
 
 template <typename TA, typename TW, typename TC>
 static int launch_f32(const TA* A, const TW* W, TC* C, int M, int N, int K, hipStream_t stream) {
+  if constexpr (std::is_same_v<TA, float> && std::is_same_v<TW, float> && std::is_same_v<TC, float>) {
+    if (gemm_f32_split_fits(K)) return gemm_f32_split_launch(A, W, C, M, N, K, stream);
+  }
   const dim3 block(kRuns * kWave), grid((N + 15) / 16);
   if (M <= 16) {
     hipLaunchKernelGGL((gemm_f32_rows_kernel<TA, TW, TC, 1>), grid, block, 0, stream, A, W, C, M, N, K);
