@@ -60,6 +60,14 @@ class Dispatch:
     #: form) instead of the library's product and a norm kernel.
     tiled_stream_rows: int = 512
     tiled_stream_weight: int = 1 << 28
+    #: Weights of `tiled_stream_few_weight` to `large_weight` elements take it from fewer rows: a
+    #: step of the 0.6B shape with 300 tokens 2,117 -> 2,042 us on the GPU, with 128 1,738 -> 2,116
+    #: (N = 1,024 fills few units), but in an eager step, where two norm kernels and three library
+    #: calls a layer held the host up, 3,400 -> 2,050 and 2,150.  (Fewer rows leave the tiles of 128
+    #: half empty; smaller weights keep the separate kernels, through which portions below 512 rows
+    #: of small models are tested.)
+    tiled_stream_few_rows: int = 96
+    tiled_stream_few_weight: int = 1 << 20
     #: Plain products: from `tiled_stream_rows` rows and up to so many elements the tiled
     #: kernel's (the same time on the GPU, 22.5 against 22.4 us for the 0.6B model's qkv at 2,048
     #: rows, and a fifth of the library call's 20 to 30 us on the host, which the GPU waits for

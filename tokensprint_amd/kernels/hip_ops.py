@@ -124,6 +124,8 @@ class HipOps:
         # for the vendor library's algorithms that want scratch memory during a product
         self._library_workspace = torch.empty(64 << 20, dtype=torch.uint8, device=self.device)
         self._timed_plans = False
+        # which kernels end a sub-layer, by sizes, as `_stream_routes_of` (a dispatch table) has it
+        self._stream_routes, self._stream_routes_of = {}, self.dispatch
         self._staging, self._staging_turn = [None] * 4, -1      # pinned buffers of _upload_ints
         # products of few rows with large weights: ours or the library's, per weight shape
         # (see large_weight_choices)
@@ -159,7 +161,7 @@ class HipOps:
         # (written for the case that all is well, which is every call of a working engine:
         # this runs several times before every kernel)
         try:
-            ok = t.device == self.device and t.is_contiguous()
+            ok = t.get_device() == self._device_index and t.is_contiguous()
         except AttributeError:
             if isinstance(t, UnmergedRows):
                 raise TypeError(f"{name}: an unmerged attention output; this call does not "
@@ -170,7 +172,7 @@ class HipOps:
         if ok and ndim is not None:
             ok = t.dim() == ndim
         if ok and shape is not None:
-            ok = t.shape == tuple(shape)
+            ok = t.shape == (shape if shape.__class__ is tuple else tuple(shape))
         if ok:
             return t
         if t.device != self.device:
@@ -483,24 +485,19 @@ class HipOps:
         N = weight.shape[0]
         if weight.shape[1] != K:
             raise ValueError(f"linear_into_stream: x has {K} columns, weight has {weight.shape[1]}")
-        next_n = hint.weight.shape[0] // 2 if hint.silu_mul else hint.weight.shape[0]
-        if self._tiled_stream_ok(M, N, K, hint):
+        tiled, parts = self._stream_route(M, N, K, hint)
+        if parts == 0:
+            return None
+        if tiled:
             # a prompt's portion: the LDS-tiled product in its tail form
             self._check("resid", resid, torch.float32, shape=(M, N))
             self._check("norm weight", hint.norm_weight, torch.float32, shape=(N,))
             rows = torch.empty(M, N, dtype=torch.bfloat16, device=self.device)
-            sumsq = torch.empty(self.lib.ts_gemm_tiled_tail_parts(N), M, dtype=torch.float32,
-                                device=self.device)
+            sumsq = torch.empty(parts, M, dtype=torch.float32, device=self.device)
             self._call(self.lib.ts_gemm_tiled_tail_bf16, _ptr(x), _ptr(weight), _ptr(resid),
                        _ptr(hint.norm_weight), _ptr(rows), _ptr(sumsq), M, N, K, 0,
                        self._stream())
-            return PreparedRows(rows, sumsq, sumsq.shape[0], hint)
-        parts = self.lib.ts_gemm_tail_parts(M, N)
-        if hint.weight.shape[1] != N or self._library_rows(M, N, K) \
-                or self._library_rows(M, next_n, N, hint.weight.numel() if hint.silu_mul else 0) \
-                or self.lib.ts_gemm_tail_fits(M, N, K) != 1 \
-                or self.lib.ts_gemm_scaled_fits(M, next_n, N, int(hint.silu_mul), parts) != 1:
-            return None
+            return PreparedRows(rows, sumsq, parts, hint, tiled=True)
         self._check("resid", resid, torch.float32, shape=(M, N))
         self._check("norm weight", hint.norm_weight, torch.float32, shape=(N,))
         rows = torch.empty(M, N, dtype=torch.bfloat16, device=self.device)
@@ -509,12 +506,44 @@ class HipOps:
                    _ptr(hint.norm_weight), _ptr(rows), _ptr(sumsq), M, N, K, self._stream())
         return PreparedRows(rows, sumsq, parts, hint)
 
+    def _stream_route(self, M, N, K, hint):
+        """(whether it is the LDS-tiled product's tail form, slices of a row's sum of squares) for
+        the product that ends a sub-layer and the hinted norm and product behind it; no slices:
+        separate kernels.  Sizes and the dispatch table decide (and, for large weights, the
+        warm-up's choice), so the answer for small weights is kept by sizes: a step asks for every
+        layer, in half a dozen calls into the library."""
+        wn = hint.weight
+        small = N * K <= self.dispatch.large_weight and wn.numel() <= self.dispatch.large_weight
+        key = (M, N, K, wn.shape, hint.silu_mul)
+        if small:
+            if self._stream_routes_of is not self.dispatch or len(self._stream_routes) > 4096:
+                self._stream_routes, self._stream_routes_of = {}, self.dispatch
+            found = self._stream_routes.get(key)
+            if found is not None:
+                return found
+        next_n = wn.shape[0] // 2 if hint.silu_mul else wn.shape[0]
+        if self._tiled_stream_ok(M, N, K, hint):
+            route = True, self.lib.ts_gemm_tiled_tail_parts(N)
+        else:
+            parts = self.lib.ts_gemm_tail_parts(M, N)
+            if wn.shape[1] != N or self._library_rows(M, N, K) \
+                    or self._library_rows(M, next_n, N, wn.numel() if hint.silu_mul else 0) \
+                    or self.lib.ts_gemm_tail_fits(M, N, K) != 1 \
+                    or self.lib.ts_gemm_scaled_fits(M, next_n, N, int(hint.silu_mul), parts) != 1:
+                parts = 0
+            route = False, parts
+        if small:
+            self._stream_routes[key] = route
+        return route
+
     def _tiled_stream_ok(self, M, N, K, hint):
         """Whether the product [M, K] x [N, K] that ends a sub-layer, and the hinted norm
         and product behind it, are the LDS-tiled kernel's tail and scaled forms."""
         d = self.dispatch
-        if M < d.tiled_stream_rows or hint.weight.shape[1] != N \
-                or max(N * K, hint.weight.numel()) > d.tiled_stream_weight:
+        least, largest = sorted((N * K, hint.weight.numel()))
+        if M < (d.tiled_stream_few_rows if largest <= d.large_weight and least >= d.tiled_stream_few_weight
+                else d.tiled_stream_rows) \
+                or hint.weight.shape[1] != N or largest > d.tiled_stream_weight:
             return False
         next_n = hint.weight.shape[0] // 2 if hint.silu_mul else hint.weight.shape[0]
         return (self.lib.ts_gemm_tiled_tail_fits(M, N, K) == 1
@@ -562,7 +591,7 @@ class HipOps:
         if out_dtype not in (torch.bfloat16, torch.float32) or (silu_mul and out_dtype != torch.bfloat16):
             raise ValueError(f"norm_linear: prepared rows cannot give {out_dtype}")
         out = torch.empty(M, N, dtype=out_dtype, device=self.device)
-        if M >= self.dispatch.tiled_stream_rows:      # prepared by the tiled tail form
+        if prepared.tiled:
             self._call(self.lib.ts_gemm_tiled_scaled_bf16, _ptr(prepared.rows),
                        _ptr(prepared.sumsq), prepared.slices, c_float(eps), _ptr(weight),
                        _ptr(out), _TYPE_CODE[out_dtype], M, N, K, int(silu_mul), 0, self._stream())
@@ -916,10 +945,19 @@ class HipOps:
         # (scores with extras: those of these kernels that know them take pages of a power of
         # two from 16)
         page16 = a.page_size >= 16 and a.page_size & (a.page_size - 1) == 0
-        if (not extras or page16) and self._prefill_tiles(batch, a.nkv, group) is not None:
-            tiles16 = sum(-(-n // tokens_per_tile) for n in batch.q_lens)
-            tpw = self.lib.ts_attention_prefill_tiles(a.hd, a.page_size, tiles16,
-                                                      a.nkv * head_blocks)
+        d = self.dispatch
+        # (the same for every layer of a step)
+        key = ("prefill", group, a.nkv, a.hd, a.page_size, d.portion_tiles, d.portion_tokens,
+               d.single_token_tiles)
+        if key not in batch.plans:
+            tpw = 0
+            if self._prefill_tiles(batch, a.nkv, group) is not None:
+                tiles16 = sum(-(-n // tokens_per_tile) for n in batch.q_lens)
+                tpw = self.lib.ts_attention_prefill_tiles(a.hd, a.page_size, tiles16,
+                                                          a.nkv * head_blocks)
+            batch.plans[key] = tpw
+        tpw = batch.plans[key]
+        if (not extras or page16) and tpw:
             tiles_dev, num_tiles = self._attention_tiles(batch, tokens_per_tile * tpw,
                                                          longest_first=True)
             m.tiles, m.num_tiles, m.tiles_per_wave = tiles_dev.data_ptr(), num_tiles, tpw
@@ -938,7 +976,6 @@ class HipOps:
         max_chunks = max(1, -(-span // chunk))
         # few tiles (decode): a workgroup per tile and chunk, its waves share the chunk;
         # many tiles (prompts): a wavefront per tile walks its keys
-        d = self.dispatch
         cooperative = items <= d.cooperative_items
         splits = min(max_chunks, max(1, (d.cooperative_workgroups if cooperative
                                          else d.per_wave_workgroups) // items))

@@ -30,13 +30,14 @@ class PreparedRows:
     not yet divided by the row's root mean square) and `sumsq`, the rows' sums of squares
     in `slices` slices of columns, laid out as the producing kernel and its counterpart
     agree ([M, slices rounded up to four] from the kernels for few rows, [slices, M] from
-    the tiled product's).  Stands where the stream's `delta` does, and only the provider's
-    `norm_linear` with the hinted norm and weight takes it."""
+    the tiled product's, `tiled`).  Stands where the stream's `delta` does, and only the
+    provider's `norm_linear` with the hinted norm and weight takes it."""
 
     rows: torch.Tensor
     sumsq: torch.Tensor
     slices: int
     hint: NormHint
+    tiled: bool = False
 
 
 @dataclass(frozen=True)
