@@ -161,3 +161,20 @@ def test_add_norm_and_shift(gpu_device, width, entries, delta_type):
         want = ops.norm_token_shift(b, norm, 1e-6, shift, batch, other, torch.bfloat16)
         assert not got.isnan().any()
         assert torch.equal(a, b) and torch.equal(got, want) and torch.equal(one[1:-1], other[1:-1])
+
+
+@pytest.mark.parametrize("T, n_a, k_a, n_g, k_g, col", [(1, 16, 32, 16, 32, 0), (8, 512, 64, 1024, 64, 8),
+                                                        (17, 70, 96, 5, 64, 3), (300, 512, 64, 1000, 32, 4)])
+def test_low_rank_pair(T, n_a, k_a, n_g, k_g, col):
+    """Two products over columns of float32 rows (also where they do not begin on 16 bytes) against
+    copies of the columns and products of their own."""
+    ops = load_hip_ops("cuda:0")
+    ld = col + k_a + k_g + 3
+    x = rand((T, ld), 90)
+    w_a, w_g = (rand((n, k), 91, 0.1).to(torch.bfloat16) for n, k in ((n_a, k_a), (n_g, k_g)))
+    z, gate = ops.low_rank_pair(x, col, w_a, col + k_a, w_g, torch.bfloat16)
+    for got, at, w in ((z, col, w_a), (gate, col + k_a, w_g)):
+        want = x[:, at:at + w.shape[1]].to(torch.bfloat16).double() @ w.double().T
+        # float32 sums of K exact products: K roundings at most of partial sums below |x| |w|
+        bound = x[:, at:at + w.shape[1]].abs().double() @ w.abs().double().T * w.shape[1] * 2.0 ** -24
+        assert ((got.double() - want).abs() <= bound + 1e-30).all()

@@ -1792,6 +1792,25 @@ class HipOps:
         return out
 
     # ------------------------------------------------------------ latent attention
+    def low_rank_pair(self, x, col_a, w_a, col_g, w_g, act_dtype):
+        """The second steps of two low-rank projections, whose first steps are the columns of x
+        (float32) from `col_a` and `col_g`: ([T, Na], [T, Ng]) in float32, the columns rounded to
+        `act_dtype` first."""
+        self._check("x", x, torch.float32, ndim=2)
+        self._check("w_a", w_a, self._FLOATS, ndim=2)
+        self._check("w_g", w_g, self._FLOATS, ndim=2)
+        (n_a, k_a), (n_g, k_g), T = w_a.shape, w_g.shape, x.shape[0]
+        if act_dtype is torch.bfloat16 and w_a.dtype is torch.bfloat16 and w_g.dtype is torch.bfloat16 \
+                and T <= 65535 * 16 and self.lib.ts_low_rank_pair_fits(k_a, k_g) == 1 \
+                and (w_a.data_ptr() | w_g.data_ptr()) % 16 == 0:
+            out_a = torch.empty(T, n_a, dtype=torch.float32, device=self.device)
+            out_g = torch.empty(T, n_g, dtype=torch.float32, device=self.device)
+            self._call(self.lib.ts_low_rank_pair, _ptr(x), x.shape[1], T, int(col_a), _ptr(w_a), n_a,
+                       k_a, _ptr(out_a), int(col_g), _ptr(w_g), n_g, k_g, _ptr(out_g), self._stream())
+            return out_a, out_g
+        return (self.linear(self.take_columns(x, col_a, k_a, act_dtype), w_a, torch.float32),
+                self.linear(self.take_columns(x, col_g, k_g, act_dtype), w_g, torch.float32))
+
     def _check_latent(self, cache, table, batch, dl):
         self._check("latent pages", cache.k_pages, self._FLOATS,
                     shape=(cache.num_pages, cache.page_size, dl))

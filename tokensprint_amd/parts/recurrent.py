@@ -239,12 +239,16 @@ class GatedDeltaRule(Mixer):
         b_col, state = self.channels, cache.states[self.state_name]
         if self.per_channel:
             # the second steps of the two low-rank projections, on the first steps' columns
-            a1 = ops.take_columns(proj, b_col + H, self.decay_rank, self.ctx.dtype)
-            g1 = ops.take_columns(proj, b_col + H + self.decay_rank, self.gate_rank,
-                                  self.ctx.dtype)
-            z = ops.linear(a1, self.w_a2, torch.float32)          # [T, heads * dim]
-            gate, gate_col = ops.linear(g1, self.w_g2, torch.float32), 0
-            z_col = 0
+            # (z [T, heads * dim])
+            a_col, g_col = b_col + H, b_col + H + self.decay_rank
+            if hasattr(ops, "low_rank_pair"):
+                z, gate = ops.low_rank_pair(proj, a_col, self.w_a2, g_col, self.w_g2, self.ctx.dtype)
+            else:
+                z = ops.linear(ops.take_columns(proj, a_col, self.decay_rank, self.ctx.dtype),
+                               self.w_a2, torch.float32)
+                gate = ops.linear(ops.take_columns(proj, g_col, self.gate_rank, self.ctx.dtype),
+                                  self.w_g2, torch.float32)
+            z_col = gate_col = 0
         else:
             z, z_col = proj, b_col + H
             gate, gate_col = proj, b_col + 2 * H
