@@ -54,6 +54,13 @@ class Dispatch:
     #: wait for `tiled_pair_rows_large` rows.
     tiled_pair_weight: int = 1 << 27
     tiled_pair_rows_large: int = 512
+    #: From `tiled_fill_rows` rows of weights above `large_weight` elements, gate/up products and
+    #: the forms below also have to fill so many per cent of their tiles' rounds
+    #: (`ts_gemm_tiled_fill`): gate/up products at 23 row counts from 520 to 3,600 take 0.90 of the
+    #: library's and the SiLU kernel's time in the mean from 65 per cent on, 1.04 at most, and 1.03
+    #: below, up to 1.18; plain products 0.97 and 1.07 of the library's, without the norm kernel.
+    tiled_fill: int = 65
+    tiled_fill_rows: int = 256
     #: rows from which, and elements of a weight [N, K] up to which, the product that ends a
     #: sub-layer is the LDS-tiled kernel's tail form (it adds itself into the float32 stream
     #: and prepares the rows for the norm behind it, whose product then takes the scaled
@@ -63,10 +70,10 @@ class Dispatch:
     #: Weights of `tiled_stream_few_weight` to `large_weight` elements take it from fewer rows: a
     #: step of the 0.6B shape with 300 tokens 2,117 -> 2,042 us on the GPU, with 128 1,738 -> 2,116
     #: (N = 1,024 fills few units), but in an eager step, where two norm kernels and three library
-    #: calls a layer held the host up, 3,400 -> 2,050 and 2,150.  (Fewer rows leave the tiles of 128
-    #: half empty; smaller weights keep the separate kernels, through which portions below 512 rows
+    #: calls a layer held the host up, 3,400 -> 2,050 and 2,150.  (Fewer rows leave nearly half of a tile
+    #: of 128 empty; smaller weights keep the separate kernels, through which portions below 512 rows
     #: of small models are tested.)
-    tiled_stream_few_rows: int = 96
+    tiled_stream_few_rows: int = 72
     tiled_stream_few_weight: int = 1 << 20
     #: Plain products: from `tiled_stream_rows` rows and up to so many elements the tiled
     #: kernel's (the same time on the GPU, 22.5 against 22.4 us for the 0.6B model's qkv at 2,048
