@@ -67,7 +67,8 @@ class Dispatch:
     #: form) instead of the library's product and a norm kernel.
     tiled_stream_rows: int = 512
     tiled_stream_weight: int = 1 << 28
-    #: Weights of `tiled_stream_few_weight` to `large_weight` elements take it from fewer rows: a
+    #: Weights of `tiled_stream_few_weight` to `large_weight` elements take it from fewer rows in
+    #: an eager step (captured ones, of up to 256 single tokens, do not: 4.99 against 4.77 ms): a
     #: step of the 0.6B shape with 300 tokens 2,117 -> 2,042 us on the GPU, with 128 1,738 -> 2,116
     #: (N = 1,024 fills few units), but in an eager step, where two norm kernels and three library
     #: calls a layer held the host up, 3,400 -> 2,050 and 2,150.  (Fewer rows leave nearly half of a tile

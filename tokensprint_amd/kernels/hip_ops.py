@@ -516,7 +516,9 @@ class HipOps:
         layer, in half a dozen calls into the library."""
         wn = hint.weight
         small = N * K <= self.dispatch.large_weight and wn.numel() <= self.dispatch.large_weight
-        key = (M, N, K, wn.shape, hint.silu_mul)
+        # a step that is captured, or run to be, does not wait for the host
+        eager = not (self._timed_plans or torch.cuda.is_current_stream_capturing())
+        key = (M, N, K, wn.shape, hint.silu_mul, eager)
         if small:
             if self._stream_routes_of is not self.dispatch or len(self._stream_routes) > 4096:
                 self._stream_routes, self._stream_routes_of = {}, self.dispatch
@@ -524,7 +526,7 @@ class HipOps:
             if found is not None:
                 return found
         next_n = wn.shape[0] // 2 if hint.silu_mul else wn.shape[0]
-        if self._tiled_stream_ok(M, N, K, hint):
+        if self._tiled_stream_ok(M, N, K, hint, eager):
             route = True, self.lib.ts_gemm_tiled_tail_parts(N)
         else:
             parts = self.lib.ts_gemm_tail_parts(M, N)
@@ -538,13 +540,13 @@ class HipOps:
             self._stream_routes[key] = route
         return route
 
-    def _tiled_stream_ok(self, M, N, K, hint):
+    def _tiled_stream_ok(self, M, N, K, hint, eager=True):
         """Whether the product [M, K] x [N, K] that ends a sub-layer, and the hinted norm
         and product behind it, are the LDS-tiled kernel's tail and scaled forms."""
         d = self.dispatch
         least, largest = sorted((N * K, hint.weight.numel()))
-        if M < (d.tiled_stream_few_rows if largest <= d.large_weight and least >= d.tiled_stream_few_weight
-                else d.tiled_stream_rows) \
+        few = eager and largest <= d.large_weight and least >= d.tiled_stream_few_weight
+        if M < (d.tiled_stream_few_rows if few else d.tiled_stream_rows) \
                 or hint.weight.shape[1] != N or largest > d.tiled_stream_weight:
             return False
         next_n = hint.weight.shape[0] // 2 if hint.silu_mul else hint.weight.shape[0]
