@@ -193,3 +193,17 @@ def test_products_with_numbers_that_have_no_three_parts(gpu_device, M):
     assert torch.equal(torch.isinf(out), torch.isinf(want))
     fine = torch.isfinite(want)
     torch.testing.assert_close(out[fine], want[fine], rtol=1e-5, atol=1e-3)
+
+
+@pytest.mark.parametrize("M", [1, 20, 40, 64, 70, 300, 600])
+def test_a_row_of_a_single_product(gpu_device, M):
+    """Nothing averages out: what is left out of a product of parts, 2^-25 of it twice at most, and
+    one rounding, 2^-24, with a sixteenth of that for the roundings of the smaller parts."""
+    ops = load_hip_ops(gpu_device)
+    g = torch.Generator().manual_seed(24)
+    x, w = torch.zeros(M, 1088), rand((1100, 1088), 25)
+    x[torch.arange(M), torch.randint(0, 1088, (M,), generator=g)] = 1 + torch.rand(M, generator=g)
+    w[7] = x[M - 1, x[M - 1].argmax()] = 1 + 2.0 ** -8 - 2.0 ** -23       # the parts behind the first are largest
+    want = x.double() @ w.double().T
+    got = ops.linear(x.to(gpu_device), w.to(gpu_device), torch.float32).double().cpu()
+    assert ((got - want).abs() <= 2.1 * 2.0 ** -24 * want.abs()).all()

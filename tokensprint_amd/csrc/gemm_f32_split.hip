@@ -1,31 +1,38 @@
 // C[M,N] = A[M,K] W[N,K]^T in float32 with float32 precision, on the bfloat16 matrix cores, for K a
 // multiple of 64.
 //
-// A float32 number is the exact sum of three bfloat16 numbers: a0 = bf16(a), a1 the upper eight bits
-// of a - a0, a2 the rest (both differences are exact: 24 bits are three times 8, with signs).  Of
-// the nine products of a pair's parts six are made, (2,0) (0,2) (1,1) (1,0) (0,1) (0,0); what is left
-// out is below 2^-24 of the pair's product, either way.  Products of parts are exact in the matrix
+// The splitting of an operand into words of lower precision and their products in descending order
+// of size are Dekker's (A floating-point technique for extending the available precision, 1971),
+// with bfloat16 words as in Henry, Tang and Heinecke (Leveraging the bfloat16 artificial
+// intelligence datatype for higher-precision computations, 2019).  A float32 number is the exact
+// sum of three bfloat16 numbers: a0 = bf16(a), a1 = bf16(a - a0), a2 the rest (both differences are
+// exact, and a2 has at most seven bits; below 2^-110 the last bits of a2 are below bfloat16's
+// smallest number and are lost).  Of the nine products of a pair's parts six are made: (2,0) (0,2)
+// (1,1) (1,0) (0,1) and (0,0).  Of those left out, (1,2) and (2,1) are at most 2^-25 of the pair's
+// product each, to either side, (2,2) is far smaller.  (With a1 cut off instead of rounded they were
+// up to 2^-24 each, both to the side of the product.)  Products of parts are exact in the matrix
 // core, and v_mfma_f32_16x16x32_bf16 adds 32 of them with little more than one rounding, where the
 // float32 instruction rounds at every one.  That rounding is to one side (a sum's errors had a mean
 // of 0.4 of themselves, the same for all rows, and a model's logits were 20 % further off), so of
-// every second 32 of K the negative product is made and subtracted.
-// Error, of the result's root mean square, beside chains of eight float32 products (gemm_fma.hip):
-// K = 64 4.8e-8 / 7.2e-8, 1,024 7.5e-8 / 9.6e-8, 3,072 9.3e-8 / 1.21e-7, 12,288 1.44e-7 / 1.96e-7;
-// logits of the 0.6B model behind 501 tokens, eight seeds, 1.32e-6 / 1.34e-6.
+// every second 32 of K the negative product is made and subtracted; and (0,0), in whose sum it would
+// be largest, is added to the five others' outside the matrix core, to nearest.
+// Error, of the result's root mean square in 2^-24, beside chains of eight float32 products
+// (gemm_fma.hip): K = 64 0.80 / 1.24, 1,024 1.26 / 1.61, 3,072 1.55 / 2.05, 12,288 2.38 / 3.28.
+// A row of a single product, in 2^-24 of it: root mean square 0.43 / 0.43, at most 1.5 / 1.0 (the
+// two products left out, where one multiply-add rounds once).
 //
-// Sums: K is cut into eight runs of whole stretches of 64; a run adds the sums of its 32s (six
-// instructions from zero, in the order above), the result the sums of pairs of runs, in order.
-// Every kernel here adds in that order, so an element depends on neither the other rows of a call
-// nor their number.
+// Sums: K is cut into eight runs of whole stretches of 64; a run adds the sums of its 32s (five
+// instructions from zero, in the order above, and the sixth's), the result the sums of pairs of runs,
+// in order.  Every kernel here adds in that order, so an element depends on neither the other rows
+// of a call nor their number.
 // Where a result is not finite, it may be because a part was not (infinities, and numbers that
 // bfloat16 rounds to one, leave a NaN behind): such an element is made again, in float32, one
 // product after the other.
 //
 // What bounds it: LDS, the matrix cores (six instructions of 16 cycles for 32 of K against eight of
 // 32) and what cuts operands in parts, 5.5 instructions a number, one after the other in most of a
-// turn.  501 rows, before (float32 instructions) and now, us: 6,144 x 1,024 72.0 -> 48.0, 4,096 x
-// 1,024 50.1 -> 36.7, 1,024 x 2,048 26.7 -> 22.9, 1,024 x 3,072 37.2 -> 32; 2,048 rows of 4,096 x
-// 4,096 793 -> 403.  (The wavefronts of a SIMD cutting and multiplying in turns, or every one for
+// turn.  501 rows, before (float32 instructions) and now, us: 6,144 x 1,024 71 -> 49, 4,096 x 1,024
+// 50 -> 36, 1,024 x 2,048 27 -> 25, 1,024 x 3,072 38 -> 35; 2,048 rows of 4,096 x 4,096 794 -> 409.  (The wavefronts of a SIMD cutting and multiplying in turns, or every one for
 // itself without LDS in tiles of 32 x 64, is no faster; nor are float32 instructions with operands
 // straight into LDS, 65.9 for the first.)
 #include "gemm_f32_split.h"
@@ -37,26 +44,27 @@ typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
+constexpr f32x4 kZero = {0.f, 0.f, 0.f, 0.f};
 constexpr int kRuns = 8;            // of K
 constexpr int kTerms = 6;
+constexpr int kSmall = kTerms - 1;  // that are added in the matrix core
 // parts of A and W that a term multiplies
-constexpr int kPartA[kTerms] = {2, 0, 1, 1, 0, 0}, kPartW[kTerms] = {0, 2, 1, 0, 1, 0};
+constexpr int kPartA[kSmall] = {2, 0, 1, 1, 0}, kPartW[kSmall] = {0, 2, 1, 0, 1};
 
-// Two numbers' parts, packed.  a0 is rounded; what is left has 16 bits, of which a1 takes the upper
-// eight as they stand.
+// Two numbers' parts, packed.
 __device__ __forceinline__ void split2(float x, float y, unsigned (&part)[3]) {
   typedef float f32x2 __attribute__((ext_vector_type(2)));
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  const unsigned head = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{x, y}, bf16x2));
-  auto upper = [](float v) { return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, v) & 0xffff0000u); };
-  auto both = [](float low, float high) {
-    return __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, high), __builtin_bit_cast(unsigned, low), 0x07060302u);
+  auto rounded = [](float a, float b) {
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{a, b}, bf16x2));
   };
-  const float x1 = x - __builtin_bit_cast(float, head << 16);
-  const float y1 = y - __builtin_bit_cast(float, head & 0xffff0000u);
-  part[0] = head;
-  part[1] = both(x1, y1);
-  part[2] = both(x1 - upper(x1), y1 - upper(y1));
+  auto low = [](unsigned two) { return __builtin_bit_cast(float, two << 16); };
+  auto high = [](unsigned two) { return __builtin_bit_cast(float, two & 0xffff0000u); };
+  part[0] = rounded(x, y);
+  const float x1 = x - low(part[0]), y1 = y - high(part[0]);
+  part[1] = rounded(x1, y1);
+  const float x2 = x1 - low(part[1]), y2 = y1 - high(part[1]);
+  part[2] = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, y2), __builtin_bit_cast(unsigned, x2), 0x07060302u);
 }
 __device__ __forceinline__ void split(f32x4 v, u32x2 (&part)[3]) {
   unsigned low[3], high[3];
@@ -109,7 +117,7 @@ __global__ __launch_bounds__(kRuns* kWave) void gemm_f32_split_rows_kernel(Split
   for (int i = 0; i < MT; ++i) a_row[i] = a.a + (int64_t)min(16 * i + l, a.M - 1) * a.K + 8 * g;
   f32x4 sum[MT], w[2][4], x[2][MT][4];      // [set][2 step + half]
 #pragma unroll
-  for (int i = 0; i < MT; ++i) sum[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < MT; ++i) sum[i] = kZero;
   auto fetch = [&](int set, int k) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -128,10 +136,12 @@ __global__ __launch_bounds__(kRuns* kWave) void gemm_f32_split_rows_kernel(Split
 #pragma unroll
       for (int i = 0; i < MT; ++i) parts(x[set][i][2 * step], x[set][i][2 * step + 1], false, xp[i]);
 #pragma unroll
-      for (int t = 0; t < kTerms; ++t)
+      for (int t = 0; t < kSmall; ++t)
 #pragma unroll
         for (int i = 0; i < MT; ++i)
-          chain[i] = mfma(wp[kPartW[t]], xp[i][kPartA[t]], t ? chain[i] : f32x4{0.f, 0.f, 0.f, 0.f});
+          chain[i] = mfma(wp[kPartW[t]], xp[i][kPartA[t]], t ? chain[i] : kZero);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) chain[i] += mfma(wp[0], xp[i][0], kZero);
 #pragma unroll
       for (int i = 0; i < MT; ++i) sum[i] = step & 1 ? sum[i] - chain[i] : sum[i] + chain[i];
     }
@@ -194,7 +204,7 @@ __global__ __launch_bounds__(kRuns* kWave) void gemm_f32_split_kernel(SplitArgs 
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < TN; ++j) sum[i][j] = kZero;
   auto fetch = [](f32x4 (&to)[2], const float* from) {
     to[0] = *(const f32x4*)from;
     to[1] = *(const f32x4*)(from + 4);
@@ -228,13 +238,16 @@ __global__ __launch_bounds__(kRuns* kWave) void gemm_f32_split_kernel(SplitArgs 
             fetch(x[s][i0 + i], a_row[i0 + i] + ahead);
           }
 #pragma unroll
-          for (int t = 0; t < kTerms; ++t)
+          for (int t = 0; t < kSmall; ++t)
 #pragma unroll
             for (int i = 0; i < AT_ONCE; ++i)
 #pragma unroll
               for (int j = 0; j < TN; ++j)
-                chain[i][j] = mfma(wp[j][kPartW[t]], xp[i][kPartA[t]],
-                                   t ? chain[i][j] : f32x4{0.f, 0.f, 0.f, 0.f});
+                chain[i][j] = mfma(wp[j][kPartW[t]], xp[i][kPartA[t]], t ? chain[i][j] : kZero);
+#pragma unroll
+          for (int i = 0; i < AT_ONCE; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) chain[i][j] += mfma(wp[j][0], xp[i][0], kZero);
 #pragma unroll
           for (int i = 0; i < AT_ONCE; ++i)
 #pragma unroll
@@ -253,7 +266,7 @@ __global__ __launch_bounds__(kRuns* kWave) void gemm_f32_split_kernel(SplitArgs 
   // a thread takes four columns of a row
   for (int e = threadIdx.x; e < TM * TN * 64; e += kRuns * kWave) {
     const int block = e / 64, of = e % 64;
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    f32x4 v = kZero;
 #pragma unroll
     for (int r = 0; r < kRuns; r += 2) v += *place(r, block, of) + *place(r + 1, block, of);
     const int m = m0 + block / TN * 16 + of % 16, n = n0 + block % TN * 16 + of / 16 * 4;
@@ -351,7 +364,7 @@ __global__ __launch_bounds__(64 * GM * GN * G) void gemm_f32_split_tile_kernel(S
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) sums[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < TN; ++j) sums[i][j] = kZero;
   };
   auto gather = [&](f32x4 (&sums)[TM][TN], const f32x4 (&more)[TM][TN]) {
 #pragma unroll
@@ -379,18 +392,21 @@ __global__ __launch_bounds__(64 * GM * GN * G) void gemm_f32_split_tile_kernel(S
       fetch_piece(set ^ 1, t + 3, u);
     }
 #pragma unroll
-    for (int term = 0; term < kTerms; ++term)
+    for (int term = 0; term < kSmall; ++term)
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-          step[i][j] = mfma(wp[kPartW[term]][j], ap[kPartA[term]][i],
-                            term ? step[i][j] : f32x4{0.f, 0.f, 0.f, 0.f});
+          step[i][j] = mfma(wp[kPartW[term]][j], ap[kPartA[term]][i], term ? step[i][j] : kZero);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) step[i][j] += mfma(wp[0][j], ap[0][i], kZero);
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        const f32x4 more = G == 1 || t < mine ? step[i][j] : f32x4{0.f, 0.f, 0.f, 0.f};
+        const f32x4 more = G == 1 || t < mine ? step[i][j] : kZero;
         run[i][j] = set == 1 ? run[i][j] - more : run[i][j] + more;
       }
 #pragma unroll
