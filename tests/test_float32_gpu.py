@@ -2,6 +2,8 @@
 tiles, runs of K and key blocks: against float64, and a row the same to the bit however it is
 batched."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -9,6 +11,9 @@ from scenarios import paged_scenario
 from tokensprint_amd.kernels import load_hip_ops
 
 pytestmark = pytest.mark.gpu
+
+#: tiles of the product cut in parts; the first ones take 16, 32, ... rows at most
+TILES, ROW_TILES = 8, 2
 
 
 def rand(shape, seed, dtype=torch.float32):
@@ -168,7 +173,7 @@ def test_product_rounds_no_more_than_short_chains_do(gpu_device, N, K, M):
 @pytest.mark.parametrize("M", [1, 17, 33, 64, 65, 200, 513])
 @pytest.mark.parametrize("N", [3, 130, 1100])
 def test_products_of_numbers_cut_in_three_parts(gpu_device, M, N, K):
-    """Runs that are empty or shorter than others, edges of every tile; results are not off to one
+    """Runs that are empty or shorter than others; results are not off to one
     side: the mean error of M N elements, each rounded by itself, is within five standard errors."""
     ops = load_hip_ops(gpu_device)
     x, w = rand((M, K), 20).to(gpu_device), (rand((N, K), 21) * 0.05).to(gpu_device)
@@ -207,3 +212,45 @@ def test_a_row_of_a_single_product(gpu_device, M):
     want = x.double() @ w.double().T
     got = ops.linear(x.to(gpu_device), w.to(gpu_device), torch.float32).double().cpu()
     assert ((got - want).abs() <= 2.1 * 2.0 ** -24 * want.abs()).all()
+
+
+def by_tile(ops, x, w, tile, offset=0):
+    """The product by a named tile, into a buffer that begins `offset` floats behind 16 bytes."""
+    (M, K), N = x.shape, w.shape[0]
+    out = torch.full((M * N + 8,), 7.0, device=x.device)
+    p = [ctypes.c_void_p(t.data_ptr()) for t in (x, w, out[offset:])]
+    ops._call(ops.lib.ts_gemm_f32_split, *p, M, N, K, tile, ops._stream())
+    assert (out[:offset] == 7).all() and (out[offset + M * N:] == 7).all()
+    return out[offset:offset + M * N].view(M, N)
+
+
+@pytest.mark.parametrize("tile", range(1, TILES + 1))
+@pytest.mark.parametrize("K", [64, 192, 1088])
+@pytest.mark.parametrize("N", [3, 130, 1100])
+def test_every_tile_of_products_cut_in_parts(gpu_device, tile, N, K):
+    """Each tile at its edges, with runs of K that are empty or shorter than others, equal to the bit
+    to the largest one, whose sums are within a unit in the last place for every addition."""
+    ops = load_hip_ops(gpu_device)
+    for M in (1, 15, 16 * tile) if tile <= ROW_TILES else (1, 63, 133, 261):
+        x, w = rand((M, K), 26).to(gpu_device), (rand((N, K), 27) * 0.05).to(gpu_device)
+        whole = by_tile(ops, x, w, TILES)
+        bound = (x.abs().double() @ w.abs().double().T) * 2.0 ** -24 * (10 + K / 256)
+        assert ((whole.double() - x.double() @ w.double().T).abs() <= bound).all()
+        assert torch.equal(by_tile(ops, x, w, tile), whole)
+        assert torch.equal(by_tile(ops, x, w, tile, offset=1), whole)
+
+
+@pytest.mark.parametrize("tile", range(1, TILES + 1))
+@pytest.mark.parametrize("N", [203, 300])
+def test_every_tile_with_numbers_that_have_no_three_parts(gpu_device, tile, N):
+    ops = load_hip_ops(gpu_device)
+    M = 16 * tile if tile <= ROW_TILES else 261
+    x, w = rand((M, 192), 28), rand((N, 192), 29)
+    x[3, 5], x[4, 7], w[9, 100], x[6, 100], x[8, 2] = float("inf"), float("nan"), -3.4e38, 1.5, 3.402e38
+    x[7], w[:, 2], w[N - 1, 191], x[M - 1, 0] = 0.0, 0.25, float("nan"), float("-inf")
+    want = (x.double() @ w.double().T).float()
+    out = by_tile(ops, x.to(gpu_device), w.to(gpu_device), tile).cpu()
+    assert torch.equal(torch.isnan(out), torch.isnan(want))
+    assert torch.equal(torch.isinf(out), torch.isinf(want))
+    fine = torch.isfinite(want)
+    torch.testing.assert_close(out[fine], want[fine], rtol=1e-5, atol=1e-3)

@@ -98,6 +98,7 @@ struct SplitArgs {
   const float *a, *w;
   float* c;
   int M, N, K;
+  int wide;                 // C's fours of columns begin on 16 bytes
   int tiles_m, tiles_n, panel;
 };
 
@@ -278,7 +279,7 @@ __global__ __launch_bounds__(kRuns* kWave) void gemm_f32_split_kernel(SplitArgs 
           v[r] = product_again(a.a + (int64_t)m * a.K, a.w + (int64_t)(n + r) * a.K, a.K);
     }
     float* out = a.c + (int64_t)m * a.N + n;
-    if (n + 4 <= a.N && a.N % 4 == 0) {
+    if (n + 4 <= a.N && a.wide) {
       *(f32x4*)out = v;
     } else {
 #pragma unroll
@@ -485,7 +486,7 @@ __global__ __launch_bounds__(64 * GM * GN * G) void gemm_f32_split_tile_kernel(S
             v[r] = product_again(a.a + (int64_t)m * a.K, a.w + (int64_t)(n + r) * a.K, a.K);
       }
       float* out = a.c + (int64_t)m * a.N + n;
-      if (n + 4 <= a.N && a.N % 4 == 0) {
+      if (n + 4 <= a.N && a.wide) {
         *(f32x4*)out = v;
       } else {
 #pragma unroll
@@ -512,32 +513,47 @@ int launch_tile(SplitArgs a, hipStream_t stream) {
 
 }  // namespace
 
-int gemm_f32_split_launch(const float* A, const float* W, float* C, int M, int N, int K, hipStream_t stream) {
-  SplitArgs a{A, W, C, M, N, K, 0, 0, 1};
-  if (M <= 32) {
-    const dim3 block(kRuns * kWave), grid((N + 15) / 16);
-    if (M <= 16) hipLaunchKernelGGL(gemm_f32_split_rows_kernel<1>, grid, block, 0, stream, a);
-    else hipLaunchKernelGGL(gemm_f32_split_rows_kernel<2>, grid, block, 0, stream, a);
-    return 0;
+int gemm_f32_split_launch(const float* A, const float* W, float* C, int M, int N, int K, int tile,
+                          hipStream_t stream) {
+  SplitArgs a{A, W, C, M, N, K, N % 4 == 0 && ((uintptr_t)C & 15) == 0, 0, 0, 1};
+  const dim3 block(kRuns * kWave), grid((N + 15) / 16);
+  if (tile == 0 && M <= 64) tile = M <= 16 ? 1 : M <= 32 ? 2 : 3;
+  if (tile == 0) {
+    // The tile with the least estimate: rounds of 256 units by what a tile takes, a part of its own
+    // and one for every 1,024 of K, both measured with weights in memory.
+    struct Tile { int bm, bn; float fixed_us, k_us; };
+    constexpr Tile kTiles[] = {{32, 64, 4.5f, 8.8f}, {64, 64, 7.f, 14.f}, {128, 64, 7.f, 30.f},
+                               {128, 96, 8.f, 41.f}, {128, 128, 9.f, 49.5f}};
+    float least = -1.f;
+    for (int t = 0; t < 5; ++t) {
+      const int64_t tiles = (int64_t)((M + kTiles[t].bm - 1) / kTiles[t].bm) * ((N + kTiles[t].bn - 1) / kTiles[t].bn);
+      const float us = (float)((tiles + 255) / 256) * (kTiles[t].fixed_us + kTiles[t].k_us * (float)K / 1024.f);
+      if (least < 0.f || us < least) least = us, tile = t + 4;
+    }
   }
-  if (M <= 64) return launch_runs<4, 1, 2>(a, stream);
-  // The tile with the least estimate: rounds of 256 units by what a tile takes, a part of its own
-  // and one for every 1,024 of K, both measured with weights in memory.
-  struct Tile { int bm, bn; float fixed_us, k_us; };
-  constexpr Tile kTiles[] = {{32, 64, 4.5f, 8.8f}, {64, 64, 7.f, 14.f}, {128, 64, 7.f, 30.f},
-                             {128, 96, 8.f, 41.f}, {128, 128, 9.f, 49.5f}};
-  int best = 0;
-  float least = -1.f;
-  for (int t = 0; t < 5; ++t) {
-    const int64_t tiles = (int64_t)((M + kTiles[t].bm - 1) / kTiles[t].bm) * ((N + kTiles[t].bn - 1) / kTiles[t].bn);
-    const float us = (float)((tiles + 255) / 256) * (kTiles[t].fixed_us + kTiles[t].k_us * (float)K / 1024.f);
-    if (least < 0.f || us < least) least = us, best = t;
+  if (tile <= 2 && M > 16 * tile) return -1;
+  switch (tile) {
+    case 1: hipLaunchKernelGGL(gemm_f32_split_rows_kernel<1>, grid, block, 0, stream, a); return 0;
+    case 2: hipLaunchKernelGGL(gemm_f32_split_rows_kernel<2>, grid, block, 0, stream, a); return 0;
+    case 3: return launch_runs<4, 1, 2>(a, stream);
+    case 4: return launch_tile<32, 64, 2, 2, 4>(a, stream);
+    case 5: return launch_runs<4, 4, 1>(a, stream);
+    case 6: return launch_tile<128, 64, 4, 2, 1>(a, stream);
+    case 7: return launch_tile<128, 96, 4, 2, 1>(a, stream);
+    case 8: return launch_tile<128, 128, 4, 2, 1>(a, stream);
+    default: return -1;
   }
-  switch (best) {
-    case 0: return launch_tile<32, 64, 2, 2, 4>(a, stream);
-    case 1: return launch_runs<4, 4, 1>(a, stream);
-    case 2: return launch_tile<128, 64, 4, 2, 1>(a, stream);
-    case 3: return launch_tile<128, 96, 4, 2, 1>(a, stream);
-    default: return launch_tile<128, 128, 4, 2, 1>(a, stream);
-  }
+}
+
+extern "C" int ts_gemm_f32_split(const float* a, const float* w, float* c, int M, int N, int K, int tile,
+                                 hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (K <= 0 || !gemm_f32_split_fits(K)) TS_FAIL("gemm_f32_split: K=%d is no multiple of 64", K);
+  if (((uintptr_t)a | (uintptr_t)w) & 15) TS_FAIL("gemm_f32_split: operands must be 16-byte aligned");
+  if (tile < 0 || tile > 8 || (tile >= 1 && tile <= 2 && M > 16 * tile))
+    TS_FAIL("gemm_f32_split: tile %d does not take %d rows", tile, M);
+  if (gemm_f32_split_launch(a, w, c, M, N, K, tile, stream))
+    TS_FAIL("gemm_f32_split: a tile needs more LDS than the device gives");
+  TS_CHECK_LAUNCH("gemm_f32_split");
+  return 0;
 }

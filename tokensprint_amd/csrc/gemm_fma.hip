@@ -341,7 +341,7 @@ static int launch_tile(const TA* A, const TW* W, TC* C, int M, int N, int K, hip
 template <typename TA, typename TW, typename TC>
 static int launch_f32(const TA* A, const TW* W, TC* C, int M, int N, int K, hipStream_t stream) {
   if constexpr (std::is_same_v<TA, float> && std::is_same_v<TW, float> && std::is_same_v<TC, float>) {
-    if (gemm_f32_split_fits(K)) return gemm_f32_split_launch(A, W, C, M, N, K, stream);
+    if (gemm_f32_split_fits(K)) return gemm_f32_split_launch(A, W, C, M, N, K, 0, stream);
   }
   const dim3 block(kRuns * kWave), grid((N + 15) / 16);
   if (M <= 16) {
