@@ -13,7 +13,7 @@ from tokensprint_amd.kernels import load_hip_ops
 pytestmark = pytest.mark.gpu
 
 #: tiles of the product cut in parts; the first ones take 16, 32, ... rows at most
-TILES, ROW_TILES = 8, 2
+TILES, ROW_TILES = 10, 3
 
 
 def rand(shape, seed, dtype=torch.float32):

@@ -103,7 +103,7 @@ struct SplitArgs {
 };
 
 // ---------------------------------------------------------------- few rows
-// Up to 16 MT rows: a workgroup takes 16 columns, each of its eight wavefronts a run of K, so a
+// Up to 16 MT rows (48): a workgroup takes 16 columns, each of its eight wavefronts a run of K, so a
 // weight is read once, a stretch ahead of its use.  Bound by the weights' way from memory.
 template <int MT>
 __global__ __launch_bounds__(kRuns* kWave) void gemm_f32_split_rows_kernel(SplitArgs a) {
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(kRuns* kWave) void gemm_f32_split_rows_kernel(Split
 }
 
 // ---------------------------------------------------------------- a run a wavefront
-// A workgroup takes 16 TM rows and 16 TN columns, each of its eight wavefronts a run of K: what a
+// A workgroup takes 16 TM rows and 16 TN columns (32 x 16 to 64 x 64), each of its eight wavefronts a run of K: what a
 // wavefront cuts it multiplies itself, so nothing passes through LDS and nobody waits for others
 // until the runs are added up.  Operands are sent for SETS steps of 32 ahead, into the registers
 // that a step has just cut.
@@ -517,30 +517,36 @@ int gemm_f32_split_launch(const float* A, const float* W, float* C, int M, int N
                           hipStream_t stream) {
   SplitArgs a{A, W, C, M, N, K, N % 4 == 0 && ((uintptr_t)C & 15) == 0, 0, 0, 1};
   const dim3 block(kRuns * kWave), grid((N + 15) / 16);
-  if (tile == 0 && M <= 64) tile = M <= 16 ? 1 : M <= 32 ? 2 : 3;
+  if (tile == 0 && M <= 32) tile = M <= 16 ? 1 : 2;
   if (tile == 0) {
     // The tile with the least estimate: rounds of 256 units by what a tile takes, a part of its own
-    // and one for every 1,024 of K, both measured with weights in memory.
-    struct Tile { int bm, bn; float fixed_us, k_us; };
-    constexpr Tile kTiles[] = {{32, 64, 4.5f, 8.8f}, {64, 64, 7.f, 14.f}, {128, 64, 7.f, 30.f},
-                               {128, 96, 8.f, 41.f}, {128, 128, 9.f, 49.5f}};
+    // and one for every 1,024 of K, both measured with weights in memory.  (33 to 64 rows had a tile
+    // of their own, 64 x 16, which reads all rows for every 16 columns: 4,096 x 4,096 53 to 56 us,
+    // now 35 to 42, 1,024 x 3,072 32 to 36, now 21.)
+    struct Tile { int bm, bn, most; float fixed_us, k_us; };
+    constexpr Tile kTiles[] = {{48, 16, 48, 3.f, 8.f}, {32, 16, 0, 4.9f, 5.2f}, {32, 32, 0, 1.5f, 10.4f},
+                               {32, 64, 0, 4.5f, 8.8f}, {64, 64, 0, 7.f, 14.f}, {128, 64, 0, 7.f, 30.f},
+                               {128, 96, 0, 8.f, 41.f}, {128, 128, 0, 9.f, 49.5f}};
     float least = -1.f;
-    for (int t = 0; t < 5; ++t) {
+    for (int t = 0; t < 8; ++t) {
+      if (kTiles[t].most && M > kTiles[t].most) continue;
       const int64_t tiles = (int64_t)((M + kTiles[t].bm - 1) / kTiles[t].bm) * ((N + kTiles[t].bn - 1) / kTiles[t].bn);
       const float us = (float)((tiles + 255) / 256) * (kTiles[t].fixed_us + kTiles[t].k_us * (float)K / 1024.f);
-      if (least < 0.f || us < least) least = us, tile = t + 4;
+      if (least < 0.f || us < least) least = us, tile = t + 3;
     }
   }
-  if (tile <= 2 && M > 16 * tile) return -1;
+  if (tile <= 3 && M > 16 * tile) return -1;
   switch (tile) {
     case 1: hipLaunchKernelGGL(gemm_f32_split_rows_kernel<1>, grid, block, 0, stream, a); return 0;
     case 2: hipLaunchKernelGGL(gemm_f32_split_rows_kernel<2>, grid, block, 0, stream, a); return 0;
-    case 3: return launch_runs<4, 1, 2>(a, stream);
-    case 4: return launch_tile<32, 64, 2, 2, 4>(a, stream);
-    case 5: return launch_runs<4, 4, 1>(a, stream);
-    case 6: return launch_tile<128, 64, 4, 2, 1>(a, stream);
-    case 7: return launch_tile<128, 96, 4, 2, 1>(a, stream);
-    case 8: return launch_tile<128, 128, 4, 2, 1>(a, stream);
+    case 3: hipLaunchKernelGGL(gemm_f32_split_rows_kernel<3>, grid, block, 0, stream, a); return 0;
+    case 4: return launch_runs<2, 1, 2>(a, stream);
+    case 5: return launch_runs<2, 2, 2>(a, stream);
+    case 6: return launch_tile<32, 64, 2, 2, 4>(a, stream);
+    case 7: return launch_runs<4, 4, 1>(a, stream);
+    case 8: return launch_tile<128, 64, 4, 2, 1>(a, stream);
+    case 9: return launch_tile<128, 96, 4, 2, 1>(a, stream);
+    case 10: return launch_tile<128, 128, 4, 2, 1>(a, stream);
     default: return -1;
   }
 }
@@ -550,7 +556,7 @@ extern "C" int ts_gemm_f32_split(const float* a, const float* w, float* c, int M
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0 || !gemm_f32_split_fits(K)) TS_FAIL("gemm_f32_split: K=%d is no multiple of 64", K);
   if (((uintptr_t)a | (uintptr_t)w) & 15) TS_FAIL("gemm_f32_split: operands must be 16-byte aligned");
-  if (tile < 0 || tile > 8 || (tile >= 1 && tile <= 2 && M > 16 * tile))
+  if (tile < 0 || tile > 10 || (tile >= 1 && tile <= 3 && M > 16 * tile))
     TS_FAIL("gemm_f32_split: tile %d does not take %d rows", tile, M);
   if (gemm_f32_split_launch(a, w, c, M, N, K, tile, stream))
     TS_FAIL("gemm_f32_split: a tile needs more LDS than the device gives");
