@@ -254,3 +254,19 @@ def test_every_tile_with_numbers_that_have_no_three_parts(gpu_device, tile, N):
     assert torch.equal(torch.isinf(out), torch.isinf(want))
     fine = torch.isfinite(want)
     torch.testing.assert_close(out[fine], want[fine], rtol=1e-5, atol=1e-3)
+
+
+@pytest.mark.parametrize("tile", range(1, TILES + 1))
+@pytest.mark.parametrize("K", [64, 1088])
+def test_rows_and_columns_without_a_finite_result(gpu_device, tile, K):
+    """Elements that are made again by a whole wavefront, all of a wavefront's and some of them,
+    with fewer and with more fours of K than lanes."""
+    ops = load_hip_ops(gpu_device)
+    M, N = 16 * tile if tile <= ROW_TILES else 140, 133
+    x, w = rand((M, K), 30), rand((N, K), 31)
+    x[1], x[5, K - 1], w[16:40, 3], w[130, K - 4] = float("nan"), float("inf"), float("-inf"), float("nan")
+    want = (x.double() @ w.double().T).float()
+    out = by_tile(ops, x.to(gpu_device), w.to(gpu_device), tile).cpu()
+    assert torch.equal(out.isnan(), want.isnan())
+    fine = ~want.isnan()
+    torch.testing.assert_close(out[fine], want[fine], rtol=1e-5, atol=1e-4)

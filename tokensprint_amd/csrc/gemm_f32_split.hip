@@ -26,8 +26,10 @@
 // in order.  Every kernel here adds in that order, so an element depends on neither the other rows
 // of a call nor their number.
 // Where a result is not finite, it may be because a part was not (infinities, and numbers that
-// bfloat16 rounds to one, leave a NaN behind): such an element is made again, in float32, one
-// product after the other.
+// bfloat16 rounds to one, leave a NaN behind): such an element is made again, in float64 (in
+// whatever order, it is infinite only if it has to be), by the wavefront that has it.  501 rows of
+// NaN with 6,144 x 1,024 take 1.3 ms instead of 0.05, 2,048 with 4,096 x 4,096 3.7 instead of 0.45 (a
+// thread an element, one product after the other: 5.7 and 61).
 //
 // What bounds it: LDS, the matrix cores (six instructions of 16 cycles for 32 of K against eight of
 // 32) and what cuts operands in parts, 5.5 instructions a number, one after the other in most of a
@@ -87,13 +89,6 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// An element by itself (see above).
-__device__ __noinline__ float product_again(const float* a, const float* w, int K) {
-  float sum = 0.f;
-  for (int k = 0; k < K; ++k) sum = fmaf(a[k], w[k], sum);
-  return sum;
-}
-
 struct SplitArgs {
   const float *a, *w;
   float* c;
@@ -101,6 +96,58 @@ struct SplitArgs {
   int wide;                 // C's fours of columns begin on 16 bytes
   int tiles_m, tiles_n, panel;
 };
+
+// The elements (m, n) of the lanes in `bad`, made again (see above), one after the other: every lane
+// of the wavefront takes part.
+__device__ __noinline__ float made_again(float v, unsigned long long bad, const float* a, const float* b,
+                                         int K, int m, int n) {
+  const int lane = threadIdx.x % kWave;
+  for (; bad; bad &= bad - 1) {
+    const int of = __ffsll(bad) - 1;
+    const float* x = a + (int64_t)__shfl(m, of, kWave) * K;
+    const float* w = b + (int64_t)__shfl(n, of, kWave) * K;
+    double sum = 0.;
+    for (int k0 = 4 * lane; k0 - 4 * lane < K; k0 += 16 * kWave) {
+      f32x4 xv[4], wv[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int k = k0 + 4 * kWave * u;
+        xv[u] = k < K ? *(const f32x4*)(x + k) : kZero, wv[u] = k < K ? *(const f32x4*)(w + k) : kZero;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum = fma((double)xv[u][j], (double)wv[u][j], sum);
+      if (__any(sum != sum)) break;         // and it stays so
+    }
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, kWave);
+    if (lane == of) v = (float)sum;
+  }
+  return v;
+}
+
+// Stores a lane's four columns [n, n + 4) of row m; all lanes of a wavefront come here.
+__device__ __forceinline__ void store4(const SplitArgs& a, f32x4 v, int m, int n) {
+  const bool row = m < a.M;
+  const bool fine = !row || fabsf(v[0]) + fabsf(v[1]) + fabsf(v[2]) + fabsf(v[3]) < INFINITY;
+  if (__ballot(!fine)) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const unsigned long long bad = __ballot(row && n + r < a.N && !(fabsf(v[r]) < INFINITY));
+      if (bad) v[r] = made_again(v[r], bad, a.a, a.w, a.K, m, n + r);
+    }
+  }
+  if (!row) return;
+  float* out = a.c + (int64_t)m * a.N + n;
+  if (n + 4 <= a.N && a.wide) {
+    *(f32x4*)out = v;
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (n + r < a.N) out[r] = v[r];
+  }
+}
 
 // ---------------------------------------------------------------- few rows
 // Up to 16 MT rows (48): a workgroup takes 16 columns, each of its eight wavefronts a run of K, so a
@@ -166,10 +213,12 @@ __global__ __launch_bounds__(kRuns* kWave) void gemm_f32_split_rows_kernel(Split
     float v = 0.f;
 #pragma unroll
     for (int r = 0; r < kRuns; r += 2) v += sums[r][i][at] + sums[r + 1][i][at];
+    // (whole wavefronts come here)
     const int m = 16 * i + row, n = n0 + col;
-    if (m >= a.M || n >= a.N) continue;
-    if (!(fabsf(v) < INFINITY)) v = product_again(a.a + (int64_t)m * a.K, a.w + (int64_t)n * a.K, a.K);
-    a.c[(int64_t)m * a.N + n] = v;
+    const bool in = m < a.M && n < a.N;
+    const unsigned long long bad = __ballot(in && !(fabsf(v) < INFINITY));
+    if (bad) v = made_again(v, bad, a.a, a.w, a.K, m, n);
+    if (in) a.c[(int64_t)m * a.N + n] = v;
   }
 }
 
@@ -264,28 +313,13 @@ __global__ __launch_bounds__(kRuns* kWave) void gemm_f32_split_kernel(SplitArgs 
 #pragma unroll
     for (int j = 0; j < TN; ++j) *place(run, i * TN + j, lane) = sum[i][j];
   __syncthreads();
-  // a thread takes four columns of a row
+  // a thread takes four columns of a row, a wavefront a block
   for (int e = threadIdx.x; e < TM * TN * 64; e += kRuns * kWave) {
     const int block = e / 64, of = e % 64;
     f32x4 v = kZero;
 #pragma unroll
     for (int r = 0; r < kRuns; r += 2) v += *place(r, block, of) + *place(r + 1, block, of);
-    const int m = m0 + block / TN * 16 + of % 16, n = n0 + block % TN * 16 + of / 16 * 4;
-    if (m >= a.M || n >= a.N) continue;
-    if (!(fabsf(v[0]) + fabsf(v[1]) + fabsf(v[2]) + fabsf(v[3]) < INFINITY)) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (n + r < a.N && !(fabsf(v[r]) < INFINITY))
-          v[r] = product_again(a.a + (int64_t)m * a.K, a.w + (int64_t)(n + r) * a.K, a.K);
-    }
-    float* out = a.c + (int64_t)m * a.N + n;
-    if (n + 4 <= a.N && a.wide) {
-      *(f32x4*)out = v;
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (n + r < a.N) out[r] = v[r];
-    }
+    store4(a, v, m0 + block / TN * 16 + of % 16, n0 + block % TN * 16 + of / 16 * 4);
   }
 }
 
@@ -472,29 +506,10 @@ __global__ __launch_bounds__(64 * GM * GN * G) void gemm_f32_split_tile_kernel(S
         for (int gr = 1; gr < G; ++gr) all[i][j] += *place(gr, i, j);
   }
 #pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int m = m0 + (wm * TM + i) * 16 + l;
-    if (m >= a.M) continue;
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int n = n0 + (wn * TN + j) * 16 + 4 * g;
-      f32x4 v = all[i][j];
-      if (!(fabsf(v[0]) + fabsf(v[1]) + fabsf(v[2]) + fabsf(v[3]) < INFINITY)) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (n + r < a.N && !(fabsf(v[r]) < INFINITY))
-            v[r] = product_again(a.a + (int64_t)m * a.K, a.w + (int64_t)(n + r) * a.K, a.K);
-      }
-      float* out = a.c + (int64_t)m * a.N + n;
-      if (n + 4 <= a.N && a.wide) {
-        *(f32x4*)out = v;
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (n + r < a.N) out[r] = v[r];
-      }
-    }
-  }
+    for (int j = 0; j < TN; ++j)
+      store4(a, all[i][j], m0 + (wm * TM + i) * 16 + l, n0 + (wn * TN + j) * 16 + 4 * g);
 }
 
 template <int BM, int BN, int GM, int GN, int G>
