@@ -275,6 +275,18 @@ def test_gate_up_of_a_large_weight(ops, gpu_device, M):
                                rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("K, first", [(1024, 9), (2048, 9), (2056, 7), (4096, 7), (4104, 5), (5120, 5)])
+def test_rows_of_an_output_head(ops, gpu_device, K, first):
+    """The row count at which a head's product becomes the library's, by the length of its rows."""
+    N = 16400
+    assert not ops._library_rows(first - 1, N, K) and ops._library_rows(first, N, K)
+    w = rand((N, K), torch.bfloat16, gpu_device, 65, scale=0.05)
+    x = rand((first, K), torch.bfloat16, gpu_device, 66)
+    want = x.float() @ w.float().T
+    for M in (first - 1, first):
+        torch.testing.assert_close(ops.linear(x[:M], w, torch.float32), want[:M], rtol=1e-4, atol=1e-3)
+
+
 @pytest.mark.parametrize("M,N,K,next_n,silu", [(2051, 1024, 2048, 3072, True),
                                                (513, 320, 1024, 400, False),
                                                (700, 576, 4096, 112, True),

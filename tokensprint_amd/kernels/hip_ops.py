@@ -447,7 +447,9 @@ class HipOps:
         if pair:
             if M >= d.library_rows_pair and pair > d.pair_head_weight:
                 return True
-        elif M >= d.library_rows_head and N >= d.head_columns:
+        elif N >= d.head_columns and M >= (
+                d.library_rows_head if K <= 2048 else
+                d.library_rows_long_head if K <= 4096 else d.library_rows_longest_head):
             return True
         if N * K > d.large_weight:
             rows = self._large_rows.get((N, K))
