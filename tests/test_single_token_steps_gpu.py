@@ -178,3 +178,20 @@ def test_low_rank_pair(T, n_a, k_a, n_g, k_g, col):
         # float32 sums of K exact products: K roundings at most of partial sums below |x| |w|
         bound = x[:, at:at + w.shape[1]].abs().double() @ w.abs().double().T * w.shape[1] * 2.0 ** -24
         assert ((got.double() - want).abs() <= bound + 1e-30).all()
+
+
+@pytest.mark.parametrize("T, n_a, k_a, n_g, k_g, one", [
+    (2048, 512, 64, 1024, 64, True), (2049, 512, 64, 1024, 64, False), (8, 64, 512, 64, 512, True),
+    (8, 64, 544, 64, 512, False), (200, 4096, 512, 4096, 512, False)])
+def test_low_rank_pairs_that_are_two_products(monkeypatch, T, n_a, k_a, n_g, k_g, one):
+    """Long ranks and many rows are left to the products of their own, which share operands out."""
+    ops = load_hip_ops("cuda:0")
+    taken, linear = [], ops.linear
+    monkeypatch.setattr(ops, "linear", lambda x, w, t: taken.append(w) or linear(x, w, t))
+    x = rand((T, k_a + k_g), 92)
+    w_a, w_g = (rand((n, k), 93, 0.1).to(torch.bfloat16) for n, k in ((n_a, k_a), (n_g, k_g)))
+    z, gate = ops.low_rank_pair(x, 0, w_a, k_a, w_g, torch.bfloat16)
+    assert len(taken) == (0 if one else 2)
+    for got, at, w in ((z, 0, w_a), (gate, k_a, w_g)):
+        want = x[:, at:at + w.shape[1]].to(torch.bfloat16).float() @ w.float().T
+        torch.testing.assert_close(got, want, rtol=1e-4, atol=1e-3)

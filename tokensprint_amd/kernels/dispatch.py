@@ -87,6 +87,15 @@ class Dispatch:
     #: at a step's start); others where `ts_gemm_tiled_ahead` says so.
     tiled_plain_weight: int = 1 << 23
 
+    #: Second steps of two low-rank projections: one launch, whose wavefronts read their operands
+    #: from memory, for ranks up to `low_rank_most` and rows x ranks x columns (of both) up to
+    #: `low_rank_work`; above, two products.  One launch of the two's time: rank 64, 512 + 1,024
+    #: columns, 8 rows 0.51, 1,000 0.67, 2,048 0.95, 4,096 1.37; 2,048 + 2,048 columns 512 rows 0.74,
+    #: 1,000 1.09; rank 128, 4,096 + 4,096 200 rows 0.77, 512 1.29; rank 512, 65 rows 0.63, 200 1.29,
+    #: 16,384 7.5; rank 1,024 8 rows 1.18
+    low_rank_most: int = 512
+    low_rank_work: int = 3 << 26
+
     # ---- attention.  Measured at 16 query / 8 key-value heads of 128, page size 16.
     #: workgroups (entries x key/value heads) up to which a decode step takes the decode
     #: kernel; with more, the chip is full anyway and the smaller workgroups of the

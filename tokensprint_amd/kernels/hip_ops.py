@@ -1810,7 +1810,9 @@ class HipOps:
         self._check("w_a", w_a, self._FLOATS, ndim=2)
         self._check("w_g", w_g, self._FLOATS, ndim=2)
         (n_a, k_a), (n_g, k_g), T = w_a.shape, w_g.shape, x.shape[0]
+        d = self.dispatch
         if act_dtype is torch.bfloat16 and w_a.dtype is torch.bfloat16 and w_g.dtype is torch.bfloat16 \
+                and max(k_a, k_g) <= d.low_rank_most and T * (n_a * k_a + n_g * k_g) <= d.low_rank_work \
                 and T <= 65535 * 16 and self.lib.ts_low_rank_pair_fits(k_a, k_g) == 1 \
                 and (w_a.data_ptr() | w_g.data_ptr()) % 16 == 0:
             out_a = torch.empty(T, n_a, dtype=torch.float32, device=self.device)
