@@ -287,6 +287,28 @@ def test_rows_of_an_output_head(ops, gpu_device, K, first):
         torch.testing.assert_close(ops.linear(x[:M], w, torch.float32), want[:M], rtol=1e-4, atol=1e-3)
 
 
+@pytest.mark.parametrize("M, N, K, ahead", [
+    # N no multiple of 256: narrow products of a long K, whose few tiles each walk all of it
+    (65, 64, 8192, 0), (96, 208, 2048, 0), (66, 576, 2048, 0), (300, 288, 1024, 0), (96, 2192, 2048, 0),
+    (262, 6176, 2048, 0), (65, 48, 512, 1), (65, 4640, 1024, 1), (676, 10304, 2048, 1),
+    (300, 151936, 1024, 0), (512, 151936, 1024, 1),
+    # N a multiple of 256
+    (432, 4096, 4096, 1), (5288, 6144, 4096, 0), (3000, 5120, 8192, 0), (1536, 5120, 25600, 1),
+    (3100, 5120, 25600, 0), (8192, 5120, 25600, 1), (8192, 10240, 5120, 0)])
+def test_plain_products_by_the_faster_kernel(ops, M, N, K, ahead):
+    assert ops.lib.ts_gemm_tiled_ahead(M, N, K, 1) == ahead
+
+
+@pytest.mark.parametrize("M, N, K", [(65, 64, 2048), (130, 208, 1088), (300, 576, 2048)])
+def test_narrow_products_of_many_rows(ops, gpu_device, M, N, K):
+    assert ops.lib.ts_gemm_tiled_fits(M, N, K, 0) == 1 and not ops.lib.ts_gemm_tiled_ahead(M, N, K, 0)
+    x = rand((M, K), torch.bfloat16, gpu_device, 67)
+    w = rand((N, K), torch.bfloat16, gpu_device, 68, scale=0.05)
+    for dtype in (torch.float32, torch.bfloat16):
+        torch.testing.assert_close(ops.linear(x, w, dtype).float(), x.float() @ w.float().T,
+                                   rtol=1e-2, atol=1e-2)
+
+
 @pytest.mark.parametrize("M,N,K,next_n,silu", [(2051, 1024, 2048, 3072, True),
                                                (513, 320, 1024, 400, False),
                                                (700, 576, 4096, 112, True),

@@ -28,20 +28,49 @@ extern "C" int ts_gemm_tiled_fill(int M, int N, int K, int pair) {
 }
 
 // 1 if the plain product of these sizes (that ts_gemm_tiled_fits) is this kernel's rather than
-// the library's.  Both timed at 65 to 8,192 rows of 18 weights (N 1,024 to 10,304, K 1,024 to
-// 25,600), the weights in memory, bfloat16 out: where N is no multiple of 256 (4,384, 4,640,
-// 6,176, 10,304) this kernel takes 0.59 to 1.11 of the library's time, 0.86 in the mean; where
-// N is one and the product fills four fifths of its tiles' rounds 0.54 to 1.07, 0.97 in the mean
-// (5,120 x 25,600 at 8,192 rows 1,610 / 2,090 us; below four fifths 1.01 in the mean and up to
-// 1.30), but for products that the library's tile of 256 x 256 cuts in whole rounds of the units:
-// 0.97 to 1.11, 1.08 in the mean, so those stay the library's (with float32 out, whose stores it
-// does worse, they do not: 2,048 x 8,192 x 2,048 59 / 66 us).
+// the library's, which shares a tile's K out over units where there are few tiles.  Both timed at
+// 65 to 8,192 rows, the weights in memory; times of the library's.
+// N no multiple of 256, N 16 to 10,304: the longer K, the more of the tiles' rounds has to be
+// filled.  K = 512 0.22 to 1.01 from 48 columns; K = 1,024 0.74 to 0.92 from 1,296 columns, 1.1 to
+// 1.3 below with less than a third filled; K = 2,048 0.78 to 1.05 from two thirds on, up to 1.8 below;
+// K = 4,096 and 8,192 0.81 to 1.01 from seven tenths on (up to 1,024 rows of up to 4,096 columns of
+// 4,096 0.90 to 1.04 from a half on), up to 3.4 below (65 rows of 64 columns of 8,192).  151,936
+// columns: 0.82 to 0.95 from seven tenths on, up to 1.11 below.
+// N a multiple of 256, float32 out: 0.87 to 1.05 from four fifths filled, 0.95 in the mean.  bfloat16
+// out, four fifths filled: 0.62 to 1.00 where the tiles are 128 x 128 or smaller; with larger ones the
+// library's 256 x 256 mostly is as good or ahead (0.97 to 1.17), but for long K (K from 5,120): one
+// round of 256 x 128 0.67 to 0.99, and more than two rounds of 256 x 256 of which the last is not
+// full 0.72 to 0.87.  With the longest K the library often is at half of its rate: K = 25,600 0.65
+// to 0.97 in one round of up to 256 x 128, whatever it fills (5,120 columns, 1,536 rows 338 / 507
+// us), with larger tiles 0.58 to 1.08 from six (one round) or seven tenths on, 0.87 in the mean (8,192
+// rows 1,610 / 2,090).
 extern "C" int ts_gemm_tiled_ahead(int M, int N, int K, int c_type) {
   if (!ts_gemm_tiled_fits(M, N, K, 0)) return 0;
-  if (N % 256 != 0) return 1;
-  const int64_t squares = (int64_t)((M + 255) / 256) * (N / 256);
-  if (c_type == TS_BF16 && squares % compute_units() == 0) return 0;
-  return ts_gemm_tiled_fill(M, N, K, 0) >= 80;
+  const int fill = ts_gemm_tiled_fill(M, N, K, 0);
+  if (N % 256 != 0) {
+    if (N < 16384 && (K <= 512 ? N >= 48 : K <= 1024 && N >= 1280)) return 1;
+    if (N < 16384 && K < 2240) return fill >= K / 32;
+    return fill >= (K <= 6144 && N <= 4096 && M <= 1024 ? 49 : 70);
+  }
+  const bool longest = K >= 16384;
+  if (fill < (longest ? 45 : 80)) return 0;
+  if (c_type != TS_BF16 && fill >= 80) return 1;
+  TiledArgs g{};
+  g.M = M, g.N = N, g.K = K;
+  const int tile = cheapest_tile(g, false), units = compute_units();
+  for (const TileCost& t : kTileCosts) {
+    if (t.tile != tile) continue;
+    const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    if (t.bm * t.bn <= 128 * 128) return 1;
+    if (K < 5120) return 0;
+    if (t.bm * t.bn == 256 * 128) {
+      if (tiles <= units) return 1;
+    } else if (longest) {
+      return fill >= (tiles <= units ? 60 : 70);
+    }
+  }
+  const int64_t squares = (int64_t)((M + 255) / 256) * (N / 256), rounds = (squares + units - 1) / units;
+  return rounds > 2 && squares * 10 < rounds * units * 9;
 }
 
 // C[M, N] = A[M, K] W[N, K]^T, or with `pair` C[M, N] = silu(A Wg^T) * (A Wu^T) (or, with a
