@@ -309,6 +309,25 @@ def test_narrow_products_of_many_rows(ops, gpu_device, M, N, K):
                                    rtol=1e-2, atol=1e-2)
 
 
+@pytest.mark.parametrize("M, inner, K, tiled", [
+    (900, 25600, 5120, False), (960, 25600, 5120, False), (1000, 25600, 5120, True),
+    (520, 12288, 4096, False), (700, 12288, 4096, True)])
+def test_gate_up_products_that_fill_their_rounds(ops, M, inner, K, tiled):
+    x = torch.empty(M, K, dtype=torch.bfloat16, device="meta")
+    w = torch.empty(2 * inner, K, dtype=torch.bfloat16, device="meta")
+    assert ops._tiled_pair_ok(x, w, torch.bfloat16) == tiled
+
+
+@pytest.mark.parametrize("M", [72, 600, 2048, 8192])
+@pytest.mark.parametrize("N, K, next_n, silu", [(4096, 4096, 12288, True), (5120, 25600, 10240, False),
+                                                (1024, 1024, 16384, False)])
+def test_large_weights_keep_norms_of_their_own(ops, M, N, K, next_n, silu):
+    """A layer's products and norms at the 8B and 32B shapes take longer in the stream's forms."""
+    from tokensprint_amd.kernels.stream import NormHint
+    wn = torch.empty(next_n * (1 + silu), N, dtype=torch.bfloat16, device="meta")
+    assert not ops._tiled_stream_ok(M, N, K, NormHint(torch.empty(N, device="meta"), 1e-6, wn, silu))
+
+
 @pytest.mark.parametrize("M,N,K,next_n,silu", [(2051, 1024, 2048, 3072, True),
                                                (513, 320, 1024, 400, False),
                                                (700, 576, 4096, 112, True),

@@ -59,19 +59,24 @@ class Dispatch:
     #: wait for `tiled_pair_rows_large` rows.
     tiled_pair_weight: int = 1 << 27
     tiled_pair_rows_large: int = 512
-    #: From `tiled_fill_rows` rows of weights above `large_weight` elements, gate/up products and
-    #: the forms below also have to fill so many per cent of their tiles' rounds
-    #: (`ts_gemm_tiled_fill`): gate/up products at 23 row counts from 520 to 3,600 take 0.90 of the
-    #: library's and the SiLU kernel's time in the mean from 65 per cent on, 1.04 at most, and 1.03
-    #: below, up to 1.18; plain products 0.97 and 1.07 of the library's, without the norm kernel.
+    #: From `tiled_fill_rows` rows of weights above `large_weight` elements, gate/up products
+    #: also have to fill so many per cent of their tiles' rounds
+    #: (`ts_gemm_tiled_fill`): gate/up products at 46 row counts from 260 to 6,400 take 0.79 to 1.04
+    #: of the library's and the SiLU kernel's time from 65 per cent on, 0.92 in the mean, and 1.04
+    #: below, up to 1.14; the largest weights (above `tiled_pair_weight`) 0.80 to 0.95 from 75 per
+    #: cent on, and 0.87 to 1.04 from 65 to 75, in a step of 900 rows of the 32B shape 1.10.
     tiled_fill: int = 65
+    tiled_fill_large: int = 75
     tiled_fill_rows: int = 256
     #: rows from which, and elements of a weight [N, K] up to which, the product that ends a
     #: sub-layer is the LDS-tiled kernel's tail form (it adds itself into the float32 stream
     #: and prepares the rows for the norm behind it, whose product then takes the scaled
     #: form) instead of the library's product and a norm kernel.
     tiled_stream_rows: int = 512
-    tiled_stream_weight: int = 1 << 28
+    #: Larger weights keep the separate kernels, whose products are each the faster one's: a layer's
+    #: products and norms at 26 row counts from 512 to 8,192 take 1.00 to 1.11 of their time in
+    #: these forms at the 8B shape, 0.98 to 1.06 at the 32B shape.
+    tiled_stream_weight: int = 1 << 23
     #: Weights of `tiled_stream_few_weight` to `large_weight` elements take it from fewer rows in
     #: an eager step (captured ones, of up to 256 single tokens, do not: 4.99 against 4.77 ms): a
     #: step of the 0.6B shape with 300 tokens 2,117 -> 2,042 us on the GPU, with 128 1,738 -> 2,116

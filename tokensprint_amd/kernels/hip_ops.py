@@ -397,7 +397,8 @@ class HipOps:
                 and self._library_rows(M, weight.shape[0], K, weight.numel())
                 and self.lib.ts_gemm_tiled_fits(M, inner, K, 1) == 1
                 and (weight.numel() <= d.large_weight or M < d.tiled_fill_rows
-                     or self.lib.ts_gemm_tiled_fill(M, inner, K, 1) >= d.tiled_fill))
+                     or self.lib.ts_gemm_tiled_fill(M, inner, K, 1) >= (
+                         d.tiled_fill if weight.numel() <= d.tiled_pair_weight else d.tiled_fill_large)))
 
     def _tiled_plain_ok(self, M, N, K, x_dtype, w_dtype, out_dtype):
         d = self.dispatch
@@ -552,10 +553,6 @@ class HipOps:
                 or hint.weight.shape[1] != N or largest > d.tiled_stream_weight:
             return False
         next_n = hint.weight.shape[0] // 2 if hint.silu_mul else hint.weight.shape[0]
-        if largest > d.large_weight and (
-                self.lib.ts_gemm_tiled_fill(M, N, K, 0) < d.tiled_fill
-                or self.lib.ts_gemm_tiled_fill(M, next_n, N, int(hint.silu_mul)) < d.tiled_fill):
-            return False
         return (self.lib.ts_gemm_tiled_tail_fits(M, N, K) == 1
                 and self.lib.ts_gemm_tiled_scaled_fits(
                     M, next_n, N, int(hint.silu_mul), self.lib.ts_gemm_tiled_tail_parts(N)) == 1)
