@@ -6,7 +6,7 @@ between parts that do."""
 
 from __future__ import annotations
 
-from dataclasses import dataclass, replace
+from dataclasses import dataclass
 
 import torch
 
@@ -58,18 +58,31 @@ class NormAhead:
 @dataclass(frozen=True)
 class ShiftAhead:
     """What a block that opens with an RMSNorm and a token shift behind it tells the block before
-    it: the norm's weight and eps, the shift's weight, and (`at_cache`, from whoever knows which
-    run reads next) the requests' last rows.  A block of the same kind in front may then make the
-    shifted rows in the kernel of its last add."""
+    it in a step of single tokens: the norm's weight and eps, the shift's weight, and the requests'
+    last rows.  A block of the same kind in front may then make the shifted rows in the kernel of
+    its last add."""
 
     norm_weight: torch.Tensor
     eps: float
     weight: torch.Tensor
-    state: torch.Tensor | None = None
+    state: torch.Tensor
 
-    def at_cache(self, cache) -> "ShiftAhead | None":
-        state = cache.states.get("shift") if cache is not None else None
-        return None if state is None else replace(self, state=state)
+
+class ShiftEntry:
+    """The entry hint of such a block, made with the block.  Whoever knows which run reads next and
+    what the step is made of gets the ShiftAhead from it: in steps of single tokens, in others (where
+    the add and the norm behind a shift are kernels of their own anyway) none."""
+
+    def __init__(self, norm, shift) -> None:
+        self.norm, self.shift = norm, shift
+
+    def at_cache(self, cache, batch) -> ShiftAhead | None:
+        if batch.max_q_len != 1 or batch.num_tokens != batch.num_entries or cache is None:
+            return None
+        fused, state = fused_rmsnorm_of(self.norm), cache.states.get("shift")
+        if fused is None or state is None or not hasattr(self.shift.ops, "postnorm_add_shift"):
+            return None
+        return ShiftAhead(fused[0], fused[1], self.shift.weight, state)
 
 
 @dataclass(frozen=True)
@@ -181,9 +194,8 @@ class StreamProducts:
 
 def product_and_conv(ops, x, weight, col, channels, conv_w, bias, batch, state):
     """(x weight^T in float32, the short convolution of its columns [col, col + channels)); a
-    provider that has the two in one call chooses how."""
-    fused = getattr(ops, "linear_conv_silu", None)
-    if fused is not None:
-        return fused(x, weight, col, channels, conv_w, bias, batch, state)
+    provider that has the two in one call for steps of single tokens chooses how."""
+    if batch.max_q_len == 1 and hasattr(ops, "linear_conv_silu"):
+        return ops.linear_conv_silu(x, weight, col, channels, conv_w, bias, batch, state)
     proj = ops.linear(x, weight, torch.float32)
     return proj, ops.conv_silu(proj, col, channels, conv_w, bias, batch, state)

@@ -118,7 +118,7 @@ class Model:
                     if hasattr(next_hint, "entering") else None
             if hasattr(next_hint, "at_cache"):
                 next_hint = next_hint.at_cache(
-                    caches[r + 1 if nxt.cache_of is None else nxt.cache_of])
+                    caches[r + 1 if nxt.cache_of is None else nxt.cache_of], batch)
             if run.enter is not None and not getattr(delta, "entered", False):
                 # what is still to be added, then the row of this pass
                 ops.stream_add(resid, delta, None, entering(run))

@@ -203,6 +203,12 @@ class StreamFilter(Part):
     def cache_need(self):
         return None
 
+    def stream_hint(self, norm: "Norm"):
+        """The entry hint of a block that opens with `norm` and this filter, or None.  Asked for
+        once, when the block is made and no weight is loaded yet.  A hint with an
+        `at_cache(cache, batch)` is asked in every step for what the block in front gets."""
+        return None
+
     def forward_from_stream(self, resid: torch.Tensor, norm: "Norm", batch, cache) -> torch.Tensor:
         """The filtered norm of the rows of the stream."""
         raise NotImplementedError

@@ -9,7 +9,7 @@ from __future__ import annotations
 import torch
 
 from tokensprint_amd.kernels.stream import (NormAhead, NormedPair, NormedRows, RowsAhead, ShiftAhead,
-                                            StreamRows,                                            fused_rmsnorm_of)
+                                            ShiftEntry, StreamRows, fused_rmsnorm_of)
 from tokensprint_amd.parts.base import (BLOCKS, FEED_FORWARDS, FILTERS, MIXERS, NORMS, SIDES, Block,
                                         StreamFilter, TensorDecl, SlotStateNeed, register)
 
@@ -70,11 +70,12 @@ class SandwichNormBlock(Block):
             raise ValueError("sandwich_norm: a feed-forward comes with both of its norms")
         if (self.side is None) != (self.side_post_norm is None):
             raise ValueError("sandwich_norm: a side input and its norm come together")
+        hint_of = getattr(self.mixer_filter, "stream_hint", None)
+        self._filter_hint = hint_of(self.mixer_norm) if callable(hint_of) else None
 
     def entry_hint(self):
         if self.mixer_filter is not None:
-            probe = getattr(self.mixer_filter, "stream_hint", None)
-            return probe(self.mixer_norm) if callable(probe) else None
+            return self._filter_hint
         fused = fused_rmsnorm_of(self.mixer_norm)
         return None if fused is None else NormAhead(fused[0], fused[1])
 
@@ -117,9 +118,9 @@ class SandwichNormBlock(Block):
             h = delta.rows
         elif self.mixer_filter is not None:
             if delta is not None:
-                # a block in front that hands on a delta (with a filter this one gives no entry
-                # hint, so it is a plain tensor): added through the mixer's norm, whose output
-                # is not used
+                # a block in front of another kind, which takes no notice of the filter's hint
+                # and hands on a plain delta: added through the mixer's norm, whose output is
+                # not used
                 self.mixer_norm.add_forward(resid, delta)
             h = self.mixer_filter.forward_from_stream(resid, self.mixer_norm, batch, cache)
         else:
@@ -266,12 +267,7 @@ class TokenShift(StreamFilter):
         return SlotStateNeed((self.dim,), torch.float32, "shift")
 
     def stream_hint(self, norm):
-        """For the block in front: the norm and the shift, if its provider has them behind an
-        add."""
-        fused = fused_rmsnorm_of(norm)
-        if fused is None or not hasattr(self.ops, "postnorm_add_shift"):
-            return None
-        return ShiftAhead(fused[0], fused[1], self.weight)
+        return ShiftEntry(norm, self)
 
     def forward_from_stream(self, resid, norm, batch, cache):
         fused = fused_rmsnorm_of(norm)

@@ -253,7 +253,7 @@ class GatedDeltaRule(Mixer):
             z, z_col = proj, b_col + H
             gate, gate_col = proj, b_col + 2 * H
         gate_kind = "sigmoid" if self.per_channel else "silu"
-        if hasattr(ops, "delta_step"):       # steps of single tokens: the rest in one kernel
+        if batch.max_q_len == 1 and hasattr(ops, "delta_step"):    # single tokens: the rest in one kernel
             gated = ops.delta_step(qkv, proj, b_col, z, z_col, self.a_log, self.dt_bias, gate,
                                    gate_col, self.norm_w, batch, state, heads=H,
                                    kv_heads=self.kv_heads, dim=self.dim, vdim=self.vdim,
