@@ -419,6 +419,57 @@ def test_gemm_tiled_into_stream(ops, gpu_device, M, N, K, next_n, silu):
             assert excess <= 0, f"{name}: {excess} beyond the rounding bound"
 
 
+@pytest.mark.parametrize("M", [72, 128, 300, 511])
+@pytest.mark.parametrize("next_n, silu", [(3072, True), (1040, False)])
+def test_few_rows_into_the_stream(ops, gpu_device, monkeypatch, M, next_n, silu):
+    """Eager steps of 72 to 511 rows: the tiled forms through the provider, where the table and what
+    the step is run for send them there, and the same function of the stream as separate kernels."""
+    from dataclasses import replace
+    from tokensprint_amd.kernels.stream import NormHint, PreparedRows
+    bf, N, K, eps = torch.bfloat16, 1024, 1024, 1e-5
+    x, w = rand((M, K), bf, gpu_device, 70), rand((N, K), bf, gpu_device, 71, scale=0.03)
+    resid = rand((M, N), torch.float32, gpu_device, 72)
+    g = rand((N,), torch.float32, gpu_device, 73).abs() + 0.5
+    wn = rand((next_n * (1 + silu), N), bf, gpu_device, 74, scale=0.05)
+    hint = NormHint(g, eps, wn, silu)
+
+    def taken(rows=x, weight=w, stream=None):
+        return ops.linear_into_stream(rows, weight, resid.clone() if stream is None else stream, hint)
+
+    stream = resid.clone()
+    prepared = taken(stream=stream)
+    assert isinstance(prepared, PreparedRows) and prepared.tiled
+    # the product is rounded to bfloat16 before it is added
+    torch.testing.assert_close(stream - resid, x.float() @ w.float().T, rtol=1e-2, atol=1e-2)
+    out, same = ops.norm_linear(stream, prepared, g, eps, wn, bf, silu_mul=silu)
+    assert same is stream
+    h = stream.double() * torch.rsqrt((stream.double() ** 2).mean(1, keepdim=True) + eps) * g.double()
+    want = h @ wn.double().T
+    # operands 2^-9 off: noise of 2^-9 sqrt(N) rms(h) rms(w), six of it for the largest of so many
+    slack = 6 * 2.0 ** -9 * N ** 0.5 * float(h.pow(2).mean().sqrt() * wn.double().pow(2).mean().sqrt())
+    if silu:
+        gate, up = want[:, :next_n], want[:, next_n:]
+        want, slack = gate * torch.sigmoid(gate) * up, slack * (1 + gate.abs() + up.abs())
+    assert ((out.double() - want).abs() <= slack + 0.01 * want.abs()).all()
+
+    # fewer rows and smaller weights keep the separate kernels, and nothing is done to the stream
+    kept = resid.clone()
+    assert taken(rows=x[:71].contiguous(), stream=kept[:71]) is None and torch.equal(kept, resid)
+    assert taken(rows=x[:, :512].contiguous(), weight=w[:, :512].contiguous()) is None
+    # a step that is run to be captured does, too; then an eager one takes them again
+    before = ops.timed_plans(True)
+    try:
+        assert taken() is None
+    finally:
+        ops.timed_plans(before)
+    assert taken().tiled
+    # another table is asked anew
+    monkeypatch.setattr(ops, "dispatch", replace(ops.dispatch, tiled_stream_few_rows=512))
+    assert taken() is None
+    monkeypatch.undo()
+    assert taken().tiled
+
+
 def test_gemm_tiled_refuses_what_it_cannot_take(ops, gpu_device):
     x = rand((100, 200), torch.bfloat16, gpu_device, 54)
     w = rand((64, 200), torch.bfloat16, gpu_device, 55)

@@ -124,8 +124,8 @@ class HipOps:
         # for the vendor library's algorithms that want scratch memory during a product
         self._library_workspace = torch.empty(64 << 20, dtype=torch.uint8, device=self.device)
         self._timed_plans = False
-        # which kernels end a sub-layer, by sizes, as `_stream_routes_of` (a dispatch table) has it
-        self._stream_routes, self._stream_routes_of = {}, self.dispatch
+        # which kernels make a product, by sizes, as `_routes_of` (a dispatch table) has it
+        self._routes, self._routes_of = {}, self.dispatch
         self._staging, self._staging_turn = [None] * 4, -1      # pinned buffers of _upload_ints
         # products of few rows with large weights: ours or the library's, per weight shape
         # (see large_weight_choices)
@@ -402,12 +402,23 @@ class HipOps:
 
     def _tiled_plain_ok(self, M, N, K, x_dtype, w_dtype, out_dtype):
         d = self.dispatch
-        return (x_dtype == torch.bfloat16 and w_dtype == torch.bfloat16
-                and out_dtype in (torch.bfloat16, torch.float32)
-                and self.lib.ts_gemm_tiled_fits(M, N, K, 0) == 1
-                and (M >= d.tiled_stream_rows and N * K <= d.tiled_plain_weight
-                     or M >= d.library_rows
-                     and self.lib.ts_gemm_tiled_ahead(M, N, K, _TYPE_CODE[out_dtype]) == 1))
+        if M < min(d.tiled_stream_rows, d.library_rows) or x_dtype != torch.bfloat16 \
+                or w_dtype != torch.bfloat16 or out_dtype not in (torch.bfloat16, torch.float32):
+            return False
+        routes, key = self._kept_routes(), (M, N, K, out_dtype)
+        if key not in routes:
+            routes[key] = self.lib.ts_gemm_tiled_fits(M, N, K, 0) == 1 and (
+                M >= d.tiled_stream_rows and N * K <= d.tiled_plain_weight
+                or M >= d.library_rows
+                and self.lib.ts_gemm_tiled_ahead(M, N, K, _TYPE_CODE[out_dtype]) == 1)
+        return routes[key]
+
+    def _kept_routes(self):
+        """Answers by sizes alone, of the dispatch table that is in use (a step asks for every layer,
+        in calls into the library)."""
+        if self._routes_of is not self.dispatch or len(self._routes) > 4096:
+            self._routes, self._routes_of = {}, self.dispatch
+        return self._routes
 
     def _library_ok(self, x, weight, pair=False):
         if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
@@ -517,17 +528,15 @@ class HipOps:
         separate kernels.  Sizes and the dispatch table decide (and, for large weights, the
         warm-up's choice), so the answer for small weights is kept by sizes: a step asks for every
         layer, in half a dozen calls into the library."""
-        wn = hint.weight
-        small = N * K <= self.dispatch.large_weight and wn.numel() <= self.dispatch.large_weight
+        wn, d = hint.weight, self.dispatch
+        small = N * K <= d.large_weight and wn.numel() <= d.large_weight
         # a step that is captured, or run to be, does not wait for the host
-        eager = not (self._timed_plans or torch.cuda.is_current_stream_capturing())
+        eager = d.tiled_stream_few_rows <= M < d.tiled_stream_rows \
+            and not (self._timed_plans or torch.cuda.is_current_stream_capturing())
         key = (M, N, K, wn.shape, hint.silu_mul, eager)
-        if small:
-            if self._stream_routes_of is not self.dispatch or len(self._stream_routes) > 4096:
-                self._stream_routes, self._stream_routes_of = {}, self.dispatch
-            found = self._stream_routes.get(key)
-            if found is not None:
-                return found
+        routes = self._kept_routes() if small else {}
+        if key in routes:
+            return routes[key]
         next_n = wn.shape[0] // 2 if hint.silu_mul else wn.shape[0]
         if self._tiled_stream_ok(M, N, K, hint, eager):
             route = True, self.lib.ts_gemm_tiled_tail_parts(N)
@@ -539,8 +548,7 @@ class HipOps:
                     or self.lib.ts_gemm_scaled_fits(M, next_n, N, int(hint.silu_mul), parts) != 1:
                 parts = 0
             route = False, parts
-        if small:
-            self._stream_routes[key] = route
+        routes[key] = route
         return route
 
     def _tiled_stream_ok(self, M, N, K, hint, eager=True):
