@@ -78,12 +78,14 @@ class Dispatch:
     #: these forms at the 8B shape, 0.98 to 1.06 at the 32B shape.
     tiled_stream_weight: int = 1 << 23
     #: Weights of `tiled_stream_few_weight` to `large_weight` elements take it from fewer rows in
-    #: an eager step (captured ones, of up to 256 single tokens, do not: 4.99 against 4.77 ms): a
-    #: step of the 0.6B shape with 300 tokens 2,117 -> 2,042 us on the GPU, with 128 1,738 -> 2,116
-    #: (N = 1,024 fills few units), but in an eager step, where two norm kernels and three library
-    #: calls a layer held the host up, 3,400 -> 2,050 and 2,150.  (Fewer rows leave nearly half of a tile
-    #: of 128 empty; smaller weights keep the separate kernels, through which portions below 512 rows
-    #: of small models are tested.)
+    #: an eager step (captured ones, of up to 256 single tokens, do not: 4.99 against 4.77 ms), where
+    #: two norm kernels and three library calls a layer hold the host up: a step of the 0.6B shape
+    #: with 300 tokens 3,400 -> 2,050 us (2,117 -> 2,042 on the GPU), with 128 3,400 -> 2,150 (1,738 ->
+    #: 2,116 on the GPU: N = 1,024 fills few units).  Fewer rows leave nearly half of a tile of 128
+    #: empty.  The lower line of weights is none of speed: below it the forms are ahead as well
+    #: (products and norms of a layer of hidden size 512, 72 to 511 rows, 76 -> 35 us eager and 30 to 33
+    #: -> 27 to 31 on the GPU), but portions below 512 rows of such models have had the separate kernels,
+    #: and their sums in another order, all along.
     tiled_stream_few_rows: int = 72
     tiled_stream_few_weight: int = 1 << 20
     #: Plain products: from `tiled_stream_rows` rows and up to so many elements the tiled
