@@ -326,11 +326,14 @@ class HipOps:
         N = weight.shape[0]
         if weight.shape[1] != K:
             raise ValueError(f"linear: x has {K} columns, weight has {weight.shape[1]}")
-        if self._tiled_plain_ok(M, N, K, x.dtype, weight.dtype, out_dtype):
+        d = self.dispatch
+        many = (M >= d.library_rows or M >= d.tiled_stream_rows) \
+            and x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16
+        if many and self._tiled_plain_ok(M, N, K, out_dtype):
             # a prompt's portion at small weights: as fast as the library's product on the
             # GPU and a fifth of its cost on the host (which a step's first layer waits for)
             return self.gemm_tiled(x, weight, out_dtype)
-        if self._library_ok(x, weight):
+        if many and M >= d.library_rows or self._library_ok(x, weight):
             # the library's float32 sums leave in the type asked for: bfloat16 activations,
             # float32 logits at the output head (not rounded to bfloat16 and widened, so
             # that logits are of one precision on both sides of the row count at which
@@ -400,18 +403,19 @@ class HipOps:
                      or self.lib.ts_gemm_tiled_fill(M, inner, K, 1) >= (
                          d.tiled_fill if weight.numel() <= d.tiled_pair_weight else d.tiled_fill_large)))
 
-    def _tiled_plain_ok(self, M, N, K, x_dtype, w_dtype, out_dtype):
-        d = self.dispatch
-        if M < min(d.tiled_stream_rows, d.library_rows) or x_dtype != torch.bfloat16 \
-                or w_dtype != torch.bfloat16 or out_dtype not in (torch.bfloat16, torch.float32):
-            return False
+    def _tiled_plain_ok(self, M, N, K, out_dtype):
+        """Whether a bfloat16 product of many rows is the LDS-tiled kernel's."""
         routes, key = self._kept_routes(), (M, N, K, out_dtype)
-        if key not in routes:
-            routes[key] = self.lib.ts_gemm_tiled_fits(M, N, K, 0) == 1 and (
-                M >= d.tiled_stream_rows and N * K <= d.tiled_plain_weight
-                or M >= d.library_rows
-                and self.lib.ts_gemm_tiled_ahead(M, N, K, _TYPE_CODE[out_dtype]) == 1)
-        return routes[key]
+        found = routes.get(key)
+        if found is None:
+            d = self.dispatch
+            found = routes[key] = (
+                out_dtype in (torch.bfloat16, torch.float32)
+                and self.lib.ts_gemm_tiled_fits(M, N, K, 0) == 1
+                and (M >= d.tiled_stream_rows and N * K <= d.tiled_plain_weight
+                     or M >= d.library_rows
+                     and self.lib.ts_gemm_tiled_ahead(M, N, K, _TYPE_CODE[out_dtype]) == 1))
+        return found
 
     def _kept_routes(self):
         """Answers by sizes alone, of the dispatch table that is in use (a step asks for every layer,
