@@ -25,12 +25,13 @@ class Dispatch:
     #: in the wide layout (a short K: four waves along N) the library is ahead from 17 rows
     library_rows_wide: int = 17
     #: at the output head (N from `head_columns`: every one of thousands of workgroups
-    #: reads all rows of x, so the line lies lower the longer they are) from 9 rows, with K above
-    #: 2,048 from 7, above 4,096 from 5; float32 logits here, of the time of the library's
-    #: algorithm that is fastest with the weights in memory: N = 151,936, K = 1,024 8 rows 0.98,
-    #: 9 rows 1.01, K = 2,048 0.95 and 1.01, K = 4,096 6 rows 0.97, 7 rows 1.00, 8 rows 1.02,
-    #: K = 5,120 4 rows 0.99, 5 rows 1.01; 128,256 x 4,096 0.97, 1.01, 1.02; 65,536 x 2,048 8 rows
-    #: 0.95, 9 rows 0.99; 20,000 x 8,192 6 rows 0.99, 7 rows 1.01
+    #: reads all rows of x) from 9 rows: float32 logits of 8 and 9 rows here, of the time of the
+    #: library's first algorithm, N = 151,936 and K = 1,024 0.98 and 1.02, K = 4,096 0.89 and 0.96,
+    #: K = 5,120 1.00 and 1.09; 128,256 x 4,096 1.00 and 1.09; 32,000 x 2,048 0.85 and 0.90.  Steps that
+    #: are captured, or run to be, have the algorithm that is fastest with the weights in memory:
+    #: there from 7 rows with K above 2,048 (K = 4,096 6 rows 0.97, 7 rows 1.00, 8 rows 1.02) and from
+    #: 5 above 4,096 (K = 5,120 4 rows 0.99, 5 rows 1.01; 8,192 6 rows 0.99, 7 rows 1.01), below as
+    #: before (K = 2,048 8 rows 0.95, 9 rows 1.01)
     library_rows_head: int = 9
     library_rows_long_head: int = 7
     library_rows_longest_head: int = 5

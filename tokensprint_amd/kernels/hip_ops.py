@@ -463,10 +463,13 @@ class HipOps:
         if pair:
             if M >= d.library_rows_pair and pair > d.pair_head_weight:
                 return True
-        elif N >= d.head_columns and M >= (
-                d.library_rows_head if K <= 2048 else
-                d.library_rows_long_head if K <= 4096 else d.library_rows_longest_head):
-            return True
+        elif N >= d.head_columns and M >= d.library_rows_longest_head:
+            rows = d.library_rows_head
+            if K > 2048 and M < rows and (self._timed_plans
+                                          or torch.cuda.is_current_stream_capturing()):
+                rows = d.library_rows_long_head if K <= 4096 else d.library_rows_longest_head
+            if M >= rows:
+                return True
         if N * K > d.large_weight:
             rows = self._large_rows.get((N, K))
             if rows is None:
