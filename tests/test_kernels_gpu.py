@@ -300,7 +300,8 @@ def test_rows_of_an_output_head(ops, gpu_device, K, first):
     (300, 151936, 1024, 0), (512, 151936, 1024, 1),
     # N a multiple of 256
     (432, 4096, 4096, 1), (5288, 6144, 4096, 0), (3000, 5120, 8192, 0), (1536, 5120, 25600, 1),
-    (3100, 5120, 25600, 0), (8192, 5120, 25600, 1), (8192, 10240, 5120, 0)])
+    (3100, 5120, 25600, 0), (3400, 5120, 25600, 1), (8192, 5120, 25600, 1), (1600, 4096, 12288, 1),
+    (4200, 4096, 12288, 1), (4700, 4096, 4096, 0), (4000, 10240, 5120, 1), (8192, 10240, 5120, 0)])
 def test_plain_products_by_the_faster_kernel(ops, M, N, K, ahead):
     assert ops.lib.ts_gemm_tiled_ahead(M, N, K, 1) == ahead
 

@@ -36,14 +36,15 @@ extern "C" int ts_gemm_tiled_fill(int M, int N, int K, int pair) {
 // K = 4,096 and 8,192 0.81 to 1.01 from seven tenths on (up to 1,024 rows of up to 4,096 columns of
 // 4,096 0.90 to 1.04 from a half on), up to 3.4 below (65 rows of 64 columns of 8,192).  151,936
 // columns: 0.82 to 0.95 from seven tenths on, up to 1.11 below.
-// N a multiple of 256, float32 out: 0.87 to 1.05 from four fifths filled, 0.95 in the mean.  bfloat16
-// out, four fifths filled: 0.62 to 1.00 where the tiles are 128 x 128 or smaller; with larger ones the
-// library's 256 x 256 mostly is as good or ahead (0.97 to 1.17), but for long K (K from 5,120): one
-// round of 256 x 128 0.67 to 0.99, and more than two rounds of 256 x 256 of which the last is not
-// full 0.72 to 0.87.  With the longest K the library often is at half of its rate: K = 25,600 0.65
-// to 0.97 in one round of up to 256 x 128, whatever it fills (5,120 columns, 1,536 rows 338 / 507
-// us), with larger tiles 0.58 to 1.08 from six (one round) or seven tenths on, 0.87 in the mean (8,192
-// rows 1,610 / 2,090).
+// N a multiple of 256, float32 out: 0.87 to 1.06 from four fifths filled, 0.95 in the mean.  bfloat16
+// out, timed at 74 row counts of eight weights (N 2,048 to 10,240, K 2,048 to 25,600): where the
+// tiles are 128 x 128 or smaller and four fifths filled 0.62 to 1.00; with larger ones the
+// library's 256 x 256 mostly is as good or ahead (0.97 to 1.17), but for long K, where it often
+// falls to half of its rate.  K from 5,120: one round of 256 x 128 three quarters filled 0.54 to 1.04,
+// and two to three rounds of 256 x 256 0.65 to 1.11, 0.83 in the mean.  K = 12,288 and 25,600: more
+// than one such round 0.59 to 1.09, 0.80 in the mean, filled by two thirds (tiles of 256 x 128 in
+// several rounds 1.11 to 1.19).  K = 25,600: one round of up to 256 x 128 0.65 to 0.97 whatever it fills
+// (5,120 columns, 1,536 rows 338 / 507 us), of larger tiles 0.58 to 1.10, 0.88 in the mean.
 extern "C" int ts_gemm_tiled_ahead(int M, int N, int K, int c_type) {
   if (!ts_gemm_tiled_fits(M, N, K, 0)) return 0;
   const int fill = ts_gemm_tiled_fill(M, N, K, 0);
@@ -52,25 +53,21 @@ extern "C" int ts_gemm_tiled_ahead(int M, int N, int K, int c_type) {
     if (N < 16384 && K < 2240) return fill >= K / 32;
     return fill >= (K <= 6144 && N <= 4096 && M <= 1024 ? 49 : 70);
   }
-  const bool longest = K >= 16384;
-  if (fill < (longest ? 45 : 80)) return 0;
   if (c_type != TS_BF16 && fill >= 80) return 1;
   TiledArgs g{};
   g.M = M, g.N = N, g.K = K;
   const int tile = cheapest_tile(g, false), units = compute_units();
+  int64_t area = 0, tiles = 0;
   for (const TileCost& t : kTileCosts) {
     if (t.tile != tile) continue;
-    const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-    if (t.bm * t.bn <= 128 * 128) return 1;
-    if (K < 5120) return 0;
-    if (t.bm * t.bn == 256 * 128) {
-      if (tiles <= units) return 1;
-    } else if (longest) {
-      return fill >= (tiles <= units ? 60 : 70);
-    }
+    area = t.bm * t.bn, tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
   }
-  const int64_t squares = (int64_t)((M + 255) / 256) * (N / 256), rounds = (squares + units - 1) / units;
-  return rounds > 2 && squares * 10 < rounds * units * 9;
+  const int64_t squares = (int64_t)((M + 255) / 256) * (N / 256);
+  if (K >= 12288 && squares > units) return area != 256 * 128 && fill >= 66;
+  if (K >= 5120 && squares > 2 * units && squares <= 3 * units) return fill >= 73;
+  if (K >= 16384) return fill >= (area <= 256 * 128 ? 45 : 60);
+  if (area == 256 * 128) return K >= 5120 && tiles <= units && fill >= 75;
+  return area <= 128 * 128 && fill >= 80;
 }
 
 // C[M, N] = A[M, K] W[N, K]^T, or with `pair` C[M, N] = silu(A Wg^T) * (A Wu^T) (or, with a
