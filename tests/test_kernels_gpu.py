@@ -317,7 +317,8 @@ def test_narrow_products_of_many_rows(ops, gpu_device, M, N, K):
 
 
 @pytest.mark.parametrize("M, inner, K, tiled", [
-    (900, 25600, 5120, False), (960, 25600, 5120, False), (1000, 25600, 5120, True),
+    (600, 25600, 5120, False), (650, 25600, 5120, True), (900, 25600, 5120, False),
+    (960, 25600, 5120, False), (1000, 25600, 5120, True),
     (520, 12288, 4096, False), (700, 12288, 4096, True)])
 def test_gate_up_products_that_fill_their_rounds(ops, M, inner, K, tiled):
     x = torch.empty(M, K, dtype=torch.bfloat16, device="meta")

@@ -64,10 +64,12 @@ class Dispatch:
     #: also have to fill so many per cent of their tiles' rounds
     #: (`ts_gemm_tiled_fill`): gate/up products at 46 row counts from 260 to 6,400 take 0.79 to 1.04
     #: of the library's and the SiLU kernel's time from 65 per cent on, 0.92 in the mean, and 1.04
-    #: below, up to 1.14; the largest weights (above `tiled_pair_weight`) 0.80 to 0.95 from 75 per
-    #: cent on, and 0.87 to 1.04 from 65 to 75, in a step of 900 rows of the 32B shape 1.10.
+    #: below, up to 1.14; the largest weights (above `tiled_pair_weight`) 0.85 to 0.87 at 650 to 750
+    #: rows, above `tiled_fill_large_rows` 0.80 to 0.95 from 75 per cent on, and 1.00 to 1.04 from 65 to
+    #: 75, in a step of 900 rows of the 32B shape 1.10.
     tiled_fill: int = 65
     tiled_fill_large: int = 75
+    tiled_fill_large_rows: int = 768
     tiled_fill_rows: int = 256
     #: rows from which, and elements of a weight [N, K] up to which, the product that ends a
     #: sub-layer is the LDS-tiled kernel's tail form (it adds itself into the float32 stream

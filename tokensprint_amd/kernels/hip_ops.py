@@ -401,7 +401,8 @@ class HipOps:
                 and self.lib.ts_gemm_tiled_fits(M, inner, K, 1) == 1
                 and (weight.numel() <= d.large_weight or M < d.tiled_fill_rows
                      or self.lib.ts_gemm_tiled_fill(M, inner, K, 1) >= (
-                         d.tiled_fill if weight.numel() <= d.tiled_pair_weight else d.tiled_fill_large)))
+                         d.tiled_fill if weight.numel() <= d.tiled_pair_weight
+                         or M <= d.tiled_fill_large_rows else d.tiled_fill_large)))
 
     def _tiled_plain_ok(self, M, N, K, out_dtype):
         """Whether a bfloat16 product of many rows is the LDS-tiled kernel's."""
