@@ -566,6 +566,8 @@ int gemm_f32_split_launch(const float* A, const float* W, float* C, int M, int N
   }
 }
 
+// The product by a tile's number (0: the sizes' choice), for tests and measuring; ts_gemm_fma is the
+// call for everything else.
 extern "C" int ts_gemm_f32_split(const float* a, const float* w, float* c, int M, int N, int K, int tile,
                                  hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
