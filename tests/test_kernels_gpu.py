@@ -296,7 +296,7 @@ def test_rows_of_an_output_head(ops, gpu_device, K, first):
 @pytest.mark.parametrize("M, N, K, ahead", [
     # N no multiple of 256: narrow products of a long K, whose few tiles each walk all of it
     (65, 64, 8192, 0), (96, 208, 2048, 0), (66, 576, 2048, 0), (300, 288, 1024, 0), (96, 2192, 2048, 0),
-    (262, 6176, 2048, 0), (65, 48, 512, 1), (65, 4640, 1024, 1), (676, 10304, 2048, 1),
+    (262, 6176, 2048, 0), (700, 6176, 2048, 0), (330, 6176, 2048, 1), (66, 10304, 2048, 1), (65, 48, 512, 1), (65, 4640, 1024, 1), (676, 10304, 2048, 1),
     (300, 151936, 1024, 0), (512, 151936, 1024, 1),
     # N a multiple of 256
     (432, 4096, 4096, 1), (5288, 6144, 4096, 0), (3000, 5120, 8192, 0), (1536, 5120, 25600, 1),

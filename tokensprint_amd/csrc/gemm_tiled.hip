@@ -32,7 +32,9 @@ extern "C" int ts_gemm_tiled_fill(int M, int N, int K, int pair) {
 // 65 to 8,192 rows, the weights in memory; times of the library's.
 // N no multiple of 256, N 16 to 10,304: the longer K, the more of the tiles' rounds has to be
 // filled.  K = 512 0.22 to 1.01 from 48 columns; K = 1,024 0.74 to 0.92 from 1,296 columns, 1.1 to
-// 1.3 below with less than a third filled; K = 2,048 0.78 to 1.05 from two thirds on, up to 1.8 below;
+// 1.3 below with less than a quarter filled; K = 2,048 below 512 rows 0.79 to 1.06 from a half on, 0.92 in
+// the mean, and up to 128 rows of at least 6,176 columns 0.93 to 1.00, up to 1.8 else; from 512 rows 0.78 to
+// 1.05 from two thirds on, up to 1.13 below;
 // K = 4,096 and 8,192 0.81 to 1.01 from seven tenths on (up to 1,024 rows of up to 4,096 columns of
 // 4,096 0.90 to 1.04 from a half on), up to 3.4 below (65 rows of 64 columns of 8,192).  151,936
 // columns: 0.82 to 0.95 from seven tenths on, up to 1.11 below.
@@ -50,7 +52,7 @@ extern "C" int ts_gemm_tiled_ahead(int M, int N, int K, int c_type) {
   const int fill = ts_gemm_tiled_fill(M, N, K, 0);
   if (N % 256 != 0) {
     if (N < 16384 && (K <= 512 ? N >= 48 : K <= 1024 && N >= 1280)) return 1;
-    if (N < 16384 && K < 2240) return fill >= K / 32;
+    if (N < 16384 && K < 2240) return M <= 128 && N >= 6144 ? 1 : fill >= (M < 512 ? 3 * K / 128 : K / 32);
     return fill >= (K <= 6144 && N <= 4096 && M <= 1024 ? 49 : 70);
   }
   if (c_type != TS_BF16 && fill >= 80) return 1;

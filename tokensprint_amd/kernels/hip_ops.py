@@ -406,11 +406,10 @@ class HipOps:
 
     def _tiled_plain_ok(self, M, N, K, out_dtype):
         """Whether a bfloat16 product of many rows is the LDS-tiled kernel's."""
-        routes, key = self._kept_routes(), (M, N, K, out_dtype)
-        found = routes.get(key)
+        d, key = self.dispatch, (M, N, K, out_dtype)
+        found = self._routes.get(key) if self._routes_of is d else None
         if found is None:
-            d = self.dispatch
-            found = routes[key] = (
+            found = self._kept_routes()[key] = (
                 out_dtype in (torch.bfloat16, torch.float32)
                 and self.lib.ts_gemm_tiled_fits(M, N, K, 0) == 1
                 and (M >= d.tiled_stream_rows and N * K <= d.tiled_plain_weight
@@ -420,7 +419,7 @@ class HipOps:
 
     def _kept_routes(self):
         """Answers by sizes alone, of the dispatch table that is in use (a step asks for every layer,
-        in calls into the library)."""
+        in calls into the library): where a new one is put."""
         if self._routes_of is not self.dispatch or len(self._routes) > 4096:
             self._routes, self._routes_of = {}, self.dispatch
         return self._routes
@@ -537,14 +536,13 @@ class HipOps:
         warm-up's choice), so the answer for small weights is kept by sizes: a step asks for every
         layer, in half a dozen calls into the library."""
         wn, d = hint.weight, self.dispatch
-        small = N * K <= d.large_weight and wn.numel() <= d.large_weight
         # a step that is captured, or run to be, does not wait for the host
         eager = d.tiled_stream_few_rows <= M < d.tiled_stream_rows \
             and not (self._timed_plans or torch.cuda.is_current_stream_capturing())
         key = (M, N, K, wn.shape, hint.silu_mul, eager)
-        routes = self._kept_routes() if small else {}
-        if key in routes:
-            return routes[key]
+        found = self._routes.get(key) if self._routes_of is d else None
+        if found is not None:
+            return found
         next_n = wn.shape[0] // 2 if hint.silu_mul else wn.shape[0]
         if self._tiled_stream_ok(M, N, K, hint, eager):
             route = True, self.lib.ts_gemm_tiled_tail_parts(N)
@@ -556,7 +554,8 @@ class HipOps:
                     or self.lib.ts_gemm_scaled_fits(M, next_n, N, int(hint.silu_mul), parts) != 1:
                 parts = 0
             route = False, parts
-        routes[key] = route
+        if N * K <= d.large_weight and wn.numel() <= d.large_weight:
+            self._kept_routes()[key] = route
         return route
 
     def _tiled_stream_ok(self, M, N, K, hint, eager=True):
