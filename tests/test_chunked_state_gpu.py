@@ -184,6 +184,82 @@ def test_state_space_scan_in_chunks(gpu_device, heads, groups, rows, vdim):
         no_further_off(st[slots], st_walked[slots], torch.stack(want_state))
 
 
+# (eight workgroups of 16 columns to every 64 tokens of the longest portion: two launches)
+@pytest.mark.parametrize("mode, heads, kv_heads, dim, vdim", [
+    ("per_head_plain", 32, 4, 20, 5), ("per_head_plain", 12, 3, 50, 40), ("per_head_plain", 8, 8, 128, 64),
+    ("fixed", 4, 4, 20, 113), ("fixed", 4, 2, 50, 128), ("fixed", 4, 1, 100, 115),
+    ("turned", 4, 4, 20, 128), ("turned", 4, 1, 65, 120), ("turned", 4, 2, 36, 113)])
+def test_linear_recurrence_in_two_launches(gpu_device, mode, heads, kv_heads, dim, vdim):
+    test_linear_recurrence_in_chunks(gpu_device, mode, heads, kv_heads, dim, vdim)
+
+
+@pytest.mark.parametrize("heads, groups, rows, vdim", [(64, 8, 32, 16), (32, 4, 33, 15), (16, 2, 65, 18)])
+def test_state_space_scan_in_two_launches(gpu_device, heads, groups, rows, vdim):
+    test_state_space_scan_in_chunks(gpu_device, heads, groups, rows, vdim)
+
+
+@pytest.mark.parametrize("tokens", [16, 17, 63, 64, 65, 128, 129, 192, 193, 209, 272])
+def test_two_launches_at_every_number_of_chunks(gpu_device, tokens):
+    """The walk's loops turn by turn: one chunk to five, the last of one tile, of more, whole."""
+    ops, gen = load_hip_ops(gpu_device), torch.Generator().manual_seed(15)
+    heads, dim, vdim = 40, 40, 17
+    requests = Requests(gpu_device, (heads, dim, vdim), 2)
+    spans = [tokens, 1]
+    batch = requests.step(spans)
+    x = torch.randn(sum(spans), heads * (2 * dim + vdim), generator=gen)
+    gates = torch.cat([torch.rand(sum(spans), heads, generator=gen),
+                       torch.rand(sum(spans), heads, generator=gen) ** 0.1], 1)
+    x_dev, gates_dev = x.to(gpu_device), gates.to(gpu_device)
+    (got, st), (walked, st_walked) = in_chunks_and_walked(
+        ops, lambda: ops.linear_recurrence(
+            x_dev, 0, heads * dim, 2 * heads * dim, batch, requests.state, heads=heads, kv_heads=heads,
+            dim=dim, vdim=vdim, silu_inputs=False, gates=gates_dev), requests.state)
+    q, k, v = x.double().split([heads * dim] * 2 + [heads * vdim], 1)
+    q, k, v = q.view(-1, heads, dim), k.view(-1, heads, dim), v.view(-1, heads, vdim)
+    g, at, want, states = gates[:, heads:, None].double(), 0, [], []
+    for n in spans:
+        r = slice(at, at + n)
+        out, S = walk(q[r], k[r], v[r], g[r], None, torch.zeros(heads, dim, vdim, dtype=torch.float64))
+        want.append(out)
+        states.append(S)
+        at += n
+    no_further_off(got, walked, torch.cat(want).view(at, -1))
+    slots = batch.slot_ids.long()
+    no_further_off(st[slots], st_walked[slots], torch.stack(states))
+
+
+@pytest.mark.parametrize("what", ["q", "k", "v"])
+def test_two_launches_keep_what_is_not_finite_from_earlier_tokens(gpu_device, what):
+    ops, gen = load_hip_ops(gpu_device), torch.Generator().manual_seed(16)
+    kept, spans = ops.dispatch, [150, 70]
+    heads, kv_heads, dim, vdim = 16, 4, 64, 33
+    x = torch.randn(sum(spans), 2 * kv_heads * dim + heads * vdim, generator=gen)
+    decay = 0.9 + 0.02 * torch.randn(heads, generator=gen).tanh().to(gpu_device)
+    column = {"q": 0, "k": kv_heads * dim, "v": 2 * kv_heads * dim}[what]
+
+    def run(x):
+        requests = Requests(gpu_device, (heads, dim, vdim), 2)
+        batch = requests.step(spans)
+        ops.dispatch = dataclasses.replace(kept, scan_whole_tokens=16)
+        try:
+            return ops.linear_recurrence(
+                x.to(gpu_device), 0, kv_heads * dim, 2 * kv_heads * dim, batch, requests.state,
+                heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, silu_inputs=False, decay=decay)
+        finally:
+            ops.dispatch = kept
+
+    want = run(x)
+    for t in (0, 5, 37, 63, 64, 79, 140):
+        for value in (float("inf"), float("nan")):
+            xs = x.clone()
+            xs[t, column] = value
+            out = run(xs)
+            assert torch.equal(out[:t], want[:t]) and torch.equal(out[150:], want[150:]), (t, value)
+            assert not out[t].isfinite().all(), (t, value)
+            if what == "q":
+                assert torch.equal(out[t + 1:], want[t + 1:]), (t, value)
+
+
 @pytest.mark.parametrize("per_channel", [False, True])
 def test_delta_rule_takes_silu_of_its_operands_in_long_portions(gpu_device, per_channel):
     ops, gen = load_hip_ops(gpu_device), torch.Generator().manual_seed(9)

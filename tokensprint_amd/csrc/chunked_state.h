@@ -33,9 +33,10 @@ struct ChunkedArgs {
   const int* chunks;          // [num_chunks, 3]: first token, one past the last, entry
   const int* entry_chunks;    // [B + 1]
   int num_chunks, num_entries;
+  int max_len;                // the most tokens an entry brings
   float* scratch;             // chunked_scratch_floats of them, 16-byte aligned
 };
 
 // Floats of scratch that launch_chunked wants; -1: these sizes are not built in chunks.
-int64_t chunked_scratch_floats(int num_chunks, int heads, int N, int P, int delta);
+int64_t chunked_scratch_floats(int num_chunks, int heads, int kv_heads, int N, int P, int delta);
 int launch_chunked(ChunkedArgs a, hipStream_t stream);

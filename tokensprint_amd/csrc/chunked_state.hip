@@ -14,7 +14,8 @@
 //
 //   u_t + beta_t sum_(s < t) M(t, s) (k_t . k_s) u_s = beta_t v_t - beta_t D(t) S0^T k_t,
 //
-// whose solution is Y - W S0 with Y and W that do not know S0.  So there are three launches:
+// whose solution is Y - W S0 with Y and W that do not know S0.  So there are three launches (or, for
+// linear forms in portions that are not too long, two: chunk_prepare and chunk_scan, below):
 //   * every chunk by itself: its contribution to S (linear forms: chunk_local), or Y, W and the
 //     decayed keys (delta rule: chunk_solve);
 //   * the chunks of an entry in order: the state in front of each (chunk_carry, a multiply-add
@@ -35,8 +36,8 @@
 // brackets the launches as they run in a prompt's step): delta rule, 16 heads of 128 x 128, 592 and
 // 126 us (solve 37, walk 60, output 37); 8 heads of 64 x 128 with a decay per row 469 and 81 (27,
 // 35, 24); fixed decays, 16 heads of 128 x 128, 230 and 78 (local 29, carry 22, output 44); state
-// space, 64 heads of 128 x 64, 386 and 123 (41, 31, 67).  The short chains of product_step and the
-// decays in 64 bits are 1 to 10 us of that.
+// space, 64 heads of 128 x 64, 386 and 123 (41, 31, 67), in two launches 101 (27, 73).  The short
+// chains of product_step and the decays in 64 bits are 1 to 10 us of that.
 //
 // Matrix operands: lane (g, l) = (lane / 16, lane % 16) holds row l of A, column l of B, and rows
 // 4 g + r, column l of the sum.  The four steps of a 16-deep product take k = 4 g + r in step r
@@ -45,6 +46,7 @@
 // order, so every access to it is 16 bytes a lane, side by side.
 #include "chunked_state.h"
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -95,9 +97,10 @@ __device__ __forceinline__ int tri_row(int t) { return t >= 6 ? 3 : t >= 3 ? 2 :
 struct Parts {
   int64_t starts, totals, u, w, kt, end;
 };
+__host__ __device__ inline int64_t padded_rows(int N) { return N <= 32 ? 32 : N <= 64 ? 64 : N <= 128 ? 128 : 256; }
 __host__ __device__ inline Parts parts_of(int num_chunks, int heads, int N, int P, int delta) {
   const int64_t units = (int64_t)num_chunks * heads;
-  const int64_t np = (N + 15) / 16 * 16 <= 32 ? 32 : N <= 64 ? 64 : N <= 128 ? 128 : 256;
+  const int64_t np = padded_rows(N);
   const int64_t pp = (P + 15) / 16 * 16;
   Parts p;
   p.starts = 0;                                            // S in front of a chunk, [PT][NT][64][4]
@@ -106,6 +109,22 @@ __host__ __device__ inline Parts parts_of(int num_chunks, int heads, int N, int 
   p.w = p.u + (delta ? units * kTok * pp : 0);             // -W: [4][NT][64][4]
   p.kt = p.w + (delta ? units * kTok * np : 0);            // decayed keys: [NT][4][64][4]
   p.end = p.kt + (delta ? units * kTok * np : 0);
+  return p;
+}
+
+// The same for linear forms in two launches.
+struct ScanParts {
+  int64_t q, k, p, d0, scale, end;
+};
+__host__ __device__ inline ScanParts scan_parts_of(int num_chunks, int heads, int kv_heads, int N) {
+  const int64_t units = (int64_t)num_chunks * heads, shared = (int64_t)num_chunks * kv_heads;
+  ScanParts p;
+  p.q = 0;                                                 // [4][NT][64][4]
+  p.k = p.q + shared * kTok * padded_rows(N);              // [NT][4][64][4]
+  p.p = p.k + shared * kTok * padded_rows(N);              // (q . k) M vs: [10][64][4]
+  p.d0 = p.p + units * kTiles * 256;                       // D(t), [64]
+  p.scale = p.d0 + units * kTok;                           // M(last, s) vs, [64]
+  p.end = p.scale + units * kTok;
   return p;
 }
 
@@ -243,6 +262,31 @@ __device__ __forceinline__ f32x4 tile_decays(HeadDecays d, int i, int j, int l, 
   return m;
 }
 
+// The same for row t = l and columns s = 4 g + r: a lane's part of the tile as a left operand.
+__device__ __forceinline__ f32x4 tile_decays_left(HeadDecays d, int i, int j, int l, int g) {
+  f32x4 m;
+  const f32x4 vs = read4(d.vs() + 16 * j + 4 * g);
+  if (i == j) {
+    const float* gb = d.g() + 16 * i;
+    double run = 1.;                       // from 4 g + 4 through t, then one more at a time
+#pragma unroll
+    for (int u = 4; u < 16; ++u) run = u > 4 * g + 3 && u <= l ? run * gb[u] : run;
+    const f32x4 own = read4(gb + 4 * g);
+#pragma unroll
+    for (int r = 3; r >= 0; --r) {
+      m[r] = l >= 4 * g + r ? (float)(run * vs[r]) : 0.f;
+      run = l >= 4 * g + r ? run * own[r] : run;
+    }
+    return m;
+  }
+  double row = d.pre()[16 * i + l];
+  for (int b = j + 1; b < i; ++b) row *= d.total()[b];
+  const f32x4 suf = read4(d.suf() + 16 * j + 4 * g);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) m[r] = (float)(row * ((double)suf[r] * vs[r]));
+  return m;
+}
+
 // One 16 x 16 tile of rows a . rows b over NP columns, both in LDS.
 template <int NT>
 __device__ __forceinline__ f32x4 gram_tile(const float* a, const float* b, int l, int g) {
@@ -285,11 +329,10 @@ __device__ __forceinline__ void read_run(const float* p, float (&v)[PER]) {
   }
 }
 
-// T u for a diagonal tile T in LDS, zero above its diagonal: row t takes u of its own and of
+// T u for a diagonal tile T (its left operand), zero above its diagonal: row t takes u of its own and of
 // earlier tokens.  Zero times what is not finite is not zero, so where such u are among the
 // sixteen a row at a time is made, with the later ones left out, and taken.
-__device__ __forceinline__ f32x4 causal_product(const float* tile, f32x4 u, int l, int g) {
-  const f32x4 a = read4(tile + l * kTileLd + 4 * g);
+__device__ __forceinline__ f32x4 causal_product(f32x4 a, f32x4 u, int g) {
   if (__builtin_amdgcn_ballot_w64(!(fabsf(u[0]) + fabsf(u[1]) + fabsf(u[2]) + fabsf(u[3]) < INFINITY)) == 0)
     return product4(a, u);
   f32x4 out;
@@ -531,6 +574,301 @@ __global__ __launch_bounds__(kThreads) void chunk_carry_kernel(ChunkedArgs a) {
     if (n0 + r < a.N && p < a.P) st[(int64_t)(n0 + r) * a.P + p] = S[r];
 }
 
+// ---------------------------------------------------------------- linear forms in two launches
+// Three launches write the state in front of every chunk, add them up and read them again (at 64 heads
+// of 128 x 64 and 2,048 tokens 270 MB of their 123 us).  Here one makes what does not hang on the
+// state, in the order in which the matrix cores take it: q, k, and (q . k) times the decays; the other
+// walks, with the state in registers, and nothing of it is written but the last.
+// A workgroup of the first takes one chunk and `heads_each` (up to 8) heads that read the same q and k.
+template <int NT, int FORM, int RT>
+__device__ __forceinline__ void prepare_chunk(const ChunkedArgs& a, const ChunkRange& c, int heads_each,
+                                              int wide) {
+  constexpr int NP = 16 * NT, LD = NP + 4;
+  extern __shared__ __align__(16) float lds[];
+  float* Qs = lds;
+  float* Ks = Qs + kTok * LD;
+  float* decays = Ks + kTok * LD;         // [heads_each] of HeadDecays
+  const int chunk = blockIdx.y, h0 = blockIdx.x * heads_each;
+  const int group = a.heads / a.kv_heads, hk = h0 / group;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64, l = lane % 16, g = lane / 16;
+  const ScanParts parts = scan_parts_of(a.num_chunks, a.heads, a.kv_heads, a.N);
+  float dec[2] = {1.f, 1.f}, vs[2] = {0.f, 0.f};          // of heads w and w + 4, a token a lane
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+    if (w + 4 * u < heads_each && lane < c.nt)
+      token_scalars(a, c.first + lane, h0 + w + 4 * u, dec[u], vs[u]);
+  stage_rows<NP, FORM>(a, Qs, a.q_col + hk * a.N, c.first, c.nt, c.pos0, false, wide);
+  stage_rows<NP, FORM>(a, Ks, a.k_col + hk * a.N, c.first, c.nt, c.pos0, true, wide);
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    if (w + 4 * u < heads_each) {
+      const HeadDecays d{decays + (w + 4 * u) * HeadDecays::kFloats};
+      spread_decays(d, dec[u], vs[u], lane);
+      const int64_t unit = (int64_t)chunk * a.heads + h0 + w + 4 * u;
+      a.scratch[parts.d0 + unit * kTok + lane] = d.d0()[lane];
+      a.scratch[parts.scale + unit * kTok + lane] = d.vs()[lane] * d.es()[lane];
+    }
+  }
+  __syncthreads();
+  f32x4 gram[3];
+#pragma unroll
+  for (int u = 0; u < 3; ++u) {
+    const int t = w + 4 * u, i = tri_row(t), j = t - tri(i, 0);
+    if (t < kTiles && i < RT) gram[u] = gram_tile<NT>(Ks + 16 * j * LD, Qs + 16 * i * LD, l, g);
+  }
+  if (h0 % group == 0) {                  // q and k themselves, by the first workgroup that reads them
+    const int64_t unit = (int64_t)chunk * a.kv_heads + hk;
+    if (w < RT) {
+      float* to = a.scratch + parts.q + (unit * 4 + w) * NT * 256 + lane * 4;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) write4(to + j * 256, read4(Qs + (16 * w + l) * LD + 16 * j + 4 * g));
+    }
+    for (int n = w; n < NT; n += 4) {
+      float* to = a.scratch + parts.k + (unit * NT + n) * 4 * 256 + lane * 4;
+#pragma unroll
+      for (int j = 0; j < RT; ++j) {
+        f32x4 v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = Ks[(16 * j + 4 * g + r) * LD + 16 * n + l];
+        write4(to + j * 256, v);
+      }
+    }
+  }
+  for (int h = 0; h < heads_each; ++h) {
+    const HeadDecays d{decays + h * HeadDecays::kFloats};
+    float* to = a.scratch + parts.p + ((int64_t)chunk * a.heads + h0 + h) * kTiles * 256 + lane * 4;
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+      const int t = w + 4 * u, i = tri_row(t), j = t - tri(i, 0);
+      if (t < kTiles && i < RT) {
+        const f32x4 m = tile_decays_left(d, i, j, l, g);
+        f32x4 p;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) p[r] = i > j || l >= 4 * g + r ? gram[u][r] * m[r] : 0.f;
+        write4(to + t * 256, p);
+      }
+    }
+  }
+}
+
+template <int NT, int FORM>
+__global__ __launch_bounds__(kThreads) void chunk_prepare_kernel(ChunkedArgs a, int heads_each, int wide) {
+  const ChunkRange c = chunk_range(a, blockIdx.y);
+  if (c.tiles == 1) prepare_chunk<NT, FORM, 1>(a, c, heads_each, wide);
+  else prepare_chunk<NT, FORM, 4>(a, c, heads_each, wide);
+}
+
+// The chunks of an entry in order, sixteen columns of S a workgroup, with their outputs.  Of eight
+// wavefronts, two to a SIMD, w = 0 to 3 keep the rows of tiles w, w + 4, ... of S and make their new
+// values; a chunk's own share of S does not hang on S, so they meet the others, which make the outputs
+// of 16 tokens each, once a chunk, when the state in front of it and v lie in LDS (in one of two
+// buffers: whoever still reads the other is in the chunk before).  An operand of a chunk some turns
+// ahead is asked for as soon as its registers have been read; nothing in the loops that touches memory
+// hangs on a condition, so that a wait is for the operands it is for.
+// A chunk of 128 x 16 of S takes 2.3 us: 1.2 are a SIMD's products, 1.4 the 108 loads that a unit takes
+// in 28 cycles each, and neither hides the other whole (without loads 1.8, without the meetings 1.9; as
+// four wavefronts that do both parts 2.6).
+constexpr int kScanThreads = 512;
+
+// Four bytes a lane, at `offset` from a base that the lanes share; offsets from `bytes` on go nowhere.
+__device__ __forceinline__ void store_inside(float* base, int bytes, int offset, float v) {
+  const auto to = __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000);
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), to, offset, 0, 0);
+}
+
+template <int NT>
+struct StateOperands {
+  static constexpr int OWN = (NT + 3) / 4;
+  f32x4 k[OWN][4], v, scale;
+  float total;
+};
+
+template <int NT>
+struct OutputOperands {
+  f32x4 q[NT], p[4], d0;
+};
+
+// turn(i, c) for c = 0 to count - 1, i = c % RING known to the compiler.
+template <int RING, typename F>
+__device__ __forceinline__ void in_turns(int count, F turn) {
+  int c = 0;
+  for (; c + RING <= count; c += RING) {
+#pragma unroll
+    for (int i = 0; i < RING; ++i) turn(i, c + i);
+  }
+#pragma unroll
+  for (int i = 0; i < RING - 1; ++i)
+    if (c + i < count) turn(i, c + i);
+}
+
+template <int NT, int FORM>
+__global__ __launch_bounds__(kScanThreads, 1) void chunk_scan_kernel(ChunkedArgs a) {
+  constexpr int OWN = (NT + 3) / 4;
+  __shared__ __align__(16) float s_lds[2][NT][256];
+  __shared__ __align__(16) float v_lds[2][2][4][256];     // scaled, and as it stands
+  // (heads that read the same q and k on one XCD: they lie next to each other, workgroups do not)
+  const int h = a.heads % 8 == 0 ? (int)(blockIdx.x % 8) * (a.heads / 8) + (int)blockIdx.x / 8 : (int)blockIdx.x;
+  const int e = blockIdx.z, ct = blockIdx.y, hk = h / (a.heads / a.kv_heads);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), w = wave % 4;
+  const int lane = threadIdx.x % 64, l = lane % 16, g = lane / 16;
+  const int p = 16 * ct + l, first_row = 16 * w + 4 * g;
+  const ScanParts parts = scan_parts_of(a.num_chunks, a.heads, a.kv_heads, a.N);
+  const int q0 = a.b.q_start[e], tokens = a.b.q_start[e + 1] - q0;
+  const int begin = a.entry_chunks[e], count = a.entry_chunks[e + 1] - begin;
+  if (count < 1) return;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  const float* v_col = a.x + a.v_col + h * a.P + min(p, a.P - 1);
+  auto unit_of = [&](int c) { return (int64_t)(begin + min(c, count - 1)) * a.heads + h; };
+  auto shared_of = [&](int c) { return (int64_t)(begin + min(c, count - 1)) * a.kv_heads + hk; };
+
+  if (wave < 4) {
+    float* st = a.state + ((int64_t)a.b.slot_ids[e] * a.heads + h) * a.N * a.P;
+    const bool fresh = a.b.positions[q0] == 0;
+    f32x4 S[OWN];
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) {
+      S[o] = zero;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int n = 16 * (w + 4 * o) + 4 * g + r;
+        if (!fresh && n < a.N && p < a.P) S[o][r] = st[(int64_t)n * a.P + p];
+      }
+    }
+    // only the last chunk may be short; of one of a single tile nothing else was left
+    const int one_tile = tokens - (count - 1) * kTok <= 16 ? count - 1 : count;
+    const bool owns_last = NT % 4 == 0 || w + 4 * (OWN - 1) < NT;
+    auto fetch_v = [&](StateOperands<NT>& f, int c) {
+      const int64_t unit = unit_of(c);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) f.v[r] = v_col[(int64_t)(q0 + min(c * kTok + first_row + r, tokens - 1)) * a.ld];
+      f.scale = read4(a.scratch + parts.scale + unit * kTok + first_row);
+      f.total = a.scratch[parts.d0 + unit * kTok + kTok - 1];
+    };
+    auto fetch_k = [&](StateOperands<NT>& f, int c, int o) {
+      const float* at = a.scratch + parts.k + shared_of(c) * NT * 1024 + min(w + 4 * o, NT - 1) * 1024;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) f.k[o][j] = read4(at + j * 256 + lane * 4);
+    };
+    auto walk = [&](auto size) {
+      constexpr bool MORE = decltype(size)::value > 0;
+      constexpr int RING = MORE ? decltype(size)::value : 1;
+      StateOperands<NT> ring[RING];
+#pragma unroll
+      for (int i = 0; i < RING; ++i) {
+        fetch_v(ring[i], i);
+#pragma unroll
+        for (int o = 0; o < OWN; ++o) fetch_k(ring[i], i, o);
+      }
+      in_turns<RING>(count, [&](int i, int c) {
+        StateOperands<NT>& f = ring[i];
+        float (&v_buf)[2][4][256] = v_lds[c & 1];
+        f32x4 mine, scaled;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          mine[r] = c * kTok + first_row + r < tokens ? (FORM == kSilu ? silu(f.v[r]) : f.v[r]) : 0.f;
+          scaled[r] = mine[r] * f.scale[r];
+        }
+        const float total = f.total;
+        write4(&v_buf[0][w][lane * 4], scaled);
+        write4(&v_buf[1][w][lane * 4], mine);
+#pragma unroll
+        for (int o = 0; o < OWN; ++o)
+          if (o < OWN - 1 || owns_last) write4(&s_lds[c & 1][w + 4 * o][lane * 4], S[o]);
+        __syncthreads();
+        f32x4 v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = read4(&v_buf[0][j][lane * 4]);
+        if (MORE) fetch_v(f, c + RING);
+        if (c == one_tile) {
+#pragma unroll
+          for (int o = 0; o < OWN; ++o)
+#pragma unroll
+            for (int j = 1; j < 4; ++j) f.k[o][j] = zero;
+        }
+#pragma unroll
+        for (int o = 0; o < OWN; ++o) {
+          const f32x4 early = product2(f.k[o][0], v[0]) + product2(f.k[o][1], v[1]);
+          const f32x4 share = early + (product2(f.k[o][2], v[2]) + product2(f.k[o][3], v[3]));
+#pragma unroll
+          for (int r = 0; r < 4; ++r) S[o][r] = fmaf(total, S[o][r], share[r]);
+        }
+        if (MORE) {
+#pragma unroll
+          for (int o = 0; o < OWN; ++o) fetch_k(f, c + RING, o);
+        }
+      });
+    };
+    if (count == 1) walk(std::integral_constant<int, 0>{});
+    else walk(std::integral_constant<int, 3>{});
+#pragma unroll
+    for (int o = 0; o < OWN; ++o)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int n = 16 * (w + 4 * o) + 4 * g + r;
+        if (n < a.N && p < a.P) st[(int64_t)n * a.P + p] = S[o][r];
+      }
+    return;
+  }
+
+  const float skip = a.d_skip ? a.d_skip[h] : 0.f;
+  const int out_ld = a.heads * a.P, out_at = p < a.P ? (first_row * out_ld + h * a.P + p) * 4 : -16 * out_ld;
+  const float* q_at = a.scratch + parts.q + w * NT * 256 + lane * 4;
+  const float* p_at = a.scratch + parts.p + tri(w, 0) * 256 + lane * 4;
+  auto fetch_q = [&](OutputOperands<NT>& f, const float* at, int j) { f.q[j] = read4(at + j * 256); };
+  auto fetch_p = [&](OutputOperands<NT>& f, int c) {      // (the last: the diagonal's)
+    const float* at = p_at + unit_of(c) * kTiles * 256;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) f.p[j] = read4(at + (j < 3 ? min(j, w) : w) * 256);
+    f.d0 = read4(a.scratch + parts.d0 + unit_of(c) * kTok + first_row);
+  };
+  auto walk = [&](auto size) {
+    constexpr bool MORE = decltype(size)::value > 0;
+    constexpr int RING = MORE ? decltype(size)::value : 1;
+    OutputOperands<NT> ring[RING];
+#pragma unroll
+    for (int i = 0; i < RING; ++i) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j) fetch_q(ring[i], q_at + shared_of(i) * 4 * NT * 256, j);
+      fetch_p(ring[i], i);
+    }
+    in_turns<RING>(count, [&](int i, int c) {
+      OutputOperands<NT>& f = ring[i];
+      const float* later = q_at + shared_of(c + RING) * 4 * NT * 256;
+      __syncthreads();
+      f32x4 s[NT], v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = read4(&v_lds[c & 1][1][j < 3 ? j : w][lane * 4]);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) s[j] = read4(&s_lds[c & 1][j][lane * 4]);
+      // (products of earlier tokens with tiles that are not there count nothing, whatever v is)
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[j][r] = j < w ? v[j][r] : 0.f;
+      const f32x4 x0 = product2(f.p[0], v[0]), x1 = product2(f.p[1], v[1]), x2 = product2(f.p[2], v[2]);
+      const f32x4 own = causal_product(f.p[3], v[3], g);
+      f32x4 acc = zero;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        acc += product2(f.q[j], s[j]);
+        asm volatile("" : "+v"(acc));        // (left alone, every sum is put off to the end)
+        if (MORE) fetch_q(f, later, j);
+      }
+      acc *= f.d0;
+      acc += w == 1 ? x0 + own : w == 0 ? own : x0 + x1;
+      if (w > 1) acc += w == 2 ? own : x2 + own;
+      if (MORE) fetch_p(f, c + RING);
+      const int nt = min(tokens - c * kTok, kTok);
+      float* out = a.out + (int64_t)(q0 + c * kTok) * out_ld;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        store_inside(out, nt * out_ld * 4, out_at + r * out_ld * 4, fmaf(skip, v[3][r], acc[r]));
+    });
+  };
+  if (count == 1) walk(std::integral_constant<int, 0>{});
+  else walk(std::integral_constant<int, NT <= 4 ? 3 : 2>{});
+}
+
 // ---------------------------------------------------------------- delta rule: Y, W, decayed keys
 // A workgroup takes one chunk of one head: the 64 x 64 triangular matrix in LDS, its diagonal
 // blocks inverted (a wavefront each, a column a lane), then block by block the solution for the
@@ -632,7 +970,7 @@ __device__ __forceinline__ void solve_chunk(const ChunkedArgs& a, const ChunkRan
 #pragma unroll
       for (int m = 0; m < i; ++m)
         acc += product4(read4(tiles + tri(i, m) * kTile + l * kTileLd + 4 * g), X[m]);
-      X[i] = causal_product(tiles + tri(i, i) * kTile, acc, l, g);
+      X[i] = causal_product(read4(tiles + tri(i, i) * kTile + l * kTileLd + 4 * g), acc, g);
       if (ct < NT) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
@@ -962,8 +1300,8 @@ __device__ __forceinline__ void output_chunk(const ChunkedArgs& a, const ChunkRa
         f32x4 pair = zero;
 #pragma unroll
         for (int j = 0; j <= i; ++j) {
-          const f32x4 p = i == j ? causal_product(tiles + tri(i, i) * kTile, v[j], l, g)
-                                 : product2(read4(tiles + tri(i, j) * kTile + l * kTileLd + 4 * g), v[j]);
+          const f32x4 t = read4(tiles + tri(i, j) * kTile + l * kTileLd + 4 * g);
+          const f32x4 p = i == j ? causal_product(t, v[j], g) : product2(t, v[j]);
           pair = j & 1 ? pair + p : p;
           if (j & 1 || j == i) acc[i] += pair;
         }
@@ -1005,6 +1343,30 @@ int launch_output(const ChunkedArgs& a, int heads_each, int wide, hipStream_t st
   return 0;
 }
 
+// Whether linear forms go in two launches, which walk 64 tokens in 2.3 us (up to 64 rows of S: 1.4)
+// whatever else the chip does, or in three, whose work is spread over it: us in two and three launches,
+// 256 workgroups in the walk (64 heads of 128 x 64) 170 tokens 26 / 35, 1,000 63 / 80, 2,048 98 / 123,
+// 8,192 360 / 464; 128 (16 heads of 128 x 128) 300 tokens 30 / 44, 1,000 55 / 55, 2,048 93 / 84;
+// 64 (16 heads of 64 x 64) 300 tokens 20 / 26, 1,000 39 / 29.  (More rows than 128 do not fit the walk's
+// registers; an output's place in a chunk is counted in 32 bits.)
+bool in_two_launches(const ChunkedArgs& a) {
+  const int64_t chunks = (a.max_len + kTok - 1) / kTok;
+  return a.N <= 128 && (int64_t)a.heads * a.P <= 1 << 22 &&
+         (int64_t)a.heads * ((a.P + 15) / 16) >= 8 * std::min<int64_t>(chunks, 32);
+}
+
+template <int NT, int FORM>
+int launch_scan(const ChunkedArgs& a, int each, int wide, hipStream_t stream) {
+  constexpr int NP = 16 * NT, LD = NP + 4;
+  const size_t lds = sizeof(float) * (2 * kTok * LD + each * HeadDecays::kFloats);
+  auto* prepare = chunk_prepare_kernel<NT, FORM>;
+  if (!raise_lds(prepare, lds)) return -1;
+  hipLaunchKernelGGL(prepare, dim3(a.heads / each, a.num_chunks), dim3(kThreads), lds, stream, a, each, wide);
+  hipLaunchKernelGGL((chunk_scan_kernel<NT, FORM>), dim3(a.heads, (a.P + 15) / 16, a.num_entries),
+                     dim3(kScanThreads), 0, stream, a);
+  return 0;
+}
+
 template <int NT, int FORM>
 int launch_linear(const ChunkedArgs& a, int wide, hipStream_t stream) {
   constexpr int NP = 16 * NT, LD = NP + 4;
@@ -1012,6 +1374,8 @@ int launch_linear(const ChunkedArgs& a, int wide, hipStream_t stream) {
   int each = a.heads / a.kv_heads;
   while (each % 2 == 0 && (each > 8 || (int64_t)(a.heads / each) * a.num_chunks < 512)) each /= 2;
   if (each > 8) each = 1;
+  if constexpr (NT <= 8)
+    if (in_two_launches(a)) return launch_scan<NT, FORM>(a, each, wide, stream);
   const size_t lds = sizeof(float) * (kTok * LD + kTok * 68 + each * kTok);
   auto* local = chunk_local_kernel<NT, FORM>;
   if (!raise_lds(local, lds)) return -1;
@@ -1043,19 +1407,20 @@ int launch_delta(const ChunkedArgs& a, int wide, hipStream_t stream) {
 
 }  // namespace
 
-int64_t chunked_scratch_floats(int num_chunks, int heads, int N, int P, int delta) {
+int64_t chunked_scratch_floats(int num_chunks, int heads, int kv_heads, int N, int P, int delta) {
   if (N < 1 || P < 1 || N > (delta ? 128 : 256)) return -1;
-  return parts_of(num_chunks, heads, N, P, delta).end;
+  const int64_t end = parts_of(num_chunks, heads, N, P, delta).end;
+  return delta ? end : std::max(end, scan_parts_of(num_chunks, heads, kv_heads, N).end);
 }
 
-extern "C" int64_t ts_chunked_scratch(int num_chunks, int heads, int N, int P, int delta) {
-  return chunked_scratch_floats(num_chunks, heads, N, P, delta);
+extern "C" int64_t ts_chunked_scratch(int num_chunks, int heads, int kv_heads, int N, int P, int delta) {
+  return chunked_scratch_floats(num_chunks, heads, kv_heads, N, P, delta);
 }
 
 extern "C" int ts_chunk_tokens() { return kChunkTokens; }
 
 int launch_chunked(ChunkedArgs a, hipStream_t stream) {
-  if (chunked_scratch_floats(a.num_chunks, a.heads, a.N, a.P, a.delta) < 0)
+  if (chunked_scratch_floats(a.num_chunks, a.heads, a.kv_heads, a.N, a.P, a.delta) < 0)
     TS_FAIL("chunked recurrence: %d rows of S are not built", a.N);
   if (a.num_chunks > 65535 || a.num_entries > 65535 || a.P > 1 << 19)
     TS_FAIL("chunked recurrence: %d chunks, %d entries, %d columns", a.num_chunks, a.num_entries, a.P);

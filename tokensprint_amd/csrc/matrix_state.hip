@@ -351,7 +351,7 @@ extern "C" int ts_linear_recurrence(const float* x, int ld, int q_col, int k_col
     c.decay = decay, c.gates = gates, c.ldg = ldg, c.delta = delta, c.per_row = per_row;
     c.turn = a.turn, c.turn_dims = turn_dims, c.k_scale = k_scale;
     c.chunks = chunks, c.entry_chunks = entry_chunks;
-    c.num_chunks = num_chunks, c.num_entries = num_entries, c.scratch = scratch;
+    c.num_chunks = num_chunks, c.num_entries = num_entries, c.max_len = max_q_len, c.scratch = scratch;
     return launch_chunked(c, stream);
   }
   if (max_q_len == 1 && num_tokens == num_entries) {       // a token an entry

@@ -454,7 +454,7 @@ extern "C" int ts_ssm_scan(const float* xbc, const float* proj, int ld, int dt_c
     c.heads = heads, c.kv_heads = groups, c.N = N, c.P = P;
     c.dt = proj + dt_col, c.ldg = ld, c.dt_bias = dt_bias, c.a_log = a_log, c.d_skip = d_skip;
     c.k_scale = 1.f, c.chunks = chunks, c.entry_chunks = entry_chunks;
-    c.num_chunks = num_chunks, c.num_entries = num_entries, c.scratch = scratch;
+    c.num_chunks = num_chunks, c.num_entries = num_entries, c.max_len = max_q_len, c.scratch = scratch;
     return launch_chunked(c, stream);
   }
   const ScanStepArgs one{xbc, proj + dt_col, dt_bias, a_log, d_skip, state, y, positions, slot_ids,

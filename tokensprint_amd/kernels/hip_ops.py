@@ -1421,18 +1421,18 @@ class HipOps:
         # the step's: every recurrent layer of the model uses the same)
         chunks, entry_chunks, num_chunks = self._scan_chunks(
             batch, self.dispatch.state_space_whole_tokens)
-        scratch = self._chunk_scratch(num_chunks, heads, N, vdim)
+        scratch = self._chunk_scratch(num_chunks, heads, groups, N, vdim)
         self._call(self.lib.ts_ssm_scan, _ptr(xbc), _ptr(proj), proj.shape[1], dt_col,
                    _ptr(dt_bias), _ptr(a_log), _ptr(d_skip), _ptr(state), _ptr(y), pos, eot, qs,
                    slots, T, batch.num_entries, int(batch.max_q_len), heads, vdim, N, groups,
                    _ptr(chunks), _ptr(entry_chunks), num_chunks, _ptr(scratch), self._stream())
         return y
 
-    def _chunk_scratch(self, num_chunks, heads, rows, cols, delta=False):
+    def _chunk_scratch(self, num_chunks, heads, kv_heads, rows, cols, delta=False):
         """What the kernels of a recurrence in chunks hand each other; None without chunks."""
         if not num_chunks:
             return None
-        count = self.lib.ts_chunked_scratch(num_chunks, heads, rows, cols, int(delta))
+        count = self.lib.ts_chunked_scratch(num_chunks, heads, kv_heads, rows, cols, int(delta))
         if count < 0:
             raise KernelError(f"recurrence in chunks: {rows} x {cols} states are not built")
         return torch.empty(count, dtype=torch.float32, device=self.device)
@@ -1565,7 +1565,7 @@ class HipOps:
         if dim <= (128 if delta else 256) and not walk and not (delta and silu_inputs):
             whole = self.dispatch.scan_whole_tokens + delta * self.dispatch.delta_whole_more
             chunks, entry_chunks, num_chunks = self._scan_chunks(batch, whole)
-        scratch = self._chunk_scratch(num_chunks, heads, dim, vdim, delta)
+        scratch = self._chunk_scratch(num_chunks, heads, kv_heads, dim, vdim, delta)
         self._call(self.lib.ts_linear_recurrence, _ptr(x), ld, int(q_col), int(k_col), int(v_col),
                    _ptr(decay), _ptr(gates), ldg, _ptr(state), _ptr(out), pos, eot, qs, slots, T,
                    batch.num_entries, int(batch.max_q_len), heads, kv_heads, dim, vdim,
