@@ -31,13 +31,16 @@
 // (`sumsq_out` [N / 32, M]; a slice is added up in the same order whatever the tile).
 // SCALED (the product behind that norm): A is such prepared rows, and the epilogue
 // multiplies row m by rsqrt(sum of its slices / K + eps), which a workgroup works out for
-// its BM rows before it sends for its first operands.
+// its BM rows before it sends for its first operands.  HEADS is SCALED for a q/k/v projection with
+// heads of as many elements as a tile has columns: the tile, rounded, passes LDS and leaves as
+// qk_prepare.hip would have left it (normed and turned queries, keys and values in their pages).
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
 
 #include "gemm_common.h"
+#include "qk_prepare.h"
 
 namespace {
 
@@ -61,7 +64,12 @@ struct TiledArgs {
   float limit;          // PAIR: gated_unit's limit (0: silu, below: gelu)
 };
 
-constexpr int kPlain = 0, kScaled = 1, kTail = 2;
+// HEADS: `qkv`, `paged`, `store_kv` and `row_extra` of the preparation's arguments are not looked at.
+struct TiledHeadsArgs : TiledArgs {
+  QkPrepareArgs heads;
+};
+
+constexpr int kPlain = 0, kScaled = 1, kTail = 2, kHeads = 3;
 constexpr int kSliceColumns = 32;   // columns per slice of a row's sum of squares (TAIL)
 
 // One 16-byte piece per lane from global memory (uniform base + per-lane byte offset)
@@ -79,8 +87,127 @@ __device__ __forceinline__ void wait_loads() {
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
 }
 
+// Rows of a tile's bfloat16 results in LDS, on their way out (HEADS): 16 bytes further from one another
+// than they are long.
+constexpr int kHeadRow = 128 + 8;
+
+// HEADS: what becomes of one head of BM tokens from row m0 on.  `put` writes the tile into LDS, where
+// sixteen lanes take a row, eight elements each, as qk_prepare.hip's do (the same sums in the same
+// order), the tables' rows and pages asked for before the tile is there.  The preparation kernel read
+// and wrote what the product had just written (50 MB and 9 us a layer of 2,048 rows of 4,096 columns);
+// this is 3.8 us at the product's end, of shuffles, LDS and the tables' trip.  Values go into their pages
+// sixteen tokens at a time: where these fill a run of sixteen places (a prompt's mostly do), 16 bytes a
+// lane, eight tokens of one element, else an element at a time.
+template <int BM, int THREADS, typename PUT>
+__device__ __forceinline__ void heads_out(const TiledHeadsArgs& g, int head, int m0, const int* row_pos,
+                                          const int* row_entry, bf16_t* rows, PUT put) {
+  constexpr int HD = 128, L = HD / 8, AT_ONCE = THREADS / L, TURNS = BM / AT_ONCE, AHEAD = 4;
+  static_assert(BM % AT_ONCE == 0 && TURNS % AHEAD == 0, "whole turns");
+  const QkPrepareArgs& a = g.heads;
+  const int sub = threadIdx.x % L, row0 = threadIdx.x / L;
+  auto page_of = [&](int row) {
+    return a.table[(int64_t)row_entry[row] * a.table_width + row_pos[row] / a.page_size];
+  };
+  if (head >= a.nq + a.nkv) {
+    const int kvh = head - a.nq - a.nkv;
+    __syncthreads();                                // the slabs have been read
+    put(rows);
+    __syncthreads();
+    // 256 threads take sixteen tokens, sixteen lanes of them eight elements of each
+    constexpr int TILES = THREADS / 256;            // of sixteen tokens at a time
+    const int part = threadIdx.x / 16 % 16, lane = threadIdx.x % 16;
+    for (int t0 = threadIdx.x / 256 * 16; t0 < BM; t0 += TILES * 16) {
+      if (m0 + t0 >= g.M) break;
+      const int row = t0 + lane, page = page_of(row), pos = row_pos[row];
+      const int first = __shfl(pos, 0, 16), first_page = __shfl(page, 0, 16);
+      const bool in_run = m0 + row < g.M && pos == first + lane && page == first_page &&
+                          first % 16 == 0 && a.page_size % 16 == 0;
+      const unsigned long long runs = __builtin_amdgcn_ballot_w64(in_run);
+      bf16_t* pages = (bf16_t*)a.v_dst;
+      if (runs == ~0ull) {
+        if (first_page < 0) continue;
+        bf16_t* dst = pages + ((int64_t)first_page * a.nkv + kvh) * a.page_size * HD + first % a.page_size;
+        const int d = part * 8 + lane / 2, half = lane % 2 * 8;
+        bf16x8 v;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = rows[(t0 + half + j) * kHeadRow + d];
+        *(bf16x8*)(dst + (int64_t)d * a.page_size + half) = v;
+      } else if (m0 + row < g.M && page >= 0) {
+        bf16_t* dst = pages + ((int64_t)page * a.nkv + kvh) * a.page_size * HD + pos % a.page_size;
+        const bf16x8 v = *(const bf16x8*)(rows + row * kHeadRow + part * 8);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) dst[(int64_t)(part * 8 + j) * a.page_size] = v[j];
+      }
+    }
+    return;
+  }
+  const bool key = head >= a.nq;
+  const float* w = key ? a.k_weight : a.q_weight;
+  const bool first = sub < L / 2;
+  float own_w[8], other_w[8];
+  if (w) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) own_w[j] = w[sub * 8 + j], other_w[j] = w[(sub ^ (L / 2)) * 8 + j];
+  }
+  f32x4 cs[AHEAD][4];
+  int page[AHEAD];
+  auto fetch = [&](int u, int turn) {
+    const int row = row0 + turn * AT_ONCE;
+    if (a.cos) {
+      const int64_t at = (int64_t)row_pos[row] * (HD / 2) + sub % (L / 2) * 8;
+      cs[u][0] = *(const f32x4*)(a.cos + at);
+      cs[u][1] = *(const f32x4*)(a.cos + at + 4);
+      cs[u][2] = *(const f32x4*)(a.sin + at);
+      cs[u][3] = *(const f32x4*)(a.sin + at + 4);
+    }
+    page[u] = key ? page_of(row) : 0;
+  };
+#pragma unroll
+  for (int u = 0; u < AHEAD; ++u) fetch(u, u);
+  __syncthreads();                                  // the slabs have been read
+  put(rows);
+  __syncthreads();
+  for (int turn0 = 0; turn0 < TURNS; turn0 += AHEAD) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const int row = row0 + (turn0 + u) * AT_ONCE;
+      const bf16x8 x = *(const bf16x8*)(rows + row * kHeadRow + sub * 8);
+      const bf16x8 y = *(const bf16x8*)(rows + row * kHeadRow + (sub ^ (L / 2)) * 8);
+      float v[8], other[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = (float)x[j], other[j] = (float)y[j];
+      if (w) {
+        const float rstd = head_rstd(v, L, HD, a.eps);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] *= rstd * own_w[j], other[j] *= rstd * other_w[j];
+      }
+      bf16x8 o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        o[j] = (bf16_t)(a.cos ? head_turned(v[j], other[j], cs[u][j / 4][j % 4], cs[u][2 + j / 4][j % 4], first)
+                              : v[j]);
+      const int m = m0 + row;
+      if (m < g.M) {
+        if (!key) {
+          *(bf16x8*)((bf16_t*)a.q_out + ((int64_t)m * a.nq + head) * HD + sub * 8) = o;
+        } else if (page[u] >= 0) {
+          *(bf16x8*)((bf16_t*)a.k_dst + (((int64_t)page[u] * a.nkv + head - a.nq) * a.page_size +
+                                         row_pos[row] % a.page_size) * HD + sub * 8) = o;
+        }
+      }
+      if (turn0 + AHEAD < TURNS) fetch(u, turn0 + AHEAD + u);
+    }
+  }
+}
+
+template <int FORM>
+using TiledArgsOf = std::conditional_t<FORM == kHeads, TiledHeadsArgs, TiledArgs>;
+
 template <int BM, int BN, int GM, int GN, int STAGES, bool PAIR, typename TO, int FORM = kPlain>
-__global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgs g) {
+__global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgsOf<FORM> g) {
+  constexpr bool kRowScaled = FORM == kScaled || FORM == kHeads;
+  static_assert(FORM != kHeads || (BN == 128 && !PAIR && BM * kHeadRow * 2 <= STAGES * (BM + BN) * 128),
+                "a tile is one head of 128 elements, and has room in LDS");
   static_assert(!(FORM == kTail && PAIR), "the product that ends a sub-layer has one weight");
   constexpr int NW = GM * GN;                        // waves: GM along the rows, GN along the columns
   static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "whole load instructions per operand");
@@ -117,8 +244,10 @@ __global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgs g
   // those before them, which the first turn needs anyway.  A row's slices are asked for
   // 32 at a time and added in their order.
   float* row_scale = (float*)(tiled_lds + STAGES * ((BM + BN) * 128));
+  int* row_pos = (int*)(row_scale + BM);             // HEADS: position and entry of the tile's rows
+  int* row_entry = row_pos + BM;
   auto row_scales = [&]() {
-    if constexpr (FORM == kScaled) {
+    if constexpr (kRowScaled) {
       for (int row = threadIdx.x; row < BM; row += 64 * NW) {
         const int m = min(m0 + row, g.M - 1);
         float sq = 0.f;
@@ -131,6 +260,10 @@ __global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgs g
           for (int i = 0; i < 32; ++i) sq += p0 + i < g.parts ? part[i] : 0.f;
         }
         row_scale[row] = rsqrtf(sq / (float)g.K + g.eps);
+        if constexpr (FORM == kHeads) {
+          row_pos[row] = g.heads.positions[m];
+          row_entry[row] = g.heads.entry_of_token[m];
+        }
       }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
@@ -458,7 +591,7 @@ __global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgs g
   const float slope = clamped ? -1.702f * 1.44269504f
                               : (gelu ? -1.59576912160573f * 1.44269504f : -1.44269504f);
   const float cubic = gelu ? 0.044715f * slope : 0.f;
-  if constexpr (FORM == kScaled) {
+  if constexpr (kRowScaled) {
     // (the barriers of the K loop lie between the factors' writes and these reads)
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) {
@@ -468,6 +601,20 @@ __global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgs g
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[tn][tm][e] *= scale;
     }
+  }
+  if constexpr (FORM == kHeads) {
+    heads_out<BM, 64 * NW>(g, tile_n, m0, row_pos, row_entry, (bf16_t*)tiled_lds, [&](bf16_t* rows) {
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn) {
+          bf16x4_t v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = (bf16_t)acc[tn][tm][e];
+          *(bf16x4_t*)(rows + (wm * WM + tm * 16 + r) * kHeadRow + wn * WN + tn * 16 + gq * 4) = v;
+        }
+    });
+    return;
   }
 #pragma unroll
   for (int tm = 0; tm < TM; ++tm) {
@@ -506,9 +653,9 @@ __global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgs g
 }
 
 template <int BM, int BN, int GM, int GN, int STAGES, bool PAIR, typename TO, int FORM>
-int launch_tiled(TiledArgs g, hipStream_t stream) {
+int launch_tiled(TiledArgsOf<FORM> g, hipStream_t stream) {
   auto kernel = gemm_tiled_kernel<BM, BN, GM, GN, STAGES, PAIR, TO, FORM>;
-  constexpr int lds = STAGES * (BM + BN) * 128 + (FORM == kScaled ? BM * 4 : 0);
+  constexpr int lds = STAGES * (BM + BN) * 128 + (FORM == kScaled ? BM * 4 : FORM == kHeads ? BM * 12 : 0);
   static_assert(lds <= 160 * 1024, "LDS of a compute unit");
   static bool raised[64] = {};
   int device = 0;

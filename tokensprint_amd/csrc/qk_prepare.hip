@@ -1,27 +1,7 @@
 // What happens to q, k and v between their projection and attention: per-head RMSNorm
 // on q and k, rotate-half position rotation, and the write of k and v into cache pages.
 // One wavefront per (token, head); sums and the rotation in float32.
-#include "common.h"
-
-struct QkPrepareArgs {
-  const void* qkv;       // [T, (nq + 2*nkv) * hd + row_extra]
-  void* q_out;           // [T, nq, hd]
-  void* k_dst;           // pages [num_pages, nkv, P, hd], or flat [T, nkv, hd] if !paged
-  void* v_dst;           // pages [num_pages, nkv, hd, P] (transposed), or flat [T, nkv, hd]
-  const float* q_weight; // [hd] or null: no norm
-  const float* k_weight;
-  const float* cos;      // [max_pos, hd/2] or null: no rotation
-  const float* sin;
-  const int* positions;      // [T]
-  const int* entry_of_token; // [T]
-  const int* table;          // [B, table_width]
-  int table_width;
-  int num_tokens, nq, nkv, hd, page_size, max_pos;
-  int paged;             // 1: k_dst/v_dst are cache pages; 0: flat buffers
-  int store_kv;          // 0: q only
-  float eps;
-  int row_extra;         // further columns of a qkv row behind the heads (another product's)
-};
+#include "qk_prepare.h"
 
 template <typename T, typename TC>
 __global__ void qk_prepare_kernel(QkPrepareArgs a) {
@@ -104,29 +84,6 @@ __global__ void qk_prepare_kernel(QkPrepareArgs a) {
 // head, eight consecutive elements per lane in one 16-byte load, the rotation partner
 // (the element hd/2 further) fetched from the lane hd/16 further.  `with_v` = 0 leaves the
 // value heads to the workgroups that store them tile by tile (v_store_tile).
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_qk;
-typedef __attribute__((ext_vector_type(4))) float f32x4_qk;
-
-// Eight consecutive elements of a row as they are loaded, and as they are stored.
-template <typename T>
-struct Eight;
-template <>
-struct Eight<bf16_t> {
-  bf16x8_qk x;
-  __device__ __forceinline__ void load(const bf16_t* p) { x = *(const bf16x8_qk*)p; }
-  __device__ __forceinline__ void store(bf16_t* p) const { *(bf16x8_qk*)p = x; }
-  __device__ __forceinline__ float get(int j) const { return (float)x[j]; }
-  __device__ __forceinline__ void set(int j, float v) { x[j] = (bf16_t)v; }
-};
-template <>
-struct Eight<float> {
-  f32x4_qk lo, hi;
-  __device__ __forceinline__ void load(const float* p) { lo = *(const f32x4_qk*)p; hi = *(const f32x4_qk*)(p + 4); }
-  __device__ __forceinline__ void store(float* p) const { *(f32x4_qk*)p = lo; *(f32x4_qk*)(p + 4) = hi; }
-  __device__ __forceinline__ float get(int j) const { return j < 4 ? lo[j] : hi[j - 4]; }
-  __device__ __forceinline__ void set(int j, float v) { if (j < 4) lo[j] = v; else hi[j - 4] = v; }
-};
-
 // Values of many tokens into their pages (of the rows' own type).  A page holds values
 // transposed, [head element][position], so a token's head vector lands an element at a
 // time, hd rows apart: here 16 lanes take 16 consecutive tokens for the same 8 head
@@ -225,11 +182,7 @@ __global__ __launch_bounds__(256) void qk_prepare_vec_kernel(QkPrepareArgs a, in
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = p.x.get(j);
     if (p.norm) {
-      float ss = 0.f;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) ss += v[j] * v[j];
-      for (int o = 1; o < L; o <<= 1) ss += __shfl_xor(ss, o, kWave);
-      const float rstd = rsqrtf(ss / (float)hd + a.eps);
+      const float rstd = head_rstd(v, L, hd, a.eps);
 #pragma unroll
       for (int j = 0; j < 4; ++j) { v[j] *= rstd * p.w0[j]; v[4 + j] *= rstd * p.w1[j]; }
     }
@@ -239,8 +192,7 @@ __global__ __launch_bounds__(256) void qk_prepare_vec_kernel(QkPrepareArgs a, in
       for (int j = 0; j < 8; ++j) {
         const float other = __shfl_xor(v[j], L / 2, kWave);
         const float c = j < 4 ? p.c0[j] : p.c1[j - 4], sn = j < 4 ? p.s0[j] : p.s1[j - 4];
-        // first half: re*c - im*s with im = other; second half: im*c + re*s with re = other
-        v[j] = first ? v[j] * c - other * sn : v[j] * c + other * sn;
+        v[j] = head_turned(v[j], other, c, sn, first);
       }
     }
     if (!p.live) continue;

@@ -623,6 +623,49 @@ class HipOps:
                    int(silu_mul), self._stream())
         return out, resid
 
+    def norm_heads(self, resid, delta, norm_weight, eps, weight, batch, table, cache, *, num_heads,
+                   num_kv_heads, head_dim, q_weight, k_weight, head_eps, cos_sin, tile=0):
+        """`norm_linear` for a q/k/v projection and `qk_norm_rope_store` behind it in one kernel:
+        the queries [T, num_heads, head_dim], keys and values being in their pages then.  None where
+        that is not built or not the faster way (and nothing has been done): a prompt's rows that
+        the tiled product before has prepared, heads of 128, a bfloat16 cache.  `tile` as in
+        `gemm_tiled` (the tiles that hold a head: 1 and 2)."""
+        if not (isinstance(delta, PreparedRows) and delta.tiled and head_dim == 128
+                and cache.k_pages.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16
+                and not self._decode_fits(batch, num_kv_heads, num_heads // num_kv_heads, head_dim,
+                                          cache.page_size, True)):
+            return None
+        M, K = delta.rows.shape
+        N = (num_heads + 2 * num_kv_heads) * head_dim
+        d, key = self.dispatch, ("heads", M, N, K, delta.slices, cache.page_size)
+        fits = self._routes.get(key) if self._routes_of is d else None
+        if fits is None:
+            fits = self._kept_routes()[key] = self.lib.ts_gemm_tiled_heads_fits(
+                M, N, K, delta.slices, head_dim, cache.page_size) == 1
+        if not fits and tile == 0:
+            return None
+        hint = delta.hint
+        if hint.norm_weight is not norm_weight or hint.eps != eps or hint.weight is not weight \
+                or hint.silu_mul:
+            raise ValueError("norm_heads: the rows were prepared for another norm or product")
+        if resid.shape != (M, K):
+            raise ValueError("norm_heads: prepared rows and stream differ in shape")
+        self._check("weight", weight, torch.bfloat16, shape=(N, K))
+        self._check_cache(cache, table, batch, num_kv_heads, head_dim)
+        a = QkPrepareArgs()
+        self._fill_qk_args(a, batch, M, num_heads, num_kv_heads, head_dim, q_weight, k_weight,
+                           head_eps, cos_sin)
+        if ((a.cos or 0) | (a.sin or 0) | cache.k_pages.data_ptr() | cache.v_pages.data_ptr()) % 16:
+            return None                    # (16 bytes at a time: others have the separate kernels)
+        q = torch.empty(M, num_heads, head_dim, dtype=torch.bfloat16, device=self.device)
+        a.q_out = q.data_ptr()
+        a.k_dst, a.v_dst = cache.k_pages.data_ptr(), cache.v_pages.data_ptr()
+        a.table, a.table_width = table.data_ptr(), table.shape[1]
+        a.page_size, a.paged, a.store_kv = cache.page_size, 1, 1
+        self._call(self.lib.ts_gemm_tiled_heads_bf16, _ptr(delta.rows), _ptr(delta.sumsq),
+                   delta.slices, c_float(eps), _ptr(weight), byref(a), M, K, tile, self._stream())
+        return q
+
     def norm_linear(self, resid, delta, norm_weight, eps, weight, out_dtype, silu_mul=False):
         """(RMSNorm(resid + delta) W^T, resid + delta): the residual add, the norm and
         the product in one kernel where it can be (bfloat16 weights, at most 16 rows);
@@ -697,9 +740,14 @@ class HipOps:
         if head_dim % 2:
             raise ValueError(f"head_dim={head_dim} must be even")
         a = QkPrepareArgs()
-        a.qkv = qkv.data_ptr()
-        a.num_tokens, a.nq, a.nkv, a.hd = T, num_heads, kv_in_row, head_dim
-        a.eps, a.row_extra = eps, row_extra
+        a.qkv, a.row_extra = qkv.data_ptr(), row_extra
+        self._fill_qk_args(a, batch, T, num_heads, kv_in_row, head_dim, q_weight, k_weight, eps,
+                           cos_sin)
+        return a
+
+    def _fill_qk_args(self, a, batch, T, num_heads, kv_in_row, head_dim, q_weight, k_weight, eps,
+                      cos_sin):
+        a.num_tokens, a.nq, a.nkv, a.hd, a.eps = T, num_heads, kv_in_row, head_dim, eps
         if q_weight is not None:
             a.q_weight = self._check("q norm weight", q_weight, torch.float32,
                                      shape=(head_dim,)).data_ptr()
@@ -721,7 +769,6 @@ class HipOps:
         self._check("entry_of_token", batch.entry_of_token, torch.int32, shape=(T,))
         a.positions = batch.positions.data_ptr()
         a.entry_of_token = batch.entry_of_token.data_ptr()
-        return a
 
     def _check_cache(self, cache, table, batch, nkv, head_dim):
         P = cache.page_size

@@ -12,7 +12,7 @@ from __future__ import annotations
 
 import torch
 
-from tokensprint_amd.kernels.stream import StreamProducts, fused_rmsnorm_of
+from tokensprint_amd.kernels.stream import PreparedRows, StreamProducts, fused_rmsnorm_of
 from tokensprint_amd.parts.base import MIXERS, Mixer, PagedKVNeed, TensorDecl, register
 
 
@@ -80,10 +80,34 @@ class GroupedQueryAttention(StreamProducts, Mixer):
         fused = fused_rmsnorm_of(norm)
         if fused is None:
             return super().forward_from_stream(resid, delta, norm, batch, cache, write_cache)
-        qkv, resid = self.ops.norm_linear(resid, delta, fused[0], fused[1], self.w_qkv,
-                                          self.ctx.dtype)
-        o = self._attend(qkv, batch, cache, write_cache)
+        o = self._attend_prepared(resid, delta, fused, batch, cache, write_cache)
+        if o is None:
+            qkv, resid = self.ops.norm_linear(resid, delta, fused[0], fused[1], self.w_qkv,
+                                              self.ctx.dtype)
+            o = self._attend(qkv, batch, cache, write_cache)
         return self.last_product(o, self.w_o, resid, hint), resid
+
+    def _attend_prepared(self, resid, delta, norm, batch, cache, write_cache):
+        """The projection of rows that the product before has prepared, and what `_attend` makes of
+        it, where the provider has the projection and the heads' preparation in one kernel; else
+        None, and nothing has been done."""
+        if not isinstance(delta, PreparedRows) or cache is None or not write_cache \
+                or not self.own_kv or not hasattr(self.ops, "norm_heads"):
+            return None
+        tables = self.position.rotary_tables() if self.position is not None else None
+        if self.position is not None and tables is None:
+            return None
+        table = batch.tables[cache.group]
+        q = self.ops.norm_heads(
+            resid, delta, norm[0], norm[1], self.w_qkv, batch, table, cache, num_heads=self.nq,
+            num_kv_heads=self.nkv, head_dim=self.hd, q_weight=self.w_qnorm, k_weight=self.w_knorm,
+            head_eps=self.eps, cos_sin=tables)
+        if q is None:
+            return None
+        o = self.ops.paged_attention(q, batch, table, cache, num_heads=self.nq,
+                                     num_kv_heads=self.nkv, head_dim=self.hd, scale=self.scale,
+                                     window=self.window, sink=self.sink, **self.score_options)
+        return o.view(q.shape[0], self.nq * self.hd)
 
     def forward(self, h, batch, cache, write_cache):
         o = self._attend(self.ops.linear(h, self.w_qkv, self.ctx.dtype), batch, cache, write_cache)
