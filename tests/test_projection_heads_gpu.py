@@ -24,7 +24,7 @@ def rand(shape, seed):
 @pytest.mark.parametrize("page", [16, 64, 4])
 @pytest.mark.parametrize("nq, nkv, K, normed, turned, tile", [
     (4, 2, 256, True, True, 1), (4, 2, 256, True, True, 2), (5, 1, 512, False, True, 1),
-    (3, 3, 320, True, False, 2)])
+    (3, 3, 320, True, False, 2), (4, 2, 256, True, True, 6), (2, 1, 512, True, True, 6)])
 def test_same_bits_as_the_kernels_one_by_one(gpu_device, nq, nkv, K, normed, turned, tile, page, spans):
     ops, hd, eps = load_hip_ops(gpu_device), 128, 1e-6
     batch, cache, table, _ = paged_scenario(gpu_device, torch.bfloat16, nkv=nkv, hd=hd, page_size=page,

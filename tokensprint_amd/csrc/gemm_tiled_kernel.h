@@ -101,7 +101,7 @@ constexpr int kHeadRow = 128 + 8;
 template <int BM, int THREADS, typename PUT>
 __device__ __forceinline__ void heads_out(const TiledHeadsArgs& g, int head, int m0, const int* row_pos,
                                           const int* row_entry, bf16_t* rows, PUT put) {
-  constexpr int HD = 128, L = HD / 8, AT_ONCE = THREADS / L, TURNS = BM / AT_ONCE, AHEAD = 4;
+  constexpr int HD = 128, L = HD / 8, AT_ONCE = THREADS / L, TURNS = BM / AT_ONCE, AHEAD = TURNS < 4 ? TURNS : 4;
   static_assert(BM % AT_ONCE == 0 && TURNS % AHEAD == 0, "whole turns");
   const QkPrepareArgs& a = g.heads;
   const int sub = threadIdx.x % L, row0 = threadIdx.x / L;

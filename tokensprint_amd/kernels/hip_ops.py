@@ -629,7 +629,7 @@ class HipOps:
         the queries [T, num_heads, head_dim], keys and values being in their pages then.  None where
         that is not built or not the faster way (and nothing has been done): a prompt's rows that
         the tiled product before has prepared, heads of 128, a bfloat16 cache.  `tile` as in
-        `gemm_tiled` (the tiles that hold a head: 1 and 2)."""
+        `gemm_tiled` (the tiles that hold a head: 1, 2 and 6)."""
         if not (isinstance(delta, PreparedRows) and delta.tiled and head_dim == 128
                 and cache.k_pages.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16
                 and not self._decode_fits(batch, num_kv_heads, num_heads // num_kv_heads, head_dim,
