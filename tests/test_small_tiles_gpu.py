@@ -1,0 +1,81 @@
+"""The tiles of 64 rows of the LDS-tiled product against its others: K is summed in index order by one
+accumulator whatever the tile, so every tile gives the same bits, in every form."""
+
+import pytest
+import torch
+
+from tokensprint_amd.kernels import load_hip_ops
+from tokensprint_amd.kernels.hip_ops import _ptr
+
+pytestmark = pytest.mark.gpu
+TILES = (6, 7, 8)
+
+
+def rand(shape, seed, device):
+    gen = torch.Generator().manual_seed(seed)
+    return (0.1 * torch.randn(shape, generator=gen)).to(device, torch.bfloat16)
+
+
+@pytest.mark.parametrize("M", [1, 15, 64, 65, 130])
+@pytest.mark.parametrize("N, K", [(16, 256), (48, 320), (144, 512), (1344, 256)])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+def test_plain_and_paired(gpu_device, out_dtype, M, N, K):
+    ops = load_hip_ops(gpu_device)
+    x, w = rand((M, K), 1, gpu_device), rand((N, K), 2, gpu_device)
+    want = ops.gemm_tiled(x, w, out_dtype, tile=3)
+    exact = x.double().cpu() @ w.double().cpu().T
+    # K products of 8-bit operands, added in 32 bits; then rounded to the output's type
+    tol = 2.0 ** -8 if out_dtype == torch.bfloat16 else K * 2.0 ** -24
+    assert (want.double().cpu() - exact).abs().max() <= tol * (x.double().cpu().abs() @ w.double().cpu().abs().T).max()
+    for tile in (0,) + TILES:
+        assert torch.equal(ops.gemm_tiled(x, w, out_dtype, tile=tile), want), tile
+    if out_dtype == torch.bfloat16:
+        pair = rand((2 * N, K), 3, gpu_device)
+        want = ops.gemm_tiled(x, pair, out_dtype, pair=True, tile=3)
+        for tile in (0,) + TILES:
+            assert torch.equal(ops.gemm_tiled(x, pair, out_dtype, pair=True, tile=tile), want), tile
+
+
+@pytest.mark.parametrize("M", [1, 63, 65, 200])
+@pytest.mark.parametrize("N, K", [(32, 256), (96, 576), (256, 320)])
+def test_tail_and_scaled(gpu_device, M, N, K):
+    ops = load_hip_ops(gpu_device)
+    x, w = rand((M, K), 1, gpu_device), rand((N, K), 2, gpu_device)
+    norm_w = (1 + rand((N,), 3, gpu_device)).float()
+    stream = rand((M, N), 4, gpu_device).float()
+    parts = ops.lib.ts_gemm_tiled_tail_parts(N)
+    results = []
+    for tile in (3, 0) + TILES:
+        resid, rows = stream.clone(), torch.empty(M, N, device=gpu_device, dtype=torch.bfloat16)
+        sums = torch.empty(parts, M, device=gpu_device)
+        ops._call(ops.lib.ts_gemm_tiled_tail_bf16, _ptr(x), _ptr(w), _ptr(resid), _ptr(norm_w), _ptr(rows),
+                  _ptr(sums), M, N, K, tile, ops._stream())
+        results.append((resid, rows, sums))
+    assert torch.equal(results[0][0], stream + ops.gemm_tiled(x, w, torch.bfloat16, tile=3).float())
+    for got in results[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got, results[0]))
+    if N < 256:
+        return
+    behind = rand((48, N), 5, gpu_device)
+    outs = []
+    for tile in (3, 0) + TILES:
+        outs.append(torch.empty(M, 48, device=gpu_device))
+        ops._call(ops.lib.ts_gemm_tiled_scaled_bf16, _ptr(results[0][1]), _ptr(results[0][2]), parts,
+                  _f(1e-6), _ptr(behind), _ptr(outs[-1]), 0, M, 48, N, 0, tile, ops._stream())
+    assert all(torch.equal(o, outs[0]) for o in outs[1:])
+
+
+@pytest.mark.parametrize("M", [8, 9, 12, 13, 33, 64])
+@pytest.mark.parametrize("K", [1024, 2048])
+def test_output_heads_of_few_rows(gpu_device, M, K):
+    """Whichever kernel's: a row's logits against float64, float32 sums of K products."""
+    ops = load_hip_ops(gpu_device)
+    x, w = rand((M, K), 6, gpu_device), rand((16400, K), 7, gpu_device)
+    out = ops.linear(x, w, torch.float32)
+    exact = x.double() @ w.double().T
+    assert (out.double() - exact).norm() <= 4e-6 * exact.norm()
+
+
+def _f(value):
+    from ctypes import c_float
+    return c_float(value)

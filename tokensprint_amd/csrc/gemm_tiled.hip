@@ -9,14 +9,14 @@ extern "C" int ts_gemm_tiled_fits(int M, int N, int K, int pair) {
          (int64_t)M * K * 2 < (1ll << 32) && rows_w * K * 2 < (1ll << 32);
 }
 
-// Per cent of the rounds of the units that the product's elements fill in the tile that its sizes
-// take: what edges and a last round leave empty is time in which the library, whose kernels share
+// Per cent of the rounds of the units that the product's elements fill in the tile of 128 rows or more
+// that its sizes take: what edges and a last round leave empty is time in which the library, whose kernels share
 // a tile's K out over units, gets ahead.
 extern "C" int ts_gemm_tiled_fill(int M, int N, int K, int pair) {
   if (!ts_gemm_tiled_fits(M, N, K, pair)) return 0;
   TiledArgs g{};
   g.M = M, g.N = N, g.K = K;
-  const int tile = cheapest_tile(g, pair), units = compute_units();
+  const int tile = cheapest_tile(g, pair, 128), units = compute_units();
   const int64_t cols = pair ? 2 * (int64_t)N : N;
   for (const TileCost& t : kTileCosts) {
     if (t.tile != tile) continue;
@@ -47,8 +47,17 @@ extern "C" int ts_gemm_tiled_fill(int M, int N, int K, int pair) {
 // than one such round 0.59 to 1.09, 0.80 in the mean, filled by two thirds (tiles of 256 x 128 in
 // several rounds 1.11 to 1.19).  K = 25,600: one round of up to 256 x 128 0.65 to 0.97 whatever it fills
 // (5,120 columns, 1,536 rows 338 / 507 us), of larger tiles 0.58 to 1.10, 0.88 in the mean.
+// N a multiple of 256 in the small tiles (64 x 64 and 64 x 32), timed at 65 to 1,500 rows of 13 weights (N 512
+// to 9,216): K up to 2,048 0.49 to 0.97, 0.70 in the mean, whatever they fill (against the fastest of the
+// library's first eight algorithms 0.57 to 0.92 at 65 to 600 rows of five of them); K = 4,096 0.80 to 0.94
+// above 256 rows, 1.03 to 1.27 below; K = 8,192 0.90 to 1.38.
 extern "C" int ts_gemm_tiled_ahead(int M, int N, int K, int c_type) {
   if (!ts_gemm_tiled_fits(M, N, K, 0)) return 0;
+  TiledArgs g{};
+  g.M = M, g.N = N, g.K = K;
+  const int small = cheapest_tile(g, false);
+  if (N % 256 == 0 && (small == 7 || small == 8)) return K <= 2048 || (K <= 4096 && M > 256);
+  const int tile = cheapest_tile(g, false, 128), units = compute_units();
   const int fill = ts_gemm_tiled_fill(M, N, K, 0);
   if (N % 256 != 0) {
     if (N < 16384 && (K <= 512 ? N >= 48 : K <= 1024 && N >= 1280)) return 1;
@@ -56,9 +65,6 @@ extern "C" int ts_gemm_tiled_ahead(int M, int N, int K, int c_type) {
     return fill >= (K <= 6144 && N <= 4096 && M <= 1024 ? 49 : 70);
   }
   if (c_type != TS_BF16 && fill >= 80) return 1;
-  TiledArgs g{};
-  g.M = M, g.N = N, g.K = K;
-  const int tile = cheapest_tile(g, false), units = compute_units();
   int64_t area = 0, tiles = 0;
   for (const TileCost& t : kTileCosts) {
     if (t.tile != tile) continue;
@@ -74,7 +80,7 @@ extern "C" int ts_gemm_tiled_ahead(int M, int N, int K, int c_type) {
 
 // C[M, N] = A[M, K] W[N, K]^T, or with `pair` C[M, N] = silu(A Wg^T) * (A Wu^T) (or, with a
 // `limit` other than 0, gated_unit's other forms) for W = [Wg; Wu] of 2 N rows.  `c_type`: bfloat16 or float32 (float32 not with `pair`).
-// `tile`: 0 lets the sizes choose; 1 to 5 name a tile (for measuring; the result is the
+// `tile`: 0 lets the sizes choose; 1 to 8 name a tile (for measuring; the result is the
 // same to the bit).
 extern "C" int ts_gemm_tiled_bf16(const void* a, const void* w, void* c, int c_type, int M, int N,
                                   int K, int pair, int tile, float limit, hipStream_t stream) {

@@ -31,14 +31,16 @@ float estimate(int M, int N, int K, const TileCost (&costs)[COUNT], int* tile) {
 
 // 1 if ts_gemm_tiled_heads_bf16 takes a projection of these sizes and is the faster way: by the estimate
 // of its tile, 2.5 us of epilogue, that of the tile which the product would take, and the preparation
-// kernel's time.  One kernel and two, 4,096 columns (24 + 8 heads), K = 1,024, weights from memory, us:
+// kernel's time.  Rows below 512 are prepared in eager steps only, which wait for the host: four
+// microseconds more for a launch less.  One kernel and two, 4,096 columns (24 + 8 heads), K = 1,024, weights from memory, us:
 // 72 rows 10.0 / 11.7, 300 10.3 / 13.8, 512 11.0 / 15.5, 800 16.0 / 21.0, 1,024 16.7 / 21.9, 1,500 25.0 /
 // 29.4, 2,048 26.6 / 32.4, 2,500 40.6 / 41.4, 4,096 48 / 58, 8,192 92 / 103.  (128 x 128 as the smallest
 // tile: 300 rows 14.4.)
 extern "C" int ts_gemm_tiled_heads_fits(int M, int N, int K, int parts, int hd, int page_size) {
   if (hd != 128 || N % 128 != 0 || page_size <= 0 || !ts_gemm_tiled_scaled_fits(M, N, K, 0, parts)) return 0;
-  const float prepare_us = 3.5f + 7.f * ((float)M * N / (2048.f * 4096.f));
-  return estimate(M, N, K, kHeadTiles, nullptr) + 2.5f <= estimate(M, N, K, kTileCosts, nullptr) + prepare_us;
+  const float prepare_us = 3.5f + 7.f * ((float)M * N / (2048.f * 4096.f)), host_us = M < 512 ? 4.f : 0.f;
+  return estimate(M, N, K, kHeadTiles, nullptr) + 2.5f <=
+         estimate(M, N, K, kTileCosts, nullptr) + prepare_us + host_us;
 }
 
 // q, and k and v into their pages, of rows[M, K] W[N, K]^T (ts_gemm_tiled_scaled_bf16's rows and sums),

@@ -696,12 +696,21 @@ int launch_tiled(TiledArgsOf<FORM> g, hipStream_t stream) {
 // ordinary data up to 1.5, with zeros 1.2), a small one's by the rate at which a unit takes
 // direct loads (0.33 us for 128 x 64, 2.3 times the matrix cores' time), but a tile is one
 // workgroup and a unit without one idles.
+// The tiles of 64 rows are for portions of few rows.  With 128 x 64 as the smallest, 300 rows of 1,024
+// columns were 48 workgroups; the product that ends a sub-layer took 12.4 us with K = 2,048 and 16.6 with
+// K = 3,072, and takes 7.3 and 9.5 in 64 x 32 tiles (160 workgroups of four wavefronts); 1,024 rows 13.2 and
+// 18.0, in 64 x 64 tiles 10.3 and 13.5.  64 x 128 is for up to 64 rows of many columns, where a tile of 128
+// rows brings every row of A twice (64 rows of 151,936 columns of 4,096: 244 us, 243 and 267 in 128 x 128
+// and 128 x 64; 16 rows 224, 236, 242).  Their fixed parts are what 65 to 1,024 rows of 21 weights show, and
+// make a second round as long as the first, which for tiles that share a unit it is not (so the
+// larger tiles are chosen there, which are about as fast).
 struct TileCost {
   int tile, bm, bn;
   float fixed_us, step_us, pair_us;
 };
 constexpr TileCost kTileCosts[] = {
-    {3, 128, 64, 1.2f, 0.329f, 0.5f}, {2, 128, 128, 2.4f, 0.491f, 0.8f}, {1, 256, 128, 4.5f, 0.721f, 1.4f},
+    {8, 64, 32, 2.2f, 0.1375f, 0.5f}, {7, 64, 64, 2.9f, 0.18f, 0.5f}, {3, 128, 64, 1.2f, 0.329f, 0.5f},
+    {6, 64, 128, 1.2f, 0.329f, 0.5f}, {2, 128, 128, 2.4f, 0.491f, 0.8f}, {1, 256, 128, 4.5f, 0.721f, 1.4f},
     {5, 256, 192, 6.6f, 0.931f, 1.1f}, {4, 256, 256, 7.7f, 1.126f, 1.6f},
 };
 
@@ -719,12 +728,14 @@ inline int compute_units() {
   return units[device];
 }
 
-inline int cheapest_tile(const TiledArgs& g, bool pair) {
+// (`least_rows`: of the tiles with so many rows or more)
+inline int cheapest_tile(const TiledArgs& g, bool pair, int least_rows = 0) {
   const int units = compute_units();
   const int64_t cols = pair ? 2 * (int64_t)g.N : g.N;
   int best = 3;
   float best_us = -1.f;
   for (const TileCost& t : kTileCosts) {
+    if (t.bm < least_rows) continue;
     const int64_t tiles = (int64_t)((g.M + t.bm - 1) / t.bm) * ((cols + t.bn - 1) / t.bn);
     const int64_t rounds = (tiles + units - 1) / units;
     const float us = rounds * (t.fixed_us + (pair ? t.pair_us : 0.f) + t.step_us * (g.K / 64));
@@ -742,6 +753,9 @@ int choose_tile(const TiledArgs& g, int tile, hipStream_t stream) {
     case 3: return launch_tiled<128, 64, 4, 2, 4, PAIR, TO, FORM>(g, stream);
     case 4: return launch_tiled<256, 256, 2, 4, 2, PAIR, TO, FORM>(g, stream);
     case 5: return launch_tiled<256, 192, 4, 2, 2, PAIR, TO, FORM>(g, stream);
+    case 6: return launch_tiled<64, 128, 2, 4, 4, PAIR, TO, FORM>(g, stream);
+    case 7: return launch_tiled<64, 64, 4, 2, 4, PAIR, TO, FORM>(g, stream);
+    case 8: return launch_tiled<64, 32, 4, 1, 4, PAIR, TO, FORM>(g, stream);
   }
   TS_FAIL("gemm_tiled: no tile %d", tile);
 }
