@@ -62,7 +62,39 @@ def test_tail_and_scaled(gpu_device, M, N, K):
         outs.append(torch.empty(M, 48, device=gpu_device))
         ops._call(ops.lib.ts_gemm_tiled_scaled_bf16, _ptr(results[0][1]), _ptr(results[0][2]), parts,
                   _f(1e-6), _ptr(behind), _ptr(outs[-1]), 0, M, 48, N, 0, tile, ops._stream())
-    assert all(torch.equal(o, outs[0]) for o in outs[1:])
+    # the same sums with a row's side by side, what is behind the last left as it is
+    by_row = torch.full((M, -(-parts // 4) * 4), float("nan"), device=gpu_device)
+    by_row[:, :parts] = results[0][2].T
+    for pair, out in ((0, torch.empty(M, 48, device=gpu_device)),
+                      (1, torch.empty(M, 16, device=gpu_device, dtype=torch.bfloat16))):
+        w_behind = behind[:32].contiguous() if pair else behind
+        got, want = out.clone(), out
+        for name, sums, o in (("ts_gemm_tiled_scaled_rows_bf16", by_row, got),
+                              ("ts_gemm_tiled_scaled_bf16", results[0][2], want)):
+            ops._call(getattr(ops.lib, name), _ptr(results[0][1]), _ptr(sums), parts, _f(1e-6),
+                      _ptr(w_behind), _ptr(o), pair, M, o.shape[1], N, pair, 0, ops._stream())
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("M", [16, 17, 33, 64])
+@pytest.mark.parametrize("N, silu_mul", [(1040, False), (1024, True)])
+def test_rows_of_the_weight_streaming_tail(gpu_device, M, N, silu_mul):
+    """linear_into_stream and norm_linear at the rows where the second changes its kernel, against
+    float64: two roundings to bfloat16 of operands, and of the results."""
+    from tokensprint_amd.kernels.stream import NormHint
+    ops, K, width, eps = load_hip_ops(gpu_device), 2048, 1024, 1e-6
+    x, w_o = rand((M, K), 8, gpu_device), rand((width, K), 9, gpu_device)
+    resid, norm_w = rand((M, width), 10, gpu_device).float() * 30, (1 + rand((width,), 11, gpu_device)).float()
+    weight = rand((N * (2 if silu_mul else 1), width), 12, gpu_device)
+    want = resid.double() + (x.double() @ w_o.double().T)
+    normed = want / (want.square().mean(-1, keepdim=True) + eps).sqrt() * norm_w.double()
+    want_out = normed @ weight.double().T
+    if silu_mul:
+        want_out = torch.nn.functional.silu(want_out[:, :N]) * want_out[:, N:]
+    prepared = ops.linear_into_stream(x, w_o, resid, NormHint(norm_w, eps, weight, silu_mul))
+    assert prepared is not None and not prepared.tiled
+    out, _ = ops.norm_linear(resid, prepared, norm_w, eps, weight, torch.bfloat16, silu_mul)
+    assert (out.double() - want_out).norm() <= 1e-2 * want_out.norm()
 
 
 @pytest.mark.parametrize("M", [8, 9, 12, 13, 33, 64])

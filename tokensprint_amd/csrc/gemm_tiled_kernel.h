@@ -51,9 +51,10 @@ struct TiledArgs {
   int M, N, K;          // N: columns of C (with PAIR: of each half of W)
   int tiles_m, tiles_n;
   int panel;            // tiles of a panel along M
-  // SCALED: the sums of squares of A's rows [parts, M]
+  // SCALED: the sums of squares of A's rows [parts, M], or (`row_stride` not 0, a multiple of 4) a row's
+  // side by side, as the weight-streaming tail form leaves them
   const float* sumsq_in;
-  int parts;
+  int parts, row_stride;
   float eps;
   // TAIL: the float32 stream [M, N] (read and written), the norm's weight [N], what is
   // handed on [M, N], the sums of squares of the new stream's rows [N / 32, M]
@@ -253,9 +254,19 @@ __global__ __launch_bounds__(64 * GM * GN, 1) void gemm_tiled_kernel(TiledArgsOf
         float sq = 0.f;
         for (int p0 = 0; p0 < g.parts; p0 += 32) {
           float part[32];
+          if (g.row_stride == 0) {
 #pragma unroll
-          for (int i = 0; i < 32; ++i)
-            part[i] = g.sumsq_in[(int64_t)min(p0 + i, g.parts - 1) * g.M + m];
+            for (int i = 0; i < 32; ++i)
+              part[i] = g.sumsq_in[(int64_t)min(p0 + i, g.parts - 1) * g.M + m];
+          } else {
+            const float* at = g.sumsq_in + (int64_t)m * g.row_stride;
+#pragma unroll
+            for (int i = 0; i < 32; i += 4) {
+              const f32x4 four = *(const f32x4*)(at + min(p0 + i, g.row_stride - 4));
+#pragma unroll
+              for (int e = 0; e < 4; ++e) part[i + e] = four[e];
+            }
+          }
 #pragma unroll
           for (int i = 0; i < 32; ++i) sq += p0 + i < g.parts ? part[i] : 0.f;
         }

@@ -40,26 +40,45 @@ extern "C" int ts_gemm_tiled_scaled_fits(int M, int N, int K, int pair, int part
   return ts_gemm_tiled_fits(M, N, K, pair) && parts > 0 && parts <= 4096;
 }
 
+namespace {
+
+int scaled(const char* who, const void* rows, const float* sumsq, int parts, int row_stride, float eps,
+           const void* w, void* c, int c_type, int M, int N, int K, int pair, int tile, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (!ts_gemm_tiled_scaled_fits(M, N, K, pair, parts))
+    TS_FAIL("%s: M=%d N=%d K=%d parts=%d not taken", who, M, N, K, parts);
+  if (((uintptr_t)rows | (uintptr_t)w | (uintptr_t)c | (row_stride ? (uintptr_t)sumsq : 0)) & 15)
+    TS_FAIL("%s: operands must be 16-byte aligned", who);
+  TiledArgs g{(const bf16_t*)rows, (const bf16_t*)w, c, M, N, K, 0, 0, 1};
+  g.sumsq_in = sumsq;
+  g.parts = parts;
+  g.row_stride = row_stride;
+  g.eps = eps;
+  if (pair) {
+    if (c_type != TS_BF16) TS_FAIL("%s: the paired form writes bfloat16", who);
+    return choose_tile<true, bf16_t, kScaled>(g, tile, stream);
+  }
+  if (c_type == TS_BF16) return choose_tile<false, bf16_t, kScaled>(g, tile, stream);
+  if (c_type == TS_F32) return choose_tile<false, float, kScaled>(g, tile, stream);
+  TS_FAIL("%s: output type %d", who, c_type);
+}
+
+}  // namespace
+
 // C[M, N] = rsqrt(sum_p sumsq[p, m] / K + eps) * (rows[M, K] W[N, K]^T), or with `pair` the
 // same for both halves of W = [Wg; Wu] and C = silu(gate) * up.  `c_type`: bfloat16, or
 // float32 without `pair`.
 extern "C" int ts_gemm_tiled_scaled_bf16(const void* rows, const float* sumsq, int parts,
                                          float eps, const void* w, void* c, int c_type, int M,
                                          int N, int K, int pair, int tile, hipStream_t stream) {
-  if (M <= 0 || N <= 0) return 0;
-  if (!ts_gemm_tiled_scaled_fits(M, N, K, pair, parts))
-    TS_FAIL("gemm_tiled_scaled: M=%d N=%d K=%d parts=%d not taken", M, N, K, parts);
-  if (((uintptr_t)rows | (uintptr_t)w | (uintptr_t)c) & 15)
-    TS_FAIL("gemm_tiled_scaled: operands must be 16-byte aligned");
-  TiledArgs g{(const bf16_t*)rows, (const bf16_t*)w, c, M, N, K, 0, 0, 1};
-  g.sumsq_in = sumsq;
-  g.parts = parts;
-  g.eps = eps;
-  if (pair) {
-    if (c_type != TS_BF16) TS_FAIL("gemm_tiled_scaled: the paired form writes bfloat16");
-    return choose_tile<true, bf16_t, kScaled>(g, tile, stream);
-  }
-  if (c_type == TS_BF16) return choose_tile<false, bf16_t, kScaled>(g, tile, stream);
-  if (c_type == TS_F32) return choose_tile<false, float, kScaled>(g, tile, stream);
-  TS_FAIL("gemm_tiled_scaled: output type %d", c_type);
+  return scaled("gemm_tiled_scaled", rows, sumsq, parts, 0, eps, w, c, c_type, M, N, K, pair, tile, stream);
+}
+
+// The same for rows that the weight-streaming tail form has prepared: sumsq[M, parts rounded up to four],
+// as ts_gemm_tail_bf16 leaves it.
+extern "C" int ts_gemm_tiled_scaled_rows_bf16(const void* rows, const float* sumsq, int parts,
+                                              float eps, const void* w, void* c, int c_type, int M,
+                                              int N, int K, int pair, int tile, hipStream_t stream) {
+  return scaled("gemm_tiled_scaled_rows", rows, sumsq, parts, (parts + 3) & ~3, eps, w, c, c_type, M, N, K,
+                pair, tile, stream);
 }

@@ -15,6 +15,17 @@ from dataclasses import dataclass
 
 @dataclass(frozen=True)
 class Dispatch:
+    # ---- the product behind a norm whose rows the weight-streaming kernel in front has prepared: the
+    # same kernels', or from `tiled_scaled_rows` rows the LDS-tiled kernel's in tiles of 64 rows, whose
+    # workgroups read the rows once in 32 or 64 columns, not in 16.  Here and there, us, weights from
+    # memory: 4,096 x 1,024 17 rows 5.2 / 5.5, 32 rows 6.0 / 5.5, 64 rows 8.3 / 5.8; 1,536 x 1,024 5.4 / 5.4, 6.3 /
+    # 5.4, 8.2 / 5.6; gate/up 2 x 3,072 x 1,024 16 rows 6.8 / 6.8, 17 rows 9.0 / 6.8, 64 rows 12.4 / 7.4.  One line
+    # for both, at the rows where a row's sums change their order anyway.  K = 512 gains nothing (1,024
+    # columns 3.4 / 4.2, 3.5 / 4.3, 4.7 / 4.4), K = 2,048 as much as it loses (4,096 columns 17 rows 8.9 / 10.7,
+    # 33 rows 11.9 / 10.9).
+    tiled_scaled_rows: int = 17
+    tiled_scaled_k: tuple[int, int] = (1024, 1536)
+
     # ---- plain bfloat16 products: from how many rows the vendor library (hipBLASLt)
     # takes them, as the reference sends every linear layer to its vendor library
     # (engine/nn/base_layers.py:7-10).  Measured inside captured graphs at the Qwen3-0.6B

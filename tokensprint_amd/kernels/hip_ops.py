@@ -612,6 +612,13 @@ class HipOps:
                    self._stream())
         return PreparedRows(rows, sumsq, parts, hint)
 
+    def _tiled_scaled_ok(self, M, N, K, silu_mul, slices):
+        """Whether the product of rows that the weight-streaming kernel has prepared is the
+        LDS-tiled kernel's."""
+        d = self.dispatch
+        return (M >= d.tiled_scaled_rows and d.tiled_scaled_k[0] <= K <= d.tiled_scaled_k[1]
+                and self.lib.ts_gemm_tiled_scaled_fits(M, N, K, int(silu_mul), slices) == 1)
+
     def _prepared_linear(self, resid, prepared, norm_weight, eps, weight, out_dtype, silu_mul):
         hint = prepared.hint
         if hint.norm_weight is not norm_weight or hint.eps != eps or hint.weight is not weight \
@@ -624,8 +631,9 @@ class HipOps:
         if out_dtype not in (torch.bfloat16, torch.float32) or (silu_mul and out_dtype != torch.bfloat16):
             raise ValueError(f"norm_linear: prepared rows cannot give {out_dtype}")
         out = torch.empty(M, N, dtype=out_dtype, device=self.device)
-        if prepared.tiled:
-            self._call(self.lib.ts_gemm_tiled_scaled_bf16, _ptr(prepared.rows),
+        if prepared.tiled or self._tiled_scaled_ok(M, N, K, silu_mul, prepared.slices):
+            self._call(self.lib.ts_gemm_tiled_scaled_bf16 if prepared.tiled
+                       else self.lib.ts_gemm_tiled_scaled_rows_bf16, _ptr(prepared.rows),
                        _ptr(prepared.sumsq), prepared.slices, c_float(eps), _ptr(weight),
                        _ptr(out), _TYPE_CODE[out_dtype], M, N, K, int(silu_mul), 0, self._stream())
             return out, resid
