@@ -61,6 +61,20 @@ extern "C" int ts_attention_decode(const AttentionDecodeArgs* p, hipStream_t str
     TS_CHECK_LAUNCH("attention_decode");
     return 0;
   }
+  // (positions times 64 are ranked in 32 bits)
+  const int64_t items = (int64_t)m.num_tiles * a.nkv * m.head_blocks;
+  if (args.qkv && m.num_splits == 1 && m.num_tiles <= 64 && items > 256 &&
+      (int64_t)a.table_width * a.page_size < 1 << 25) {
+    switch (a.hd) {
+#define TS_CASE(HD) case HD: rc = launch_decode<HD, false, true>(args, stream); break;
+      TS_CASE(32) TS_CASE(64) TS_CASE(96) TS_CASE(128) TS_CASE(160) TS_CASE(192) TS_CASE(224) TS_CASE(256)
+#undef TS_CASE
+      default: TS_FAIL("attention_decode: head_dim=%d not built", a.hd);
+    }
+    if (rc) return rc;
+    TS_CHECK_LAUNCH("attention_decode");
+    return 0;
+  }
   switch (a.hd) {
 #define TS_CASE(HD) case HD: rc = launch_decode<HD, false>(args, stream); break;
     TS_CASE(16) TS_CASE(32) TS_CASE(48) TS_CASE(64) TS_CASE(80) TS_CASE(96) TS_CASE(112)

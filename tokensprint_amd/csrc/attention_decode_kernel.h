@@ -147,8 +147,29 @@ __device__ __forceinline__ void merge_splits_here(const float* partial_o, const 
   }
 }
 
+// The entry with the rank-th longest context of up to 64 (equal ones in order), and its position.
+struct Ranked {
+  int entry, pos;
+};
+__device__ __forceinline__ Ranked ranked_entry(const int* positions, int entries, int rank, int lane) {
+  const int pos = positions[min(lane, entries - 1)];
+  const int key = lane < entries ? pos * 64 + 63 - lane : -1;
+  int before = 0;
+#pragma unroll
+  for (int j = 0; j < kWave; ++j) before += __builtin_amdgcn_readlane(key, j) > key ? 1 : 0;
+  const int entry = __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < entries && before == rank));
+  return {entry, __builtin_amdgcn_readlane(pos, entry)};
+}
+
 // EXTRA: scores with a cap, a distance bias or a query temperature (attention.h).
-template <int HD, bool FUSED, bool EXTRA>
+// RANKED (more items than the chip has units, up to 64 entries, no splits): the items are the entries'
+// in the order of their contexts, longest first.  A unit holds one workgroup at a time (its eight
+// wavefronts take 206 registers), so a long context that comes late is walked alone at the end: 64
+// entries of 100 to 2,047 tokens in no order 64.3 us (4.4 TB/s), ranked 55.9 (5.0), of 128 to 4,096
+// tokens 117.9 and 99.4 (5.6), 40 entries 50.7 and 41.7; entries of one length, which have nothing to
+// rank, 54.4 and 55.6.  A captured step's contexts are known on the device only, so every wavefront
+// ranks them for itself.  (Workgroups of four wavefronts, two to a unit: 61.1 and 114 us, ranked too.)
+template <int HD, bool FUSED, bool EXTRA, bool RANKED = false>
 __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_kernel(
     AttentionDecodeArgs args) {
   constexpr int NW = decode_waves<HD>();
@@ -159,7 +180,9 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
   const int r = lane % 16, g = lane / 16;
   const int group = a.nq / a.nkv;
   const int item = blockIdx.x, split = blockIdx.y;
-  const int entry = item / (a.nkv * ma.head_blocks);
+  Ranked place{item / (a.nkv * ma.head_blocks), 0};
+  if constexpr (RANKED) place = ranked_entry(a.positions, ma.num_tiles, place.entry, lane);
+  const int entry = place.entry;
   const int kvh = (item / ma.head_blocks) % a.nkv;
   const int hb = item % ma.head_blocks;
   const int token = entry;
@@ -178,7 +201,7 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
   const bool prep_wave = FUSED && wave == NW - 1;
   const bool key_wave = adds_new && wave == NW - 2;
   const bool walker = !prep_wave && !key_wave;
-  const int pos_lane = a.positions[token];
+  const int pos_lane = RANKED ? place.pos : a.positions[token];
   bf16x8 kq[KS];            // the head vector such a wave prepares: query rows, or the new key
   f32x4 cs[KS][4];          // cos (2 x 4) and sin (2 x 4) of the lane's elements
   f32x4 pw[KS][2];          // norm weight
@@ -431,7 +454,7 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
 
 int launch_attention_merge(const AttentionMfmaArgs& args, hipStream_t stream);
 
-template <int HD, bool EXTRA>
+template <int HD, bool EXTRA, bool RANKED = false>
 static int launch_decode(const AttentionDecodeArgs& args, hipStream_t stream) {
   const AttentionMfmaArgs& m = args.m;
   const int items = m.num_tiles * m.base.nkv * m.head_blocks;
@@ -440,7 +463,7 @@ static int launch_decode(const AttentionDecodeArgs& args, hipStream_t stream) {
   const size_t lds = (size_t)decode_waves<HD>() * (kWave * 2 * 4 + (HD / 16) * kWave * 16);
   if (args.qkv) {
     if constexpr (HD % 32 == 0) {
-      auto kernel = attention_decode_kernel<HD, true, EXTRA>;
+      auto kernel = attention_decode_kernel<HD, true, EXTRA, RANKED>;
       static bool raised = false;     // per head size
       if (lds > 48 * 1024 && !raised) {
         if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
