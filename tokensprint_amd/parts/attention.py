@@ -12,7 +12,7 @@ from __future__ import annotations
 
 import torch
 
-from tokensprint_amd.kernels.stream import PreparedRows, StreamProducts, fused_rmsnorm_of
+from tokensprint_amd.kernels.stream import NormHint, PreparedRows, StreamProducts, fused_rmsnorm_of
 from tokensprint_amd.parts.base import MIXERS, Mixer, PagedKVNeed, TensorDecl, register
 
 
@@ -80,34 +80,42 @@ class GroupedQueryAttention(StreamProducts, Mixer):
         fused = fused_rmsnorm_of(norm)
         if fused is None:
             return super().forward_from_stream(resid, delta, norm, batch, cache, write_cache)
-        o = self._attend_prepared(resid, delta, fused, batch, cache, write_cache)
+        o = None
+        if isinstance(delta, PreparedRows) and delta.tiled:
+            o, prepared = self._attend_prepared(resid, delta, fused, batch, cache, write_cache, hint)
+            if prepared is not None:
+                return prepared, resid
         if o is None:
             qkv, resid = self.ops.norm_linear(resid, delta, fused[0], fused[1], self.w_qkv,
                                               self.ctx.dtype)
             o = self._attend(qkv, batch, cache, write_cache)
         return self.last_product(o, self.w_o, resid, hint), resid
 
-    def _attend_prepared(self, resid, delta, norm, batch, cache, write_cache):
-        """The projection of rows that the product before has prepared, and what `_attend` makes of
-        it, where the provider has the projection and the heads' preparation in one kernel; else
-        None, and nothing has been done."""
-        if not isinstance(delta, PreparedRows) or cache is None or not write_cache \
-                or not self.own_kv or not hasattr(self.ops, "norm_heads"):
-            return None
+    def _attend_prepared(self, resid, delta, norm, batch, cache, write_cache, hint):
+        """(What `_attend` makes of the projection of rows that a prompt's product has prepared, None),
+        where the provider has the projection and the heads' preparation in one kernel; (None, the
+        rows prepared for `hint`) where it does the whole sub-layer in one call; else (None, None),
+        and nothing has been done."""
+        ops = self.ops
+        if cache is None or not write_cache or not self.own_kv or not hasattr(ops, "norm_heads"):
+            return None, None
         tables = self.position.rotary_tables() if self.position is not None else None
         if self.position is not None and tables is None:
-            return None
+            return None, None
         table = batch.tables[cache.group]
-        q = self.ops.norm_heads(
-            resid, delta, norm[0], norm[1], self.w_qkv, batch, table, cache, num_heads=self.nq,
-            num_kv_heads=self.nkv, head_dim=self.hd, q_weight=self.w_qnorm, k_weight=self.w_knorm,
-            head_eps=self.eps, cos_sin=tables)
+        args = (resid, delta, norm[0], norm[1], self.w_qkv, batch, table, cache)
+        heads = dict(num_heads=self.nq, num_kv_heads=self.nkv, head_dim=self.hd)
+        scores = dict(scale=self.scale, window=self.window, sink=self.sink, **self.score_options)
+        kinds = dict(q_weight=self.w_qnorm, k_weight=self.w_knorm, head_eps=self.eps, cos_sin=tables)
+        if isinstance(hint, NormHint):
+            prepared = ops.attend_into_stream(*args, self.w_o, hint, **heads, **kinds, **scores)
+            if prepared is not None:
+                return None, prepared
+        q = ops.norm_heads(*args, **heads, **kinds)
         if q is None:
-            return None
-        o = self.ops.paged_attention(q, batch, table, cache, num_heads=self.nq,
-                                     num_kv_heads=self.nkv, head_dim=self.hd, scale=self.scale,
-                                     window=self.window, sink=self.sink, **self.score_options)
-        return o.view(q.shape[0], self.nq * self.hd)
+            return None, None
+        o = ops.paged_attention(q, batch, table, cache, **heads, **scores)
+        return o.view(q.shape[0], self.nq * self.hd), None
 
     def forward(self, h, batch, cache, write_cache):
         o = self._attend(self.ops.linear(h, self.w_qkv, self.ctx.dtype), batch, cache, write_cache)

@@ -9,7 +9,7 @@ from __future__ import annotations
 
 import torch
 
-from tokensprint_amd.kernels.stream import StreamProducts, fused_rmsnorm_of
+from tokensprint_amd.kernels.stream import NormHint, PreparedRows, StreamProducts, fused_rmsnorm_of
 from tokensprint_amd.parts.base import FEED_FORWARDS, FeedForward, TensorDecl, register
 
 
@@ -61,6 +61,12 @@ class SwiGLU(StreamProducts, FeedForward):
         fused = fused_rmsnorm_of(norm)
         if fused is None or self.form:
             return super().forward_from_stream(resid, delta, norm, batch)
+        if isinstance(delta, PreparedRows) and isinstance(hint, NormHint) \
+                and hasattr(self.ops, "feed_into_stream"):
+            prepared = self.ops.feed_into_stream(resid, delta, fused[0], fused[1], self.w_gate_up,
+                                                 self.w_down, hint)
+            if prepared is not None:
+                return prepared, resid
         act, resid = self.ops.norm_linear(resid, delta, fused[0], fused[1], self.w_gate_up,
                                           self.ctx.dtype, silu_mul=True)
         return self.last_product(act, self.w_down, resid, hint), resid
