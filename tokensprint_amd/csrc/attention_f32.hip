@@ -3,7 +3,7 @@
 // of a multiple of 16 keys; what else there is goes to attention_generic.hip.
 //
 // A workgroup takes a tile of 16 rows (tokens of one entry x the query heads of a key/value head);
-// its eight wavefronts take every eighth block of 64 keys, counted from position 0, and their
+// its eight wavefronts take every eighth block of 16 keys, counted from position 0, and their
 // results are merged in wavefront order.  So what a row adds up, and in which order, depends on
 // its position and window alone, however the step was cut or batched.
 //
@@ -13,10 +13,20 @@
 // passes through LDS but the merge.  Keys and values come straight from their pages, 16 bytes a
 // lane (values lie transposed in a page).
 //
-// What bounds it: at a prompt of 501 tokens (16 heads over 8, 128 wide) 1.1 GFLOP of useful
-// products, 7 us at the float32 matrix rate, and a wavefront's chain of loads and products for
-// each of its blocks.  The kernel before it, a workgroup per token and head with a key a lane,
-// read every key row 32 times as 16-byte pieces 512 bytes apart.
+// A wavefront asks for a block's values before its scores and for the next block's keys behind them,
+// in the registers of the keys that the scores have used: 16 loads are under way beneath each of its
+// two products.  Blocks of 64 keys, all loaded and then waited for, left half of the wavefronts of a
+// prompt of 501 tokens without a block.  Blocks of 32 in this form spill.
+//
+// The tiles of all heads lie one behind the other in the grid, heads fastest: the longest tiles of every
+// head begin first, and with eight heads an XCD has one head's pages in its cache.
+//
+// What bounds it: at a prompt of 501 tokens (16 heads over 8, 128 wide) 1.1 GFLOP of useful products, 7 us
+// at the float32 matrix rate, and two wavefronts a SIMD (registers) whose products wait for the scores'
+// maximum and their loads.  Measured, blocks of 64 -> here: 501 tokens 43.5 -> 29.6 us, 2,048 tokens
+// 305 -> 245, 32 heads 68.5 -> 54.8, 64 single tokens over 100 to 1,990 positions 148 -> 112, one over
+// 501 21.4 -> 18.5.  Error against float64 (relative, 501 tokens): 3.1e-7 -> 2.0e-7; two chains of
+// products make a score.
 #include "attention_mfma.h"
 #include <type_traits>
 
@@ -25,7 +35,8 @@ int ts_check_attention_args(const AttentionArgs& a, const char* who);
 namespace {
 
 constexpr int kWaves = 8;
-constexpr int kBlock = 64;                 // keys of a block
+constexpr int kBlock = 16;                 // keys of a block
+constexpr int kGridTiles = 32768;          // tiles in the grid's second dimension
 
 __device__ __forceinline__ f32x4 read4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 __device__ __forceinline__ f32x4 mfma4(f32x4 a, f32x4 b, f32x4 c) {
@@ -43,7 +54,8 @@ __global__ __launch_bounds__(kWaves* kWave) void attention_f32_kernel(AttentionM
   float* m_s = o_s + kWaves * 16 * LD;                // [kWaves][16]
   float* l_s = m_s + kWaves * 16;                     // [kWaves][16]
   const AttentionArgs& a = m.base;
-  const int tile = blockIdx.x, kvh = blockIdx.y, group = m.rows_per_token;
+  const int tile = blockIdx.z * kGridTiles + blockIdx.y, kvh = blockIdx.x, group = m.rows_per_token;
+  if (tile >= m.num_tiles) return;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
   const int l = lane % 16, g = lane / 16, P = a.page_size;
   const int entry = m.tiles ? m.tiles[3 * tile] : tile;
@@ -70,51 +82,39 @@ __global__ __launch_bounds__(kWaves* kWave) void attention_f32_kernel(AttentionM
 #pragma unroll
     for (int j = 0; j < NT; ++j) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
     top = -INFINITY, sum = 0.f;
-    int b = begin / kBlock;
-    b += (w - b) & (kWaves - 1);             // the first block of this wavefront's
-    for (; b * kBlock <= last; b += kWaves) {
-      // (every load is made, from page 0 where there is none: what it brings is not used)
-      int64_t row[4];                        // of the block's four tiles of 16 keys: their page
-      bool have[4];
+    f32x4 kf[NT], vf[NT], s;
+    int page;                                // of the block whose keys are loaded or under way
+    bool have;                               // whether the block that has scores has a page
+    // (every load is made, from page 0 where there is none: what it brings is not used)
+    auto place = [&] { return ((int64_t)max(page, 0) * a.nkv + kvh) * P * HD; };
+    auto load_keys = [&](int b) {            // b * kBlock <= last
+      page = __builtin_amdgcn_readfirstlane(table[b * kBlock / P]);
+      const float* k = (const float*)a.k_pages + place() + (int64_t)(b * kBlock % P + l) * HD + 4 * g;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int key = b * kBlock + 16 * t;
-        const int page = __builtin_amdgcn_readfirstlane(table[min(key, last) / P]);
-        have[t] = key <= last && page >= 0;
-        row[t] = ((int64_t)max(page, 0) * a.nkv + kvh) * P * HD;
-      }
-      f32x4 kf[4][NT], vf[4][NT], s[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const float* k = (const float*)a.k_pages + row[t] + (int64_t)((b * kBlock + 16 * t) % P + l) * HD + 4 * g;
-#pragma unroll
-        for (int j = 0; j < NT; ++j) kf[t][j] = read4(k + 16 * j);
-      }
+      for (int j = 0; j < NT; ++j) kf[j] = read4(k + 16 * j);
       __builtin_amdgcn_sched_barrier(0);
+    };
+    auto score = [&](int b) {
+      have = page >= 0;
+      const float* v = (const float*)a.v_pages + place() + (int64_t)l * P + b * kBlock % P + 4 * g;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < NT; ++j) s[t] = mfma4(kf[t][j], qf[j], s[t]);
-      }
-      __builtin_amdgcn_sched_barrier(0);     // (the values in the keys' registers)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const float* v = (const float*)a.v_pages + row[t] + (int64_t)l * P + (b * kBlock + 16 * t) % P + 4 * g;
-#pragma unroll
-        for (int c = 0; c < NT; ++c) vf[t][c] = read4(v + (int64_t)16 * c * P);
-      }
+      for (int c = 0; c < NT; ++c) vf[c] = read4(v + (int64_t)16 * c * P);
       __builtin_amdgcn_sched_barrier(0);
+      f32x4 chain[2] = {};
+#pragma unroll
+      for (int j = 0; j < NT; ++j) chain[j & 1] = mfma4(kf[j], qf[j], chain[j & 1]);
+      s = chain[0] + chain[1];
+      __builtin_amdgcn_sched_barrier(0);     // (the next keys in these keys' registers)
+    };
+    auto add = [&](int b) {
+      const int key = b * kBlock + 4 * g;    // of s[0]
       float high = top;
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int key = b * kBlock + 16 * t + 4 * g + r;
-          const float v = EXTRAS ? extra_score(x, s[t][r], key) : s[t][r] * a.scale;
-          s[t][r] = have[t] && mine && key <= pos && key >= from ? v : -INFINITY;
-          high = fmaxf(high, s[t][r]);
-        }
+      for (int r = 0; r < 4; ++r) {
+        const float v = EXTRAS ? extra_score(x, s[r], key + r) : s[r] * a.scale;
+        s[r] = have && mine && key + r <= pos && key + r >= from ? v : -INFINITY;
+        high = fmaxf(high, s[r]);
+      }
       high = fmaxf(high, __shfl_xor(high, 16, kWave));
       high = fmaxf(high, __shfl_xor(high, 32, kWave));
       // (`high` stays -inf only while the row has seen no key: zeros are kept)
@@ -122,48 +122,55 @@ __global__ __launch_bounds__(kWaves* kWave) void attention_f32_kernel(AttentionM
       top = high;
       sum *= fall;
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          s[t][r] = s[t][r] == -INFINITY ? 0.f : expf(s[t][r] - high);
-          sum += s[t][r];
-        }
+      for (int r = 0; r < 4; ++r) {
+        s[r] = s[r] == -INFINITY ? 0.f : expf(s[r] - high);
+        sum += s[r];
+      }
 #pragma unroll
       for (int c = 0; c < NT; ++c) o[c] *= fall;
+      // (a page's places behind the last key hold anything; selects: as a branch for the last block
+      // alone it became a branch for each register of every block)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int key = b * kBlock + 16 * t;
-        if (!have[t] || key + 15 > last) {   // a page's places behind the last key hold anything
+      for (int r = 0; r < 4; ++r) {
+        const bool there = have && key + r <= last;
+#pragma unroll
+        for (int c = 0; c < NT; ++c) vf[c][r] = there ? vf[c][r] : 0.f;
+      }
+      if constexpr (APART) {
+#pragma unroll 1
+        for (int row = 0; row < tokens * group; ++row) {
+          const int to = __shfl(pos, row, kWave), lo = __shfl(from, row, kWave);
+#pragma unroll
+          for (int c = 0; c < NT; ++c) {
+            f32x4 sums = o[c];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const bool sees = key + r <= to && key + r >= lo;
+              sums = __builtin_amdgcn_mfma_f32_16x16x4f32(sees ? vf[c][r] : 0.f, s[r], sums, 0, 0, 0);
+            }
+            if (l == row) o[c] = sums;
+          }
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
 #pragma unroll
           for (int c = 0; c < NT; ++c)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (!have[t] || key + 4 * g + r > last) vf[t][c][r] = 0.f;
-        }
-        if constexpr (APART) {
-#pragma unroll 1
-          for (int row = 0; row < tokens * group; ++row) {
-            const int to = __shfl(pos, row, kWave), lo = __shfl(from, row, kWave);
-#pragma unroll
-            for (int c = 0; c < NT; ++c) {
-              f32x4 sums = o[c];
-#pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                const bool sees = key + 4 * g + r <= to && key + 4 * g + r >= lo;
-                sums = __builtin_amdgcn_mfma_f32_16x16x4f32(sees ? vf[t][c][r] : 0.f, s[t][r], sums, 0, 0, 0);
-              }
-              if (l == row) o[c] = sums;
-            }
-          }
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int c = 0; c < NT; ++c)
-              o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][c][r], s[t][r], o[c], 0, 0, 0);
-        }
+            o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[c][r], s[r], o[c], 0, 0, 0);
       }
+    };
+    int b = begin / kBlock;
+    b += (w - b) & (kWaves - 1);             // the first block of this wavefront's
+    if (b * kBlock > last) return;
+    load_keys(b);
+#pragma unroll 1
+    for (; (b + kWaves) * kBlock <= last; b += kWaves) {
+      score(b);
+      load_keys(b + kWaves);
+      add(b);
     }
+    score(b);
+    add(b);
   };
   walk(std::false_type{});
   // (a value of that kind leaves NaN in every row that meets it, whatever comes behind)
@@ -214,7 +221,8 @@ int launch(const AttentionMfmaArgs& m, hipStream_t stream) {
   if (lds > 64 * 1024 &&
       hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return -1;
-  const dim3 grid(m.num_tiles, m.base.nkv), block(kWaves * kWave);
+  const dim3 grid(m.base.nkv, min(m.num_tiles, kGridTiles), (m.num_tiles + kGridTiles - 1) / kGridTiles);
+  const dim3 block(kWaves * kWave);
   if (extras) hipLaunchKernelGGL((attention_f32_kernel<NT, true>), grid, block, lds, stream, m);
   else hipLaunchKernelGGL((attention_f32_kernel<NT, false>), grid, block, lds, stream, m);
   return 0;
