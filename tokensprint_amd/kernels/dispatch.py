@@ -100,9 +100,9 @@ class Dispatch:
     #: Weights of `tiled_stream_few_weight` to `large_weight` elements take it from fewer rows in
     #: an eager step (captured ones, of up to 256 single tokens, do not: 4.99 against 4.77 ms), where
     #: two norm kernels and three library calls a layer hold the host up: a step of the 0.6B shape
-    #: with 300 tokens 3,400 -> 2,050 us (2,117 -> 2,042 on the GPU), with 128 3,400 -> 2,150 (1,738 ->
-    #: 2,116 on the GPU: N = 1,024 fills few units).  Fewer rows leave nearly half of a tile of 128
-    #: empty.  The lower line of weights is none of speed: below it the forms are ahead as well
+    #: with 300 tokens 3,400 -> 2,050 us when it had tiles of 128 rows only (N = 1,024 fills few units
+    #: with them), 1,740 with tiles of 64 and a sub-layer a call.  Fewer rows were measured in
+    #: tiles of 128, nearly half empty.  The lower line of weights is none of speed: below it the forms are ahead as well
     #: (products and norms of a layer of hidden size 512, 72 to 511 rows, 76 -> 35 us eager and 30 to 33
     #: -> 27 to 31 on the GPU), but portions below 512 rows of such models have had the separate kernels,
     #: and their sums in another order, all along.
