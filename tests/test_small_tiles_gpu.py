@@ -6,6 +6,7 @@ import torch
 
 from tokensprint_amd.kernels import load_hip_ops
 from tokensprint_amd.kernels.hip_ops import _ptr
+from tokensprint_amd.kernels.stream import NormHint
 
 pytestmark = pytest.mark.gpu
 TILES = (6, 7, 8)
@@ -111,3 +112,24 @@ def test_output_heads_of_few_rows(gpu_device, M, K):
 def _f(value):
     from ctypes import c_float
     return c_float(value)
+
+
+@pytest.mark.parametrize("T", [16, 17, 64])
+def test_prepared_rows_by_kind_of_step(gpu_device, monkeypatch, T):
+    """Steps that are captured, or run to be, take the tiled kernel from 17 rows; others do not.  Both sums
+    are of the same products, 1,024 of about 0.05 a piece, in bfloat16."""
+    ops, K, N = load_hip_ops(gpu_device), 1024, 1536
+    x, w, norm_w = (torch.randn(s, generator=torch.Generator().manual_seed(i)).to(gpu_device)
+                    for i, s in enumerate([(T, 512), (K, 512), (K,)]))
+    w2 = (0.05 * torch.randn(N, K, generator=torch.Generator().manual_seed(4))).to(gpu_device, torch.bfloat16)
+    hint, called, results = NormHint(norm_w, 1e-6, w2), [], []
+    call = type(ops)._call
+    monkeypatch.setattr(type(ops), "_call", lambda self, fn, *a: (called.append(fn.__name__), call(self, fn, *a))[1])
+    for timed in (False, True):
+        monkeypatch.setattr(ops, "_timed_plans", timed)
+        resid = torch.zeros(T, K, device=gpu_device)
+        delta = ops.linear_into_stream(x.bfloat16(), w.bfloat16(), resid, hint)
+        results.append(ops.norm_linear(resid, delta, norm_w, 1e-6, w2, torch.bfloat16)[0].float())
+    assert called.count("ts_gemm_tiled_scaled_rows_bf16") == (T >= 17)
+    # float32 sums of 1,024 terms in two orders, then one rounding to bfloat16 each
+    assert (results[0] - results[1]).abs().max() <= 2 ** -7 * results[0].abs().max()

@@ -16,7 +16,7 @@ from dataclasses import dataclass
 @dataclass(frozen=True)
 class Dispatch:
     # ---- the product behind a norm whose rows the weight-streaming kernel in front has prepared: the
-    # same kernels', or from `tiled_scaled_rows` rows the LDS-tiled kernel's in tiles of 64 rows, whose
+    # same kernels', or in captured steps from `tiled_scaled_rows` rows the LDS-tiled kernel's in tiles of 64 rows, whose
     # workgroups read the rows once in 32 or 64 columns, not in 16.  Here and there, us, weights from
     # memory: 4,096 x 1,024 17 rows 5.2 / 5.5, 32 rows 6.0 / 5.5, 64 rows 8.3 / 5.8; 1,536 x 1,024 5.4 / 5.4, 6.3 /
     # 5.4, 8.2 / 5.6; gate/up 2 x 3,072 x 1,024 16 rows 6.8 / 6.8, 17 rows 9.0 / 6.8, 64 rows 12.4 / 7.4.  One line

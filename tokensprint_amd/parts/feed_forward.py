@@ -61,7 +61,7 @@ class SwiGLU(StreamProducts, FeedForward):
         fused = fused_rmsnorm_of(norm)
         if fused is None or self.form:
             return super().forward_from_stream(resid, delta, norm, batch)
-        if isinstance(delta, PreparedRows) and isinstance(hint, NormHint) \
+        if isinstance(delta, PreparedRows) and delta.tiled and isinstance(hint, NormHint) \
                 and hasattr(self.ops, "feed_into_stream"):
             prepared = self.ops.feed_into_stream(resid, delta, fused[0], fused[1], self.w_gate_up,
                                                  self.w_down, hint)
