@@ -187,7 +187,7 @@ def test_low_rank_pairs_that_are_two_products(monkeypatch, T, n_a, k_a, n_g, k_g
     """Long ranks and many rows are left to the products of their own, which share operands out."""
     ops = load_hip_ops("cuda:0")
     taken, linear = [], ops.linear
-    monkeypatch.setattr(ops, "linear", lambda x, w, t: taken.append(w) or linear(x, w, t))
+    monkeypatch.setitem(vars(ops), "linear", lambda x, w, t: taken.append(w) or linear(x, w, t))
     x = rand((T, k_a + k_g), 92)
     w_a, w_g = (rand((n, k), 93, 0.1).to(torch.bfloat16) for n, k in ((n_a, k_a), (n_g, k_g)))
     z, gate = ops.low_rank_pair(x, 0, w_a, k_a, w_g, torch.bfloat16)

@@ -114,6 +114,14 @@ def _f(value):
     return c_float(value)
 
 
+def calls_of(ops, monkeypatch):
+    """The names of the library's functions that `ops` calls from now on, in order.  (In the provider's
+    own dict, which loses the entry again: all tests share the provider.)"""
+    called, call = [], ops._call
+    monkeypatch.setitem(vars(ops), "_call", lambda fn, *args: (called.append(fn.__name__), call(fn, *args))[1])
+    return called
+
+
 @pytest.mark.parametrize("T", [16, 17, 64])
 def test_prepared_rows_by_kind_of_step(gpu_device, monkeypatch, T):
     """Steps that are captured, or run to be, take the tiled kernel from 17 rows; others do not.  Both sums
@@ -122,14 +130,13 @@ def test_prepared_rows_by_kind_of_step(gpu_device, monkeypatch, T):
     x, w, norm_w = (torch.randn(s, generator=torch.Generator().manual_seed(i)).to(gpu_device)
                     for i, s in enumerate([(T, 512), (K, 512), (K,)]))
     w2 = (0.05 * torch.randn(N, K, generator=torch.Generator().manual_seed(4))).to(gpu_device, torch.bfloat16)
-    hint, called, results = NormHint(norm_w, 1e-6, w2), [], []
-    call = type(ops)._call
-    monkeypatch.setattr(type(ops), "_call", lambda self, fn, *a: (called.append(fn.__name__), call(self, fn, *a))[1])
+    hint, called, results = NormHint(norm_w, 1e-6, w2), calls_of(ops, monkeypatch), []
     for timed in (False, True):
         monkeypatch.setattr(ops, "_timed_plans", timed)
         resid = torch.zeros(T, K, device=gpu_device)
         delta = ops.linear_into_stream(x.bfloat16(), w.bfloat16(), resid, hint)
         results.append(ops.norm_linear(resid, delta, norm_w, 1e-6, w2, torch.bfloat16)[0].float())
-    assert called.count("ts_gemm_tiled_scaled_rows_bf16") == (T >= 17)
+    captured = "ts_gemm_tiled_scaled_rows_bf16" if T >= 17 else "ts_gemm_scaled_bf16"
+    assert called == ["ts_gemm_tail_bf16", "ts_gemm_scaled_bf16", "ts_gemm_tail_bf16", captured]
     # float32 sums of 1,024 terms in two orders, then one rounding to bfloat16 each
     assert (results[0] - results[1]).abs().max() <= 2 ** -7 * results[0].abs().max()
