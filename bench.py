@@ -113,7 +113,7 @@ def decode_run(engine, batch, prompt_len, steps, warmup, vocab, max_tokens):
 
 
 PRODUCTS = ("linear", "norm_linear", "linear_into_stream", "linear_silu_mul")
-ATTENTION = ("attend", "paged_attention")
+ATTENTION = ("attend", "paged_attention", "norm_heads", "attend_into_stream")
 
 
 class Without:
@@ -141,6 +141,9 @@ class Without:
             def paged_attention(q, *args, **kw):
                 return block(q.shape, q.dtype)
             ops.attend, ops.paged_attention = attend, paged_attention
+            # (a prompt's sub-layer as one call, and its projection with the heads' preparation in
+            # the epilogue: not these ways, so that the calls above are the ones made)
+            ops.norm_heads = ops.attend_into_stream = lambda *a, **k: None
         else:
             def linear(x, weight, out_dtype):
                 return block((x.shape[0], weight.shape[0]), out_dtype)
@@ -206,6 +209,16 @@ def step_split(model, page, entries_of, max_len):
         no_products = captured_seconds(runner, batch)
     batch.plans.clear()
     return whole, whole - no_products, whole - no_attention
+
+
+def tflops(flops, seconds, peak):
+    """The rate in TFLOP/s, or None if it is above the `peak` (FLOP/s) or no time is left over:
+    then what was taken out of the step was not what the rate is of."""
+    if seconds <= 0 or flops / seconds > peak:
+        print(f"a rate of {flops:.3g} operations in {seconds:.3g} s is none of this card's: left out",
+              file=sys.stderr)
+        return None
+    return round(flops / seconds / 1e12, 1)
 
 
 def decode_entries(batch, context):
@@ -799,9 +812,9 @@ def main() -> int:
                           "frac": round(flops / sec / peak, 4)}
         attn_flops = layers * prefill_attention_flops(raw, T)
         _, t_products, t_attention = step_split(model, page, prefill_entries(T), ctx_len)
-        out["prefill"]["products_tflops"] = round((flops - attn_flops) / t_products / 1e12, 1)
+        out["prefill"]["products_tflops"] = tflops(flops - attn_flops, t_products, peak)
         out["prefill"]["products_us"] = round(t_products * 1e6, 1)
-        out["prefill"]["attention_tflops"] = round(attn_flops / t_attention / 1e12, 1)
+        out["prefill"]["attention_tflops"] = tflops(attn_flops, t_attention, peak)
         out["prefill"]["attention_us"] = round(t_attention * 1e6, 1)
         del pre_engine
         torch.cuda.empty_cache()

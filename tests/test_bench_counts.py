@@ -153,3 +153,9 @@ def test_sisepel_and_palelix_are_compared_at_equal_size():
         assert {"softcap", "mask", "rot"} <= set(left) and sise["token_side"]
         other = next(e["mixer"] for e in pale["layers"] if e["type"] == "lightning")
         assert [right[k] for k in ("heads", "dim", "vdim")] == [other[k] for k in ("heads", "dim", "vdim")]
+
+
+def test_a_rate_above_the_peak_is_left_out(capsys):
+    assert bench.tflops(1e12, 1e-3, 2.5e15) == 1000.0 and not capsys.readouterr().err
+    assert bench.tflops(1e12, 1e-4, 2.5e15) is None and bench.tflops(1e12, -1e-6, 2.5e15) is None
+    assert capsys.readouterr().err.count("left out") == 2
