@@ -77,12 +77,20 @@ def test_tail_and_scaled(gpu_device, M, N, K):
         assert torch.equal(got, want)
 
 
+def calls_of(ops, monkeypatch):
+    """The names of the library's functions that `ops` calls from now on, in order.  (In the provider's
+    own dict, which loses the entry again: all tests share the provider.)"""
+    called, call = [], ops._call
+    monkeypatch.setitem(vars(ops), "_call", lambda fn, *args: (called.append(fn.__name__), call(fn, *args))[1])
+    return called
+
+
 @pytest.mark.parametrize("M", [16, 17, 33, 64])
 @pytest.mark.parametrize("N, silu_mul", [(1040, False), (1024, True)])
-def test_rows_of_the_weight_streaming_tail(gpu_device, M, N, silu_mul):
-    """linear_into_stream and norm_linear at the rows where the second changes its kernel, against
-    float64: two roundings to bfloat16 of operands, and of the results."""
-    from tokensprint_amd.kernels.stream import NormHint
+@pytest.mark.parametrize("captured", [False, True])
+def test_rows_of_the_weight_streaming_tail(gpu_device, monkeypatch, captured, M, N, silu_mul):
+    """linear_into_stream and norm_linear at the rows where the second changes its kernel (in steps that
+    are captured, or run to be), against float64: two roundings to bfloat16 of operands, and of the results."""
     ops, K, width, eps = load_hip_ops(gpu_device), 2048, 1024, 1e-6
     x, w_o = rand((M, K), 8, gpu_device), rand((width, K), 9, gpu_device)
     resid, norm_w = rand((M, width), 10, gpu_device).float() * 30, (1 + rand((width,), 11, gpu_device)).float()
@@ -92,9 +100,13 @@ def test_rows_of_the_weight_streaming_tail(gpu_device, M, N, silu_mul):
     want_out = normed @ weight.double().T
     if silu_mul:
         want_out = torch.nn.functional.silu(want_out[:, :N]) * want_out[:, N:]
+    monkeypatch.setattr(ops, "_timed_plans", captured)
+    called = calls_of(ops, monkeypatch)
     prepared = ops.linear_into_stream(x, w_o, resid, NormHint(norm_w, eps, weight, silu_mul))
     assert prepared is not None and not prepared.tiled
     out, _ = ops.norm_linear(resid, prepared, norm_w, eps, weight, torch.bfloat16, silu_mul)
+    assert called == ["ts_gemm_tail_bf16", "ts_gemm_tiled_scaled_rows_bf16" if captured and M >= 17
+                      else "ts_gemm_scaled_bf16"]
     assert (out.double() - want_out).norm() <= 1e-2 * want_out.norm()
 
 
@@ -112,14 +124,6 @@ def test_output_heads_of_few_rows(gpu_device, M, K):
 def _f(value):
     from ctypes import c_float
     return c_float(value)
-
-
-def calls_of(ops, monkeypatch):
-    """The names of the library's functions that `ops` calls from now on, in order.  (In the provider's
-    own dict, which loses the entry again: all tests share the provider.)"""
-    called, call = [], ops._call
-    monkeypatch.setitem(vars(ops), "_call", lambda fn, *args: (called.append(fn.__name__), call(fn, *args))[1])
-    return called
 
 
 @pytest.mark.parametrize("T", [16, 17, 64])
