@@ -198,6 +198,85 @@ def test_state_space_scan_in_two_launches(gpu_device, heads, groups, rows, vdim)
     test_state_space_scan_in_chunks(gpu_device, heads, groups, rows, vdim)
 
 
+# (fewer than that at both of SPANS: three; heads that share q and k, 128 rows of S)
+@pytest.mark.parametrize("mode", ["fixed", "per_head_plain", "turned"])
+@pytest.mark.parametrize("vdim", [100, 128])
+def test_linear_recurrence_in_three_launches(gpu_device, mode, vdim):
+    test_linear_recurrence_in_chunks(gpu_device, mode, 2, 1, 128, vdim)
+
+
+def test_state_space_scan_in_three_launches(gpu_device):
+    test_state_space_scan_in_chunks(gpu_device, 4, 2, 128, 64)
+
+
+def in_two_and_in_three(ops, monkeypatch, state, slot, batch, x, columns, **kw):
+    """The output and the slot's state as a step makes them by itself, and beside a portion of 4,000 tokens
+    (whose length says how many launches it is)."""
+    scratch, make, before, results = [], ops._chunk_scratch, state.clone(), []
+    # (scratch begins as a mark, so that what a form writes can be counted)
+    monkeypatch.setitem(vars(ops), "_chunk_scratch",
+                        lambda *args: scratch.append(make(*args).fill_(-2.0 ** 100)) or scratch[-1])
+    monkeypatch.setattr(ops, "dispatch", dataclasses.replace(ops.dispatch, scan_whole_tokens=16))
+    for longest in (batch.max_q_len, 4000):
+        state.copy_(before)
+        out = ops.linear_recurrence(x, *columns, dataclasses.replace(batch, max_q_len=longest, plans={}),
+                                    state, silu_inputs=False, **kw)
+        results.append((out, state[slot].clone()))
+    two, three = ((s != -2.0 ** 100).sum().item() for s in scratch)
+    assert two != three
+    return results
+
+
+@pytest.mark.parametrize("heads, kv_heads, dim, vdim", [(8, 2, 128, 128), (12, 4, 40, 50), (8, 8, 64, 80)])
+@pytest.mark.parametrize("tokens", [40, 200, 300])
+def test_two_launches_and_three_give_the_same_bits(gpu_device, monkeypatch, tokens, heads, kv_heads, dim, vdim):
+    ops, gen = load_hip_ops(gpu_device), torch.Generator().manual_seed(17)
+    requests = Requests(gpu_device, (heads, dim, vdim), 1)
+    x = torch.randn(2, tokens, 2 * kv_heads * dim + heads * vdim, generator=gen).to(gpu_device)
+    gates = torch.cat([torch.rand(tokens, heads, generator=gen),
+                       torch.rand(tokens, heads, generator=gen) ** 0.1], 1).to(gpu_device)
+    for rows in x:                                         # at position 0, and behind that
+        batch = requests.step([tokens])
+        two, three = in_two_and_in_three(
+            ops, monkeypatch, requests.state, batch.slot_ids[0].item(), batch, rows,
+            (0, kv_heads * dim, 2 * kv_heads * dim), heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim,
+            gates=gates)
+        assert torch.equal(two[0], three[0]) and torch.equal(two[1], three[1])
+        monkeypatch.undo()
+
+
+# 2^24 times four decays whose product in 64 bits, then rounded to 32, hangs on the order (for all tokens
+# but four the decay is 1)
+ROUNDED_APART = {
+    "tokens 1 to 4": [(8455556, 16707183, 16586236, 11763250), (14533896, 15783492, 11605631, 12895099)],
+    "a block each": [(10746809, 12595570, 9500064, 14306753), (11433115, 11517348, 10958803, 13946748),
+                     (14191418, 13858469, 13507899, 10767477), (13046945, 8467980, 9204622, 11222547)]}
+
+
+def test_two_launches_and_three_multiply_decays_in_one_order(gpu_device, monkeypatch):
+    """Every k and q a unit vector and v of one token alone: outputs and state are that token's decays."""
+    ops = load_hip_ops(gpu_device)
+    heads, dim, vdim, tokens = 16, 16, 16, 128
+    gates, v = torch.ones(tokens, 2 * heads), torch.zeros(tokens, heads, vdim)
+    planted = [(place, four, chunk) for place, fours in ROUNDED_APART.items() for four in fours
+               for chunk in (0, 64)]
+    v[0] = 1
+    for h, (place, four, chunk) in enumerate(planted):     # in the chunk of that v, or in the one behind it
+        at = (1, 2, 3, 4) if place == "tokens 1 to 4" else (5, 20, 40, 50)
+        gates[[chunk + t for t in at], heads + h] = torch.tensor(four) / 2.0 ** 24
+    x = torch.cat([torch.eye(1, dim).expand(tokens, dim)] * 2 + [v.view(tokens, -1)], 1).contiguous()
+    requests = Requests(gpu_device, (heads, dim, vdim), 1)
+    batch = requests.step([tokens])
+    two, three = in_two_and_in_three(
+        ops, monkeypatch, requests.state, batch.slot_ids[0].item(), batch, x.to(gpu_device), (0, dim, 2 * dim),
+        heads=heads, kv_heads=1, dim=dim, vdim=vdim, gates=gates.to(gpu_device))
+    assert torch.equal(two[0], three[0]) and torch.equal(two[1], three[1])
+    # and to 32 bits what 64 give: two to four products rounded to 53, one to 24
+    want = torch.cumprod(gates[:, heads:].double(), 0)
+    got = two[0].double().cpu().view(tokens, heads, vdim)[:, :, 0]
+    assert ((got - want).abs() <= 2.0 ** -22 * want).all()
+
+
 @pytest.mark.parametrize("tokens", [16, 17, 63, 64, 65, 128, 129, 192, 193, 209, 272])
 def test_two_launches_at_every_number_of_chunks(gpu_device, tokens):
     """The walk's loops turn by turn: one chunk to five, the last of one tile, of more, whole."""

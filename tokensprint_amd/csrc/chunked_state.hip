@@ -36,7 +36,7 @@
 // brackets the launches as they run in a prompt's step): delta rule, 16 heads of 128 x 128, 592 and
 // 126 us (solve 37, walk 60, output 37); 8 heads of 64 x 128 with a decay per row 469 and 81 (27,
 // 35, 24); fixed decays, 16 heads of 128 x 128, 230 and 78 (local 29, carry 22, output 44); state
-// space, 64 heads of 128 x 64, 386 and 123 (41, 31, 67), in two launches 101 (27, 73).  The short
+// space, 64 heads of 128 x 64, 386 and 123 (41, 31, 67), in two launches 99 (29, 77).  The short
 // chains of product_step and the decays in 64 bits are 1 to 10 us of that.
 //
 // Matrix operands: lane (g, l) = (lane / 16, lane % 16) holds row l of A, column l of B, and rows
@@ -114,7 +114,7 @@ __host__ __device__ inline Parts parts_of(int num_chunks, int heads, int N, int 
 
 // The same for linear forms in two launches.
 struct ScanParts {
-  int64_t q, k, p, d0, scale, end;
+  int64_t q, k, p, d0, scale, whole, end;
 };
 __host__ __device__ inline ScanParts scan_parts_of(int num_chunks, int heads, int kv_heads, int N) {
   const int64_t units = (int64_t)num_chunks * heads, shared = (int64_t)num_chunks * kv_heads;
@@ -124,7 +124,8 @@ __host__ __device__ inline ScanParts scan_parts_of(int num_chunks, int heads, in
   p.p = p.k + shared * kTok * padded_rows(N);              // (q . k) M vs: [10][64][4]
   p.d0 = p.p + units * kTiles * 256;                       // D(t), [64]
   p.scale = p.d0 + units * kTok;                           // M(last, s) vs, [64]
-  p.end = p.scale + units * kTok;
+  p.whole = p.scale + units * kTok;                        // M(last, first) times the first's own
+  p.end = p.whole + units;
   return p;
 }
 
@@ -239,6 +240,20 @@ __device__ __forceinline__ void spread_decays(HeadDecays d, float dec, float vs,
   if (l == 15) d.total()[blk] = (float)p;
 }
 
+// One wavefront, a token of a chunk a lane (dec 1 behind its end): M(last, token), and the chunk's whole
+// decay in lane 0.  Products by doubling, in 64 bits, as above.
+__device__ __forceinline__ float decay_behind(float dec, int lane, float& whole) {
+  double p = dec;                          // from this token through the last
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const double q = __shfl_down(p, o, 64);
+    p *= lane + o < 64 ? q : 1.;
+  }
+  const double behind = __shfl_down(p, 1, 64);
+  whole = (float)p;
+  return (float)(lane < 63 ? behind : 1.);
+}
+
 // M(t, s) times vs(s) for rows t = 4 g + r and column s = l of tile (i, j), j <= i; zero above the
 // diagonal.  Multiplied up in 64 bits and rounded once.
 __device__ __forceinline__ f32x4 tile_decays(HeadDecays d, int i, int j, int l, int g) {
@@ -259,31 +274,6 @@ __device__ __forceinline__ f32x4 tile_decays(HeadDecays d, int i, int j, int l, 
   const f32x4 row = read4(d.pre() + 16 * i + 4 * g);
 #pragma unroll
   for (int r = 0; r < 4; ++r) m[r] = (float)(row[r] * col);
-  return m;
-}
-
-// The same for row t = l and columns s = 4 g + r: a lane's part of the tile as a left operand.
-__device__ __forceinline__ f32x4 tile_decays_left(HeadDecays d, int i, int j, int l, int g) {
-  f32x4 m;
-  const f32x4 vs = read4(d.vs() + 16 * j + 4 * g);
-  if (i == j) {
-    const float* gb = d.g() + 16 * i;
-    double run = 1.;                       // from 4 g + 4 through t, then one more at a time
-#pragma unroll
-    for (int u = 4; u < 16; ++u) run = u > 4 * g + 3 && u <= l ? run * gb[u] : run;
-    const f32x4 own = read4(gb + 4 * g);
-#pragma unroll
-    for (int r = 3; r >= 0; --r) {
-      m[r] = l >= 4 * g + r ? (float)(run * vs[r]) : 0.f;
-      run = l >= 4 * g + r ? run * own[r] : run;
-    }
-    return m;
-  }
-  double row = d.pre()[16 * i + l];
-  for (int b = j + 1; b < i; ++b) row *= d.total()[b];
-  const f32x4 suf = read4(d.suf() + 16 * j + 4 * g);
-#pragma unroll
-  for (int r = 0; r < 4; ++r) m[r] = (float)(row * ((double)suf[r] * vs[r]));
   return m;
 }
 
@@ -471,15 +461,9 @@ __global__ __launch_bounds__(kThreads, 2) void chunk_local_kernel(ChunkedArgs a,
   for (int i = w; i < heads_each; i += 4) {
     float dec = 1.f, vs = 0.f;
     if (lane < c.nt) token_scalars(a, c.first + lane, h0 + i, dec, vs);
-    double p = dec;                        // the product from this token through the last (64 bits:
-#pragma unroll                             // see spread_decays)
-    for (int o = 1; o < 64; o <<= 1) {
-      const double q = __shfl_down(p, o, 64);
-      p *= lane + o < 64 ? q : 1.;
-    }
-    const double behind = __shfl_down(p, 1, 64);
-    scale[i * kTok + lane] = vs * (float)(lane < 63 ? behind : 1.);
-    if (lane == 0) a.scratch[parts.totals + ((int64_t)chunk * a.heads + h0 + i) * NP] = (float)p;
+    float whole;
+    scale[i * kTok + lane] = vs * decay_behind(dec, lane, whole);
+    if (lane == 0) a.scratch[parts.totals + ((int64_t)chunk * a.heads + h0 + i) * NP] = whole;
   }
   stage_rows<NP, FORM>(a, Ks, a.k_col + hk * a.N, c.first, c.nt, c.pos0, true, wide);
   __syncthreads();
@@ -580,6 +564,9 @@ __global__ __launch_bounds__(kThreads) void chunk_carry_kernel(ChunkedArgs a) {
 // state, in the order in which the matrix cores take it: q, k, and (q . k) times the decays; the other
 // walks, with the state in registers, and nothing of it is written but the last.
 // A workgroup of the first takes one chunk and `heads_each` (up to 8) heads that read the same q and k.
+// Decays are multiplied up in the order that the three launches have, and every sum is theirs: the bits
+// are the same.  (In an order of this form's own the first took 28.5 us instead of 29.5 at that size;
+// with the tiles dealt out in turn, two of the diagonal to one wavefront, 32.5.)
 template <int NT, int FORM, int RT>
 __device__ __forceinline__ void prepare_chunk(const ChunkedArgs& a, const ChunkRange& c, int heads_each,
                                               int wide) {
@@ -606,16 +593,20 @@ __device__ __forceinline__ void prepare_chunk(const ChunkedArgs& a, const ChunkR
       spread_decays(d, dec[u], vs[u], lane);
       const int64_t unit = (int64_t)chunk * a.heads + h0 + w + 4 * u;
       a.scratch[parts.d0 + unit * kTok + lane] = d.d0()[lane];
-      a.scratch[parts.scale + unit * kTok + lane] = d.vs()[lane] * d.es()[lane];
+      float whole;
+      a.scratch[parts.scale + unit * kTok + lane] = vs[u] * decay_behind(dec[u], lane, whole);
+      if (lane == 0) a.scratch[parts.whole + unit] = whole;
     }
   }
   __syncthreads();
+  // A wavefront's tiles: one on the diagonal, whose decays take longest, one or two below it (row 4 or
+  // more: none).
+  auto tile_row = [&](int u) { return u == 0 ? w : u == 1 ? min(w + 1, 3) : w < 2 ? w + 2 : 4; };
+  auto tile_col = [&](int u) { return u == 0 ? w : u == 1 ? (w < 2 ? w : w - 1) : 0; };
   f32x4 gram[3];
 #pragma unroll
-  for (int u = 0; u < 3; ++u) {
-    const int t = w + 4 * u, i = tri_row(t), j = t - tri(i, 0);
-    if (t < kTiles && i < RT) gram[u] = gram_tile<NT>(Ks + 16 * j * LD, Qs + 16 * i * LD, l, g);
-  }
+  for (int u = 0; u < 3; ++u)
+    if (tile_row(u) < RT) gram[u] = gram_tile<NT>(Qs + 16 * tile_row(u) * LD, Ks + 16 * tile_col(u) * LD, l, g);
   if (h0 % group == 0) {                  // q and k themselves, by the first workgroup that reads them
     const int64_t unit = (int64_t)chunk * a.kv_heads + hk;
     if (w < RT) {
@@ -636,16 +627,17 @@ __device__ __forceinline__ void prepare_chunk(const ChunkedArgs& a, const ChunkR
   }
   for (int h = 0; h < heads_each; ++h) {
     const HeadDecays d{decays + h * HeadDecays::kFloats};
-    float* to = a.scratch + parts.p + ((int64_t)chunk * a.heads + h0 + h) * kTiles * 256 + lane * 4;
+    // (row 4 g + r and column l of a tile go where a left operand has them: 16 bytes at a time)
+    float* to = a.scratch + parts.p + ((int64_t)chunk * a.heads + h0 + h) * kTiles * 256 +
+                (l / 4 * 16 + 4 * g) * 4 + l % 4;
 #pragma unroll
     for (int u = 0; u < 3; ++u) {
-      const int t = w + 4 * u, i = tri_row(t), j = t - tri(i, 0);
-      if (t < kTiles && i < RT) {
-        const f32x4 m = tile_decays_left(d, i, j, l, g);
-        f32x4 p;
+      const int i = tile_row(u), j = tile_col(u);
+      if (i < RT) {
+        const f32x4 m = tile_decays(d, i, j, l, g);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) p[r] = i > j || l >= 4 * g + r ? gram[u][r] * m[r] : 0.f;
-        write4(to + t * 256, p);
+        for (int r = 0; r < 4; ++r)
+          to[tri(i, j) * 256 + r * 4] = i > j || 4 * g + r >= l ? gram[u][r] * m[r] : 0.f;
       }
     }
   }
@@ -742,7 +734,7 @@ __global__ __launch_bounds__(kScanThreads, 1) void chunk_scan_kernel(ChunkedArgs
 #pragma unroll
       for (int r = 0; r < 4; ++r) f.v[r] = v_col[(int64_t)(q0 + min(c * kTok + first_row + r, tokens - 1)) * a.ld];
       f.scale = read4(a.scratch + parts.scale + unit * kTok + first_row);
-      f.total = a.scratch[parts.d0 + unit * kTok + kTok - 1];
+      f.total = a.scratch[parts.whole + unit];
     };
     auto fetch_k = [&](StateOperands<NT>& f, int c, int o) {
       const float* at = a.scratch + parts.k + shared_of(c) * NT * 1024 + min(w + 4 * o, NT - 1) * 1024;
@@ -1347,7 +1339,8 @@ int launch_output(const ChunkedArgs& a, int heads_each, int wide, hipStream_t st
 // whatever else the chip does, or in three, whose work is spread over it: us in two and three launches,
 // 256 workgroups in the walk (64 heads of 128 x 64) 170 tokens 26 / 35, 1,000 63 / 80, 2,048 98 / 123,
 // 8,192 360 / 464; 128 (16 heads of 128 x 128) 300 tokens 30 / 44, 1,000 55 / 55, 2,048 93 / 84;
-// 64 (16 heads of 64 x 64) 300 tokens 20 / 26, 1,000 39 / 29.  (More rows than 128 do not fit the walk's
+// 64 (16 heads of 64 x 64) 300 tokens 20 / 26, 1,000 39 / 29.  The longest portion of a step decides for
+// all of its requests, whose results do not hang on it: both give the same bits.  (More rows than 128 do not fit the walk's
 // registers; an output's place in a chunk is counted in 32 bits.)
 bool in_two_launches(const ChunkedArgs& a) {
   const int64_t chunks = (a.max_len + kTok - 1) / kTok;
