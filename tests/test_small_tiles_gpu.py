@@ -144,3 +144,20 @@ def test_prepared_rows_by_kind_of_step(gpu_device, monkeypatch, T):
     assert called == ["ts_gemm_tail_bf16", "ts_gemm_scaled_bf16", "ts_gemm_tail_bf16", captured]
     # float32 sums of 1,024 terms in two orders, then one rounding to bfloat16 each
     assert (results[0] - results[1]).abs().max() <= 2 ** -7 * results[0].abs().max()
+
+
+@pytest.mark.parametrize("T", [17, 33, 64])
+def test_float32_rows_are_the_same_in_both_kinds_of_step(gpu_device, monkeypatch, T):
+    """Float32 results keep the weight-streaming kernel, whose sums round less (a third at K = 1,024)."""
+    ops, K, N = load_hip_ops(gpu_device), 1024, 1536
+    x, w, resid = (torch.randn(s, generator=torch.Generator().manual_seed(i)).to(gpu_device)
+                   for i, s in enumerate([(T, 512), (K, 512), (T, K)]))
+    w2, ones = rand((N, K), 4, gpu_device), torch.ones(K, device=gpu_device)
+    hint, called, results = NormHint(ones, 1e-6, w2), calls_of(ops, monkeypatch), []
+    for captured in (False, True):
+        monkeypatch.setattr(ops, "_timed_plans", captured)
+        stream = resid.clone()
+        prepared = ops.linear_into_stream(x.bfloat16(), w.bfloat16(), stream, hint)
+        results.append(ops.norm_linear(stream, prepared, ones, 1e-6, w2, torch.float32)[0])
+    assert called == ["ts_gemm_tail_bf16", "ts_gemm_scaled_bf16"] * 2
+    assert torch.equal(*results)

@@ -23,6 +23,9 @@ class Dispatch:
     # for both, at the rows where a row's sums change their order anyway.  K = 512 gains nothing (1,024
     # columns 3.4 / 4.2, 3.5 / 4.3, 4.7 / 4.4), K = 2,048 as much as it loses (4,096 columns 17 rows 8.9 / 10.7,
     # 33 rows 11.9 / 10.9).
+    # Results that leave in float32 stay with the weight-streaming kernel, whose short runs of K round
+    # less: K = 1,024 1.1e-7 against 3.2e-7 of float64, 1,536 1.2e-7 and 4.3e-7.  In bfloat16 both are off by
+    # its rounding, 1.6556e-3 and 1.6556e-3 (gate/up 3.040e-3 and 3.040e-3); 2 to 4 values in 10,000 differ.
     tiled_scaled_rows: int = 17
     tiled_scaled_k: tuple[int, int] = (1024, 1536)
 

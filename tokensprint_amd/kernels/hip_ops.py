@@ -628,7 +628,7 @@ class HipOps:
         return PreparedRows(rows, sumsq, parts, hint)
 
     def _tiled_scaled_ok(self, M, N, K, silu_mul, slices):
-        """Whether the product of rows that the weight-streaming kernel has prepared is the
+        """Whether the bfloat16 product of rows that the weight-streaming kernel has prepared is the
         LDS-tiled kernel's: in steps that are captured, or run to be (an eager one of so few rows waits
         for the host, and this launch is the longer one there: 25 rows 1.95 against 2.02 to 2.08 ms a
         step)."""
@@ -656,7 +656,8 @@ class HipOps:
         if out_dtype not in (torch.bfloat16, torch.float32) or (silu_mul and out_dtype != torch.bfloat16):
             raise ValueError(f"norm_linear: prepared rows cannot give {out_dtype}")
         out = torch.empty(M, N, dtype=out_dtype, device=self.device)
-        if prepared.tiled or self._tiled_scaled_ok(M, N, K, silu_mul, prepared.slices):
+        if prepared.tiled or out_dtype is torch.bfloat16 \
+                and self._tiled_scaled_ok(M, N, K, silu_mul, prepared.slices):
             self._call(self.lib.ts_gemm_tiled_scaled_bf16 if prepared.tiled
                        else self.lib.ts_gemm_tiled_scaled_rows_bf16, _ptr(prepared.rows),
                        _ptr(prepared.sumsq), prepared.slices, c_float(eps), _ptr(weight),
