@@ -110,15 +110,29 @@ def test_rows_of_the_weight_streaming_tail(gpu_device, monkeypatch, captured, M,
     assert (out.double() - want_out).norm() <= 1e-2 * want_out.norm()
 
 
-@pytest.mark.parametrize("M", [8, 9, 12, 13, 33, 64])
+@pytest.mark.parametrize("M", [8, 9, 12, 16, 17, 33, 64])
 @pytest.mark.parametrize("K", [1024, 2048])
-def test_output_heads_of_few_rows(gpu_device, M, K):
-    """Whichever kernel's: a row's logits against float64, float32 sums of K products."""
+def test_output_heads_of_few_rows(gpu_device, monkeypatch, M, K):
+    """The weight-streaming kernel's up to 8 rows, the library's up to 16, the tiled kernel's from there:
+    float32 sums of K products, and never further from float64 than the library's (which up to 16 rows
+    are shared out over K)."""
     ops = load_hip_ops(gpu_device)
     x, w = rand((M, K), 6, gpu_device), rand((16400, K), 7, gpu_device)
+    called = calls_of(ops, monkeypatch)
     out = ops.linear(x, w, torch.float32)
+    assert called == ["ts_gemm_mfma_bf16" if M <= 8 else "ts_gemm_library_bf16" if M <= 16
+                      else "ts_gemm_tiled_bf16"]
     exact = x.double() @ w.double().T
     assert (out.double() - exact).norm() <= 4e-6 * exact.norm()
+    assert (out.double() - exact).norm() <= 1.1 * (library(ops, x, w).double() - exact).norm()
+
+
+def library(ops, x, w):
+    from ctypes import c_size_t
+    out, space = torch.empty(x.shape[0], w.shape[0], device=x.device), ops._library_workspace
+    ops._call(ops.lib.ts_gemm_library_bf16, _ptr(x), _ptr(w), _ptr(out), 0, x.shape[0], w.shape[0], x.shape[1],
+              _ptr(space), c_size_t(space.numel()), ops._stream())
+    return out
 
 
 def _f(value):

@@ -425,8 +425,7 @@ class HipOps:
         """Whether an output head's product of less than `library_rows` rows is the LDS-tiled
         kernel's."""
         (M, K), d = x.shape, self.dispatch
-        return (M >= (d.tiled_head_rows_short if K <= 1024 else d.tiled_head_rows)
-                and x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16
+        return (M >= d.tiled_head_rows and x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16
                 and out_dtype in (torch.bfloat16, torch.float32)
                 and self.lib.ts_gemm_tiled_fits(M, weight.shape[0], K, 0) == 1)
 
