@@ -127,6 +127,22 @@ def test_output_heads_of_few_rows(gpu_device, monkeypatch, M, K):
     assert (out.double() - exact).norm() <= 1.1 * (library(ops, x, w).double() - exact).norm()
 
 
+@pytest.mark.parametrize("M, N, K, tiled", [
+    (65, 256, 1024, True), (65, 3072, 1024, True), (65, 3072, 1088, False), (128, 1024, 2048, False),
+    (144, 1792, 1088, False), (256, 512, 1536, False), (300, 256, 4096, False), (500, 1024, 1024, True)])
+def test_float32_results_of_small_tiles(gpu_device, monkeypatch, M, N, K, tiled):
+    """Plain products that leave in float32 are no further from float64 than the library's, which shares K out
+    where there are few tiles; in bfloat16 the tiled kernel's in all of these sizes."""
+    ops = load_hip_ops(gpu_device)
+    x, w = rand((M, K), 13, gpu_device), rand((N, K), 14, gpu_device)
+    exact, called = x.double() @ w.double().T, calls_of(ops, monkeypatch)
+    out = ops.linear(x, w, torch.float32)
+    ops.linear(x, w, torch.bfloat16)
+    error, theirs = ((o.double() - exact).norm() for o in (out, library(ops, x, w)))
+    assert error <= 1.05 * theirs
+    assert called[:2] == ["ts_gemm_tiled_bf16" if tiled else "ts_gemm_library_bf16", "ts_gemm_tiled_bf16"]
+
+
 def library(ops, x, w):
     from ctypes import c_size_t
     out, space = torch.empty(x.shape[0], w.shape[0], device=x.device), ops._library_workspace

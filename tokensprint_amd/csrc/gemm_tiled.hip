@@ -50,13 +50,17 @@ extern "C" int ts_gemm_tiled_fill(int M, int N, int K, int pair) {
 // N a multiple of 256 in the small tiles (64 x 64 and 64 x 32), timed at 65 to 1,500 rows of 13 weights (N 512
 // to 9,216): K up to 2,048 0.49 to 0.97, 0.70 in the mean, whatever they fill (against the fastest of the
 // library's first eight algorithms 0.57 to 0.92 at 65 to 600 rows of five of them); K = 4,096 0.80 to 0.94
-// above 256 rows, 1.03 to 1.27 below; K = 8,192 0.90 to 1.38.
+// above 256 rows, 1.03 to 1.27 below; K = 8,192 0.90 to 1.38.  Float32 results only up to K = 1,024: above, the
+// library shares K out where there are few tiles (at 65 to 513 rows of up to 3,072 columns, by no rule of
+// sizes) and is half as far from float64 as one chain of K (K = 2,048 1.3e-7 and 2.7e-7); up to there both
+// are one chain (2,362 sizes).
 extern "C" int ts_gemm_tiled_ahead(int M, int N, int K, int c_type) {
   if (!ts_gemm_tiled_fits(M, N, K, 0)) return 0;
   TiledArgs g{};
   g.M = M, g.N = N, g.K = K;
   const int small = cheapest_tile(g, false);
-  if (N % 256 == 0 && (small == 7 || small == 8)) return K <= 2048 || (K <= 4096 && M > 256);
+  if (N % 256 == 0 && (small == 7 || small == 8) && (c_type == TS_BF16 || K <= 1024))
+    return K <= 2048 || (K <= 4096 && M > 256);
   const int tile = cheapest_tile(g, false, 128), units = compute_units();
   const int fill = ts_gemm_tiled_fill(M, N, K, 0);
   if (N % 256 != 0) {
