@@ -110,21 +110,19 @@ def test_rows_of_the_weight_streaming_tail(gpu_device, monkeypatch, captured, M,
     assert (out.double() - want_out).norm() <= 1e-2 * want_out.norm()
 
 
-@pytest.mark.parametrize("M", [8, 9, 12, 16, 17, 33, 64])
-@pytest.mark.parametrize("K", [1024, 2048])
-def test_output_heads_of_few_rows(gpu_device, monkeypatch, M, K):
-    """The weight-streaming kernel's up to 8 rows, the library's up to 16, the tiled kernel's from there:
-    float32 sums of K products, and never further from float64 than the library's (which up to 16 rows
-    are shared out over K)."""
+@pytest.mark.parametrize("M", [8, 9, 16, 17, 33, 48, 64])
+@pytest.mark.parametrize("N, K", [(16400, 1024), (16400, 2048), (119552, 1088)])
+def test_output_heads_of_few_rows(gpu_device, monkeypatch, M, N, K):
+    """The weight-streaming kernel's up to 8 rows, the library's from there (which shares K out at up to 16 rows,
+    and at some numbers of columns for the last of its tiles): float32 sums of K products."""
     ops = load_hip_ops(gpu_device)
-    x, w = rand((M, K), 6, gpu_device), rand((16400, K), 7, gpu_device)
+    x, w = rand((M, K), 6, gpu_device), rand((N, K), 7, gpu_device)
     called = calls_of(ops, monkeypatch)
     out = ops.linear(x, w, torch.float32)
-    assert called == ["ts_gemm_mfma_bf16" if M <= 8 else "ts_gemm_library_bf16" if M <= 16
-                      else "ts_gemm_tiled_bf16"]
+    assert called == ["ts_gemm_mfma_bf16" if M <= 8 else "ts_gemm_library_bf16"]
     exact = x.double() @ w.double().T
     assert (out.double() - exact).norm() <= 4e-6 * exact.norm()
-    assert (out.double() - exact).norm() <= 1.1 * (library(ops, x, w).double() - exact).norm()
+    assert (out.double() - exact).norm() <= 1.02 * (library(ops, x, w).double() - exact).norm()
 
 
 @pytest.mark.parametrize("M, N, K, tiled", [

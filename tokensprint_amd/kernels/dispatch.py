@@ -47,11 +47,6 @@ class Dispatch:
     #: 5 above 4,096 (K = 5,120 4 rows 0.99, 5 rows 1.01; 8,192 6 rows 0.99, 7 rows 1.01), below as
     #: before (K = 2,048 8 rows 0.95, 9 rows 1.01)
     library_rows_head: int = 9
-    #: and from 17 rows the LDS-tiled kernel's.  Its time of the fastest of the library's first eight
-    #: algorithms, 17 to 64 rows: K = 1,024 0.90 to 0.93, K = 2,048 0.88 to 0.98, K = 4,096 0.87 to 1.00,
-    #: K = 5,120 0.97 to 0.99.  Its sums are as far from float64 as theirs there (0.92 to 1.00 of them); up to
-    #: 16 rows theirs, of K shared out, are half as far (K = 2,048 1.3e-7 against 2.7e-7)
-    tiled_head_rows: int = 17
     library_rows_long_head: int = 7
     library_rows_longest_head: int = 5
     head_columns: int = 16384

@@ -348,8 +348,6 @@ class HipOps:
             # a prompt's portion at small weights: as fast as the library's product on the
             # GPU and a fifth of its cost on the host (which a step's first layer waits for)
             return self.gemm_tiled(x, weight, out_dtype)
-        if not many and N >= d.head_columns and self._tiled_head_ok(x, weight, out_dtype):
-            return self.gemm_tiled(x, weight, out_dtype)
         if many and M >= d.library_rows or self._library_ok(x, weight):
             # the library's float32 sums leave in the type asked for: bfloat16 activations,
             # float32 logits at the output head (not rounded to bfloat16 and widened, so
@@ -420,14 +418,6 @@ class HipOps:
                      or self.lib.ts_gemm_tiled_fill(M, inner, K, 1) >= (
                          d.tiled_fill if weight.numel() <= d.tiled_pair_weight
                          or M <= d.tiled_fill_large_rows else d.tiled_fill_large)))
-
-    def _tiled_head_ok(self, x, weight, out_dtype):
-        """Whether an output head's product of less than `library_rows` rows is the LDS-tiled
-        kernel's."""
-        (M, K), d = x.shape, self.dispatch
-        return (M >= d.tiled_head_rows and x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16
-                and out_dtype in (torch.bfloat16, torch.float32)
-                and self.lib.ts_gemm_tiled_fits(M, weight.shape[0], K, 0) == 1)
 
     def _tiled_plain_ok(self, M, N, K, out_dtype):
         """Whether a bfloat16 product of many rows is the LDS-tiled kernel's."""
