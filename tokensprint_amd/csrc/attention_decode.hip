@@ -63,7 +63,7 @@ extern "C" int ts_attention_decode(const AttentionDecodeArgs* p, hipStream_t str
   }
   // (positions times 64 are ranked in 32 bits)
   const int64_t items = (int64_t)m.num_tiles * a.nkv * m.head_blocks;
-  if (args.qkv && m.num_splits == 1 && m.num_tiles <= 64 && items > 256 &&
+  if (args.qkv && m.num_splits == 1 && m.num_tiles <= 64 && items > compute_units() &&
       (int64_t)a.table_width * a.page_size < 1 << 25) {
     switch (a.hd) {
 #define TS_CASE(HD) case HD: rc = launch_decode<HD, false, true>(args, stream); break;

@@ -763,7 +763,6 @@ void attention_prefill_wide_kernel8(AttentionMfmaArgs args, int paired) {
 // Query tiles per wavefront: as many as the register file holds accumulators for.
 constexpr int tiles_per_wave(int hd) { return hd <= 32 ? 4 : (hd <= 64 ? 2 : 1); }
 
-static int compute_units();
 // Which kernel takes the long portions of head sizes 64 and 128.  2 (the default): turns of
 // 64 keys for few items (two sets of waves per item) and for many (eight tiles an item),
 // turns of 32 keys between; 1: for few items only; 0: turns of 32 keys everywhere; 3: eight
@@ -781,18 +780,6 @@ extern "C" int ts_attention_prefill_tiles(int head_dim, int page_size, int tiles
   const bool wide = g_prefill_variant >= 2 && head_dim % 64 == 0 && head_dim <= 128;
   const int64_t items4 = (int64_t)((tiles16 + 3) / 4) * heads;
   return wide && (g_prefill_variant == 3 || items4 >= 6 * compute_units()) ? 8 : 4;
-}
-
-int compute_units() {
-  static int cus = 0;       // of the device current when first asked; a host's GPUs are alike
-  if (cus == 0) {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    cus = n;
-  }
-  return cus;
 }
 
 template <int HD, int H>

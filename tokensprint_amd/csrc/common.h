@@ -29,6 +29,20 @@ void ts_set_error(const char* fmt, ...);
     if (e_ != hipSuccess) TS_FAIL("%s: launch failed: %s", name, hipGetErrorString(e_)); \
   } while (0)
 
+// Compute units of the current device (256 where it cannot be asked).
+inline int compute_units() {
+  static int units[64] = {};
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return 256;
+  if (units[device] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0)
+      n = 256;
+    units[device] = n;
+  }
+  return units[device];
+}
+
 __device__ __forceinline__ float to_f32(float x) { return x; }
 __device__ __forceinline__ float to_f32(bf16_t x) { return (float)x; }
 template <typename T> __device__ __forceinline__ T from_f32(float x);

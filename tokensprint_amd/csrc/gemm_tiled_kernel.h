@@ -725,20 +725,6 @@ constexpr TileCost kTileCosts[] = {
     {5, 256, 192, 6.6f, 0.931f, 1.1f}, {4, 256, 256, 7.7f, 1.126f, 1.6f},
 };
 
-// Compute units of the current device (256 where it cannot be asked).
-inline int compute_units() {
-  static int units[64] = {};
-  int device = 0;
-  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return 256;
-  if (units[device] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0)
-      n = 256;
-    units[device] = n;
-  }
-  return units[device];
-}
-
 // (`least_rows`: of the tiles with so many rows or more)
 inline int cheapest_tile(const TiledArgs& g, bool pair, int least_rows = 0) {
   const int units = compute_units();

@@ -623,7 +623,7 @@ class HipOps:
         step)."""
         d = self.dispatch
         if M < d.tiled_scaled_rows or not (
-                self._timed_plans or torch._C._cuda_isCurrentStreamCapturing()):
+                self._timed_plans or torch.cuda.is_current_stream_capturing()):
             return False
         key = (M, N, K, silu_mul, slices)
         found = self._routes.get(key) if self._routes_of is d else None
