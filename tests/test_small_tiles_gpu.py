@@ -85,10 +85,10 @@ def calls_of(ops, monkeypatch):
     return called
 
 
-@pytest.mark.parametrize("M", [16, 17, 33, 64])
-@pytest.mark.parametrize("N, silu_mul", [(1040, False), (1024, True)])
+@pytest.mark.parametrize("M", [16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N, silu_mul, rows", [(1040, False, 33), (2048, True, 33), (2064, True, 17)])
 @pytest.mark.parametrize("captured", [False, True])
-def test_rows_of_the_weight_streaming_tail(gpu_device, monkeypatch, captured, M, N, silu_mul):
+def test_rows_of_the_weight_streaming_tail(gpu_device, monkeypatch, captured, M, N, silu_mul, rows):
     """linear_into_stream and norm_linear at the rows where the second changes its kernel (in steps that
     are captured, or run to be), against float64: two roundings to bfloat16 of operands, and of the results."""
     ops, K, width, eps = load_hip_ops(gpu_device), 2048, 1024, 1e-6
@@ -105,7 +105,7 @@ def test_rows_of_the_weight_streaming_tail(gpu_device, monkeypatch, captured, M,
     prepared = ops.linear_into_stream(x, w_o, resid, NormHint(norm_w, eps, weight, silu_mul))
     assert prepared is not None and not prepared.tiled
     out, _ = ops.norm_linear(resid, prepared, norm_w, eps, weight, torch.bfloat16, silu_mul)
-    assert called == ["ts_gemm_tail_bf16", "ts_gemm_tiled_scaled_rows_bf16" if captured and M >= 17
+    assert called == ["ts_gemm_tail_bf16", "ts_gemm_tiled_scaled_rows_bf16" if captured and M >= rows
                       else "ts_gemm_scaled_bf16"]
     assert (out.double() - want_out).norm() <= 1e-2 * want_out.norm()
 
@@ -154,9 +154,9 @@ def _f(value):
     return c_float(value)
 
 
-@pytest.mark.parametrize("T", [16, 17, 64])
+@pytest.mark.parametrize("T", [32, 33, 64])
 def test_prepared_rows_by_kind_of_step(gpu_device, monkeypatch, T):
-    """Steps that are captured, or run to be, take the tiled kernel from 17 rows; others do not.  Both sums
+    """Steps that are captured, or run to be, take the tiled kernel from 33 rows; others do not.  Both sums
     are of the same products, 1,024 of about 0.05 a piece, in bfloat16."""
     ops, K, N = load_hip_ops(gpu_device), 1024, 1536
     x, w, norm_w = (torch.randn(s, generator=torch.Generator().manual_seed(i)).to(gpu_device)
@@ -168,7 +168,7 @@ def test_prepared_rows_by_kind_of_step(gpu_device, monkeypatch, T):
         resid = torch.zeros(T, K, device=gpu_device)
         delta = ops.linear_into_stream(x.bfloat16(), w.bfloat16(), resid, hint)
         results.append(ops.norm_linear(resid, delta, norm_w, 1e-6, w2, torch.bfloat16)[0].float())
-    captured = "ts_gemm_tiled_scaled_rows_bf16" if T >= 17 else "ts_gemm_scaled_bf16"
+    captured = "ts_gemm_tiled_scaled_rows_bf16" if T >= 33 else "ts_gemm_scaled_bf16"
     assert called == ["ts_gemm_tail_bf16", "ts_gemm_scaled_bf16", "ts_gemm_tail_bf16", captured]
     # float32 sums of 1,024 terms in two orders, then one rounding to bfloat16 each
     assert (results[0] - results[1]).abs().max() <= 2 ** -7 * results[0].abs().max()

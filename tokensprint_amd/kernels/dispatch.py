@@ -16,17 +16,23 @@ from dataclasses import dataclass
 @dataclass(frozen=True)
 class Dispatch:
     # ---- the product behind a norm whose rows the weight-streaming kernel in front has prepared: the
-    # same kernels', or in captured steps from `tiled_scaled_rows` rows the LDS-tiled kernel's in tiles of 64 rows, whose
-    # workgroups read the rows once in 32 or 64 columns, not in 16.  Here and there, us, weights from
-    # memory: 4,096 x 1,024 17 rows 5.2 / 5.5, 32 rows 6.0 / 5.5, 64 rows 8.3 / 5.8; 1,536 x 1,024 5.4 / 5.4, 6.3 /
-    # 5.4, 8.2 / 5.6; gate/up 2 x 3,072 x 1,024 16 rows 6.8 / 6.8, 17 rows 9.0 / 6.8, 64 rows 12.4 / 7.4.  One line
-    # for both, at the rows where a row's sums change their order anyway.  K = 512 gains nothing (1,024
-    # columns 3.4 / 4.2, 3.5 / 4.3, 4.7 / 4.4), K = 2,048 as much as it loses (4,096 columns 17 rows 8.9 / 10.7,
-    # 33 rows 11.9 / 10.9).
+    # same kernels', or in captured steps from `tiled_scaled_rows` rows (gate/up products of more than
+    # `tiled_scaled_pair_columns` columns from `tiled_scaled_pair_rows`) the LDS-tiled kernel's in tiles of 64
+    # rows, whose workgroups read the rows once in 32 or 64 columns, not in 16.  The one and the other, us,
+    # weights from memory, launch after launch in a graph, 17, 32 and 48 rows: 3,072 x 1,024 6.5 / 6.9, 7.5 /
+    # 7.1, 9.7 / 7.4; 1,536 x 1,536 6.6 / 9.0, 7.9 / 9.2, 10.3 / 9.5; gate/up 2 x 3,072 x 1,024 9.1 / 7.2,
+    # 10.0 / 7.5, 12.9 / 7.7; 2 x 2,048 x 1,024 6.8 / 7.0, 6.7 / 7.3, 9.9 / 7.4.  Captured steps with the
+    # streaming kernels alone and so: 0.6B 17 rows 1,404 / 1,351, 32 1,535 / 1,461, 33 1,635 / 1,513, 64
+    # 2,078 / 1,911 (the tiled kernel for both from 17 rows on: 1,388 and 1,480); its layers with an inner size of
+    # 2,048 17 rows 1,285 / 1,287 (1,336), 33 1,520 / 1,458.
+    # K = 512 gains nothing (1,024 columns 3.4 / 4.2, 3.5 / 4.3, 4.7 / 4.4), K = 2,048 as much as it loses
+    # (4,096 columns 17 rows 8.9 / 10.7, 33 rows 11.9 / 10.9).
     # Results that leave in float32 stay with the weight-streaming kernel, whose short runs of K round
     # less: K = 1,024 1.1e-7 against 3.2e-7 of float64, 1,536 1.2e-7 and 4.3e-7.  In bfloat16 both are off by
     # its rounding, 1.6556e-3 and 1.6556e-3 (gate/up 3.040e-3 and 3.040e-3); 2 to 4 values in 10,000 differ.
-    tiled_scaled_rows: int = 17
+    tiled_scaled_rows: int = 33
+    tiled_scaled_pair_rows: int = 17
+    tiled_scaled_pair_columns: int = 2048
     tiled_scaled_k: tuple[int, int] = (1024, 1536)
 
     # ---- plain bfloat16 products: from how many rows the vendor library (hipBLASLt)

@@ -622,7 +622,8 @@ class HipOps:
         for the host, and this launch is the longer one there: 25 rows 1.95 against 2.02 to 2.08 ms a
         step)."""
         d = self.dispatch
-        if M < d.tiled_scaled_rows or not (
+        wide = silu_mul and N > d.tiled_scaled_pair_columns
+        if M < (d.tiled_scaled_pair_rows if wide else d.tiled_scaled_rows) or not (
                 self._timed_plans or torch.cuda.is_current_stream_capturing()):
             return False
         key = (M, N, K, silu_mul, slices)
