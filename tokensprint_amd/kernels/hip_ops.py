@@ -160,6 +160,12 @@ class HipOps:
         # the current stream's handle, by the short way: this runs before every kernel
         return c_void_p(self._raw_stream(self._device_index))
 
+    def _captured(self):
+        """Whether the step is captured, or run to be.  (The default stream cannot be captured; asking the
+        runtime takes 1 us, which a step of few rows would spend on every layer.)"""
+        return self._timed_plans or (self._raw_stream(self._device_index) != 0
+                                     and torch.cuda.is_current_stream_capturing())
+
     def _call(self, fn, *args):
         if fn(*args) != 0:
             message = self.lib.ts_last_error().decode()
@@ -480,8 +486,7 @@ class HipOps:
                 return True
         elif N >= d.head_columns and M >= d.library_rows_longest_head:
             rows = d.library_rows_head
-            if K > 2048 and M < rows and (self._timed_plans
-                                          or torch.cuda.is_current_stream_capturing()):
+            if K > 2048 and M < rows and self._captured():
                 rows = d.library_rows_long_head if K <= 4096 else d.library_rows_longest_head
             if M >= rows:
                 return True
@@ -553,7 +558,7 @@ class HipOps:
         wn, d = hint.weight, self.dispatch
         # a step that is captured, or run to be, does not wait for the host
         eager = d.tiled_stream_few_rows <= M < d.tiled_stream_rows \
-            and not (self._timed_plans or torch.cuda.is_current_stream_capturing())
+            and not self._captured()
         key = (M, N, K, wn.shape, hint.silu_mul, eager)
         found = self._routes.get(key) if self._routes_of is d else None
         if found is not None:
@@ -616,15 +621,15 @@ class HipOps:
                    self._stream())
         return PreparedRows(rows, sumsq, parts, hint)
 
-    def _tiled_scaled_ok(self, M, N, K, silu_mul, slices):
-        """Whether the bfloat16 product of rows that the weight-streaming kernel has prepared is the
-        LDS-tiled kernel's: in steps that are captured, or run to be (an eager one of so few rows waits
-        for the host, and this launch is the longer one there: 25 rows 1.95 against 2.02 to 2.08 ms a
-        step)."""
+    def _tiled_scaled_ok(self, M, N, K, silu_mul, slices, out_dtype):
+        """Whether the product of rows that the weight-streaming kernel has prepared is the LDS-tiled
+        kernel's: in steps that are captured, or run to be (an eager one of so few rows waits for the host,
+        and this launch is the longer one there: 25 rows 1.95 against 2.02 to 2.08 ms a step), with results
+        in bfloat16."""
         d = self.dispatch
         wide = silu_mul and N > d.tiled_scaled_pair_columns
-        if M < (d.tiled_scaled_pair_rows if wide else d.tiled_scaled_rows) or not (
-                self._timed_plans or torch.cuda.is_current_stream_capturing()):
+        if out_dtype is not torch.bfloat16 \
+                or M < (d.tiled_scaled_pair_rows if wide else d.tiled_scaled_rows) or not self._captured():
             return False
         key = (M, N, K, silu_mul, slices)
         found = self._routes.get(key) if self._routes_of is d else None
@@ -646,16 +651,18 @@ class HipOps:
         if out_dtype not in (torch.bfloat16, torch.float32) or (silu_mul and out_dtype != torch.bfloat16):
             raise ValueError(f"norm_linear: prepared rows cannot give {out_dtype}")
         out = torch.empty(M, N, dtype=out_dtype, device=self.device)
-        if prepared.tiled or out_dtype is torch.bfloat16 \
-                and self._tiled_scaled_ok(M, N, K, silu_mul, prepared.slices):
+        stream = self._stream()
+        # (an eager step on the default stream, which cannot be captured, asks nothing)
+        if prepared.tiled or (stream.value or self._timed_plans) \
+                and self._tiled_scaled_ok(M, N, K, silu_mul, prepared.slices, out_dtype):
             self._call(self.lib.ts_gemm_tiled_scaled_bf16 if prepared.tiled
                        else self.lib.ts_gemm_tiled_scaled_rows_bf16, _ptr(prepared.rows),
                        _ptr(prepared.sumsq), prepared.slices, c_float(eps), _ptr(weight),
-                       _ptr(out), _TYPE_CODE[out_dtype], M, N, K, int(silu_mul), 0, self._stream())
+                       _ptr(out), _TYPE_CODE[out_dtype], M, N, K, int(silu_mul), 0, stream)
             return out, resid
         self._call(self.lib.ts_gemm_scaled_bf16, _ptr(prepared.rows), _ptr(prepared.sumsq),
                    prepared.slices, c_float(eps), _ptr(weight), _ptr(out), _TYPE_CODE[out_dtype], M, N, K,
-                   int(silu_mul), self._stream())
+                   int(silu_mul), stream)
         return out, resid
 
     def norm_heads(self, resid, delta, norm_weight, eps, weight, batch, table, cache, *, num_heads,
@@ -702,8 +709,8 @@ class HipOps:
             raise ValueError("norm_heads: prepared rows and stream differ in shape")
         self._check("weight", weight, torch.bfloat16, shape=(N, K))
         self._check_cache(cache, table, batch, num_kv_heads, head_dim)
-        self._fill_qk_args(a, batch, M, num_heads, num_kv_heads, head_dim, q_weight, k_weight,
-                           head_eps, cos_sin)
+        self._qk_args(M, batch, num_heads=num_heads, kv_in_row=num_kv_heads, head_dim=head_dim,
+                      q_weight=q_weight, k_weight=k_weight, eps=head_eps, cos_sin=cos_sin, a=a)
         if ((a.cos or 0) | (a.sin or 0) | cache.k_pages.data_ptr() | cache.v_pages.data_ptr()) % 16:
             return None                    # (16 bytes at a time: others have the separate kernels)
         q = torch.empty(M, num_heads, head_dim, dtype=torch.bfloat16, device=self.device)
@@ -735,8 +742,7 @@ class HipOps:
         self._fill_attention_args(a, q, out, batch, table, cache, num_heads, num_kv_heads, head_dim,
                                   scale, window, sink, **options)
         extras = any(options.get(k) is not None for k in ("softcap", "slopes", "q_temp"))
-        p.prefill, kept = self._plan_attention_mfma(p.attention, a, batch, num_heads // num_kv_heads,
-                                                    extras)
+        p.prefill, kept = self._attention_mfma(p.attention, a, batch, num_heads // num_kv_heads, extras)
         p.w_qkv, p.w_o = weight.data_ptr(), w_o.data_ptr()
         prepared = self._prompt_stream(p.s, resid, delta, hint, route, w_o.shape[0])
         self._call(self.lib.ts_prompt_attention, byref(p), self._stream())
@@ -855,22 +861,21 @@ class HipOps:
 
     # ------------------------------------------------------------ q/k preparation
     def _qk_args(self, qkv, batch, *, num_heads, kv_in_row, head_dim, q_weight, k_weight, eps,
-                 cos_sin, row_extra=0):
-        T = qkv.shape[0]
-        if row_extra < 0 or row_extra % 8:
-            raise ValueError(f"row_extra={row_extra} must be a multiple of 8")
-        self._check("qkv", qkv, self._FLOATS,
-                    shape=(T, (num_heads + 2 * kv_in_row) * head_dim + row_extra))
-        if head_dim % 2:
-            raise ValueError(f"head_dim={head_dim} must be even")
-        a = QkPrepareArgs()
-        a.qkv, a.row_extra = qkv.data_ptr(), row_extra
-        self._fill_qk_args(a, batch, T, num_heads, kv_in_row, head_dim, q_weight, k_weight, eps,
-                           cos_sin)
-        return a
-
-    def _fill_qk_args(self, a, batch, T, num_heads, kv_in_row, head_dim, q_weight, k_weight, eps,
-                      cos_sin):
+                 cos_sin, row_extra=0, a=None):
+        """The preparation's arguments for `qkv`; with `a`, those but for the rows, which are not there yet
+        (`qkv` then says how many), into it."""
+        if a is None:
+            T = qkv.shape[0]
+            if row_extra < 0 or row_extra % 8:
+                raise ValueError(f"row_extra={row_extra} must be a multiple of 8")
+            self._check("qkv", qkv, self._FLOATS,
+                        shape=(T, (num_heads + 2 * kv_in_row) * head_dim + row_extra))
+            if head_dim % 2:
+                raise ValueError(f"head_dim={head_dim} must be even")
+            a = QkPrepareArgs()
+            a.qkv, a.row_extra = qkv.data_ptr(), row_extra
+        else:
+            T = qkv
         a.num_tokens, a.nq, a.nkv, a.hd, a.eps = T, num_heads, kv_in_row, head_dim, eps
         if q_weight is not None:
             a.q_weight = self._check("q norm weight", q_weight, torch.float32,
@@ -893,6 +898,7 @@ class HipOps:
         self._check("entry_of_token", batch.entry_of_token, torch.int32, shape=(T,))
         a.positions = batch.positions.data_ptr()
         a.entry_of_token = batch.entry_of_token.data_ptr()
+        return a
 
     def _check_cache(self, cache, table, batch, nkv, head_dim):
         P = cache.page_size
@@ -1002,7 +1008,10 @@ class HipOps:
                                  cache.page_size, False):
                 self._attention_decode(a, batch, num_heads // num_kv_heads)
             else:
-                self._attention_mfma(a, batch, num_heads // num_kv_heads, extras)
+                m = AttentionMfmaArgs()
+                prefill, kept = self._attention_mfma(m, a, batch, num_heads // num_kv_heads, extras)
+                self._call(self.lib.ts_attention_prefill if prefill else self.lib.ts_attention_mfma,
+                           byref(m), self._stream())
         elif (q.dtype == torch.float32 and cache.k_pages.dtype == torch.float32
                 # (its loads are of 16 bytes; buffers that begin elsewhere take the general kernel)
                 and (q.data_ptr() | cache.k_pages.data_ptr() | cache.v_pages.data_ptr()) % 16 == 0
@@ -1125,14 +1134,7 @@ class HipOps:
         reach = min(a.window, a.chunk) if a.window and a.chunk else a.window or a.chunk
         return reach + -(-a.keep // 64) * 64 if reach else 0
 
-    def _attention_mfma(self, a, batch, group, extras=False):
-        """The plan of `_plan_attention_mfma`, launched."""
-        m = AttentionMfmaArgs()
-        prefill, kept = self._plan_attention_mfma(m, a, batch, group, extras)
-        self._call(self.lib.ts_attention_prefill if prefill else self.lib.ts_attention_mfma,
-                   byref(m), self._stream())
-
-    def _plan_attention_mfma(self, m, a, batch, group, extras):
+    def _attention_mfma(self, m, a, batch, group, extras):
         """Tile the batch's queries (16 rows of q heads x tokens per wavefront) and choose how
         many waves share a tile's keys, in `m`: (whether it is the kernel for long portions,
         what has to live until the launch)."""

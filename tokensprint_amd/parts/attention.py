@@ -80,15 +80,15 @@ class GroupedQueryAttention(StreamProducts, Mixer):
         fused = fused_rmsnorm_of(norm)
         if fused is None:
             return super().forward_from_stream(resid, delta, norm, batch, cache, write_cache)
-        o = None
         if isinstance(delta, PreparedRows) and delta.tiled:
             o, prepared = self._attend_prepared(resid, delta, fused, batch, cache, write_cache, hint)
             if prepared is not None:
                 return prepared, resid
-        if o is None:
-            qkv, resid = self.ops.norm_linear(resid, delta, fused[0], fused[1], self.w_qkv,
-                                              self.ctx.dtype)
-            o = self._attend(qkv, batch, cache, write_cache)
+            if o is not None:
+                return self.last_product(o, self.w_o, resid, hint), resid
+        qkv, resid = self.ops.norm_linear(resid, delta, fused[0], fused[1], self.w_qkv,
+                                          self.ctx.dtype)
+        o = self._attend(qkv, batch, cache, write_cache)
         return self.last_product(o, self.w_o, resid, hint), resid
 
     def _attend_prepared(self, resid, delta, norm, batch, cache, write_cache, hint):
