@@ -96,7 +96,8 @@ constexpr int kHeadRow = 128 + 8;
 // sixteen lanes take a row, eight elements each, as qk_prepare.hip's do (the same sums in the same
 // order), the tables' rows and pages asked for before the tile is there.  The preparation kernel read
 // and wrote what the product had just written (50 MB and 9 us a layer of 2,048 rows of 4,096 columns);
-// this is 3.8 us at the product's end, of shuffles, LDS and the tables' trip.  Values go into their pages
+// this is 1.7, 2.7 and 4.2 us at the end of a tile of 64, 128 and 256 rows (K = 1,024, against the same tile
+// written as it is), of shuffles, LDS and the tables' trip.  Values go into their pages
 // sixteen tokens at a time: where these fill a run of sixteen places (a prompt's mostly do), 16 bytes a
 // lane, eight tokens of one element, else an element at a time.
 template <int BM, int THREADS, typename PUT>
@@ -712,7 +713,8 @@ int launch_tiled(TiledArgsOf<FORM> g, hipStream_t stream) {
 // K = 3,072, and takes 7.3 and 9.5 in 64 x 32 tiles (160 workgroups of four wavefronts); 1,024 rows 13.2 and
 // 18.0, in 64 x 64 tiles 10.3 and 13.5.  64 x 128 is for up to 64 rows of many columns, where a tile of 128
 // rows brings every row of A twice (64 rows of 151,936 columns of 4,096: 244 us, 243 and 267 in 128 x 128
-// and 128 x 64; 16 rows 224, 236, 242).  Their fixed parts are what 65 to 1,024 rows of 21 weights show, and
+// and 128 x 64; 16 rows 224, 236, 242), and for rows that leave most of a last tile of 128 empty (192 rows of
+// 10,240 columns: 240 tiles, 320 of 128 x 64).  Their fixed parts are what 65 to 1,024 rows of 21 weights show, and
 // make a second round as long as the first, which for tiles that share a unit it is not (so the
 // larger tiles are chosen there, which are about as fast).
 struct TileCost {
