@@ -1,0 +1,138 @@
+"""The kernel of 32 query rows a wavefront that prompts' attention takes at head sizes 64 and 128:
+each of its forms (one, two and four sets of wavefronts that split an item's keys) against the plain
+attention, at the edges of its tiles (32 rows, items of 64 and 128), of its turns (32 and 64 keys) and
+of pages, with every option that reaches it."""
+
+import ctypes
+
+import pytest
+import torch
+
+from kernel_refs import TorchOps
+from scenarios import paged_scenario
+
+pytestmark = pytest.mark.gpu
+
+REF = TorchOps()
+FORMS = {"one-set": 3, "two-sets": 4, "four-sets": 5}
+
+
+@pytest.fixture(scope="module")
+def ops(gpu_device):
+    from tokensprint_amd.kernels import load_hip_ops
+    return load_hip_ops(gpu_device)
+
+
+@pytest.fixture(params=FORMS.values(), ids=FORMS.keys())
+def form(ops, request):
+    ops.lib.ts_attention_prefill_variant(request.param)
+    yield request.param
+    ops.lib.ts_attention_prefill_variant(2)
+
+
+def rand(shape, device, seed, scale=1.0):
+    g = torch.Generator().manual_seed(seed)
+    return (torch.randn(shape, generator=g) * scale).to(device)
+
+
+def check(ops, device, nq, nkv, hd, page, spans, **options):
+    """bfloat16 outputs against float32 attention over the same bfloat16 operands: weights are
+    rounded to 8 bits (2^-9 of the largest value each, at random) and so is the result (2^-9)."""
+    batch, cache, table, _ = paged_scenario(device, torch.bfloat16, nkv=nkv, hd=hd, page_size=page,
+                                            spans=spans, seed=11)
+    assert ops._prefill_tiles(batch, nkv, nq // nkv) is not None
+    q = rand((batch.num_tokens, nq, hd), device, 12).bfloat16()
+    kw = dict(num_heads=nq, num_kv_heads=nkv, head_dim=hd, scale=hd ** -0.5, window=None)
+    kw.update(options)
+    got = ops.paged_attention(q, batch, table, cache, **kw)
+    T, only, first = batch.num_tokens, set(), 0
+    for _, n in spans:          # a span's ends and the tokens around borders of items and tiles
+        only |= {first + t for t in (0, 1, 7, 8, 15, 16, 31, 32, 63, 64, 127, 128, n // 2, n - 2, n - 1)
+                 if 0 <= t < n}
+        first += n
+    only = sorted(only)
+    want = REF.paged_attention(q, batch, table, cache, only=only, **kw)
+    torch.testing.assert_close(got[only].float(), want[only].float(), rtol=1.6e-2, atol=1.6e-2)
+    assert torch.isfinite(got.float()).all()
+    return got, T
+
+
+@pytest.mark.parametrize("nq,nkv,hd,page", [(16, 8, 128, 16), (8, 8, 64, 16), (24, 8, 128, 32),
+                                            (32, 4, 64, 64), (40, 2, 128, 16), (16, 1, 128, 128)])
+@pytest.mark.parametrize("spans", [
+    [(0, 1000), (333, 1), (64, 33), (31, 65), (0, 17)],
+    [(448, 515), (63, 64), (1023, 1), (17, 191)],
+], ids=["from-the-start", "behind-others"])
+def test_spans(ops, gpu_device, form, nq, nkv, hd, page, spans):
+    check(ops, gpu_device, nq, nkv, hd, page, spans)
+
+
+@pytest.mark.parametrize("options", [
+    dict(window=1), dict(window=33), dict(window=200), dict(chunk=96), dict(window=40, keep_first=5),
+    dict(window=100, keep_first=70), dict(chunk=64, keep_first=130), dict(scale=2.5), dict(softcap=3.0),
+    dict(q_temp=(0.3, 100)), dict(softcap=20.0, window=90, keep_first=3),
+], ids=lambda o: "-".join(f"{k}{v}" for k, v in o.items()))
+@pytest.mark.parametrize("nq,nkv,hd", [(16, 8, 128), (12, 4, 64)])
+def test_options(ops, gpu_device, form, nq, nkv, hd, options):
+    check(ops, gpu_device, nq, nkv, hd, 16, [(0, 700), (450, 1), (300, 260)], **options)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+def test_sinks_and_slopes(ops, gpu_device, form, hd):
+    sink, slopes = rand((16,), gpu_device, 13, 2.0), rand((16,), gpu_device, 14).abs() * 0.05
+    check(ops, gpu_device, 16, 8, hd, 16, [(0, 600), (100, 200)], sink=sink)
+    check(ops, gpu_device, 16, 8, hd, 16, [(0, 600), (100, 200)], slopes=slopes, sink=sink)
+
+
+def test_growing_scores(ops, gpu_device, form):
+    """Scores that rise along the keys by far more than the 2^8 at which sums are rescaled, and fall
+    again: every block brings new largest scores for some rows, or none."""
+    nq, nkv, hd, S = 16, 8, 128, 900
+    batch, cache, table, _ = paged_scenario(gpu_device, torch.bfloat16, nkv=nkv, hd=hd, page_size=16,
+                                            spans=[(0, S)], seed=15)
+    direction = rand((hd,), gpu_device, 16)
+    direction = direction / direction.norm()
+    q = (rand((S, nq, hd), gpu_device, 17) * 0.3 + 4.0 * direction).bfloat16()
+    for shape in (lambda x: x, lambda x: 1 - x, lambda x: (x * 6).sin()):
+        for page in range(-(-S // 16)):
+            x = (torch.arange(16, device=gpu_device) + page * 16) / S
+            k = rand((nkv, 16, hd), gpu_device, 18 + page) * 0.2 + shape(x)[:, None] * 12.0 * direction
+            cache.k_pages[table[0, page]] = k.bfloat16()
+        kw = dict(num_heads=nq, num_kv_heads=nkv, head_dim=hd, scale=1.0, window=None)
+        got = ops.paged_attention(q, batch, table, cache, **kw)
+        only = list(range(0, S, 13)) + [31, 32, 63, 64, S - 1]
+        want = REF.paged_attention(q, batch, table, cache, only=only, **kw)
+        # (a few keys hold most of the weight, so the weights' rounding does not average out: 2^-8 of
+        # values up to 4)
+        torch.testing.assert_close(got[only].float(), want[only].float(), rtol=2e-2, atol=2e-2)
+
+
+def test_the_same_every_time(ops, gpu_device, form):
+    """Waves with blocks to skip run ahead of the others of their workgroup; a block sent for too
+    early would show as a result that differs from launch to launch."""
+    batch, cache, table, _ = paged_scenario(gpu_device, torch.bfloat16, nkv=8, hd=128, page_size=16,
+                                            spans=[(0, 1212), (333, 1), (50, 1027)], seed=19)
+    q = rand((batch.num_tokens, 16, 128), gpu_device, 20).bfloat16()
+    for window in (None, 40, 333):
+        kw = dict(num_heads=16, num_kv_heads=8, head_dim=128, scale=128 ** -0.5, window=window)
+        first = ops.paged_attention(q, batch, table, cache, **kw).clone()
+        for _ in range(20):
+            assert torch.equal(ops.paged_attention(q, batch, table, cache, **kw), first)
+
+
+def test_which_form(ops):
+    """The plan of a step: sets by how many items there are and how long they are."""
+    def plan(q_lens, starts, head_dim=128, page=16, heads=8, reach=0, rows=2):
+        n, sets = len(q_lens), ctypes.c_int(-1)
+        tiles = ops.lib.ts_attention_prefill_plan(head_dim, page, rows, heads, reach, n,
+                                                  (ctypes.c_int * n)(*q_lens), (ctypes.c_int * n)(*starts),
+                                                  ctypes.byref(sets))
+        return tiles, sets.value
+    assert plan([1024], [0]) == (4, 4)
+    assert plan([2600], [0]) == (8, 2)
+    assert plan([8192], [0], rows=8) == (8, 1)
+    # under a window the items are short, however long the sequence: one round is not what decides
+    assert plan([8192], [0], reach=128) == (8, 1)
+    assert plan([1] * 200, [4000] * 200) == (4, 0)
+    assert plan([1024], [0], head_dim=96) == (4, 0)
+    assert plan([1024], [0], page=24) == (1, 0)

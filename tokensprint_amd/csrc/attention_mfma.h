@@ -18,6 +18,7 @@ struct AttentionMfmaArgs {
   int head_blocks;       // ceil(group / 16)
   int num_splits;
   int cooperative;       // 1: a workgroup per item (few tiles), 0: a wavefront per item
-  int tiles_per_wave;    // prompt kernel: 16-row tiles a wavefront works on (1, 2 or 4)
+  int tiles_per_wave;    // prompt kernels: 16-row tiles of a work item
+  int sets;              // prompt kernel of 32 rows a wavefront: sets that split an item's keys; else 0
 };
 

@@ -18,7 +18,7 @@ from tokensprint_amd.kernels.build import build, find_library
 from tokensprint_amd.kernels.dispatch import default_dispatch
 from tokensprint_amd.kernels.stream import NormedPair, PreparedRows, UnmergedRows
 
-ABI_VERSION = 1
+ABI_VERSION = 2
 _TYPE_CODE = {torch.float32: 0, torch.bfloat16: 1}
 
 
@@ -58,7 +58,7 @@ AttentionMfmaArgs._fields_ = [
     ("base", AttentionArgs), ("tiles", c_void_p), ("partial_o", c_void_p),
     ("partial_ml", c_void_p), ("num_tiles", c_int), ("rows_per_token", c_int),
     ("head_blocks", c_int), ("num_splits", c_int), ("cooperative", c_int),
-    ("tiles_per_wave", c_int),
+    ("tiles_per_wave", c_int), ("sets", c_int),
 ]
 
 
@@ -1148,17 +1148,20 @@ class HipOps:
         # two from 16)
         page16 = a.page_size >= 16 and a.page_size & (a.page_size - 1) == 0
         d = self.dispatch
-        # (the same for every layer of a step)
-        key = ("prefill", group, a.nkv, a.hd, a.page_size, d.portion_tiles, d.portion_tokens,
-               d.single_token_tiles)
+        # (the same for every layer of a step with the same reach)
+        reach = self._reach(a)
+        key = ("prefill", group, a.nkv, a.hd, a.page_size, reach, d.portion_tiles,
+               d.portion_tokens, d.single_token_tiles)
         if key not in batch.plans:
-            tpw = 0
+            plan = 0, 0
             if self._prefill_tiles(batch, a.nkv, group) is not None:
-                tiles16 = sum(-(-n // tokens_per_tile) for n in batch.q_lens)
-                tpw = self.lib.ts_attention_prefill_tiles(a.hd, a.page_size, tiles16,
-                                                          a.nkv * head_blocks)
-            batch.plans[key] = tpw
-        tpw = batch.plans[key]
+                n, sets = batch.num_entries, c_int()
+                tpw = self.lib.ts_attention_prefill_plan(
+                    a.hd, a.page_size, rows_per_token, a.nkv * head_blocks, reach, n,
+                    (c_int * n)(*batch.q_lens), (c_int * n)(*batch.starts), byref(sets))
+                plan = tpw, sets.value
+            batch.plans[key] = plan
+        tpw, m.sets = batch.plans[key]
         if (not extras or page16) and tpw:
             tiles_dev, num_tiles = self._attention_tiles(batch, tokens_per_tile * tpw,
                                                          longest_first=True)
@@ -1171,7 +1174,6 @@ class HipOps:
             tiles_dev, num_tiles = self._attention_tiles(batch, tokens_per_tile)
         items = num_tiles * a.nkv * head_blocks
         chunk = self._attn_chunk
-        reach = self._reach(a)
         span = batch.max_ctx_len if reach == 0 else min(batch.max_ctx_len,
                                                         reach + batch.max_q_len + chunk)
         max_chunks = max(1, -(-span // chunk))
@@ -1206,7 +1208,7 @@ class HipOps:
         """Device list of (entry, first flat token, tokens) cutting every entry of the batch
         into runs of at most `tokens` consecutive tokens; made once per step and size.
         `longest_first`: sorted by the number of keys a run's last token sees, most first
-        (the kernels for long portions pair runs from both ends of that order)."""
+        (the kernels for long portions take them in that order)."""
         key = ("attn_tiles", tokens, longest_first)
         if key not in batch.plans and batch.max_q_len == 1:
             # a step of single tokens: tile i is entry i.  No order: the host's `starts` of a
