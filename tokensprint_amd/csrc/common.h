@@ -77,6 +77,79 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
   return total;
 }
 
+// The same of several sums at once.  `scratch`: N floats per wave.
+template <int N>
+__device__ __forceinline__ void block_sums(float (&v)[N], float* scratch) {
+#pragma unroll
+  for (int n = 0; n < N; ++n) v[n] = wave_sum(v[n]);
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int nwaves = (blockDim.x + kWave - 1) / kWave;
+  __syncthreads();
+  if (lane == 0) {
+#pragma unroll
+    for (int n = 0; n < N; ++n) scratch[N * wave + n] = v[n];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int n = 0; n < N; ++n) v[n] = 0.f;
+  for (int w = 0; w < nwaves; ++w) {
+#pragma unroll
+    for (int n = 0; n < N; ++n) v[n] += scratch[N * w + n];
+  }
+}
+
+// A thread's share of a row that a workgroup keeps in registers: eight elements, number k at `at(k)`.
+// QUADS: two fours side by side, moved 16 (bfloat16: 8) bytes at a time, for rows of a multiple of four
+// elements whose operands begin on 16 bytes; else an element at a time, a workgroup's threads apart.
+constexpr int kRowItems = 8;
+
+template <bool QUADS>
+struct RowShare {
+  int width;
+  __device__ __forceinline__ int at(int k) const {
+    return QUADS ? ((int)threadIdx.x + k / 4 * (int)blockDim.x) * 4 + k % 4 : (int)threadIdx.x + k * (int)blockDim.x;
+  }
+  __device__ __forceinline__ bool has(int k) const { return at(k) < width; }
+  // (zeros behind the row's end, or where there is nothing to read)
+  template <typename T>
+  __device__ __forceinline__ void load(const T* row, float (&v)[kRowItems], bool there = true) const {
+    typedef T four __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int k = 0; k < kRowItems; k += QUADS ? 4 : 1) {
+      if constexpr (QUADS) {
+        four x = {};
+        if (there && has(k)) x = *(const four*)(row + at(k));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[k + j] = to_f32(x[j]);
+      } else {
+        v[k] = there && has(k) ? to_f32(row[at(k)]) : 0.f;
+      }
+    }
+  }
+  template <typename T>
+  __device__ __forceinline__ void store(T* row, const float (&v)[kRowItems]) const {
+    typedef T four __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int k = 0; k < kRowItems; k += QUADS ? 4 : 1) {
+      if (!has(k)) continue;
+      if constexpr (QUADS) {
+        four x;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] = from_f32<T>(v[k + j]);
+        *(four*)(row + at(k)) = x;
+      } else {
+        row[at(k)] = from_f32<T>(v[k]);
+      }
+    }
+  }
+};
+
+// Whether rows of `width` elements of these operands (null or not) can be moved in fours.
+template <typename... P>
+inline bool rows_in_fours(int width, P... operand) {
+  return width % 4 == 0 && (((uintptr_t)operand | ...) & 15) == 0;
+}
+
 // 0.5 z (1 + tanh(sqrt(2 / pi) (z + 0.044715 z^3))), the tanh form of GELU.
 __device__ __forceinline__ float gelu_tanh(float z) {
   return 0.5f * z * (1.0f + tanhf(0.79788456080286536f * (z + 0.044715f * z * z * z)));

@@ -21,8 +21,10 @@ __device__ __forceinline__ float inv_rms(float sumsq, int n, float eps) {
 // A thread keeps the first kRowItems elements of its share of a row in registers between
 // the passes over the row (sum of squares, then the scaled values), so a row of up to
 // kRowItems x threads elements is read once; what lies beyond is read again.  A step of
-// few rows is a chain of trips to memory and barriers, and this halves the trips.
-constexpr int kRowItems = 8;
+// few rows is a chain of trips to memory and barriers, and this halves the trips.  (kRowItems and how
+// the share is moved: common.h.  In fours, 2,048 rows of 2,048: the add with the next norm 13.7 ->
+// 12.4 us, the norm with a token shift 10.2 -> 8.2, PolyNorm of 8,192 24.4 -> 22.8, with its three sums
+// added up together; 8 rows: 4.8 -> 4.2 and 5.1 -> 4.6.  What is left is the memory's rate, 4.4 TB/s.)
 
 // Threads for a row of `width` elements: eight elements a thread, 64 to 1024 threads.
 static int row_threads(int width) {
@@ -105,7 +107,7 @@ struct ShiftArgs {
   const int *positions, *slot_ids;      // of the rows
 };
 
-template <typename TD, typename TO, int THEN>
+template <typename TD, typename TO, int THEN, bool QUADS>
 __global__ __launch_bounds__(1024) void postnorm_add_kernel(
     float* __restrict__ resid, const TD* __restrict__ delta, const float* __restrict__ post_w,
     const float* __restrict__ norm_w, TO* __restrict__ out, int width, float post_eps,
@@ -119,58 +121,54 @@ __global__ __launch_bounds__(1024) void postnorm_add_kernel(
   float* x = resid + row * width;
   const TD* d = delta + row * width;
   TO* o = out + row * width;
+  const RowShare<QUADS> share{width};
   // (the weights are asked for with the row, not behind the sum that they wait for)
-  float dc[kRowItems], xc[kRowItems], pc[kRowItems], nc[kRowItems];
-  float mc[kShift ? kRowItems : 1], sc[kShift ? kRowItems : 1];
+  float dc[kRowItems], xc[kRowItems], pc[kRowItems], nc[kRowItems], mc[kRowItems], sc[kRowItems];
   float ss = 0.f;
-#pragma unroll
-  for (int k = 0; k < kRowItems; ++k) {
-    const int i = threadIdx.x + k * nt;
-    dc[k] = i < width ? to_f32(d[i]) : 0.f;
-    xc[k] = i < width ? x[i] : 0.f;
-    pc[k] = i < width ? post_w[i] : 0.f;
-    nc[k] = kNorm && i < width ? norm_w[i] : 0.f;
-    if constexpr (kShift) {
-      mc[k] = i < width ? shift.weight[i] : 0.f;
-      sc[k] = i < width && from_state ? st[i] : 0.f;
-    }
+  share.load(d, dc);
+  share.load(x, xc);
+  share.load(post_w, pc);
+  if (kNorm) share.load(norm_w, nc);
+  if constexpr (kShift) {
+    share.load(shift.weight, mc);
+    share.load(st, sc, from_state);
   }
 #pragma unroll
-  for (int k = 0; k < kRowItems; ++k) ss += dc[k] * dc[k];
+  for (int k = 0; k < kRowItems; ++k) ss = fmaf(dc[k], dc[k], ss);
   for (int i = threadIdx.x + kRowItems * nt; i < width; i += nt) {
     const float v = to_f32(d[i]);
-    ss += v * v;
+    ss = fmaf(v, v, ss);
   }
   const float r = inv_rms(block_sum(ss, scratch), width, post_eps);
   float ss2 = 0.f;
 #pragma unroll
   for (int k = 0; k < kRowItems; ++k) {
-    const int i = threadIdx.x + k * nt;
-    if (i < width) {
-      xc[k] = xc[k] + dc[k] * r * pc[k];
-      x[i] = xc[k];
-      if (THEN == kThenRows) o[i] = from_f32<TO>(xc[k]);
-      ss2 += xc[k] * xc[k];
-    }
+    xc[k] = xc[k] + dc[k] * r * pc[k];            // (zeros behind the row's end stay zeros)
+    if (share.has(k)) ss2 = fmaf(xc[k], xc[k], ss2);
   }
+  share.store(x, xc);
+  if (THEN == kThenRows) share.store(o, xc);
   for (int i = threadIdx.x + kRowItems * nt; i < width; i += nt) {
     const float v = x[i] + to_f32(d[i]) * r * post_w[i];
     x[i] = v;
     if (THEN == kThenRows) o[i] = from_f32<TO>(v);
-    ss2 += v * v;
+    ss2 = fmaf(v, v, ss2);
   }
   if (kNorm) {
     const float r2 = inv_rms(block_sum(ss2, scratch), width, norm_eps);
+    float h[kRowItems], shifted[kRowItems];
+#pragma unroll
+    for (int k = 0; k < kRowItems; ++k) {
+      h[k] = xc[k] * r2 * nc[k];
+      shifted[k] = kShift ? h[k] + (sc[k] - h[k]) * mc[k] : h[k];
+    }
+    share.store(o, shifted);
+    if constexpr (kShift) share.store(st, h);
     auto finish = [&](int i, float h, float prev, float mix) {
       if (!kShift) { o[i] = from_f32<TO>(h); return; }
       o[i] = from_f32<TO>(h + (prev - h) * mix);
       st[i] = h;
     };
-#pragma unroll
-    for (int k = 0; k < kRowItems; ++k) {
-      const int i = threadIdx.x + k * nt;
-      if (i < width) finish(i, xc[k] * r2 * nc[k], kShift ? sc[kShift ? k : 0] : 0.f, kShift ? mc[kShift ? k : 0] : 0.f);
-    }
     // each thread reads back the elements it wrote itself
     for (int i = threadIdx.x + kRowItems * nt; i < width; i += nt)
       finish(i, x[i] * r2 * norm_w[i], from_state ? st[i] : 0.f, kShift ? shift.weight[i] : 0.f);
@@ -186,20 +184,27 @@ extern "C" int ts_postnorm_add(float* resid, const void* delta, int delta_type,
   if (width <= 0) TS_FAIL("postnorm_add: bad width %d", width);
   if (norm_w && !out) TS_FAIL("postnorm_add: a norm without an output");
   const dim3 grid(rows), block(row_threads(width));
+  const bool quads = rows_in_fours(width, resid, delta, post_w, norm_w, out);
   TS_DISPATCH_TYPE(delta_type, TD, {
     if (!out) {
-      hipLaunchKernelGGL((postnorm_add_kernel<TD, float, kThenNothing>), grid, block, 0, stream,
-                         resid, (const TD*)delta, post_w, nullptr, nullptr, width, post_eps, 0.f, ShiftArgs{});
+      const auto kernel = quads ? postnorm_add_kernel<TD, float, kThenNothing, true>
+                                : postnorm_add_kernel<TD, float, kThenNothing, false>;
+      hipLaunchKernelGGL(kernel, grid, block, 0, stream, resid, (const TD*)delta, post_w, nullptr, nullptr,
+                         width, post_eps, 0.f, ShiftArgs{});
     } else if (norm_w) {
-      TS_DISPATCH_TYPE(out_type, TO,
-                       hipLaunchKernelGGL((postnorm_add_kernel<TD, TO, kThenNorm>), grid, block, 0,
-                                          stream, resid, (const TD*)delta, post_w, norm_w,
-                                          (TO*)out, width, post_eps, norm_eps, ShiftArgs{}));
+      TS_DISPATCH_TYPE(out_type, TO, {
+        const auto kernel = quads ? postnorm_add_kernel<TD, TO, kThenNorm, true>
+                                  : postnorm_add_kernel<TD, TO, kThenNorm, false>;
+        hipLaunchKernelGGL(kernel, grid, block, 0, stream, resid, (const TD*)delta, post_w, norm_w, (TO*)out,
+                           width, post_eps, norm_eps, ShiftArgs{});
+      });
     } else {
-      TS_DISPATCH_TYPE(out_type, TO,
-                       hipLaunchKernelGGL((postnorm_add_kernel<TD, TO, kThenRows>), grid, block, 0,
-                                          stream, resid, (const TD*)delta, post_w, nullptr,
-                                          (TO*)out, width, post_eps, 0.f, ShiftArgs{}));
+      TS_DISPATCH_TYPE(out_type, TO, {
+        const auto kernel = quads ? postnorm_add_kernel<TD, TO, kThenRows, true>
+                                  : postnorm_add_kernel<TD, TO, kThenRows, false>;
+        hipLaunchKernelGGL(kernel, grid, block, 0, stream, resid, (const TD*)delta, post_w, nullptr, (TO*)out,
+                           width, post_eps, 0.f, ShiftArgs{});
+      });
     }
   });
   TS_CHECK_LAUNCH("postnorm_add");
@@ -217,10 +222,13 @@ extern "C" int ts_postnorm_add_shift(float* resid, const void* delta, int delta_
   if (rows <= 0) return 0;
   if (width <= 0) TS_FAIL("postnorm_add_shift: bad width %d", width);
   const ShiftArgs shift{shift_w, state, positions, slot_ids};
-  TS_DISPATCH_TYPE(delta_type, TD, TS_DISPATCH_TYPE(out_type, TO,
-      hipLaunchKernelGGL((postnorm_add_kernel<TD, TO, kThenShift>), dim3(rows),
-                         dim3(row_threads(width)), 0, stream, resid, (const TD*)delta, post_w,
-                         norm_w, (TO*)out, width, post_eps, norm_eps, shift)));
+  const bool quads = rows_in_fours(width, resid, delta, post_w, norm_w, shift_w, state, out);
+  TS_DISPATCH_TYPE(delta_type, TD, TS_DISPATCH_TYPE(out_type, TO, {
+    const auto kernel = quads ? postnorm_add_kernel<TD, TO, kThenShift, true>
+                              : postnorm_add_kernel<TD, TO, kThenShift, false>;
+    hipLaunchKernelGGL(kernel, dim3(rows), dim3(row_threads(width)), 0, stream, resid, (const TD*)delta, post_w,
+                       norm_w, (TO*)out, width, post_eps, norm_eps, shift);
+  }));
   TS_CHECK_LAUNCH("postnorm_add_shift");
   return 0;
 }
@@ -491,7 +499,7 @@ extern "C" int ts_token_gate_product(const float* z, const void* table, const in
 // h_t = resid_t / rms(resid_t) * w;  out_t = h_t + (h_(t-1) - h_t) * shift.
 // h_(t-1) is recomputed from the row before inside a portion, read from the request's
 // state at a portion's first token, and zero at position 0.
-template <typename TO>
+template <typename TO, bool QUADS>
 __global__ __launch_bounds__(1024) void norm_token_shift_kernel(
     const float* __restrict__ resid, const float* __restrict__ norm_w,
     const float* __restrict__ shift_w, float* __restrict__ state, TO* __restrict__ out,
@@ -500,15 +508,12 @@ __global__ __launch_bounds__(1024) void norm_token_shift_kernel(
   __shared__ float scratch[16];
   const int t = blockIdx.x, nt = blockDim.x;
   const float* x = resid + (int64_t)t * width;
+  const RowShare<QUADS> share{width};
   // the row and the weights, asked for before it is known which other rows are wanted
   float xc[kRowItems], yc[kRowItems], sc[kRowItems], wc[kRowItems], mc[kRowItems];
-#pragma unroll
-  for (int k = 0; k < kRowItems; ++k) {
-    const int i = threadIdx.x + k * nt;
-    xc[k] = i < width ? x[i] : 0.f;
-    wc[k] = i < width ? norm_w[i] : 0.f;
-    mc[k] = i < width ? shift_w[i] : 0.f;
-  }
+  share.load(x, xc);
+  share.load(norm_w, wc);
+  share.load(shift_w, mc);
   const int e = entry_of_token[t], slot = slot_ids[e];
   const int first = q_start[e], last = q_start[e + 1] - 1;
   const bool is_first = t == first;
@@ -522,38 +527,40 @@ __global__ __launch_bounds__(1024) void norm_token_shift_kernel(
   const float* y = !is_first ? xp : xl;
   const bool need_y = !is_first || other_last;
   float ss = 0.f, ssy = 0.f;
+  share.load(y, yc, need_y);
+  share.load(st, sc, from_state);
 #pragma unroll
   for (int k = 0; k < kRowItems; ++k) {
-    const int i = threadIdx.x + k * nt;
-    yc[k] = (need_y && i < width) ? y[i] : 0.f;
-    sc[k] = (from_state && i < width) ? st[i] : 0.f;
-  }
-#pragma unroll
-  for (int k = 0; k < kRowItems; ++k) {
-    ss += xc[k] * xc[k];
-    ssy += yc[k] * yc[k];
+    ss = fmaf(xc[k], xc[k], ss);
+    ssy = fmaf(yc[k], yc[k], ssy);
   }
   for (int i = threadIdx.x + kRowItems * nt; i < width; i += nt) {
-    ss += x[i] * x[i];
-    if (need_y) ssy += y[i] * y[i];
+    ss = fmaf(x[i], x[i], ss);
+    if (need_y) ssy = fmaf(y[i], y[i], ssy);
   }
   const float r = inv_rms(block_sum(ss, scratch), width, eps);
   float ry = r;
   if (need_y) ry = inv_rms(block_sum(ssy, scratch), width, eps);
   TO* o = out + (int64_t)t * width;
-  auto finish = [&](int i, float xv, float yv, float sv, float w, float mix) {
+  auto parts = [&](float xv, float yv, float sv, float w, float mix, float& shifted, float& kept) {
     const float h = xv * r * w;
     float prev = 0.f;
     if (!is_first) prev = yv * ry * w;
     else if (from_state) prev = sv;
-    o[i] = from_f32<TO>(h + (prev - h) * mix);
-    if (is_first) st[i] = other_last ? yv * ry * w : h;
+    shifted = h + (prev - h) * mix;
+    kept = other_last ? yv * ry * w : h;
   };
+  float shifted[kRowItems], kept[kRowItems];
 #pragma unroll
-  for (int k = 0; k < kRowItems; ++k) {
-    const int i = threadIdx.x + k * nt;
-    if (i < width) finish(i, xc[k], yc[k], sc[k], wc[k], mc[k]);
-  }
+  for (int k = 0; k < kRowItems; ++k) parts(xc[k], yc[k], sc[k], wc[k], mc[k], shifted[k], kept[k]);
+  share.store(o, shifted);
+  if (is_first) share.store(st, kept);
+  auto finish = [&](int i, float xv, float yv, float sv, float w, float mix) {
+    float shifted, kept;
+    parts(xv, yv, sv, w, mix, shifted, kept);
+    o[i] = from_f32<TO>(shifted);
+    if (is_first) st[i] = kept;
+  };
   for (int i = threadIdx.x + kRowItems * nt; i < width; i += nt)
     finish(i, x[i], need_y ? y[i] : 0.f, from_state ? st[i] : 0.f, norm_w[i], shift_w[i]);
 }
@@ -566,43 +573,42 @@ extern "C" int ts_norm_token_shift(const float* resid, const float* norm_w, floa
   if (num_tokens <= 0) return 0;
   if (width <= 0) TS_FAIL("norm_token_shift: bad width %d", width);
   TS_DISPATCH_TYPE(out_type, TO,
-                   hipLaunchKernelGGL(norm_token_shift_kernel<TO>, dim3(num_tokens),
-                                      dim3(row_threads(width)), 0, stream, resid, norm_w, shift_w,
-                                      state, (TO*)out, positions, entry_of_token, q_start,
-                                      slot_ids, width, eps));
+                   {
+                     const auto kernel = rows_in_fours(width, resid, norm_w, shift_w, state, out)
+                         ? norm_token_shift_kernel<TO, true> : norm_token_shift_kernel<TO, false>;
+                     hipLaunchKernelGGL(kernel, dim3(num_tokens), dim3(row_threads(width)), 0, stream, resid,
+                                        norm_w, shift_w, state, (TO*)out, positions, entry_of_token, q_start,
+                                        slot_ids, width, eps);
+                   });
   TS_CHECK_LAUNCH("norm_token_shift");
   return 0;
 }
 
 // ---------------------------------------------------------------- PolyNorm
 // out = a z/rms(z) + b z^2/rms(z^2) + c z^3/rms(z^3) + e, powers element by element.
-template <typename TO>
+template <typename TO, bool QUADS>
 __global__ __launch_bounds__(1024) void polynorm_kernel(const float* __restrict__ z,
                                                         const float* __restrict__ coef,
                                                         TO* __restrict__ out, int width,
                                                         float eps) {
-  __shared__ float scratch[16];
+  __shared__ float scratch[48];
   const int64_t row = blockIdx.x;
   const int nt = blockDim.x;
   const float* x = z + row * width;
-  float zc[kRowItems];
-  float s2 = 0.f, s4 = 0.f, s6 = 0.f;
+  const RowShare<QUADS> share{width};
+  float zc[kRowItems], sum[3] = {0.f, 0.f, 0.f};      // of squares, fourth and sixth powers
   auto add = [&](float v) {
     const float v2 = v * v, v3 = v2 * v;
-    s2 += v2;
-    s4 += v2 * v2;
-    s6 += v3 * v3;
+    sum[0] += v2;
+    sum[1] += v2 * v2;
+    sum[2] += v3 * v3;
   };
+  share.load(x, zc);
 #pragma unroll
-  for (int k = 0; k < kRowItems; ++k) {
-    const int i = threadIdx.x + k * nt;
-    zc[k] = i < width ? x[i] : 0.f;
-    add(zc[k]);
-  }
+  for (int k = 0; k < kRowItems; ++k) add(zc[k]);
   for (int i = threadIdx.x + kRowItems * nt; i < width; i += nt) add(x[i]);
-  const float r1 = inv_rms(block_sum(s2, scratch), width, eps);
-  const float r2 = inv_rms(block_sum(s4, scratch), width, eps);
-  const float r3 = inv_rms(block_sum(s6, scratch), width, eps);
+  block_sums(sum, scratch);
+  const float r1 = inv_rms(sum[0], width, eps), r2 = inv_rms(sum[1], width, eps), r3 = inv_rms(sum[2], width, eps);
   const float a = coef[0], b = coef[1], c = coef[2], e = coef[3];
   TO* o = out + row * width;
   auto value = [&](float v) {
@@ -610,10 +616,8 @@ __global__ __launch_bounds__(1024) void polynorm_kernel(const float* __restrict_
     return a * (v * r1) + b * (v2 * r2) + c * (v2 * v * r3) + e;
   };
 #pragma unroll
-  for (int k = 0; k < kRowItems; ++k) {
-    const int i = threadIdx.x + k * nt;
-    if (i < width) o[i] = from_f32<TO>(value(zc[k]));
-  }
+  for (int k = 0; k < kRowItems; ++k) zc[k] = value(zc[k]);
+  share.store(o, zc);
   for (int i = threadIdx.x + kRowItems * nt; i < width; i += nt) o[i] = from_f32<TO>(value(x[i]));
 }
 
@@ -622,8 +626,8 @@ extern "C" int ts_polynorm(const float* z, const float* coef, void* out, int out
   if (rows <= 0) return 0;
   if (width <= 0) TS_FAIL("polynorm: bad width %d", width);
   TS_DISPATCH_TYPE(out_type, TO,
-                   hipLaunchKernelGGL(polynorm_kernel<TO>, dim3(rows), dim3(row_threads(width)), 0,
-                                      stream, z, coef, (TO*)out, width, eps));
+                   hipLaunchKernelGGL((rows_in_fours(width, z, out) ? polynorm_kernel<TO, true> : polynorm_kernel<TO, false>),
+                                      dim3(rows), dim3(row_threads(width)), 0, stream, z, coef, (TO*)out, width, eps));
   TS_CHECK_LAUNCH("polynorm");
   return 0;
 }

@@ -96,7 +96,9 @@ __global__ __launch_bounds__(256) void conv_silu_run_kernel(
 // The same with four channels a thread, for up to four taps and rows whose channels lie in fours
 // on 16 bytes: loads and stores of 16 bytes, and no look at a token's entry where the thread's
 // tokens and the inputs in front of them are one entry's (30 against 39 us for 2,048 tokens of
-// 6,144 channels: 3.4 TB/s).
+// 6,144 channels).  Four taps are a channel's 16 bytes: one by one, four of 64 lanes' 256 bytes a load, they
+// cost a unit more than the inputs (a load takes 2.1 cycles per line of 128 bytes it names, and sixteen of
+// those named 32 each; 31.3 -> 27.3 us, 4.4 TB/s).  Sixteen tokens a thread: 28.8.
 constexpr int kConvRunTaps = 4;
 __global__ __launch_bounds__(256) void conv_silu_run4_kernel(
     const float* __restrict__ proj, int ld, int col, int channels, int taps,
@@ -110,11 +112,21 @@ __global__ __launch_bounds__(256) void conv_silu_run4_kernel(
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   const f32x4 ib = in_bias ? *(const f32x4*)(in_bias + c) : zero;
   const f32x4 bc = bias ? *(const f32x4*)(bias + c) : zero;
+  const bool wide = taps == kConvRunTaps && ((uintptr_t)w & 15) == 0;
   f32x4 wk[kConvRunTaps], raw[kConvRun + kConvRunTaps - 1];
 #pragma unroll
-  for (int k = 0; k < kConvRunTaps; ++k)
+  for (int j = 0; j < 4; ++j) {
+    f32x4 of = zero;                  // one channel's
+    if (wide) {
+      of = *(const f32x4*)(w + (int64_t)(c + j) * kConvRunTaps);
+    } else {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) wk[k][j] = k < taps ? w[(c + j) * taps + k] : 0.f;
+      for (int k = 0; k < kConvRunTaps; ++k)
+        if (k < taps) of[k] = w[(int64_t)(c + j) * taps + k];
+    }
+#pragma unroll
+    for (int k = 0; k < kConvRunTaps; ++k) wk[k][j] = of[k];
+  }
   // raw[j]: the input of flat row t0 - (taps - 1) + j (whatever entry it belongs to)
 #pragma unroll
   for (int j = 0; j < kConvRun + kConvRunTaps - 1; ++j) {
@@ -247,7 +259,8 @@ extern "C" int ts_conv_silu(const float* proj, int ld, int col, int channels, in
                        (uintptr_t)in_bias) & 15) == 0;
   if (quads && num_tokens >= 256 && (num_tokens + kConvRun - 1) / kConvRun <= 65535) {
     hipLaunchKernelGGL(conv_silu_run4_kernel,
-                       dim3((unsigned)((channels / 4 + 255) / 256), (unsigned)((num_tokens + kConvRun - 1) / kConvRun)),
+                       dim3((unsigned)((channels / 4 + 255) / 256),
+                            (unsigned)((num_tokens + kConvRun - 1) / kConvRun)),
                        dim3(256), 0, stream, proj, ld, col, channels, taps, w, bias, state, out, b,
                        num_tokens, in_bias, plain);
     TS_CHECK_LAUNCH("conv_silu (runs of four channels)");

@@ -36,39 +36,30 @@ extern "C" int ts_stream_add(float* resid, const void* a, int a_type, const void
 // The same sum, and the RMS norm of the new stream: out = resid / sqrt(mean(resid^2) + eps) * w.
 // One workgroup a row; the row's values wait in registers between the two passes (up to
 // eight a thread), or are read back.
-template <typename TA, typename TB, typename TO>
+template <typename TA, typename TB, typename TO, bool QUADS>
 __global__ __launch_bounds__(256) void stream_add_norm_kernel(
     float* __restrict__ resid, const TA* __restrict__ a, const TB* __restrict__ b,
     const float* __restrict__ row, int row_stride, const float* __restrict__ w,
     TO* __restrict__ out, int width, float eps) {
   __shared__ float scratch[8];
-  constexpr int kKeep = 8;
   const int64_t base = (int64_t)blockIdx.x * width;
+  const RowShare<QUADS> share{width};
   if (row) row += (int64_t)blockIdx.x * row_stride;
   // (everything is asked for before the first store, which every later wait would wait for)
-  float keep[kKeep], av[kKeep], bv[kKeep], rv[kKeep], wv[kKeep], ss = 0.f;
+  float keep[kRowItems], av[kRowItems], bv[kRowItems], rv[kRowItems], wv[kRowItems], ss = 0.f;
+  share.load(resid + base, keep);
+  share.load(a + base, av);
+  share.load(b + base, bv, b != nullptr);
+  share.load(row, rv, row != nullptr);
+  share.load(w, wv);
 #pragma unroll
-  for (int j = 0; j < kKeep; ++j) {
-    const int c = j * blockDim.x + threadIdx.x;
-    const bool in = c < width;
-    keep[j] = in ? resid[base + c] : 0.f;
-    av[j] = in ? to_f32(a[base + c]) : 0.f;
-    bv[j] = in && b ? to_f32(b[base + c]) : 0.f;
-    rv[j] = in && row ? row[c] : 0.f;
-    wv[j] = in ? w[c] : 0.f;
-  }
-#pragma unroll
-  for (int j = 0; j < kKeep; ++j) {
+  for (int j = 0; j < kRowItems; ++j) {
     keep[j] += b ? av[j] + bv[j] : av[j];
     if (row) keep[j] += rv[j];
     ss = fmaf(keep[j], keep[j], ss);
   }
-#pragma unroll
-  for (int j = 0; j < kKeep; ++j) {
-    const int c = j * blockDim.x + threadIdx.x;
-    if (c < width) resid[base + c] = keep[j];
-  }
-  for (int c = kKeep * blockDim.x + threadIdx.x; c < width; c += blockDim.x) {
+  share.store(resid + base, keep);
+  for (int c = kRowItems * blockDim.x + threadIdx.x; c < width; c += blockDim.x) {
     float v = resid[base + c];
     v += b ? to_f32(a[base + c]) + to_f32(b[base + c]) : to_f32(a[base + c]);
     if (row) v += row[c];
@@ -77,11 +68,9 @@ __global__ __launch_bounds__(256) void stream_add_norm_kernel(
   }
   const float r = 1.0f / sqrtf(block_sum(ss, scratch) / (float)width + eps);
 #pragma unroll
-  for (int j = 0; j < kKeep; ++j) {
-    const int c = j * blockDim.x + threadIdx.x;
-    if (c < width) out[base + c] = from_f32<TO>(keep[j] * r * wv[j]);
-  }
-  for (int c = kKeep * blockDim.x + threadIdx.x; c < width; c += blockDim.x)
+  for (int j = 0; j < kRowItems; ++j) keep[j] = keep[j] * r * wv[j];
+  share.store(out + base, keep);
+  for (int c = kRowItems * blockDim.x + threadIdx.x; c < width; c += blockDim.x)
     out[base + c] = from_f32<TO>(resid[base + c] * r * w[c]);
 }
 
@@ -95,10 +84,12 @@ extern "C" int ts_stream_add_norm(float* resid, const void* a, int a_type, const
   const int threads = width >= 1024 ? 256 : (width >= 256 ? 128 : 64);
   TS_DISPATCH_TYPE(a_type, TA,
     TS_DISPATCH_TYPE(b ? b_type : TS_F32, TB,
-      TS_DISPATCH_TYPE(out_type, TO,
-        hipLaunchKernelGGL((stream_add_norm_kernel<TA, TB, TO>), dim3(rows), dim3(threads), 0,
-                           stream, resid, (const TA*)a, (const TB*)b, row, row_stride, w,
-                           (TO*)out, width, eps))));
+      TS_DISPATCH_TYPE(out_type, TO, {
+        const auto kernel = rows_in_fours(width, resid, a, b, row, w, out) ? stream_add_norm_kernel<TA, TB, TO, true>
+                                                                           : stream_add_norm_kernel<TA, TB, TO, false>;
+        hipLaunchKernelGGL(kernel, dim3(rows), dim3(threads), 0, stream, resid, (const TA*)a, (const TB*)b, row,
+                           row_stride, w, (TO*)out, width, eps);
+      })));
   TS_CHECK_LAUNCH("stream_add_norm");
   return 0;
 }
