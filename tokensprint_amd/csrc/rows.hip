@@ -3,13 +3,21 @@
 #include "common.h"
 
 // ---------------------------------------------------------------- embedding
-template <typename TW>
-__global__ void embed_kernel(const TW* __restrict__ table, const int* __restrict__ ids,
-                             float* __restrict__ out, int width, float scale) {
+// (In fours, 64 rows of 4,096: 9.8 -> 4.8 us, 8,192 of 5,120: 77.7 -> 42.9.)
+template <typename TW, bool QUADS>
+__global__ __launch_bounds__(256) void embed_kernel(const TW* __restrict__ table, const int* __restrict__ ids,
+                                                    float* __restrict__ out, int width, float scale) {
   const int64_t t = blockIdx.x;
   const TW* row = table + (int64_t)ids[t] * width;
   float* o = out + t * width;
-  for (int i = threadIdx.x; i < width; i += blockDim.x) o[i] = to_f32(row[i]) * scale;
+  for (int begin = 0; begin < width; begin += kRowItems * blockDim.x) {
+    const RowShare<QUADS> share{width - begin};
+    float v[kRowItems];
+    share.load(row + begin, v);
+#pragma unroll
+    for (int k = 0; k < kRowItems; ++k) v[k] *= scale;
+    share.store(o + begin, v);
+  }
 }
 
 // out[t] = table[ids[t]] * scale, in float32 (a scale of 1 changes no bit).
@@ -19,8 +27,8 @@ extern "C" int ts_embed(const void* table, int table_type, int vocab, const int*
   if (num_tokens <= 0) return 0;
   if (width <= 0 || vocab <= 0) TS_FAIL("embed: bad sizes width=%d vocab=%d", width, vocab);
   TS_DISPATCH_TYPE(table_type, TW,
-                   hipLaunchKernelGGL(embed_kernel<TW>, dim3(num_tokens), dim3(256), 0, stream,
-                                      (const TW*)table, ids, out, width, scale));
+                   hipLaunchKernelGGL((rows_in_fours(width, table, out) ? embed_kernel<TW, true> : embed_kernel<TW, false>),
+                                      dim3(num_tokens), dim3(256), 0, stream, (const TW*)table, ids, out, width, scale));
   TS_CHECK_LAUNCH("embed");
   return 0;
 }
