@@ -188,6 +188,74 @@ __device__ __forceinline__ void load_kv_block_wide(KvBlock<HD>& b, const Attenti
   cur.start(v + stride);
 }
 
+// The same block with its keys as they lie in memory, 64 lanes asking for 1 KB of a page's rows in
+// one run; spread_keys then brings them into the operand's order through LDS.  A compute unit takes
+// a load in about 2 cycles for each 128-byte line that a quarter of its lanes touches: lanes that each
+// ask for 16 bytes of a row of their own take 27 ns a kilobyte, these 8.  It counts where a unit
+// has little more than the loads of a first block to wait for (one request of 541 tokens,
+// 16 / 8 heads of 128: 7.5 -> 7.1 us a launch) and is nothing where memory is the limit.
+template <int HD>
+__device__ __forceinline__ void load_kv_block_rows(KvBlock<HD>& b, const AttentionArgs& a, PageCursor& cur,
+                                                   int kvh, int v, int stride, int lane) {
+  constexpr int KS = KvBlock<HD>::KS, DB = KvBlock<HD>::DB;
+  const int r = lane % 16, g = lane / 16;
+  const int kb = cur.walk.real(v);
+  const bf16_t* kp = (const bf16_t*)a.k_pages;
+  const bf16_t* vp = (const bf16_t*)a.v_pages;
+  const int P = a.page_size;
+  const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+  const int page0 = cur.next0, page1 = cur.next1;
+  const int in0 = kb & (P - 1), in1 = (kb + 16) & (P - 1);
+  const int64_t h0 = ((int64_t)max(page0, 0) * a.nkv + kvh) * P, h1 = ((int64_t)max(page1, 0) * a.nkv + kvh) * P;
+  const bf16_t* k0 = kp + (h0 + in0) * HD + lane * 8;
+  const bf16_t* k1 = kp + (h1 + in1) * HD + lane * 8;
+  const bool v_second = g >= 2;
+  const bf16_t* vcol = vp + (v_second ? h1 * HD + in1 : h0 * HD + in0) + (int64_t)r * P + (g % 2) * 8;
+#pragma unroll
+  for (int s = 0; s < KS; ++s) b.k[0][s] = *(const bf16x8*)(k0 + s * 512);
+#pragma unroll
+  for (int s = 0; s < KS; ++s) b.k[1][s] = *(const bf16x8*)(k1 + s * 512);
+#pragma unroll
+  for (int db = 0; db < DB; ++db) b.v[db] = *(const bf16x8*)(vcol + (int64_t)db * 16 * P);
+  if (page0 < 0 || page1 < 0) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      if (page0 < 0) b.k[0][s] = zero8;
+      if (page1 < 0) b.k[1][s] = zero8;
+    }
+    const bool v_ok = (v_second ? page1 : page0) >= 0;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) b.v[db] = v_ok ? b.v[db] : zero8;
+  }
+  cur.start(v + stride);
+}
+
+// From rows to the operand's order (the keys of load_kv_block_wide), by one wavefront through HD * 64
+// bytes of LDS of its own, 16-byte pieces of a row in an order that changes from row to row so that
+// the 16 rows of a read lie in different banks.
+template <int HD>
+__device__ __forceinline__ void spread_keys(KvBlock<HD>& b, unsigned char* scratch, int lane) {
+  constexpr int KS = HD / 32, CH = HD / 8;
+  constexpr int LOW = (CH & -CH) < 16 ? (CH & -CH) : 16, SHIFT = LOW == 16 ? 0 : LOW == 8 ? 1 : 2;
+  const int r = lane % 16, g = lane / 16;
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int u = s * 64 + lane, key = h * 16 + u / CH, c = u % CH;
+      const int i = key / 8 * 4 + key % 4;
+      *(bf16x8*)(scratch + (key * CH + (c ^ ((i >> SHIFT) & (LOW - 1)))) * 16) = b.k[h][s];
+    }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+  for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int key = r / 4 * 8 + blk * 4 + r % 4, c = g * KS + s;
+      b.k[blk][s] = *(const bf16x8*)(scratch + (key * CH + (c ^ ((r >> SHIFT) & (LOW - 1)))) * 16);
+    }
+}
+
 // One query tile's running state.
 template <int HD>
 struct TileState {

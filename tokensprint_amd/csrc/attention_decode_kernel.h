@@ -1,6 +1,7 @@
 // The kernel of attention_decode.hip as a template, so that its forms with and without
 // score extras compile in translation units of their own, side by side.
 #pragma once
+#include <type_traits>
 #include "attention_core.h"
 
 struct AttentionDecodeArgs {
@@ -23,63 +24,93 @@ struct AttentionDecodeArgs {
 int launch_attention_merge(const AttentionMfmaArgs& args, hipStream_t stream);
 
 template <int HD> constexpr int decode_waves() { return HD <= 128 ? 8 : 4; }
+// floats of a row of partial sums in LDS: neighbouring rows start four banks apart
+template <int HD> constexpr int merge_row() { return HD + 4; }
 
-// Norm and rotation of one head vector held in the query operand layout: `v` has the
-// lane's HD/4 elements [g*HD/4 + s*8 + j] as they come from the projection and gets them
-// back normed, rotated and rounded to bfloat16.  The elements are widened to float32 twice
-// (for the sum of squares, then slice by slice) rather than kept widened: registers are
-// short here, next to the first key block in flight.  `w` and `cs` are the lane's slices
-// of the norm weight and of the position's cos and sin, loaded by the caller together
-// with everything else the kernel starts with.
+// What the host works out for the kernel: the divisions by numbers that are the same for all.
+struct DecodeShape {
+  unsigned group;                  // query heads of a key/value head
+  unsigned heads, heads_inv;       // workgroups of an entry (key/value heads times blocks of their heads)
+  unsigned splits_inv;
+};
+inline unsigned inverse32(unsigned d) { return d <= 1 ? 0xffffffffu : (unsigned)((1ull << 32) / d); }
+// n / d for any n, with inv = inverse32(d): the estimate is at most one short.
+__device__ __forceinline__ unsigned divided(unsigned n, unsigned d, unsigned inv) {
+  const unsigned q = __umulhi(n, inv);
+  return q + (n - q * d >= d ? 1u : 0u);
+}
+
+// A lane's share of a head vector while it is normed and turned: four elements of the first half and
+// the four that they turn with.  HD / 8 lanes hold a head, so a wavefront does several at once (four
+// of 128 elements) and nothing crosses lanes but the sum of squares.  One wavefront does this while
+// the others wait for it, so what counts is how many instructions it issues (1.8 ns each) and how
+// many loads stand before its last: in the operand's layout, a quarter of a head to a lane and most
+// lanes without a row, this was 0.8 us of a step's 7.5 at one request.
 template <int HD>
-__device__ __forceinline__ void prepare_head(bf16x8 (&v)[HD / 32], bool live, bool weight,
-                                             const f32x4 (&w)[HD / 32][2], float eps,
-                                             const f32x4 (&cs)[HD / 32][4], bool rotate, int g) {
-  constexpr int KS = HD / 32;
-  const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-  float rstd = 1.f;
-  if (weight) {
-    float ss = 0.f;
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) ss += (float)v[s][j] * (float)v[s][j];
-    ss = col4_sum(live ? ss : 0.f);
-    rstd = rsqrtf(ss / (float)HD + eps);
+struct HeadShare {
+  static constexpr int USED = HD / 8;                                           // lanes of a head
+  static constexpr int LANES = USED <= 4 ? 4 : USED <= 8 ? 8 : USED <= 16 ? 16 : 32;
+  static constexpr int AT_ONCE = kWave / LANES;
+  bf16x4 lo, hi;
+  __device__ __forceinline__ void load(const bf16_t* head, int c) {
+    lo = *(const bf16x4*)(head + c * 4);
+    hi = *(const bf16x4*)(head + HD / 2 + c * 4);
   }
-  const bool first = g < 2;            // elements below hd/2
+  // where element e (a multiple of 4) of operand row `row` of `rows` stands, in units of four
+  static __device__ __forceinline__ int place(int e, int row, int rows) {
+    return ((e % (HD / 4) / 8 * 4 + e / (HD / 4)) * rows + row) * 2 + e % 8 / 4;
+  }
+  __device__ __forceinline__ void store(bf16x4* operand, int c, int row, int rows) const {
+    operand[place(c * 4, row, rows)] = lo;
+    operand[place(HD / 2 + c * 4, row, rows)] = hi;
+  }
+  __device__ __forceinline__ void prepare(bool norm, const f32x4 (&w)[2], float eps, bool turn, const f32x4& cs,
+                                          const f32x4& sn, int c) {
+    float x[4], y[4];
 #pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    float x[8];
+    for (int j = 0; j < 4; ++j) { x[j] = (float)lo[j]; y[j] = (float)hi[j]; }
+    if (norm) {
+      float ss = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = (float)v[s][j];
-    if (weight) {
+      for (int j = 0; j < 4; ++j) ss = fmaf(y[j], y[j], fmaf(x[j], x[j], ss));
+      if (USED < LANES && c >= USED) ss = 0.f;
+      // the neighbour's, the other pair's, then mirrored eights and sixteens
+      auto add_from = [&](auto lanes) {
+        ss += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(ss), decltype(lanes)::value, 0xf, 0xf, true));
+      };
+      add_from(std::integral_constant<int, 0xB1>());
+      add_from(std::integral_constant<int, 0x4E>());
+      if (LANES >= 8) add_from(std::integral_constant<int, 0x141>());
+      if (LANES >= 16) add_from(std::integral_constant<int, 0x140>());
+      if (LANES >= 32) {
+        auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(ss), __float_as_uint(ss), false, false);
+        ss = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+      }
+      const float rstd = rsqrtf(ss / (float)HD + eps);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) { x[j] *= rstd * w[s][0][j]; x[4 + j] *= rstd * w[s][1][j]; }
+      for (int j = 0; j < 4; ++j) { x[j] *= rstd * w[0][j]; y[j] *= rstd * w[1][j]; }
     }
-    if (rotate) {
+    if (turn) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        // the partner's element, from the lane 32 further: a row-swap instruction, fed
-        // the same value twice, returns each half's value in both halves
-        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[j]), __float_as_uint(x[j]),
-                                                         false, false);
-        const float other = __uint_as_float(first ? sw[1] : sw[0]);
-        const float c = cs[s][j / 4][j % 4], sn = cs[s][2 + j / 4][j % 4];
-        x[j] = first ? x[j] * c - other * sn : x[j] * c + other * sn;
+      for (int j = 0; j < 4; ++j) {
+        const float a = x[j], b = y[j];
+        x[j] = a * cs[j] - b * sn[j];
+        y[j] = b * cs[j] + a * sn[j];
       }
     }
-    bf16x8 o;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = (bf16_t)x[j];
-    v[s] = live ? o : zero8;
+    for (int j = 0; j < 4; ++j) { lo[j] = (bf16_t)x[j]; hi[j] = (bf16_t)y[j]; }
   }
-}
+};
 
 // A float32 to memory, and back, at device scope without ordering: such accesses pass the
 // caches that another XCD does not share.
 __device__ __forceinline__ void store_past_caches(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void store_past_caches(float* p, float v, float w) {     // p: of 8 bytes
+  __hip_atomic_store((uint64_t*)p, (uint64_t)__float_as_uint(w) << 32 | __float_as_uint(v), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ float load_past_caches(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -88,62 +119,47 @@ __device__ __forceinline__ float load_past_caches(const float* p) {
 // The merge of attention_merge_kernel (same order, same arithmetic per element, so the same
 // bits) by the THREADS threads of one workgroup, over the `used` first splits of one item:
 // slot (first_slot + split * 16 + row) holds a row's statistics and HD partial sums.  A
-// thread takes two elements at a time and asks for all of a group of eight splits before it
-// uses the first.
-template <int HD, int THREADS>
+// thread takes an element and asks for all of a group of GROUP splits before it uses the first:
+// the workgroup's last act, bound by one trip to memory and by its instructions (two elements a
+// thread and always eight splits: 1.5 us of 10.9 for four splits of 2 rows of 128, now 0.8).
+template <int HD, int THREADS, int GROUP>
 __device__ __forceinline__ void merge_splits_here(const float* partial_o, const float* partial_ml,
                                                   int64_t first_slot, int used, int rows, bf16_t* out,
                                                   const float* sink = nullptr, int first_head = 0) {
-  constexpr int kGroup = 8, E = 2;
-  const int count = rows * HD;
-  for (int e0 = threadIdx.x; e0 < count; e0 += E * THREADS) {
-    int row[E], d[E];
+  partial_o += first_slot * HD;
+  partial_ml += first_slot * 2;
+  for (int e = threadIdx.x; e < rows * HD; e += THREADS) {
+    const int row = e / HD, d = e % HD;
+    float M = -INFINITY, L = 0.f, acc = 0.f;
+    for (int s0 = 0; s0 < used; s0 += GROUP) {
+      float ms[GROUP], ls[GROUP], part[GROUP];
 #pragma unroll
-    for (int k = 0; k < E; ++k) {
-      const int e = min(e0 + k * THREADS, count - 1);    // past the end: the last again, not stored
-      row[k] = e / HD;
-      d[k] = e % HD;
-    }
-    float M[E], L[E], acc[E];
-#pragma unroll
-    for (int k = 0; k < E; ++k) { M[k] = -INFINITY; L[k] = 0.f; acc[k] = 0.f; }
-    for (int s0 = 0; s0 < used; s0 += kGroup) {
-      float ms[E][kGroup], ls[E][kGroup], part[E][kGroup];
-#pragma unroll
-      for (int j = 0; j < kGroup; ++j)
-#pragma unroll
-        for (int k = 0; k < E; ++k) {
-          const int64_t slot = first_slot + (int64_t)min(s0 + j, used - 1) * 16 + row[k];
-          ms[k][j] = load_past_caches(partial_ml + slot * 2);
-          ls[k][j] = load_past_caches(partial_ml + slot * 2 + 1);
-          part[k][j] = load_past_caches(partial_o + slot * HD + d[k]);
-        }
-#pragma unroll
-      for (int k = 0; k < E; ++k) {
-        float Mg = M[k];
-#pragma unroll
-        for (int j = 0; j < kGroup; ++j) Mg = (s0 + j < used) ? fmaxf(Mg, ms[k][j]) : Mg;
-        if (Mg == -INFINITY) continue;
-        const float keep = __builtin_amdgcn_exp2f(M[k] - Mg);
-        L[k] *= keep;
-        acc[k] *= keep;
-#pragma unroll
-        for (int j = 0; j < kGroup; ++j) {
-          const bool live = s0 + j < used && ms[k][j] != -INFINITY;
-          const float w = live ? __builtin_amdgcn_exp2f(ms[k][j] - Mg) : 0.f;
-          L[k] += live ? ls[k][j] * w : 0.f;
-          acc[k] += live ? part[k][j] * w : 0.f;
-        }
-        M[k] = Mg;
+      for (int j = 0; j < GROUP; ++j) {
+        const unsigned slot = min(s0 + j, used - 1) * 16 + row;
+        const uint64_t ml = __hip_atomic_load((const uint64_t*)partial_ml + slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        ms[j] = __uint_as_float((unsigned)ml);
+        ls[j] = __uint_as_float((unsigned)(ml >> 32));
+        part[j] = load_past_caches(partial_o + slot * HD + d);
       }
-    }
+      float Mg = M;
 #pragma unroll
-    for (int k = 0; k < E; ++k) {
-      if (e0 + k * THREADS >= count) break;
-      const float sum = sum_with_sink(L[k], M[k], sink, first_head + row[k]);
-      const float inv = sum > 0.f ? 1.f / sum : 0.f;
-      out[(int64_t)row[k] * HD + d[k]] = (bf16_t)(acc[k] * inv);
+      for (int j = 0; j < GROUP; ++j) Mg = (s0 + j < used) ? fmaxf(Mg, ms[j]) : Mg;
+      if (Mg == -INFINITY) continue;
+      const float keep = __builtin_amdgcn_exp2f(M - Mg);
+      L *= keep;
+      acc *= keep;
+#pragma unroll
+      for (int j = 0; j < GROUP; ++j) {
+        const bool live = s0 + j < used && ms[j] != -INFINITY;
+        const float w = live ? __builtin_amdgcn_exp2f(ms[j] - Mg) : 0.f;
+        L += live ? ls[j] * w : 0.f;
+        acc += live ? part[j] * w : 0.f;
+      }
+      M = Mg;
     }
+    const float sum = sum_with_sink(L, M, sink, first_head + row);
+    const float inv = sum > 0.f ? 1.f / sum : 0.f;
+    out[(int64_t)row * HD + d] = (bf16_t)(acc * inv);
   }
 }
 
@@ -164,27 +180,28 @@ __device__ __forceinline__ Ranked ranked_entry(const int* positions, int entries
 // EXTRA: scores with a cap, a distance bias or a query temperature (attention.h).
 // RANKED (more items than the chip has units, up to 64 entries, no splits): the items are the entries'
 // in the order of their contexts, longest first.  A unit holds one workgroup at a time (its eight
-// wavefronts take 206 registers), so a long context that comes late is walked alone at the end: 64
+// wavefronts take over 200 registers), so a long context that comes late is walked alone at the end: 64
 // entries of 100 to 2,047 tokens in no order 64.3 us (4.4 TB/s), ranked 55.9 (5.0), of 128 to 4,096
 // tokens 117.9 and 99.4 (5.6), 40 entries 50.7 and 41.7; entries of one length, which have nothing to
 // rank, 54.4 and 55.6.  A captured step's contexts are known on the device only, so every wavefront
 // ranks them for itself.  (Workgroups of four wavefronts, two to a unit: 61.1 and 114 us, ranked too.)
 template <int HD, bool FUSED, bool EXTRA, bool RANKED = false>
 __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_kernel(
-    AttentionDecodeArgs args) {
+    AttentionDecodeArgs args, DecodeShape sh) {
   constexpr int NW = decode_waves<HD>();
   constexpr int DB = HD / 16, KS = (HD + 31) / 32;
   const AttentionMfmaArgs& ma = args.m;
   const AttentionArgs& a = ma.base;
   const int wave = uniform(threadIdx.x / kWave), lane = threadIdx.x % kWave;
   const int r = lane % 16, g = lane / 16;
-  const int group = a.nq / a.nkv;
+  const int group = sh.group;
   const int item = blockIdx.x, split = blockIdx.y;
-  Ranked place{item / (a.nkv * ma.head_blocks), 0};
+  // a division by a number the compiler does not know costs 40 instructions before the first load
+  Ranked place{(int)divided(item, sh.heads, sh.heads_inv), 0};
+  int kvh = item - place.entry * sh.heads, hb = 0;
+  if (ma.head_blocks > 1) { hb = kvh % ma.head_blocks; kvh /= ma.head_blocks; }
   if constexpr (RANKED) place = ranked_entry(a.positions, ma.num_tiles, place.entry, lane);
   const int entry = place.entry;
-  const int kvh = (item / ma.head_blocks) % a.nkv;
-  const int hb = item % ma.head_blocks;
   const int token = entry;
   const int* table = a.table + (int64_t)entry * a.table_width;
 
@@ -202,44 +219,51 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
   const bool key_wave = adds_new && wave == NW - 2;
   const bool walker = !prep_wave && !key_wave;
   const int pos_lane = RANKED ? place.pos : a.positions[token];
-  bf16x8 kq[KS];            // the head vector such a wave prepares: query rows, or the new key
-  f32x4 cs[KS][4];          // cos (2 x 4) and sin (2 x 4) of the lane's elements
-  f32x4 pw[KS][2];          // norm weight
+  const int rows = min(ma.rows_per_token, group - hb * 16);
+  using Share = HeadShare<HD>;
+  const int share_row = lane / Share::LANES, share_lane = lane % Share::LANES;
+  const int share_at = min(share_lane, Share::USED - 1);
+  const bf16_t* row = FUSED ? args.qkv : nullptr;
+  if (FUSED) row += (int64_t)token * ((a.nq + 2 * args.kv_in_row) * HD + args.row_extra);
+  Share part;
+  f32x4 pw[2], cs, sn;
+  bf16x4 nv[DB], nv_slot = {0, 0, 0, 0};       // the new key's value: as a partial sum, and as its slot takes it
   const float* prep_weight = nullptr;
+  const bf16_t* first_head = nullptr;          // of the query heads, or the new key
   if constexpr (FUSED) {
     if (!walker) {
       prep_weight = prep_wave ? args.q_weight : args.k_weight;
-      const bf16_t* src = args.qkv + (int64_t)token * ((a.nq + 2 * args.kv_in_row) * HD + args.row_extra) +
-                          (int64_t)(prep_wave ? head : a.nq + kvh) * HD + g * (HD / 4);
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        kq[s] = *(const bf16x8*)(src + s * 8);
-        if (prep_weight) {
-          pw[s][0] = *(const f32x4*)(prep_weight + g * (HD / 4) + s * 8);
-          pw[s][1] = *(const f32x4*)(prep_weight + g * (HD / 4) + s * 8 + 4);
-        }
+      first_head = row + (int64_t)(prep_wave ? kvh * group + hb * 16 : a.nq + kvh) * HD;
+      part.load(first_head + (int64_t)(prep_wave ? min(share_row, rows - 1) : 0) * HD, share_at);
+      if (prep_weight) {
+        pw[0] = *(const f32x4*)(prep_weight + share_at * 4);
+        pw[1] = *(const f32x4*)(prep_weight + HD / 2 + share_at * 4);
       }
     }
   }
   const int pos = uniform(pos_lane);
   if constexpr (FUSED) {
-    if (!walker && args.cos != nullptr) {
+    if (!walker) {
+      if (args.cos != nullptr) {
+        cs = *(const f32x4*)(args.cos + (int64_t)pos * (HD / 2) + share_at * 4);
+        sn = *(const f32x4*)(args.sin + (int64_t)pos * (HD / 2) + share_at * 4);
+      }
+      if (key_wave) {
+        const bf16_t* vrow = row + (int64_t)(a.nq + args.kv_in_row + kvh) * HD;
 #pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const int64_t i = (int64_t)pos * (HD / 2) + (g & 1) * (HD / 4) + s * 8;
-        cs[s][0] = *(const f32x4*)(args.cos + i);
-        cs[s][1] = *(const f32x4*)(args.cos + i + 4);
-        cs[s][2] = *(const f32x4*)(args.sin + i);
-        cs[s][3] = *(const f32x4*)(args.sin + i + 4);
+        for (int db = 0; db < DB; ++db) nv[db] = *(const bf16x4*)(vrow + db * 16 + g * 4);
+        nv_slot = *(const bf16x4*)(vrow + min(r, DB - 1) * 16 + g * 4);
       }
     }
   }
+  int new_page = -1;
+  if (FUSED && key_wave && hb == 0 && pos >= 0) new_page = ((ConstTable)table)[pos >> __builtin_ctz(a.page_size)];
   const int last = new_key ? pos - 1 : pos;                   // last key walked from the cache
   const int lo = first_visible(a, pos);
   // chunks of this split: the arithmetic of attention_merge (from pos, not from last)
   const KeyWalk walk = key_walk<32>(a, lo);
   const int c_first = walk.origin / kChunk, c_last = pos / kChunk;
-  const int per = (c_last - c_first + ma.num_splits) / ma.num_splits;
+  const int per = divided(c_last - c_first + ma.num_splits, ma.num_splits, sh.splits_inv);
   const int c0 = c_first + split * per, c1 = min(c0 + per, c_last + 1);
   if (c0 > c_last) {   // more splits than chunks: a neutral partial, no data touched
     if (g == 0 && wave == 0) {
@@ -267,73 +291,61 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
   // head sizes in whole 32-element slices take the blocks with 16-byte value loads
   constexpr bool kWide = HD % 32 == 0;
   auto load_block = [&](KvBlock<HD>& b, int kb) {
-    if constexpr (kWide) load_kv_block_wide<HD>(b, a, cur, kvh, kb, stride, r, g);
+    if constexpr (kWide) load_kv_block_rows<HD>(b, a, cur, kvh, kb, stride, lane);
     else load_kv_block<HD, true>(b, a, table, cur, kvh, kb, stride, r, g);
   };
 
   if constexpr (FUSED) {
     // The last wave prepares the query rows for all of them (through LDS): the others
-    // have their first key block in flight meanwhile and no registers to spare for the
-    // cos, sin and norm weight slices.
-    __shared__ bf16x8 s_q[KS][kWave];
-    const int row_width = (a.nq + 2 * args.kv_in_row) * HD + args.row_extra;
-    const bf16_t* row = args.qkv + (int64_t)token * row_width;
+    // have their first key block in flight meanwhile.
+    __shared__ bf16x8 s_q[KS * kWave];         // [slice][lane of the operand]
+    __shared__ bf16x8 s_k[KS * 4];             // the new key: [slice][g]
     const bool rotate = args.cos != nullptr;
     if (walker) {
       cur.start(key_begin);
       if (key_begin < key_end) load_block(A, key_begin);
     }
     if (!walker) {
-      prepare_head<HD>(kq, prep_wave ? row_ok : true, prep_weight != nullptr, pw, args.eps, cs, rotate, g);
       if (prep_wave) {
-#pragma unroll
-        for (int s = 0; s < KS; ++s) s_q[s][lane] = kq[s];
+        for (int row0 = 0;;) {
+          Share coming = part;
+          if (row0 + Share::AT_ONCE < rows)
+            coming.load(first_head + (int64_t)min(row0 + Share::AT_ONCE + share_row, rows - 1) * HD, share_at);
+          part.prepare(prep_weight != nullptr, pw, args.eps, rotate, cs, sn, share_lane);
+          if (share_lane < Share::USED && row0 + share_row < rows)
+            part.store((bf16x4*)s_q, share_lane, row0 + share_row, 16);
+          row0 += Share::AT_ONCE;
+          if (row0 >= rows) break;
+          part = coming;
+        }
+      } else {
+        part.prepare(prep_weight != nullptr, pw, args.eps, rotate, cs, sn, share_lane);
+        if (lane < Share::USED) part.store((bf16x4*)s_k, lane, 0, 1);
       }
     }
     __syncthreads();
+    const int q_row = g * 16 + min(r, rows - 1);      // rows past the last take its query: nobody reads them
 #pragma unroll
-    for (int s = 0; s < KS; ++s) t.q[s] = s_q[s][lane];
+    for (int s = 0; s < KS; ++s) t.q[s] = s_q[s * kWave + q_row];
 #pragma unroll
     for (int db = 0; db < DB; ++db) t.o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
     t.m = -INFINITY;
     t.l = 0.f;
 
     if (key_wave) {
-      const bf16_t* vrow = row + (int64_t)(a.nq + args.kv_in_row + kvh) * HD;
-      float dot = 0.f;
+      f32x4 dots = {0.f, 0.f, 0.f, 0.f};                    // every row of the product's keys is the new key
 #pragma unroll
       for (int s = 0; s < KS; ++s)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) dot += (float)t.q[s][j] * (float)kq[s][j];
+        dots = __builtin_amdgcn_mfma_f32_16x16x32_bf16(s_k[s * 4 + g], t.q[s], dots, 0, 0, 0);
+      const float dot = dots[0];
       // this wave's partial: one key with weight 1
-      t.m = EXTRA ? extra_score_log2(x, col4_sum(dot), pos)
-                  : col4_sum(dot) * scale_log2;
+      t.m = EXTRA ? extra_score_log2(x, dot, pos)
+                  : dot * scale_log2;
       t.l = g == 0 ? 1.f : 0.f;
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
-        const bf16x4 v = *(const bf16x4*)(vrow + db * 16 + g * 4);
+        const bf16x4 v = nv[db];
         t.o[db] = f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
-      }
-      if (hb == 0) {   // into the cache slot of position pos, once per key/value head
-        const int P = a.page_size;
-        const int page = uniform(table[pos >> __builtin_ctz(P)]);
-        const int off = pos & (P - 1);
-        if (page >= 0) {
-          bf16_t* kdst = (bf16_t*)a.k_pages + (((int64_t)page * a.nkv + kvh) * P + off) * HD;
-          if (r == 0) {
-#pragma unroll
-            for (int s = 0; s < KS; ++s) *(bf16x8*)(kdst + g * (HD / 4) + s * 8) = kq[s];
-          }
-          bf16_t* vdst = (bf16_t*)a.v_pages + ((int64_t)page * a.nkv + kvh) * HD * P + off;
-          if (r < DB) {
-            const bf16x4 v = *(const bf16x4*)(vrow + r * 16 + g * 4);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) vdst[(int64_t)(r * 16 + g * 4 + i) * P] = v[i];
-          }
-        }
-        // vmcnt(0): no store is in flight where this path joins the walkers' (this wave
-        // has nothing else to do meanwhile)
-        __builtin_amdgcn_s_waitcnt(0x0F70);
       }
     }
   } else {
@@ -342,7 +354,11 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
     load_query<HD>(t, (const bf16_t*)a.q + ((int64_t)token * a.nq + head) * HD, row_ok, g);
   }
 
-  auto update = [&](const KvBlock<HD>& b, int v) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char merge_lds[];
+  // a wavefront's keys are spread where its partial sums will stand: nobody else's
+  unsigned char* scratch = merge_lds + NW * kWave * 2 * 4 + wave * (16 * merge_row<HD>() * 4);
+  auto update = [&](KvBlock<HD>& b, int v) {
+    if constexpr (kWide) spread_keys<HD>(b, scratch, lane);
     const int kb = walk.real(v);
     tile_update<HD, false, kWide, EXTRA>(t, b, kb, scale_log2, kb + 31 <= last && kb >= lo, g, &x);
   };
@@ -361,14 +377,34 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
   // The waves' partial results (the new key's among them) all go to LDS, and every wave
   // merges, in wave order, its share of the head's blocks of 16 elements and stores that
   // share: the merge is as wide as the workgroup instead of one wave's long tail.
-  extern __shared__ __attribute__((aligned(16))) unsigned char merge_lds[];
   float (*s_ml)[kWave][2] = (float (*)[kWave][2])merge_lds;                        // [NW]
-  f32x4 (*s_o)[DB][kWave] = (f32x4 (*)[DB][kWave])(merge_lds + NW * kWave * 2 * 4);  // [NW]
+  constexpr int kRow = merge_row<HD>();
+  float (*s_o)[16][kRow] = (float (*)[16][kRow])(merge_lds + NW * kWave * 2 * 4);    // [NW]
   s_ml[wave][lane][0] = m;
   s_ml[wave][lane][1] = l;
 #pragma unroll
-  for (int db = 0; db < DB; ++db) s_o[wave][db][lane] = o[db];
+  for (int db = 0; db < DB; ++db) *(f32x4*)&s_o[wave][r][db * 16 + g * 4] = o[db];
   __syncthreads();
+  if constexpr (FUSED) {
+    // The new key and value into the cache slot of position pos, once per key/value head: behind
+    // the last barrier that others wait at, with nothing loaded after them here (loads and stores
+    // share a counter, and a wait for a load would wait for these).
+    if (key_wave && hb == 0) {
+      const int P = a.page_size, off = pos & (P - 1);
+      if (new_page >= 0) {
+        bf16_t* kdst = (bf16_t*)a.k_pages + (((int64_t)new_page * a.nkv + kvh) * P + off) * HD;
+        if (lane < Share::USED) {
+          *(bf16x4*)(kdst + lane * 4) = part.lo;
+          *(bf16x4*)(kdst + HD / 2 + lane * 4) = part.hi;
+        }
+        bf16_t* vdst = (bf16_t*)a.v_pages + ((int64_t)new_page * a.nkv + kvh) * HD * P + off;
+        if (r < DB) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) vdst[(int64_t)(r * 16 + g * 4 + i) * P] = nv_slot[i];
+        }
+      }
+    }
+  }
   constexpr int kShare = (DB + NW - 1) / NW;         // blocks of 16 elements per wave
   // Merge by the last to finish: the partial results go out past the caches (their readers
   // may sit on another XCD, behind another L2), each wave waits until its own have been
@@ -377,10 +413,47 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
   // the order and arithmetic of attention_merge.  Nothing here needs the caches written
   // back or dropped, which is what release and acquire at device scope would cost.
   const bool fold = ma.num_splits > 1 && !args.defer_merge && args.arrivals != nullptr;
-  const bool has_share = wave * kShare < DB;
+  const bool has_share = rows * HD <= NW * kWave ? wave * kWave < rows * HD : wave * kShare < DB;
   if (!has_share && !fold) return;
   const int64_t slot = ((int64_t)item * ma.num_splits + split) * 16 + r;
-  if (has_share) {
+  if (rows * HD <= NW * kWave) {
+    // few rows (4 of 128): an element a thread, which is a quarter of the instructions that the
+    // operand's layout takes with most of its rows empty (0.3 us of 5.6)
+    const int e = threadIdx.x, mrow = e / HD, d = e % HD;
+    if (mrow < rows) {
+      float mw[NW], lw[NW], ow[NW];
+#pragma unroll
+      for (int w = 0; w < NW; ++w) { mw[w] = s_ml[w][mrow][0]; lw[w] = s_ml[w][mrow][1]; ow[w] = s_o[w][mrow][d]; }
+      float M = mw[0];
+#pragma unroll
+      for (int w = 1; w < NW; ++w) M = fmaxf(M, mw[w]);
+      const float Mc = fmaxf(M, -1e30f);
+      float acc = 0.f, sum = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float ww = __builtin_amdgcn_exp2f(mw[w] - Mc);
+        sum = fmaf(lw[w], ww, sum);
+        acc += ww == 0.f ? 0.f : ow[w] * ww;
+      }
+      const int h = kvh * group + hb * 16 + mrow;
+      if (ma.num_splits == 1) {
+        sum = sum_with_sink(sum, M, a.sink, h);
+        const float inv = sum > 0.f ? 1.f / sum : 0.f;
+        ((bf16_t*)a.out)[((int64_t)token * a.nq + h) * HD + d] = (bf16_t)(acc * inv);
+      } else {
+        const int64_t at_slot = ((int64_t)item * ma.num_splits + split) * 16 + mrow;
+        float* po = ma.partial_o + at_slot * HD + d;
+        float* pm = ma.partial_ml + at_slot * 2;
+        if (fold) {
+          store_past_caches(po, acc);
+          if (d == 0) store_past_caches(pm, M, sum);
+        } else {
+          *po = acc;
+          if (d == 0) { pm[0] = M; pm[1] = sum; }
+        }
+      }
+    }
+  } else if (has_share) {
     float M = -INFINITY;
 #pragma unroll
     for (int w = 0; w < NW; ++w) M = fmaxf(M, s_ml[w][lane][0]);
@@ -405,7 +478,7 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int w = 0; w < NW; ++w) {
-        const f32x4 ow = s_o[w][db][lane];
+        const f32x4 ow = *(const f32x4*)&s_o[w][r][db * 16 + g * 4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[i] += ww[w] == 0.f ? 0.f : ow[i] * ww[w];   // never 0 * garbage
       }
@@ -423,8 +496,7 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
     }
     if (ma.num_splits > 1 && wave == 0 && g == 0) {
       if (fold) {
-        store_past_caches(ma.partial_ml + slot * 2, m);
-        store_past_caches(ma.partial_ml + slot * 2 + 1, l);
+        store_past_caches(ma.partial_ml + slot * 2, m, l);
       } else {
         ma.partial_ml[slot * 2] = m;
         ma.partial_ml[slot * 2 + 1] = l;
@@ -446,10 +518,13 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
   if (threadIdx.x == 0)
     __hip_atomic_store(args.arrivals + item, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const int rows = min(ma.rows_per_token, group - hb * 16);
   bf16_t* out = (bf16_t*)a.out + ((int64_t)token * a.nq + kvh * group + hb * 16) * HD;
-  merge_splits_here<HD, NW * kWave>(ma.partial_o, ma.partial_ml, (int64_t)item * ma.num_splits * 16,
-                                    used, rows, out, a.sink, kvh * group + hb * 16);
+  auto merge = [&](auto at_once) {
+    merge_splits_here<HD, NW * kWave, decltype(at_once)::value>(ma.partial_o, ma.partial_ml, (int64_t)item * ma.num_splits * 16,
+                                                                used, rows, out, a.sink, kvh * group + hb * 16);
+  };
+  if (used <= 4) merge(std::integral_constant<int, 4>());
+  else merge(std::integral_constant<int, 8>());
 }
 
 int launch_attention_merge(const AttentionMfmaArgs& args, hipStream_t stream);
@@ -458,9 +533,12 @@ template <int HD, bool EXTRA, bool RANKED = false>
 static int launch_decode(const AttentionDecodeArgs& args, hipStream_t stream) {
   const AttentionMfmaArgs& m = args.m;
   const int items = m.num_tiles * m.base.nkv * m.head_blocks;
+  const AttentionArgs& a = m.base;
+  const unsigned heads = a.nkv * m.head_blocks;
+  const DecodeShape sh{(unsigned)(a.nq / a.nkv), heads, inverse32(heads), inverse32(m.num_splits)};
   const dim3 grid(items, m.num_splits), block(decode_waves<HD>() * kWave);
   // the merge area: per wave its row statistics and HD/16 blocks of partial sums
-  const size_t lds = (size_t)decode_waves<HD>() * (kWave * 2 * 4 + (HD / 16) * kWave * 16);
+  const size_t lds = (size_t)decode_waves<HD>() * (kWave * 2 * 4 + 16 * merge_row<HD>() * 4);
   if (args.qkv) {
     if constexpr (HD % 32 == 0) {
       auto kernel = attention_decode_kernel<HD, true, EXTRA, RANKED>;
@@ -471,7 +549,7 @@ static int launch_decode(const AttentionDecodeArgs& args, hipStream_t stream) {
           TS_FAIL("attention_decode: cannot raise the LDS limit to %zu bytes", lds);
         raised = true;
       }
-      hipLaunchKernelGGL(kernel, grid, block, lds, stream, args);
+      hipLaunchKernelGGL(kernel, grid, block, lds, stream, args, sh);
     } else {
       TS_FAIL("attention_decode: the fused form needs a head size that is a multiple of 32");
     }
@@ -484,7 +562,7 @@ static int launch_decode(const AttentionDecodeArgs& args, hipStream_t stream) {
         TS_FAIL("attention_decode: cannot raise the LDS limit to %zu bytes", lds);
       raised = true;
     }
-    hipLaunchKernelGGL(kernel, grid, block, lds, stream, args);
+    hipLaunchKernelGGL(kernel, grid, block, lds, stream, args, sh);
   }
   if (m.num_splits > 1 && !args.defer_merge && !args.arrivals) return launch_attention_merge(m, stream);
   return 0;
