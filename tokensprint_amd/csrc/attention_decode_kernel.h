@@ -33,12 +33,6 @@ struct DecodeShape {
   unsigned heads, heads_inv;       // workgroups of an entry (key/value heads times blocks of their heads)
   unsigned splits_inv;
 };
-inline unsigned inverse32(unsigned d) { return d <= 1 ? 0xffffffffu : (unsigned)((1ull << 32) / d); }
-// n / d for any n, with inv = inverse32(d): the estimate is at most one short.
-__device__ __forceinline__ unsigned divided(unsigned n, unsigned d, unsigned inv) {
-  const unsigned q = __umulhi(n, inv);
-  return q + (n - q * d >= d ? 1u : 0u);
-}
 
 // A lane's share of a head vector while it is normed and turned: four elements of the first half and
 // the four that they turn with.  HD / 8 lanes hold a head, so a wavefront does several at once (four

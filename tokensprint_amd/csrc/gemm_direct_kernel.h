@@ -31,7 +31,7 @@ __device__ __forceinline__ bf16x8 row_down_by(bf16x8 v, int n) {
 template <int MT, int WK, typename TC, bool PAIR, bool NORM, int S, int PD, bool SCALED = false,
           bool TAIL = false, int CW = 16, int AR = 16, bool MERGE = false, bool CONV = false>
 __global__ __launch_bounds__(WK* kWave) void gemm_direct_kernel(
-    std::conditional_t<CONV, ConvArgs, DirectArgs> a) {
+    std::conditional_t<CONV, ConvArgs, std::conditional_t<MERGE, MergedArgs, DirectArgs>> a) {
   static_assert(!NORM || MT == 1, "the fused form holds one tile of rows");
   static_assert(!MERGE || (TAIL && MT == 1), "the merged form: a tail product of one tile of rows");
   static_assert(!CONV || (MT == 1 && !PAIR && !NORM && !SCALED && !TAIL), "the convolved form is a plain product");
@@ -286,101 +286,94 @@ __global__ __launch_bounds__(WK* kWave) void gemm_direct_kernel(
   Step st[PD];
   int kb = kb0;
   if constexpr (MERGE) {
-    // The first steps' rows of W are asked for, then every thread merges pieces of eight
-    // elements of A (the arithmetic of attention_merge, split by split in groups of
-    // eight, so the rows are bit for bit what that kernel would have stored), then the
-    // K loop runs with A out of LDS.
+    // The first steps' rows of W are asked for, then every thread merges fours of elements of A
+    // (the arithmetic of attention_merge, split by split in groups of eight, so the rows are bit
+    // for bit what that kernel would have stored), then the K loop runs with A out of LDS.  Fours,
+    // so that a load names whole lines and one row of 2,048 elements keeps all eight wavefronts at
+    // it; what the launch knows is divided by with a multiplication.  Bound by the trip to what
+    // the attention's other XCDs have written.
 #pragma unroll
     for (int p = 0; p < PD; ++p)
       if (kb0 + p * stride < kfull) load(st[p], kb0 + p * stride, true, false);
-    const int hd = a.merge_hd, splits = a.merge_splits, grp = a.merge_group;
+    typedef float Pair __attribute__((ext_vector_type(2), aligned(4)));
+    const int hd = a.merge_hd, splits = a.merge_splits, grp = a.merge_group, heads = grp * a.merge_nkv;
     const int head_blocks = (grp + 15) / 16;
-    const int pieces = K / 8;
-    bf16x8* rows = (bf16x8*)merged_rows;
-    // U pieces of a thread at a time, the loads of all of them asked for before the first
-    // is used (a piece after the other would cost a trip to memory each), in groups of G
-    // splits: few splits (decode steps of several rows) take four pieces of up to four
-    // splits, many (one or two rows) a piece of eight splits at a time.
-    auto merge_pieces = [&](auto group_size, auto at_a_time) {
+    const int fours = M * (K / 4), row_fours = row_pieces * 2;
+    bf16x4_t* rows = (bf16x4_t*)merged_rows;
+    // U fours of a thread at a time, the loads of all of them asked for before the first is used (one
+    // after the other would cost a trip to memory each), in groups of G splits.
+    auto merge_fours = [&](auto group_size, auto at_a_time) {
       constexpr int G = decltype(group_size)::value, U = decltype(at_a_time)::value;
       constexpr int kThreads = WK * kWave;
-      for (int idx0 = threadIdx.x; idx0 < M * pieces; idx0 += U * kThreads) {
-        int64_t base[U];
-        int used[U], d[U];
-        float ms[U][G], ls[U][G];
-        f32x4 lo4[U][G], hi4[U][G];
+      for (int idx0 = threadIdx.x; idx0 < fours; idx0 += U * kThreads) {
+        unsigned base[U];                  // slot of the first split
+        int d[U], at[U], pos[U];
+        Pair ml[U][G];
+        f32x4 part[U][G];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const int idx = min(idx0 + u * kThreads, M * pieces - 1);     // past the end: the last again
-          const int m = idx / pieces, p8 = idx % pieces;
-          const int head = p8 * 8 / hd;
-          d[u] = p8 * 8 % hd;
-          const int kvh = head / grp, hh = head % grp;
-          base[u] = ((int64_t)((m * a.merge_nkv + kvh) * head_blocks + hh / 16) * splits) * 16 + hh % 16;
-          const int pos = a.merge_pos[m];
-          const int lo = a.merge_window > 0 ? max(0, pos - a.merge_window + 1) : 0;
-          const int nchunks = pos / a.merge_chunk - lo / a.merge_chunk + 1;
-          const int per = (nchunks - 1 + splits) / splits;
-          used[u] = min(splits, (nchunks + per - 1) / per);
+          const int e = min(idx0 + u * kThreads, fours - 1) * 4;        // past the end: the last again
+          const int all = divided(e, hd, a.hd_inv), m = divided(all, heads, a.heads_inv), head = all - m * heads;
+          const int kvh = divided(head, grp, a.group_inv), hh = head - kvh * grp;
+          d[u] = e - all * hd;
+          at[u] = m * row_fours + (e - m * K) / 4;
+          pos[u] = max(a.merge_pos[m], 0);
+          base[u] = (unsigned)((m * a.merge_nkv + kvh) * head_blocks + hh / 16) * splits * 16 + hh % 16;
           // (the first group is asked for without waiting for the position, which says
           // how many splits hold keys at all; an empty one says so itself)
 #pragma unroll
           for (int j = 0; j < G; ++j) {
-            const int64_t slot = base[u] + (int64_t)min(j, splits - 1) * 16;
-            const bool holds = j < splits;
-            ms[u][j] = holds ? a.merge_ml[slot * 2] : -INFINITY;
-            ls[u][j] = holds ? a.merge_ml[slot * 2 + 1] : 0.f;
-            lo4[u][j] = holds ? *(const f32x4*)(a.merge_o + slot * hd + d[u]) : fzero;
-            hi4[u][j] = holds ? *(const f32x4*)(a.merge_o + slot * hd + d[u] + 4) : fzero;
+            const int64_t slot = base[u] + (unsigned)min(j, splits - 1) * 16;
+            ml[u][j] = *(const Pair*)(a.merge_ml + slot * 2);
+            part[u][j] = *(const f32x4*)(a.merge_o + slot * hd + d[u]);
           }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          float mx = -INFINITY, sum = 0.f, o[8] = {};
-          for (int s0 = 0; s0 == 0 || s0 < used[u]; s0 += G) {
+          const int lo = a.merge_window > 0 ? max(0, pos[u] - a.merge_window + 1) : 0;
+          const int chunks = divided(pos[u], a.merge_chunk, a.chunk_inv) - divided(lo, a.merge_chunk, a.chunk_inv);
+          const int per = divided(chunks + splits, splits, a.splits_inv);      // chunks of a split
+          float mx = -INFINITY, sum = 0.f;
+          f32x4 o = fzero;
+          // split s holds keys if s * per <= chunks (a chunk less than there are)
+          for (int s0 = 0; s0 == 0 || (s0 < splits && s0 * per <= chunks); s0 += G) {
             if (s0 > 0) {      // later groups only if they hold keys: every workgroup merges all rows
 #pragma unroll
               for (int j = 0; j < G; ++j) {
-                const int64_t slot = base[u] + (int64_t)min(s0 + j, splits - 1) * 16;
-                const bool holds = s0 + j < used[u];
-                ms[u][j] = holds ? a.merge_ml[slot * 2] : -INFINITY;
-                ls[u][j] = holds ? a.merge_ml[slot * 2 + 1] : 0.f;
-                lo4[u][j] = holds ? *(const f32x4*)(a.merge_o + slot * hd + d[u]) : fzero;
-                hi4[u][j] = holds ? *(const f32x4*)(a.merge_o + slot * hd + d[u] + 4) : fzero;
+                const int64_t slot = base[u] + (unsigned)min(s0 + j, splits - 1) * 16;
+                const bool holds = s0 + j < splits && (s0 + j) * per <= chunks;
+                ml[u][j] = holds ? *(const Pair*)(a.merge_ml + slot * 2) : Pair{-INFINITY, 0.f};
+                part[u][j] = holds ? *(const f32x4*)(a.merge_o + slot * hd + d[u]) : fzero;
               }
             }
             float mg = mx;
 #pragma unroll
-            for (int j = 0; j < G; ++j) mg = (s0 + j < splits) ? fmaxf(mg, ms[u][j]) : mg;
+            for (int j = 0; j < G; ++j) mg = (s0 + j < splits) ? fmaxf(mg, ml[u][j][0]) : mg;
             if (mg == -INFINITY) continue;
             const float keep = __builtin_amdgcn_exp2f(mx - mg);
             sum *= keep;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) o[i] *= keep;
+            for (int i = 0; i < 4; ++i) o[i] *= keep;
 #pragma unroll
             for (int j = 0; j < G; ++j) {
-              const bool live = s0 + j < splits && ms[u][j] != -INFINITY;
-              const float w = live ? __builtin_amdgcn_exp2f(ms[u][j] - mg) : 0.f;
-              sum += live ? ls[u][j] * w : 0.f;
+              const bool live = s0 + j < splits && ml[u][j][0] != -INFINITY;
+              const float w = live ? __builtin_amdgcn_exp2f(ml[u][j][0] - mg) : 0.f;
+              sum += live ? ml[u][j][1] * w : 0.f;
 #pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                o[i] += live ? lo4[u][j][i] * w : 0.f;
-                o[4 + i] += live ? hi4[u][j][i] * w : 0.f;
-              }
+              for (int i = 0; i < 4; ++i) o[i] += live ? part[u][j][i] * w : 0.f;
             }
             mx = mg;
           }
           const float inv = sum > 0.f ? 1.f / sum : 0.f;
-          bf16x8 out;
+          bf16x4_t out;
 #pragma unroll
-          for (int i = 0; i < 8; ++i) out[i] = (bf16_t)(o[i] * inv);
-          const int idx = idx0 + u * kThreads;
-          if (idx < M * pieces) rows[(idx / pieces) * row_pieces + idx % pieces] = out;
+          for (int i = 0; i < 4; ++i) out[i] = (bf16_t)(o[i] * inv);
+          if (idx0 + u * kThreads < fours) rows[at[u]] = out;
         }
       }
     };
-    if (splits <= 4) merge_pieces(std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});
-    else merge_pieces(std::integral_constant<int, 8>{}, std::integral_constant<int, 1>{});
+    if (splits <= 4) merge_fours(std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});
+    else merge_fours(std::integral_constant<int, 8>{}, std::integral_constant<int, 1>{});
     __syncthreads();
 #pragma unroll
     for (int p = 0; p < PD; ++p)
@@ -585,7 +578,7 @@ static inline void launch(const std::conditional_t<CONV, ConvArgs, DirectArgs>& 
 // The merged tail form: dynamic LDS for the rows of A.  Returns false if the device
 // refuses that much.
 template <int WK, int CW, int AR>
-static inline bool launch_merged(const DirectArgs& a, hipStream_t stream) {
+static inline bool launch_merged(const MergedArgs& a, hipStream_t stream) {
   auto kernel = gemm_direct_kernel<1, WK, bf16_t, false, false, 4, 4, false, true, CW, AR, true>;
   const size_t lds = (size_t)AR * (a.K / 8 + 1) * 16;
   static size_t raised = 48 * 1024;      // per instantiation
@@ -610,7 +603,7 @@ static inline int gemm_direct_packed_rows(int M) { return M <= 4 ? 4 : M <= 8 ? 
 int gemm_direct_plain(const DirectArgs& a, int c_type, hipStream_t stream);
 int gemm_direct_conv(const ConvArgs& a, hipStream_t stream);
 int gemm_direct_tail(const DirectArgs& a, hipStream_t stream);
-int gemm_direct_merged(const DirectArgs& a, hipStream_t stream);
+int gemm_direct_merged(const MergedArgs& a, hipStream_t stream);
 int gemm_direct_scaled(const DirectArgs& a, int c_type, bool pair, hipStream_t stream);
 int gemm_direct_pair(const DirectArgs& a, hipStream_t stream);
 int gemm_direct_norm(const DirectArgs& a, int c_type, bool pair, hipStream_t stream);

@@ -8,7 +8,7 @@
 #include "attention_mfma.h"
 #include "gemm_direct_kernel.h"
 
-int gemm_direct_merged(const DirectArgs& a, hipStream_t stream) {
+int gemm_direct_merged(const MergedArgs& a, hipStream_t stream) {
   const bool deep = layout_deep(a.N, a.K);
   const int cw = gemm_direct_columns(a.M, a.N);
   bool ok = true;
@@ -58,12 +58,14 @@ extern "C" int ts_gemm_tail_merged_bf16(const float* partial_o, const float* par
   if (((uintptr_t)prepared) & 7) TS_FAIL("gemm_tail_merged: the prepared rows must be 8-byte aligned");
   if (!partial_o || !partial_ml || !positions || !w || !resid || !norm_w || !prepared || !sumsq)
     TS_FAIL("gemm_tail_merged: null operand");
-  DirectArgs da = {};
+  MergedArgs da = {};
   da.W = (const bf16_t*)w; da.M = M; da.N = N; da.K = nq * hd;
   da.resid = resid; da.tail_w = norm_w; da.prepared = (bf16_t*)prepared; da.sumsq_out = sumsq;
   da.merge_o = partial_o; da.merge_ml = partial_ml; da.merge_pos = positions;
   da.merge_splits = splits; da.merge_nkv = nkv; da.merge_group = nq / nkv; da.merge_hd = hd;
   da.merge_window = window; da.merge_chunk = kChunk;
+  da.heads_inv = inverse32(nq); da.splits_inv = inverse32(splits); da.group_inv = inverse32(nq / nkv);
+  da.hd_inv = inverse32(hd); da.chunk_inv = inverse32(kChunk);
   if (gemm_direct_merged(da, stream)) return -1;
   TS_CHECK_LAUNCH("gemm_tail_merged");
   return 0;
