@@ -193,7 +193,8 @@ __device__ __forceinline__ void load_kv_block_wide(KvBlock<HD>& b, const Attenti
 // a load in about 2 cycles for each 128-byte line that a quarter of its lanes touches: lanes that each
 // ask for 16 bytes of a row of their own take 27 ns a kilobyte, these 8.  It counts where a unit
 // has little more than the loads of a first block to wait for (one request of 541 tokens,
-// 16 / 8 heads of 128: 7.5 -> 7.1 us a launch) and is nothing where memory is the limit.
+// 16 / 8 heads of 128: 7.5 -> 7.1 us a launch); where memory is the limit the way through LDS is a
+// loss of 1 % (attention_decode_kernel's ranked form).
 template <int HD>
 __device__ __forceinline__ void load_kv_block_rows(KvBlock<HD>& b, const AttentionArgs& a, PageCursor& cur,
                                                    int kvh, int v, int stride, int lane) {

@@ -282,10 +282,14 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
   const int key_end = (prep_wave || key_wave) ? 0 : min(c1 * kChunk, last + 1);
   PageCursor cur{(ConstTable)table, a.page_size, last, walk, -1, -1};
   KvBlock<HD> A, B;
-  // head sizes in whole 32-element slices take the blocks with 16-byte value loads
+  // Head sizes in whole 32-element slices take the blocks with 16-byte value loads.  Ranked items are
+  // more than the chip has units and wait for memory, not for a unit's loads: their keys go straight
+  // into the operand's order (64 entries of 100 to 2,047 tokens, whole steps: 2,472 us spread through
+  // LDS, 2,457 straight; of 128 to 4,096 tokens at the 8B shape 1,193 and 1,172).
   constexpr bool kWide = HD % 32 == 0;
   auto load_block = [&](KvBlock<HD>& b, int kb) {
-    if constexpr (kWide) load_kv_block_rows<HD>(b, a, cur, kvh, kb, stride, lane);
+    if constexpr (kWide && RANKED) load_kv_block_wide<HD>(b, a, cur, kvh, kb, stride, r, g);
+    else if constexpr (kWide) load_kv_block_rows<HD>(b, a, cur, kvh, kb, stride, lane);
     else load_kv_block<HD, true>(b, a, table, cur, kvh, kb, stride, r, g);
   };
 
@@ -352,7 +356,7 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
   // a wavefront's keys are spread where its partial sums will stand: nobody else's
   unsigned char* scratch = merge_lds + NW * kWave * 2 * 4 + wave * (16 * merge_row<HD>() * 4);
   auto update = [&](KvBlock<HD>& b, int v) {
-    if constexpr (kWide) spread_keys<HD>(b, scratch, lane);
+    if constexpr (kWide && !RANKED) spread_keys<HD>(b, scratch, lane);
     const int kb = walk.real(v);
     tile_update<HD, false, kWide, EXTRA>(t, b, kb, scale_log2, kb + 31 <= last && kb >= lo, g, &x);
   };
