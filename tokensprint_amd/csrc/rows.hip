@@ -126,28 +126,25 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(float* __restrict__ x,
   __shared__ float scratch[16];
   const int64_t base = (int64_t)blockIdx.x * width;
   const int n4 = width / 4;
-  f32x4_rows v[VPT];
+  // (no load hangs on a condition, past the row's end its last four again: each under one of its own
+  // was waited for before the next was asked for)
+  f32x4_rows v[VPT], d[VPT], wv[VPT];
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) {
+    const int at = min((int)(threadIdx.x + j * blockDim.x), n4 - 1) * 4;
+    v[j] = load4(x + base + at);
+    if (ADD) d[j] = load4(delta + base + at);
+    wv[j] = load4(w + at);
+  }
   float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
-    const int i = threadIdx.x + j * blockDim.x;
-    v[j] = f32x4_rows{0.f, 0.f, 0.f, 0.f};
-    if (i < n4) {
-      v[j] = load4(x + base + i * 4);
-      if (ADD) {
-        const f32x4_rows d = load4(delta + base + i * 4);
+    const bool in = (int)(threadIdx.x + j * blockDim.x) < n4;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[j][e] += d[e];
-      }
+    for (int e = 0; e < 4; ++e) {
+      if (ADD) v[j][e] += d[j][e];
+      ss += in ? v[j][e] * v[j][e] : 0.f;
     }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) ss += v[j][e] * v[j][e];
-  }
-  f32x4_rows wv[VPT];
-#pragma unroll
-  for (int j = 0; j < VPT; ++j) {
-    const int i = threadIdx.x + j * blockDim.x;
-    wv[j] = i < n4 ? load4(w + i * 4) : f32x4_rows{0.f, 0.f, 0.f, 0.f};
   }
   const float rstd = rsqrtf(block_sum(ss, scratch) / (float)width + eps);
 #pragma unroll
