@@ -63,14 +63,14 @@ __global__ __launch_bounds__(256) void conv_silu_run_kernel(
   const float ib = in_bias ? in_bias[c] : 0.f, bc = bias ? bias[c] : 0.f;
   float wk[kConvMaxTaps], raw[kConvRun + kConvMaxTaps - 1];
 #pragma unroll
-  for (int k = 0; k < kConvMaxTaps; ++k) wk[k] = k < taps ? w[c * taps + k] : 0.f;
-  // raw[j]: the input of flat row t0 - (taps - 1) + j (whatever entry it belongs to)
+  for (int k = 0; k < kConvMaxTaps; ++k) wk[k] = w[c * taps + min(k, taps - 1)];
+  // raw[j]: the input of flat row t0 - (taps - 1) + j, whatever entry it belongs to (another row's
+  // where there is none: no output takes that)
 #pragma unroll
-  for (int j = 0; j < kConvRun + kConvMaxTaps - 1; ++j) {
-    const int row = t0 - (taps - 1) + j;
-    raw[j] = (j < kConvRun + taps - 1 && row >= 0 && row < num_tokens)
-                 ? proj[(int64_t)row * ld + col + c] + ib : 0.f;
-  }
+  for (int j = 0; j < kConvRun + kConvMaxTaps - 1; ++j)
+    raw[j] = proj[(int64_t)min(max(t0 - (taps - 1) + j, 0), num_tokens - 1) * ld + col + c];
+#pragma unroll
+  for (int j = 0; j < kConvRun + kConvMaxTaps - 1; ++j) raw[j] += ib;
 #pragma unroll
   for (int i = 0; i < kConvRun; ++i) {
     const int t = t0 + i;
@@ -98,43 +98,46 @@ __global__ __launch_bounds__(256) void conv_silu_run_kernel(
 // tokens and the inputs in front of them are one entry's (30 against 39 us for 2,048 tokens of
 // 6,144 channels).  Four taps are a channel's 16 bytes: one by one, four of 64 lanes' 256 bytes a load, they
 // cost a unit more than the inputs (a load takes 2.1 cycles per line of 128 bytes it names, and sixteen of
-// those named 32 each; 31.3 -> 27.3 us, 4.4 TB/s).  Sixteen tokens a thread: 28.8.
+// those named 32 each; 31.3 -> 27.3 us).  No load hangs on a condition (each was waited for before the
+// next was sent; in a prompt's step 27.9 -> 24.2 us, 4,096 channels 17.7 -> 14.5).
 constexpr int kConvRunTaps = 4;
+template <bool WIDE>        // four taps, and w on 16 bytes
 __global__ __launch_bounds__(256) void conv_silu_run4_kernel(
-    const float* __restrict__ proj, int ld, int col, int channels, int taps,
+    const float* __restrict__ proj, int ld, int col, int channels, int num_taps,
     const float* __restrict__ w, const float* __restrict__ bias, const float* __restrict__ state,
     float* __restrict__ out, BatchView b, int num_tokens, const float* __restrict__ in_bias,
     int plain) {
+  const int taps = WIDE ? kConvRunTaps : num_taps;
   typedef float f32x4 __attribute__((ext_vector_type(4)));
   const int c = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (c >= channels) return;
   const int t0 = blockIdx.y * kConvRun, back0 = taps - 1;
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  const f32x4 ib = in_bias ? *(const f32x4*)(in_bias + c) : zero;
-  const f32x4 bc = bias ? *(const f32x4*)(bias + c) : zero;
-  const bool wide = taps == kConvRunTaps && ((uintptr_t)w & 15) == 0;
+  // (no load hangs on a condition: what is not there is read from a place that is, and dropped)
+  const float* some = proj + col + c;
+  f32x4 ib = *(const f32x4*)(in_bias ? in_bias + c : some), bc = *(const f32x4*)(bias ? bias + c : some);
   f32x4 wk[kConvRunTaps], raw[kConvRun + kConvRunTaps - 1];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    f32x4 of = zero;                  // one channel's
-    if (wide) {
+    f32x4 of;                         // one channel's
+    if constexpr (WIDE) {
       of = *(const f32x4*)(w + (int64_t)(c + j) * kConvRunTaps);
     } else {
 #pragma unroll
-      for (int k = 0; k < kConvRunTaps; ++k)
-        if (k < taps) of[k] = w[(int64_t)(c + j) * taps + k];
+      for (int k = 0; k < kConvRunTaps; ++k) of[k] = w[(int64_t)(c + j) * taps + min(k, taps - 1)];
     }
 #pragma unroll
     for (int k = 0; k < kConvRunTaps; ++k) wk[k][j] = of[k];
   }
-  // raw[j]: the input of flat row t0 - (taps - 1) + j (whatever entry it belongs to)
+  // raw[j]: the input of flat row t0 - (taps - 1) + j, whatever entry it belongs to (another row's
+  // where there is none: no output takes that)
 #pragma unroll
-  for (int j = 0; j < kConvRun + kConvRunTaps - 1; ++j) {
-    const int row = t0 - back0 + j;
-    raw[j] = zero;
-    if (j < kConvRun + back0 && row >= 0 && row < num_tokens)
-      raw[j] = *(const f32x4*)(proj + (int64_t)row * ld + col + c) + ib;
-  }
+  for (int j = 0; j < kConvRun + kConvRunTaps - 1; ++j)
+    raw[j] = *(const f32x4*)(proj + (int64_t)min(max(t0 - back0 + j, 0), num_tokens - 1) * ld + col + c);
+  if (!in_bias) ib = zero;
+  if (!bias) bc = zero;
+#pragma unroll
+  for (int j = 0; j < kConvRun + kConvRunTaps - 1; ++j) raw[j] += ib;
   const int e0 = b.entry_of_token[t0], first0 = b.q_start[e0];
   const bool one = b.entry_of_token[min(t0 + kConvRun, num_tokens) - 1] == e0 && first0 <= t0 - back0;
 #pragma unroll
@@ -184,12 +187,20 @@ __global__ __launch_bounds__(256) void conv_state_kernel(
   const int first = b.q_start[e], n = b.q_start[e + 1] - first;
   const int start = b.positions[first];
   float* st = state + (int64_t)b.slot_ids[e] * (taps - 1) * channels;
-  for (int j = 0; j < taps - 1; ++j) {
-    const int p = start + n - (taps - 1) + j;
-    float v = 0.f;
-    if (p >= start) v = proj[(int64_t)(first + p - start) * ld + col + c] + (in_bias ? in_bias[c] : 0.f);
-    else if (p >= 0) v = st[(int64_t)(j + n) * channels + c];
-    st[(int64_t)j * channels + c] = v;
+  const float ib = in_bias ? in_bias[c] : 0.f;
+  constexpr int kAtOnce = 4;          // rows asked for before the first is written
+  for (int j0 = 0; j0 < taps - 1; j0 += kAtOnce) {
+    float v[kAtOnce];
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u) {
+      const int j = min(j0 + u, taps - 2), p = start + n - (taps - 1) + j;
+      v[u] = *(p >= start ? proj + (int64_t)(first + p - start) * ld + col + c
+                          : st + (int64_t)(j + n) * channels + c);
+      v[u] = p >= start ? v[u] + ib : p >= 0 ? v[u] : 0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u)
+      if (j0 + u < taps - 1) st[(int64_t)(j0 + u) * channels + c] = v[u];
   }
 }
 
@@ -258,7 +269,8 @@ extern "C" int ts_conv_silu(const float* proj, int ld, int col, int channels, in
                      (((uintptr_t)proj | (uintptr_t)out | (uintptr_t)state | (uintptr_t)bias |
                        (uintptr_t)in_bias) & 15) == 0;
   if (quads && num_tokens >= 256 && (num_tokens + kConvRun - 1) / kConvRun <= 65535) {
-    hipLaunchKernelGGL(conv_silu_run4_kernel,
+    const bool wide = taps == kConvRunTaps && ((uintptr_t)w & 15) == 0;
+    hipLaunchKernelGGL((wide ? conv_silu_run4_kernel<true> : conv_silu_run4_kernel<false>),
                        dim3((unsigned)((channels / 4 + 255) / 256),
                             (unsigned)((num_tokens + kConvRun - 1) / kConvRun)),
                        dim3(256), 0, stream, proj, ld, col, channels, taps, w, bias, state, out, b,
