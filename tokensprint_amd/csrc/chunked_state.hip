@@ -34,9 +34,9 @@
 // token at a time (the linear forms in chunks side by side, twice the arithmetic) and were bound
 // by the chain of a token's multiply-adds and sums.  At 2,048 tokens, before and now (alone; in
 // brackets the launches as they run in a prompt's step): delta rule, 16 heads of 128 x 128, 592 and
-// 126 us (solve 37, walk 60, output 37); 8 heads of 64 x 128 with a decay per row 469 and 81 (27,
-// 35, 24); fixed decays, 16 heads of 128 x 128, 230 and 78 (local 29, carry 22, output 44); state
-// space, 64 heads of 128 x 64, 386 and 123 (41, 31, 67), in two launches 99 (29, 77).  The short
+// 125 us (solve 31, walk 61, output 33); 8 heads of 64 x 128 with a decay per row 469 and 76 (21,
+// 36, 19); fixed decays, 16 heads of 128 x 128, 230 and 78 (local 29, carry 22, output 44); state
+// space, 64 heads of 128 x 64, 386 and 123 (41, 31, 67), in two launches 102 (25, 77).  The short
 // chains of product_step and the decays in 64 bits are 1 to 10 us of that.
 //
 // Matrix operands: lane (g, l) = (lane / 16, lane % 16) holds row l of A, column l of B, and rows
@@ -138,55 +138,72 @@ __device__ __forceinline__ void stage_rows(const ChunkedArgs& a, float* dst, int
   constexpr int Q = NP / 4, STEP = kThreads / Q, COUNT = kTok / STEP;
   const int t0 = threadIdx.x / Q, n = threadIdx.x % Q * 4, left = a.N - n;
   const float* row = a.x + (int64_t)first * a.ld + col + n;
-  f32x4 v[COUNT];
+  auto put = [&](int t, f32x4 v) {
+    if (FORM == kSilu) {
 #pragma unroll
-  for (int u = 0; u < COUNT; ++u) {
-    const int t = t0 + u * STEP;
-    v[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (wide) {
-      if (t < nt && left > 0) v[u] = read4(row + (int64_t)t * a.ld);
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (t < nt && left > j) v[u][j] = row[(int64_t)t * a.ld + j];
+      for (int j = 0; j < 4; ++j) v[j] = silu(v[j]);
     }
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  if (FORM == kSilu) {
-#pragma unroll
-    for (int u = 0; u < COUNT; ++u)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) v[u][j] = silu(v[u][j]);
-  }
-  if (FORM == kTurned) {
-#pragma unroll
-    for (int u = 0; u < COUNT; ++u) {
-      const int t = min(t0 + u * STEP, nt - 1);        // (rows behind the last are zeros)
+    if (FORM == kTurned) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        if (n + 2 * j < a.turn_dims) {
-          const float2 c = a.turn[(int64_t)(pos0 + t) * (a.turn_dims / 2) + n / 2 + j];
-          const float even = v[u][2 * j], odd = v[u][2 * j + 1];
-          v[u][2 * j] = fmaf(odd, -c.y, even * c.x);
-          v[u][2 * j + 1] = fmaf(even, c.y, odd * c.x);
+        if (n + 2 * j < a.turn_dims) {                 // (rows behind the last are zeros)
+          const float2 c = a.turn[(int64_t)(pos0 + min(t, nt - 1)) * (a.turn_dims / 2) + n / 2 + j];
+          const float even = v[2 * j], odd = v[2 * j + 1];
+          v[2 * j] = fmaf(odd, -c.y, even * c.x);
+          v[2 * j + 1] = fmaf(even, c.y, odd * c.x);
         }
       }
-      if (key) v[u] *= a.k_scale;
-      __builtin_amdgcn_sched_barrier(0);               // (or every angle is asked for at once)
+      if (key) v *= a.k_scale;
+    }
+    write4(dst + t * (NP + 4) + n, v);
+    if (FORM == kTurned) __builtin_amdgcn_sched_barrier(0);      // (or every angle is asked for at once)
+  };
+  if (wide) {
+    // (no load under a condition of its own: the compiler waits inside it, and what was to be asked for
+    // at once was a trip to memory after the other)
+    const float* from = left > 0 ? row : row - n;
+    f32x4 v[COUNT];
+#pragma unroll
+    for (int u = 0; u < COUNT; ++u) v[u] = read4(from + (int64_t)min(t0 + u * STEP, nt - 1) * a.ld);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < COUNT; ++u) {
+      const int t = t0 + u * STEP;
+      put(t, t < nt && left > 0 ? v[u] : f32x4{0.f, 0.f, 0.f, 0.f});
+    }
+  } else {
+#pragma unroll 1
+    for (int u = 0; u < COUNT; ++u) {
+      const int t = t0 + u * STEP;
+      f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (t < nt && left > j) v[j] = row[(int64_t)t * a.ld + j];
+      put(t, v);
     }
   }
-#pragma unroll
-  for (int u = 0; u < COUNT; ++u) write4(dst + (t0 + u * STEP) * (NP + 4) + n, v[u]);
   __builtin_amdgcn_sched_barrier(0);
 }
 
 // Decays per row of S, gates rows of head h, into dst [64][NP + 4]; ones elsewhere.
 template <int NP>
 __device__ __forceinline__ void stage_decays(const ChunkedArgs& a, float* dst, int h, int first, int nt) {
-  for (int i = threadIdx.x; i < kTok * NP; i += kThreads) {
-    const int t = i / NP, n = i % NP;
-    dst[t * (NP + 4) + n] = t < nt && n < a.N
-        ? a.gates[(int64_t)(first + t) * a.ldg + a.heads + h * a.N + n] : 1.f;
+  constexpr int COUNT = kTok * NP / kThreads, AT_ONCE = COUNT < 16 ? COUNT : 16;
+  static_assert(kTok * NP % kThreads == 0 && COUNT % AT_ONCE == 0, "whole turns");
+  const float* from = a.gates + (int64_t)first * a.ldg + a.heads + h * a.N;
+#pragma unroll 1
+  for (int u0 = 0; u0 < COUNT; u0 += AT_ONCE) {
+    float v[AT_ONCE];
+#pragma unroll
+    for (int u = 0; u < AT_ONCE; ++u) {
+      const int i = threadIdx.x + (u0 + u) * kThreads;
+      v[u] = from[(int64_t)min(i / NP, nt - 1) * a.ldg + min(i % NP, a.N - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < AT_ONCE; ++u) {
+      const int i = threadIdx.x + (u0 + u) * kThreads, t = i / NP, n = i % NP;
+      dst[t * (NP + 4) + n] = t < nt && n < a.N ? v[u] : 1.f;
+    }
   }
 }
 
@@ -946,6 +963,14 @@ __device__ __forceinline__ void solve_chunk(const ChunkedArgs& a, const ChunkRan
     f32x4 X[4];
     const int n = 16 * ct + l, p = n - NP;
     float whole = 1.f;                     // ROW: the decay of the blocks in front
+    float vx[RT][4];                       // a column of v, all of it asked for at once
+    if (ct >= NT) {
+      const float* from = a.x + (int64_t)c.first * a.ld + a.v_col + h * a.P + min(p, a.P - 1);
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) vx[i][r] = from[(int64_t)min(16 * i + 4 * g + r, c.nt - 1) * a.ld];
+    }
 #pragma unroll
     for (int i = 0; i < RT; ++i) {
       f32x4 acc;
@@ -954,8 +979,7 @@ __device__ __forceinline__ void solve_chunk(const ChunkedArgs& a, const ChunkRan
         const int t = 16 * i + 4 * g + r;
         float v;
         if (ct < NT) v = ROW ? Ks[t * LD + n] * whole : Ks[t * LD + n] * dec.d0()[t];
-        else v = t < c.nt && p < a.P
-            ? a.x[(int64_t)(c.first + t) * a.ld + a.v_col + h * a.P + p] : 0.f;
+        else v = t < c.nt && p < a.P ? vx[i][r] : 0.f;
         acc[r] = beta[t] * v;
       }
       if (ROW && ct < NT) whole *= blocks[i * NP + n];
