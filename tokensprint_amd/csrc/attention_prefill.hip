@@ -11,6 +11,7 @@
 #include "attention_core.h"
 
 #include <algorithm>
+#include <exception>
 #include <functional>
 #include <vector>
 
@@ -360,20 +361,25 @@ extern "C" int ts_attention_prefill_plan(int head_dim, int page_size, int rows_p
     return *sets == 4 ? 4 : 8;
   }
   if (entries <= 0 || *std::max_element(q_lens, q_lens + entries) <= 1) return 4;
-  const int tokens16 = 16 / rows_per_token, bins = std::max(1, compute_units() / heads);
-  const std::vector<int> four = item_turns(4 * tokens16, reach, entries, q_lens, starts),
-                         eight = item_turns(8 * tokens16, reach, entries, q_lens, starts);
-  const double of_head = head_dim == 64 ? 0.6 : 1.0;
-  // one set: a unit has two items at a time, which slow one another down
-  const double crowd = std::min(1.0, std::max(0.0, (double)eight.size() / bins - 1.0));
-  double sum = 0.0;
-  for (int n : eight) sum += n;
-  const double one_set = std::max(0.5 + eight[0] * (1.04 + 0.26 * crowd) * of_head,
-                                  (sum * 0.97 * of_head + 0.25 * eight.size()) / bins);
-  const double two_sets = handed_out(eight, bins, 3.0, 0.78 * of_head, 1.05 * of_head);
-  const double four_sets = handed_out(four, bins, 2.0, 0.53 * of_head, 0.68 * of_head);
-  *sets = four_sets < one_set && four_sets < two_sets ? 4 : two_sets < one_set ? 2 : 1;
-  return *sets == 4 ? 4 : 8;
+  try {
+    const int tokens16 = 16 / rows_per_token, bins = std::max(1, compute_units() / heads);
+    const std::vector<int> four = item_turns(4 * tokens16, reach, entries, q_lens, starts),
+                           eight = item_turns(8 * tokens16, reach, entries, q_lens, starts);
+    const double of_head = head_dim == 64 ? 0.6 : 1.0;
+    // one set: a unit has two items at a time, which slow one another down
+    const double crowd = std::min(1.0, std::max(0.0, (double)eight.size() / bins - 1.0));
+    double sum = 0.0;
+    for (int n : eight) sum += n;
+    const double one_set = std::max(0.5 + eight[0] * (1.04 + 0.26 * crowd) * of_head,
+                                    (sum * 0.97 * of_head + 0.25 * eight.size()) / bins);
+    const double two_sets = handed_out(eight, bins, 3.0, 0.78 * of_head, 1.05 * of_head);
+    const double four_sets = handed_out(four, bins, 2.0, 0.53 * of_head, 0.68 * of_head);
+    *sets = four_sets < one_set && four_sets < two_sets ? 4 : two_sets < one_set ? 2 : 1;
+    return *sets == 4 ? 4 : 8;
+  } catch (const std::exception&) {      // no memory for the estimate: any step may take this kernel
+    *sets = 0;
+    return 4;
+  }
 }
 
 int launch_attention_prefill_tall(const AttentionMfmaArgs& args, hipStream_t stream);
