@@ -4,6 +4,7 @@ attention, at the edges of its tiles (32 rows, items of 64 and 128), of its turn
 of pages, with every option that reaches it."""
 
 import ctypes
+import math
 
 import pytest
 import torch
@@ -85,8 +86,8 @@ def test_sinks_and_slopes(ops, gpu_device, form, hd):
 
 
 def test_growing_scores(ops, gpu_device, form):
-    """Scores that rise along the keys by far more than the 2^8 at which sums are rescaled, and fall
-    again: every block brings new largest scores for some rows, or none."""
+    """Scores that rise along the keys, by far more than a weight's range, and fall again: every block
+    brings new largest scores for some rows, or none."""
     nq, nkv, hd, S = 16, 8, 128, 900
     batch, cache, table, _ = paged_scenario(gpu_device, torch.bfloat16, nkv=nkv, hd=hd, page_size=16,
                                             spans=[(0, S)], seed=15)
@@ -105,6 +106,37 @@ def test_growing_scores(ops, gpu_device, form):
         # (a few keys hold most of the weight, so the weights' rounding does not average out: 2^-8 of
         # values up to 4)
         torch.testing.assert_close(got[only].float(), want[only].float(), rtol=2e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("sharpness", [1.0, 3.0, 8.0])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_error_against_float64(ops, gpu_device, form, hd, sharpness):
+    """How far outputs are from float64: the rounding of the result and of the weights, but not of a row's
+    largest weight, which is one.  A relative rounding to 8 bits has a root mean square of
+    2^-7 / sqrt(12) sqrt(E[1 / m^2]), m spread over [1, 2) as a logarithm's: 1.66e-3; errors of different weights
+    add as squares.  (With the largest weight rounded too, rows that few keys dominate are 1.14 to 1.25 times as far.)"""
+    nq, nkv, start, n = 16, 8, 512, 700
+    batch, cache, table, _ = paged_scenario(gpu_device, torch.bfloat16, nkv=nkv, hd=hd, page_size=16,
+                                            spans=[(start, n)], seed=21)
+    q = rand((n, nq, hd), gpu_device, 22, sharpness).bfloat16()
+    got = ops.paged_attention(q, batch, table, cache, num_heads=nq, num_kv_heads=nkv, head_dim=hd,
+                              scale=hd ** -0.5, window=None)
+    pages = table[0, :-(-(start + n) // 16)].long()
+    k = cache.k_pages[pages].double().permute(1, 0, 2, 3).reshape(nkv, -1, hd)[:, :start + n]
+    v = cache.v_pages[pages].double().permute(1, 0, 3, 2).reshape(nkv, -1, hd)[:, :start + n]
+    hidden = (torch.arange(start + n, device=gpu_device)[None, :]
+              > (start + torch.arange(n, device=gpu_device))[:, None])
+    off = size = weights = 0.0
+    for h in range(nq):
+        scores = q[:, h].double() @ k[h // 2].T.contiguous() * hd ** -0.5
+        w = scores.masked_fill(hidden, float("-inf")).softmax(-1)
+        want = w @ v[h // 2]
+        off += (got[:, h].double() - want).square().sum().item()
+        size += want.square().sum().item()
+        w.scatter_(1, w.argmax(1, keepdim=True), 0.0)
+        weights += (w.square() @ v[h // 2].square()).sum().item()
+    rounding = 2.0 ** -7 / 12 ** 0.5 * (0.375 / math.log(2)) ** 0.5
+    assert off ** 0.5 <= 1.05 * rounding * (size + weights) ** 0.5
 
 
 def test_the_same_every_time(ops, gpu_device, form):

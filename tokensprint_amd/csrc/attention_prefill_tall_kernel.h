@@ -2,9 +2,10 @@
 // head sizes 64 and 128, pages of a power of two from 16 up), as a template so that its forms
 // compile in translation units of their own.
 //
-// What bounds it: at 8,192 tokens of 64 query heads, where it runs at 1,100 TFLOP/s (with 16 rows a
-// wavefront 780), the card's power (zeros in place of ordinary data take 812 instead of 1,005 us); at 2,048
-// tokens of 16 the longest item, and 8 us of launch and dependent trips to memory.  Thirty-two rows
+// What bounds it: at 8,192 tokens of 64 query heads, where it takes 1,043 us (1,050 TFLOP/s; with 16 rows
+// a wavefront 1,394), the card's power (before sums were rescaled for every new largest score, zeros in
+// place of ordinary data took 812 instead of 1,005); at 2,048 tokens of 16 (36 us, before 40) the longest
+// item, and 8 us of launch and dependent trips to memory.  Thirty-two rows
 // a wavefront halve what LDS has to read out per product and the softmax's instructions; a row's
 // scores lie in two lanes, so its maximum is one exchange.  The scores of the next block and the values
 // of the one before beside a block's softmax, in one wavefront, was slower (all 256 registers; 1,106 us).
@@ -258,15 +259,18 @@ __device__ __forceinline__ void attention_prefill_tall(const AttentionMfmaArgs& 
 #pragma unroll
       for (int i = 1; i < 16; ++i) mx[b] = max2(mx[b], st[b][i]);
     }
-    // The weights are relative to a score at most 2^8 below the row's largest: what has been
-    // summed is only rescaled for rows that have gone above that, mostly in the first turns.  (A
-    // condition of the lane's, not of the wavefront's: the sums then stay in the registers they are
-    // in, where the compiler would copy all 64 beside a branch that the wavefront takes as one.)
+    // The weights are relative to the row's largest score so far, and what has been summed is rescaled
+    // for rows that have met a larger one.  (A reference left up to 2^8 below it, as published attention
+    // kernels have it, saves most of that, 1,015 us in place of 1,043 at 8,192 tokens of 64 heads, but a row's
+    // largest weight is then no longer the one that bfloat16 holds exactly: rows that few keys dominate
+    // were 1.14 to 1.25 times as far from float64.  A condition of the lane's, not of the wavefront's: the sums
+    // then stay in the registers they are in, where the compiler would copy all 64 beside a branch that the
+    // wavefront takes as one; without a condition 18.5 in place of 18.8 us at 1,024 tokens of 16, 1,072 at the
+    // 8,192 of 64.)
     const float top = halves_max(B == 2 ? max2(mx[0], mx[B - 1]) : mx[0]) * scale_log2;
-    if (top > m + 8.f) {
-      const float m_new = max2(m, top);
-      const float corr = __builtin_amdgcn_exp2f(m - max2(m_new, -1e30f));
-      m = m_new;
+    if (top > m) {
+      const float corr = __builtin_amdgcn_exp2f(m - max2(top, -1e30f));
+      m = top;
       l *= corr;
 #pragma unroll
       for (int db = 0; db < DB; ++db)
