@@ -425,7 +425,7 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
       float M = mw[0];
 #pragma unroll
       for (int w = 1; w < NW; ++w) M = fmaxf(M, mw[w]);
-      const float Mc = fmaxf(M, -1e30f);
+      const float Mc = M == -INFINITY ? 0.f : M;      // (no key: all weights are 0)
       float acc = 0.f, sum = 0.f;
 #pragma unroll
       for (int w = 0; w < NW; ++w) {
