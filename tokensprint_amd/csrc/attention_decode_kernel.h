@@ -113,47 +113,67 @@ __device__ __forceinline__ float load_past_caches(const float* p) {
 // The merge of attention_merge_kernel (same order, same arithmetic per element, so the same
 // bits) by the THREADS threads of one workgroup, over the `used` first splits of one item:
 // slot (first_slot + split * 16 + row) holds a row's statistics and HD partial sums.  A
-// thread takes an element and asks for all of a group of GROUP splits before it uses the first:
-// the workgroup's last act, bound by one trip to memory and by its instructions (two elements a
-// thread and always eight splits: 1.5 us of 10.9 for four splits of 2 rows of 128, now 0.8).
-template <int HD, int THREADS, int GROUP>
+// thread takes E elements and asks for all of a group of GROUP splits of each before it uses the first:
+// the workgroup's last act, bound by its trips to memory and by its instructions (two elements a
+// thread and always eight splits: 1.5 us of 10.9 for four splits of 2 rows of 128, with one and four 0.8;
+// where a thread has more than one, one at a time is a trip each: 16 query heads of 128 over one key/value head,
+// 2,000 tokens, 15.4 us, now 14.6).
+template <int HD, int THREADS, int GROUP, int E>
 __device__ __forceinline__ void merge_splits_here(const float* partial_o, const float* partial_ml,
                                                   int64_t first_slot, int used, int rows, bf16_t* out,
                                                   const float* sink = nullptr, int first_head = 0) {
   partial_o += first_slot * HD;
   partial_ml += first_slot * 2;
-  for (int e = threadIdx.x; e < rows * HD; e += THREADS) {
-    const int row = e / HD, d = e % HD;
-    float M = -INFINITY, L = 0.f, acc = 0.f;
-    for (int s0 = 0; s0 < used; s0 += GROUP) {
-      float ms[GROUP], ls[GROUP], part[GROUP];
+  const int count = rows * HD;
+  for (int e0 = threadIdx.x; e0 < count; e0 += E * THREADS) {
+    int row[E], d[E];
+    float M[E], L[E], acc[E];
 #pragma unroll
-      for (int j = 0; j < GROUP; ++j) {
-        const unsigned slot = min(s0 + j, used - 1) * 16 + row;
-        const uint64_t ml = __hip_atomic_load((const uint64_t*)partial_ml + slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        ms[j] = __uint_as_float((unsigned)ml);
-        ls[j] = __uint_as_float((unsigned)(ml >> 32));
-        part[j] = load_past_caches(partial_o + slot * HD + d);
-      }
-      float Mg = M;
-#pragma unroll
-      for (int j = 0; j < GROUP; ++j) Mg = (s0 + j < used) ? fmaxf(Mg, ms[j]) : Mg;
-      if (Mg == -INFINITY) continue;
-      const float keep = __builtin_amdgcn_exp2f(M - Mg);
-      L *= keep;
-      acc *= keep;
-#pragma unroll
-      for (int j = 0; j < GROUP; ++j) {
-        const bool live = s0 + j < used && ms[j] != -INFINITY;
-        const float w = live ? __builtin_amdgcn_exp2f(ms[j] - Mg) : 0.f;
-        L += live ? ls[j] * w : 0.f;
-        acc += live ? part[j] * w : 0.f;
-      }
-      M = Mg;
+    for (int k = 0; k < E; ++k) {
+      const int e = E == 1 ? e0 : min(e0 + k * THREADS, count - 1);    // past the end: the last again, not stored
+      row[k] = e / HD;
+      d[k] = e % HD;
+      M[k] = -INFINITY;
+      L[k] = acc[k] = 0.f;
     }
-    const float sum = sum_with_sink(L, M, sink, first_head + row);
-    const float inv = sum > 0.f ? 1.f / sum : 0.f;
-    out[(int64_t)row * HD + d] = (bf16_t)(acc * inv);
+    for (int s0 = 0; s0 < used; s0 += GROUP) {
+      float ms[E][GROUP], ls[E][GROUP], part[E][GROUP];
+#pragma unroll
+      for (int j = 0; j < GROUP; ++j)
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+          const unsigned slot = min(s0 + j, used - 1) * 16 + row[k];
+          const uint64_t ml = __hip_atomic_load((const uint64_t*)partial_ml + slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          ms[k][j] = __uint_as_float((unsigned)ml);
+          ls[k][j] = __uint_as_float((unsigned)(ml >> 32));
+          part[k][j] = load_past_caches(partial_o + slot * HD + d[k]);
+        }
+#pragma unroll
+      for (int k = 0; k < E; ++k) {
+        float Mg = M[k];
+#pragma unroll
+        for (int j = 0; j < GROUP; ++j) Mg = (s0 + j < used) ? fmaxf(Mg, ms[k][j]) : Mg;
+        if (Mg == -INFINITY) continue;
+        const float keep = __builtin_amdgcn_exp2f(M[k] - Mg);
+        L[k] *= keep;
+        acc[k] *= keep;
+#pragma unroll
+        for (int j = 0; j < GROUP; ++j) {
+          const bool live = s0 + j < used && ms[k][j] != -INFINITY;
+          const float w = live ? __builtin_amdgcn_exp2f(ms[k][j] - Mg) : 0.f;
+          L[k] += live ? ls[k][j] * w : 0.f;
+          acc[k] += live ? part[k][j] * w : 0.f;
+        }
+        M[k] = Mg;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < E; ++k) {
+      if (E > 1 && e0 + k * THREADS >= count) break;
+      const float sum = sum_with_sink(L[k], M[k], sink, first_head + row[k]);
+      const float inv = sum > 0.f ? 1.f / sum : 0.f;
+      out[(int64_t)row[k] * HD + d[k]] = (bf16_t)(acc[k] * inv);
+    }
   }
 }
 
@@ -517,12 +537,20 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
   if (threadIdx.x == 0)
     __hip_atomic_store(args.arrivals + item, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   bf16_t* out = (bf16_t*)a.out + ((int64_t)token * a.nq + kvh * group + hb * 16) * HD;
-  auto merge = [&](auto at_once) {
-    merge_splits_here<HD, NW * kWave, decltype(at_once)::value>(ma.partial_o, ma.partial_ml, (int64_t)item * ma.num_splits * 16,
-                                                                used, rows, out, a.sink, kvh * group + hb * 16);
+  auto merge = [&](auto at_once, auto each) {
+    merge_splits_here<HD, NW * kWave, decltype(at_once)::value, decltype(each)::value>(
+        ma.partial_o, ma.partial_ml, (int64_t)item * ma.num_splits * 16, used, rows, out, a.sink, kvh * group + hb * 16);
   };
-  if (used <= 4) merge(std::integral_constant<int, 4>());
-  else merge(std::integral_constant<int, 8>());
+  constexpr std::integral_constant<int, 1> one;
+  constexpr std::integral_constant<int, 4> four;
+  constexpr std::integral_constant<int, 8> eight;
+  if (rows * HD <= NW * kWave) {
+    if (used <= 4) merge(four, one);
+    else merge(eight, one);
+  } else {
+    if (used <= 4) merge(four, four);
+    else merge(eight, std::integral_constant<int, 2>());
+  }
 }
 
 int launch_attention_merge(const AttentionMfmaArgs& args, hipStream_t stream);
