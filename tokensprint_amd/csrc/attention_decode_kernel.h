@@ -305,10 +305,14 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
   // Head sizes in whole 32-element slices take the blocks with 16-byte value loads.  Ranked items are
   // more than the chip has units and wait for memory, not for a unit's loads: their keys go straight
   // into the operand's order (64 entries of 100 to 2,047 tokens, whole steps: 2,472 us spread through
-  // LDS, 2,457 straight; of 128 to 4,096 tokens at the 8B shape 1,193 and 1,172).
-  constexpr bool kWide = HD % 32 == 0;
+  // LDS, 2,457 straight; of 128 to 4,096 tokens at the 8B shape 1,193 and 1,172).  Above 128 it is the
+  // registers of two blocks that count, and what is left for the compiler to send loads ahead with: us
+  // straight / through LDS, 40 entries of 2,500 tokens, ranked (8 key/value heads) 160 113 / 98, 192 123 / 117, 224
+  // 143 / 138, 256 173 / 161; 20 entries of 8 heads or 40 of 4, not ranked, 160 56 / 61, 192 84 / 81, 224 112 / 113,
+  // 256, one request of 800, 25 / 23.
+  constexpr bool kWide = HD % 32 == 0, kStraight = RANKED ? HD <= 128 : HD == 160 || HD == 224;
   auto load_block = [&](KvBlock<HD>& b, int kb) {
-    if constexpr (kWide && RANKED) load_kv_block_wide<HD>(b, a, cur, kvh, kb, stride, r, g);
+    if constexpr (kWide && kStraight) load_kv_block_wide<HD>(b, a, cur, kvh, kb, stride, r, g);
     else if constexpr (kWide) load_kv_block_rows<HD>(b, a, cur, kvh, kb, stride, lane);
     else load_kv_block<HD, true>(b, a, table, cur, kvh, kb, stride, r, g);
   };
@@ -376,7 +380,7 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
   // a wavefront's keys are spread where its partial sums will stand: nobody else's
   unsigned char* scratch = merge_lds + NW * kWave * 2 * 4 + wave * (16 * merge_row<HD>() * 4);
   auto update = [&](KvBlock<HD>& b, int v) {
-    if constexpr (kWide && !RANKED) spread_keys<HD>(b, scratch, lane);
+    if constexpr (kWide && !kStraight) spread_keys<HD>(b, scratch, lane);
     const int kb = walk.real(v);
     tile_update<HD, false, kWide, EXTRA>(t, b, kb, scale_log2, kb + 31 <= last && kb >= lo, g, &x);
   };
