@@ -3,13 +3,18 @@
 #include "common.h"
 
 // ---------------------------------------------------------------- embedding
-// (In fours, 64 rows of 4,096: 9.8 -> 4.8 us, 8,192 of 5,120: 77.7 -> 42.9.)
+// (In fours, 64 rows of 4,096: 9.8 -> 4.8 us, 8,192 of 5,120: 77.7 -> 42.9.  Other rows an element at a time:
+// by eights with a condition each 2,048 of 8,190 took 21.7 us, so 19.1.)
 template <typename TW, bool QUADS>
 __global__ __launch_bounds__(256) void embed_kernel(const TW* __restrict__ table, const int* __restrict__ ids,
                                                     float* __restrict__ out, int width, float scale) {
   const int64_t t = blockIdx.x;
   const TW* row = table + (int64_t)ids[t] * width;
   float* o = out + t * width;
+  if constexpr (!QUADS) {
+    for (int i = threadIdx.x; i < width; i += blockDim.x) o[i] = to_f32(row[i]) * scale;
+    return;
+  }
   for (int begin = 0; begin < width; begin += kRowItems * blockDim.x) {
     const RowShare<QUADS> share{width - begin};
     float v[kRowItems];
@@ -26,9 +31,12 @@ extern "C" int ts_embed(const void* table, int table_type, int vocab, const int*
                         hipStream_t stream) {
   if (num_tokens <= 0) return 0;
   if (width <= 0 || vocab <= 0) TS_FAIL("embed: bad sizes width=%d vocab=%d", width, vocab);
+  const bool quads = rows_in_fours(width, table, out);
+  // (fours: eight elements a thread, of narrow rows no more wavefronts than these take)
+  const int threads = !quads || width > 3 * 64 * kRowItems ? 256 : (width + 64 * kRowItems - 1) / (64 * kRowItems) * 64;
   TS_DISPATCH_TYPE(table_type, TW,
-                   hipLaunchKernelGGL((rows_in_fours(width, table, out) ? embed_kernel<TW, true> : embed_kernel<TW, false>),
-                                      dim3(num_tokens), dim3(256), 0, stream, (const TW*)table, ids, out, width, scale));
+                   hipLaunchKernelGGL((quads ? embed_kernel<TW, true> : embed_kernel<TW, false>), dim3(num_tokens),
+                                      dim3(threads), 0, stream, (const TW*)table, ids, out, width, scale));
   TS_CHECK_LAUNCH("embed");
   return 0;
 }

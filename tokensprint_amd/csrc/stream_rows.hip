@@ -35,9 +35,10 @@ extern "C" int ts_stream_add(float* resid, const void* a, int a_type, const void
 
 // The same sum, and the RMS norm of the new stream: out = resid / sqrt(mean(resid^2) + eps) * w.
 // One workgroup a row; the row's values wait in registers between the two passes (up to
-// eight a thread), or are read back.
+// eight a thread), or are read back.  (Eight wavefronts a SIMD: an element at a time would take 68 registers,
+// and 2,048 rows of 4,098 23.8 us in place of 20.9.)
 template <typename TA, typename TB, typename TO, bool QUADS>
-__global__ __launch_bounds__(256) void stream_add_norm_kernel(
+__global__ __launch_bounds__(256, 8) void stream_add_norm_kernel(
     float* __restrict__ resid, const TA* __restrict__ a, const TB* __restrict__ b,
     const float* __restrict__ row, int row_stride, const float* __restrict__ w,
     TO* __restrict__ out, int width, float eps) {
