@@ -30,7 +30,7 @@ def test_norms_of_rows(gpu_device, dtype, width):
     torch.testing.assert_close(got, want, **tol)
 
 
-@pytest.mark.parametrize("taps", [2, 4, 5, 6, 8, 9])
+@pytest.mark.parametrize("taps", [2, 3, 4, 5, 6, 8, 9])
 @pytest.mark.parametrize("shifted", [False, True])
 @pytest.mark.parametrize("bias", [False, True])
 def test_convolution_taps(gpu_device, taps, shifted, bias):

@@ -99,45 +99,46 @@ __global__ __launch_bounds__(256) void conv_silu_run_kernel(
 // 6,144 channels).  Four taps are a channel's 16 bytes: one by one, four of 64 lanes' 256 bytes a load, they
 // cost a unit more than the inputs (a load takes 2.1 cycles per line of 128 bytes it names, and sixteen of
 // those named 32 each; 31.3 -> 27.3 us).  No load hangs on a condition (each was waited for before the
-// next was sent; in a prompt's step 27.9 -> 24.2 us, 4,096 channels 17.7 -> 14.5).
+// next was sent; in a prompt's step 27.9 -> 24.2 us, 4,096 channels 17.7 -> 14.5), and there are no more of
+// them than TAPS taps take.
 constexpr int kConvRunTaps = 4;
-template <bool WIDE>        // four taps, and w on 16 bytes
+template <int TAPS, bool WIDE>        // WIDE: four taps, and w on 16 bytes
 __global__ __launch_bounds__(256) void conv_silu_run4_kernel(
-    const float* __restrict__ proj, int ld, int col, int channels, int num_taps,
-    const float* __restrict__ w, const float* __restrict__ bias, const float* __restrict__ state,
-    float* __restrict__ out, BatchView b, int num_tokens, const float* __restrict__ in_bias,
-    int plain) {
-  const int taps = WIDE ? kConvRunTaps : num_taps;
+    const float* __restrict__ proj, int ld, int col, int channels, const float* __restrict__ w,
+    const float* __restrict__ bias, const float* __restrict__ state, float* __restrict__ out, BatchView b,
+    int num_tokens, const float* __restrict__ in_bias, int plain) {
+  static_assert(!WIDE || TAPS == 4, "a channel's taps in one load");
   typedef float f32x4 __attribute__((ext_vector_type(4)));
   const int c = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (c >= channels) return;
-  const int t0 = blockIdx.y * kConvRun, back0 = taps - 1;
+  const int t0 = blockIdx.y * kConvRun;
+  constexpr int back0 = TAPS - 1;
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   // (no load hangs on a condition: what is not there is read from a place that is, and dropped)
   const float* some = proj + col + c;
   f32x4 ib = *(const f32x4*)(in_bias ? in_bias + c : some), bc = *(const f32x4*)(bias ? bias + c : some);
-  f32x4 wk[kConvRunTaps], raw[kConvRun + kConvRunTaps - 1];
+  f32x4 wk[TAPS], raw[kConvRun + back0];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     f32x4 of;                         // one channel's
     if constexpr (WIDE) {
-      of = *(const f32x4*)(w + (int64_t)(c + j) * kConvRunTaps);
+      of = *(const f32x4*)(w + (int64_t)(c + j) * TAPS);
     } else {
 #pragma unroll
-      for (int k = 0; k < kConvRunTaps; ++k) of[k] = w[(int64_t)(c + j) * taps + min(k, taps - 1)];
+      for (int k = 0; k < TAPS; ++k) of[k] = w[(int64_t)(c + j) * TAPS + k];
     }
 #pragma unroll
-    for (int k = 0; k < kConvRunTaps; ++k) wk[k][j] = of[k];
+    for (int k = 0; k < TAPS; ++k) wk[k][j] = of[k];
   }
-  // raw[j]: the input of flat row t0 - (taps - 1) + j, whatever entry it belongs to (another row's
+  // raw[j]: the input of flat row t0 - (TAPS - 1) + j, whatever entry it belongs to (another row's
   // where there is none: no output takes that)
 #pragma unroll
-  for (int j = 0; j < kConvRun + kConvRunTaps - 1; ++j)
+  for (int j = 0; j < kConvRun + back0; ++j)
     raw[j] = *(const f32x4*)(proj + (int64_t)min(max(t0 - back0 + j, 0), num_tokens - 1) * ld + col + c);
   if (!in_bias) ib = zero;
   if (!bias) bc = zero;
 #pragma unroll
-  for (int j = 0; j < kConvRun + kConvRunTaps - 1; ++j) raw[j] += ib;
+  for (int j = 0; j < kConvRun + back0; ++j) raw[j] += ib;
   const int e0 = b.entry_of_token[t0], first0 = b.q_start[e0];
   const bool one = b.entry_of_token[min(t0 + kConvRun, num_tokens) - 1] == e0 && first0 <= t0 - back0;
 #pragma unroll
@@ -147,8 +148,7 @@ __global__ __launch_bounds__(256) void conv_silu_run4_kernel(
     f32x4 acc = bc;
     if (one) {
 #pragma unroll
-      for (int k = 0; k < kConvRunTaps; ++k) {
-        if (k >= taps) break;
+      for (int k = 0; k < TAPS; ++k) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[j] = fmaf(wk[k][j], raw[i + k][j], acc[j]);
       }
@@ -157,8 +157,7 @@ __global__ __launch_bounds__(256) void conv_silu_run4_kernel(
       const int first = b.q_start[e], pos = b.positions[t];
       const float* st = state + (int64_t)b.slot_ids[e] * back0 * channels;
 #pragma unroll
-      for (int k = 0; k < kConvRunTaps; ++k) {
-        if (k >= taps) break;
+      for (int k = 0; k < TAPS; ++k) {
         const int back = back0 - k;
         if (pos - back < 0) continue;
         const f32x4 v = t - back >= first
@@ -270,11 +269,15 @@ extern "C" int ts_conv_silu(const float* proj, int ld, int col, int channels, in
                        (uintptr_t)in_bias) & 15) == 0;
   if (quads && num_tokens >= 256 && (num_tokens + kConvRun - 1) / kConvRun <= 65535) {
     const bool wide = taps == kConvRunTaps && ((uintptr_t)w & 15) == 0;
-    hipLaunchKernelGGL((wide ? conv_silu_run4_kernel<true> : conv_silu_run4_kernel<false>),
-                       dim3((unsigned)((channels / 4 + 255) / 256),
-                            (unsigned)((num_tokens + kConvRun - 1) / kConvRun)),
-                       dim3(256), 0, stream, proj, ld, col, channels, taps, w, bias, state, out, b,
-                       num_tokens, in_bias, plain);
+    const auto kernel = wide        ? conv_silu_run4_kernel<4, true>
+                        : taps == 4 ? conv_silu_run4_kernel<4, false>
+                        : taps == 3 ? conv_silu_run4_kernel<3, false>
+                        : taps == 2 ? conv_silu_run4_kernel<2, false>
+                                    : conv_silu_run4_kernel<1, false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((channels / 4 + 255) / 256),
+                                    (unsigned)((num_tokens + kConvRun - 1) / kConvRun)),
+                       dim3(256), 0, stream, proj, ld, col, channels, w, bias, state, out, b, num_tokens, in_bias,
+                       plain);
     TS_CHECK_LAUNCH("conv_silu (runs of four channels)");
   } else if (taps <= kConvMaxTaps && num_tokens >= 256 && (num_tokens + kConvRun - 1) / kConvRun <= 65535) {
     hipLaunchKernelGGL(conv_silu_run_kernel,
