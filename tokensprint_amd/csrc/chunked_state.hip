@@ -172,13 +172,15 @@ __device__ __forceinline__ void stage_rows(const ChunkedArgs& a, float* dst, int
       put(t, t < nt && left > 0 ? v[u] : f32x4{0.f, 0.f, 0.f, 0.f});
     }
   } else {
-#pragma unroll 1
+#pragma unroll 2
     for (int u = 0; u < COUNT; ++u) {
       const int t = t0 + u * STEP;
-      f32x4 v = {0.f, 0.f, 0.f, 0.f};
+      const float* from = row - n + (int64_t)min(t, nt - 1) * a.ld;
+      f32x4 v;
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (t < nt && left > j) v[j] = row[(int64_t)t * a.ld + j];
+      for (int j = 0; j < 4; ++j) v[j] = from[min(n + j, a.N - 1)];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = t < nt && left > j ? v[j] : 0.f;
       put(t, v);
     }
   }
