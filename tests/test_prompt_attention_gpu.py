@@ -5,6 +5,7 @@ of pages, with every option that reaches it."""
 
 import ctypes
 import math
+import time
 
 import pytest
 import torch
@@ -168,3 +169,46 @@ def test_which_form(ops):
     assert plan([1] * 200, [4000] * 200) == (4, 0)
     assert plan([1024], [0], head_dim=96) == (4, 0)
     assert plan([1024], [0], page=24) == (1, 0)
+
+
+def plan_of(ops, q_lens, starts, head_dim=128, heads=8, rows=2, scores=False):
+    n, sets = len(q_lens), ctypes.c_int(-1)
+    choose = ops.lib.ts_attention_prefill_plan_scores if scores else ops.lib.ts_attention_prefill_plan
+    tiles = choose(head_dim, 16, rows, heads, 0, n, (ctypes.c_int * n)(*q_lens), (ctypes.c_int * n)(*starts),
+                   ctypes.byref(sets))
+    return tiles, sets.value
+
+
+@pytest.mark.parametrize("lanes, ctx, portion", [(200, 300, 33), (400, 300, 33), (200, 300, 256), (400, 1500, 33)])
+def test_single_tokens_are_most_of_the_work(ops, lanes, ctx, portion):
+    """A portion beside many single tokens does not take their kernel from them; it does where it is most
+    of the work, or where scores are more than a product and that kernel is the slower one."""
+    for head_dim in (64, 128):
+        q_lens, starts = [1] * lanes + [portion], [ctx] * lanes + [0]
+        assert plan_of(ops, q_lens, starts, head_dim) == (4, 0)
+        assert plan_of(ops, [1] * 12 + [2000], [ctx] * 12 + [0], head_dim)[1] > 0
+    assert plan_of(ops, q_lens, starts, 128, scores=True)[1] > 0
+    if ctx == 300:
+        assert plan_of(ops, q_lens, starts, 64, scores=True) == (4, 0)
+
+
+def test_what_a_plan_costs(ops):
+    """Many items for many units (one key/value head): each goes to the unit that is free first out of a
+    heap, where a look at all units for every item took 0.8 to 1.2 ms."""
+    for q_lens, starts in (([1] * 1000 + [33], list(range(1000)) + [0]), ([8192], [0])):
+        least = float("inf")
+        for _ in range(20):
+            t = time.perf_counter()
+            plan_of(ops, q_lens, starts, heads=1, rows=16)
+            least = min(least, time.perf_counter() - t)
+        assert least < 5e-4
+
+
+@pytest.mark.parametrize("nq, nkv, hd", [(16, 8, 64), (16, 8, 128), (24, 3, 64)])
+@pytest.mark.parametrize("options", [{}, dict(window=40, keep_first=5), dict(softcap=3.0)], ids=str)
+def test_many_single_tokens_beside_a_portion(ops, gpu_device, nq, nkv, hd, options):
+    spans = [((37 * i) % 600, 1) for i in range(210)] + [(130, 45), (0, 33)]
+    if not options:
+        rows = nq // nkv
+        assert plan_of(ops, [n for _, n in spans], [s for s, _ in spans], hd, nkv, rows) == (4, 0) or nkv == 3
+    check(ops, gpu_device, nq, nkv, hd, 16, spans, **options)

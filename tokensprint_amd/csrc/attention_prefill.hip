@@ -11,8 +11,8 @@
 #include "attention_core.h"
 
 #include <algorithm>
+#include <cmath>
 #include <exception>
-#include <functional>
 #include <vector>
 
 template <int HD, int TPW, bool PAGE16>
@@ -139,10 +139,10 @@ __device__ __forceinline__ void lds_dma16(const void* src, void* dst) {
                : "memory", "m0");
 }
 
-// Steps of single tokens take it (a workgroup's four waves walk one request's keys with one row
-// each in use, three workgroups a unit): there it waits for memory, and tiles of 32 rows, two
-// workgroups a unit, are behind (136 entries of 300 tokens 29 against 34 us, 200 of 4,000 575
-// against 588).
+// Steps of single tokens take it, and those in which single tokens are most of the work (a workgroup's four
+// waves walk one request's keys with one row each in use, three workgroups a unit): there it waits for
+// memory, and tiles of 32 rows, two workgroups a unit, are behind (136 entries of 300 tokens 29 against
+// 34 us, 200 of 4,000 575 against 588).
 template <int HD>
 __global__ __launch_bounds__(256, 3) void attention_prefill_async_kernel(AttentionMfmaArgs args) {
   constexpr int KS = HD / 32, DB = HD / 16;
@@ -292,7 +292,7 @@ __global__ __launch_bounds__(256, 3) void attention_prefill_async_kernel(Attenti
 constexpr int tiles_per_wave(int hd) { return hd <= 32 ? 4 : (hd <= 64 ? 2 : 1); }
 
 // Which kernel takes the long portions of head sizes 64 and 128 (so that tests reach each at small
-// sizes).  2 (the default): the rule below; 0: turns of 32 keys everywhere; 3, 4, 5: the kernel of 32
+// sizes).  2, as any other value: the rule below; 0: turns of 32 keys everywhere; 3, 4, 5: the kernel of 32
 // rows a wavefront with one set, two and four.
 static int g_prefill_variant = 2;
 extern "C" void ts_attention_prefill_variant(int v) { g_prefill_variant = v; }
@@ -300,86 +300,142 @@ extern "C" void ts_attention_prefill_variant(int v) { g_prefill_variant = v; }
 // What a step's portions are cut into: 16-row tiles per work item (the returned number) and, where
 // the kernel of 32 rows a wavefront takes them, sets of wavefronts that split an item's keys (`sets`,
 // else 0).  `q_lens` and `starts` are the entries' tokens and first positions, `reach` the keys that a
-// query sees at most (0: all), `heads` the key/value heads (x blocks of 16 query heads).
+// query sees at most (0: all), `heads` the key/value heads (x blocks of 16 query heads); `extras`, the second
+// entry point's: scores are more than scale times the product.
 //
 // The forms of that kernel: eight tiles an item in one set (two workgroups a unit, the best rate), eight
 // tiles in two sets (half the time for a long item), four tiles in four sets (a quarter, for
 // portions that would leave units without an item, at two thirds of the rate, since half as many rows share
-// what the unit loads).  A step takes the one with the smallest estimate: 7 us for launch, first trips to
-// memory and stores, a part per item, and its turns of 64 keys, which take longer where a unit has
-// items on end (`together_us`) than where it has one (`alone_us`); items go to the units of a head's
-// share of the chip longest first, each to the one that is free first, as the hardware hands them out.
-// At 16 query and 8 key/value heads of 128, in us (one set / two / four / the kernels of 16 rows a
-// wavefront that were there before): 300 tokens 11.0 / 11.5 / 10.7 / 10.9, 1,024 23.3 / 21.2 / 16.3 / 17.9,
-// 2,048 41.6 / 35.0 / 31.8 / 34.4, 2,600 52.1 / 42.7 / 52.2 / 58.3, 4,096 89.1 / 78.5 / 101 / 107, 5,600 135 / 149 / 179
-// / 206, 8,192 279 / 279 / 352 / 379; three of 683 18.8 / 17.7 / 25.0 / 20.5; 64 query heads, 512 tokens 15.2 / 15.4 /
-// 18.0 / 17.0, 2,048 78.8 / 90.3 / 120 / 111, 8,192 998 (1,100 TFLOP/s) / 1,118 / 1,409 / 1,405; 32 query heads, 1,000
-// tokens behind 2,048 beside 30 single tokens 70.9 / 76.9 / 84.6 / 84.2.  Of 126 such steps the choice is the
-// fastest or within four per cent of it in 121, and 0.4 per cent behind it in the mean.
+// what the unit loads).  Beside them the kernel of 16 rows a wavefront (three workgroups a unit), for steps in
+// which single tokens are most of the work: those wait for memory, and it is the fewer rows of an item and the
+// more workgroups that count.  A step takes the form with the smallest estimate.
+//
+// An estimate is launch and first trips to memory, then its items handed out to the units of a head's
+// share of the chip, longest first, each to the one that is free first, as the hardware does it; where a unit
+// holds several workgroups, or has four items and more, the items' mean share of a unit or the longest
+// item, whichever is more.  An item takes its turns of 64 keys (of a portion: the products', longer where units
+// have items on end than alone; of a single token: the memory's, the same in every form) and a part of its own.
+// The numbers are fitted to the times of 755 steps (prompts, and single tokens beside portions; 2 to 16 key/value
+// heads of 64 and 128): the choice is the fastest form or within 4 per cent of it in 735, 0.4 per cent behind
+// it in the mean; of 100 steps of random sizes that were timed afterwards in 98, 0.3.
+// In us, one set / two / four / 16 rows: 16 and 8 heads of 128, 300 tokens 12.3 / 12.6 / 11.3 / 11.9, 2,048
+// 47 / 40 / 36 / 50, 4,096 97 / 84 / 107 / 103, 8,192 286 / 303 / 382 / 370; 64 query heads, 8,192
+// 1,009 / 1,136 / 1,410 / 1,326; 200 single tokens of 300 beside 33 tokens, 16 and 8 heads of 128
+// 56 / 78 / 72 / 49, of 64 34 / 54 / 48 / 27; 400 of 1,500 beside 2,000
+// 433 / 461 / 450 / 423 and 226 / 276 / 263 / 218.
 namespace {
-// Turns of 64 keys of the step's items of so many tokens at most, most first.
-std::vector<int> item_turns(int tokens, int reach, int entries, const int* q_lens, const int* starts) {
-  std::vector<int> turns;
+struct Item {
+  int turns;        // of 64 keys
+  bool single;      // of an entry of one token
+};
+
+// A step's items of so many tokens at most, longest first.
+std::vector<Item> items_of(int tokens, int reach, int entries, const int* q_lens, const int* starts) {
+  std::vector<Item> items;
   for (int e = 0; e < entries; ++e)
     for (int t = 0; t < q_lens[e]; t += tokens) {
       const int n = t + tokens < q_lens[e] ? tokens : q_lens[e] - t;
       int keys = starts[e] + t + n;
       if (reach > 0 && keys - n > reach) keys = reach + n;
-      turns.push_back((keys + 63) / 64);
+      items.push_back({(keys + 63) / 64, q_lens[e] == 1});
     }
-  std::sort(turns.begin(), turns.end(), std::greater<int>());
-  return turns;
+  std::stable_sort(items.begin(), items.end(), [](const Item& a, const Item& b) { return a.turns > b.turns; });
+  return items;
 }
 
-double handed_out(const std::vector<int>& turns, int bins, double item_us, double alone_us, double together_us) {
-  if ((int64_t)turns.size() > 8 * (int64_t)bins) {
-    double sum = 0.0;
-    for (int n : turns) sum += item_us + n * together_us;
-    return sum / bins;
+// us of a form: `launch`; of a portion's item `item` and, a turn, `alone` or `together`; of a single token's
+// `single` and `single_alone`.  Times of turns are at head size 128.
+struct Form {
+  double launch, item, alone, together, single, single_alone;
+};
+constexpr double kSingleTogether = 1.19;     // a single token's turn where its unit has others
+constexpr Form kOneSet{5.2, 1.3, 1.42, 0.97, 2.0, 1.75}, kTwoSets{2.3, 4.45, 1.0, 1.12, 6.0, 0.94},
+    kFourSets{0.0, 5.0, 0.81, 0.715, 4.5, 0.845}, kRows16{3.8, 0.86, 1.53, 0.64, 0.0, 1.55};
+
+// The estimate's two kinds of times, by head size and by what makes a score.
+struct Rates {
+  double products, memory;
+  double alone(const Form& f, const Item& i) const {
+    return i.turns * (i.single ? f.single_alone * memory : f.alone * products);
   }
-  struct Bin { double us; int items, last; };
-  std::vector<Bin> bin(bins, Bin{0.0, 0, 0});
-  for (int n : turns) {
-    Bin* least = &bin[0];
-    for (Bin& b : bin)
-      if (b.us < least->us) least = &b;
-    least->us += item_us + n * together_us, least->items += 1, least->last = n;
+  double own(const Form& f, const Item& i) const { return i.single ? f.single : f.item; }
+  double together(const Form& f, const Item& i) const {
+    return own(f, i) + i.turns * (i.single ? kSingleTogether * memory : f.together * products);
+  }
+};
+
+double mean_share(const Form& f, const Rates& r, const std::vector<Item>& items, int bins) {
+  double sum = 0.0;
+  for (const Item& i : items) sum += r.together(f, i);
+  return sum / bins;
+}
+
+// Several workgroups a unit: `rest` of what is not the bound is not hidden behind it.
+double side_by_side(const Form& f, const Rates& r, const std::vector<Item>& items, int bins, double rest) {
+  double longest = 0.0;
+  for (const Item& i : items) longest = std::max(longest, r.alone(f, i));
+  const double share = mean_share(f, r, items, bins);
+  return f.launch + std::max(longest, share) + rest * std::min(longest, share);
+}
+
+double handed_out(const Form& f, const Rates& r, const std::vector<Item>& items, int bins) {
+  if ((int64_t)items.size() > 4 * (int64_t)bins) return f.launch + mean_share(f, r, items, bins);
+  struct Unit {
+    double us, shown;       // with every item's time together; with that of its only item alone
+    bool operator<(const Unit& o) const { return us > o.us; }       // the heap's first is free first
+  };
+  std::vector<Unit> units(bins, Unit{0.0, 0.0});
+  for (const Item& i : items) {
+    std::pop_heap(units.begin(), units.end());
+    Unit& u = units.back();
+    const bool first = u.us == 0.0;
+    u.us += r.together(f, i);
+    u.shown = first ? r.own(f, i) + r.alone(f, i) : u.us;
+    std::push_heap(units.begin(), units.end());
   }
   double most = 0.0;
-  for (const Bin& b : bin) most = std::max(most, b.items > 1 ? b.us : item_us + b.last * alone_us);
-  return most;
+  for (const Unit& u : units) most = std::max(most, u.shown);
+  return f.launch + most;
 }
-}  // namespace
 
-extern "C" int ts_attention_prefill_plan(int head_dim, int page_size, int rows_per_token, int heads, int reach,
-                                         int entries, const int* q_lens, const int* starts, int* sets) {
+int plan(int head_dim, int page_size, int rows_per_token, int heads, int reach, int entries, const int* q_lens,
+         const int* starts, bool extras, int* sets) {
   *sets = 0;
   if (!(page_size >= 16 && (page_size & (page_size - 1)) == 0)) return tiles_per_wave(head_dim);
   if ((head_dim != 64 && head_dim != 128) || g_prefill_variant == 0) return 4;
-  if (g_prefill_variant >= 3) {
+  if (g_prefill_variant >= 3 && g_prefill_variant <= 5) {
     *sets = g_prefill_variant == 3 ? 1 : g_prefill_variant == 4 ? 2 : 4;
     return *sets == 4 ? 4 : 8;
   }
   if (entries <= 0 || *std::max_element(q_lens, q_lens + entries) <= 1) return 4;
   try {
     const int tokens16 = 16 / rows_per_token, bins = std::max(1, compute_units() / heads);
-    const std::vector<int> four = item_turns(4 * tokens16, reach, entries, q_lens, starts),
-                           eight = item_turns(8 * tokens16, reach, entries, q_lens, starts);
-    const double of_head = head_dim == 64 ? 0.6 : 1.0;
-    // one set: a unit has two items at a time, which slow one another down
-    const double crowd = std::min(1.0, std::max(0.0, (double)eight.size() / bins - 1.0));
-    double sum = 0.0;
-    for (int n : eight) sum += n;
-    const double one_set = std::max(0.5 + eight[0] * (1.04 + 0.26 * crowd) * of_head,
-                                    (sum * 0.97 * of_head + 0.25 * eight.size()) / bins);
-    const double two_sets = handed_out(eight, bins, 3.0, 0.78 * of_head, 1.05 * of_head);
-    const double four_sets = handed_out(four, bins, 2.0, 0.53 * of_head, 0.68 * of_head);
-    *sets = four_sets < one_set && four_sets < two_sets ? 4 : two_sets < one_set ? 2 : 1;
-    return *sets == 4 ? 4 : 8;
+    const std::vector<Item> four = items_of(4 * tokens16, reach, entries, q_lens, starts),
+                            eight = items_of(8 * tokens16, reach, entries, q_lens, starts);
+    Rates tall = head_dim == 64 ? Rates{0.68, 0.57} : Rates{1.0, 1.0}, rows16 = tall;
+    // (with scores of more than a product that kernel is another, at 128 half as fast: 200 single tokens of 300
+    // beside 33 80 us, in one set 60; at 64 33 and 39)
+    if (extras) tall.products *= 1.34, rows16.products *= 1.27, rows16.memory *= 1.24;
+    const double us[] = {side_by_side(kOneSet, tall, eight, bins, 0.0), handed_out(kTwoSets, tall, eight, bins),
+                         handed_out(kFourSets, tall, four, bins),
+                         extras && head_dim == 128 ? HUGE_VAL : side_by_side(kRows16, rows16, four, bins, 0.28)};
+    constexpr int kSets[] = {1, 2, 4, 0}, kTiles[] = {8, 8, 4, 4};
+    const int best = (int)(std::min_element(us, us + 4) - us);
+    *sets = kSets[best];
+    return kTiles[best];
   } catch (const std::exception&) {      // no memory for the estimate: any step may take this kernel
-    *sets = 0;
     return 4;
   }
+}
+}  // namespace
+
+extern "C" int ts_attention_prefill_plan(int head_dim, int page_size, int rows_per_token, int heads, int reach,
+                                         int entries, const int* q_lens, const int* starts, int* sets) {
+  return plan(head_dim, page_size, rows_per_token, heads, reach, entries, q_lens, starts, false, sets);
+}
+extern "C" int ts_attention_prefill_plan_scores(int head_dim, int page_size, int rows_per_token, int heads, int reach,
+                                                int entries, const int* q_lens, const int* starts, int* sets) {
+  return plan(head_dim, page_size, rows_per_token, heads, reach, entries, q_lens, starts, true, sets);
 }
 
 int launch_attention_prefill_tall(const AttentionMfmaArgs& args, hipStream_t stream);

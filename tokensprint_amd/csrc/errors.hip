@@ -13,4 +13,4 @@ void ts_set_error(const char* fmt, ...) {
 extern "C" const char* ts_last_error() { return g_error; }
 
 // Version of the C interface; the Python loader refuses a library with another one.
-extern "C" int ts_abi_version() { return 2; }
+extern "C" int ts_abi_version() { return 3; }

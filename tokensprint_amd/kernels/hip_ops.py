@@ -18,7 +18,7 @@ from tokensprint_amd.kernels.build import build, find_library
 from tokensprint_amd.kernels.dispatch import default_dispatch
 from tokensprint_amd.kernels.stream import NormedPair, PreparedRows, UnmergedRows
 
-ABI_VERSION = 2
+ABI_VERSION = 3
 _TYPE_CODE = {torch.float32: 0, torch.bfloat16: 1}
 
 
@@ -1150,15 +1150,16 @@ class HipOps:
         d = self.dispatch
         # (the same for every layer of a step with the same reach)
         reach = self._reach(a)
-        key = ("prefill", group, a.nkv, a.hd, a.page_size, reach, d.portion_tiles,
+        key = ("prefill", group, a.nkv, a.hd, a.page_size, reach, extras, d.portion_tiles,
                d.portion_tokens, d.single_token_tiles)
         if key not in batch.plans:
             plan = 0, 0
             if self._prefill_tiles(batch, a.nkv, group) is not None:
                 n, sets = batch.num_entries, c_int()
-                tpw = self.lib.ts_attention_prefill_plan(
-                    a.hd, a.page_size, rows_per_token, a.nkv * head_blocks, reach, n,
-                    (c_int * n)(*batch.q_lens), (c_int * n)(*batch.starts), byref(sets))
+                choose = (self.lib.ts_attention_prefill_plan_scores if extras
+                          else self.lib.ts_attention_prefill_plan)
+                tpw = choose(a.hd, a.page_size, rows_per_token, a.nkv * head_blocks, reach, n,
+                             (c_int * n)(*batch.q_lens), (c_int * n)(*batch.starts), byref(sets))
                 plan = tpw, sets.value
             batch.plans[key] = plan
         tpw, m.sets = batch.plans[key]
