@@ -762,18 +762,22 @@ def test_paged_attention_long_portions(ops, gpu_device, nq, nkv, hd, page, windo
     torch.testing.assert_close(out[pick].float(), ref.float(), **tol(dtype))
 
 
+MANY_ITEMS = [(0, 1212), (333, 1), (50, 1027), (700, 700)]
+FEW_ITEMS = [(0, 700), (333, 1), (50, 500), (700, 300)]
+
+
 @pytest.mark.parametrize("window", [40, 100, 333])
 @pytest.mark.parametrize("spans,kernel", [
-    ([(0, 1212), (333, 1), (50, 1027), (700, 700)], 2),     # many items: turns of 32 keys
-    ([(0, 700), (333, 1), (50, 500), (700, 300)], 2),       # few items: turns of 64, two sets
-    ([(0, 1212), (333, 1), (50, 1027), (700, 700)], 3),     # turns of 64, eight tiles an item
-], ids=["turns-of-32", "two-sets", "eight-tiles"])
+    (MANY_ITEMS, 2), (MANY_ITEMS, 0), (MANY_ITEMS, 3), (FEW_ITEMS, 4), (FEW_ITEMS, 5),
+    ([(37 * i % 1100, 1) for i in range(143)], 2),          # single tokens: 16 rows, three waves of four idle
+], ids=["default", "16-rows", "one-set", "two-sets", "four-sets", "single-tokens"])
 def test_long_portions_under_a_window_come_out_the_same_every_time(ops, gpu_device, window, spans,
                                                                    kernel):
     """Under a window the waves of a workgroup have different blocks to skip, so some run a
     turn ahead of the others; a block sent for into a buffer that a slower wave still reads
-    would show as a result that differs from launch to launch.  Each of the three kernels
-    for long portions of this head size."""
+    would show as a result that differs from launch to launch.  Each kernel for long portions
+    of this head size: 16 rows a wavefront with a ring of three buffers, 32 rows with rings
+    of two and one, two and four sets of wavefronts."""
     dtype, nq, nkv, hd, page = torch.bfloat16, 16, 8, 128, 16
     batch, cache, table, _ = paged_scenario(gpu_device, dtype, nkv=nkv, hd=hd, page_size=page,
                                             spans=spans, seed=35)
@@ -1069,15 +1073,15 @@ def test_paged_attention_finds_one_far_key(ops, gpu_device, dtype):
 @pytest.mark.parametrize("nq,nkv,hd,page,window", [(16, 8, 128, 16, None), (16, 8, 128, 64, 700),
                                                    (8, 8, 96, 16, None), (6, 2, 64, 32, None),
                                                    (40, 2, 32, 16, 300)])
-@pytest.mark.parametrize("kernel", [2, 0, 3], ids=["default", "turns-of-32", "eight-tiles"])
+@pytest.mark.parametrize("kernel", [2, 0, 3], ids=["default", "16-rows", "one-set"])
 def test_attend_long_portions(ops, gpu_device, nq, nkv, hd, page, window, kernel):
     """Portions of prompts long enough for the kernels in which a wavefront walks several
     query tiles: with and without norm weights, rotation, and keys in the row; groups of
     3 and 20 heads, whose 16 rows are not a whole number of tokens (a row past a tile's
     tokens must not be computed with that tile's key range and stored).  Head sizes 64 and
-    128 have three kernels for this (turns of 64 keys with two sets of waves an item, with
-    eight tiles an item, and turns of 32 keys), chosen by the number of items: each is
-    made to take the same step."""
+    128 have two kernels for this (16 rows a wavefront, and 32 with one, two and four sets of
+    waves an item), chosen by an estimate of the step's items: both are made to take the
+    same step, beside the choice."""
     if kernel != 2 and hd not in (64, 128):
         pytest.skip("one kernel for this head size")
     ops.lib.ts_attention_prefill_variant(kernel)
@@ -1123,7 +1127,7 @@ def _attend_long_portions(ops, gpu_device, nq, nkv, hd, page, window):
 
 
 @pytest.mark.parametrize("page", [16, 64])
-@pytest.mark.parametrize("kernel", [2, 0, 3], ids=["default", "turns-of-32", "eight-tiles"])
+@pytest.mark.parametrize("kernel", [2, 0, 3], ids=["default", "16-rows", "one-set"])
 def test_long_portion_finds_one_far_key(ops, gpu_device, kernel, page):
     """Random keys would hide a block that a kernel for long portions skips, reads from the
     wrong page or masks by mistake: among two thousand keys one more changes a bfloat16

@@ -1208,8 +1208,9 @@ class HipOps:
     def _attention_tiles(self, batch, tokens, longest_first=False):
         """Device list of (entry, first flat token, tokens) cutting every entry of the batch
         into runs of at most `tokens` consecutive tokens; made once per step and size.
-        `longest_first`: sorted by the number of keys a run's last token sees, most first
-        (the kernels for long portions take them in that order)."""
+        `longest_first`: sorted by the number of keys a run's last token sees, most first (of
+        the kernels for long portions, those of head sizes 64 and 128 take them in that order,
+        the others pair runs from both ends of it)."""
         key = ("attn_tiles", tokens, longest_first)
         if key not in batch.plans and batch.max_q_len == 1:
             # a step of single tokens: tile i is entry i.  No order: the host's `starts` of a
