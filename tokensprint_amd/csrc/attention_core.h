@@ -190,8 +190,8 @@ __device__ __forceinline__ void load_kv_block_wide(KvBlock<HD>& b, const Attenti
 
 // The same block with its keys as they lie in memory, 64 lanes asking for 1 KB of a page's rows in
 // one run; spread_keys then brings them into the operand's order through LDS.  A compute unit takes
-// a load in about 2 cycles for each 128-byte line that a quarter of its lanes touches: lanes that each
-// ask for 16 bytes of a row of their own take 27 ns a kilobyte, these 8.  It counts where a unit
+// a kilobyte in 7 ns where neighbouring lanes ask for neighbouring pieces, in 27 where each asks for 16 bytes
+// of a row of its own (of 32 lines, of 16 or of 8).  It counts where a unit
 // has little more than the loads of a first block to wait for (one request of 541 tokens,
 // 16 / 8 heads of 128: 7.5 -> 7.1 us a launch); where memory is the limit the way through LDS is a
 // loss of 1 % (attention_decode_kernel's ranked form).

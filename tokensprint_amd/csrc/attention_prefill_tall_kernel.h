@@ -74,9 +74,9 @@ __device__ __forceinline__ void attention_prefill_tall(const AttentionMfmaArgs& 
   // Where things lie in LDS.  A key's row, in key order, its 16-byte pieces exchanged so that
   // the sixteen rows that lanes read together lie in different banks; values as their pages hold
   // them (a head element's sixteen keys, 32 bytes), halves exchanged every eight elements for
-  // the same reason.  A load of 64 pieces then names whole lines of 128 bytes: a compute unit
-  // takes a load in 2.1 cycles per line it touches, 18 for a load of eight lines and 66 for one that
-  // names 16 or 32 bytes of 32 lines.
+  // the same reason.  Neighbouring lanes then name neighbouring pieces: a compute unit takes a load of
+  // 1 KB in 18 cycles where they do, in 66 where each names 16 bytes in a line that its neighbours do not (in
+  // the order of the operands, 32 lines in all).
   unsigned k_off[OFFS], v_off[OFFS];           // of this lane's piece in its sixteen keys, bytes
 #pragma unroll
   for (int i = 0; i < OFFS; ++i) {

@@ -97,10 +97,10 @@ __global__ __launch_bounds__(256) void conv_silu_run_kernel(
 // on 16 bytes: loads and stores of 16 bytes, and no look at a token's entry where the thread's
 // tokens and the inputs in front of them are one entry's (30 against 39 us for 2,048 tokens of
 // 6,144 channels).  Four taps are a channel's 16 bytes: one by one, four of 64 lanes' 256 bytes a load, they
-// cost a unit more than the inputs (a load takes 2.1 cycles per line of 128 bytes it names, and sixteen of
-// those named 32 each; 31.3 -> 27.3 us).  No load hangs on a condition (each was waited for before the
-// next was sent; in a prompt's step 27.9 -> 24.2 us, 4,096 channels 17.7 -> 14.5), and there are no more of
-// them than TAPS taps take (two taps of 6,144 channels 29.4 us with those of four, 21.9).
+// cost a unit more than the inputs (sixteen loads, each naming 32 lines of 128 bytes; 31.3 -> 27.3 us).  No load
+// hangs on a condition (each was waited for before the next was sent; in a prompt's step 27.9 -> 24.2 us, 4,096
+// channels 17.7 -> 14.5), and there are no more of them than TAPS taps take (two taps of 6,144 channels 29.4 us
+// with those of four, 21.9).
 constexpr int kConvRunTaps = 4;
 template <int TAPS, bool WIDE>        // WIDE: four taps, and w on 16 bytes
 __global__ __launch_bounds__(256) void conv_silu_run4_kernel(

@@ -133,8 +133,9 @@ class Dispatch:
     decode_items: int = 512
     #: a step that holds a portion of at least `portion_tokens` tokens takes the kernel
     #: for long portions from this many 16-row wave tiles (one portion of 256 tokens 11.0
-    #: against the general kernel's 16.6 us, 1,024 tokens 21.5 against 34.4, 1,536 tokens
-    #: 34.0 against 96.8; below that the two are equal)
+    #: against the general kernel's 16.6 us in tiles of 16 rows, and since in tiles of 32
+    #: 1,024 tokens 18.7 against 34.4, 1,536 tokens 25.5 against 96.8; below that the two
+    #: are equal)
     portion_tiles: int = 256
     portion_tokens: int = 32
     #: a step of single tokens only takes it where the chip is full without splitting

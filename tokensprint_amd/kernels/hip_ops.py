@@ -1002,8 +1002,8 @@ class HipOps:
         extras = softcap is not None or slopes is not None or q_temp is not None
         if (q.dtype == torch.bfloat16 and cache.k_pages.dtype == torch.bfloat16
                 and head_dim % 16 == 0 and head_dim <= 256 and cache.page_size % 4 == 0):
-            # (scores with extras: the decode kernel and the kernel for short portions and
-            # mixed steps know them, the LDS-tiled kernels for long portions do not)
+            # (scores with extras: of the kernels for long portions those for pages of a power
+            # of two know them)
             if self._decode_fits(batch, num_kv_heads, num_heads // num_kv_heads, head_dim,
                                  cache.page_size, False):
                 self._attention_decode(a, batch, num_heads // num_kv_heads)
