@@ -116,8 +116,8 @@ __device__ __forceinline__ float load_past_caches(const float* p) {
 // thread takes E elements and asks for all of a group of GROUP splits of each before it uses the first:
 // the workgroup's last act, bound by its trips to memory and by its instructions (two elements a
 // thread and always eight splits: 1.5 us of 10.9 for four splits of 2 rows of 128, with one and four 0.8;
-// where a thread has more than one, one at a time is a trip each: 16 query heads of 128 over one key/value head,
-// 2,000 tokens, 15.4 us, now 14.6).
+// more splits and more than an element to a thread, two at a time: 16 query heads of 128 over one key/value head,
+// 2,000 tokens, 15.4 us one at a time, 14.5).
 template <int HD, int THREADS, int GROUP, int E>
 __device__ __forceinline__ void merge_splits_here(const float* partial_o, const float* partial_ml,
                                                   int64_t first_slot, int used, int rows, bf16_t* out,
@@ -546,15 +546,14 @@ __global__ __launch_bounds__(decode_waves<HD>() * kWave) void attention_decode_k
         ma.partial_o, ma.partial_ml, (int64_t)item * ma.num_splits * 16, used, rows, out, a.sink, kvh * group + hb * 16);
   };
   constexpr std::integral_constant<int, 1> one;
+  constexpr std::integral_constant<int, 2> two;
   constexpr std::integral_constant<int, 4> four;
   constexpr std::integral_constant<int, 8> eight;
-  if (rows * HD <= NW * kWave) {
-    if (used <= 4) merge(four, one);
-    else merge(eight, one);
-  } else {
-    if (used <= 4) merge(four, four);
-    else merge(eight, std::integral_constant<int, 2>());
-  }
+  // (up to four splits an element at a time whatever a thread has: four at a time 8.1 us in place of 7.0 where it
+  // has two, and a fourth form beside these three costs every launch 0.15)
+  if (__builtin_expect(used <= 4, 1)) merge(four, one);
+  else if (__builtin_expect(rows * HD <= NW * kWave, 1)) merge(eight, one);
+  else merge(eight, two);
 }
 
 int launch_attention_merge(const AttentionMfmaArgs& args, hipStream_t stream);
